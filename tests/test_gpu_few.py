@@ -1,0 +1,107 @@
+"""GPU: short-list rows shared between workgroups that hold them in registers (ws_few.h), through the C ABI against the CPU
+oracle on identical seeded inputs, at the sizes where its split can go wrong: vocabularies one token either side of a vector,
+of a chunk and of a share, rows off every alignment, the longest history it takes, tokens with several bias entries, ties at
+the threshold, rows it has to hand back. Bars as in test_gpu_sample.py (gpu_cases.compare_rows)."""
+import numpy as np
+import pytest
+import torch
+
+import gpu_cases as gc
+
+pytestmark = pytest.mark.gpu
+
+
+def case(rows, V, dtype="f32", top_k=40, min_p=0.0, n_hist=300, n_bias=20, allowed=None, seed=3):
+    c = gc.make_cfg2(rows=rows, V=V, n_hist=n_hist, n_bias=n_bias)
+    rng = np.random.default_rng(seed)
+    c["top_k"][:] = top_k
+    c["min_p"][:] = min_p
+    if dtype == "bf16":
+        c["logits"], c["dtype"] = gc.f32_to_bf16_bits(c["logits"]), "bf16"
+    if allowed is not None:
+        words = (V + 31) // 32
+        c["allow"] = np.ascontiguousarray(np.packbits(rng.random((rows, words * 32)) < allowed, axis=1, bitorder="little").view(np.uint32))
+    return c
+
+
+def run(c, handed_back=0, max_differ=0, max_split=0, **more):
+    m = gc.pkg()
+    d = gc.upload(c, hints=True, min_p_hint=True)
+    smp = gc.sampler_for(c, d, 1, kept_cap=1024, max_split=max_split, **more)
+    assert m.lib().ws_sample_batch_workspace_use(smp.desc) == m.WORK_MEETING  # (the rows are shared)
+    for _ in range(2):  # the second launch finds the workspace as the first left it
+        smp.run()
+    res = gc.compare_rows(c, smp, range(c["rows"]), 1)
+    assert res["differ"] <= max_differ and res["exact"] + res["differ"] == c["rows"], res
+    fl = smp.flags.cpu().numpy()
+    back = int(((fl & m.FLAG_ROUTE_HANDED_BACK) != 0).sum())
+    assert back <= handed_back and int(((fl & m.FLAG_ROUTE_SHORT) != 0).sum()) + back == c["rows"], fl
+    assert not smp.workspace.any().item(), "the workspace is not zero after the launch"
+    return smp
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("V", [4097, 8191, 8200, 32771, 50257, 65535, 151935, 151937])
+def test_vocabularies_off_every_boundary(V, dtype):
+    run(case(3, V, dtype))
+
+
+@pytest.mark.parametrize("max_split", [2, 3, 4, 7, 16])
+def test_any_number_of_parts(max_split):
+    """Parts that are no power of two; two parts of 40960 tokens, the most a workgroup holds."""
+    run(case(2, 81920, top_k=50), max_split=max_split)
+
+
+@pytest.mark.parametrize("dtype,top_k", [("f32", 1), ("f32", 512), ("bf16", 513), ("f32", 1024), ("bf16", 64)])
+def test_top_k_from_one_to_the_largest(dtype, top_k):
+    run(case(2, 40003, dtype, top_k=top_k), max_differ=1 if dtype == "bf16" else 0)
+
+
+@pytest.mark.parametrize("dtype,allowed", [("f32", 0.1), ("bf16", 0.5)])
+def test_rows_with_an_allow_mask(dtype, allowed):
+    run(case(3, 33001, dtype, allowed=allowed))
+
+
+@pytest.mark.parametrize("min_p", [1.0, 0.2, 0.05])
+def test_min_p_without_a_top_k(min_p):
+    run(case(4, 60001, top_k=0, min_p=min_p), max_differ=1, handed_back=1 if min_p < 0.1 else 0)
+
+
+def test_long_histories_and_repeated_bias_entries():
+    """9000 ids of few tokens, so that counts are in the hundreds, and bias lists that name tokens of the history, some of
+    them three times (their values are added in the order of the list)."""
+    c = case(2, 90001, n_hist=9000, n_bias=60)
+    c["hist"] %= 700
+    c["bias_ids"][:, 20:40] = c["bias_ids"][:, :20]
+    c["bias_ids"][:, 40:50] = c["bias_ids"][:, :10]
+    c["bias_ids"][:, 50:] = c["hist"][:, :10]
+    run(c)
+
+
+def test_ties_at_the_threshold_and_a_row_of_one_value():
+    """Logits rounded to halves: the threshold falls among ties; more of them than a wave lists, and the row is handed back.
+    A row of equal logits is handed back as well and still the oracle's."""
+    c = case(4, 30000, top_k=20, n_hist=0, n_bias=0)
+    c["logits"][:2] = np.round(c["logits"][:2] * 2) / 2
+    c["logits"][3] = 1.25
+    run(c, handed_back=3)
+
+
+def test_query_and_entropy():
+    """Probability of a named token and the kept set's entropy from the sorted candidates."""
+    m = gc.pkg()
+    c = case(6, 32003, top_k=40)
+    want = [gc.oracle_row(c, r, 1) for r in range(6)]
+    query = np.array([w[1]["id"][r % 2] for r, w in enumerate(want)], np.int32)
+    query[4] = np.setdiff1d(np.arange(c["V"]), want[4][1]["id"])[0]
+    query[5] = -1
+    smp = run(c, query=torch.from_numpy(query).cuda(), want_entropy=True)
+    qp, ent = smp.query_prob.cpu().numpy(), smp.entropy.cpu().numpy()
+    for r, (o, kept, _) in enumerate(want):
+        hit = kept["p"][kept["id"] == query[r]]
+        p_want = float(hit[0]) if hit.size else 0.0
+        assert abs(qp[r] - p_want) <= 1e-6 * max(p_want, 1e-300), (r, qp[r], p_want)  # the bar of the token's probability
+        pk = kept["p"][kept["p"] > 0]
+        h_want = float(-(pk * np.log(pk)).sum())
+        assert abs(ent[r] - h_want) <= 1e-6 * max(1.0, h_want), (r, ent[r], h_want)
+    assert not (smp.flags.cpu().numpy() & m.FLAG_APPROX_ENTROPY).any()

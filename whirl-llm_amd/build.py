@@ -17,6 +17,7 @@ SRC_FUSED = os.path.join(HERE, "csrc", "ws_fused.hip")  # the single-sweep sampl
 SRC_SPLIT = os.path.join(HERE, "csrc", "ws_split.hip")  # the same kernel for rows split over several workgroups
 SRC_KEPT = [os.path.join(HERE, "csrc", f) for f in ("ws_fused_kept.hip", "ws_split_kept.hip")]  # both once more, with the kept-set dump
 SRC_SHORT = os.path.join(HERE, "csrc", "ws_short.hip")  # the short-list kernel for batches whose rows all have a bounded top-k
+SRC_FEW = os.path.join(HERE, "csrc", "ws_few.hip")  # short-list rows shared between workgroups that hold them in registers
 SRC_LEAN = os.path.join(HERE, "csrc", "ws_lean.hip")  # the lean single-sweep kernel for batches of unsplit rows
 # packed FP32 instructions are switched off for every device compile of this repository
 FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
@@ -43,10 +44,10 @@ def build(verbose=True):
     so = os.path.join(HERE, "libwhirl_sampling_hip.so")
     co = os.path.join(HERE, "whirl_sampling_gfx950.co")
     host = os.path.join(HERE, "libwhirl_sampling_host.so")
-    # the five translation units and the bare code object side by side (each takes a minute or two), then the link
+    # the translation units and the bare code object side by side (each takes a minute or two), then the link
     objdir = os.path.join(HERE, "csrc", "obj")
     os.makedirs(objdir, exist_ok=True)
-    srcs = (SRC, SRC_FUSED, SRC_SPLIT, *SRC_KEPT, SRC_LEAN, SRC_SHORT)
+    srcs = (SRC, SRC_FUSED, SRC_SPLIT, *SRC_KEPT, SRC_LEAN, SRC_SHORT, SRC_FEW)
     objs = [os.path.join(objdir, os.path.basename(src)[:-4] + ".o") for src in srcs]
     jobs = [[hipcc, *FLAGS, "-fPIC", "-c", "-o", obj, src] for obj, src in zip(objs, srcs)]
     jobs.append([hipcc, *FLAGS, "--genco", "-o", co, SRC])

@@ -37,6 +37,9 @@ int prepare_lean(unsigned lds_limit);
 // ws_short.hip: the short-list kernel for batches whose rows all have a bounded top-k
 int launch_short(hipStream_t stream, const BatchArgs& a, unsigned blocks, unsigned lds_bytes, unsigned lds_limit);
 int prepare_short(unsigned lds_limit);
+// ws_few.hip: the same rows shared between workgroups that hold them in registers
+int launch_few(hipStream_t stream, const BatchArgs& a, unsigned lds_bytes, unsigned lds_limit);
+int prepare_few(unsigned lds_limit);
 }  // namespace ws
 
 namespace {
@@ -53,6 +56,8 @@ constexpr uint32_t kStaticLds = 4096u;
 #endif
 // the short-list kernel's own words and those of both builds of the three-pass code it calls (8.2 KiB)
 constexpr uint32_t kStaticShort = 9216u;
+// the same for the kernel of few rows
+constexpr uint32_t kStaticFew = 10240u;
 // the lean kernel's own tables and those of the three-pass code it calls
 #ifdef WS_PHASE_TIMERS
 constexpr uint32_t kStaticLean = 11776u + 768u;
@@ -71,8 +76,10 @@ struct BatchPlan {
     uint32_t lean_tie;    // its second histogram copy (0: none), its dynamic LDS, and the spare LDS of the three-pass code it calls
     uint32_t lean_total;
     uint32_t lean_fb_tie;
+    bool vec_rows;        // rows of whole aligned 128-bit vectors
     bool shortlist;       // the short-list kernel takes the batch: every row has a top-k of at most top_k_max (the caller's word)
     uint32_t short_ab, short_cnt, short_total, short_fb_tie, short_fb_ab;  // its LDS: bitmap at short_ab, rank words at short_cnt
+    uint32_t few_parts, few_total;  // short-list rows shared between this many workgroups each (0: not), and the dynamic LDS of those
     uint32_t split_log2;  // the most parts per row that pay for this batch
     uint64_t workspace_min;  // split rows: the least that lets them split (no staging areas), 0 when nothing is split
     uint64_t workspace;   // bytes for that
@@ -90,6 +97,32 @@ int compute_units() {
         known[dev].store(n, std::memory_order_relaxed);
     }
     return n > 0 ? n : 0;
+}
+
+// Few rows of the short-list kind: how many workgroups share a row. A share fits the registers of 512 threads (80 tokens
+// each) and has 2048 tokens at least; as many parts as the compute units allow, up to 16 - a wide top-k gets 8 at most, its
+// waves' lists need the room. Nobody waits for anybody, so more workgroups than compute units are no danger, only slower.
+void few_plan(const ws_batch* b, uint64_t cap, uint64_t maps, BatchPlan& p) {
+    p.few_parts = 0;
+    if (b->max_split == 1u || cap > ws::kFewLists) return;
+    const uint32_t cus = static_cast<uint32_t>(compute_units());
+    const uint32_t share = ws::kFewShare;
+    uint32_t most = b->top_k_max > 512u ? 8u : ws::kFewMaxParts;
+    if (b->max_split && b->max_split < most) most = b->max_split;
+    const uint32_t least = (b->vocab + share - 1u) / share;
+    uint32_t parts = cus / b->rows;
+    if (parts > most) parts = most;
+    if (parts > b->vocab / 2048u) parts = b->vocab / 2048u;
+    if (parts < least) parts = least;
+    if (cap > uint64_t{parts} * 1600u) return;  // (touched tokens of a share: room for 2048)
+    if (parts < 2u || parts > most || static_cast<uint64_t>(b->rows) * parts > 2ull * cus) return;
+    const uint64_t three = (cap * 8u > 65536u ? ((cap * 8u + 15u) & ~uint64_t{15}) : 65536u) + maps;
+    const uint64_t own = 32768u + ws::kFewShare * 2u;
+    const uint64_t total = own > three ? own : three;
+    if (total + kStaticFew > kMaxLds) return;
+    p.few_parts = parts;
+    p.few_total = static_cast<uint32_t>(total);
+    p.workspace = p.workspace_min = uint64_t{b->rows} * ws::kFewRowBytes;
 }
 
 BatchPlan plan_batch(const ws_batch* b) {
@@ -111,7 +144,7 @@ BatchPlan plan_batch(const ws_batch* b) {
     // fused sweep: rows of whole 128-bit vectors that fit the register cache, and LDS room for the per-rank counters
     // next to the histogram (the exact path reuses the histogram's LDS for them)
     const uint64_t esz = b->dtype == WS_DTYPE_F32 ? 4 : 2;
-    const bool vec_rows = b->vocab % 8u == 0 && (b->row_stride * esz) % 16u == 0 && reinterpret_cast<uintptr_t>(b->logits) % 16u == 0;
+    const bool vec_rows = p.vec_rows = b->vocab % 8u == 0 && (b->row_stride * esz) % 16u == 0 && reinterpret_cast<uintptr_t>(b->logits) % 16u == 0;
     const uint64_t fused_total = 65536u + maps + cap * 8u;
     // (a token's bias entries are counted in 11 bits of its rank word)
     const bool can_fuse = vec_rows && b->vocab <= 163840u && fused_total + kStaticLds <= kMaxLds && (!b->bias_ids || b->max_bias <= 2047u);
@@ -167,8 +200,8 @@ BatchPlan plan_batch(const ws_batch* b) {
     // per history / bias entry), and under it room for the three-pass layout of the rows it hands back.
     const bool word_k = b->top_k && b->top_k_max >= 1u && b->top_k_max <= 1024u;  // every row with a top-k: at most top_k_max
     const bool word_p = b->min_p && b->min_p_min > 0.0;                            // every row without: a min-p
-    p.shortlist = (b->top_k ? (word_k || word_p) : word_p) && (!b->top_k || b->top_k_max <= 1024u) && b->mode == WS_MODE_AUTO && vec_rows && !b->race &&
-                  !b->query_prob && !b->entropy && (!b->bias_ids || b->max_bias <= 2047u);
+    p.shortlist = (b->top_k ? (word_k || word_p) : word_p) && (!b->top_k || b->top_k_max <= 1024u) && b->mode == WS_MODE_AUTO && b->vocab >= 8u && !b->race &&
+                  (!b->bias_ids || b->max_bias <= 2047u);
     if (p.shortlist) {
         const uint64_t maps_s = uint64_t{nW} * 4u + ((uint64_t{nW} * 2u + 15u) & ~uint64_t{15});
         const uint64_t tabs_s = ((cap * 4u + 15u) & ~uint64_t{15}) + ((cap * 2u + 15u) & ~uint64_t{15});
@@ -189,18 +222,11 @@ BatchPlan plan_batch(const ws_batch* b) {
             p.short_total = static_cast<uint32_t>(st);
         }
     }
-    if (p.shortlist) {  // few rows: a row is shared by up to 16 workgroups of at least 8192 tokens each; nobody waits, so there is no bound on rows * parts but usefulness
+    if (p.shortlist) {
         p.lean = false;
         p.split_log2 = 0;
         p.workspace = p.workspace_min = 0;
-        if (b->max_split != 1u) {
-            const uint32_t cus = static_cast<uint32_t>(compute_units());
-            const uint32_t most = b->max_split ? b->max_split : 16u;
-            uint32_t lg = 0;
-            while (lg < 4u && (2u << lg) <= most && b->rows * (2u << lg) <= cus && b->vocab / (2u << lg) >= 8192u) ++lg;
-            p.split_log2 = lg;
-            if (lg) p.workspace = p.workspace_min = uint64_t{b->rows} * ws::kShortSplitRowBytes;
-        }
+        few_plan(b, cap, maps, p);
         p.err = WS_OK;
         return p;
     }
@@ -271,6 +297,7 @@ int prepare_all() {
     if (const int e = ws::prepare_fused_kept(kMaxLds - kStaticLds); e != 0) return e;
     if (const int e = ws::prepare_split_kept(kMaxLds - kStaticLds); e != 0) return e;
     if (const int e = ws::prepare_lean(kMaxLds - kStaticLean); e != 0) return e;
+    if (const int e = ws::prepare_few(kMaxLds - kStaticFew); e != 0) return e;
     return ws::prepare_short(kMaxLds - kStaticShort);
 }
 
@@ -499,7 +526,7 @@ uint64_t ws_sample_batch_workspace(const ws_batch* b) {
 int ws_sample_batch_workspace_use(const ws_batch* b) {
     const BatchPlan p = plan_batch(b);
     if (p.err != WS_OK || p.workspace == 0) return WS_WORK_NONE;
-    return p.split_log2 ? WS_WORK_MEETING : WS_WORK_TABLES;
+    return p.split_log2 || p.few_parts ? WS_WORK_MEETING : WS_WORK_TABLES;
 }
 
 namespace {
@@ -555,13 +582,24 @@ int sample_batch_on(void* stream, const ws_batch* b, const BatchPlan& p, unsigne
     a.query = b->query;
     a.query_prob = b->query_prob;
     a.entropy = b->entropy;
+    if (p.few_parts && can_split) {
+        a.few_parts = p.few_parts;
+        const uint32_t waves = p.few_parts * 8u;  // (512 threads a workgroup)
+        a.few_magic = static_cast<uint32_t>(((uint64_t{1} << 32) + waves - 1u) / waves);
+        // chunks of eight lanes, a line of memory; where rows lie off the lines a chunk straddles two, and longer ones straddle fewer
+        a.few_chunk_log2 = p.vec_rows ? 3u : 5u;
+        a.work = work;
+        a.fb_lds_tie = 0u;
+        a.fb_lds_ab = p.short_fb_ab;
+        return ws::launch_few(S(stream), a, p.few_total, kMaxLds - kStaticFew);
+    }
     if (p.shortlist) {
         a.lds_ab = p.short_ab;
         a.lds_cnt = p.short_cnt;
         a.fb_lds_tie = p.short_fb_tie;
         a.fb_lds_ab = p.short_fb_ab;
-        a.work = a.split_log2 ? work : nullptr;
-        return ws::launch_short(S(stream), a, b->rows << a.split_log2, p.short_total, kMaxLds - kStaticShort);
+        a.work = nullptr;
+        return ws::launch_short(S(stream), a, b->rows, p.short_total, kMaxLds - kStaticShort);
     }
     if (p.fused && a.split_log2)
         return (a.kept_ids ? ws::launch_split_kept : ws::launch_split)(S(stream), a, b->rows << a.split_log2, p.lds_total, kMaxLds - kStaticLds);
@@ -589,7 +627,10 @@ int ws_sample_batch_static(void* stream, const ws_batch* b) {
     const BatchPlan p = plan_batch(b);
     if (p.err != WS_OK) return p.err;
     if (!p.fused && !p.shortlist) return sample_batch_on(stream, b, p, nullptr, 0);  // (nothing may be left in the split rows' memory)
-    if (p.workspace_min > sizeof(scratch)) return WS_E_STATIC_LIMIT;  // more split rows than the library's own memory holds
+    if (p.workspace_min > sizeof(scratch)) {  // more split rows than the library's own memory holds
+        if (p.few_parts && b->max_split == 0u) return sample_batch_on(stream, b, p, nullptr, 0);  // (split by the library's own choice: not here)
+        return WS_E_STATIC_LIMIT;
+    }
     unsigned char* at = nullptr;
     if (const int e = scratch_address(&at); e != WS_OK) return e;
     return sample_batch_on(stream, b, p, at, sizeof(scratch));

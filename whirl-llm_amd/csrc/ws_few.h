@@ -1,0 +1,569 @@
+// The sampler for few rows: every row is shared by up to sixteen workgroups, each of which keeps its share of the row in
+// registers. It takes the rows the short-list kernel (ws_short.h) takes - a top-k of at most kShortMaxK, or no top-k but a
+// min-p - and ends with the same sort and rules.
+//
+// With few rows nothing streams: 600 KB over sixteen compute units are 3 us of loads, and what counts is the chain of
+// dependent steps. Against the short-list kernel's shared rows, whose workgroups met over a histogram of the head each,
+// this one is built to make that chain short:
+//   * the eight waves of a workgroup work on their own until they publish: a wave's threshold is the d-th largest of its
+//     64 lanes' maxima (ballots, no barrier, no histogram), its list and its sum of exp go straight from registers to the
+//     row's workspace. A row of P parts is 8 P wave shares;
+//   * the vectors of a row are dealt to the waves in chunks of eight lanes, so that tokens that are large together - the
+//     low ids of a vocabulary - end up in different waves' lists;
+//   * history counts are 16-bit words indexed by the token's place in the share (no ranks, no prefix sums): two barriers;
+//     a touched token's logit is asked for as soon as its id is known;
+//   * the part that arrives last - a ticket, nobody waits - reads the waves' headers and lists. With top_k at most the
+//     number of waves, the top_k-th largest of the waves' maxima bounds the row's top_k-th largest logit from below, so
+//     that about as many keys as top_k are left to sort.
+// What bounds it is that chain: parameters, ids, their tokens' logits, headers, keys are five trips to memory of about
+// 0.7 us, between them some 2500 instructions of the slowest wave. 512 threads rather than 1024: the cost of a wave's own
+// work (threshold, sums, publishing) is paid half as often, and a share still fits the registers. Measured against the
+// short-list kernel's shared rows (151936 fp32, microseconds a launch): one row, top-k 40: 20.6 -> 11.5; 64 rows of mixed
+// filters with 4096-id histories: 50 (126 when a row's min-p list ran over) -> 33; 32 rows of 50257, which went through
+// the three-pass kernel: 55.6 -> 15.0.
+#pragma once
+#include "ws_short.h"
+
+namespace ws {
+
+constexpr uint32_t kFewWaves = kFewMaxParts * WS_WAVES;
+// Workspace of a row: kFewKeys keys, slot by slot with one key a wave in each, then two words a wave ({maximum, threshold} as
+// order keys; the sum of exp against the maximum, its low thirteen bits holding the number of keys plus one, all of them
+// set when the wave could not list its share), then {parts arrived, largest logit so far as an order key}. Zero-filled
+// between launches; a word that has been written is not zero.
+constexpr uint32_t kFewKeys = 7648u, kFewHead = kFewKeys * 8u, kFewCtrl = kFewHead + kFewWaves * 16u;
+static_assert(kFewCtrl + 256u <= kFewRowBytes, "a row's workspace");
+constexpr uint32_t kFewBad = 0x1fffu;
+constexpr uint32_t kFewExt = 2048u;  // touched tokens of a share
+constexpr uint32_t kFewDup = 0x4000u, kFewTaken = 0x8000u;  // in a token's 16-bit word, above its history count: a second bias entry, somebody takes it
+constexpr uint32_t kFewDups = 64u;  // bias entries of tokens that another entry has taken
+
+struct FewShared {
+    ShortShared sh;
+    uint32_t dup_at[kFewDups], dup_j[kFewDups];
+    float dup_v[kFewDups];
+    float red_f[WS_WAVES];
+    uint32_t w[16];
+    double u;
+};
+
+// the largest prefix (bits 31 .. 14) of an order key that at least d lanes of the wave reach, two bits a step
+__device__ __forceinline__ uint32_t few_lane_threshold(uint32_t k32, uint32_t d) {
+    uint32_t at = 0u;
+#pragma unroll 1
+    for (int b = 30; b >= 14; b -= 2) {
+        const uint32_t c1 = at | (1u << b), c2 = at | (2u << b), c3 = at | (3u << b);
+        const uint32_t n1 = static_cast<uint32_t>(__popcll(__ballot(k32 >= c1))), n2 = static_cast<uint32_t>(__popcll(__ballot(k32 >= c2))),
+                       n3 = static_cast<uint32_t>(__popcll(__ballot(k32 >= c3)));
+        at = n3 >= d ? c3 : (n2 >= d ? c2 : (n1 >= d ? c1 : at));
+    }
+    return at;
+}
+__device__ __forceinline__ uint32_t lanes_before(uint64_t m) {  // set bits of m below this lane
+    return __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(m >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(m), 0u));
+}
+
+// LDS: [0, 32 KiB) the list, [32 KiB, 64 KiB) its sorted copy while it is short; the history counts from 32 KiB on (they are
+// dead by then).
+template <int DT, bool MASKED, int NV>
+__device__ __forceinline__ bool few_row(const BatchArgs& A, const uint32_t row, const uint32_t part, FewShared& F, bool& finisher) {
+    extern __shared__ __align__(16) unsigned char lds[];
+    constexpr uint32_t TPV = DT == 0 ? 4u : 8u;  // tokens in a 128-bit vector
+    static_assert(NV * TPV * WS_BLOCK <= kFewShare, "tokens a share");
+    ShortShared& S = F.sh;
+    const uint32_t t = threadIdx.x, lane = t & 63u;
+    const uint32_t wv = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(t >> 6)));
+    const uint32_t V = A.vocab;
+    const unsigned char* base = static_cast<const unsigned char*>(A.logits) + static_cast<size_t>(row) * A.row_stride * (DT == 0 ? 4u : 2u);
+    const uint32_t* allow = MASKED ? A.allow + static_cast<size_t>(row) * A.allow_stride : nullptr;
+    finisher = false;
+#ifdef WS_SHORT_TIMERS
+    const long long wss_t0 = clock64();
+#endif
+
+    // ---- this thread's vectors: chunk c of the row is wave c mod G's; vector k of a lane lies in its wave's chunk number
+    // k * (chunks a load) + lane / (lanes a chunk)
+    const uint32_t G = A.few_parts * WS_WAVES, g = part * WS_WAVES + wv, cl = A.few_chunk_log2;
+    const uint32_t nv = (V + TPV - 1u) / TPV;
+    const uint32_t j_part = V % TPV ? nv - 1u : 0xffffffffu;
+    const uint32_t n_vec = (nv + 64u * G - 1u) / (64u * G);  // vectors a lane has
+    uint4 q[NV];
+    uint32_t na[NV];
+    auto vec_of = [&](uint32_t k) { return ((((k << (6u - cl)) + (lane >> cl)) * G + g) << cl) + (lane & ((1u << cl) - 1u)); };
+#pragma unroll
+    for (uint32_t k = 0; k < NV; ++k) {
+        const uint32_t j = vec_of(k);
+        q[k] = row_vector<DT>(base, j, V);
+        na[k] = MASKED ? allow[min(j * TPV, V - 1u) >> 5] : 0xffffffffu;
+    }
+    uint32_t* cnt = reinterpret_cast<uint32_t*>(lds + 32768);  // two 16-bit counts a word; bit 15 of a count: somebody takes the token
+    const bool lists = A.hist || A.bias_ids;
+    if (lists)
+#pragma unroll
+        for (uint32_t k = 0; k < NV * TPV / 8u + (NV * TPV % 8u ? 1u : 0u); ++k) reinterpret_cast<uint4*>(cnt)[k * WS_BLOCK + t] = make_uint4(0u, 0u, 0u, 0u);
+
+    // ---- the row's parameters
+    const LeanRowParams P = load_row_params(A, row);
+    WSS_MARK(0);  // parameters in
+    const float inv_t = P.inv_t;
+    const uint32_t top_k = P.top_k, nh = P.nh, nb = P.nb, n_all = nh + nb;
+    const double min_p = P.min_p;
+    const bool by_k = top_k >= 1u && top_k <= kShortMaxK && top_k <= V;  // the top_k largest decide
+    const bool by_p = top_k == 0u && min_p > 0.0 && min_p <= 1.0;      // no top-k: what the min-p floor lets through decides
+    const bool not_mine = !(by_k || by_p) || !(inv_t > 0.f) || n_all > A.patch_cap;
+
+    // ---- history and bias entries: those of this share are counted, and the first entry of each token puts it, with its
+    // logit, on a list (touched tokens: `ext`). A token that both lists name stands there twice; the bias entry's stays.
+    const uint32_t slots = kFewKeys / G;
+    uint4* ext = reinterpret_cast<uint4*>(lds);  // {token | kExtBias, logit, bias, place in the bias list}
+    constexpr uint32_t kExtBias = 0x80000000u;
+    const bool any_ext = lists && !not_mine && n_all;  // uniform
+    if (t < 2u) F.w[t] = 0u;                           // bias entries of tokens another entry has taken; length of `ext`
+    // this share's place of a token; 0xffffffff: not of this share
+    auto place_of = [&](uint32_t id) {
+        const uint32_t v = id / TPV, c = v >> cl;
+        const uint32_t cq = static_cast<uint32_t>((static_cast<uint64_t>(c) * A.few_magic) >> 32), cg = c - cq * G;  // c / G, c mod G
+        const uint32_t at = (((cg % WS_WAVES) * (NV * 64u) + (cq << cl) + (v & ((1u << cl) - 1u))) * TPV) + id % TPV;
+        return id < V && cg / WS_WAVES == part ? at : 0xffffffffu;
+    };
+    if (any_ext) {
+        const int32_t* hist_ids = A.hist + P.h0;
+        const int32_t* bias_ids = A.bias_ids + P.b0;
+        const float* bias_vals = A.bias_vals + P.b0;
+        constexpr uint32_t kR = 4u;  // entries a thread at a time, their loads together
+        auto four = [&](auto is_bias, uint32_t n, uint32_t j0, bool first) __attribute__((always_inline)) {
+            constexpr bool BIAS = decltype(is_bias)::value;
+            uint32_t id[kR], li[kR], raw[kR], al[kR];
+            float bv[kR];
+#pragma unroll
+            for (uint32_t r = 0; r < kR; ++r) {
+                const uint32_t j = j0 + r * WS_BLOCK + t;
+                id[r] = 0xffffffffu;
+                if (j0 + r * WS_BLOCK < n && j < n) id[r] = static_cast<uint32_t>((BIAS ? bias_ids : hist_ids)[j]);
+            }
+            if (first) __syncthreads();  // the counts are clear
+#pragma unroll
+            for (uint32_t r = 0; r < kR; ++r) {
+                if (j0 + r * WS_BLOCK >= n) continue;  // uniform
+                li[r] = place_of(id[r]);
+                if (li[r] != 0xffffffffu) {
+                    raw[r] = DT == 0 ? reinterpret_cast<const uint32_t*>(base)[id[r]] : static_cast<uint32_t>(reinterpret_cast<const uint16_t*>(base)[id[r]]) << 16;
+                    al[r] = MASKED ? allow[id[r] >> 5] >> (id[r] & 31u) : 1u;
+                    bv[r] = BIAS ? bias_vals[j0 + r * WS_BLOCK + t] : 0.f;
+                }
+            }
+#pragma unroll
+            for (uint32_t r = 0; r < kR; ++r) {
+                if (j0 + r * WS_BLOCK >= n) continue;  // uniform
+                bool takes = false;
+                if (li[r] != 0xffffffffu) {
+                    const uint32_t sh = (li[r] & 1u) * 16u;
+                    if (!BIAS) {
+                        takes = ((atomicAdd(&cnt[li[r] >> 1], 1u << sh) >> sh) & (kFewDup - 1u)) == 0u;
+                    } else if ((atomicOr(&cnt[li[r] >> 1], kFewTaken << sh) >> sh) & kFewTaken) {  // another entry has this token: left where that one finds it
+                        atomicOr(&cnt[li[r] >> 1], kFewDup << sh);
+                        const uint32_t at = atomicAdd(&F.w[0], 1u);
+                        if (at < kFewDups) {
+                            F.dup_at[at] = li[r];
+                            F.dup_j[at] = j0 + r * WS_BLOCK + t;
+                            F.dup_v[at] = bv[r];
+                        }
+                    } else {
+                        takes = true;
+                    }
+                }
+                const uint64_t mk = __ballot(takes);
+                if (mk) {  // uniform
+                    uint32_t at0 = 0;
+                    if (lane == 0u) at0 = atomicAdd(&F.w[1], static_cast<uint32_t>(__popcll(mk)));
+                    const uint32_t at = lane_value(at0, 0u) + lanes_before(mk);
+                    if (takes && at < kFewExt)
+                        ext[at] = make_uint4(id[r] | (BIAS ? kExtBias : 0u), al[r] & 1u ? raw[r] : 0xff800000u, __float_as_uint(bv[r]), j0 + r * WS_BLOCK + t);
+                }
+            }
+        };
+        bool first = true;
+        for (uint32_t j0 = 0; j0 < nh; j0 += kR * WS_BLOCK, first = false) four(std::false_type{}, nh, j0, first);
+        for (uint32_t j0 = 0; j0 < nb; j0 += kR * WS_BLOCK, first = false) four(std::true_type{}, nb, j0, first);
+    }
+    __syncthreads();
+    WSS_MARK(1);  // history and bias entries counted
+
+    // ---- the share: tokens that do not count - masked out, NaN, past the row, touched - become -inf
+    float x[NV][TPV];
+    float lm = -INFINITY;
+#pragma unroll
+    for (uint32_t k = 0; k < NV; ++k) {
+        if (k >= n_vec) {  // uniform
+#pragma unroll
+            for (uint32_t e = 0; e < TPV; ++e) x[k][e] = -INFINITY;
+            continue;
+        }
+        const uint32_t j = vec_of(k);
+        uint4 qq = q[k];
+        if (j_part != 0xffffffffu && j == j_part) qq = part_vector<DT>(qq, TPV - V % TPV);
+        const uint32_t w[4] = {qq.x, qq.y, qq.z, qq.w};
+        uint32_t invalid = j < nv ? 0u : ~0u;  // bit e: token e does not count
+        if (MASKED) invalid |= ~(na[k] >> ((j * TPV) & 31u));
+        uint32_t c2[TPV / 2u];
+#pragma unroll
+        for (uint32_t e = 0; e < TPV / 2u; ++e) c2[e] = 0u;
+        if (any_ext) {  // uniform
+            const uint32_t at = (wv * (NV * 64u) + k * 64u + lane) * (TPV / 2u);
+#pragma unroll
+            for (uint32_t e = 0; e < TPV / 2u; e += 2u) {
+                const uint2 two = *reinterpret_cast<const uint2*>(&cnt[at + e]);
+                c2[e] = two.x;
+                c2[e + 1u] = two.y;
+            }
+        }
+#pragma unroll
+        for (uint32_t e = 0; e < TPV; ++e) {
+            const uint32_t bits = DT == 0 ? w[e] : ((e & 1u) ? (w[e >> 1] & 0xffff0000u) : (w[e >> 1] << 16));
+            const uint32_t c = (e & 1u) ? c2[e >> 1] & 0xffff0000u : c2[e >> 1] & 0xffffu;
+            const bool out = ((invalid >> e) & 1u) || c;
+            x[k][e] = out ? -INFINITY : fmaxf(__uint_as_float(bits), -INFINITY);
+            lm = fmaxf(lm, x[k][e]);
+        }
+    }
+    WSS_MARK(2);  // share in registers
+
+    // ---- the touched tokens: bias, repetition, frequency / presence (as ws_sample.h applies them); from here on the list
+    // holds {token, adjusted logit}, and every thread keeps to its own entries
+    const uint32_t n_ext = any_ext ? min(F.w[1], kFewExt) : 0u, n_ext_all = any_ext ? F.w[1] : 0u;
+    for (uint32_t i = t; i < n_ext; i += WS_BLOCK) {
+        const uint4 en = ext[i];
+        const bool bias = (en.x & kExtBias) != 0u;
+        const uint32_t id = en.x & ~kExtBias, li = place_of(id), sh = (li & 1u) * 16u, c = cnt[li >> 1] >> sh;
+        float v = fmaxf(__uint_as_float(en.y), -INFINITY);
+        if (bias) {
+            const uint32_t n_dup = F.w[0];
+            if (!(c & kFewDup)) {
+                v = __fadd_rn(v, __uint_as_float(en.z));
+            } else if (n_dup <= kFewDups) {  // the token's entries in the order of the list: this one and those left behind
+                for (uint32_t from = 0; from <= nb;) {
+                    uint32_t next = en.w >= from ? en.w : 0xfffffffeu;
+                    float val = __uint_as_float(en.z);
+                    for (uint32_t k = 0; k < n_dup; ++k)
+                        if (F.dup_at[k] == li && F.dup_j[k] >= from && F.dup_j[k] < next) {
+                            next = F.dup_j[k];
+                            val = F.dup_v[k];
+                        }
+                    if (next == 0xfffffffeu) break;
+                    v = __fadd_rn(v, val);
+                    from = next + 1u;
+                }
+            } else {
+                for (uint32_t j = 0; j < nb; ++j)
+                    if (static_cast<uint32_t>(A.bias_ids[P.b0 + j]) == id) v = __fadd_rn(v, A.bias_vals[P.b0 + j]);
+            }
+        } else if (c & kFewTaken) {
+            v = -INFINITY;  // (the bias entry has this token)
+        }
+        if ((c & (kFewDup - 1u)) && v > -INFINITY) {
+            v = v > 0.f ? __fdiv_rn(v, P.rep) : __fmul_rn(v, P.rep);
+            v = __fsub_rn(v, __fadd_rn(__fmul_rn(P.freq, static_cast<float>(c & (kFewDup - 1u))), P.pres));
+        }
+        v = fmaxf(v, -INFINITY);
+        *reinterpret_cast<uint2*>(&ext[i]) = make_uint2(id, __float_as_uint(v));
+        lm = fmaxf(lm, v);
+    }
+    const float wm = wave_max(lm);
+    WSS_MARK(11);  // touched tokens in
+
+    unsigned char* work = A.work + static_cast<size_t>(row) * kFewRowBytes;
+    unsigned long long* gkeys = reinterpret_cast<unsigned long long*>(work);
+    unsigned long long* ghead = reinterpret_cast<unsigned long long*>(work + kFewHead);
+    uint32_t* ctrl = reinterpret_cast<uint32_t*>(work + kFewCtrl);
+
+    // ---- the threshold
+    float thr = -INFINITY;  // this wave lists its tokens from here up
+    if (by_k) {
+        // A wave has top_k / G of the row's top_k largest on average; four more and five times the scatter of that number
+        // are listed, d of them in different lanes.
+        const float lambda = static_cast<float>(top_k) / static_cast<float>(G);
+        const uint32_t want = static_cast<uint32_t>(lambda + 5.f * __builtin_sqrtf(lambda) + 4.f) + 1u;
+        const uint32_t d = min(60u, want <= 20u ? want : 20u + (want - 20u) / 2u);
+        const uint32_t at = few_lane_threshold(key32(lm), d);
+        thr = at > 0x007fffffu ? unkey32(at) : -INFINITY;  // (below that prefix: -inf and the NaN patterns under it)
+    } else if (by_p) {
+        // what the floor lets through lies within -ln(min_p) / inv_t of the row's maximum: of the largest logit any part
+        // has reported so far, or this part's (0.02 units of the exponent below: roundings)
+        if (lane == 0u) F.red_f[wv] = wm;
+        __syncthreads();
+        float top = F.red_f[0];
+#pragma unroll
+        for (uint32_t w = 1; w < WS_WAVES; ++w) top = fmaxf(top, F.red_f[w]);
+        if (t == 0) {
+            __hip_atomic_fetch_max(&ctrl[1], key32(top), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            F.w[8] = __hip_atomic_load(&ctrl[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        __syncthreads();
+        top = fmaxf(top, unkey32(F.w[8]));
+        if (top > -INFINITY) thr = __fadd_rn(top, __fdiv_rn(static_cast<float>(log(min_p)) - 0.02f, inv_t));
+    }
+
+    WSS_MARK(3);  // threshold
+    // ---- the sum of exp against the wave's maximum, and the list
+    const float k2 = inv_t * 1.44269504088896340736f;
+    const float k2lo = static_cast<float>(static_cast<double>(inv_t) * 1.44269504088896340736 - static_cast<double>(k2));
+    const float ref = wm > -INFINITY ? wm : 0.f;
+    float s = 0.f;
+    auto add = [&](float v) {
+        const float a = fmaxf(__fsub_rn(v, ref), -1e30f);
+        s += __builtin_amdgcn_exp2f(fmaf(a, k2lo, a * k2));
+    };
+    uint32_t n_list = 0;  // uniform
+    const float thr_list = fmaxf(thr, -3.402823466e38f);  // (-inf is no token)
+    auto push = [&](float v, uint32_t id) {
+        const bool yes = v >= thr_list;
+        const uint64_t m = __ballot(yes);
+        if (m) {  // uniform
+            const uint32_t slot = n_list + lanes_before(m);
+            if (yes && slot < slots) __hip_atomic_store(&gkeys[slot * G + g], key64(v, id), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            n_list += static_cast<uint32_t>(__popcll(m));
+        }
+    };
+    if (!not_mine && wm < INFINITY) {
+#pragma unroll
+        for (uint32_t k = 0; k < NV; ++k)
+#pragma unroll
+            for (uint32_t e = 0; e < TPV; ++e)
+                if (k < n_vec) push(x[k][e], vec_of(k) * TPV + e);
+        for (uint32_t i0 = 0; i0 < n_ext; i0 += WS_BLOCK) {  // uniform
+            uint2 en = make_uint2(0u, 0xff800000u);
+            if (i0 + t < n_ext) en = *reinterpret_cast<const uint2*>(&ext[i0 + t]);
+            push(__uint_as_float(en.y), en.x);
+            add(__uint_as_float(en.y));
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < NV; ++k)
+#pragma unroll
+            for (uint32_t e = 0; e < TPV; ++e)
+                if (k < n_vec) add(x[k][e]);
+    }
+    {
+        const double z = wm > -INFINITY && wm < INFINITY ? wave_sum(static_cast<double>(s)) : 0.0;
+        const uint32_t n = not_mine || !(wm < INFINITY) || n_list > slots || n_ext_all > kFewExt ? kFewBad : n_list + 1u;
+        if (lane == 0u) {
+            const uint64_t zw = static_cast<uint64_t>(__double_as_longlong(z));
+            __hip_atomic_store(&ghead[g], (static_cast<unsigned long long>(key32(wm)) << 32) | key32(thr), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(&ghead[kFewWaves + g], (zw & ~uint64_t{kFewBad}) | n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
+    // (The ticket orders nothing by itself and need not: every word the parts exchange is written and read by device-scope
+    // atomic accesses, which go past this unit's caches, and a word still on its way reads as zero and is read again.)
+    WSS_MARK(4);  // listed, summed
+    __syncthreads();  // every wave's stores have been issued
+    WSS_MARK(5);
+    if (t == 0) F.w[2] = __hip_atomic_fetch_add(&ctrl[0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    if (F.w[2] != A.few_parts - 1u) return true;  // not the last: done
+    finisher = true;
+    WSS_MARK(6);  // ticket
+    // ---- the last part: everybody's keys asked for (those of the first slots right away), then the headers. Four waves read
+    // them side by side, each for what it works out: the threshold, the normaliser, how many keys there are, the uniform.
+    constexpr uint32_t kTries = 64u, kBlind = 4096u / WS_BLOCK, kHL = kFewWaves / 64u;
+    uint64_t got[kBlind];
+#pragma unroll
+    for (uint32_t i = 0; i < kBlind; ++i) got[i] = __hip_atomic_load(&gkeys[i * WS_BLOCK + t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (t < 2u) F.w[5u + t] = 0u;  // keys taken, keys seen
+    if (wv == 3u) {
+        // (the seed by way of a vector register: as scalar arithmetic the generator's rounds are moved out of this branch)
+        uint32_t seed_lo = static_cast<uint32_t>(P.seed);
+        asm volatile("" : "+v"(seed_lo));
+        const double u_ = batch_uniform(A.rng, (P.seed & 0xffffffff00000000ull) | seed_lo, row, P.step, 0);
+        if (lane == 0u) F.u = u_;
+    } else if (wv < 3u) {
+        uint64_t h0[kHL], h1[kHL];
+        bool late = false;
+        for (uint32_t tries = 0; tries < kTries; ++tries) {
+            bool zero = false;
+#pragma unroll
+            for (uint32_t i = 0; i < kHL; ++i) {
+                const uint32_t w = min(i * 64u + lane, G - 1u);
+                h0[i] = __hip_atomic_load(&ghead[w], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                h1[i] = __hip_atomic_load(&ghead[kFewWaves + w], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+#pragma unroll
+            for (uint32_t i = 0; i < kHL; ++i) zero = zero || h0[i] == 0ull || h1[i] == 0ull;
+            late = __ballot(zero) != 0ull;
+            if (!late) break;
+        }
+        float m4[kHL], mx = -INFINITY;
+#pragma unroll
+        for (uint32_t i = 0; i < kHL; ++i) {
+            m4[i] = i * 64u + lane < G ? unkey32(static_cast<uint32_t>(h0[i] >> 32)) : -INFINITY;
+            mx = fmaxf(mx, m4[i]);
+        }
+        mx = wave_max(mx);
+        if (wv == 0u) {
+            float tx = -INFINITY;
+#pragma unroll
+            for (uint32_t i = 0; i < kHL; ++i) tx = fmaxf(tx, unkey32(static_cast<uint32_t>(h0[i])));
+            tx = wave_max(tx);
+            // the keys that are looked at: from the largest of the waves' thresholds up (every wave has listed what it has
+            // there), or - higher - from the top_k-th largest of the waves' maxima
+            float floor_v = tx;
+            if (by_k && top_k <= G) {
+                float lo = tx, hi = mx;
+                auto reach = [&](float v) {
+                    uint32_t n = 0;
+#pragma unroll
+                    for (uint32_t i = 0; i < kHL; ++i) n += static_cast<uint32_t>(__popcll(__ballot(m4[i] >= v)));
+                    return n;
+                };
+                if (lo > -INFINITY && reach(lo) >= top_k)
+                    for (int i = 0; i < 5; ++i) {  // two halvings a step
+                        const float m2 = 0.5f * lo + 0.5f * hi, m1 = 0.5f * lo + 0.5f * m2, m3 = 0.5f * m2 + 0.5f * hi;
+                        const uint32_t n1 = reach(m1), n2 = reach(m2), n3 = reach(m3);
+                        hi = n1 < top_k ? m1 : (n2 < top_k ? m2 : (n3 < top_k ? m3 : hi));
+                        lo = n3 >= top_k ? m3 : (n2 >= top_k ? m2 : (n1 >= top_k ? m1 : lo));
+                    }
+                floor_v = lo;
+            }
+            if (by_p) floor_v = __fadd_rn(mx, __fdiv_rn(static_cast<float>(log(min_p)) - 0.02f, inv_t));
+            if (lane == 0u) {
+                F.red_f[0] = mx;
+                F.red_f[1] = floor_v;
+            }
+        } else if (wv == 1u) {
+            double z = 0.0;
+#pragma unroll
+            for (uint32_t i = 0; i < kHL; ++i)
+                if (m4[i] > -INFINITY) {
+                    const float a = fmaxf(__fsub_rn(m4[i], mx), -1e30f);
+                    z += __longlong_as_double(static_cast<long long>(h1[i] & ~uint64_t{kFewBad})) * static_cast<double>(__builtin_amdgcn_exp2f(fmaf(a, k2lo, a * k2)));
+                }
+            z = wave_sum(z);
+            if (lane == 0u) S.s_d[0] = z;
+        } else {
+            uint32_t most = 0, all = 0;
+            bool bad = late || !(mx > -INFINITY);
+#pragma unroll
+            for (uint32_t i = 0; i < kHL; ++i)
+                if (i * 64u + lane < G) {
+                    const uint32_t n = static_cast<uint32_t>(h1[i]) & kFewBad;
+                    bad = bad || n == kFewBad || n == 0u;
+                    most = max(most, n - 1u);
+                    all += n - 1u;
+                }
+            most = wave_max_u32(most);
+            all = wave_sum(all);
+            bad = __ballot(bad) != 0ull;
+            if (lane == 0u) {
+                F.w[3] = bad ? slots : most;  // (a wave that could not list its share may have left keys in every slot)
+                F.w[4] = bad ? 1u : 0u;
+                F.w[7] = all;
+            }
+        }
+    }
+    __syncthreads();
+    WSS_MARK(7);  // headers
+    const float m = F.red_f[0];
+    const uint32_t floor_key = key32(F.red_f[1]);
+    const double z = S.s_d[0];
+    const uint32_t n_read = F.w[3] * G;
+    bool bad = F.w[4] != 0u;
+    uint64_t* list = reinterpret_cast<uint64_t*>(lds);
+    uint32_t seen = 0;  // uniform
+    auto keep = [&](uint64_t key, uint32_t at) {
+        if (key != 0ull) __hip_atomic_store(&gkeys[at], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // the workspace as the next launch needs it
+        seen += static_cast<uint32_t>(__popcll(__ballot(key != 0ull)));
+        const bool yes = static_cast<uint32_t>(key >> 32) >= floor_key && key != 0ull;
+        const uint64_t mk = __ballot(yes);
+        if (mk) {  // uniform
+            uint32_t at0 = 0;
+            if (lane == 0u) at0 = atomicAdd(&F.w[5], static_cast<uint32_t>(__popcll(mk)));
+            const uint32_t slot = lane_value(at0, 0u) + lanes_before(mk);
+            if (yes && slot < kShortCap) list[slot] = key;
+        }
+    };
+#pragma unroll
+    for (uint32_t i = 0; i < kBlind; ++i)
+        if (i * WS_BLOCK < n_read) keep(got[i], i * WS_BLOCK + t);  // uniform
+    for (uint32_t i0 = kBlind * WS_BLOCK; i0 < n_read; i0 += WS_BLOCK) {
+        const uint32_t at = i0 + t;
+        keep(at < n_read ? __hip_atomic_load(&gkeys[at], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0ull, at);
+    }
+    if (lane == 0u && seen) atomicAdd(&F.w[6], seen);
+    if (t < G) {
+        __hip_atomic_store(&ghead[t], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(&ghead[kFewWaves + t], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if (t < 2u) __hip_atomic_store(&ctrl[t], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    // (a key still on its way was read as zero: looked for again, place by place, until all have come)
+    for (uint32_t tries = 0; !bad && F.w[6] != F.w[7]; ++tries) {  // uniform, rare
+        if (tries == kTries) bad = true;
+        __syncthreads();
+        seen = 0;
+        for (uint32_t i0 = 0; i0 < n_read; i0 += WS_BLOCK)
+            keep(i0 + t < n_read ? __hip_atomic_load(&gkeys[i0 + t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0ull, i0 + t);
+        if (lane == 0u && seen) atomicAdd(&F.w[6], seen);
+        __syncthreads();
+    }
+    const uint32_t n_keys = F.w[5];
+    const uint32_t n_cand = by_k ? top_k : n_keys;
+    if (bad || n_keys < n_cand || n_cand == 0u || n_keys > kShortCap) return false;
+
+    WSS_MARK(8);  // keys
+    // ---- the candidates in order
+    if (n_keys <= 64u) {
+        // WS_BLOCK / 64 threads a key, each counting the larger keys among its share of the 64 places: one barrier
+        constexpr uint32_t kPer = WS_BLOCK / 64u, kEach = 64u / kPer;
+        static_assert(kPer == 8u, "the sum below is over eight lanes");
+        uint64_t* sorted = list + 4096;
+        const uint32_t ki = t / kPer, q0 = (t % kPer) * kEach;
+        const uint64_t own = ki < n_keys ? list[ki] : 0ull;
+        uint32_t above = 0;
+        if (wv * (64u / kPer) < n_keys) {  // (per wave)
+#pragma unroll
+            for (uint32_t i = 0; i < kEach; i += 2u) {
+                const ulonglong2 o = *reinterpret_cast<const ulonglong2*>(&list[q0 + i]);
+                above += (q0 + i < n_keys && o.x > own ? 1u : 0u) + (q0 + i + 1u < n_keys && o.y > own ? 1u : 0u);
+            }
+            above += dpp_or_zero<0x111, 0xf>(above);
+            above += dpp_or_zero<0x112, 0xf>(above);
+            above += dpp_or_zero<0x114, 0xf>(above);  // lanes 7 and 15 of a row of sixteen have the sums of their eight
+            if (ki < n_keys && t % kPer == kPer - 1u) sorted[above] = own;
+        }
+        __syncthreads();
+        list = sorted;
+    } else {
+        short_sort(list, n_keys, m, inv_t * 64.f, S);
+    }
+    WSS_MARK(9);  // sorted
+    ShortRow R;
+    R.top_p = P.top_p;
+    R.min_p = min_p;
+    R.u = F.u;
+    R.z = z;
+    R.inv_t = inv_t;
+    R.m = m;
+    R.n_cand = n_cand;
+    R.by_k = by_k;
+    short_rules(list, row, R, S);
+#ifdef WS_SHORT_TIMERS
+    WSS_MARK(10);
+    __syncthreads();
+    if (t < 16 && A.kept_logits) A.kept_logits[static_cast<size_t>(row) * A.kept_cap + 100u + t] = t == 15 ? static_cast<float>(n_keys) : (t == 14 ? static_cast<float>(n_read) : S.marks[t]);
+#endif
+    return true;
+}
+
+template <int DT, bool MASKED, int NV>
+__global__ void __launch_bounds__(WS_BLOCK) few_batch_kernel(BatchArgs A) {
+    __shared__ FewShared shared;
+    const uint32_t row = blockIdx.y, part = blockIdx.x;
+    bool finisher;
+    if (!few_row<DT, MASKED, NV>(A, row, part, shared, finisher) && finisher) {
+        __syncthreads();
+        LeanArgPtr Ap = (LeanArgPtr)__builtin_amdgcn_kernarg_segment_ptr();
+        asm volatile("" : "+s"(Ap));
+        if (Ap->kept_ids) three_pass_row<true>(Ap, row);
+        else three_pass_row<false>(Ap, row);
+    }
+}
+
+}  // namespace ws

@@ -12,7 +12,8 @@ namespace ws {
 
 // `done`: one bit per device (setting the attribute twice does no harm, so two threads that both find the bit clear may
 // both go on). Returns 0 or the hipError_t.
-inline int raise_lds_limit(std::atomic<uint64_t>& done, std::initializer_list<const void*> kernels, unsigned lds_limit) {
+template <class Kernels>  // a range of kernel addresses
+inline int raise_lds_limit_of(std::atomic<uint64_t>& done, const Kernels& kernels, unsigned lds_limit) {
     int dev = 0;
     if (const hipError_t e = hipGetDevice(&dev); e != hipSuccess) return static_cast<int>(e);
     const uint64_t bit = 1ull << (dev & 63);
@@ -23,6 +24,9 @@ inline int raise_lds_limit(std::atomic<uint64_t>& done, std::initializer_list<co
     }
     done.fetch_or(bit, std::memory_order_release);
     return 0;
+}
+inline int raise_lds_limit(std::atomic<uint64_t>& done, std::initializer_list<const void*> kernels, unsigned lds_limit) {
+    return raise_lds_limit_of(done, kernels, lds_limit);
 }
 
 }  // namespace ws

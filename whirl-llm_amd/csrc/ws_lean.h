@@ -239,6 +239,59 @@ struct LeanRowParams {
     bool race;
 };
 
+// Every one of a row's parameters with one scalar load, all asked for together and waited for once. (Written as plain reads
+// they become vector loads, each behind the test of its pointer and each waited for on its own: a dozen trips to memory one
+// after the other.) An absent array is read at the kernel's argument segment instead and the value dropped.
+__device__ __forceinline__ LeanRowParams load_row_params(const BatchArgs& A, const uint32_t row) {
+    LeanRowParams P;
+    const uint64_t dummy = reinterpret_cast<uint64_t>((const __attribute__((address_space(4))) void*)__builtin_amdgcn_kernarg_segment_ptr());
+    auto at = [&](const void* base, uint64_t byte_off) { return base ? reinterpret_cast<uint64_t>(base) + byte_off : dummy; };
+    const uint64_t r4 = static_cast<uint64_t>(row) * 4u, r8 = static_cast<uint64_t>(row) * 8u;
+    const uint64_t p_inv_t = at(A.inv_t, r4), p_top_k = at(A.top_k, r4), p_race = at(A.race, r4), p_top_p = at(A.top_p, r8), p_min_p = at(A.min_p, r8);
+    // (the history's length: its own array, or else the next row's offset - which an offsets array with lengths beside it need not have)
+    const uint64_t p_hoff = at(A.hist ? A.hist_off : nullptr, r4);
+    const uint64_t p_hlen = A.hist ? (A.hist_len ? at(A.hist_len, r4) : at(A.hist_off, r4 + 4u)) : dummy;
+    const uint64_t p_boff = at(A.bias_ids ? A.bias_off : nullptr, r4), p_seed = at(A.seed, r8), p_step = at(A.step, r8);
+    const uint64_t p_rep = at(A.rep, r4), p_pres = at(A.pres, r4), p_freq = at(A.freq, r4);
+    uint32_t v_inv_t, v_top_k, v_race, v_hoff, v_hlen, v_rep, v_pres, v_freq;
+    uint64_t v_top_p, v_min_p, v_boff, v_seed, v_step;
+    asm volatile(
+        "s_load_dword %0, %13, 0x0\n\t"
+        "s_load_dword %1, %14, 0x0\n\t"
+        "s_load_dword %2, %15, 0x0\n\t"
+        "s_load_dwordx2 %3, %16, 0x0\n\t"
+        "s_load_dwordx2 %4, %17, 0x0\n\t"
+        "s_load_dword %5, %18, 0x0\n\t"
+        "s_load_dword %6, %19, 0x0\n\t"
+        "s_load_dwordx2 %7, %20, 0x0\n\t"
+        "s_load_dwordx2 %8, %21, 0x0\n\t"
+        "s_load_dwordx2 %9, %22, 0x0\n\t"
+        "s_load_dword %10, %23, 0x0\n\t"
+        "s_load_dword %11, %24, 0x0\n\t"
+        "s_load_dword %12, %25, 0x0\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&s"(v_inv_t), "=&s"(v_top_k), "=&s"(v_race), "=&s"(v_top_p), "=&s"(v_min_p), "=&s"(v_hoff), "=&s"(v_hlen), "=&s"(v_boff),
+          "=&s"(v_seed), "=&s"(v_step), "=&s"(v_rep), "=&s"(v_pres), "=&s"(v_freq)
+        : "s"(p_inv_t), "s"(p_top_k), "s"(p_race), "s"(p_top_p), "s"(p_min_p), "s"(p_hoff), "s"(p_hlen), "s"(p_boff), "s"(p_seed),
+          "s"(p_step), "s"(p_rep), "s"(p_pres), "s"(p_freq)
+        : "memory");
+    P.inv_t = __uint_as_float(v_inv_t);
+    P.top_k = A.top_k ? v_top_k : 0u;
+    P.race = A.race != nullptr && v_race != 0u;
+    P.top_p = A.top_p ? __longlong_as_double(static_cast<long long>(v_top_p)) : 1.0;
+    P.min_p = A.min_p ? __longlong_as_double(static_cast<long long>(v_min_p)) : 0.0;
+    P.h0 = A.hist ? v_hoff : 0u;
+    P.nh = A.hist ? (A.hist_len ? v_hlen : v_hlen - P.h0) : 0u;
+    P.b0 = A.bias_ids ? static_cast<uint32_t>(v_boff) : 0u;
+    P.nb = A.bias_ids ? static_cast<uint32_t>(v_boff >> 32) - P.b0 : 0u;
+    P.seed = v_seed;
+    P.step = v_step;
+    P.rep = A.rep ? __uint_as_float(v_rep) : 1.f;
+    P.pres = A.pres ? __uint_as_float(v_pres) : 0.f;
+    P.freq = A.freq ? __uint_as_float(v_freq) : 0.f;
+    return P;
+}
+
 // what wave 0 works out from the searches' answers for everybody
 struct LeanSel {
     double X, m0base, m1base;
@@ -361,58 +414,7 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const uint32_t row,
         }
     }
 
-    // The row's parameters, every one of them with one scalar load, all asked for together and waited for once. (Written
-    // as plain reads they become vector loads, each behind the test of its pointer and each waited for on its own: a
-    // dozen trips to memory one after the other, here and again behind the sweep.) An absent array is read at the
-    // kernel's argument segment instead and the value dropped.
-    LeanRowParams P;
-    {
-        const uint64_t dummy = reinterpret_cast<uint64_t>((const __attribute__((address_space(4))) void*)__builtin_amdgcn_kernarg_segment_ptr());
-        auto at = [&](const void* base, uint64_t byte_off) { return base ? reinterpret_cast<uint64_t>(base) + byte_off : dummy; };
-        const uint64_t r4 = static_cast<uint64_t>(row) * 4u, r8 = static_cast<uint64_t>(row) * 8u;
-        const uint64_t p_inv_t = at(A.inv_t, r4), p_top_k = at(A.top_k, r4), p_race = at(A.race, r4), p_top_p = at(A.top_p, r8), p_min_p = at(A.min_p, r8);
-        // (the history's length: its own array, or else the next row's offset - which an offsets array with lengths beside it need not have)
-        const uint64_t p_hoff = at(A.hist ? A.hist_off : nullptr, r4);
-        const uint64_t p_hlen = A.hist ? (A.hist_len ? at(A.hist_len, r4) : at(A.hist_off, r4 + 4u)) : dummy;
-        const uint64_t p_boff = at(A.bias_ids ? A.bias_off : nullptr, r4), p_seed = at(A.seed, r8), p_step = at(A.step, r8);
-        const uint64_t p_rep = at(A.rep, r4), p_pres = at(A.pres, r4), p_freq = at(A.freq, r4);
-        uint32_t v_inv_t, v_top_k, v_race, v_hoff, v_hlen, v_rep, v_pres, v_freq;
-        uint64_t v_top_p, v_min_p, v_boff, v_seed, v_step;
-        asm volatile(
-            "s_load_dword %0, %13, 0x0\n\t"
-            "s_load_dword %1, %14, 0x0\n\t"
-            "s_load_dword %2, %15, 0x0\n\t"
-            "s_load_dwordx2 %3, %16, 0x0\n\t"
-            "s_load_dwordx2 %4, %17, 0x0\n\t"
-            "s_load_dword %5, %18, 0x0\n\t"
-            "s_load_dword %6, %19, 0x0\n\t"
-            "s_load_dwordx2 %7, %20, 0x0\n\t"
-            "s_load_dwordx2 %8, %21, 0x0\n\t"
-            "s_load_dwordx2 %9, %22, 0x0\n\t"
-            "s_load_dword %10, %23, 0x0\n\t"
-            "s_load_dword %11, %24, 0x0\n\t"
-            "s_load_dword %12, %25, 0x0\n\t"
-            "s_waitcnt lgkmcnt(0)"
-            : "=&s"(v_inv_t), "=&s"(v_top_k), "=&s"(v_race), "=&s"(v_top_p), "=&s"(v_min_p), "=&s"(v_hoff), "=&s"(v_hlen), "=&s"(v_boff),
-              "=&s"(v_seed), "=&s"(v_step), "=&s"(v_rep), "=&s"(v_pres), "=&s"(v_freq)
-            : "s"(p_inv_t), "s"(p_top_k), "s"(p_race), "s"(p_top_p), "s"(p_min_p), "s"(p_hoff), "s"(p_hlen), "s"(p_boff), "s"(p_seed),
-              "s"(p_step), "s"(p_rep), "s"(p_pres), "s"(p_freq)
-            : "memory");
-        P.inv_t = __uint_as_float(v_inv_t);
-        P.top_k = A.top_k ? v_top_k : 0u;
-        P.race = A.race != nullptr && v_race != 0u;
-        P.top_p = A.top_p ? __longlong_as_double(static_cast<long long>(v_top_p)) : 1.0;
-        P.min_p = A.min_p ? __longlong_as_double(static_cast<long long>(v_min_p)) : 0.0;
-        P.h0 = A.hist ? v_hoff : 0u;
-        P.nh = A.hist ? (A.hist_len ? v_hlen : v_hlen - P.h0) : 0u;
-        P.b0 = A.bias_ids ? static_cast<uint32_t>(v_boff) : 0u;
-        P.nb = A.bias_ids ? static_cast<uint32_t>(v_boff >> 32) - P.b0 : 0u;
-        P.seed = v_seed;
-        P.step = v_step;
-        P.rep = A.rep ? __uint_as_float(v_rep) : 1.f;
-        P.pres = A.pres ? __uint_as_float(v_pres) : 0.f;
-        P.freq = A.freq ? __uint_as_float(v_freq) : 0.f;
-    }
+    const LeanRowParams P = load_row_params(A, row);
     const float inv_t = P.inv_t;
     const uint32_t top_k = P.top_k;
     const bool race = P.race;

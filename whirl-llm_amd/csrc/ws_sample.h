@@ -101,6 +101,7 @@ struct BatchArgs {
     uint32_t stage_cap;        // entries of a row's staging area (kSplitStageCap), 0: none
     uint32_t fb_lds_tie;       // the lean and the short-list kernel: lds_tie and lds_ab of the three-pass code they hand rows back to
     uint32_t fb_lds_ab;
+    uint32_t few_parts, few_magic, few_chunk_log2;  // ws_few.h: parts a row, 2^32 / waves a row rounded up, log2 of the lanes a chunk
 };
 
 // Global memory of a split row: the merged histogram, the merged candidate list, and four control words (parts that
@@ -111,12 +112,10 @@ constexpr uint32_t kSplitHist = 0u, kSplitList = 32768u, kSplitCtrl = 65536u, kS
 // slices there, in id order, and the part that finishes the row picks the kept tokens out - no workgroup reads the whole
 // row again. Control words 4 (entries staged), 8 + part (where the part's entries start) and 24 + part (how many).
 constexpr uint32_t kSplitStage = kSplitRowBytes, kSplitStageCap = 8192u, kSplitRowBytesKept = kSplitStage + kSplitStageCap * 8u;
-// The short-list kernel (ws_short.h). Global memory of a row shared by several workgroups (zero-filled once, left
-// zero-filled): kShortCap keys - the tokens a row lists, a stretch of kShortCap / parts for each part -, then 64 + 8 * 16
-// words: [0] parts arrived; from word 64 on, eight words a part: maximum (as an order key), threshold (order key), the
-// part's sum as a double against its maximum, and how many keys it listed (all bits set: it could not list its slice).
+// The short-list kernels (ws_short.h, ws_few.h): keys a row may list, tokens a workgroup of ws_few.h holds, history and bias
+// entries its rows may have, workgroups a row at most, and the workspace of a row (its layout: ws_few.h)
 constexpr uint32_t kShortCap = 4096u;
-constexpr uint32_t kShortSplitCtrl = kShortCap * 8u, kShortSplitRowBytes = kShortSplitCtrl + 4u * (64u + 8u * 16u);
+constexpr uint32_t kFewShare = 40960u, kFewLists = 10240u, kFewMaxParts = 16u, kFewRowBytes = 65536u;
 // Workspace of one row of the three-pass kernel: per history / bias entry a word of each of phase 0's two rank
 // tables, which sit out the first sweep there. Whole memory lines, so that rows share none.
 __host__ __device__ constexpr uint64_t capture_row_bytes(uint32_t patch_cap) {
