@@ -105,3 +105,23 @@ def test_query_and_entropy():
         h_want = float(-(pk * np.log(pk)).sum())
         assert abs(ent[r] - h_want) <= 1e-6 * max(1.0, h_want), (r, ent[r], h_want)
     assert not (smp.flags.cpu().numpy() & m.FLAG_APPROX_ENTROPY).any()
+
+
+@pytest.mark.parametrize("rows,n,K", [(2, 32768, 512), (100, 81920, 40), (5, 163844, 300), (1, 655360, 64), (16, 100000, 17)])
+def test_top_lists_at_the_edges_of_a_share(rows, n, K):
+    """ws_topk_rows_ws and ws_dflash_topk_ws (ws_top.h) with the smallest and the largest shares: ids, values and maxima equal to
+    those of the kernels that give a row to one workgroup, twice on one workspace, which is zero again afterwards."""
+    m = gc.pkg()
+    rng = np.random.default_rng(n)
+    x = torch.from_numpy((rng.standard_normal((rows, n)) * 2).astype(np.float32)).cuda()
+    work = m.topk_rows_workspace(n, K, rows)
+    want = m.topk_rows(x, K, 1.25)
+    k = min(K, 64)
+    first = m.dflash_topk(x, k)
+    for _ in range(2):
+        got = m.topk_rows(x, K, 1.25, workspace=work)
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1]) and torch.equal(got[2][:, 0], want[2][:, 0])
+        assert torch.allclose(got[2][:, 1], want[2][:, 1], rtol=2e-6, atol=0)  # (float sums in another order: the bar of ws_topk_rows_ws)
+        again = m.dflash_topk(x, k, workspace=work)
+        assert torch.equal(again[0], first[0]) and torch.equal(again[1], first[1])
+    assert not work.any().item()

@@ -8,7 +8,9 @@ The directory name holds a hyphen, so import it through `load_package()` of the 
 `importlib` (module name `whirl_llm_amd`).
 """
 import ctypes as C
+import operator
 import os
+import struct
 
 import torch
 
@@ -175,17 +177,38 @@ def check(code, what):
 
 
 def _stream():
-    return C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    """The current stream's handle, as an integer (what ctypes makes a void* of): without the torch.cuda.Stream object in between, a
+    third of the host time of a small launch."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _p(t):
-    return C.c_void_p(t.data_ptr()) if t is not None else None
+    return t.data_ptr() if t is not None else None
 
 
 def _dev_f32(x):
     if not (x.is_cuda and x.dtype == torch.float32 and x.is_contiguous()):
         raise WsError("expected a contiguous float32 device tensor")
     return x
+
+
+_DSAMP_FIELDS = operator.itemgetter("top_k", "qoff", "inv_t", "top_p", "min_p", "key")
+_dsamp_structs = {}
+
+
+def _dsamp_struct(n):
+    """The first n entries of every array of a DSampArgs, as one struct format."""
+    st = _dsamp_structs.get(n)
+    if st is None:
+        gap = f"{4 * (32 - n)}x"
+        st = _dsamp_structs[n] = struct.Struct("=" + f"{n}i{gap}" * 3 + f"{n}f{gap}" * 3 + f"{n}I{gap}" * 2)
+    return st
+
+
+def _row_idx(values):
+    ri = RowIdx()
+    ri.v[:len(values)] = values
+    return ri
 
 
 def argmax_rows(x):
@@ -206,9 +229,7 @@ def argmax(x, ids, pos, advance=1):
 
 def argmax_rows_to(x, out, dst):
     _dev_f32(x)
-    ri = RowIdx()
-    for i, d in enumerate(dst):
-        ri.v[i] = d
+    ri = _row_idx(dst)
     check(lib().ws_argmax_rows_to(_stream(), _p(x), x.shape[1], _p(out), C.byref(ri), x.shape[0]), "ws_argmax_rows_to")
     return out
 
@@ -238,9 +259,7 @@ def draft_pick(x, tok, prob, ctl, r, n_min, p_min, vmap=None, workspace=None):
 
 def draft_pick_rows(x, ctl_all, area, r, n_min, p_min, vmap=None, workspace=None):
     _dev_f32(x)
-    ri = RowIdx()
-    for i, d in enumerate(area):
-        ri.v[i] = d
+    ri = _row_idx(area)
     if workspace is not None:
         check(lib().ws_draft_pick_rows_ws(_stream(), _p(x), x.shape[1], _p(ctl_all), C.byref(ri), r, n_min, p_min, _p(vmap),
                                           x.shape[0], _p(workspace), workspace.numel()), "ws_draft_pick_rows_ws")
@@ -252,13 +271,11 @@ def draft_pick_rows(x, ctl_all, area, r, n_min, p_min, vmap=None, workspace=None
 def draft_sample_rows(x, ctl_all, area, r, args, qbuf, vmap=None, workspace=None):
     """args: list of per-row dicts (on, top_k, qoff, inv_t, top_p, min_p, key). workspace: as for topk_rows (K = 32)."""
     _dev_f32(x)
-    ri, da = RowIdx(), DSampArgs()
-    for i, d in enumerate(area):
-        ri.v[i] = d
-    for i, a in enumerate(args):
-        da.on[i], da.top_k[i], da.qoff[i] = a.get("on", 1), a["top_k"], a["qoff"]
-        da.inv_t[i], da.top_p[i], da.min_p[i] = a["inv_t"], a["top_p"], a["min_p"]
-        da.key_lo[i], da.key_hi[i] = a["key"] & 0xFFFFFFFF, a["key"] >> 32
+    ri, da = _row_idx(area), DSampArgs()
+    if args:
+        top_k, qoff, inv_t, top_p, min_p, key = zip(*map(_DSAMP_FIELDS, args))
+        _dsamp_struct(len(args)).pack_into(da, 0, *[a.get("on", 1) for a in args], *top_k, *qoff, *inv_t, *top_p, *min_p,
+                                           *[k & 0xFFFFFFFF for k in key], *[k >> 32 for k in key])
     if workspace is not None:
         check(lib().ws_draft_sample_rows_ws(_stream(), _p(x), x.shape[1], _p(ctl_all), C.byref(ri), r, _p(vmap), C.byref(da),
                                             _p(qbuf), x.shape[0], _p(workspace), workspace.numel()), "ws_draft_sample_rows_ws")
@@ -272,15 +289,19 @@ def topk_rows(x, K, inv_t, workspace=None):
     workspace: a zero-filled uint8 device tensor of ws_topk_rows_workspace bytes kept between calls - small batches then
     share each row between several workgroups (ws_topk_rows_ws)."""
     _dev_f32(x)
-    rows = x.shape[0]
-    ids = torch.full((rows, K), -1, dtype=torch.int32, device=x.device)
-    vals = torch.zeros((rows, K), dtype=torch.float32, device=x.device)
+    rows, n = x.shape
+    if K <= n:  # (every entry is written)
+        ids = torch.empty((rows, K), dtype=torch.int32, device=x.device)
+        vals = torch.empty((rows, K), dtype=torch.float32, device=x.device)
+    else:
+        ids = torch.full((rows, K), -1, dtype=torch.int32, device=x.device)
+        vals = torch.zeros((rows, K), dtype=torch.float32, device=x.device)
     stats = torch.empty((rows, 2), dtype=torch.float32, device=x.device)
     if workspace is not None:
-        check(lib().ws_topk_rows_ws(_stream(), _p(x), x.shape[1], K, inv_t, _p(ids), _p(vals), _p(stats), rows, _p(workspace),
+        check(lib().ws_topk_rows_ws(_stream(), _p(x), n, K, inv_t, _p(ids), _p(vals), _p(stats), rows, _p(workspace),
                                     workspace.numel()), "ws_topk_rows_ws")
     else:
-        check(lib().ws_topk_rows(_stream(), _p(x), x.shape[1], K, inv_t, _p(ids), _p(vals), _p(stats), rows), "ws_topk_rows")
+        check(lib().ws_topk_rows(_stream(), _p(x), n, K, inv_t, _p(ids), _p(vals), _p(stats), rows), "ws_topk_rows")
     return ids, vals, stats
 
 
@@ -295,8 +316,8 @@ def dflash_topk(x, k, workspace=None):
     if not x.is_cuda or x.dim() != 2 or x.dtype != torch.float32 or x.stride(1) != 1:
         raise WsError("x: [rows, n] float32 device tensor with unit inner stride")
     rows, n = x.shape
-    ids = torch.full((rows, k), -1, dtype=torch.int32, device=x.device)
-    vals = torch.zeros((rows, k), dtype=torch.float32, device=x.device)
+    ids = torch.empty((rows, k), dtype=torch.int32, device=x.device)  # (every entry is written, those past a short row as well)
+    vals = torch.empty((rows, k), dtype=torch.float32, device=x.device)
     if workspace is not None:
         check(lib().ws_dflash_topk_ws(_stream(), _p(x), n, x.stride(0), k, _p(ids), _p(vals), rows, _p(workspace),
                                       workspace.numel()), "ws_dflash_topk_ws")
@@ -356,10 +377,7 @@ def accept_sampled(token, flags, row0, ctl_all, area, typical=None, hist=None, s
         if not v.is_cuda or v.dtype != torch.int32 or not v.is_contiguous():
             raise WsError(f"{name}: contiguous int32 device tensor")
     n_seq = row0.numel()
-    n_acc = torch.empty(n_seq, dtype=torch.int32, device=token.device)
-    chosen = torch.empty(n_seq, dtype=torch.int32, device=token.device)
-    status = torch.empty(n_seq, dtype=torch.int32, device=token.device)
-    relaxed = torch.zeros(n_seq, dtype=torch.int32, device=token.device)
+    n_acc, chosen, status, relaxed = torch.zeros((4, n_seq), dtype=torch.int32, device=token.device).unbind()
     a = Accept(token=_p(token), flags=_p(flags), row0=_p(row0), ctl_all=_p(ctl_all), area=_p(area), n_seq=n_seq,
                n_accepted=_p(n_acc), chosen=_p(chosen), status=_p(status), relaxed=_p(relaxed))
     if typical is not None:
@@ -377,10 +395,7 @@ def accept_greedy(ctl_all, area, row0, relax=None, hist=None, slot=None):
     largest logits as ws_topk_rows wrote them. Returns (n_accepted, chosen, status, relaxed, relax_gap)."""
     n_seq = row0.numel()
     dev = row0.device
-    n_acc = torch.empty(n_seq, dtype=torch.int32, device=dev)
-    chosen = torch.empty(n_seq, dtype=torch.int32, device=dev)
-    status = torch.empty(n_seq, dtype=torch.int32, device=dev)
-    relaxed = torch.zeros(n_seq, dtype=torch.int32, device=dev)
+    n_acc, chosen, status, relaxed = torch.zeros((4, n_seq), dtype=torch.int32, device=dev).unbind()
     gap = torch.zeros(n_seq, dtype=torch.float64, device=dev)
     a = AcceptGreedy(ctl_all=_p(ctl_all), area=_p(area), row0=_p(row0), n_seq=n_seq, n_accepted=_p(n_acc), chosen=_p(chosen),
                      status=_p(status), relaxed=_p(relaxed), relax_gap=_p(gap))
@@ -449,14 +464,12 @@ class BatchSampler:
         self.desc = b
 
     def run(self, stream=None):
-        s = _stream() if stream is None else C.c_void_p(stream)
-        check(lib().ws_sample_batch(s, C.byref(self.desc)), "ws_sample_batch")
+        check(lib().ws_sample_batch(_stream() if stream is None else stream, C.byref(self.desc)), "ws_sample_batch")
         return self
 
     def run_static(self, stream=None):
         """The same launch over the library's own workspace (ws_sample_batch_static): nothing of this object's workspace is used."""
-        s = _stream() if stream is None else C.c_void_p(stream)
-        check(lib().ws_sample_batch_static(s, C.byref(self.desc)), "ws_sample_batch_static")
+        check(lib().ws_sample_batch_static(_stream() if stream is None else stream, C.byref(self.desc)), "ws_sample_batch_static")
         return self
 
 

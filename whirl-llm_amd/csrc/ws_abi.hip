@@ -40,6 +40,14 @@ int prepare_short(unsigned lds_limit);
 // ws_few.hip: the same rows shared between workgroups that hold them in registers
 int launch_few(hipStream_t stream, const BatchArgs& a, unsigned lds_bytes, unsigned lds_limit);
 int prepare_few(unsigned lds_limit);
+// ws_top.hip: topk_rows, dflash_topk and draft_sample_rows with rows shared between workgroups
+int launch_topk_shared(hipStream_t stream, const float* x, int n, int K, float inv_t, int* ids, float* vals, float* stats, unsigned rows, unsigned parts,
+                       unsigned chunk_log2, unsigned char* work);
+int launch_dflash_shared(hipStream_t stream, const float* x, int n, int ld, int k, int* ids, float* vals, unsigned rows, unsigned parts, unsigned chunk_log2,
+                         unsigned char* work);
+int launch_draft_shared(hipStream_t stream, const float* x, int n, int* ctl_all, const void* area, int r, const int* map, const void* args, int* qbuf,
+                        unsigned rows, unsigned parts, unsigned chunk_log2, unsigned char* work);
+int prepare_top();
 }  // namespace ws
 
 namespace {
@@ -298,6 +306,7 @@ int prepare_all() {
     if (const int e = ws::prepare_split_kept(kMaxLds - kStaticLds); e != 0) return e;
     if (const int e = ws::prepare_lean(kMaxLds - kStaticLean); e != 0) return e;
     if (const int e = ws::prepare_few(kMaxLds - kStaticFew); e != 0) return e;
+    if (const int e = ws::prepare_top(); e != 0) return e;
     return ws::prepare_short(kMaxLds - kStaticShort);
 }
 
@@ -440,7 +449,9 @@ int ws_draft_sample_rows(void* stream, const float* x, int n, int* ctl_all, cons
 }
 
 namespace {
-unsigned topk_split_log2(const float* x, int n, int K, unsigned rows);
+unsigned top_parts(int n, int K, unsigned rows);
+unsigned chunk_log2(const void* x, uint64_t row_bytes);
+bool top_workspace_ok(const void* w, uint64_t bytes, unsigned rows);
 }
 uint64_t ws_topk_rows_workspace(int n, int K, unsigned rows);
 
@@ -451,16 +462,11 @@ int ws_draft_sample_rows_ws(void* stream, const float* x, int n, int* ctl_all, c
                             const ws_dsamp_args* a, int* qbuf, unsigned rows, void* workspace, uint64_t workspace_bytes) {
     if (!x || !ctl_all || !area || !a || !qbuf || n <= 0 || r < 0 || r >= 16 || rows == 0 || rows > WS_MAX_TABLE_ROWS)
         return WS_E_INVALID;
-    const unsigned lg = topk_split_log2(x, n, 32, rows);
-    if (!lg || !workspace || workspace_bytes < uint64_t{rows} * ws::kTopkSplitRowBytes || reinterpret_cast<uintptr_t>(workspace) % 8u != 0)
+    const unsigned parts = top_parts(n, 32, rows);
+    if (!parts || !top_workspace_ok(workspace, workspace_bytes, rows))
         return ws_draft_sample_rows(stream, x, n, ctl_all, area, r, map, a, qbuf, rows);
-    RowIdx ar;
-    DSampArgs da;
-    std::memcpy(&ar, area, sizeof ar);
-    std::memcpy(&da, a, sizeof da);
-    hipLaunchKernelGGL(draft_sample_rows_split, dim3(rows << lg), dim3(WS_BLOCK), 0, S(stream), x, n, ctl_all, ar, r, map, da, qbuf, lg,
-                       static_cast<unsigned char*>(workspace));
-    return done();
+    return ws::launch_draft_shared(S(stream), x, n, ctl_all, area, r, map, a, qbuf, rows, parts, chunk_log2(x, uint64_t{4} * static_cast<unsigned>(n)),
+                                   static_cast<unsigned char*>(workspace));
 }
 
 int ws_topk_rows(void* stream, const float* x, int n, int K, float inv_t, int* ids, float* vals, float* stats, unsigned rows) {
@@ -470,46 +476,47 @@ int ws_topk_rows(void* stream, const float* x, int n, int K, float inv_t, int* i
 }
 
 namespace {
-// parts per row that pay for ws_topk_rows_ws: a short list (the route that needs no second pass), whole aligned vectors,
-// the launch within the compute units, at least 16384 tokens a part
-unsigned topk_split_log2(const float* x, int n, int K, unsigned rows) {
-    if (K > static_cast<int>(ws::kTopkCap / 4u) || (n & 3) != 0 || (reinterpret_cast<uintptr_t>(x) & 15u) != 0) return 0u;
+// workgroups a row of the shared top-k kernels (0: rows are not shared): a short list, shares that fit the registers of 512
+// threads and have 2048 tokens at least, fewer rows than half the compute units
+unsigned top_parts(int n, int K, unsigned rows) {
+    if (n < 32768 || n % 4 != 0 || rows == 0 || K <= 0 || K > 512) return 0u;  // (the shapes the workspace functions have always named)
     const uint64_t cus = static_cast<uint64_t>(compute_units());
-    unsigned lg = 0;
-    while (lg < 4u && (static_cast<uint64_t>(rows) << (lg + 1u)) <= cus && (n >> (lg + 1u)) >= 16384) ++lg;
-    return lg;
+    const unsigned least = (static_cast<unsigned>(n) + ws::kFewShare - 1u) / ws::kFewShare;
+    uint64_t parts = cus / rows;
+    if (parts > ws::kFewMaxParts) parts = ws::kFewMaxParts;
+    if (parts > static_cast<unsigned>(n) / 2048u) parts = static_cast<unsigned>(n) / 2048u;
+    if (parts < least) parts = least;
+    return parts < 2u || parts > ws::kFewMaxParts || rows * parts > 2u * cus || 2u * rows > cus ? 0u : static_cast<unsigned>(parts);
+}
+// chunks of eight lanes, a line of memory; where rows lie off the lines a chunk straddles two, and longer ones straddle fewer
+unsigned chunk_log2(const void* x, uint64_t row_bytes) { return reinterpret_cast<uintptr_t>(x) % 16u == 0 && row_bytes % 16u == 0 ? 3u : 5u; }
+bool top_workspace_ok(const void* w, uint64_t bytes, unsigned rows) {
+    return w && bytes >= uint64_t{rows} * ws::kFewRowBytes && reinterpret_cast<uintptr_t>(w) % 8u == 0;
 }
 }  // namespace
 
-uint64_t ws_topk_rows_workspace(int n, int K, unsigned rows) {
-    // (the row pointer's alignment is looked at when the launch comes; an aligned one is assumed here)
-    return topk_split_log2(nullptr, n, K, rows) ? uint64_t{rows} * ws::kTopkSplitRowBytes : 0ull;
-}
+uint64_t ws_topk_rows_workspace(int n, int K, unsigned rows) { return top_parts(n, K, rows) ? uint64_t{rows} * ws::kFewRowBytes : 0ull; }
 
 int ws_topk_rows_ws(void* stream, const float* x, int n, int K, float inv_t, int* ids, float* vals, float* stats, unsigned rows,
                     void* workspace, uint64_t workspace_bytes) {
     if (!x || !ids || !vals || !stats || n <= 0 || K <= 0 || rows == 0) return WS_E_INVALID;
-    const unsigned lg = topk_split_log2(x, n, K, rows);
-    if (!lg || !workspace || workspace_bytes < uint64_t{rows} * ws::kTopkSplitRowBytes || reinterpret_cast<uintptr_t>(workspace) % 8u != 0)
-        return ws_topk_rows(stream, x, n, K, inv_t, ids, vals, stats, rows);
-    hipLaunchKernelGGL(topk_rows_split, dim3(rows << lg), dim3(WS_BLOCK), 0, S(stream), x, n, K, inv_t, ids, vals, stats, lg,
-                       static_cast<unsigned char*>(workspace));
-    return done();
+    const unsigned parts = top_parts(n, K, rows);
+    if (!parts || !top_workspace_ok(workspace, workspace_bytes, rows)) return ws_topk_rows(stream, x, n, K, inv_t, ids, vals, stats, rows);
+    return ws::launch_topk_shared(S(stream), x, n, K, inv_t, ids, vals, stats, rows, parts, chunk_log2(x, uint64_t{4} * static_cast<unsigned>(n)),
+                                  static_cast<unsigned char*>(workspace));
 }
 
 uint64_t ws_dflash_topk_workspace(int n, int ld, unsigned rows) {
-    return (ld & 3) == 0 && topk_split_log2(nullptr, n, 64, rows) ? uint64_t{rows} * ws::kTopkSplitRowBytes : 0ull;
+    return ld >= n && ld % 4 == 0 && top_parts(n, 64, rows) ? uint64_t{rows} * ws::kFewRowBytes : 0ull;
 }
 
 int ws_dflash_topk_ws(void* stream, const float* x, int n, int ld, int k, int* ids, float* vals, unsigned rows, void* workspace,
                       uint64_t workspace_bytes) {
     if (!x || !ids || !vals || n <= 0 || ld < n || k <= 0 || k > 64 || rows == 0) return WS_E_INVALID;
-    const unsigned lg = (ld & 3) == 0 ? topk_split_log2(x, n, k, rows) : 0u;  // (rows ld floats apart: whole vectors when ld is)
-    if (!lg || !workspace || workspace_bytes < uint64_t{rows} * ws::kTopkSplitRowBytes || reinterpret_cast<uintptr_t>(workspace) % 8u != 0)
-        return ws_dflash_topk(stream, x, n, ld, k, ids, vals, rows);
-    hipLaunchKernelGGL(dflash_topk_split, dim3(rows << lg), dim3(WS_BLOCK), 0, S(stream), x, n, ld, k, ids, vals, lg,
-                       static_cast<unsigned char*>(workspace));
-    return done();
+    const unsigned parts = ld % 4 == 0 ? top_parts(n, k, rows) : 0u;
+    if (!parts || !top_workspace_ok(workspace, workspace_bytes, rows)) return ws_dflash_topk(stream, x, n, ld, k, ids, vals, rows);
+    return ws::launch_dflash_shared(S(stream), x, n, ld, k, ids, vals, rows, parts, chunk_log2(x, uint64_t{4} * static_cast<unsigned>(ld)),
+                                    static_cast<unsigned char*>(workspace));
 }
 
 int ws_dflash_topk(void* stream, const float* x, int n, int ld, int k, int* ids, float* vals, unsigned rows) {
@@ -586,8 +593,7 @@ int sample_batch_on(void* stream, const ws_batch* b, const BatchPlan& p, unsigne
         a.few_parts = p.few_parts;
         const uint32_t waves = p.few_parts * 8u;  // (512 threads a workgroup)
         a.few_magic = static_cast<uint32_t>(((uint64_t{1} << 32) + waves - 1u) / waves);
-        // chunks of eight lanes, a line of memory; where rows lie off the lines a chunk straddles two, and longer ones straddle fewer
-        a.few_chunk_log2 = p.vec_rows ? 3u : 5u;
+        a.few_chunk_log2 = chunk_log2(b->logits, b->row_stride * (b->dtype == WS_DTYPE_F32 ? 4u : 2u));
         a.work = work;
         a.fb_lds_tie = 0u;
         a.fb_lds_ab = p.short_fb_ab;

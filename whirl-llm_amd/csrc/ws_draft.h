@@ -22,97 +22,94 @@ struct DSampArgs {
 };
 
 namespace ws {
-// one row (b: its place in the tables; sp: the row shared by several workgroups, as in topk_rows_split)
-__device__ __forceinline__ void draft_sample_row(const float* x, int n, int* ctl_all, const RowIdx& area, int r, const int* map,
-                                                 const DSampArgs& a, int* qbuf, int b, TopkSplit sp) {
-    constexpr int QMAX = 32;
-    __shared__ int s_id[QMAX];
-    __shared__ float s_lg[QMAX];
-    __shared__ float s_stats[2];
-    if (a.on[b] == 0) return;
-    int* c = ctl_all + area.v[b];
-    if (c[49] != 0 && c[48] <= r) return;  // chain stopped by the p-min cutoff at or before r
-    x += static_cast<size_t>(b) * n;
+constexpr int kDraftMax = 32;  // candidates of a draft distribution
+// whether row b (its place in the tables) is drawn at draft position r, and with how many candidates
+__device__ __forceinline__ int draft_candidates(const int* ctl_all, const RowIdx& area, int r, const DSampArgs& a, int n, int b) {
+    if (a.on[b] == 0) return 0;
+    const int* c = ctl_all + area.v[b];
+    if (c[49] != 0 && c[48] <= r) return 0;  // chain stopped by the p-min cutoff at or before r
     const int tk = a.top_k[b];
-    int K = (tk > 0 && tk < QMAX) ? tk : QMAX;
-    if (K > n) K = n;
+    return min((tk > 0 && tk < kDraftMax) ? tk : kDraftMax, n);
+}
+// The draw of row b from its K largest logits (LDS: s_id, s_lg; any order that puts the lower of two equal logits' ids first),
+// maximum and normaliser. One wave calls it.
+template <bool SORTED>  // s_id, s_lg: in order (logit desc, id asc)
+__device__ __forceinline__ void draft_finish(int* ctl_all, const RowIdx& area, int r, const int* map, const DSampArgs& a, int* qbuf, int b, int K,
+                                             const int* s_id, const float* s_lg, float top, float sum) {
+    constexpr int QMAX = kDraftMax;
+    int* c = ctl_all + area.v[b];
+    const int tk = a.top_k[b];
     const float inv_t = a.inv_t[b];
-    // one pass over the row: {max, sum exp((x - max) * inv_t)} and the K largest logits in id order, ties at the cut to
-    // the lowest ids (the short-list route of topk_rows)
-    if (!ws::topk_one_row(x, n, K, inv_t, s_id, s_lg, s_stats, sp)) return;  // (a part of a shared row that is not the last to arrive)
-    __syncthreads();
-    const float top = s_stats[0], sum = s_stats[1];
-    if (threadIdx.x >= 64) return;
-    // ---- the rest on one wave, lane i = candidate i (QMAX = 32 <= 64 lanes). What the reference's single thread does in
-    // a fixed order - the running float sums of the filters - is done in that order by every lane for itself, with the
-    // candidates' values read from their lanes; what is independent per candidate (its place in the order, its
-    // probability, its race key with a double-precision logarithm) is done by the candidate's lane.
+    // ---- one wave, lane i = candidate i (QMAX = 32 <= 64 lanes). What the reference's single thread does in a fixed order -
+    // the running float sums of the filters - is done in that order by every lane for itself, with the candidates' values
+    // read from their lanes (v_readlane, a few clocks a term; through the LDS crossbar the loops below took 7 us); what is
+    // independent per candidate (its place in the order, its probability and its share, its race key with a
+    // double-precision logarithm) is done by the candidate's lane.
     const int lane = threadIdx.x;
     const bool live = lane < K;
+    auto value_at = [](float v, int j_) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), j_)); };
+    // front to back over the first n lanes (all the terms there can be, none of them behind a branch: x + 0 is x)
+    auto sum_of = [&](float v, int n) {
+        const float own = lane < n ? v : 0.f;
+        float z = 0.f;
+#pragma unroll
+        for (int i = 0; i < QMAX; ++i) z = __fadd_rn(z, value_at(own, i));
+        return z;
+    };
     const int my_id = live ? (map ? map[s_id[lane]] : s_id[lane]) : 0x7fffffff;
     const float my_lg = live ? s_lg[lane] : -INFINITY;
-    int place = 0;  // logit desc, (mapped) id asc, then the position in the list
-    for (int j = 0; j < K; ++j) {
-        const float lj = __shfl(my_lg, j);
-        const int ij = __shfl(my_id, j);
-        place += (lj > my_lg || (lj == my_lg && (ij < my_id || (ij == my_id && j < lane)))) ? 1 : 0;
+    int place = lane;  // logit desc, (mapped) id asc, then the position in the list
+    if (!SORTED || map) {  // uniform
+        place = 0;
+        for (int j = 0; j < K; ++j) {
+            const float lj = value_at(my_lg, j);
+            const int ij = __builtin_amdgcn_readlane(my_id, j);
+            place += (lj > my_lg || (lj == my_lg && (ij < my_id || (ij == my_id && j < lane)))) ? 1 : 0;
+        }
     }
     // lane r takes the candidate of place r
     const int dst = (live ? place : lane) << 2;
     const int id = __builtin_amdgcn_ds_permute(dst, my_id);
     const float lg = __int_as_float(__builtin_amdgcn_ds_permute(dst, __float_as_int(my_lg)));
     float p = live ? __fdiv_rn(expf(__fmul_rn(__fsub_rn(lg, top), inv_t)), sum) : 0.f;
-    auto p_of = [&](int j) { return __shfl(p, j); };
     int nk = K;
     const bool closed = tk > 0 && tk <= K;
     if (closed) nk = tk;
     const float top_p = a.top_p[b];
     if (top_p < 1.f) {
-        float z = 1.f;
-        if (closed) {
-            z = 0.f;
-            for (int i = 0; i < nk; ++i) z = __fadd_rn(z, p_of(i));
-        }
+        const float z = closed ? sum_of(p, nk) : 1.f;
+        const float share = lane < nk ? __fdiv_rn(p, z) : 0.f;
         float cum = 0.f;
-        for (int j = 0; j < nk; ++j) {
-            cum = __fadd_rn(cum, __fdiv_rn(p_of(j), z));
-            if (cum >= top_p) {
-                nk = j + 1;
-                break;
-            }
+        int before = 0;  // candidates at which the running share has not reached top_p
+#pragma unroll
+        for (int j = 0; j < QMAX; ++j) {
+            cum = __fadd_rn(cum, value_at(share, j));
+            before += cum >= top_p ? 0 : 1;
         }
+        nk = min(nk, before + 1);
     }
     const float min_p = a.min_p[b];
     if (min_p > 0.f && nk > 0) {
-        const float floor_p = __fmul_rn(min_p, p_of(0));
-        int j = 0;
-        while (j < nk && p_of(j) >= floor_p) ++j;
-        nk = j > 1 ? j : 1;
+        const float floor_p = __fmul_rn(min_p, value_at(p, 0));
+        const uint64_t below = __ballot(lane < nk && !(p >= floor_p));  // the first of them ends the kept candidates
+        if (below) nk = max(1, __ffsll(static_cast<unsigned long long>(below)) - 1);
     }
-    float z = 0.f;
-    for (int i = 0; i < nk; ++i) z = __fadd_rn(z, p_of(i));
+    const float z = sum_of(p, nk);
     p = lane < nk ? __fdiv_rn(p, z) : 0.f;
     // race: argmin E(v) / q(v), E(v) = -ln(1 - U(key, v)) (src/common/spec_sample.cpp:83-101); the earlier candidate on
     // equal keys, candidate 0 when none has a probability
     const uint64_t rkey = (static_cast<uint64_t>(a.key_hi[b]) << 32) | a.key_lo[b];
-    const double inf = __longlong_as_double(0x7FF0000000000000ll);
-    double k = inf;
+    double k = __longlong_as_double(0x7FF0000000000000ll);
     if (lane < nk && p > 0.f) {
         const uint64_t h = ws::mix64(rkey + (static_cast<uint64_t>(static_cast<uint32_t>(id)) + 1ull) * 0xE7037ED1A0B428DBull);
-        k = -log(1.0 - ws::unit53(h)) / static_cast<double>(p);
+        k = __builtin_fabs(log(1.0 - ws::unit53(h)) / static_cast<double>(p));  // (the logarithm is not above 0; and no -0)
     }
-    int pick = lane;
-#pragma unroll
-    for (int o = 32; o; o >>= 1) {
-        const double ko = __shfl_xor(k, o);
-        const int po = __shfl_xor(pick, o);
-        if (ko < k || (ko == k && po < pick)) {
-            k = ko;
-            pick = po;
-        }
-    }
-    if (!(k < inf)) pick = 0;
-    const int picked = __shfl(id, pick);
+    // (keys are not negative: their order is that of their bits)
+    const uint64_t kb = static_cast<uint64_t>(__double_as_longlong(k));
+    const uint32_t k_hi = static_cast<uint32_t>(kb >> 32), least_hi = wave_min_u32(k_hi);
+    const uint32_t k_lo = k_hi == least_hi ? static_cast<uint32_t>(kb) : 0xffffffffu, least_lo = wave_min_u32(k_lo);
+    const int pick = least_hi < 0x7FF00000u ? __ffsll(static_cast<unsigned long long>(__ballot(k_hi == least_hi && k_lo == least_lo))) - 1 : 0;
+    const int picked = __builtin_amdgcn_readlane(id, pick);
     int* q = qbuf + a.qoff[b];
     if (lane == 0) {
         c[16 + r] = picked;
@@ -123,22 +120,24 @@ __device__ __forceinline__ void draft_sample_row(const float* x, int n, int* ctl
         q[1 + QMAX + lane] = __float_as_int(p);
     }
 }
+
+__device__ __forceinline__ void draft_sample_row(const float* x, int n, int* ctl_all, const RowIdx& area, int r, const int* map,
+                                                 const DSampArgs& a, int* qbuf, int b, int K) {
+    __shared__ int s_id[kDraftMax];
+    __shared__ float s_lg[kDraftMax];
+    __shared__ float s_stats[2];
+    // one pass over the row: {max, sum exp((x - max) * inv_t)} and the K largest logits in id order, ties at the cut to
+    // the lowest ids (the short-list route of topk_rows)
+    ws::topk_one_row(x + static_cast<size_t>(b) * n, n, K, a.inv_t[b], s_id, s_lg, s_stats);
+    __syncthreads();
+    if (threadIdx.x < 64) draft_finish<false>(ctl_all, area, r, map, a, qbuf, b, K, s_id, s_lg, s_stats[0], s_stats[1]);
+}
 }  // namespace ws
 
+#ifndef WS_NO_NAMED_KERNELS
 extern "C" __global__ void __launch_bounds__(WS_BLOCK)
     draft_sample_rows(const float* x, int n, int* ctl_all, RowIdx area, int r, const int* map, DSampArgs a, int* qbuf) {
-    ws::draft_sample_row(x, n, ctl_all, area, r, map, a, qbuf, static_cast<int>(blockIdx.x), ws::TopkSplit{});
+    const int b = static_cast<int>(blockIdx.x), K = ws::draft_candidates(ctl_all, area, r, a, n, b);
+    if (K > 0) ws::draft_sample_row(x, n, ctl_all, area, r, map, a, qbuf, b, K);
 }
-
-// draft_sample_rows with every row shared by 1 << split_log2 consecutive workgroups (no counterpart in the reference;
-// ws_draft_sample_rows_ws launches it: the draft head's rows come one position after the other, a few rows at a time)
-extern "C" __global__ void __launch_bounds__(WS_BLOCK)
-    draft_sample_rows_split(const float* x, int n, int* ctl_all, RowIdx area, int r, const int* map, DSampArgs a, int* qbuf,
-                            unsigned split_log2, unsigned char* work) {
-    const unsigned row = blockIdx.x >> split_log2;
-    ws::TopkSplit sp;
-    sp.parts = 1u << split_log2;
-    sp.part = blockIdx.x & (sp.parts - 1u);
-    sp.work = work + static_cast<size_t>(row) * ws::kTopkSplitRowBytes;
-    ws::draft_sample_row(x, n, ctl_all, area, r, map, a, qbuf, static_cast<int>(row), sp);
-}
+#endif

@@ -38,13 +38,22 @@ constexpr uint32_t kFewExt = 2048u;  // touched tokens of a share
 constexpr uint32_t kFewDup = 0x4000u, kFewTaken = 0x8000u;  // in a token's 16-bit word, above its history count: a second bias entry, somebody takes it
 constexpr uint32_t kFewDups = 64u;  // bias entries of tokens that another entry has taken
 
+#ifdef WS_SHORT_TIMERS  // (debug builds: clocks since the kernel began, at the unused end of the row's workspace)
+#define WSF_MARK(k) \
+    if (threadIdx.x == 0) reinterpret_cast<long long*>(work + 64512)[k] = clock64() - F.t0
+#else
+#define WSF_MARK(k)
+#endif
 struct FewShared {
+#ifdef WS_SHORT_TIMERS
+    long long t0;
+#endif
     ShortShared sh;
     uint32_t dup_at[kFewDups], dup_j[kFewDups];
     float dup_v[kFewDups];
-    float red_f[WS_WAVES];
+    float red_f[WS_WAVES];  // (few_collect: the row's maximum, and the lowest logit looked at)
     uint32_t w[16];
-    double u;
+    double u, z;
 };
 
 // the largest prefix (bits 31 .. 14) of an order key that at least d lanes of the wave reach, two bits a step
@@ -63,6 +72,331 @@ __device__ __forceinline__ uint32_t lanes_before(uint64_t m) {  // set bits of m
     return __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(m >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(m), 0u));
 }
 
+// What a workgroup of a shared row is given: which share of the row is its own, and how the row is dealt out. Chunk c of the
+// row (2^cl vectors) is wave c mod G's; vector k of a lane lies in its wave's chunk number k * (chunks a load) + lane / (lanes a
+// chunk).
+struct FewShare {
+    uint32_t parts, part, G, g, cl, V, nv, n_vec;  // G: waves a row, g: this one, nv: vectors of the row, n_vec: of a lane
+    template <int DT>
+    __device__ __forceinline__ static FewShare of(uint32_t V, uint32_t parts, uint32_t part, uint32_t cl) {
+        constexpr uint32_t TPV = DT == 0 ? 4u : 8u;
+        FewShare L;
+        L.parts = parts;
+        L.part = part;
+        L.G = parts * WS_WAVES;
+        L.g = part * WS_WAVES + static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)));
+        L.cl = cl;
+        L.V = V;
+        L.nv = (V + TPV - 1u) / TPV;
+        L.n_vec = (L.nv + 64u * L.G - 1u) / (64u * L.G);
+        return L;
+    }
+    __device__ __forceinline__ uint32_t vec_of(uint32_t k) const {
+        const uint32_t lane = threadIdx.x & 63u;
+        return ((((k << (6u - cl)) + (lane >> cl)) * G + g) << cl) + (lane & ((1u << cl) - 1u));
+    }
+};
+// What is wanted of the row: its top_k largest logits, or everything within min_p of its largest
+struct FewWant {
+    bool by_k, by_p;
+    uint32_t top_k;
+    float inv_t;
+    double min_p;
+};
+__device__ __forceinline__ void few_exp_scale(float inv_t, float& k2, float& k2lo) {  // exp(a inv_t) = 2^(a k2 + a k2lo)
+    k2 = inv_t * 1.44269504088896340736f;
+    k2lo = static_cast<float>(static_cast<double>(inv_t) * 1.44269504088896340736 - static_cast<double>(k2));
+}
+
+// Threshold, list and sum of every wave of this workgroup, published in the row's workspace. x: the share in registers (-inf:
+// no token), lm: this thread's largest logit, ext: n_ext more tokens {id, logit}; ok false: the share cannot be listed. SUM
+// false: nobody asks for the normaliser. Returns whether this workgroup is the last of the row's: it has everything to go on.
+template <int DT, int NV, bool SUM>
+__device__ __forceinline__ bool few_publish(const FewShare& L, const FewWant& W, const float (&x)[NV][DT == 0 ? 4 : 8], float lm, const uint4* ext, uint32_t n_ext,
+                                            bool ok, unsigned char* work, FewShared& F) {
+    constexpr uint32_t TPV = DT == 0 ? 4u : 8u;
+    const uint32_t t = threadIdx.x, lane = t & 63u;
+    const uint32_t wv = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(t >> 6)));
+    const uint32_t slots = kFewKeys / L.G;
+    const float wm = wave_max(lm);
+    unsigned long long* gkeys = reinterpret_cast<unsigned long long*>(work);
+    unsigned long long* ghead = reinterpret_cast<unsigned long long*>(work + kFewHead);
+    uint32_t* ctrl = reinterpret_cast<uint32_t*>(work + kFewCtrl);
+
+    WSF_MARK(1);
+    // ---- the threshold
+    float thr = -INFINITY;  // this wave lists its tokens from here up
+    if (W.by_k) {
+        // A wave has top_k / G of the row's top_k largest on average; two more and five times the scatter of that number
+        // are listed, d of them in different lanes.
+        const float lambda = static_cast<float>(W.top_k) / static_cast<float>(L.G);
+        const uint32_t want = static_cast<uint32_t>(lambda + 5.f * __builtin_sqrtf(lambda) + 2.f) + 1u;
+        const uint32_t d = min(60u, want <= 20u ? want : 20u + (want - 20u) / 2u);
+        const uint32_t at = few_lane_threshold(key32(lm), d);
+        thr = at > 0x007fffffu ? unkey32(at) : -INFINITY;  // (below that prefix: -inf and the NaN patterns under it)
+    } else if (W.by_p) {
+        // what the floor lets through lies within -ln(min_p) / W.inv_t of the row's maximum: of the largest logit any part
+        // has reported so far, or this part's (0.02 units of the exponent below: roundings)
+        if (lane == 0u) F.red_f[wv] = wm;
+        __syncthreads();
+        float top = F.red_f[0];
+#pragma unroll
+        for (uint32_t w = 1; w < WS_WAVES; ++w) top = fmaxf(top, F.red_f[w]);
+        if (t == 0) {
+            __hip_atomic_fetch_max(&ctrl[1], key32(top), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            F.w[8] = __hip_atomic_load(&ctrl[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        __syncthreads();
+        top = fmaxf(top, unkey32(F.w[8]));
+        if (top > -INFINITY) thr = __fadd_rn(top, __fdiv_rn(static_cast<float>(log(W.min_p)) - 0.02f, W.inv_t));
+    }
+
+    WSF_MARK(2);
+    // ---- the sum of exp against the wave's maximum, and the list
+    float k2, k2lo;
+    few_exp_scale(W.inv_t, k2, k2lo);
+    const float ref = wm > -INFINITY ? wm : 0.f;
+    float s = 0.f;
+    auto add = [&](float v) {
+        const float a = fmaxf(__fsub_rn(v, ref), -1e30f);
+        s += __builtin_amdgcn_exp2f(fmaf(a, k2lo, a * k2));
+    };
+    uint32_t n_list = 0;  // uniform
+    const float thr_list = fmaxf(thr, -3.402823466e38f);  // (-inf is no token)
+    auto push = [&](float v, uint32_t id) {
+        const bool yes = v >= thr_list;
+        const uint64_t m = __ballot(yes);
+        if (m) {  // uniform
+            const uint32_t slot = n_list + lanes_before(m);
+            if (yes && slot < slots) __hip_atomic_store(&gkeys[slot * L.G + L.g], key64(v, id), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            n_list += static_cast<uint32_t>(__popcll(m));
+        }
+    };
+    if (ok && wm < INFINITY) {
+#pragma unroll
+        for (uint32_t k = 0; k < NV; ++k)
+#pragma unroll
+            for (uint32_t e = 0; e < TPV; ++e)
+                if (k < L.n_vec) push(x[k][e], L.vec_of(k) * TPV + e);
+        for (uint32_t i0 = 0; i0 < n_ext; i0 += WS_BLOCK) {  // uniform
+            uint2 en = make_uint2(0u, 0xff800000u);
+            if (i0 + t < n_ext) en = *reinterpret_cast<const uint2*>(&ext[i0 + t]);
+            push(__uint_as_float(en.y), en.x);
+            if (SUM) add(__uint_as_float(en.y));
+        }
+        if (SUM)
+#pragma unroll
+            for (uint32_t k = 0; k < NV; ++k)
+#pragma unroll
+                for (uint32_t e = 0; e < TPV; ++e)
+                    if (k < L.n_vec) add(x[k][e]);
+    }
+    {
+        const double z = wm > -INFINITY && wm < INFINITY ? wave_sum(static_cast<double>(s)) : 0.0;
+        const uint32_t n = !ok || !(wm < INFINITY) || n_list > slots ? kFewBad : n_list + 1u;
+        if (lane == 0u) {
+            const uint64_t zw = static_cast<uint64_t>(__double_as_longlong(z));
+            __hip_atomic_store(&ghead[L.g], (static_cast<unsigned long long>(key32(wm)) << 32) | key32(thr), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(&ghead[kFewWaves + L.g], (zw & ~uint64_t{kFewBad}) | n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
+    // (The ticket orders nothing by itself and need not: every word the parts exchange is written and read by device-scope
+    // atomic accesses, which go past this unit's caches, and a word still on its way reads as zero and is read again.)
+    WSF_MARK(3);
+    __syncthreads();  // every wave's stores have been issued
+    WSF_MARK(4);
+    if (t == 0) F.w[2] = __hip_atomic_fetch_add(&ctrl[0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    WSF_MARK(5);
+    return F.w[2] == L.parts - 1u;
+}
+
+// The last part: everybody's keys from the larger of the waves' thresholds up - or from a higher bound of the row's top_k-th
+// largest logit - to `list` (LDS, kShortCap keys), in no order; F.red_f[0] and F.z: the row's maximum and normaliser. Every place of
+// the workspace is zero again afterwards. Returns the number of keys (which may be more than the list holds); 0 when a share could not be listed.
+// fourth(): work of the caller's for the fourth wave, while others read the headers.
+template <bool SUM, class FOURTH>
+__device__ __forceinline__ uint32_t few_collect(const FewShare& L, const FewWant& W, unsigned char* work, FewShared& F, uint64_t* list, FOURTH&& fourth) {
+    const uint32_t t = threadIdx.x, lane = t & 63u;
+    const uint32_t wv = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(t >> 6)));
+    unsigned long long* gkeys = reinterpret_cast<unsigned long long*>(work);
+    unsigned long long* ghead = reinterpret_cast<unsigned long long*>(work + kFewHead);
+    uint32_t* ctrl = reinterpret_cast<uint32_t*>(work + kFewCtrl);
+    const uint32_t G = L.G, slots = kFewKeys / G;
+    float k2, k2lo;
+    few_exp_scale(W.inv_t, k2, k2lo);
+    // everybody's keys asked for (those of the first slots right away), then the headers. Four waves read
+    // them side by side, each for what it works out: the threshold, the normaliser, how many keys there are, the uniform.
+    constexpr uint32_t kTries = 64u, kBlind = 4096u / WS_BLOCK, kHL = kFewWaves / 64u;
+    uint64_t got[kBlind];
+#pragma unroll
+    for (uint32_t i = 0; i < kBlind; ++i) got[i] = __hip_atomic_load(&gkeys[i * WS_BLOCK + t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (t < 2u) F.w[5u + t] = 0u;  // keys taken, keys seen
+    if (wv == 3u) {
+        fourth();
+    } else if (wv < 3u) {
+        uint64_t h0[kHL], h1[kHL];
+        bool late = false;
+        for (uint32_t tries = 0; tries < kTries; ++tries) {
+            bool zero = false;
+#pragma unroll
+            for (uint32_t i = 0; i < kHL; ++i) {
+                const uint32_t w = min(i * 64u + lane, G - 1u);
+                h0[i] = __hip_atomic_load(&ghead[w], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                h1[i] = __hip_atomic_load(&ghead[kFewWaves + w], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+#pragma unroll
+            for (uint32_t i = 0; i < kHL; ++i) zero = zero || h0[i] == 0ull || h1[i] == 0ull;
+            late = __ballot(zero) != 0ull;
+            if (!late) break;
+        }
+        float m4[kHL], mx = -INFINITY;
+#pragma unroll
+        for (uint32_t i = 0; i < kHL; ++i) {
+            m4[i] = i * 64u + lane < G ? unkey32(static_cast<uint32_t>(h0[i] >> 32)) : -INFINITY;
+            mx = fmaxf(mx, m4[i]);
+        }
+        mx = wave_max(mx);
+        if (wv == 0u) {
+            float tx = -INFINITY;
+#pragma unroll
+            for (uint32_t i = 0; i < kHL; ++i) tx = fmaxf(tx, unkey32(static_cast<uint32_t>(h0[i])));
+            tx = wave_max(tx);
+            // the keys that are looked at: from the largest of the waves' thresholds up (every wave has listed what it has
+            // there), or - higher - from the top_k-th largest of the waves' maxima
+            float floor_v = tx;
+            if (W.by_k && W.top_k <= G) {
+                float lo = tx, hi = mx;
+                auto reach = [&](float v) {
+                    uint32_t n = 0;
+#pragma unroll
+                    for (uint32_t i = 0; i < kHL; ++i) n += static_cast<uint32_t>(__popcll(__ballot(m4[i] >= v)));
+                    return n;
+                };
+                if (lo > -INFINITY && reach(lo) >= W.top_k)
+                    for (int i = 0; i < 5; ++i) {  // two halvings a step
+                        const float m2 = 0.5f * lo + 0.5f * hi, m1 = 0.5f * lo + 0.5f * m2, m3 = 0.5f * m2 + 0.5f * hi;
+                        const uint32_t n1 = reach(m1), n2 = reach(m2), n3 = reach(m3);
+                        hi = n1 < W.top_k ? m1 : (n2 < W.top_k ? m2 : (n3 < W.top_k ? m3 : hi));
+                        lo = n3 >= W.top_k ? m3 : (n2 >= W.top_k ? m2 : (n1 >= W.top_k ? m1 : lo));
+                    }
+                floor_v = lo;
+            }
+            if (W.by_p) floor_v = __fadd_rn(mx, __fdiv_rn(static_cast<float>(log(W.min_p)) - 0.02f, W.inv_t));
+            if (lane == 0u) {
+                F.red_f[0] = mx;
+                F.red_f[1] = floor_v;
+            }
+        } else if (wv == 1u) {
+            double z = 0.0;
+            if (SUM) {
+#pragma unroll
+                for (uint32_t i = 0; i < kHL; ++i)
+                    if (m4[i] > -INFINITY) {
+                        const float a = fmaxf(__fsub_rn(m4[i], mx), -1e30f);
+                        z += __longlong_as_double(static_cast<long long>(h1[i] & ~uint64_t{kFewBad})) * static_cast<double>(__builtin_amdgcn_exp2f(fmaf(a, k2lo, a * k2)));
+                    }
+                z = wave_sum(z);
+            }
+            if (lane == 0u) F.z = z;
+        } else {
+            uint32_t most = 0, all = 0;
+            bool bad = late || !(mx > -INFINITY);
+#pragma unroll
+            for (uint32_t i = 0; i < kHL; ++i)
+                if (i * 64u + lane < G) {
+                    const uint32_t n = static_cast<uint32_t>(h1[i]) & kFewBad;
+                    bad = bad || n == kFewBad || n == 0u;
+                    most = max(most, n - 1u);
+                    all += n - 1u;
+                }
+            most = wave_max_u32(most);
+            all = wave_sum(all);
+            bad = __ballot(bad) != 0ull;
+            if (lane == 0u) {
+                F.w[3] = bad ? slots : most;  // (a wave that could not list its share may have left keys in every slot)
+                F.w[4] = bad ? 1u : 0u;
+                F.w[7] = all;
+            }
+        }
+    }
+    __syncthreads();
+    WSF_MARK(6);
+    const uint32_t floor_key = key32(F.red_f[1]);
+    const uint32_t n_read = F.w[3] * G;
+    bool bad = F.w[4] != 0u;
+    uint32_t seen = 0;  // uniform
+    auto keep = [&](uint64_t key, uint32_t at) {
+        if (key != 0ull) __hip_atomic_store(&gkeys[at], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // the workspace as the next launch needs it
+        seen += static_cast<uint32_t>(__popcll(__ballot(key != 0ull)));
+        const bool yes = static_cast<uint32_t>(key >> 32) >= floor_key && key != 0ull;
+        const uint64_t mk = __ballot(yes);
+        if (mk) {  // uniform
+            uint32_t at0 = 0;
+            if (lane == 0u) at0 = atomicAdd(&F.w[5], static_cast<uint32_t>(__popcll(mk)));
+            const uint32_t slot = lane_value(at0, 0u) + lanes_before(mk);
+            if (yes && slot < kShortCap) list[slot] = key;
+        }
+    };
+#pragma unroll
+    for (uint32_t i = 0; i < kBlind; ++i)
+        if (i * WS_BLOCK < n_read) keep(got[i], i * WS_BLOCK + t);  // uniform
+    for (uint32_t i0 = kBlind * WS_BLOCK; i0 < n_read; i0 += WS_BLOCK) {
+        const uint32_t at = i0 + t;
+        keep(at < n_read ? __hip_atomic_load(&gkeys[at], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0ull, at);
+    }
+    if (lane == 0u && seen) atomicAdd(&F.w[6], seen);
+    if (t < G) {
+        __hip_atomic_store(&ghead[t], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(&ghead[kFewWaves + t], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if (t < 2u) __hip_atomic_store(&ctrl[t], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    // (a key still on its way was read as zero: looked for again, place by place, until all have come)
+    for (uint32_t tries = 0; !bad && F.w[6] != F.w[7]; ++tries) {  // uniform, rare
+        if (tries == kTries) bad = true;
+        __syncthreads();
+        seen = 0;
+        for (uint32_t i0 = 0; i0 < n_read; i0 += WS_BLOCK)
+            keep(i0 + t < n_read ? __hip_atomic_load(&gkeys[i0 + t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0ull, i0 + t);
+        if (lane == 0u && seen) atomicAdd(&F.w[6], seen);
+        __syncthreads();
+    }
+    WSF_MARK(7);
+    return bad ? 0u : F.w[5];
+}
+
+// The keys of the list (n_keys <= kShortCap) in descending order; returns where they lie.
+__device__ __forceinline__ uint64_t* few_sort(uint64_t* list, uint32_t n_keys, FewShared& F) {
+    const uint32_t t = threadIdx.x;
+    const uint32_t wv = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(t >> 6)));
+    if (n_keys <= 64u) {
+        // WS_BLOCK / 64 threads a key, each counting the larger keys among its share of the 64 places: one barrier
+        constexpr uint32_t kPer = WS_BLOCK / 64u, kEach = 64u / kPer;
+        static_assert(kPer == 8u, "the sum below is over eight lanes");
+        uint64_t* sorted = list + 4096;
+        const uint32_t ki = t / kPer, q0 = (t % kPer) * kEach;
+        const uint64_t own = ki < n_keys ? list[ki] : 0ull;
+        uint32_t above = 0;
+        if (wv * (64u / kPer) < n_keys) {  // (per wave)
+#pragma unroll
+            for (uint32_t i = 0; i < kEach; i += 2u) {
+                const ulonglong2 o = *reinterpret_cast<const ulonglong2*>(&list[q0 + i]);
+                above += (q0 + i < n_keys && o.x > own ? 1u : 0u) + (q0 + i + 1u < n_keys && o.y > own ? 1u : 0u);
+            }
+            above += dpp_or_zero<0x111, 0xf>(above);
+            above += dpp_or_zero<0x112, 0xf>(above);
+            above += dpp_or_zero<0x114, 0xf>(above);  // lanes 7 and 15 of a row of sixteen have the sums of their eight
+            if (ki < n_keys && t % kPer == kPer - 1u) sorted[above] = own;
+        }
+        __syncthreads();
+        list = sorted;
+    } else {
+        short_sort(list, n_keys, F.red_f[0], F.sh);
+    }
+    return list;
+}
+
 // LDS: [0, 32 KiB) the list, [32 KiB, 64 KiB) its sorted copy while it is short; the history counts from 32 KiB on (they are
 // dead by then).
 template <int DT, bool MASKED, int NV>
@@ -78,21 +412,18 @@ __device__ __forceinline__ bool few_row(const BatchArgs& A, const uint32_t row, 
     const uint32_t* allow = MASKED ? A.allow + static_cast<size_t>(row) * A.allow_stride : nullptr;
     finisher = false;
 #ifdef WS_SHORT_TIMERS
+    if (threadIdx.x == 0) F.t0 = clock64();
     const long long wss_t0 = clock64();
 #endif
 
-    // ---- this thread's vectors: chunk c of the row is wave c mod G's; vector k of a lane lies in its wave's chunk number
-    // k * (chunks a load) + lane / (lanes a chunk)
-    const uint32_t G = A.few_parts * WS_WAVES, g = part * WS_WAVES + wv, cl = A.few_chunk_log2;
-    const uint32_t nv = (V + TPV - 1u) / TPV;
+    const FewShare L = FewShare::of<DT>(V, A.few_parts, part, A.few_chunk_log2);
+    const uint32_t G = L.G, cl = L.cl, nv = L.nv, n_vec = L.n_vec;
     const uint32_t j_part = V % TPV ? nv - 1u : 0xffffffffu;
-    const uint32_t n_vec = (nv + 64u * G - 1u) / (64u * G);  // vectors a lane has
     uint4 q[NV];
     uint32_t na[NV];
-    auto vec_of = [&](uint32_t k) { return ((((k << (6u - cl)) + (lane >> cl)) * G + g) << cl) + (lane & ((1u << cl) - 1u)); };
 #pragma unroll
     for (uint32_t k = 0; k < NV; ++k) {
-        const uint32_t j = vec_of(k);
+        const uint32_t j = L.vec_of(k);
         q[k] = row_vector<DT>(base, j, V);
         na[k] = MASKED ? allow[min(j * TPV, V - 1u) >> 5] : 0xffffffffu;
     }
@@ -114,7 +445,6 @@ __device__ __forceinline__ bool few_row(const BatchArgs& A, const uint32_t row, 
 
     // ---- history and bias entries: those of this share are counted, and the first entry of each token puts it, with its
     // logit, on a list (touched tokens: `ext`). A token that both lists name stands there twice; the bias entry's stays.
-    const uint32_t slots = kFewKeys / G;
     uint4* ext = reinterpret_cast<uint4*>(lds);  // {token | kExtBias, logit, bias, place in the bias list}
     constexpr uint32_t kExtBias = 0x80000000u;
     const bool any_ext = lists && !not_mine && n_all;  // uniform
@@ -199,7 +529,7 @@ __device__ __forceinline__ bool few_row(const BatchArgs& A, const uint32_t row, 
             for (uint32_t e = 0; e < TPV; ++e) x[k][e] = -INFINITY;
             continue;
         }
-        const uint32_t j = vec_of(k);
+        const uint32_t j = L.vec_of(k);
         uint4 qq = q[k];
         if (j_part != 0xffffffffu && j == j_part) qq = part_vector<DT>(qq, TPV - V % TPV);
         const uint32_t w[4] = {qq.x, qq.y, qq.z, qq.w};
@@ -268,277 +598,37 @@ __device__ __forceinline__ bool few_row(const BatchArgs& A, const uint32_t row, 
         *reinterpret_cast<uint2*>(&ext[i]) = make_uint2(id, __float_as_uint(v));
         lm = fmaxf(lm, v);
     }
-    const float wm = wave_max(lm);
     WSS_MARK(11);  // touched tokens in
-
     unsigned char* work = A.work + static_cast<size_t>(row) * kFewRowBytes;
-    unsigned long long* gkeys = reinterpret_cast<unsigned long long*>(work);
-    unsigned long long* ghead = reinterpret_cast<unsigned long long*>(work + kFewHead);
-    uint32_t* ctrl = reinterpret_cast<uint32_t*>(work + kFewCtrl);
-
-    // ---- the threshold
-    float thr = -INFINITY;  // this wave lists its tokens from here up
-    if (by_k) {
-        // A wave has top_k / G of the row's top_k largest on average; four more and five times the scatter of that number
-        // are listed, d of them in different lanes.
-        const float lambda = static_cast<float>(top_k) / static_cast<float>(G);
-        const uint32_t want = static_cast<uint32_t>(lambda + 5.f * __builtin_sqrtf(lambda) + 4.f) + 1u;
-        const uint32_t d = min(60u, want <= 20u ? want : 20u + (want - 20u) / 2u);
-        const uint32_t at = few_lane_threshold(key32(lm), d);
-        thr = at > 0x007fffffu ? unkey32(at) : -INFINITY;  // (below that prefix: -inf and the NaN patterns under it)
-    } else if (by_p) {
-        // what the floor lets through lies within -ln(min_p) / inv_t of the row's maximum: of the largest logit any part
-        // has reported so far, or this part's (0.02 units of the exponent below: roundings)
-        if (lane == 0u) F.red_f[wv] = wm;
-        __syncthreads();
-        float top = F.red_f[0];
-#pragma unroll
-        for (uint32_t w = 1; w < WS_WAVES; ++w) top = fmaxf(top, F.red_f[w]);
-        if (t == 0) {
-            __hip_atomic_fetch_max(&ctrl[1], key32(top), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            F.w[8] = __hip_atomic_load(&ctrl[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-        __syncthreads();
-        top = fmaxf(top, unkey32(F.w[8]));
-        if (top > -INFINITY) thr = __fadd_rn(top, __fdiv_rn(static_cast<float>(log(min_p)) - 0.02f, inv_t));
-    }
-
-    WSS_MARK(3);  // threshold
-    // ---- the sum of exp against the wave's maximum, and the list
-    const float k2 = inv_t * 1.44269504088896340736f;
-    const float k2lo = static_cast<float>(static_cast<double>(inv_t) * 1.44269504088896340736 - static_cast<double>(k2));
-    const float ref = wm > -INFINITY ? wm : 0.f;
-    float s = 0.f;
-    auto add = [&](float v) {
-        const float a = fmaxf(__fsub_rn(v, ref), -1e30f);
-        s += __builtin_amdgcn_exp2f(fmaf(a, k2lo, a * k2));
-    };
-    uint32_t n_list = 0;  // uniform
-    const float thr_list = fmaxf(thr, -3.402823466e38f);  // (-inf is no token)
-    auto push = [&](float v, uint32_t id) {
-        const bool yes = v >= thr_list;
-        const uint64_t m = __ballot(yes);
-        if (m) {  // uniform
-            const uint32_t slot = n_list + lanes_before(m);
-            if (yes && slot < slots) __hip_atomic_store(&gkeys[slot * G + g], key64(v, id), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            n_list += static_cast<uint32_t>(__popcll(m));
-        }
-    };
-    if (!not_mine && wm < INFINITY) {
-#pragma unroll
-        for (uint32_t k = 0; k < NV; ++k)
-#pragma unroll
-            for (uint32_t e = 0; e < TPV; ++e)
-                if (k < n_vec) push(x[k][e], vec_of(k) * TPV + e);
-        for (uint32_t i0 = 0; i0 < n_ext; i0 += WS_BLOCK) {  // uniform
-            uint2 en = make_uint2(0u, 0xff800000u);
-            if (i0 + t < n_ext) en = *reinterpret_cast<const uint2*>(&ext[i0 + t]);
-            push(__uint_as_float(en.y), en.x);
-            add(__uint_as_float(en.y));
-        }
-#pragma unroll
-        for (uint32_t k = 0; k < NV; ++k)
-#pragma unroll
-            for (uint32_t e = 0; e < TPV; ++e)
-                if (k < n_vec) add(x[k][e]);
-    }
-    {
-        const double z = wm > -INFINITY && wm < INFINITY ? wave_sum(static_cast<double>(s)) : 0.0;
-        const uint32_t n = not_mine || !(wm < INFINITY) || n_list > slots || n_ext_all > kFewExt ? kFewBad : n_list + 1u;
-        if (lane == 0u) {
-            const uint64_t zw = static_cast<uint64_t>(__double_as_longlong(z));
-            __hip_atomic_store(&ghead[g], (static_cast<unsigned long long>(key32(wm)) << 32) | key32(thr), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(&ghead[kFewWaves + g], (zw & ~uint64_t{kFewBad}) | n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-    }
-    // (The ticket orders nothing by itself and need not: every word the parts exchange is written and read by device-scope
-    // atomic accesses, which go past this unit's caches, and a word still on its way reads as zero and is read again.)
-    WSS_MARK(4);  // listed, summed
-    __syncthreads();  // every wave's stores have been issued
-    WSS_MARK(5);
-    if (t == 0) F.w[2] = __hip_atomic_fetch_add(&ctrl[0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __syncthreads();
-    if (F.w[2] != A.few_parts - 1u) return true;  // not the last: done
+    FewWant W;
+    W.by_k = by_k;
+    W.by_p = by_p;
+    W.top_k = top_k;
+    W.inv_t = inv_t;
+    W.min_p = min_p;
+    if (!few_publish<DT, NV, true>(L, W, x, lm, ext, n_ext, !not_mine && n_ext_all <= kFewExt, work, F)) return true;  // not the last: done
     finisher = true;
     WSS_MARK(6);  // ticket
-    // ---- the last part: everybody's keys asked for (those of the first slots right away), then the headers. Four waves read
-    // them side by side, each for what it works out: the threshold, the normaliser, how many keys there are, the uniform.
-    constexpr uint32_t kTries = 64u, kBlind = 4096u / WS_BLOCK, kHL = kFewWaves / 64u;
-    uint64_t got[kBlind];
-#pragma unroll
-    for (uint32_t i = 0; i < kBlind; ++i) got[i] = __hip_atomic_load(&gkeys[i * WS_BLOCK + t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (t < 2u) F.w[5u + t] = 0u;  // keys taken, keys seen
-    if (wv == 3u) {
-        // (the seed by way of a vector register: as scalar arithmetic the generator's rounds are moved out of this branch)
-        uint32_t seed_lo = static_cast<uint32_t>(P.seed);
-        asm volatile("" : "+v"(seed_lo));
-        const double u_ = batch_uniform(A.rng, (P.seed & 0xffffffff00000000ull) | seed_lo, row, P.step, 0);
-        if (lane == 0u) F.u = u_;
-    } else if (wv < 3u) {
-        uint64_t h0[kHL], h1[kHL];
-        bool late = false;
-        for (uint32_t tries = 0; tries < kTries; ++tries) {
-            bool zero = false;
-#pragma unroll
-            for (uint32_t i = 0; i < kHL; ++i) {
-                const uint32_t w = min(i * 64u + lane, G - 1u);
-                h0[i] = __hip_atomic_load(&ghead[w], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                h1[i] = __hip_atomic_load(&ghead[kFewWaves + w], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
-#pragma unroll
-            for (uint32_t i = 0; i < kHL; ++i) zero = zero || h0[i] == 0ull || h1[i] == 0ull;
-            late = __ballot(zero) != 0ull;
-            if (!late) break;
-        }
-        float m4[kHL], mx = -INFINITY;
-#pragma unroll
-        for (uint32_t i = 0; i < kHL; ++i) {
-            m4[i] = i * 64u + lane < G ? unkey32(static_cast<uint32_t>(h0[i] >> 32)) : -INFINITY;
-            mx = fmaxf(mx, m4[i]);
-        }
-        mx = wave_max(mx);
-        if (wv == 0u) {
-            float tx = -INFINITY;
-#pragma unroll
-            for (uint32_t i = 0; i < kHL; ++i) tx = fmaxf(tx, unkey32(static_cast<uint32_t>(h0[i])));
-            tx = wave_max(tx);
-            // the keys that are looked at: from the largest of the waves' thresholds up (every wave has listed what it has
-            // there), or - higher - from the top_k-th largest of the waves' maxima
-            float floor_v = tx;
-            if (by_k && top_k <= G) {
-                float lo = tx, hi = mx;
-                auto reach = [&](float v) {
-                    uint32_t n = 0;
-#pragma unroll
-                    for (uint32_t i = 0; i < kHL; ++i) n += static_cast<uint32_t>(__popcll(__ballot(m4[i] >= v)));
-                    return n;
-                };
-                if (lo > -INFINITY && reach(lo) >= top_k)
-                    for (int i = 0; i < 5; ++i) {  // two halvings a step
-                        const float m2 = 0.5f * lo + 0.5f * hi, m1 = 0.5f * lo + 0.5f * m2, m3 = 0.5f * m2 + 0.5f * hi;
-                        const uint32_t n1 = reach(m1), n2 = reach(m2), n3 = reach(m3);
-                        hi = n1 < top_k ? m1 : (n2 < top_k ? m2 : (n3 < top_k ? m3 : hi));
-                        lo = n3 >= top_k ? m3 : (n2 >= top_k ? m2 : (n1 >= top_k ? m1 : lo));
-                    }
-                floor_v = lo;
-            }
-            if (by_p) floor_v = __fadd_rn(mx, __fdiv_rn(static_cast<float>(log(min_p)) - 0.02f, inv_t));
-            if (lane == 0u) {
-                F.red_f[0] = mx;
-                F.red_f[1] = floor_v;
-            }
-        } else if (wv == 1u) {
-            double z = 0.0;
-#pragma unroll
-            for (uint32_t i = 0; i < kHL; ++i)
-                if (m4[i] > -INFINITY) {
-                    const float a = fmaxf(__fsub_rn(m4[i], mx), -1e30f);
-                    z += __longlong_as_double(static_cast<long long>(h1[i] & ~uint64_t{kFewBad})) * static_cast<double>(__builtin_amdgcn_exp2f(fmaf(a, k2lo, a * k2)));
-                }
-            z = wave_sum(z);
-            if (lane == 0u) S.s_d[0] = z;
-        } else {
-            uint32_t most = 0, all = 0;
-            bool bad = late || !(mx > -INFINITY);
-#pragma unroll
-            for (uint32_t i = 0; i < kHL; ++i)
-                if (i * 64u + lane < G) {
-                    const uint32_t n = static_cast<uint32_t>(h1[i]) & kFewBad;
-                    bad = bad || n == kFewBad || n == 0u;
-                    most = max(most, n - 1u);
-                    all += n - 1u;
-                }
-            most = wave_max_u32(most);
-            all = wave_sum(all);
-            bad = __ballot(bad) != 0ull;
-            if (lane == 0u) {
-                F.w[3] = bad ? slots : most;  // (a wave that could not list its share may have left keys in every slot)
-                F.w[4] = bad ? 1u : 0u;
-                F.w[7] = all;
-            }
-        }
-    }
-    __syncthreads();
-    WSS_MARK(7);  // headers
-    const float m = F.red_f[0];
-    const uint32_t floor_key = key32(F.red_f[1]);
-    const double z = S.s_d[0];
-    const uint32_t n_read = F.w[3] * G;
-    bool bad = F.w[4] != 0u;
     uint64_t* list = reinterpret_cast<uint64_t*>(lds);
-    uint32_t seen = 0;  // uniform
-    auto keep = [&](uint64_t key, uint32_t at) {
-        if (key != 0ull) __hip_atomic_store(&gkeys[at], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // the workspace as the next launch needs it
-        seen += static_cast<uint32_t>(__popcll(__ballot(key != 0ull)));
-        const bool yes = static_cast<uint32_t>(key >> 32) >= floor_key && key != 0ull;
-        const uint64_t mk = __ballot(yes);
-        if (mk) {  // uniform
-            uint32_t at0 = 0;
-            if (lane == 0u) at0 = atomicAdd(&F.w[5], static_cast<uint32_t>(__popcll(mk)));
-            const uint32_t slot = lane_value(at0, 0u) + lanes_before(mk);
-            if (yes && slot < kShortCap) list[slot] = key;
-        }
-    };
-#pragma unroll
-    for (uint32_t i = 0; i < kBlind; ++i)
-        if (i * WS_BLOCK < n_read) keep(got[i], i * WS_BLOCK + t);  // uniform
-    for (uint32_t i0 = kBlind * WS_BLOCK; i0 < n_read; i0 += WS_BLOCK) {
-        const uint32_t at = i0 + t;
-        keep(at < n_read ? __hip_atomic_load(&gkeys[at], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0ull, at);
-    }
-    if (lane == 0u && seen) atomicAdd(&F.w[6], seen);
-    if (t < G) {
-        __hip_atomic_store(&ghead[t], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(&ghead[kFewWaves + t], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    if (t < 2u) __hip_atomic_store(&ctrl[t], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __syncthreads();
-    // (a key still on its way was read as zero: looked for again, place by place, until all have come)
-    for (uint32_t tries = 0; !bad && F.w[6] != F.w[7]; ++tries) {  // uniform, rare
-        if (tries == kTries) bad = true;
-        __syncthreads();
-        seen = 0;
-        for (uint32_t i0 = 0; i0 < n_read; i0 += WS_BLOCK)
-            keep(i0 + t < n_read ? __hip_atomic_load(&gkeys[i0 + t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0ull, i0 + t);
-        if (lane == 0u && seen) atomicAdd(&F.w[6], seen);
-        __syncthreads();
-    }
-    const uint32_t n_keys = F.w[5];
+    const uint32_t n_keys = few_collect<true>(L, W, work, F, list, [&]() {
+            // (the seed by way of a vector register: as scalar arithmetic the generator's rounds are moved out of this branch)
+            uint32_t seed_lo = static_cast<uint32_t>(P.seed);
+            asm volatile("" : "+v"(seed_lo));
+            const double u_ = batch_uniform(A.rng, (P.seed & 0xffffffff00000000ull) | seed_lo, row, P.step, 0);
+            if (lane == 0u) F.u = u_;
+    });
+    const float m = F.red_f[0];
     const uint32_t n_cand = by_k ? top_k : n_keys;
-    if (bad || n_keys < n_cand || n_cand == 0u || n_keys > kShortCap) return false;
+    if (n_keys < n_cand || n_cand == 0u || n_keys > kShortCap) return false;
 
     WSS_MARK(8);  // keys
-    // ---- the candidates in order
-    if (n_keys <= 64u) {
-        // WS_BLOCK / 64 threads a key, each counting the larger keys among its share of the 64 places: one barrier
-        constexpr uint32_t kPer = WS_BLOCK / 64u, kEach = 64u / kPer;
-        static_assert(kPer == 8u, "the sum below is over eight lanes");
-        uint64_t* sorted = list + 4096;
-        const uint32_t ki = t / kPer, q0 = (t % kPer) * kEach;
-        const uint64_t own = ki < n_keys ? list[ki] : 0ull;
-        uint32_t above = 0;
-        if (wv * (64u / kPer) < n_keys) {  // (per wave)
-#pragma unroll
-            for (uint32_t i = 0; i < kEach; i += 2u) {
-                const ulonglong2 o = *reinterpret_cast<const ulonglong2*>(&list[q0 + i]);
-                above += (q0 + i < n_keys && o.x > own ? 1u : 0u) + (q0 + i + 1u < n_keys && o.y > own ? 1u : 0u);
-            }
-            above += dpp_or_zero<0x111, 0xf>(above);
-            above += dpp_or_zero<0x112, 0xf>(above);
-            above += dpp_or_zero<0x114, 0xf>(above);  // lanes 7 and 15 of a row of sixteen have the sums of their eight
-            if (ki < n_keys && t % kPer == kPer - 1u) sorted[above] = own;
-        }
-        __syncthreads();
-        list = sorted;
-    } else {
-        short_sort(list, n_keys, m, inv_t * 64.f, S);
-    }
+    list = few_sort(list, n_keys, F);
     WSS_MARK(9);  // sorted
     ShortRow R;
     R.top_p = P.top_p;
     R.min_p = min_p;
     R.u = F.u;
-    R.z = z;
+    R.z = F.z;
     R.inv_t = inv_t;
     R.m = m;
     R.n_cand = n_cand;
@@ -547,7 +637,7 @@ __device__ __forceinline__ bool few_row(const BatchArgs& A, const uint32_t row, 
 #ifdef WS_SHORT_TIMERS
     WSS_MARK(10);
     __syncthreads();
-    if (t < 16 && A.kept_logits) A.kept_logits[static_cast<size_t>(row) * A.kept_cap + 100u + t] = t == 15 ? static_cast<float>(n_keys) : (t == 14 ? static_cast<float>(n_read) : S.marks[t]);
+    if (t < 16 && A.kept_logits) A.kept_logits[static_cast<size_t>(row) * A.kept_cap + 100u + t] = t == 15 ? static_cast<float>(n_keys) : (t == 14 ? 0.f : S.marks[t]);
 #endif
     return true;
 }

@@ -174,7 +174,7 @@ __device__ __forceinline__ T pick4(uint32_t k, T a0, T a1, T a2, T a3) {
 }
 
 // Sorts the n (<= kShortCap) different 64-bit keys keys[0 .. n) in LDS into descending order. bucket_of(key) in [0, nb)
-// (nb: 64 or 256; bcnt, bstart: nb words of LDS each) must not rise along that order (equal for keys it cannot tell apart): a key's place is the start of its bucket plus
+// (nb: 64 or 512; bcnt, bstart: nb words of LDS each, 16-byte aligned) must not rise along that order (equal for keys it cannot tell apart): a key's place is the start of its bucket plus
 // the number of larger keys among the bucket's members, which it reads after all keys have been laid out bucket by
 // bucket - a few dozen reads a key where a full comparison sort takes dozens of barriers. Every thread calls it.
 template <class B>
@@ -184,34 +184,37 @@ __device__ __forceinline__ void bucket_sort_desc(uint64_t* keys, uint32_t n, uin
     uint64_t key[K];
     uint32_t bk[K], pos[K];
 #pragma unroll
-    for (uint32_t k = 0; k < K; ++k) key[k] = k * WS_BLOCK + t < n ? keys[k * WS_BLOCK + t] : 0ull;
-    if (t < nb) bcnt[t] = 0u;
+    for (uint32_t k = 0; k < K; ++k)
+        if (k * WS_BLOCK < n) key[k] = k * WS_BLOCK + t < n ? keys[k * WS_BLOCK + t] : 0ull;  // (uniform: rounds past the list issue nothing)
+    for (uint32_t i = t; i < nb; i += WS_BLOCK) bcnt[i] = 0u;
     __syncthreads();
 #pragma unroll
     for (uint32_t k = 0; k < K; ++k)
-        if (k * WS_BLOCK + t < n) {
+        if (k * WS_BLOCK < n && k * WS_BLOCK + t < n) {
             bk[k] = min(nb - 1u, bucket_of(key[k]));
             pos[k] = atomicAdd(&bcnt[bk[k]], 1u);
         }
     __syncthreads();
-    if (t < 64u) {  // one wave: nb / 64 consecutive counts a lane
-        const uint32_t per = nb >> 6;
-        uint32_t c = 0;
-        for (uint32_t i = 0; i < per; ++i) c += bcnt[t * per + i];
-        uint32_t run = wave_incl_scan(c) - c;
-        for (uint32_t i = 0; i < per; ++i) {
-            bstart[t * per + i] = run;
-            run += bcnt[t * per + i];
+    if (t < 64u) {  // one wave: one or eight consecutive counts a lane
+        if (nb == 64u) {
+            const uint32_t c = bcnt[t];
+            bstart[t] = wave_incl_scan(c) - c;
+        } else {
+            const uint4 a = *reinterpret_cast<const uint4*>(&bcnt[t * 8u]), b = *reinterpret_cast<const uint4*>(&bcnt[t * 8u + 4u]);
+            const uint32_t sa = a.x + a.y + a.z + a.w, sum = sa + b.x + b.y + b.z + b.w;
+            const uint32_t run = wave_incl_scan(sum) - sum, mid = run + sa;
+            *reinterpret_cast<uint4*>(&bstart[t * 8u]) = make_uint4(run, run + a.x, run + a.x + a.y, run + a.x + a.y + a.z);
+            *reinterpret_cast<uint4*>(&bstart[t * 8u + 4u]) = make_uint4(mid, mid + b.x, mid + b.x + b.y, mid + b.x + b.y + b.z);
         }
     }
     __syncthreads();
 #pragma unroll
     for (uint32_t k = 0; k < K; ++k)
-        if (k * WS_BLOCK + t < n) keys[bstart[bk[k]] + pos[k]] = key[k];
+        if (k * WS_BLOCK < n && k * WS_BLOCK + t < n) keys[bstart[bk[k]] + pos[k]] = key[k];
     __syncthreads();
 #pragma unroll
     for (uint32_t k = 0; k < K; ++k)
-        if (k * WS_BLOCK + t < n) {
+        if (k * WS_BLOCK < n && k * WS_BLOCK + t < n) {
             const uint32_t b0 = bstart[bk[k]], c = bcnt[bk[k]];
             uint32_t above = 0;
             for (uint32_t i = 0; i < c; i += 4u) {  // four reads on their way together
@@ -226,7 +229,7 @@ __device__ __forceinline__ void bucket_sort_desc(uint64_t* keys, uint32_t n, uin
     __syncthreads();
 #pragma unroll
     for (uint32_t k = 0; k < K; ++k)
-        if (k * WS_BLOCK + t < n) keys[pos[k]] = key[k];
+        if (k * WS_BLOCK < n && k * WS_BLOCK + t < n) keys[pos[k]] = key[k];
     __syncthreads();
 }
 

@@ -183,6 +183,7 @@ struct RowIdx {
     int v[32];
 };
 
+#ifndef WS_NO_NAMED_KERNELS  // (a translation unit that only wants the functions)
 extern "C" __global__ void __launch_bounds__(WS_BLOCK) argmax(const float* x, int n, int* out, int* ids, int* pos, int advance) {
     const ws::RowTop t = ws::row_top<false>(x, n);
     if (threadIdx.x == 0) {
@@ -261,3 +262,4 @@ extern "C" __global__ void __launch_bounds__(WS_BLOCK)
         out_prob[0] = 1.f / t.sum;
     }
 }
+#endif

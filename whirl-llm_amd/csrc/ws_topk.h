@@ -15,6 +15,8 @@
 
 namespace ws {
 
+constexpr uint32_t kTopkPer = 4096u / WS_BLOCK;  // bins a thread scans
+
 // Block-wide: the key of the kk-th largest element of x[0..n) and how many elements equal to it belong to the top kk.
 // hist: LDS, 4096 words. NaN -> -inf.
 __device__ __forceinline__ void radix_kth(const float* __restrict__ x, int n, uint32_t kk, uint32_t* hist, uint32_t* red,
@@ -32,11 +34,11 @@ __device__ __forceinline__ void radix_kth(const float* __restrict__ x, int n, ui
             if ((k & mask) == prefix) atomicAdd(&hist[(k >> shift) & (nb - 1)], 1u);
         });
         __syncthreads();
-        // bins in descending order, 4 per thread (nb = 256: thread t < 64 owns 4 bins, the rest own none)
-        uint32_t c[4], tot = 0;
+        // bins in descending order, kTopkPer per thread (nb = 256: the first threads own all of them)
+        uint32_t c[kTopkPer], tot = 0;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const uint32_t pos = 4u * threadIdx.x + j;  // rank of the bin from the top
+        for (uint32_t j = 0; j < kTopkPer; ++j) {
+            const uint32_t pos = kTopkPer * threadIdx.x + j;  // rank of the bin from the top
             c[j] = pos < nb ? hist[nb - 1 - pos] : 0u;
             tot += c[j];
         }
@@ -48,9 +50,9 @@ __device__ __forceinline__ void radix_kth(const float* __restrict__ x, int n, ui
         }
         __syncthreads();
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
+        for (uint32_t j = 0; j < kTopkPer; ++j) {
             if (above < need && above + c[j] >= need) {
-                s_sel[0] = nb - 1 - (4u * threadIdx.x + j);
+                s_sel[0] = nb - 1 - (kTopkPer * threadIdx.x + j);
                 s_sel[1] = need - above;
             }
             above += c[j];
@@ -232,10 +234,10 @@ __device__ __forceinline__ int topk_from_list(const float* __restrict__ x, const
                                                float* vals) {
     const uint32_t t = threadIdx.x;
     // the bin of the kk-th largest, as in the count route
-    uint32_t c[4], tot = 0;
+    uint32_t c[kTopkPer], tot = 0;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        c[j] = work[4u * t + j];
+    for (uint32_t j = 0; j < kTopkPer; ++j) {
+        c[j] = work[kTopkPer * t + j];
         tot += c[j];
     }
     uint32_t all;
@@ -247,9 +249,9 @@ __device__ __forceinline__ int topk_from_list(const float* __restrict__ x, const
     }
     __syncthreads();
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (uint32_t j = 0; j < kTopkPer; ++j) {
         if (above < kk && above + c[j] >= kk) {
-            sel[0] = 4u * t + j;
+            sel[0] = kTopkPer * t + j;
             sel[1] = kk - above;
         }
         above += c[j];
@@ -315,11 +317,11 @@ __device__ __forceinline__ bool topk_by_counts(const float* __restrict__ x, int 
                                                int* ids, float* vals) {
     const uint32_t t = threadIdx.x, lane = static_cast<uint32_t>(lane_id());
     const uint32_t wv = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(t >> 6)));
-    // the bin the kk-th largest falls in: bins ascend as logits fall, 4 consecutive bins per thread
-    uint32_t c[4], tot = 0;
+    // the bin the kk-th largest falls in: bins ascend as logits fall, consecutive bins per thread
+    uint32_t c[kTopkPer], tot = 0;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        c[j] = L.hist[4u * t + j];
+    for (uint32_t j = 0; j < kTopkPer; ++j) {
+        c[j] = L.hist[kTopkPer * t + j];
         tot += c[j];
     }
     uint32_t all;
@@ -331,9 +333,9 @@ __device__ __forceinline__ bool topk_by_counts(const float* __restrict__ x, int 
     if (t < WS_WAVES) L.cnt[t] = 0u;
     __syncthreads();
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (uint32_t j = 0; j < kTopkPer; ++j) {
         if (above < kk && above + c[j] >= kk) {
-            L.sel[0] = 4u * t + j;
+            L.sel[0] = kTopkPer * t + j;
             L.sel[1] = kk - above;
         }
         above += c[j];
@@ -434,22 +436,10 @@ __device__ __forceinline__ bool topk_by_counts(const float* __restrict__ x, int 
 
 // The K largest logits of one row (x, n tokens) into ids / vals in ascending id order, ties at the cut to the lowest ids;
 // stats (unless null) = {max, sum exp((x - max) * inv_t)}. Every return is taken by the whole workgroup.
-// A row shared by several workgroups (few rows, a short list: K up to kTopkCap / 4): every part takes the bound, the
-// bins and the listing threshold from the head of the row (the same for all), runs the first pass over its slice,
-// and leaves its listed tokens, its maximum and its sum (against the common reference) in the row's workspace; the part
-// that arrives last takes them all and goes on as the one workgroup does with the same list - so the same ids and
-// values; the normaliser is the sum of the parts' sums. Rows the short-list route does not take are done by part 0 alone.
-// Workspace of a row: kTopkCap keys, then 64 words: [0] parts arrived, [1] tokens listed, [2] a wave's stretch of the
-// list overflowed, [16 + 2 p], [17 + 2 p] maximum and sum of part p. Zero-filled once; every launch leaves [0..2] at zero.
-constexpr uint64_t kTopkSplitRowBytes = kTopkCap * 8ull + 256ull;
-struct TopkSplit {
-    uint32_t parts = 1u, part = 0u;
-    unsigned char* work = nullptr;  // of this row
-};
-
+// (Few rows with a short list are shared between workgroups by the kernels of ws_top.h, which call this for the rows they
+// cannot list.)
 template <bool SUM = true>
-__device__ __forceinline__ bool topk_one_row(const float* x, int n, int K, float inv_t, int* ids, float* vals, float* stats,
-                                             TopkSplit sp = TopkSplit{}) {
+__device__ __forceinline__ void topk_one_row(const float* x, int n, int K, float inv_t, int* ids, float* vals, float* stats) {
     __shared__ __align__(16) uint32_t hist[4096];  // also viewed as 64- and 128-bit words
     __shared__ uint64_t cand[ws::kTopkCap];
     __shared__ float red_f[WS_WAVES];
@@ -495,10 +485,10 @@ __device__ __forceinline__ bool topk_one_row(const float* x, int n, int K, float
             for (int e = 0; e < 4; ++e) atomicAdd(&hist[ws::topk_bin(v[e], scale, a32, tail)], 1u);
             __syncthreads();
             const uint32_t want = min(4u * WS_BLOCK, static_cast<uint32_t>((2ull * kk * 4u * WS_BLOCK) / static_cast<uint32_t>(n)) + 8u);
-            uint32_t c[4], tot = 0;
+            uint32_t c[kTopkPer], tot = 0;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                c[j] = hist[4u * threadIdx.x + j];
+            for (uint32_t j = 0; j < kTopkPer; ++j) {
+                c[j] = hist[kTopkPer * threadIdx.x + j];
                 tot += c[j];
             }
             uint32_t all;
@@ -506,8 +496,8 @@ __device__ __forceinline__ bool topk_one_row(const float* x, int n, int K, float
             if (threadIdx.x == 0) s_sel[0] = 0xffffffffu;
             __syncthreads();
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                if (above < want && above + c[j] >= want) s_sel[0] = 4u * threadIdx.x + j;
+            for (uint32_t j = 0; j < kTopkPer; ++j) {
+                if (above < want && above + c[j] >= want) s_sel[0] = kTopkPer * threadIdx.x + j;
                 above += c[j];
             }
             __syncthreads();
@@ -523,74 +513,7 @@ __device__ __forceinline__ bool topk_one_row(const float* x, int n, int K, float
     // the maximum between the two: terms up to e^(8 inv_t), which a float holds for temperatures above 1 / 8)
     const float nan = __uint_as_float(0x7fc00000u);
     const float ref = (counted && inv_t > 0.f && inv_t <= 8.f) ? bound - 8.f : nan;
-    bool split = sp.parts > 1u;
-    if (split && !(counted && list_bin >= 0 && (!SUM || ref == ref))) {  // (every part sees the same head: the same answer)
-        if (sp.part != 0u) return false;
-        split = false;
-    }
-    if (split) {
-        __shared__ uint32_t s_meet[4];
-        const uint32_t t = threadIdx.x, w = ws::wave_id(), l = ws::lane_id();
-        const int nv_all = n >> 2, per = (nv_all + static_cast<int>(sp.parts) - 1) / static_cast<int>(sp.parts);
-        const int v0 = min(static_cast<int>(sp.part) * per, nv_all), v1 = min(v0 + per, nv_all);
-        ws::topk_first_pass<true, SUM>(x + 4 * v0, 4 * (v1 - v0), inv_t, scale, a32, hist, list_bin, cand, s_wn, ref, m, s,
-                                       static_cast<uint32_t>(4 * v0));
-        __syncthreads();  // the wave lists and their counters are complete
-        const float top_p = ws::block_max(m, red_f);
-        const float sum_p = ws::block_sum(s, red_f);  // against ref, like every part's
-        unsigned long long* glist = reinterpret_cast<unsigned long long*>(sp.work);
-        uint32_t* ctrl = reinterpret_cast<uint32_t*>(sp.work + ws::kTopkCap * 8ull);
-        {
-            // this wave's stretch of the list goes to the row's common list (stores and loads that every compute unit
-            // sees; acknowledged before the arrival counter is touched, so no cache write-back is needed)
-            const uint32_t mine = s_wn[w], cnt = min(mine, ws::kTopkWaveCap);
-            uint32_t base = 0;
-            if (l == 0 && cnt) base = __hip_atomic_fetch_add(&ctrl[1], cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            base = static_cast<uint32_t>(__shfl(static_cast<int>(base), 0));
-            for (uint32_t e = l; e < cnt; e += 64u)
-                if (base + e < ws::kTopkCap)
-                    __hip_atomic_store(&glist[base + e], static_cast<unsigned long long>(cand[w * ws::kTopkWaveCap + e]), __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_AGENT);
-            if (l == 0 && mine > ws::kTopkWaveCap) __hip_atomic_fetch_or(&ctrl[2], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (t == 0) {
-                __hip_atomic_store(&ctrl[16u + 2u * sp.part], __float_as_uint(top_p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                __hip_atomic_store(&ctrl[17u + 2u * sp.part], __float_as_uint(sum_p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
-        }
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
-        if (t == 0) s_meet[0] = __hip_atomic_fetch_add(&ctrl[0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __syncthreads();
-        if (s_meet[0] != sp.parts - 1u) return false;
-        // the last one to arrive: everything is there
-        const uint32_t total = __hip_atomic_load(&ctrl[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const uint32_t over = __hip_atomic_load(&ctrl[2], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        float top_all = -INFINITY, sum_all = 0.f;
-        for (uint32_t p = 0; p < sp.parts; ++p) {  // (every thread, in part order: the same sum everywhere)
-            top_all = fmaxf(top_all, __uint_as_float(__hip_atomic_load(&ctrl[16u + 2u * p], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)));
-            sum_all += __uint_as_float(__hip_atomic_load(&ctrl[17u + 2u * p], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-        }
-        __syncthreads();  // every thread has read the counters
-        if (t < 3) __hip_atomic_store(&ctrl[t], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // as the next launch needs them
-        const bool whole = !over && total <= ws::kTopkCap;
-        for (int b = t; b < ws::kTopkBins; b += WS_BLOCK) hist[b] = 0u;
-        if (t < WS_WAVES) {
-            const uint32_t before = t * ws::kTopkWaveCap;
-            // the common list as one stretch after the other; an overflow shows as a stretch that is too long (the row is then counted in full)
-            s_wn[t] = whole ? (total > before ? min(total - before, ws::kTopkWaveCap) : 0u) : (t == 0 ? ws::kTopkWaveCap + 1u : 0u);
-        }
-        __syncthreads();
-        if (whole) {
-            for (uint32_t i = t; i < total; i += WS_BLOCK) {
-                const uint64_t k = __hip_atomic_load(&glist[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                cand[i] = k;
-                atomicAdd(&hist[ws::topk_bin(ws::unkey32(static_cast<uint32_t>(k >> 32)), scale, a32, 4095.f)], 1u);  // the counts of the listed bins
-            }
-        }
-        m = top_all;
-        s = t == 0 ? sum_all : 0.f;
-        __syncthreads();
-    } else if (counted) {
+    if (counted) {
         ws::topk_first_pass<true, SUM>(x, n, inv_t, scale, a32, hist, list_bin, cand, s_wn, ref, m, s);
     } else {
         ws::topk_first_pass<false, SUM>(x, n, inv_t, scale, a32, hist, -1, cand, s_wn, nan, m, s);
@@ -608,7 +531,7 @@ __device__ __forceinline__ bool topk_one_row(const float* x, int n, int K, float
         stats[0] = top;
         stats[1] = sum;
     }
-    if (kk == 0) return true;
+    if (kk == 0) return;
     __syncthreads();  // the counts are complete
 
     int counts_left = counted && top <= bound;  // uniform
@@ -622,7 +545,7 @@ __device__ __forceinline__ bool topk_one_row(const float* x, int n, int K, float
         if (listed >= kk && fits) {  // the K largest are all on the list
             __shared__ uint32_t s_list[4];
             const int rc = ws::topk_from_list(x, cand, s_wn, list_bin, kk, scale, a32, hist, red_u, s_list, ids, vals);
-            if (rc == 0) return true;
+            if (rc == 0) return;
             __syncthreads();
             counts_left = rc == 1;
         }
@@ -638,7 +561,7 @@ __device__ __forceinline__ bool topk_one_row(const float* x, int n, int K, float
     }
     if (counts_left) {
         const ws::TopkLds L{hist, cand, red_f, red_u, s_sel, s_cnt, &s_n, &s_kmin};
-        if (ws::topk_by_counts(x, n, kk, scale, a32, L, ids, vals)) return true;
+        if (ws::topk_by_counts(x, n, kk, scale, a32, L, ids, vals)) return;
         __syncthreads();
     }
 
@@ -649,36 +572,26 @@ __device__ __forceinline__ bool topk_one_row(const float* x, int n, int K, float
         ids[o] = i;
         vals[o] = v;
     });
-    return true;
+    return;
 }
 
 }  // namespace ws
 
+#ifndef WS_NO_NAMED_KERNELS  // (a translation unit that only wants the functions)
 extern "C" __global__ void __launch_bounds__(WS_BLOCK)
     topk_rows(const float* x, int n, int K, float inv_t, int* ids, float* vals, float* stats) {
     const size_t row = blockIdx.x;
     ws::topk_one_row(x + row * n, n, K, inv_t, ids + row * K, vals + row * K, stats + 2 * row);
 }
-
-// topk_rows with every row shared by 1 << split_log2 consecutive workgroups (no counterpart in the reference, whose
-// kernel gives a row to one workgroup; ws_topk_rows_ws launches it for small batches)
-extern "C" __global__ void __launch_bounds__(WS_BLOCK)
-    topk_rows_split(const float* x, int n, int K, float inv_t, int* ids, float* vals, float* stats, unsigned split_log2, unsigned char* work) {
-    const size_t row = blockIdx.x >> split_log2;
-    ws::TopkSplit sp;
-    sp.parts = 1u << split_log2;
-    sp.part = blockIdx.x & (sp.parts - 1u);
-    sp.work = work + row * ws::kTopkSplitRowBytes;
-    ws::topk_one_row(x + row * n, n, K, inv_t, ids + row * K, vals + row * K, stats + 2 * row, sp);
-}
+#endif
 
 // dflash_topk(x, n, ld, k, ids, vals) of kernels/dflash.hip:36-77: the k <= 64 largest logits of each row in key order
 // (larger value first, then smaller index; NaN counts as -inf and is written out as it stands), rows ld floats apart.
 // The reference takes k passes over the row, one winner each; here the row is read once by the select above and the
 // k winners are put in order by one wave.
 namespace ws {
-__device__ __forceinline__ void dflash_topk_row(const float* x, int n, int k, int* ids, float* vals, TopkSplit sp) {
-    if (!ws::topk_one_row<false>(x, n, k, 1.f, ids, vals, nullptr, sp)) return;  // no normaliser asked for (false: a part of a shared row that is not the last to arrive)
+__device__ __forceinline__ void dflash_topk_row(const float* x, int n, int k, int* ids, float* vals) {
+    ws::topk_one_row<false>(x, n, k, 1.f, ids, vals, nullptr);  // no normaliser asked for
     __syncthreads();  // the winners are in ids / vals, in id order
     const int kk = k < n ? k : n;
     if (threadIdx.x >= 64) return;
@@ -703,18 +616,9 @@ __device__ __forceinline__ void dflash_topk_row(const float* x, int n, int k, in
 }
 }  // namespace ws
 
+#ifndef WS_NO_NAMED_KERNELS
 extern "C" __global__ void __launch_bounds__(WS_BLOCK) dflash_topk(const float* x, int n, int ld, int k, int* ids, float* vals) {
     const size_t row = blockIdx.x;
-    ws::dflash_topk_row(x + row * ld, n, k, ids + row * k, vals + row * k, ws::TopkSplit{});
+    ws::dflash_topk_row(x + row * ld, n, k, ids + row * k, vals + row * k);
 }
-
-// dflash_topk with every row shared by 1 << split_log2 consecutive workgroups (ws_dflash_topk_ws)
-extern "C" __global__ void __launch_bounds__(WS_BLOCK)
-    dflash_topk_split(const float* x, int n, int ld, int k, int* ids, float* vals, unsigned split_log2, unsigned char* work) {
-    const size_t row = blockIdx.x >> split_log2;
-    ws::TopkSplit sp;
-    sp.parts = 1u << split_log2;
-    sp.part = blockIdx.x & (sp.parts - 1u);
-    sp.work = work + row * ws::kTopkSplitRowBytes;
-    ws::dflash_topk_row(x + row * ld, n, k, ids + row * k, vals + row * k, sp);
-}
+#endif
