@@ -125,3 +125,32 @@ def test_top_lists_at_the_edges_of_a_share(rows, n, K):
         again = m.dflash_topk(x, k, workspace=work)
         assert torch.equal(again[0], first[0]) and torch.equal(again[1], first[1])
     assert not work.any().item()
+
+
+@pytest.mark.parametrize("rows,n", [(1, 8191), (1, 8192), (3, 12289), (32, 50257), (127, 8200), (128, 9001), (129, 8195)])
+def test_greedy_picks_shared_between_workgroups(rows, n):
+    """Vocabularies and row counts either side of the rule that shares a row, ties across its parts, a row of one value, a row
+    of -inf: the lowest index of the largest logit, on the current stream, on others, and twice on each."""
+    m = gc.pkg()
+    rng = np.random.default_rng(n)
+    x = (rng.standard_normal((rows, n)) * 2).astype(np.float32)
+    for r in range(rows):
+        x[r, rng.integers(0, n, 3)] = 50.0
+    x[0], x[rows - 1, :] = 1.5, (-np.inf if rows > 1 else 1.5)
+    x[rows // 2, n - 1] = 60.0 if rows > 2 else x[rows // 2, n - 1]
+    want = x.argmax(axis=1)
+    d = torch.from_numpy(x).cuda()
+    torch.cuda.synchronize()
+    for stream in [torch.cuda.current_stream(), torch.cuda.Stream(), torch.cuda.Stream()]:
+        with torch.cuda.stream(stream):
+            for _ in range(2):
+                got = m.argmax_rows(d)
+                to = torch.full((40,), -7, dtype=torch.int32, device="cuda")
+                if rows <= 32:
+                    m.argmax_rows_to(d, to, list(range(rows, 0, -1)))
+                ids, pos = torch.zeros(1, dtype=torch.int32, device="cuda"), torch.full((1,), 5, dtype=torch.int32, device="cuda")
+                one = m.argmax(d[rows - 1], ids, pos, 2)
+                stream.synchronize()
+                assert np.array_equal(got.cpu().numpy(), want)
+                assert rows > 32 or np.array_equal(to.cpu().numpy()[1:rows + 1][::-1], want)
+                assert one.item() == ids.item() == want[rows - 1] and pos.item() == 7

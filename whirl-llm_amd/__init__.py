@@ -479,9 +479,8 @@ def spec_verify_classic(p, q, draft, seed, step0, rng=RNG_PHILOX, tol=0.0, works
     it as the next needs it), None: one is made for this call when the batch is small enough to split (split=False: never)."""
     n_seq, n_pos, V = p.shape
     dev = p.device
-    out = torch.full((n_seq, n_pos), -1, dtype=torch.int32, device=dev)
-    nacc = torch.empty(n_seq, dtype=torch.int32, device=dev)
-    flags = torch.empty(n_seq, dtype=torch.int32, device=dev)
+    out = torch.empty((n_seq, n_pos), dtype=torch.int32, device=dev)  # (positions past the drawn token: -1, written by the kernel)
+    nacc, flags = torch.empty((2, n_seq), dtype=torch.int32, device=dev).unbind()
     v = SpecVerify(_p(p), _p(q), _p(draft), n_seq, n_pos, V, _p(seed), _p(step0), rng, _p(out), _p(nacc), _p(flags), None, 0,
                    tol)
     if split:

@@ -47,6 +47,8 @@ int launch_dflash_shared(hipStream_t stream, const float* x, int n, int ld, int 
                          unsigned char* work);
 int launch_draft_shared(hipStream_t stream, const float* x, int n, int* ctl_all, const void* area, int r, const int* map, const void* args, int* qbuf,
                         unsigned rows, unsigned parts, unsigned chunk_log2, unsigned char* work);
+int launch_argmax_shared(hipStream_t stream, int mode, const float* x, int n, int* out, const void* dst, int* ids, int* pos, int advance, unsigned rows,
+                         unsigned parts, unsigned long long* scratch);
 int prepare_top();
 }  // namespace ws
 
@@ -287,6 +289,53 @@ int scratch_address(unsigned char** out) {
     return WS_OK;
 }
 
+// Scratch of the greedy picks, whose entry points take no workspace: kPickStreams blocks of it in every GPU's copy of the code
+// object, each given to the first stream that asks and kept by it. Launches on one stream follow one another, so a block is
+// never in two launches at once; the streams beyond the first kPickStreams, the handle that names a stream per thread, and a
+// stream under capture (whose graph may be replayed on another) get none and take the kernels that need none.
+constexpr uint32_t kPickStreams = 64, kPickRows = 128;
+static __device__ __align__(256) unsigned char pick_scratch[kPickStreams * kPickRows * ws::kPickSplitRowBytes];
+std::atomic<unsigned char*> pick_scratch_at[64];
+std::atomic<uintptr_t> pick_owner[64][kPickStreams];  // [device][block]: the stream's handle, 1 for the null stream
+
+unsigned long long* pick_block(void* stream, unsigned rows) {
+    int dev = 0;
+    if (rows > kPickRows || stream == static_cast<void*>(hipStreamPerThread) || hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return nullptr;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(S(stream), &cap) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    if (cap != hipStreamCaptureStatusNone) return nullptr;
+    unsigned char* at = pick_scratch_at[dev].load(std::memory_order_acquire);
+    if (!at) {
+        void* sym = nullptr;
+        if (hipGetSymbolAddress(&sym, HIP_SYMBOL(pick_scratch)) != hipSuccess) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        at = static_cast<unsigned char*>(sym);
+        pick_scratch_at[dev].store(at, std::memory_order_release);
+    }
+    const uintptr_t key = stream ? reinterpret_cast<uintptr_t>(stream) : 1u;
+    const uint32_t first = static_cast<uint32_t>((key >> 4) * 0x9E3779B1u) >> 26;
+    for (uint32_t i = 0; i < kPickStreams; ++i) {
+        const uint32_t b = (first + i) % kPickStreams;
+        uintptr_t owner = pick_owner[dev][b].load(std::memory_order_relaxed);
+        if (owner == 0 && pick_owner[dev][b].compare_exchange_strong(owner, key)) owner = key;
+        if (owner == key) return reinterpret_cast<unsigned long long*>(at + size_t{b} * kPickRows * ws::kPickSplitRowBytes);
+    }
+    return nullptr;
+}
+
+// workgroups a row of a greedy pick: within the compute units, at least 4096 tokens each
+unsigned argmax_parts(int n, unsigned rows) {
+    unsigned parts = rows ? static_cast<unsigned>(compute_units()) / rows : 0u;
+    if (parts > 16u) parts = 16u;
+    if (parts > static_cast<unsigned>(n) / 4096u) parts = static_cast<unsigned>(n) / 4096u;
+    return parts < 2u ? 0u : parts;
+}
+
 // the kernels launched from this file whose dynamic LDS goes beyond the default limit
 int prepare_three_pass() {
     static std::atomic<uint64_t> done{0};
@@ -346,18 +395,24 @@ int ws_probe(void) {
 
 int ws_argmax(void* stream, const float* x, int n, int* out, int* ids, int* pos, int advance) {
     if (!x || !out || !ids || !pos || n <= 0) return WS_E_INVALID;
+    if (const unsigned parts = argmax_parts(n, 1u))
+        if (unsigned long long* scratch = pick_block(stream, 1u)) return ws::launch_argmax_shared(S(stream), 2, x, n, out, nullptr, ids, pos, advance, 1u, parts, scratch);
     hipLaunchKernelGGL(argmax, dim3(1), dim3(WS_BLOCK), 0, S(stream), x, n, out, ids, pos, advance);
     return done();
 }
 
 int ws_argmax_rows(void* stream, const float* x, int n, int* out, unsigned rows) {
     if (!x || !out || n <= 0 || rows == 0) return WS_E_INVALID;
+    if (const unsigned parts = argmax_parts(n, rows))
+        if (unsigned long long* scratch = pick_block(stream, rows)) return ws::launch_argmax_shared(S(stream), 0, x, n, out, nullptr, nullptr, nullptr, 0, rows, parts, scratch);
     hipLaunchKernelGGL(argmax_rows, dim3(rows), dim3(WS_BLOCK), 0, S(stream), x, n, out);
     return done();
 }
 
 int ws_argmax_rows_to(void* stream, const float* x, int n, int* out, const ws_row_idx* dst, unsigned rows) {
     if (!x || !out || !dst || n <= 0 || rows == 0 || rows > WS_MAX_TABLE_ROWS) return WS_E_INVALID;
+    if (const unsigned parts = argmax_parts(n, rows))
+        if (unsigned long long* scratch = pick_block(stream, rows)) return ws::launch_argmax_shared(S(stream), 1, x, n, out, dst, nullptr, nullptr, 0, rows, parts, scratch);
     RowIdx d;
     std::memcpy(&d, dst, sizeof d);
     hipLaunchKernelGGL(argmax_rows_to, dim3(rows), dim3(WS_BLOCK), 0, S(stream), x, n, out, d);
@@ -538,8 +593,12 @@ int ws_sample_batch_workspace_use(const ws_batch* b) {
 
 namespace {
 
+bool split_fits(const BatchPlan& p, const unsigned char* work, uint64_t work_bytes) {
+    return p.workspace_min && work && work_bytes >= p.workspace_min && reinterpret_cast<uintptr_t>(work) % 8u == 0;
+}
+
 int sample_batch_on(void* stream, const ws_batch* b, const BatchPlan& p, unsigned char* work, uint64_t work_bytes) {
-    const bool can_split = p.workspace_min && work && work_bytes >= p.workspace_min && reinterpret_cast<uintptr_t>(work) % 8u == 0;
+    const bool can_split = split_fits(p, work, work_bytes);
     const bool staged = can_split && work_bytes >= p.workspace && p.workspace > p.workspace_min;
     ws::BatchArgs a{};
     a.split_log2 = can_split ? p.split_log2 : 0u;

@@ -161,4 +161,78 @@ __global__ void __launch_bounds__(WS_BLOCK)
 #endif
 }
 
+// ---- greedy picks of few rows: every part leaves the largest {logit, lowest index} of its stretch as an order key (never
+// zero) in the row's 256 bytes of scratch, and the part that arrives last picks among them (a key still on its way reads as zero
+// and is read again) and puts the scratch back to zero. What bounds it: the stretch's loads (76 KB a compute unit at 32 rows of
+// 151936) and three trips to memory; 32 rows took 10.4 us with a compute unit a row.
+struct PickTable {
+    RowIdx dst;  // argmax_rows_to: where each row's pick goes
+};
+template <int MODE>  // 0: out[row]; 1: out[dst.v[row]]; 2: one row, out[0], ids[0] and pos[0] += advance
+__global__ void __launch_bounds__(WS_BLOCK)
+    argmax_shared(const float* x, int n, int* out, PickTable table, int* ids, int* pos, int advance, unsigned parts, unsigned long long* scratch) {
+    __shared__ unsigned long long red[WS_WAVES];
+    __shared__ uint32_t s_ticket;
+    const uint32_t row = blockIdx.y, part = blockIdx.x, t = threadIdx.x, lane = t & 63u, V = static_cast<uint32_t>(n);
+    const unsigned char* base = reinterpret_cast<const unsigned char*>(x + static_cast<size_t>(row) * V);
+    scratch += static_cast<size_t>(row) * (kPickSplitRowBytes / 8u);
+    const uint32_t nv = (V + 3u) / 4u, per = (nv + parts - 1u) / parts, j0 = min(part * per, nv), j1 = min(j0 + per, nv);
+    float best = -INFINITY;
+    uint32_t at = 0xffffffffu;
+    auto take = [&](const uint4& q, uint32_t j) {  // (a last vector that overlaps the one before it offers tokens twice: no harm, but their places count from the row's end)
+        const float v[4] = {fmaxf(__uint_as_float(q.x), -INFINITY), fmaxf(__uint_as_float(q.y), -INFINITY), fmaxf(__uint_as_float(q.z), -INFINITY),
+                            fmaxf(__uint_as_float(q.w), -INFINITY)};
+        const float m = fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3]));
+        if (m > best) {
+            best = m;
+            at = min(4u * j, V - 4u) + (v[0] == m ? 0u : (v[1] == m ? 1u : (v[2] == m ? 2u : 3u)));
+        }
+    };
+    constexpr uint32_t kU = 10u;  // loads of a thread on their way together
+    for (uint32_t jb = j0; jb < j1; jb += kU * WS_BLOCK) {
+        uint4 q[kU];
+#pragma unroll
+        for (uint32_t u = 0; u < kU; ++u) q[u] = row_vector<0>(base, min(jb + u * WS_BLOCK + t, j1 - 1u), V);
+#pragma unroll
+        for (uint32_t u = 0; u < kU; ++u) take(q[u], min(jb + u * WS_BLOCK + t, j1 - 1u));  // (past the stretch: its last vector once more)
+    }
+    auto wave_pick = [&](float v, uint32_t i) {  // the wave's largest, lowest index on ties, as a key
+        const float m = wave_max(v);
+        const uint32_t first = wave_min_u32(v == m ? i : 0xffffffffu);
+        return (static_cast<unsigned long long>(key32(m)) << 32) | (0xffffffffu - first);
+    };
+    const unsigned long long mine = wave_pick(best, at);
+    if (lane == 0u) red[t >> 6] = mine;
+    __syncthreads();
+    auto key_max = [](unsigned long long a, unsigned long long b) { return a > b ? a : b; };
+    if (t == 0) {
+        unsigned long long k = red[0];
+#pragma unroll
+        for (uint32_t w = 1; w < WS_WAVES; ++w) k = key_max(k, red[w]);
+        __hip_atomic_store(&scratch[part], k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        s_ticket = __hip_atomic_fetch_add(reinterpret_cast<uint32_t*>(scratch + 16), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    if (s_ticket != parts - 1u || t >= 64u) return;
+    unsigned long long k = 1ull;
+    for (uint32_t tries = 0; tries < 4096u; ++tries) {
+        k = lane < parts ? __hip_atomic_load(&scratch[lane], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 1ull;
+        if (__ballot(k == 0ull) == 0ull) break;
+    }
+    if (lane < parts) __hip_atomic_store(&scratch[lane], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (lane == 16u) __hip_atomic_store(&scratch[16], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const bool some = lane < parts;
+    const unsigned long long r = wave_pick(some ? unkey32(static_cast<uint32_t>(k >> 32)) : -INFINITY, some ? 0xffffffffu - static_cast<uint32_t>(k) : 0xffffffffu);
+    if (lane == 0u) {
+        const uint32_t i = 0xffffffffu - static_cast<uint32_t>(r);
+        const int id = i == 0xffffffffu ? 0 : static_cast<int>(i);  // (a row without a number: the first index)
+        if (MODE == 1) out[table.dst.v[row]] = id;
+        else out[row] = id;
+        if (MODE == 2) {
+            ids[0] = id;
+            pos[0] += advance;
+        }
+    }
+}
+
 }  // namespace ws

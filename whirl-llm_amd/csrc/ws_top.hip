@@ -65,4 +65,13 @@ int launch_draft_shared(hipStream_t stream, const float* x, int n, int* ctl_all,
     return static_cast<int>(hipGetLastError());
 }
 
+int launch_argmax_shared(hipStream_t stream, int mode, const float* x, int n, int* out, const void* dst, int* ids, int* pos, int advance, unsigned rows,
+                         unsigned parts, unsigned long long* scratch) {
+    PickTable t{};
+    if (mode == 1) __builtin_memcpy(&t.dst, dst, sizeof t.dst);
+    const auto f = mode == 0 ? argmax_shared<0> : (mode == 1 ? argmax_shared<1> : argmax_shared<2>);
+    hipLaunchKernelGGL(f, dim3(parts, rows), dim3(WS_BLOCK), 0, stream, x, n, out, t, ids, pos, advance, parts, scratch);
+    return static_cast<int>(hipGetLastError());
+}
+
 }  // namespace ws
