@@ -60,7 +60,7 @@ public:
     const float* loadFullRow(std::uint32_t gr) override;
     float logitAt(std::uint32_t gr, std::uint32_t t) override;
     std::uint32_t nVocab() const override { return vocab_; }
-    std::uint8_t* inCands() override { return marks_.data(); }
+    std::uint8_t* inCands() override;
     // The device drew a token when it filtered the row (same uniform, same walk: candidates in sorted order, then the
     // rest of the row in id order). It stands for the host's walk when the sampler still is as it was at prepareRow and the
     // device did not flag the draw as close to a boundary.
@@ -74,6 +74,7 @@ private:
     void uploadLists(std::uint32_t n);
     void ensureAdjusted(std::uint32_t gr);
     void filterOnDevice(const Sampler& s, std::uint32_t gr0, std::uint32_t n);
+    void waitForRows(std::uint32_t n);
     struct Dev;    // device scratch
     struct Ready;  // a row filtered on the device, held for its prepareRow
     struct ReadyKey {

@@ -330,6 +330,11 @@ enum {
 };
 int ws_sample_batch_workspace_use(const ws_batch* b);
 int ws_sample_batch(void* stream, const ws_batch* b);
+/* ws_sample_batch for a caller that waits for its results on the host (a decode loop; no counterpart in the reference, whose
+ * caller waits for the stream): the words done[0 .. rows), in memory the device writes in place (hipHostMalloc), are all `value`
+ * once everything the launch writes is visible to the host. Looking at those words costs some 5 us less than a stream wait;
+ * a caller that looks in vain asks the stream (hipStreamQuery) for an error. */
+int ws_sample_batch_notify(void* stream, const ws_batch* b, uint32_t* done, uint32_t value);
 /* ws_sample_batch for callers that cannot allocate device memory - code under HIP graph capture, tight serving loops,
  * harnesses that forbid it; it has no counterpart in the reference. The split rows of a small batch meet in memory that is
  * part of the library's code object on every GPU (WS_STATIC_SPLIT_ROWS rows of it, about 4 MiB, held until the process

@@ -378,7 +378,9 @@ const char* ws_error_string(int code) {
 }
 
 int ws_probe(void) {
-    int n = 0;
+    static std::atomic<uint64_t> ready{0};  // devices this has succeeded on
+    int n = 0, dev = -1;
+    if (hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < 64 && (ready.load(std::memory_order_acquire) >> dev & 1u)) return WS_OK;
     if (hipGetDeviceCount(&n) != hipSuccess || n <= 0) {
         (void)hipGetLastError();
         return WS_E_NO_DEVICE;
@@ -390,7 +392,9 @@ int ws_probe(void) {
     }
     unsigned char* at = nullptr;  // the current device's copy of the static workspace: resolved here, outside any capture
     if (const int e = scratch_address(&at); e != WS_OK) return e;
-    return prepare_all();
+    if (const int e = prepare_all(); e != WS_OK) return e;
+    if (dev >= 0 && dev < 64) ready.fetch_or(uint64_t{1} << dev, std::memory_order_release);
+    return WS_OK;
 }
 
 int ws_argmax(void* stream, const float* x, int n, int* out, int* ids, int* pos, int advance) {
@@ -597,7 +601,9 @@ bool split_fits(const BatchPlan& p, const unsigned char* work, uint64_t work_byt
     return p.workspace_min && work && work_bytes >= p.workspace_min && reinterpret_cast<uintptr_t>(work) % 8u == 0;
 }
 
-int sample_batch_on(void* stream, const ws_batch* b, const BatchPlan& p, unsigned char* work, uint64_t work_bytes) {
+// done: a word per row that gets `value` once the row's results are visible to the host, or nullptr (ws_sample_batch_notify)
+int sample_batch_on(void* stream, const ws_batch* b, const BatchPlan& p, unsigned char* work, uint64_t work_bytes, uint32_t* done_at = nullptr,
+                    uint32_t done_value = 0u) {
     const bool can_split = split_fits(p, work, work_bytes);
     const bool staged = can_split && work_bytes >= p.workspace && p.workspace > p.workspace_min;
     ws::BatchArgs a{};
@@ -649,6 +655,8 @@ int sample_batch_on(void* stream, const ws_batch* b, const BatchPlan& p, unsigne
     a.query_prob = b->query_prob;
     a.entropy = b->entropy;
     if (p.few_parts && can_split) {
+        a.done = done_at;
+        a.done_value = done_value;
         a.few_parts = p.few_parts;
         const uint32_t waves = p.few_parts * 8u;  // (512 threads a workgroup)
         a.few_magic = static_cast<uint32_t>(((uint64_t{1} << 32) + waves - 1u) / waves);
@@ -686,6 +694,18 @@ int ws_sample_batch(void* stream, const ws_batch* b) {
     const BatchPlan p = plan_batch(b);
     if (p.err != WS_OK) return p.err;
     return sample_batch_on(stream, b, p, static_cast<unsigned char*>(b->workspace), b->workspace_bytes);
+}
+
+int ws_sample_batch_notify(void* stream, const ws_batch* b, uint32_t* done, uint32_t value) {
+    if (!done) return WS_E_INVALID;
+    const BatchPlan p = plan_batch(b);
+    if (p.err != WS_OK) return p.err;
+    unsigned char* work = static_cast<unsigned char*>(b->workspace);
+    if (const int e = sample_batch_on(stream, b, p, work, b->workspace_bytes, done, value); e != WS_OK) return e;
+    if (p.few_parts && split_fits(p, work, b->workspace_bytes)) return WS_OK;  // (that kernel writes the words itself)
+    if (!b->rows) return WS_OK;
+    for (uint32_t r = 0; r + 1u < b->rows; ++r) done[r] = value;
+    return static_cast<int>(hipStreamWriteValue32(S(stream), done + b->rows - 1u, value, 0));
 }
 
 int ws_sample_batch_static(void* stream, const ws_batch* b) {

@@ -654,6 +654,11 @@ __global__ void __launch_bounds__(WS_BLOCK) few_batch_kernel(BatchArgs A) {
         if (Ap->kept_ids) three_pass_row<true>(Ap, row);
         else three_pass_row<false>(Ap, row);
     }
+    if (A.done && finisher) {  // a host looks at this word instead of waiting for the stream: everything written for the row first
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (threadIdx.x == 0) __hip_atomic_store(&A.done[row], A.done_value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
 }
 
 }  // namespace ws

@@ -101,6 +101,8 @@ struct BatchArgs {
     uint32_t stage_cap;        // entries of a row's staging area (kSplitStageCap), 0: none
     uint32_t fb_lds_tie;       // the lean and the short-list kernel: lds_tie and lds_ab of the three-pass code they hand rows back to
     uint32_t fb_lds_ab;
+    uint32_t* done;       // ws_few.h: a word per row for a host that waits (or nullptr), and what goes there
+    uint32_t done_value;
     uint32_t few_parts, few_magic, few_chunk_log2;  // ws_few.h: parts a row, 2^32 / waves a row rounded up, log2 of the lanes a chunk
 };
 

@@ -4,9 +4,12 @@
 // No vocabulary-sized work happens here unless the device flags the row.
 // Parameters, penalty lists, results and kept sets live in pinned host memory that the device addresses directly
 // (hipHostMalloc): the host writes the few hundred bytes a row needs, the kernel reads them over the bus, writes what
-// it kept straight back, and no copy command sits before or after the launch - a decode step is one launch and one
-// stream wait. Everything here waits for the stream before it returns, so the host never rewrites a block that a
-// launch still reads.
+// it kept straight back and then a word the host looks at (ws_sample_batch_notify), and no copy command sits before or after
+// the launch - a decode step is one launch and one wait for that word, which comes some 5 us before a stream wait would end.
+// Everything here has waited for what it launched before it returns, so the host never rewrites a block that a launch
+// still reads.
+// Pinned blocks and the sampler's zero-filled workspace outlive the object that asked for them, in a pool of bounded size
+// (a pinned allocation takes longer than ten decode steps): objects made and dropped once a request find them there.
 #include "sampling/device_rows.h"
 
 #include "whirl_sampling_abi.h"
@@ -14,9 +17,11 @@
 #include <hip/hip_runtime_api.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstring>
 #include <limits>
+#include <mutex>
 
 namespace whirl::sampling {
 
@@ -31,6 +36,92 @@ void check(int rc, const char* op) {
 void checkHip(hipError_t e, const char* op) {
     if (e != hipSuccess) throw DeviceError(op, static_cast<int>(e), std::string(op) + ": " + hipGetErrorString(e));
 }
+
+// Blocks of memory between two owners: pinned host memory, or device memory that is all zeros. A block goes back to the
+// runtime when the pool holds kMost of them or kMostBytes. Any thread may call; a block's last user has waited for its launches.
+class BlockPool {
+public:
+    explicit BlockPool(bool pinned) : pinned_(pinned) {}
+    // at least `bytes` on the current device; `got`: how much it is, `fresh`: its contents are anything
+    void* take(std::size_t bytes, std::size_t& got, bool& fresh) {
+        int dev = 0;
+        checkHip(hipGetDevice(&dev), "hipGetDevice");
+        {
+            const std::lock_guard<std::mutex> lock(mutex_);
+            std::size_t best = blocks_.size();
+            for (std::size_t i = 0; i < blocks_.size(); ++i)
+                if (blocks_[i].dev == dev && blocks_[i].bytes >= bytes && blocks_[i].bytes / 4 <= bytes && (best == blocks_.size() || blocks_[i].bytes < blocks_[best].bytes)) best = i;
+            if (best != blocks_.size()) {
+                const Block b = blocks_[best];
+                blocks_.erase(blocks_.begin() + static_cast<std::ptrdiff_t>(best));
+                held_ -= b.bytes;
+                got = b.bytes;
+                fresh = false;
+                return b.at;
+            }
+        }
+        void* p = nullptr;
+        if (pinned_) checkHip(hipHostMalloc(&p, bytes, hipHostMallocDefault), "hipHostMalloc");
+        else checkHip(hipMalloc(&p, bytes), "hipMalloc");
+        got = bytes;
+        fresh = true;
+        return p;
+    }
+    void give(void* p, std::size_t bytes) {
+        if (!p) return;
+        int dev = 0;
+        if (hipGetDevice(&dev) == hipSuccess) {
+            const std::lock_guard<std::mutex> lock(mutex_);
+            if (blocks_.size() < kMost && held_ + bytes <= kMostBytes) {
+                blocks_.push_back({p, bytes, dev});
+                held_ += bytes;
+                return;
+            }
+        }
+        drop(p);
+    }
+    void drop(void* p) {
+        if (p) (void)(pinned_ ? hipHostFree(p) : hipFree(p));
+    }
+
+private:
+    struct Block {
+        void* at;
+        std::size_t bytes;
+        int dev;
+    };
+    static constexpr std::size_t kMost = 16, kMostBytes = std::size_t{8} << 20;
+    bool pinned_;
+    std::mutex mutex_;
+    std::vector<Block> blocks_;
+    std::size_t held_ = 0;
+};
+// (never destroyed: at the end of the process the runtime may be gone before them)
+BlockPool& pinnedPool() {
+    static BlockPool& pool = *new BlockPool(true);
+    return pool;
+}
+BlockPool& zeroPool() {
+    static BlockPool& pool = *new BlockPool(false);
+    return pool;
+}
+
+// a pinned array of one owner
+struct Pinned {
+    unsigned char* at = nullptr;
+    std::size_t bytes = 0;
+    void need(std::size_t want) {
+        if (want <= bytes) return;
+        release();
+        bool fresh;
+        at = static_cast<unsigned char*>(pinnedPool().take(want, bytes, fresh));
+    }
+    void release() {
+        pinnedPool().give(at, bytes);
+        at = nullptr;
+        bytes = 0;
+    }
+};
 
 }  // namespace
 
@@ -75,6 +166,7 @@ struct DeviceRows::Dev {
         float* stats;
     };
     static std::size_t resultBytes(std::uint32_t R) { return std::size_t{R} * 24; }
+    static std::size_t up(std::size_t bytes) { return (bytes + 255u) & ~std::size_t{255}; }
     static ResultView view_res(unsigned char* base, std::uint32_t R) {
         ResultView v;
         v.token = reinterpret_cast<std::int32_t*>(base);
@@ -84,16 +176,19 @@ struct DeviceRows::Dev {
         v.stats = reinterpret_cast<float*>(v.flags + R);
         return v;
     }
-    std::uint32_t row_cap = 0;     // rows the blocks below are sized for
-    // pinned host memory, read and written by the kernels in place
+    std::uint32_t row_cap = 0;     // rows the block below is sized for
+    // pinned host memory, read and written by the kernels in place: parameters, results, arrival words and kept sets in one block
+    Pinned rows_block, hist_block, bias_block, topk_block, row_block;
     unsigned char* prm = nullptr;
     unsigned char* res = nullptr;
+    std::uint32_t* done = nullptr;     // [row_cap]
+    std::uint32_t turn = 0;            // what the last launch writes there
+    bool in_flight = false;            // a launch has not been waited for (an exception came first)
     std::int32_t* kept_ids = nullptr;  // [row_cap][cap]
     float* kept_logits = nullptr;
     std::int32_t* hist = nullptr;      // the history, once per row
     std::int32_t* bias_ids = nullptr;
     float* bias_vals = nullptr;
-    std::size_t hist_cap = 0, bias_cap = 0;
     std::int32_t* topk_ids = nullptr;  // escalation: ids | vals | stats of one row, kBig candidates
     float* topk_vals = nullptr;
     float* topk_stats = nullptr;
@@ -123,18 +218,16 @@ struct DeviceRows::Ready {
 };
 
 DeviceRows::DeviceRows(const float* d_logits, std::uint32_t rows, std::uint32_t n_vocab, void* stream)
-    : logits_(d_logits), rows_(rows), vocab_(n_vocab), stream_(stream), dev_(new Dev), marks_(n_vocab, 0) {
+    : logits_(d_logits), rows_(rows), vocab_(n_vocab), stream_(stream), dev_(new Dev) {
     check(ws_probe(), "ws_probe");
 }
 
 DeviceRows::~DeviceRows() {
-    for (void* p : {static_cast<void*>(dev_->prm), static_cast<void*>(dev_->res), static_cast<void*>(dev_->kept_ids),
-                    static_cast<void*>(dev_->kept_logits), static_cast<void*>(dev_->hist), static_cast<void*>(dev_->bias_ids),
-                    static_cast<void*>(dev_->bias_vals), static_cast<void*>(dev_->topk_ids), static_cast<void*>(dev_->topk_vals),
-                    static_cast<void*>(dev_->topk_stats), static_cast<void*>(dev_->row_host)})
-        if (p) (void)hipHostFree(p);
-    for (void* p : {static_cast<void*>(dev_->adjusted), static_cast<void*>(dev_->work)})
-        if (p) (void)hipFree(p);
+    if (dev_->in_flight) (void)hipStreamSynchronize(static_cast<hipStream_t>(stream_));
+    for (Pinned* p : {&dev_->rows_block, &dev_->hist_block, &dev_->bias_block, &dev_->topk_block, &dev_->row_block}) p->release();
+    if (dev_->adjusted) (void)hipFree(dev_->adjusted);
+    if (dev_->work_dirty || dev_->in_flight) zeroPool().drop(dev_->work);
+    else zeroPool().give(dev_->work, dev_->work_cap);
     delete dev_;
 }
 
@@ -151,12 +244,16 @@ void DeviceRows::newCycle() {
     last_token_ = -1;
 }
 
-namespace {
-template <class T>
-void pinned(T** p, std::size_t bytes) {
-    checkHip(hipHostMalloc(reinterpret_cast<void**>(p), bytes, hipHostMallocDefault), "hipHostMalloc");
+// the candidates' scratch of a sampler, at least n entries (a caller may start with less than a vocabulary's worth)
+static Cand* room(Sampler& s, std::size_t n) {
+    if (s.cands->size() < n) s.cands->resize(n);
+    return s.cands->data();
 }
-}  // namespace
+
+std::uint8_t* DeviceRows::inCands() {
+    if (marks_.size() < vocab_) marks_.resize(vocab_);
+    return marks_.data();
+}
 
 // Parameters of `n` rows that share sampler `s` and the current penalties, and the penalty lists once per row, written
 // where the device reads them (the lists are replicated because a batch addresses them through one ascending offset
@@ -179,37 +276,29 @@ void DeviceRows::uploadLists(std::uint32_t n) {
     Dev& d = *dev_;
     const std::uint32_t cap = std::min(kKeptCap, vocab_);
     if (n > d.row_cap) {
-        for (void* p : {static_cast<void*>(d.prm), static_cast<void*>(d.res), static_cast<void*>(d.kept_ids), static_cast<void*>(d.kept_logits)})
-            if (p) (void)hipHostFree(p);
-        d.prm = d.res = nullptr;
-        d.kept_ids = nullptr;
-        d.kept_logits = nullptr;
+        const std::size_t prm_b = Dev::up(Dev::paramBytes(n)), res_b = Dev::up(Dev::resultBytes(n)), done_b = Dev::up(n * sizeof(std::uint32_t)),
+                          ids_b = Dev::up(std::size_t{n} * cap * sizeof(std::int32_t));
         d.row_cap = 0;
-        pinned(&d.prm, Dev::paramBytes(n));
-        pinned(&d.res, Dev::resultBytes(n));
-        pinned(&d.kept_ids, std::size_t{n} * cap * sizeof(std::int32_t));
-        pinned(&d.kept_logits, std::size_t{n} * cap * sizeof(float));
+        d.rows_block.need(prm_b + res_b + done_b + 2 * ids_b);
+        unsigned char* at = d.rows_block.at;
+        d.prm = at;
+        d.res = at += prm_b;
+        d.done = reinterpret_cast<std::uint32_t*>(at += res_b);
+        d.kept_ids = reinterpret_cast<std::int32_t*>(at += done_b);
+        d.kept_logits = reinterpret_cast<float*>(at + ids_b);
+        std::fill_n(d.done, n, 0u);
+        d.turn = 0;
         d.row_cap = n;
     }
     const std::size_t nh = adj_.n_history, nb = adj_.n_bias;
-    if (nh * n > d.hist_cap) {
-        if (d.hist) (void)hipHostFree(d.hist);
-        d.hist = nullptr;
-        const std::size_t want = std::max(nh * n, 2 * d.hist_cap);
-        d.hist_cap = 0;
-        pinned(&d.hist, want * sizeof(std::int32_t));
-        d.hist_cap = want;
+    if (const std::size_t want = nh * n * sizeof(std::int32_t); want > d.hist_block.bytes) {
+        d.hist_block.need(std::max(want, 2 * d.hist_block.bytes));
+        d.hist = reinterpret_cast<std::int32_t*>(d.hist_block.at);
     }
-    if (nb * n > d.bias_cap) {
-        if (d.bias_ids) (void)hipHostFree(d.bias_ids);
-        if (d.bias_vals) (void)hipHostFree(d.bias_vals);
-        d.bias_ids = nullptr;
-        d.bias_vals = nullptr;
-        const std::size_t want = std::max(nb * n, 2 * d.bias_cap);
-        d.bias_cap = 0;
-        pinned(&d.bias_ids, want * sizeof(std::int32_t));
-        pinned(&d.bias_vals, want * sizeof(float));
-        d.bias_cap = want;
+    if (const std::size_t want = 2 * Dev::up(nb * n * sizeof(float)); nb && want > d.bias_block.bytes) d.bias_block.need(std::max(want, 2 * d.bias_block.bytes));
+    if (nb) {
+        d.bias_ids = reinterpret_cast<std::int32_t*>(d.bias_block.at);
+        d.bias_vals = reinterpret_cast<float*>(d.bias_block.at + Dev::up(nb * n * sizeof(float)));
     }
     for (std::uint32_t r = 0; r < n; ++r) {
         if (nh) std::memcpy(d.hist + r * nh, adj_.history, nh * sizeof(std::int32_t));
@@ -282,12 +371,15 @@ void DeviceRows::filterOnDevice(const Sampler& s, std::uint32_t gr0, std::uint32
     b.top_k_max = (s.top_k >= 1 && s.top_k <= 1024) ? static_cast<std::uint32_t>(s.top_k) : 0u;
     b.min_p_min = (s.top_k == 0 && s.min_p >= 1e-3) ? s.min_p : 0.0;  // (no top-k, but a floor that keeps the set small)
     if (const std::uint64_t need = ws_sample_batch_workspace(&b); need > d.work_cap) {
-        if (d.work) (void)hipFree(d.work);
+        if (d.work_dirty) zeroPool().drop(d.work);
+        else zeroPool().give(d.work, d.work_cap);
         d.work = nullptr;
         d.work_cap = 0;
-        checkHip(hipMalloc(reinterpret_cast<void**>(&d.work), need), "hipMalloc");
-        d.work_cap = need;
-        d.work_dirty = true;  // (fresh memory: whatever it holds)
+        std::size_t got = 0;
+        bool fresh = true;
+        d.work = static_cast<unsigned char*>(zeroPool().take(need, got, fresh));
+        d.work_cap = got;
+        d.work_dirty = fresh;  // (fresh memory: whatever it holds)
     }
     const int use = ws_sample_batch_workspace_use(&b);
     if (use == WS_WORK_MEETING && d.work_dirty) {
@@ -298,9 +390,10 @@ void DeviceRows::filterOnDevice(const Sampler& s, std::uint32_t gr0, std::uint32
     }
     b.workspace = d.work;
     b.workspace_bytes = d.work_cap;
-    check(ws_sample_batch(stream_, &b), "ws_sample_batch");
-
-    checkHip(hipStreamSynchronize(stream), "hipStreamSynchronize");  // results and kept sets are in host memory now
+    d.in_flight = true;
+    check(ws_sample_batch_notify(stream_, &b, d.done, ++d.turn), "ws_sample_batch");
+    waitForRows(n);  // results and kept sets are in host memory now
+    d.in_flight = false;
     const Dev::ResultView& h = o;
     ready_.clear();
     ready_.resize(n);
@@ -321,6 +414,23 @@ void DeviceRows::filterOnDevice(const Sampler& s, std::uint32_t gr0, std::uint32
         q.logits.assign(d.kept_logits + std::size_t{r} * cap, d.kept_logits + std::size_t{r} * cap + q.n_kept);
     }
     ready_key_ = {s.inv_t, s.top_k, s.top_p, s.min_p};
+}
+
+// Looks at the rows' words until all of them have come; now and then the stream is asked as well, which knows of errors.
+void DeviceRows::waitForRows(std::uint32_t n) {
+    Dev& d = *dev_;
+    for (std::uint32_t r = 0, looks = 0; r < n;) {
+        if (std::atomic_ref<std::uint32_t>(d.done[r]).load(std::memory_order_acquire) == d.turn) {
+            ++r;
+            continue;
+        }
+        __builtin_ia32_pause();
+        if (++looks % 16384u == 0) {
+            const hipError_t e = hipStreamQuery(static_cast<hipStream_t>(stream_));
+            if (e == hipSuccess) return;  // everything is done
+            if (e != hipErrorNotReady) checkHip(e, "hipStreamQuery");
+        }
+    }
 }
 
 void DeviceRows::prefetchRows(const Sampler& s, std::uint32_t r0, std::uint32_t n) { filterOnDevice(s, s.row_base + r0, n); }
@@ -356,7 +466,7 @@ void DeviceRows::prepareRow(Sampler& s, std::uint32_t r) {
     const std::uint32_t n = q->n_kept;
     s.m = q->m;
     s.sum = q->sum;
-    Cand* c = s.cands->data();
+    Cand* c = room(s, n);
     if (q->flags & WS_FLAG_OPEN) {
         // No filter at all: the device's list is the engine's short candidate list (the 256 largest logits, lowest ids among
         // equals), the first step of the reference's route (src/server/engine_sampling.cpp:51-66) without a launch of its
@@ -411,6 +521,7 @@ void DeviceRows::ensureAdjusted(std::uint32_t gr) {
     }
     a.out = d.adjusted;
     a.out_stride = vocab_;
+    d.in_flight = true;
     check(ws_adjust_rows(stream_, &a), "ws_adjust_rows");
     adjusted_row_ = gr;
 }
@@ -427,16 +538,19 @@ void DeviceRows::escalate(Sampler& s, std::uint32_t gr) {
         src = d.adjusted;
     }
     if (!d.topk_ids) {
-        pinned(&d.topk_ids, kBig * sizeof(std::int32_t));
-        pinned(&d.topk_vals, kBig * sizeof(float));
-        pinned(&d.topk_stats, 2 * sizeof(float));
+        d.topk_block.need(kBig * 8 + 256);
+        d.topk_ids = reinterpret_cast<std::int32_t*>(d.topk_block.at);
+        d.topk_vals = reinterpret_cast<float*>(d.topk_block.at + kBig * 4);
+        d.topk_stats = reinterpret_cast<float*>(d.topk_block.at + kBig * 8);
     }
-    Cand* c = s.cands->data();
+    Cand* c = room(s, std::min(kBig, vocab_));
     bool first = true;
     for (std::uint32_t k : {std::min(kSmall, vocab_), std::min(kBig, vocab_)}) {
+        d.in_flight = true;
         check(ws_topk_rows(stream_, src, static_cast<int>(vocab_), static_cast<int>(k), s.inv_t, d.topk_ids, d.topk_vals, d.topk_stats, 1),
               "ws_topk_rows");
         checkHip(hipStreamSynchronize(stream), "hipStreamSynchronize");  // the kernel wrote the list into host memory
+        d.in_flight = false;
         if (first) {  // the row's maximum and normaliser, once (the second call recomputes the same values)
             s.m = d.topk_stats[0];
             s.sum = d.topk_stats[1];
@@ -449,6 +563,7 @@ void DeviceRows::escalate(Sampler& s, std::uint32_t gr) {
     }
     s.full_used += 1;
     const float* x = loadFullRow(gr);
+    c = room(s, vocab_);
     for (std::uint32_t j = 0; j < vocab_; ++j) c[j] = {j, x[j], 0.0};
     filterCands(s, vocab_, true);
 }
@@ -462,13 +577,18 @@ bool DeviceRows::drawnToken(const Sampler& s, std::uint32_t& token) {
 
 const float* DeviceRows::loadFullRow(std::uint32_t gr) {
     if (gr >= rows_) throw DeviceError("loadFullRow", WS_E_INVALID, "loadFullRow: row out of range");
-    if (!dev_->row_host) pinned(&dev_->row_host, vocab_ * sizeof(float));
+    if (!dev_->row_host) {
+        dev_->row_block.need(vocab_ * sizeof(float));
+        dev_->row_host = reinterpret_cast<float*>(dev_->row_block.at);
+    }
     auto stream = static_cast<hipStream_t>(stream_);
     const bool penalised = adj_.n_history || adj_.n_bias;
     if (penalised) ensureAdjusted(gr);
     const float* src = penalised ? dev_->adjusted : logits_ + static_cast<std::size_t>(gr) * vocab_;
+    dev_->in_flight = true;
     checkHip(hipMemcpyAsync(dev_->row_host, src, vocab_ * sizeof(float), hipMemcpyDeviceToHost, stream), "hipMemcpyAsync");
     checkHip(hipStreamSynchronize(stream), "hipStreamSynchronize");
+    dev_->in_flight = false;
     return dev_->row_host;
 }
 
@@ -481,6 +601,7 @@ float DeviceRows::logitAt(std::uint32_t gr, std::uint32_t t) {
     const float* src = penalised ? dev_->adjusted : logits_ + static_cast<std::size_t>(gr) * vocab_;
     checkHip(hipMemcpyAsync(&v, src + t, sizeof v, hipMemcpyDeviceToHost, stream), "hipMemcpyAsync");
     checkHip(hipStreamSynchronize(stream), "hipStreamSynchronize");
+    dev_->in_flight = false;
     return v;
 }
 

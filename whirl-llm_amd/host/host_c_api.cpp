@@ -190,7 +190,7 @@ int wsh_decode_steps(void* stream, wsh_steps* a) {
     g_err[0] = 0;
     try {
         ws::DeviceRows src(a->d_logits, 1, a->vocab, stream);
-        std::vector<ws::Cand> scratch(a->vocab > 16384u ? a->vocab : 16384u);
+        std::vector<ws::Cand> scratch(1024);  // (DeviceRows makes room for what it keeps)
         ws::Sampler s;
         s.inv_t = a->inv_t;
         s.temp = 1.0 / s.inv_t;
