@@ -137,3 +137,22 @@ def test_a_top_k_of_the_vocabulary_size_or_beyond_closes_the_row(mode, V):
     fl = smp.flags.cpu().numpy()
     assert not (fl[[0, 1, 2, 4, 5]] & gc.pkg().FLAG_OPEN).any() and (fl[3] & gc.pkg().FLAG_OPEN)
     assert smp.n_kept.cpu().numpy()[:3].tolist() == [V, V, V]
+
+
+@pytest.mark.parametrize("V", [6, 4097, 70001, 151936])
+def test_thousands_of_ties_at_the_cut_and_the_draw(V):
+    """More equal logits in the cut's bin than the walk has room for (they are divided by id), fewer than that, a top-k that
+    reaches the masked-out tokens, cuts at the first and the last token; vocabularies off and on every vector boundary."""
+    c, rng = _base(8, V, n_hist=min(64, V // 2), seed=4)
+    c["name"] = f"ties at {V}"
+    levels = np.array([-3.0, -2.0, -1.5, -1.0, 0.0, 1.0], np.float32)
+    c["dtype"] = "bf16"
+    c["logits"] = gc.f32_to_bf16_bits(levels[rng.choice(6, size=(8, V), p=[0.2, 0.25, 0.25, 0.15, 0.1, 0.05])])
+    allow = rng.random((8, (V + 31) // 32 * 32)) < 0.7
+    allow[:, 0] = True
+    c["allow"] = np.ascontiguousarray(np.packbits(allow, axis=1, bitorder="little").view(np.uint32))
+    c["top_p"][:] = [0.95, 0.6, 1.0, 0.9, 0.99999, 0.99, 1.0, 1e-9]
+    c["top_k"][:] = [0, 0, max(1, V - 2), V // 2, 0, 0, 0, 0]
+    c["min_p"][5:7] = [0.1, 0.05]
+    res, _ = run_case(c, 1, max_differ=2)  # (cuts between equal masses lie within the rounding of a sum)
+    assert res["exact"] >= 6, res

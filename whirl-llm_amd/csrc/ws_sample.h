@@ -1220,146 +1220,331 @@ struct ExactOut {
     double Zk, ptok, mg_top_p, mg_min_p, mg_draw, list_mass, target;
 };
 
+// The row as the exact path reads it: eight tokens a thread and load, two such loads in flight. Its functions are inlined into
+// two of their own (exact_row, exact_walk), whose LDS is named and whose row is a pointer to global memory: as closures handed
+// from one to the other both went through generic addresses, and a pass over 151936 tokens took some 500 us.
+struct ExactRow {
+    typedef const __attribute__((address_space(1))) unsigned char* Bytes;
+    typedef uint32_t Loose __attribute__((ext_vector_type(4), aligned(2)));  // (rows start at any element)
+    Bytes base, allow;
+    uint32_t V, touched_at;
+    int dtype;
+    float m, inv_t, c64;
+    __device__ __forceinline__ explicit ExactRow(const ExactIn& in)
+        : base((Bytes)in.base), allow((Bytes)in.allow), V(in.V), touched_at(in.touched_at), dtype(in.dtype), m(in.m), inv_t(in.inv_t), c64(__fmul_rn(in.inv_t, 64.f)) {}
+    template <class F>
+    __device__ __forceinline__ void each_token(F&& f) const {  // every token with its adjusted logit
+        extern __shared__ __align__(16) unsigned char lds[];
+        const uint32_t t = threadIdx.x, nW = (V + 31u) >> 5;
+        const bool any = touched_at != 0xffffffffu;
+        const uint32_t at0 = any ? touched_at : 0u;
+        const uint32_t* touched = reinterpret_cast<const uint32_t*>(lds + at0);
+        const uint16_t* wprefix = reinterpret_cast<const uint16_t*>(lds + at0 + nW * 4u);
+        const float* pv = reinterpret_cast<const float*>(lds + at0 + nW * 4u + ((nW * 2u + 15u) & ~15u));
+        constexpr uint32_t kU = 2u;
+#pragma unroll 1
+        for (uint32_t i0 = 0; i0 < V; i0 += kU * 8u * WS_BLOCK) {
+            uint32_t b[kU][8], al[kU];
+#pragma unroll
+            for (uint32_t q = 0; q < kU; ++q) {
+                const uint32_t i = i0 + (q * WS_BLOCK + t) * 8u;
+                al[q] = allow ? *(const __attribute__((address_space(1))) uint32_t*)(allow + (min(i, V - 1u) >> 5) * 4u) : 0xffffffffu;
+                if (i + 8u <= V) {
+                    if (dtype == 0) {
+                        const Loose lo = *(const __attribute__((address_space(1))) Loose*)(base + size_t{i} * 4u), hi = *(const __attribute__((address_space(1))) Loose*)(base + size_t{i} * 4u + 16u);
+#pragma unroll
+                        for (uint32_t e = 0; e < 4u; ++e) {
+                            b[q][e] = lo[e];
+                            b[q][4u + e] = hi[e];
+                        }
+                    } else {
+                        const Loose lo = *(const __attribute__((address_space(1))) Loose*)(base + size_t{i} * 2u);
+#pragma unroll
+                        for (uint32_t e = 0; e < 4u; ++e) {
+                            b[q][2u * e] = lo[e] << 16;
+                            b[q][2u * e + 1u] = lo[e] & 0xffff0000u;
+                        }
+                    }
+                } else {  // the row's end
+#pragma unroll
+                    for (uint32_t e = 0; e < 8u; ++e) {
+                        const uint32_t j = min(i + e, V - 1u);
+                        b[q][e] = dtype == 0 ? *(const __attribute__((address_space(1))) uint32_t*)(base + size_t{j} * 4u)
+                                             : static_cast<uint32_t>(*(const __attribute__((address_space(1))) uint16_t*)(base + size_t{j} * 2u)) << 16;
+                    }
+                }
+            }
+#pragma unroll
+            for (uint32_t q = 0; q < kU; ++q) {
+                const uint32_t i = i0 + (q * WS_BLOCK + t) * 8u, w = min(i, V - 1u) >> 5, bit = i & 31u;  // (the eight share a word)
+                const uint32_t to = any ? touched[w] : 0u;
+#pragma unroll
+                for (uint32_t e = 0; e < 8u; ++e) {
+                    if (i + e >= V) continue;
+                    float x = (al[q] >> (bit + e)) & 1u ? fmaxf(__uint_as_float(b[q][e]), -INFINITY) : -INFINITY;
+                    if ((to >> (bit + e)) & 1u) x = pv[wprefix[w] + __popc(to & ((1u << (bit + e)) - 1u))];
+                    f(i + e, x);
+                }
+            }
+        }
+    }
+    __device__ __forceinline__ double e_of(float x) const { return exp(-(static_cast<double>(__fsub_rn(m, x)) * static_cast<double>(inv_t))); }
+    __device__ __forceinline__ uint32_t bin_at(float x) const {  // grows as x falls
+        return static_cast<uint32_t>(__builtin_fminf(__fmul_rn(__fsub_rn(m, x), c64), static_cast<float>(kTail)));
+    }
+    __device__ __forceinline__ uint64_t fx_of(float x) const {  // its mass in units of 2^-43
+        if (bin_at(x) >= 2048u) return 0ull;  // (below e^-31.9: less than half a unit)
+        return static_cast<uint64_t>(__double2ll_rn(e_of(x) * 8796093022208.0));
+    }
+};
+// LDS of the exact path: the row's tokens by distance to its maximum, 64 bins an exponent unit, bin kTail: all further ones (hm
+// masses, hc counts, as prefixes); and the same of one interval of keys (rm, rc), or the keys of an interval themselves (gk, gf)
+constexpr uint32_t kExactRoom = 1024u, kExactHc = 32768u, kExactRm = 49152u, kExactRc = 57344u;
+struct Walk {
+    uint64_t key, before_m, own_m;
+    uint32_t before_c, found;
+};
+// The first key, in descending order, at which the running total - counts (by_mass 0) or masses - reaches `want`;
+// before_c / before_m: what ranks before it. found 0: the whole row, of mass `total`, stays below `want`.
+// The bin is read off the prefixes. Inside it a token is K, its order key without the id's twelve idle bits: while the bin, or
+// what is left of it, has more tokens than LDS has room for, a pass finds the span of their keys and a pass divides it by 1024
+// (thousands of equal logits: the span is one of ids); then a pass lists them and every key is compared with every other.
+// Radix passes over all of the row from the top of the key - up to six a question, an exp of every token in each, and nearly
+// all tokens meeting in a few words of the first - took 7.2 ms
+// a launch with such rows (151936 bf16 tokens, Zipfian, top-p 0.9 and up); now 1.0 ms.
+__device__ __noinline__ Walk exact_walk(const ExactIn in, const uint64_t total, const uint32_t by_mass, const uint64_t want) {
+    extern __shared__ __align__(16) unsigned char lds[];
+    // its few words lie behind the last bin's prefix (static LDS of its own would come off what a batch may ask for)
+    static_assert(kTail + 8 + 6 + 16 + 8 + 1 <= kBins && WS_WAVES <= 16, "room behind the prefixes");
+    uint64_t* const behind = reinterpret_cast<uint64_t*>(lds) + kTail + 8;
+    unsigned long long* const x_w = reinterpret_cast<unsigned long long*>(behind);
+    uint64_t* const red_w = behind + 6;
+    uint32_t* const x_red_u = reinterpret_cast<uint32_t*>(behind + 22);
+    uint32_t& x_first = *reinterpret_cast<uint32_t*>(behind + 30);
+    constexpr uint32_t kRoom = kExactRoom;
+    const uint64_t* const hm = reinterpret_cast<const uint64_t*>(lds);
+    const uint32_t* const hc = reinterpret_cast<const uint32_t*>(lds + kExactHc);
+    uint64_t* const rm = reinterpret_cast<uint64_t*>(lds + kExactRm);
+    uint32_t* const rc = reinterpret_cast<uint32_t*>(lds + kExactRc);
+    uint64_t* const gk = rm;
+    uint64_t* const gf = reinterpret_cast<uint64_t*>(lds + kExactRc);
+    const ExactRow R(in);
+    const uint32_t t = threadIdx.x, V = in.V;
+    auto short_key = [](float x, uint32_t i) { return (static_cast<uint64_t>(key32(x)) << 20) | (0xfffffu - i); };
+            if (t == 0) x_first = 0xffffffffu;
+            __syncthreads();
+            auto end_c = [&](uint32_t d) { return d < static_cast<uint32_t>(kTail) ? hc[d + 1u] : V; };
+            for (uint32_t d = t; d <= static_cast<uint32_t>(kTail); d += WS_BLOCK)
+                if (end_c(d) > hc[d] && (by_mass ? hm[d + 1u] >= want : static_cast<uint64_t>(end_c(d)) >= want)) {
+                    atomicMin(&x_first, d);
+                    break;
+                }
+            __syncthreads();
+            const uint32_t bin = x_first;
+            if (bin == 0xffffffffu) return Walk{0ull, total, 0ull, V, 0u};
+            uint64_t base_m = hm[bin];
+            uint32_t base_c = hc[bin], n_in = end_c(bin) - base_c;
+            uint64_t lo = 0ull, hi = ~0ull;
+            auto each_inside = [&](auto&& f) __attribute__((always_inline)) {
+                R.each_token([&](uint32_t i, float x) __attribute__((always_inline)) {
+                    if (R.bin_at(x) != bin) return;
+                    const uint64_t k = short_key(x, i);
+                    if (k >= lo && k <= hi) f(k, x);
+                });
+            };
+            while (n_in > kRoom) {
+                __syncthreads();
+                if (t == 0) {
+                    x_w[0] = ~0ull;
+                    x_w[1] = 0ull;
+                    x_first = 0xffffffffu;
+                }
+                for (uint32_t d = t; d < kRoom; d += WS_BLOCK) {
+                    rm[d] = 0ull;
+                    rc[d] = 0u;
+                }
+                uint64_t mn = ~0ull, mx = 0ull;
+                each_inside([&](uint64_t k, float) __attribute__((always_inline)) {
+                    mn = k < mn ? k : mn;
+                    mx = k > mx ? k : mx;
+                });
+                __syncthreads();
+                if (mx) {
+                    atomicMin(&x_w[0], static_cast<unsigned long long>(mn));
+                    atomicMax(&x_w[1], static_cast<unsigned long long>(mx));
+                }
+                __syncthreads();
+                lo = x_w[0];
+                hi = x_w[1];
+                const int width = 64 - __clzll(static_cast<long long>(hi - lo));  // (more than kRoom different keys: hi > lo)
+                const uint32_t shift = width > 10 ? static_cast<uint32_t>(width - 10) : 0u;
+                each_inside([&](uint64_t k, float x) __attribute__((always_inline)) {
+                    const uint32_t d = static_cast<uint32_t>((hi - k) >> shift);
+                    atomicAdd(&rc[d], 1u);
+                    const uint64_t fx = R.fx_of(x);
+                    if (fx) atomicAdd(reinterpret_cast<unsigned long long*>(&rm[d]), static_cast<unsigned long long>(fx));
+                });
+                __syncthreads();
+                constexpr uint32_t kPer = kRoom / WS_BLOCK;
+                uint64_t lm[kPer], sm = 0, tot_m;
+                uint32_t lc[kPer], sc = 0, tot_c;
+    #pragma unroll
+                for (uint32_t q = 0; q < kPer; ++q) {
+                    lm[q] = rm[kPer * t + q];
+                    lc[q] = rc[kPer * t + q];
+                    sm += lm[q];
+                    sc += lc[q];
+                }
+                uint64_t run_m = base_m + block_excl_scan(sm, red_w, &tot_m);
+                uint32_t run_c = base_c + block_excl_scan(sc, x_red_u, &tot_c);
+                uint32_t at = 0xffffffffu, at_c = 0, own_c = 0;
+                uint64_t at_m = 0;
+    #pragma unroll
+                for (uint32_t q = 0; q < kPer; ++q) {
+                    const bool reached = by_mass ? run_m + lm[q] >= want : static_cast<uint64_t>(run_c + lc[q]) >= want;
+                    if (at == 0xffffffffu && lc[q] != 0u && reached) {
+                        at = kPer * t + q;
+                        at_m = run_m;
+                        at_c = run_c;
+                        own_c = lc[q];
+                    }
+                    run_m += lm[q];
+                    run_c += lc[q];
+                }
+                if (at != 0xffffffffu) atomicMin(&x_first, at);
+                __syncthreads();
+                const uint32_t first = x_first;
+                if (first == 0xffffffffu) return Walk{0ull, total, 0ull, V, 0u};  // (the prefixes say otherwise: not reached)
+                if (at == first) {
+                    x_w[2] = at_m;
+                    x_w[3] = at_c;
+                    x_w[4] = own_c;
+                }
+                __syncthreads();
+                base_m = x_w[2];
+                base_c = static_cast<uint32_t>(x_w[3]);
+                n_in = static_cast<uint32_t>(x_w[4]);
+                hi -= static_cast<uint64_t>(first) << shift;
+                const uint64_t below = (uint64_t{1} << shift) - 1ull;
+                lo = hi - lo > below ? hi - below : lo;
+            }
+            __syncthreads();
+            if (t == 0) {
+                x_first = 0u;
+                x_w[0] = 0ull;
+            }
+            __syncthreads();
+            each_inside([&](uint64_t k, float x) __attribute__((always_inline)) {
+                const uint32_t slot = atomicAdd(&x_first, 1u);
+                if (slot < kRoom) {
+                    gk[slot] = k;
+                    gf[slot] = R.fx_of(x);
+                }
+            });
+            __syncthreads();
+            const uint32_t n = min(x_first, kRoom);
+            constexpr uint32_t kOwn = kRoom / WS_BLOCK;
+            uint64_t own_k[kOwn], cum[kOwn];
+            uint32_t upto[kOwn];
+    #pragma unroll
+            for (uint32_t q = 0; q < kOwn; ++q) {
+                own_k[q] = q * WS_BLOCK + t < n ? gk[q * WS_BLOCK + t] : ~0ull;
+                cum[q] = base_m;
+                upto[q] = base_c;
+            }
+            for (uint32_t j = 0; j < n; ++j) {
+                const uint64_t kj = gk[j], fj = gf[j];
+    #pragma unroll
+                for (uint32_t q = 0; q < kOwn; ++q) {
+                    cum[q] += kj >= own_k[q] ? fj : 0ull;
+                    upto[q] += kj >= own_k[q] ? 1u : 0u;
+                }
+            }
+    #pragma unroll
+            for (uint32_t q = 0; q < kOwn; ++q)
+                if (q * WS_BLOCK + t < n && (by_mass ? cum[q] >= want : static_cast<uint64_t>(upto[q]) >= want))
+                    atomicMax(&x_w[0], static_cast<unsigned long long>(own_k[q]));
+            __syncthreads();
+            const uint64_t k = x_w[0];
+    #pragma unroll
+            for (uint32_t q = 0; q < kOwn; ++q)
+                if (own_k[q] == k) {
+                    const uint64_t f = gf[q * WS_BLOCK + t];
+                    x_w[1] = cum[q] - f;
+                    x_w[2] = upto[q] - 1u;
+                    x_w[3] = f;
+                }
+            __syncthreads();
+            const Walk w{(k >> 20 << 32) | (0xfff00000u | static_cast<uint32_t>(k & 0xfffffu)), x_w[1], x_w[3], static_cast<uint32_t>(x_w[2]), k != 0ull};
+    __syncthreads();  // (the caller may call again)
+    return w;
+}
+
 __device__ __noinline__ ExactOut exact_row(const ExactIn in) {
     extern __shared__ __align__(16) unsigned char lds[];
     __shared__ unsigned long long x_w[6];
     __shared__ unsigned long long x_red_q[WS_WAVES];
     __shared__ double x_red_d[WS_WAVES];
     __shared__ uint32_t x_red_u[WS_WAVES];
-    __shared__ uint32_t x_first;
     const uint32_t t = threadIdx.x, V = in.V;
-    const float m = in.m, inv_t = in.inv_t;
     const bool prefix_mode = in.mode & 1u, open_row = in.mode & 2u, use_top_p = in.mode & 4u, use_min_p = in.mode & 8u, race = in.mode & 16u;
-    RowView rv;
-    rv.base = in.base;
-    rv.V = V;
-    rv.dtype = in.dtype;
-    rv.vec = false;
-    rv.allow = in.allow;
-    const uint32_t nW = (V + 31u) >> 5;
-    rv.touched = in.touched_at != 0xffffffffu ? reinterpret_cast<const uint32_t*>(lds + in.touched_at) : nullptr;
-    rv.wprefix = reinterpret_cast<const uint16_t*>(lds + (in.touched_at != 0xffffffffu ? in.touched_at : 0u) + nW * 4u);
-    rv.pv = reinterpret_cast<const float*>(lds + (in.touched_at != 0xffffffffu ? in.touched_at : 0u) + nW * 4u + ((nW * 2u + 15u) & ~15u));
+    const ExactRow R(in);
     constexpr double kFx = 8796093022208.0;  // 2^43
-    uint64_t* hm = reinterpret_cast<uint64_t*>(lds);          // masses per digit
-    uint32_t* hc = reinterpret_cast<uint32_t*>(lds + 32768);  // counts per digit
-    uint64_t* red_w = reinterpret_cast<uint64_t*>(x_red_q);
+    uint64_t* const hm = reinterpret_cast<uint64_t*>(lds);
+    uint32_t* const hc = reinterpret_cast<uint32_t*>(lds + kExactHc);
+    uint64_t* const red_w = reinterpret_cast<uint64_t*>(x_red_q);
     ExactOut out{};
     out.mg_top_p = out.mg_min_p = out.mg_draw = 1.0;
-
-    auto each_token = [&](auto&& f) {  // every token with its adjusted logit, four loads in flight per thread
-        for (uint32_t i0 = 0; i0 < V; i0 += 4u * WS_BLOCK) {
-            float xr[4];
-#pragma unroll
-            for (uint32_t q = 0; q < 4u; ++q) xr[q] = raw_logit(rv, min(i0 + q * WS_BLOCK + t, V - 1u));
-#pragma unroll
-            for (uint32_t q = 0; q < 4u; ++q) {
-                const uint32_t i = i0 + q * WS_BLOCK + t;
-                if (i < V) f(i, is_touched(rv, i) ? rv.pv[rank_of(rv, i)] : (is_allowed(rv, i) ? xr[q] : -INFINITY));
-            }
-        }
-    };
-    auto e_of = [&](float x) { return exp(-(static_cast<double>(__fsub_rn(m, x)) * static_cast<double>(inv_t))); };
-    auto fx_of = [&](float x) -> uint64_t {
-        const double e = e_of(x);
-        return e > 0.0 ? static_cast<uint64_t>(__double2ll_rn(e * kFx)) : 0ull;
-    };
+    auto each_token = [&](auto&& f) __attribute__((always_inline)) { R.each_token(f); };
+    auto e_of = [&](float x) __attribute__((always_inline)) { return R.e_of(x); };
+    auto fx_of = [&](float x) __attribute__((always_inline)) { return R.fx_of(x); };
     auto id_of = [](uint64_t key) { return static_cast<int32_t>(0xffffffffu - static_cast<uint32_t>(key)); };
     auto x_of = [](uint64_t key) { return unkey32(static_cast<uint32_t>(key >> 32)); };
-    // The first key, in descending order, at which the running total - counts (by_mass false) or masses - reaches
-    // `want`; before_c / before_m: what ranks before it. found false: the whole row stays below `want`.
-    struct Walk {
-        bool found;
-        uint64_t key, before_m;
-        uint32_t before_c;
-        uint64_t own_m;
-    };
-    auto walk = [&](bool by_mass, uint64_t want) -> Walk {
-        uint64_t prefix = 0, base_m = 0;
-        uint32_t base_c = 0;
-        int hi = 64;  // bits [hi, 64) of the key are fixed to `prefix`
-        for (;;) {
-            const int width = hi >= 12 ? 12 : hi, lo = hi - width;
-            const uint32_t nd = 1u << width;
-            for (uint32_t d = t; d < nd; d += WS_BLOCK) {
-                hm[d] = 0ull;
-                hc[d] = 0u;
-            }
-            if (t == 0) x_first = 0xffffffffu;
-            __syncthreads();
-            each_token([&](uint32_t i, float x) {
-                const uint64_t k = key64(x, i);
-                if (hi == 64 || (k >> (hi & 63)) == prefix) {
-                    const uint32_t d = static_cast<uint32_t>(k >> lo) & (nd - 1u);
-                    atomicAdd(&hc[d], 1u);
-                    const uint64_t fx = fx_of(x);
-                    if (fx) atomicAdd(reinterpret_cast<unsigned long long*>(&hm[d]), static_cast<unsigned long long>(fx));
-                }
-            });
-            __syncthreads();
-            // digits from the largest down: thread t holds places 8 t .. 8 t + 7 of that order
-            uint64_t lm[8], sm = 0;
-            uint32_t lc[8], sc = 0;
-#pragma unroll
-            for (uint32_t q = 0; q < 8u; ++q) {
-                const uint32_t j = 8u * t + q;
-                const bool valid = j < nd;
-                const uint32_t d = valid ? nd - 1u - j : 0u;
-                lm[q] = valid ? hm[d] : 0ull;
-                lc[q] = valid ? hc[d] : 0u;
-                sm += lm[q];
-                sc += lc[q];
-            }
-            uint64_t tot_m;
-            uint32_t tot_c;
-            uint64_t rm = base_m + block_excl_scan(sm, red_w, &tot_m);
-            uint32_t rc = base_c + block_excl_scan(sc, x_red_u, &tot_c);
-            uint32_t at = 0xffffffffu, bc = 0, oc = 0;
-            uint64_t bm = 0, om = 0;
-#pragma unroll
-            for (uint32_t q = 0; q < 8u; ++q) {
-                const bool reached = by_mass ? rm + lm[q] >= want : static_cast<uint64_t>(rc + lc[q]) >= want;
-                if (at == 0xffffffffu && lc[q] != 0u && reached) {
-                    at = 8u * t + q;
-                    bm = rm;
-                    bc = rc;
-                    om = lm[q];
-                    oc = lc[q];
-                }
-                rm += lm[q];
-                rc += lc[q];
-            }
-            if (at != 0xffffffffu) atomicMin(&x_first, at);
-            __syncthreads();
-            const uint32_t first = x_first;
-            if (first == 0xffffffffu) return Walk{false, 0ull, base_m + tot_m, base_c + tot_c, 0ull};  // at the first level only
-            if (at == first) {
-                x_w[0] = bm;
-                x_w[1] = bc;
-                x_w[2] = om;
-                x_w[3] = oc;
-            }
-            __syncthreads();
-            base_m = x_w[0];
-            base_c = static_cast<uint32_t>(x_w[1]);
-            const uint64_t own_m = x_w[2];
-            const uint32_t own_c = static_cast<uint32_t>(x_w[3]);
-            const uint64_t d = nd - 1u - first;
-            prefix = hi == 64 ? d : ((prefix << width) | d);
-            hi = lo;
-            if (hi == 0) return Walk{true, prefix, base_m, base_c, own_m};
-            if (own_c == 1u) {  // one key is left under the prefix: one pass finds it
-                each_token([&](uint32_t i, float x) {
-                    const uint64_t k = key64(x, i);
-                    if ((k >> hi) == prefix) x_w[4] = k;
-                });
-                __syncthreads();
-                const uint64_t key = x_w[4];
-                __syncthreads();
-                return Walk{true, key, base_m, base_c, own_m};
-            }
+
+    // ---- one pass with everybody's mass: the bins, the total, and the first key in sorted order
+    for (uint32_t d = t; d < kBins; d += WS_BLOCK) {
+        hm[d] = 0ull;
+        hc[d] = 0u;
+    }
+    if (t == 0) x_w[5] = 0ull;
+    __syncthreads();
+    uint64_t k_own = 0;
+    each_token([&](uint32_t i, float x) __attribute__((always_inline)) {
+        const uint64_t k = key64(x, i);
+        k_own = k > k_own ? k : k_own;
+        const uint32_t d = R.bin_at(x);
+        if (d < static_cast<uint32_t>(kTail)) {  // (the tail's tokens are those that are left: masked-out ones by the hundred thousand)
+            atomicAdd(&hc[d], 1u);
+            const uint64_t fx = fx_of(x);
+            if (fx) atomicAdd(reinterpret_cast<unsigned long long*>(&hm[d]), static_cast<unsigned long long>(fx));
         }
-    };
+    });
+    atomicMax(&x_w[5], static_cast<unsigned long long>(k_own));
+    __syncthreads();
+    const uint64_t k_top = x_w[5];
+    uint64_t Zfx;
+    {
+        constexpr uint32_t kPer = kBins / WS_BLOCK;
+        uint64_t sm = 0;
+        uint32_t sc = 0, total_c;
+        for (uint32_t q = 0; q < kPer; ++q) {
+            sm += hm[t * kPer + q];
+            sc += hc[t * kPer + q];
+        }
+        sm = block_excl_scan(sm, red_w, &Zfx);
+        sc = block_excl_scan(sc, x_red_u, &total_c);
+        for (uint32_t q = 0; q < kPer; ++q) {
+            const uint64_t om = hm[t * kPer + q];
+            const uint32_t oc = hc[t * kPer + q];
+            hm[t * kPer + q] = sm;
+            hc[t * kPer + q] = sc;
+            sm += om;
+            sc += oc;
+        }
+    }
+    __syncthreads();
+
+    auto walk = [&](bool by_mass, uint64_t want) __attribute__((always_inline)) { return exact_walk(in, Zfx, by_mass ? 1u : 0u, want); };
     // smallest race key of the block, the candidate that is earlier in sorted order (the larger `who`) on equal keys
     const double inf = __longlong_as_double(0x7FF0000000000000ll);
     auto block_first = [&](double& k, uint64_t& who) {
@@ -1390,26 +1575,13 @@ __device__ __noinline__ ExactOut exact_row(const ExactIn in) {
         }
     };
 
-    // total mass, and the first key in sorted order
-    uint64_t z_own = 0, k_own = 0;
-    each_token([&](uint32_t i, float x) {
-        z_own += fx_of(x);
-        const uint64_t k = key64(x, i);
-        k_own = k > k_own ? k : k_own;
-    });
-    const uint64_t Zfx = block_sum(z_own, red_w);
-    if (t == 0) x_w[5] = 0ull;
-    __syncthreads();
-    atomicMax(&x_w[5], static_cast<unsigned long long>(k_own));
-    __syncthreads();
-    const uint64_t k_top = x_w[5];
     const double Zs = static_cast<double>(Zfx) / kFx, Zfs = static_cast<double>(static_cast<float>(Zs));
     const double u = in.u;
     uint64_t kk = 0ull, kept_fx = Zfx;  // the kept set: keys >= kk, nk of them, kept_fx their mass
     uint32_t nk = V;
     // the race over every token at or above a key (E = -ln(1 - U), U hashed from the row's base and the token)
-    auto race_from = [&](uint64_t from, double Zk) {
-        auto race_key = [&](uint64_t cand) {
+    auto race_from = [&](uint64_t from, double Zk) __attribute__((always_inline)) {
+        auto race_key = [&](uint64_t cand) __attribute__((always_inline)) {
             const double e = e_of(x_of(cand));
             const uint64_t h = mix64(in.rbase + (static_cast<uint64_t>(static_cast<uint32_t>(id_of(cand))) + 1ull) * 0xE7037ED1A0B428DBull);
             const double E = -log(1.0 - unit53(h));
@@ -1417,7 +1589,7 @@ __device__ __noinline__ ExactOut exact_row(const ExactIn in) {
         };
         double k1 = inf, k2nd = inf;
         uint64_t w1 = 0;
-        each_token([&](uint32_t i, float x) {
+        each_token([&](uint32_t i, float x) __attribute__((always_inline)) {
             const uint64_t c = key64(x, i);
             if (c < from) return;
             const double k = race_key(c);
@@ -1446,7 +1618,7 @@ __device__ __noinline__ ExactOut exact_row(const ExactIn in) {
         kept_fx = w1.before_m + w1.own_m;
         nk = in.n1_asked;
     }
-    auto draw_walk = [&](double Zk_fx) {  // inverse-CDF draw among the first nk keys; false: the walk left them
+    auto draw_walk = [&](double Zk_fx) __attribute__((always_inline)) {  // inverse-CDF draw among the first nk keys; false: the walk left them
         const double T = u * Zk_fx;
         const Walk wd = walk(true, static_cast<uint64_t>(floor(T)) + 1ull);
         if (!wd.found || wd.before_c >= nk) return false;
@@ -1481,7 +1653,7 @@ __device__ __noinline__ ExactOut exact_row(const ExactIn in) {
             uint32_t c_own = 0;
             uint64_t s_own = 0, kmin_own = ~0ull;
             double near = 1.0;
-            each_token([&](uint32_t i, float x) {
+            each_token([&](uint32_t i, float x) __attribute__((always_inline)) {
                 const double e = e_of(x);
                 near = fmin(near, fabs(e - min_p) / min_p);
                 if (e >= min_p) {
