@@ -111,7 +111,10 @@ int compute_units() {
 
 // Few rows of the short-list kind: how many workgroups share a row. A share fits the registers of 512 threads (80 tokens
 // each) and has 2048 tokens at least; as many parts as the compute units allow, up to 16 - a wide top-k gets 8 at most, its
-// waves' lists need the room. Nobody waits for anybody, so more workgroups than compute units are no danger, only slower.
+// waves' lists need the room. More workgroups than compute units (rows too long for the parts there are units for): nobody
+// waits for anybody, but the second round of them costs more than it saves, bf16 rows of 96000 tokens and more aside (shared
+// and unshared microseconds, top-k 40: 181 rows of 44992 fp32 32.7 / 22.4, 90 of 151936 fp32 37.6 / 33.6, 150 of 44992 bf16
+// 29.1 / 23.3; 90 of 151936 bf16 32.7 / 38.8, 60 of 220032 bf16 29.0 / 44.7).
 void few_plan(const ws_batch* b, uint64_t cap, uint64_t maps, BatchPlan& p) {
     p.few_parts = 0;
     if (b->max_split == 1u || cap > ws::kFewLists) return;
@@ -125,7 +128,8 @@ void few_plan(const ws_batch* b, uint64_t cap, uint64_t maps, BatchPlan& p) {
     if (parts > b->vocab / 2048u) parts = b->vocab / 2048u;
     if (parts < least) parts = least;
     if (cap > uint64_t{parts} * 1600u) return;  // (touched tokens of a share: room for 2048)
-    if (parts < 2u || parts > most || static_cast<uint64_t>(b->rows) * parts > 2ull * cus) return;
+    const bool twice = b->dtype == WS_DTYPE_BF16 && b->vocab >= 96000u;
+    if (parts < 2u || parts > most || static_cast<uint64_t>(b->rows) * parts > (twice ? 2ull : 1ull) * cus) return;
     const uint64_t three = (cap * 8u > 65536u ? ((cap * 8u + 15u) & ~uint64_t{15}) : 65536u) + maps;
     const uint64_t own = 32768u + ws::kFewShare * 2u;
     const uint64_t total = own > three ? own : three;
