@@ -404,3 +404,25 @@ def test_dflash_topk_and_argmax_prob_shared_between_workgroups(k, rows5):
             tok, prob = m.argmax_prob(dx[r], workspace=w1)
             assert tok.item() == first_max(x[r])
             assert abs(prob.item() - softmax_top(x[r])) <= 2e-6 * softmax_top(x[r]) + 1e-12
+
+
+@pytest.mark.parametrize("n", [4096, 4097, 4099, 50258, 151937, 163843])
+@pytest.mark.parametrize("K", [1, 256, 3000])
+def test_topk_rows_off_the_vector_boundaries(n, K):
+    """Rows of any length, so that most start off a 16-byte boundary: the K largest, ties to the lowest ids, in id order; a row
+    of ties, one whose largest logits stand behind its last whole vector, one with NaN there."""
+    m = gpu_cases.pkg()
+    rng = np.random.default_rng(n + K)
+    x = (rng.standard_normal((5, n)) * 2).astype(np.float32)
+    x[1] = np.round(x[1] * 2) / 2
+    x[2, n - 3:] = [9.0, 30.0, 9.0]
+    x[3, n - 1] = np.nan
+    ids, vals, stats = [a.cpu().numpy() for a in m.topk_rows(torch.from_numpy(x).to(DEV), K, 1.25)]
+    for r in range(5):
+        xr = np.where(np.isnan(x[r]), -np.inf, x[r]).astype(np.float64)
+        want = np.sort(np.lexsort((np.arange(n), -xr))[:K])
+        assert np.array_equal(ids[r], want), r
+        assert vals[r].tobytes() == x[r][want].tobytes(), r
+        assert stats[r, 0] == xr.max()
+        truth = np.exp((xr - xr.max()) * 1.25).sum()
+        assert abs(stats[r, 1] - truth) <= 2e-6 * truth  # (the bar of the aligned rows)

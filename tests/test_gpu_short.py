@@ -180,3 +180,27 @@ def test_min_p_rows_in_bf16_with_a_mask():
     c["min_p"][:] = [0.3, 0.1, 0.02] * 4
     res, _ = run_short(c, 0, max_differ=1)
     assert res["exact"] >= 11 and res["short"] == 12, res
+
+
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("V,allowed", [(9, None), (15, 0.8), (4099, None), (32771, 0.5), (50257, None), (151937, 0.1)])
+def test_unshared_rows_that_end_inside_a_vector(V, allowed, dtype):
+    """The tokens behind the last whole vector come in one by one: untouched, touched and masked-out ones, the row's largest
+    among them, with a head that is the whole row and one that is not."""
+    c = gc.make_cfg2(rows=6, V=V, n_hist=min(300, V // 2), n_bias=min(20, V // 3))
+    rng = np.random.default_rng(V)
+    c["top_k"][:] = [1, 2, 5, 8, 8, 3] if V < 64 else [1, 40, 25, 300, 1000, 64]
+    c["min_p"][:] = 0.0
+    x = np.array(c["logits"])
+    x[0, V - 1] = x[1, V - V % 4 - (0 if V % 4 else 1)] = 12.0
+    c["logits"] = x
+    if dtype == "bf16":
+        c["logits"], c["dtype"] = gc.f32_to_bf16_bits(x), "bf16"
+    if allowed is not None:
+        allow = rng.random((6, (V + 31) // 32 * 32)) < allowed
+        allow[:3, V - 1] = True
+        c["allow"] = np.ascontiguousarray(np.packbits(allow, axis=1, bitorder="little").view(np.uint32))
+    d = gc.upload(c, hints=True, min_p_hint=True)
+    smp = gc.sampler_for(c, d, 1, kept_cap=1024, max_split=1).run()
+    res = gc.compare_rows(c, smp, range(6), 1)
+    assert res["differ"] <= (1 if dtype == "bf16" else 0) and res["exact"] + res["differ"] == 6, res

@@ -33,6 +33,27 @@ __device__ __forceinline__ uint64_t key64(float f, uint32_t id) {
     return (static_cast<uint64_t>(key32(f)) << 32) | static_cast<uint64_t>(0xffffffffu - id);
 }
 
+// A row's vectors of 128 bits wherever the row begins (rows of an odd vocabulary lie off every boundary; the memory
+// system takes a 128-bit load at any address, and splits it where it crosses a line). A row whose size is no multiple of a
+// vector: the last vector is read where it ends with the row, and part_vector moves its tokens down to their places, the
+// places past the row filled with NaN. `drop`: tokens of the vector read that belong to the one before it.
+struct __attribute__((packed, aligned(2))) LooseVec {
+    uint32_t x, y, z, w;
+};
+template <int DT>
+__device__ __forceinline__ uint4 row_vector(const unsigned char* base, uint32_t j, uint32_t V) {
+    constexpr uint32_t TPV = DT == 0 ? 4u : 8u;
+    const uint32_t at = min(j * TPV, V - TPV) * (DT == 0 ? 4u : 2u);  // (a vector past the row: the row's end)
+    const LooseVec v = *reinterpret_cast<const LooseVec*>(base + at);
+    return make_uint4(v.x, v.y, v.z, v.w);
+}
+template <int DT>
+__device__ __forceinline__ uint4 part_vector(const uint4& q, uint32_t drop) {
+    unsigned __int128 v = (static_cast<unsigned __int128>((static_cast<uint64_t>(q.w) << 32) | q.z) << 64) | ((static_cast<uint64_t>(q.y) << 32) | q.x);
+    v = ~(~v >> (drop * (DT == 0 ? 32u : 16u)));
+    return make_uint4(static_cast<uint32_t>(v), static_cast<uint32_t>(v >> 32), static_cast<uint32_t>(v >> 64), static_cast<uint32_t>(v >> 96));
+}
+
 // ---- wave inclusive scan (sum of lanes 0..own) on the data-parallel-primitive path: four shifts inside each row of
 // 16 lanes, then lane 15 of rows 0 and 2 into rows 1 and 3, then lane 31 into rows 2 and 3. Lanes without a source,
 // and rows a step leaves out, add 0. Six dependent vector instructions instead of six trips through the LDS crossbar.

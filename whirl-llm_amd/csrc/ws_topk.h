@@ -312,6 +312,14 @@ __device__ __forceinline__ int topk_from_list(const float* __restrict__ x, const
     return 0;
 }
 
+// vector j of a row of n >= 4 tokens that may start at any token, NaN behind the last one's tokens
+__device__ __forceinline__ float4 loose_vector(const float* __restrict__ x, int n, uint32_t j) {
+    const uint32_t V = static_cast<uint32_t>(n);
+    uint4 q = row_vector<0>(reinterpret_cast<const unsigned char*>(x), j, V);
+    if (V % 4u && j == V / 4u) q = part_vector<0>(q, 4u - V % 4u);
+    return make_float4(__uint_as_float(q.x), __uint_as_float(q.y), __uint_as_float(q.z), __uint_as_float(q.w));
+}
+
 // After the first pass with counts: the rest of the histogram route.
 __device__ __forceinline__ bool topk_by_counts(const float* __restrict__ x, int n, uint32_t kk, float scale, float a32, const TopkLds& L,
                                                int* ids, float* vals) {
@@ -345,8 +353,7 @@ __device__ __forceinline__ bool topk_by_counts(const float* __restrict__ x, int 
     if (bcut >= static_cast<uint32_t>(kTopkTail)) return false;  // the cut lies among -inf / NaN / far-off logits
 
     // second pass: wave w takes the w-th stretch of the row, 64 vectors at a time in id order
-    const float4* __restrict__ x4 = reinterpret_cast<const float4*>(x);
-    const uint32_t nv = static_cast<uint32_t>(n) >> 2;
+    const uint32_t nv = (static_cast<uint32_t>(n) + 3u) >> 2;
     const uint32_t R = (nv + WS_WAVES - 1u) / WS_WAVES;
     const uint32_t j_begin = min(wv * R, nv), j_end = min(j_begin + R, nv);
     const float tail = static_cast<float>(kTopkTail + lane);
@@ -355,7 +362,7 @@ __device__ __forceinline__ bool topk_by_counts(const float* __restrict__ x, int 
     for (uint32_t j0 = j_begin; j0 < j_end; j0 += 64u * kU) {
         float4 q[kU];
 #pragma unroll
-        for (uint32_t u = 0; u < kU; ++u) q[u] = x4[min(j0 + 64u * u + lane, j_end - 1u)];
+        for (uint32_t u = 0; u < kU; ++u) q[u] = loose_vector(x, n, min(j0 + 64u * u + lane, j_end - 1u));
 #pragma unroll
         for (uint32_t u = 0; u < kU; ++u) {
             const uint32_t j = j0 + 64u * u + lane;
@@ -405,7 +412,7 @@ __device__ __forceinline__ bool topk_by_counts(const float* __restrict__ x, int 
     for (uint32_t j0 = j_begin; j0 < j_end; j0 += 64u * kU) {
         float4 q[kU];
 #pragma unroll
-        for (uint32_t u = 0; u < kU; ++u) q[u] = x4[min(j0 + 64u * u + lane, j_end - 1u)];
+        for (uint32_t u = 0; u < kU; ++u) q[u] = loose_vector(x, n, min(j0 + 64u * u + lane, j_end - 1u));
 #pragma unroll
         for (uint32_t u = 0; u < kU; ++u) {
             const uint32_t j = j0 + 64u * u + lane;
@@ -454,12 +461,14 @@ __device__ __forceinline__ void topk_one_row(const float* x, int n, int K, float
     // A bound above the maximum (+ 8 units) and the spread of the logits, both from the first 4096 of them: the bins
     // of the histogram route hang from the bound and are as fine as 3968 of them over bound - smallest allow (fine
     // bins: few tokens of a wave instruction meet on one counter, and few tokens share the cut's bin).
-    // Rows it cannot take - unaligned, short, a bound that is not finite - count nothing and go the radix way.
-    bool counted = (reinterpret_cast<uintptr_t>(x) & 15u) == 0 && (n & 3) == 0 && n >= 4 * WS_BLOCK && kk > 0 && kk < static_cast<uint32_t>(n);
+    // Rows it cannot take - short, a bound that is not finite - count nothing and go the radix way. (Rows off the 16-byte
+    // boundaries and of any length go the counting way as well, by 128-bit loads at whatever address: the radix way's
+    // five passes of 4-byte loads took 235 us for 5 rows of 232703, this way takes 36.)
+    bool counted = n >= 4 * WS_BLOCK && n < (1 << 30) && kk > 0 && kk < static_cast<uint32_t>(n);
     float scale = 0.f, a32 = 0.f, bound = 0.f;
     int list_bin = -1;
     if (counted) {  // uniform
-        const float4 q = reinterpret_cast<const float4*>(x)[threadIdx.x];
+        const float4 q = ws::loose_vector(x, n, threadIdx.x);
         const float v[4] = {q.x, q.y, q.z, q.w};
         float hi = -INFINITY, lo = INFINITY;
 #pragma unroll
