@@ -156,3 +156,25 @@ def test_thousands_of_ties_at_the_cut_and_the_draw(V):
     c["min_p"][5:7] = [0.1, 0.05]
     res, _ = run_case(c, 1, max_differ=2)  # (cuts between equal masses lie within the rounding of a sum)
     assert res["exact"] >= 6, res
+
+
+@pytest.mark.parametrize("V", [5, 8, 4099, 32771, 50257, 170001])
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_three_pass_rows_at_any_address(V, dtype):
+    """Rows that begin at any token and end inside a vector, through the three-pass kernel: history, bias and mask entries in the
+    last vector and behind it, the row's largest token there, kept sets dumped."""
+    c, rng = _base(6, V, n_hist=min(200, V), seed=5)
+    c["name"] = f"rows of {V} {dtype}"
+    x = np.array(c["logits"])
+    x[1, V - 1], x[2, max(0, V - 9)] = 9.0, 11.0
+    c["logits"] = x
+    if dtype == "bf16":
+        c["dtype"], c["logits"] = "bf16", gc.f32_to_bf16_bits(x)
+    c["hist"][:, 0], c["hist"][3, -1] = V - 1, max(0, V - 8)
+    allow = rng.random((6, (V + 31) // 32 * 32)) < 0.8
+    allow[:, V - 1] = True
+    c["allow"] = np.ascontiguousarray(np.packbits(allow, axis=1, bitorder="little").view(np.uint32))
+    c["top_p"][:] = [0.9, 0.95, 0.8, 0.99, 1.0, 0.7]
+    c["top_k"][:] = [0, 0, 50, 0, 40, 0]
+    res, _ = run_case(c, 0, max_differ=1)
+    assert res["exact"] >= 5, res
