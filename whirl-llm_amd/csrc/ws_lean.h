@@ -1001,6 +1001,7 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const uint32_t row,
             r1c1 = b2 > hi3 ? cut.cex + cut.c : fhi.cex + fhi.c;
         }
         const double m1lo = zlo;                           // mass ranked before range 1
+        if (topp_in_list && !minp_in_list && cut.b != 0xffffffffu && cut.c != 0u) kept_bounds(X, cut.c, zlo, zhi);
         if (r1lo == 0 && zlo < 1.0) zlo = fmin(1.0, zhi);  // the top token is always kept
         if (lane == 0u) {
             sel.X = X;
