@@ -52,6 +52,13 @@ def test_any_number_of_parts(max_split):
     run(case(2, 81920, top_k=50), max_split=max_split)
 
 
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("V,max_split", [(81921, 2), (114681, 2), (114688, 2), (172032, 3), (172025, 3)])
+def test_shares_of_112_tokens_a_thread(V, max_split, dtype):
+    """Too few parts for shares of 80 tokens a thread: the smallest and the largest rows of the wide ones."""
+    run(case(2, V, dtype, top_k=50, n_hist=1500, allowed=0.7 if V % 2 else None), max_split=max_split)
+
+
 @pytest.mark.parametrize("dtype,top_k", [("f32", 1), ("f32", 512), ("bf16", 513), ("f32", 1024), ("bf16", 64)])
 def test_top_k_from_one_to_the_largest(dtype, top_k):
     run(case(2, 40003, dtype, top_k=top_k), max_differ=1 if dtype == "bf16" else 0)

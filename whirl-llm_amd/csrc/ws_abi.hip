@@ -111,10 +111,11 @@ int compute_units() {
 
 // Few rows of the short-list kind: how many workgroups share a row. A share fits the registers of 512 threads (80 tokens
 // each) and has 2048 tokens at least; as many parts as the compute units allow, up to 16 - a wide top-k gets 8 at most, its
-// waves' lists need the room. More workgroups than compute units (rows too long for the parts there are units for): nobody
-// waits for anybody, but the second round of them costs more than it saves, bf16 rows of 96000 tokens and more aside (shared
-// and unshared microseconds, top-k 40: 181 rows of 44992 fp32 32.7 / 22.4, 90 of 151936 fp32 37.6 / 33.6, 150 of 44992 bf16
-// 29.1 / 23.3; 90 of 151936 bf16 32.7 / 38.8, 60 of 220032 bf16 29.0 / 44.7).
+// waves' lists need the room. Where the compute units allow fewer parts than that takes, shares of 112 tokens a thread are
+// tried (two parts hold 114688 tokens, three 172032: unshared and shared microseconds, top-k 40: 90 rows of 82000 fp32
+// 23.3 / 18.9, 70 of 151936 33.2 / 25.3, 90 of 92736 bf16 32 / 17). More workgroups than compute units: nobody waits for
+// anybody, but the second round of them costs more than it saves (181 rows of 44992 fp32 22.4 / 32.7, 160 of 82000 bf16
+// 29 / 32), bf16 rows of 130000 tokens and more aside (90 rows of 151936 38.8 / 32.7, 60 of 220032 44.7 / 29.0).
 void few_plan(const ws_batch* b, uint64_t cap, uint64_t maps, BatchPlan& p) {
     p.few_parts = 0;
     if (b->max_split == 1u || cap > ws::kFewLists) return;
@@ -126,12 +127,12 @@ void few_plan(const ws_batch* b, uint64_t cap, uint64_t maps, BatchPlan& p) {
     uint32_t parts = cus / b->rows;
     if (parts > most) parts = most;
     if (parts > b->vocab / 2048u) parts = b->vocab / 2048u;
-    if (parts < least) parts = least;
+    if (parts < least && (parts < 2u || uint64_t{parts} * ws::kFewWide < b->vocab)) parts = least;
     if (cap > uint64_t{parts} * 1600u) return;  // (touched tokens of a share: room for 2048)
-    const bool twice = b->dtype == WS_DTYPE_BF16 && b->vocab >= 96000u;
+    const bool twice = b->dtype == WS_DTYPE_BF16 && b->vocab >= 130000u;
     if (parts < 2u || parts > most || static_cast<uint64_t>(b->rows) * parts > (twice ? 2ull : 1ull) * cus) return;
     const uint64_t three = (cap * 8u > 65536u ? ((cap * 8u + 15u) & ~uint64_t{15}) : 65536u) + maps;
-    const uint64_t own = 32768u + ws::kFewShare * 2u;
+    const uint64_t own = 32768u + (parts < least ? ws::kFewWide : ws::kFewShare) * 2u;
     const uint64_t total = own > three ? own : three;
     if (total + kStaticFew > kMaxLds) return;
     p.few_parts = parts;

@@ -403,7 +403,7 @@ template <int DT, bool MASKED, int NV>
 __device__ __forceinline__ bool few_row(const BatchArgs& A, const uint32_t row, const uint32_t part, FewShared& F, bool& finisher) {
     extern __shared__ __align__(16) unsigned char lds[];
     constexpr uint32_t TPV = DT == 0 ? 4u : 8u;  // tokens in a 128-bit vector
-    static_assert(NV * TPV * WS_BLOCK <= kFewShare, "tokens a share");
+    static_assert(NV * TPV * WS_BLOCK <= kFewWide, "tokens a share");
     ShortShared& S = F.sh;
     const uint32_t t = threadIdx.x, lane = t & 63u;
     const uint32_t wv = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(t >> 6)));

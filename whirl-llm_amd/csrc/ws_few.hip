@@ -10,18 +10,18 @@ namespace ws {
 namespace {
 // [dtype][masked][size]: vectors a thread
 using FewKernel = void (*)(BatchArgs);
-constexpr uint32_t kFewVectors[2][3] = {{5u, 10u, 20u}, {3u, 5u, 10u}};
-const FewKernel kFewKernels[2][2][3] = {
-    {{few_batch_kernel<0, false, 5>, few_batch_kernel<0, false, 10>, few_batch_kernel<0, false, 20>},
-     {few_batch_kernel<0, true, 5>, few_batch_kernel<0, true, 10>, few_batch_kernel<0, true, 20>}},
-    {{few_batch_kernel<1, false, 3>, few_batch_kernel<1, false, 5>, few_batch_kernel<1, false, 10>},
-     {few_batch_kernel<1, true, 3>, few_batch_kernel<1, true, 5>, few_batch_kernel<1, true, 10>}}};
+constexpr uint32_t kFewVectors[2][4] = {{5u, 10u, 20u, 28u}, {3u, 5u, 10u, 14u}};
+const FewKernel kFewKernels[2][2][4] = {
+    {{few_batch_kernel<0, false, 5>, few_batch_kernel<0, false, 10>, few_batch_kernel<0, false, 20>, few_batch_kernel<0, false, 28>},
+     {few_batch_kernel<0, true, 5>, few_batch_kernel<0, true, 10>, few_batch_kernel<0, true, 20>, few_batch_kernel<0, true, 28>}},
+    {{few_batch_kernel<1, false, 3>, few_batch_kernel<1, false, 5>, few_batch_kernel<1, false, 10>, few_batch_kernel<1, false, 14>},
+     {few_batch_kernel<1, true, 3>, few_batch_kernel<1, true, 5>, few_batch_kernel<1, true, 10>, few_batch_kernel<1, true, 14>}}};
 }  // namespace
 
 int prepare_few(unsigned lds_limit) {
     static std::atomic<uint64_t> done{0};
-    const void* all[12];
-    for (int k = 0; k < 12; ++k) all[k] = reinterpret_cast<const void*>(kFewKernels[k / 6][k / 3 % 2][k % 3]);
+    const void* all[16];
+    for (int k = 0; k < 16; ++k) all[k] = reinterpret_cast<const void*>(kFewKernels[k / 8][k / 4 % 2][k % 4]);
     return raise_lds_limit_of(done, all, lds_limit);
 }
 
@@ -30,7 +30,7 @@ int launch_few(hipStream_t stream, const BatchArgs& a, unsigned lds_bytes, unsig
     const uint32_t per = a.dtype == 0 ? 4u : 8u, vectors = (a.vocab + per - 1u) / per, load = 64u * WS_WAVES * a.few_parts;
     const uint32_t each = (vectors + load - 1u) / load;
     int size = 0;
-    while (size < 2 && each > kFewVectors[a.dtype][size]) ++size;
+    while (size < 3 && each > kFewVectors[a.dtype][size]) ++size;
     hipLaunchKernelGGL(kFewKernels[a.dtype][a.allow ? 1 : 0][size], dim3(a.few_parts, a.rows), dim3(WS_BLOCK), lds_bytes, stream, a);
     return static_cast<int>(hipGetLastError());
 }
