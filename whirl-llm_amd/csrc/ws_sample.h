@@ -308,12 +308,6 @@ __device__ __forceinline__ float anchor_product(float anchor, float c64) {
     return __fmaf_rn(fabsf(a), 4.76837158203125e-7f, a);  // + 2^-21 |a|: above the exact product whatever the roundings
 }
 constexpr int kTail = 4032;  // first bin of the tail
-// The provisional anchor lies this many units of the exponent above the largest logit at the head of the row, and its
-// histogram stands when the row's maximum turns out at most kTooHigh bins below it (39 units of resolution are left then).
-// With 8 units, one confident row in twenty at T = 0.6 .. 1.2 - a few tokens lifted to logits of 10 to 14, none of them
-// among the first - had a token above the anchor and was swept twice, and a launch takes as long as its slowest row: 64 rows
-// of 151936 bf16 took 77 us. With 16 the same batch takes 47, and rows that 8 fitted take as long as before.
-constexpr float kAbove = 16.f, kTooHigh = 1536.f;
 __device__ __forceinline__ float bin_coord(float aq, float c64, float x, float tail = 4095.f) {
     const float t = __fmaf_rn(x, -c64, aq);
     return __builtin_fminf(t, tail);  // minNum: NaN -> tail
@@ -392,7 +386,7 @@ __device__ __forceinline__ bool fused_pass_impl(const RowView& rv, float floor_v
         }
         s = block_max(s, red);  // its barriers also publish the zeroed histogram
         if (given_s == given_s) s = given_s;  // a slice of a split row: the bound every part derives from the head of the row
-        anchor = s + kAbove / inv_t;
+        anchor = s + 8.f / inv_t;
         aq = anchor_product(anchor, c64);
         if (!(anchor > -INFINITY && anchor < INFINITY)) return false;
     }
@@ -2402,7 +2396,7 @@ __device__ __forceinline__ void sample_row(const BatchArgs& A, const uint32_t bl
             if (swept) {
                 m = m_all;
                 // the sweep stands if no token beat the anchor and the anchor is not wastefully high (a masked outlier)
-                cached = m <= anchor && (anchor - m) * c64 <= kTooHigh;
+                cached = m <= anchor && (anchor - m) * c64 <= 1024.f;
             }
         }
         if (WS_RARE(split && (!cached || gave_up || !(m > -INFINITY)))) {
@@ -2461,7 +2455,7 @@ __device__ __forceinline__ void sample_row(const BatchArgs& A, const uint32_t bl
             }
             float s = head_max(-INFINITY);  // (its barriers also end the reads of the rank tables)
             WS_MARK(9);
-            anchor = s + kAbove / inv_t;
+            anchor = s + 8.f / inv_t;
             if (anchor > -INFINITY && anchor < INFINITY) {  // uniform
                 aq = anchor_product(anchor, c64);
                 for (uint32_t b = t; b < kBins; b += WS_BLOCK) hist[b] = 0ull;
@@ -2480,7 +2474,7 @@ __device__ __forceinline__ void sample_row(const BatchArgs& A, const uint32_t bl
                 adjusted = true;
                 replay_touched([&](uint32_t i, float x) { add_to_hist(i, x, 0); });
                 m = fmaxf(block_max(m, red_f), m_adj);
-                cached = m <= anchor && (anchor - m) * c64 <= kTooHigh;  // here: the histogram stands
+                cached = m <= anchor && (anchor - m) * c64 <= 1024.f;  // here: the histogram stands
             } else {
                 __syncthreads();
             }
@@ -2491,7 +2485,7 @@ __device__ __forceinline__ void sample_row(const BatchArgs& A, const uint32_t bl
             // bound above the maximum guessed from the adjusted tokens and the head of the row (as the single-sweep
             // mode does); rows the guess does not fit fall through to the two passes below
             float s = head_max(m_adj);
-            anchor = s + kAbove / inv_t;
+            anchor = s + 8.f / inv_t;
             if (anchor > -INFINITY && anchor < INFINITY) {  // uniform
                 aq = anchor_product(anchor, c64);
                 for (uint32_t b = t; b < kBins; b += WS_BLOCK) hist[b] = 0ull;
@@ -2505,7 +2499,7 @@ __device__ __forceinline__ void sample_row(const BatchArgs& A, const uint32_t bl
                     [](uint32_t, uint32_t) {});
                 replay_touched([&](uint32_t i, float x) { add_to_hist(i, x, 0); });
                 m = fmaxf(block_max(m, red_f), m_adj);
-                cached = m <= anchor && (anchor - m) * c64 <= kTooHigh;  // here: the histogram stands
+                cached = m <= anchor && (anchor - m) * c64 <= 1024.f;  // here: the histogram stands
             }
         }
         if (WS_RARE(!cached)) {
@@ -2986,10 +2980,9 @@ __device__ __forceinline__ void sample_row(const BatchArgs& A, const uint32_t bl
                 const bool lean = !race && !open_row && !(flags & kOverflow) && n_r0 <= lean_max && n_r1 <= lean_max && n_hit <= 4u * WS_BLOCK;
                 bool lean_failed = false;
                 if (lean) {
-                    // masses of a range in units of 2^-52 of the largest mass a token of the range can have (the maximum's, 1, at most:
-                    // a range from the top of the row starts at the anchor)
+                    // masses of a range in units of 2^-52 of the largest mass a token of the range can have
                     auto edge_mass = [&](int b) { return s_exp[b >> 6] * s_exp[64 + (b & 63)] * to_max * 1.00001; };
-                    const double emax0 = fmin(edge_mass(r0lo), 1.00001), emax1 = has_r1 ? edge_mass(r1lo) : 1.0;
+                    const double emax0 = edge_mass(r0lo), emax1 = has_r1 ? edge_mass(r1lo) : 1.0;
                     const double scale0 = 4503599627370496.0 / emax0, scale1 = 4503599627370496.0 / emax1;
                     const double inv0 = emax0 * (1.0 / 4503599627370496.0), inv1 = emax1 * (1.0 / 4503599627370496.0);
                     const float step0 = 64.f / static_cast<float>(nb0), step1 = has_r1 ? 64.f / static_cast<float>(nb1) : 0.f;
@@ -4148,19 +4141,8 @@ __device__ __forceinline__ void sample_row(const BatchArgs& A, const uint32_t bl
         } else if (finished_lean) {  // the keys lie in the buckets' places
             const uint32_t* cnt_of = reinterpret_cast<const uint32_t*>(s_pool + 128);
             const uint32_t shift = A.lds_tie ? 5u : 4u;
-            // (in whichever order they arrived: added up as whole numbers, 2^-90 to the unit, so that the sum is not that order's)
-            uint64_t hi = 0, lo = 0;
             for (uint32_t slot = t; slot < (128u << shift); slot += WS_BLOCK)
-                if ((slot & ((1u << shift) - 1u)) < cnt_of[slot >> shift]) {
-                    se = 0.0;
-                    term(reinterpret_cast<const uint64_t*>(lds)[slot]);
-                    const double up = se * 1099511627776.0, whole = floor(up);  // (e a is at most 1 / e)
-                    hi += static_cast<uint64_t>(whole);
-                    lo += static_cast<uint64_t>((up - whole) * 1125899906842624.0);
-                }
-            hi = block_sum(hi, reinterpret_cast<uint64_t*>(red_q));
-            lo = block_sum(lo, reinterpret_cast<uint64_t*>(red_q));
-            se = t == 0 ? static_cast<double>(hi) * (1.0 / 1099511627776.0) + static_cast<double>(lo) * (1.0 / 1099511627776.0 / 1125899906842624.0) : 0.0;
+                if ((slot & ((1u << shift) - 1u)) < cnt_of[slot >> shift]) term(reinterpret_cast<const uint64_t*>(lds)[slot]);
         } else {
             const uint32_t n_sorted = open_row ? min(n3, n_list) : n_list;
             for (uint32_t i = t; i < n_sorted; i += WS_BLOCK) term(keys[i]);
