@@ -423,9 +423,14 @@ __device__ __forceinline__ bool short_row(const BatchArgs& A, const uint32_t row
     uint32_t* cnt = reinterpret_cast<uint32_t*>(lds + A.lds_cnt);
     uint16_t* first = reinterpret_cast<uint16_t*>(cnt + A.patch_cap);
 
-    // the row in whole vectors; the few tokens behind them (none, of most vocabularies) come in one by one after the sweep
-    const uint32_t nv = V / TPV, n_odd = V % TPV;
+    // The row in vectors. Without a mask the whole ones, and the few tokens behind them (none, of most vocabularies) one by one
+    // after the sweep; with one all of them, the last read where it ends with the row and moved down. (Either way for the registers'
+    // sake: moved vectors spill them in the unmasked bf16 kernel - 1000 rows of 24896: 118 us, now 72 -, clamped whole ones in
+    // the masked fp32 kernel - 1024 rows of 262144: 430 us and more against 390.)
+    const uint32_t nv = MASKED ? (V + TPV - 1u) / TPV : V / TPV, n_odd = MASKED ? 0u : V % TPV;
+    const uint32_t j_part = MASKED && V % TPV ? nv - 1u : 0xffffffffu;
     auto vector_at = [&](uint32_t j) __attribute__((always_inline)) {
+        if (MASKED) return row_vector<DT>(base, j, V);
         const LooseVec v = *reinterpret_cast<const LooseVec*>(base + min(j, nv - 1u) * 16u);
         return make_uint4(v.x, v.y, v.z, v.w);
     };
@@ -439,7 +444,7 @@ __device__ __forceinline__ bool short_row(const BatchArgs& A, const uint32_t row
     for (uint32_t k = 0; k < kShortHead; ++k) {
         const uint32_t j = k * WS_BLOCK + t;
         hq[k] = vector_at(j);
-        hna[k] = MASKED ? allow[(min(j, nv - 1u) * TPV) >> 5] : 0xffffffffu;
+        hna[k] = MASKED ? allow[min(j * TPV, V - 1u) >> 5] : 0xffffffffu;
     }
     for (uint32_t b = t; b < 4096u; b += WS_BLOCK) head_cnt[b] = 0u;
     // (the tables of the touched tokens as well, while the parameters travel: their sizes are the launch's, not the row's)
@@ -562,8 +567,9 @@ __device__ __forceinline__ bool short_row(const BatchArgs& A, const uint32_t row
 
     WSS_MARK(1);  // bitmap done
     // one vector: its tokens as floats, masked-out / touched / NaN ones as -inf
-    auto unpack = [&](const uint4& q, uint32_t na, uint32_t j, float (&x)[TPV]) {
+    auto unpack = [&](uint4 q, uint32_t na, uint32_t j, float (&x)[TPV]) {
         const uint32_t i0 = j * TPV;
+        if (MASKED && j_part != 0xffffffffu && j == j_part) q = part_vector<DT>(q, TPV - V % TPV);  // (uniform before per lane)
         uint32_t invalid = 0u;  // bit e: token e does not count here
         if (MASKED) invalid = ~(na >> (i0 & 31u));
         if (n_touched) invalid |= touched[i0 >> 5] >> (i0 & 31u);
@@ -586,7 +592,7 @@ __device__ __forceinline__ bool short_row(const BatchArgs& A, const uint32_t row
         for (uint32_t k = 0; k < KB; ++k) {
             const uint32_t j = jbase + k * WS_BLOCK + t;
             q[k] = vector_at(j);
-            na[k] = MASKED ? allow[(min(j, nv - 1u) * TPV) >> 5] : 0xffffffffu;
+            na[k] = MASKED ? allow[min(j * TPV, V - 1u) >> 5] : 0xffffffffu;
         }
     };
     load(qa, naa, jb);
@@ -612,7 +618,7 @@ __device__ __forceinline__ bool short_row(const BatchArgs& A, const uint32_t row
     float thr = -INFINITY;  // tokens above it are listed
     // tokens to list: the count above a threshold fitted to a sample of the row scatters like the square root of the
     // sample's rank: half of top_k on top, 150 at least
-    const uint32_t n_head = n_head_vec == nv ? V : n_head_vec * TPV;
+    const uint32_t n_head = n_head_vec == nv ? V : min(n_head_vec * TPV, V);
     // (a head that is the whole row: the count is exact but for the tokens of a bin, and twice top_k will do. 156 rows of
     // 24896, Zipfian, top-k 25: 30.6 us with 191 tokens to list, most of them in a second round of counting, 21 with 56)
     const uint32_t want = min(n_head >= V ? 2u * top_k + 6u : 0xffffffffu, top_k + max(top_k >> 1, 150u) + 16u);
@@ -727,7 +733,7 @@ __device__ __forceinline__ bool short_row(const BatchArgs& A, const uint32_t row
     if (n_odd && !not_mine && ref > -INFINITY) {  // uniform: the tokens behind the last whole vector
         float x = -INFINITY;
         const uint32_t id = nv * TPV + t;
-        if (t < n_odd && (!MASKED || ((allow[id >> 5] >> (id & 31u)) & 1u)) && !(n_touched && ((touched[id >> 5] >> (id & 31u)) & 1u)))
+        if (t < n_odd && !(n_touched && ((touched[id >> 5] >> (id & 31u)) & 1u)))
             x = fmaxf(DT == 0 ? reinterpret_cast<const float*>(base)[id] : bf16_to_f32(reinterpret_cast<const uint16_t*>(base)[id]), -INFINITY);
         if (t < n_odd) {
             const float a = fmaxf(__fsub_rn(x, ref), -1e30f);
