@@ -1,5 +1,5 @@
 """GPU: rows whose candidate ranges do not fit the sampler's list (more than 4096 candidates in the gathered bins) take the
-kernel's exact path - fixed-point masses and radix walks over the 64-bit candidate key - and must give what the oracle
+kernel's exact path - fixed-point masses, a histogram, then the keys of the cut's bin alone - and must give what the oracle
 gives, like every other row: a top-k beyond the list (the reference escalates 256 -> 16384 -> full row,
 src/server/engine_sampling.cpp:51-84), constant rows, rows of a handful of distinct values, flat rows at a high
 temperature, with penalties, masks, the race draw and open rows."""
