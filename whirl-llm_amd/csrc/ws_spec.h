@@ -171,21 +171,19 @@ __global__ void __launch_bounds__(WS_BLOCK) spec_verify_kernel(SpecArgs A) {
         unsigned long long* gsum = reinterpret_cast<unsigned long long*>(A.work + static_cast<size_t>(s) * spec_seq_bytes);
         uint32_t* arrive = reinterpret_cast<uint32_t*>(gsum + kSpecMaxSteps);
         __syncthreads();
-        // (Nothing waits for a store to be acknowledged: a sum goes out as its bits plus one, which are not zero - it is not
-        // negative -, the places are zero between launches, and whoever reads a zero reads again.)
         for (uint32_t k = k_lo + t; k < k_hi; k += WS_BLOCK)
-            __hip_atomic_store(&gsum[k], static_cast<unsigned long long>(__double_as_longlong(step_sum[k])) + 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __syncthreads();  // every wave's stores have been issued
+            __hip_atomic_store(&gsum[k], static_cast<unsigned long long>(__double_as_longlong(step_sum[k])), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        // (the wave's sums have arrived, so that whoever draws the last ticket finds them all: a sum that is looked for instead
+        // may come after its place has been cleared, and stand there for the next launch)
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
         if (t == 0) s_u[3] = __hip_atomic_fetch_add(arrive, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __syncthreads();
         if (s_u[3] != n_parts - 1u) return;
         if (t == 0) __hip_atomic_store(arrive, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // as the next launch needs it
-        for (uint32_t k = t; k < n_steps; k += WS_BLOCK) {
-            unsigned long long word = 0ull;
-            for (uint32_t tries = 0; word == 0ull && tries < 65536u; ++tries) word = __hip_atomic_load(&gsum[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(&gsum[k], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (k < k_lo || k >= k_hi) step_sum[k] = __longlong_as_double(static_cast<long long>(word - 1ull));
-        }
+        for (uint32_t k = t; k < n_steps; k += WS_BLOCK)  // (what an earlier launch left in these places has been written over)
+            if (k < k_lo || k >= k_hi)
+                step_sum[k] = __longlong_as_double(static_cast<long long>(__hip_atomic_load(&gsum[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)));
     }
     for (int attempt = 0; attempt < 2; ++attempt) {
         if (attempt == 1) sweep(0u, n_steps);  // (zero residual: the whole of p, by this workgroup alone)
