@@ -94,6 +94,27 @@ def test_ties_at_the_threshold_and_a_row_of_one_value():
     run(c, handed_back=3)
 
 
+@pytest.mark.parametrize("inv_t", [0.7, 1.25])
+def test_the_waves_sums_meet_in_64_bits(inv_t):
+    """128 tokens, every one a different wave's only one (a wave's own sum is exactly one), so that the normaliser is made of the
+    factors that bring the waves' sums to the row's maximum: it has to be the 64-bit sum, rounded once."""
+    m = gc.pkg()
+    rng = np.random.default_rng(17)
+    rows, V = 16, 32768  # sixteen parts a row, chunks of 32 tokens dealt to 128 waves
+    x = np.full((rows, V), -np.inf, np.float32)
+    at = 32 * np.arange(128) + rng.integers(0, 32, (rows, 128))
+    np.put_along_axis(x, at, rng.uniform(0.0, 9.0, (rows, 128)).astype(np.float32), 1)
+    d = [torch.full((rows,), v, dtype=dt, device="cuda") for v, dt in ((inv_t, torch.float32), (7, torch.int64), (0, torch.int64), (40, torch.int32))]
+    smp = m.BatchSampler(torch.from_numpy(x).cuda(), d[0], d[1], d[2], top_k=d[3], top_k_max=40).run()
+    got = smp.stats.cpu().numpy()
+    assert (smp.flags.cpu().numpy() & m.FLAG_ROUTE_MASK == m.FLAG_ROUTE_SHORT).all()
+    top = x.max(axis=1)
+    want = np.exp((x - top[:, None]).astype(np.float64) * np.float64(np.float32(inv_t))).sum(axis=1)
+    assert np.array_equal(got[:, 0], top)
+    # (a rounding of the 64-bit sum to 32 bits differs between two orders of it once in 2^24 or so)
+    assert np.array_equal(got[:, 1], want.astype(np.float32)), (got[:, 1] - want.astype(np.float32)) / want
+
+
 def test_query_and_entropy():
     """Probability of a named token and the kept set's entropy from the sorted candidates."""
     m = gc.pkg()

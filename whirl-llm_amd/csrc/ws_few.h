@@ -27,13 +27,12 @@
 namespace ws {
 
 constexpr uint32_t kFewWaves = kFewMaxParts * WS_WAVES;
-// Workspace of a row: kFewKeys keys, slot by slot with one key a wave in each, then two words a wave ({maximum, threshold} as
-// order keys; the sum of exp against the maximum, its low thirteen bits holding the number of keys plus one, all of them
-// set when the wave could not list its share), then {parts arrived, largest logit so far as an order key}. Zero-filled
-// between launches.
-constexpr uint32_t kFewKeys = 7648u, kFewHead = kFewKeys * 8u, kFewCtrl = kFewHead + kFewWaves * 16u;
-static_assert(kFewCtrl + 256u <= kFewRowBytes, "a row's workspace");
-constexpr uint32_t kFewBad = 0x1fffu;
+// Workspace of a row: kFewKeys keys, slot by slot with one key a wave in each, then what every wave says of its share -
+// {maximum, threshold} as order keys; the sum of exp against the maximum; how many keys it has listed, kFewBad when it could not
+// list them -, then {parts arrived, largest logit so far as an order key}. Zero-filled between launches.
+constexpr uint32_t kFewKeys = 7648u, kFewHead = kFewKeys * 8u, kFewCount = kFewHead + kFewWaves * 16u, kFewCtrl = kFewCount + kFewWaves * 4u;
+static_assert(kFewCtrl + 256u <= 64512u && 64512u < kFewRowBytes, "a row's workspace (debug builds put their clocks at 64512)");
+constexpr uint32_t kFewBad = 0xffffffffu;
 constexpr uint32_t kFewExt = 2048u;  // touched tokens of a share
 constexpr uint32_t kFewDup = 0x4000u, kFewTaken = 0x8000u;  // in a token's 16-bit word, above its history count: a second bias entry, somebody takes it
 constexpr uint32_t kFewDups = 64u;  // bias entries of tokens that another entry has taken
@@ -53,7 +52,13 @@ struct FewShared {
     float dup_v[kFewDups];
     float red_f[WS_WAVES];  // (few_collect: the row's maximum, and the lowest logit looked at)
     uint32_t w[16];
-    double u, z;
+    double u, z[kFewWaves / 64u];  // (z: the row's normaliser, in as many summands)
+    __device__ __forceinline__ double sum() const {
+        double all = z[0];
+#pragma unroll
+        for (uint32_t i = 1; i < kFewWaves / 64u; ++i) all += z[i];
+        return all;
+    }
 };
 
 // the largest prefix (bits 31 .. 14) of an order key that at least d lanes of the wave reach, two bits a step
@@ -121,6 +126,7 @@ __device__ __forceinline__ bool few_publish(const FewShare& L, const FewWant& W,
     const float wm = wave_max(lm);
     unsigned long long* gkeys = reinterpret_cast<unsigned long long*>(work);
     unsigned long long* ghead = reinterpret_cast<unsigned long long*>(work + kFewHead);
+    uint32_t* gcount = reinterpret_cast<uint32_t*>(work + kFewCount);
     uint32_t* ctrl = reinterpret_cast<uint32_t*>(work + kFewCtrl);
 
     WSF_MARK(1);
@@ -193,11 +199,10 @@ __device__ __forceinline__ bool few_publish(const FewShare& L, const FewWant& W,
     }
     {
         const double z = wm > -INFINITY && wm < INFINITY ? wave_sum(static_cast<double>(s)) : 0.0;
-        const uint32_t n = !ok || !(wm < INFINITY) || n_list > slots ? kFewBad : n_list + 1u;
         if (lane == 0u) {
-            const uint64_t zw = static_cast<uint64_t>(__double_as_longlong(z));
             __hip_atomic_store(&ghead[L.g], (static_cast<unsigned long long>(key32(wm)) << 32) | key32(thr), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(&ghead[kFewWaves + L.g], (zw & ~uint64_t{kFewBad}) | n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(&ghead[kFewWaves + L.g], static_cast<unsigned long long>(__double_as_longlong(z)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(&gcount[L.g], !ok || !(wm < INFINITY) || n_list > slots ? kFewBad : n_list, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
     // What the parts exchange is written and read by device-scope atomic accesses, which go past this unit's caches, and a wave
@@ -216,7 +221,7 @@ __device__ __forceinline__ bool few_publish(const FewShare& L, const FewWant& W,
 }
 
 // The last part: everybody's keys from the larger of the waves' thresholds up - or from a higher bound of the row's top_k-th
-// largest logit - to `list` (LDS, kShortCap keys), in no order; F.red_f[0] and F.z: the row's maximum and normaliser. Every place of
+// largest logit - to `list` (LDS, kShortCap keys), in no order; F.red_f[0] and F.sum(): the row's maximum and normaliser. Every place of
 // the workspace is zero again afterwards. Returns the number of keys (which may be more than the list holds); 0 when a share could not be listed.
 // fourth(): work of the caller's for the fourth wave, while others read the headers.
 template <bool SUM, class FOURTH>
@@ -225,12 +230,12 @@ __device__ __forceinline__ uint32_t few_collect(const FewShare& L, const FewWant
     const uint32_t wv = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(t >> 6)));
     unsigned long long* gkeys = reinterpret_cast<unsigned long long*>(work);
     unsigned long long* ghead = reinterpret_cast<unsigned long long*>(work + kFewHead);
+    uint32_t* gcount = reinterpret_cast<uint32_t*>(work + kFewCount);
     uint32_t* ctrl = reinterpret_cast<uint32_t*>(work + kFewCtrl);
     const uint32_t G = L.G, slots = kFewKeys / G;
-    float k2, k2lo;
-    few_exp_scale(W.inv_t, k2, k2lo);
-    // everybody's keys asked for (those of the first slots right away), then the headers. Four waves read
-    // them side by side, each for what it works out: the threshold, the normaliser, how many slots hold keys, the uniform.
+    // everybody's keys asked for (those of the first slots right away), then the headers. Five waves read them side by side, each
+    // for what it works out: the threshold, the normaliser (two of them: the exponentials are the longest chain here, and one a
+    // lane is 0.1 us shorter than two), how many slots hold keys; and one the uniform.
     constexpr uint32_t kBlind = 4096u / WS_BLOCK, kHL = kFewWaves / 64u;
     uint64_t got[kBlind];
 #pragma unroll
@@ -238,13 +243,18 @@ __device__ __forceinline__ uint32_t few_collect(const FewShare& L, const FewWant
     if (t == 0) F.w[5] = 0u;  // keys taken
     if (wv == 3u) {
         fourth();
-    } else if (wv < 3u) {
-        uint64_t h0[kHL], h1[kHL];
+    } else if (wv < 5u) {
+        const bool sums = wv == 1u || wv == 4u;
+        const uint32_t half = wv == 4u ? 1u : 0u;  // of the waves: the first 64, or the others
+        static_assert(kHL == 2u, "a wave of this part for every 64 of the row");
+        uint64_t h0[kHL], zs = 0ull;
+        uint32_t ns[kHL];
 #pragma unroll
         for (uint32_t i = 0; i < kHL; ++i) {
             const uint32_t w = min(i * 64u + lane, G - 1u);
             h0[i] = __hip_atomic_load(&ghead[w], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            h1[i] = __hip_atomic_load(&ghead[kFewWaves + w], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (SUM && sums && i == half) zs = __hip_atomic_load(&ghead[kFewWaves + w], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (wv == 2u) ns[i] = __hip_atomic_load(&gcount[w], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         float m4[kHL], mx = -INFINITY;
 #pragma unroll
@@ -283,27 +293,22 @@ __device__ __forceinline__ uint32_t few_collect(const FewShare& L, const FewWant
                 F.red_f[0] = mx;
                 F.red_f[1] = floor_v;
             }
-        } else if (wv == 1u) {
+        } else if (sums) {
             double z = 0.0;
-            if (SUM) {
-#pragma unroll
-                for (uint32_t i = 0; i < kHL; ++i)
-                    if (m4[i] > -INFINITY) {
-                        const float a = fmaxf(__fsub_rn(m4[i], mx), -1e30f);
-                        z += __longlong_as_double(static_cast<long long>(h1[i] & ~uint64_t{kFewBad})) * static_cast<double>(__builtin_amdgcn_exp2f(fmaf(a, k2lo, a * k2)));
-                    }
+            if (SUM) {  // (the factors in 64 bits, as the rules work out the candidates' masses)
+                const float own = half ? m4[1] : m4[0];
+                if (own > -INFINITY) z = __longlong_as_double(static_cast<long long>(zs)) * exp(static_cast<double>(__fsub_rn(own, mx)) * static_cast<double>(W.inv_t));
                 z = wave_sum(z);
             }
-            if (lane == 0u) F.z = z;
+            if (lane == 0u) F.z[half] = z;
         } else {
             uint32_t most = 0;
             bool bad = !(mx > -INFINITY);
 #pragma unroll
             for (uint32_t i = 0; i < kHL; ++i)
                 if (i * 64u + lane < G) {
-                    const uint32_t n = static_cast<uint32_t>(h1[i]) & kFewBad;
-                    bad = bad || n == kFewBad || n == 0u;
-                    most = max(most, n - 1u);
+                    bad = bad || ns[i] == kFewBad;
+                    most = max(most, ns[i]);
                 }
             most = wave_max_u32(most);
             bad = __ballot(bad) != 0ull;
@@ -339,6 +344,7 @@ __device__ __forceinline__ uint32_t few_collect(const FewShare& L, const FewWant
     if (t < G) {
         __hip_atomic_store(&ghead[t], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __hip_atomic_store(&ghead[kFewWaves + t], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(&gcount[t], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     if (t < 2u) __hip_atomic_store(&ctrl[t], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
@@ -608,7 +614,7 @@ __device__ __forceinline__ bool few_row(const BatchArgs& A, const uint32_t row, 
     R.top_p = P.top_p;
     R.min_p = min_p;
     R.u = F.u;
-    R.z = F.z;
+    R.z = F.sum();
     R.inv_t = inv_t;
     R.m = m;
     R.n_cand = n_cand;

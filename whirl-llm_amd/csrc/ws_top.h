@@ -15,7 +15,7 @@ struct TopSplit {
     unsigned char* work;  // kFewRowBytes a row
 };
 
-// The K largest logits of this row, by the part of it that arrives last: `list` in descending order (value desc, id asc), F.z
+// The K largest logits of this row, by the part of it that arrives last: `list` in descending order (value desc, id asc), F.sum()
 // the normaliser. Returns 0: another part's business; 1: listed; 2: this part has to do the row without the list.
 template <int NV, bool SUM>
 __device__ __forceinline__ int top_share(const float* x, int n, int K, float inv_t, const TopSplit& sp, uint32_t row, FewShared& F, uint64_t*& list) {
@@ -83,7 +83,7 @@ __global__ void __launch_bounds__(WS_BLOCK) topk_rows_shared(const float* x, int
     __syncthreads();
     if (t == 0) {
         stats[2 * row] = F.red_f[0];
-        stats[2 * row + 1] = static_cast<float>(F.z);
+        stats[2 * row + 1] = static_cast<float>(F.sum());
     }
     const uint32_t half = ((kk + 15u) >> 4 << 3);  // ids each of the two looks at: eight or a multiple
     for (uint32_t i0 = 0; i0 < 2u * kk; i0 += WS_BLOCK) {
@@ -154,7 +154,7 @@ __global__ void __launch_bounds__(WS_BLOCK)
         s_lg[t] = unkey32(static_cast<uint32_t>(list[t] >> 32));
     }
     __builtin_amdgcn_wave_barrier();  // (one wave: its LDS stores are done before its loads)
-    draft_finish<true>(ctl_all, area, r, map, a, qbuf, b, K, s_id, s_lg, F.red_f[0], static_cast<float>(F.z));
+    draft_finish<true>(ctl_all, area, r, map, a, qbuf, b, K, s_id, s_lg, F.red_f[0], static_cast<float>(F.sum()));
 #ifdef WS_SHORT_TIMERS
     unsigned char* work = sp.work + static_cast<size_t>(b) * kFewRowBytes;
     WSF_MARK(9);
