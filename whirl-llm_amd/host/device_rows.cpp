@@ -8,10 +8,11 @@
 // the launch - a decode step is one launch and one wait for that word, which comes some 5 us before a stream wait would end.
 // Everything here has waited for what it launched before it returns, so the host never rewrites a block that a launch
 // still reads.
-// Pinned blocks and the sampler's zero-filled workspace outlive the object that asked for them, in a pool of bounded size
-// (a pinned allocation takes longer than ten decode steps): objects made and dropped once a request find them there.
+// Pinned blocks and the sampler's zero-filled workspace outlive the object that asked for them, in pools of bounded size
+// (block_pool.h): objects made and dropped once a request find them there.
 #include "sampling/device_rows.h"
 
+#include "block_pool.h"
 #include "whirl_sampling_abi.h"
 
 #include <hip/hip_runtime_api.h>
@@ -21,7 +22,6 @@
 #include <cmath>
 #include <cstring>
 #include <limits>
-#include <mutex>
 
 namespace whirl::sampling {
 
@@ -37,90 +37,42 @@ void checkHip(hipError_t e, const char* op) {
     if (e != hipSuccess) throw DeviceError(op, static_cast<int>(e), std::string(op) + ": " + hipGetErrorString(e));
 }
 
-// Blocks of memory between two owners: pinned host memory, or device memory that is all zeros. A block goes back to the
-// runtime when the pool holds kMost of them or kMostBytes. Any thread may call; a block's last user has waited for its launches.
-class BlockPool {
-public:
-    explicit BlockPool(bool pinned) : pinned_(pinned) {}
-    // at least `bytes` on the current device; `got`: how much it is, `fresh`: its contents are anything
-    void* take(std::size_t bytes, std::size_t& got, bool& fresh) {
-        int dev = 0;
-        checkHip(hipGetDevice(&dev), "hipGetDevice");
-        {
-            const std::lock_guard<std::mutex> lock(mutex_);
-            std::size_t best = blocks_.size();
-            for (std::size_t i = 0; i < blocks_.size(); ++i)
-                if (blocks_[i].dev == dev && blocks_[i].bytes >= bytes && blocks_[i].bytes / 4 <= bytes && (best == blocks_.size() || blocks_[i].bytes < blocks_[best].bytes)) best = i;
-            if (best != blocks_.size()) {
-                const Block b = blocks_[best];
-                blocks_.erase(blocks_.begin() + static_cast<std::ptrdiff_t>(best));
-                held_ -= b.bytes;
-                got = b.bytes;
-                fresh = false;
-                return b.at;
-            }
-        }
-        void* p = nullptr;
-        if (pinned_) checkHip(hipHostMalloc(&p, bytes, hipHostMallocDefault), "hipHostMalloc");
-        else checkHip(hipMalloc(&p, bytes), "hipMalloc");
-        got = bytes;
-        fresh = true;
-        return p;
-    }
-    void give(void* p, std::size_t bytes) {
-        if (!p) return;
-        int dev = 0;
-        if (hipGetDevice(&dev) == hipSuccess) {
-            const std::lock_guard<std::mutex> lock(mutex_);
-            if (blocks_.size() < kMost && held_ + bytes <= kMostBytes) {
-                blocks_.push_back({p, bytes, dev});
-                held_ += bytes;
-                return;
-            }
-        }
-        drop(p);
-    }
-    void drop(void* p) {
-        if (p) (void)(pinned_ ? hipHostFree(p) : hipFree(p));
-    }
-
-private:
-    struct Block {
-        void* at;
-        std::size_t bytes;
-        int dev;
-    };
-    static constexpr std::size_t kMost = 16, kMostBytes = std::size_t{8} << 20;
-    bool pinned_;
-    std::mutex mutex_;
-    std::vector<Block> blocks_;
-    std::size_t held_ = 0;
-};
+int currentDevice() {
+    int dev = 0;
+    checkHip(hipGetDevice(&dev), "hipGetDevice");
+    return dev;
+}
+void* makePinned(std::size_t bytes) {
+    void* p = nullptr;
+    checkHip(hipHostMalloc(&p, bytes, hipHostMallocDefault), "hipHostMalloc");
+    return p;
+}
+void* makeDevice(std::size_t bytes) {
+    void* p = nullptr;
+    checkHip(hipMalloc(&p, bytes), "hipMalloc");
+    return p;
+}
 // (never destroyed: at the end of the process the runtime may be gone before them)
 BlockPool& pinnedPool() {
-    static BlockPool& pool = *new BlockPool(true);
+    static BlockPool& pool = *new BlockPool({currentDevice, makePinned, [](void* p) { (void)hipHostFree(p); }});
     return pool;
 }
-BlockPool& zeroPool() {
-    static BlockPool& pool = *new BlockPool(false);
+BlockPool& zeroPool() {  // device memory that is all zeros
+    static BlockPool& pool = *new BlockPool({currentDevice, makeDevice, [](void* p) { (void)hipFree(p); }});
     return pool;
 }
 
 // a pinned array of one owner
 struct Pinned {
-    unsigned char* at = nullptr;
-    std::size_t bytes = 0;
+    Block block;
+    unsigned char* at() const { return static_cast<unsigned char*>(block.at); }
     void need(std::size_t want) {
-        if (want <= bytes) return;
+        if (want <= block.bytes) return;
         release();
         bool fresh;
-        at = static_cast<unsigned char*>(pinnedPool().take(want, bytes, fresh));
+        block = pinnedPool().take(want, fresh);
     }
-    void release() {
-        pinnedPool().give(at, bytes);
-        at = nullptr;
-        bytes = 0;
-    }
+    void release() { pinnedPool().give(block); }
 };
 
 }  // namespace
@@ -201,8 +153,7 @@ struct DeviceRows::Dev {
     // changes while this object lives: the first use needs zeros and puts them back, the second leaves its tables
     // behind. `work_dirty` says that the last launch was of the second kind; the next one of the first kind clears
     // the buffer on the stream before it runs.
-    unsigned char* work = nullptr;
-    std::uint64_t work_cap = 0;
+    Block work;
     bool work_dirty = false;
 };
 
@@ -227,7 +178,7 @@ DeviceRows::~DeviceRows() {
     for (Pinned* p : {&dev_->rows_block, &dev_->hist_block, &dev_->bias_block, &dev_->topk_block, &dev_->row_block}) p->release();
     if (dev_->adjusted) (void)hipFree(dev_->adjusted);
     if (dev_->work_dirty || dev_->in_flight) zeroPool().drop(dev_->work);
-    else zeroPool().give(dev_->work, dev_->work_cap);
+    else zeroPool().give(dev_->work);
     delete dev_;
 }
 
@@ -280,7 +231,7 @@ void DeviceRows::uploadLists(std::uint32_t n) {
                           ids_b = Dev::up(std::size_t{n} * cap * sizeof(std::int32_t));
         d.row_cap = 0;
         d.rows_block.need(prm_b + res_b + done_b + 2 * ids_b);
-        unsigned char* at = d.rows_block.at;
+        unsigned char* at = d.rows_block.at();
         d.prm = at;
         d.res = at += prm_b;
         d.done = reinterpret_cast<std::uint32_t*>(at += res_b);
@@ -291,14 +242,14 @@ void DeviceRows::uploadLists(std::uint32_t n) {
         d.row_cap = n;
     }
     const std::size_t nh = adj_.n_history, nb = adj_.n_bias;
-    if (const std::size_t want = nh * n * sizeof(std::int32_t); want > d.hist_block.bytes) {
-        d.hist_block.need(std::max(want, 2 * d.hist_block.bytes));
-        d.hist = reinterpret_cast<std::int32_t*>(d.hist_block.at);
+    if (const std::size_t want = nh * n * sizeof(std::int32_t); want > d.hist_block.block.bytes) {
+        d.hist_block.need(std::max(want, 2 * d.hist_block.block.bytes));
+        d.hist = reinterpret_cast<std::int32_t*>(d.hist_block.at());
     }
-    if (const std::size_t want = 2 * Dev::up(nb * n * sizeof(float)); nb && want > d.bias_block.bytes) d.bias_block.need(std::max(want, 2 * d.bias_block.bytes));
+    if (const std::size_t want = 2 * Dev::up(nb * n * sizeof(float)); nb && want > d.bias_block.block.bytes) d.bias_block.need(std::max(want, 2 * d.bias_block.block.bytes));
     if (nb) {
-        d.bias_ids = reinterpret_cast<std::int32_t*>(d.bias_block.at);
-        d.bias_vals = reinterpret_cast<float*>(d.bias_block.at + Dev::up(nb * n * sizeof(float)));
+        d.bias_ids = reinterpret_cast<std::int32_t*>(d.bias_block.at());
+        d.bias_vals = reinterpret_cast<float*>(d.bias_block.at() + Dev::up(nb * n * sizeof(float)));
     }
     for (std::uint32_t r = 0; r < n; ++r) {
         if (nh) std::memcpy(d.hist + r * nh, adj_.history, nh * sizeof(std::int32_t));
@@ -370,26 +321,20 @@ void DeviceRows::filterOnDevice(const Sampler& s, std::uint32_t gr0, std::uint32
     // every row of the launch has the sampler's top-k: a bounded one takes the short-list kernel
     b.top_k_max = (s.top_k >= 1 && s.top_k <= 1024) ? static_cast<std::uint32_t>(s.top_k) : 0u;
     b.min_p_min = (s.top_k == 0 && s.min_p >= 1e-3) ? s.min_p : 0.0;  // (no top-k, but a floor that keeps the set small)
-    if (const std::uint64_t need = ws_sample_batch_workspace(&b); need > d.work_cap) {
+    if (const std::uint64_t need = ws_sample_batch_workspace(&b); need > d.work.bytes) {
         if (d.work_dirty) zeroPool().drop(d.work);
-        else zeroPool().give(d.work, d.work_cap);
-        d.work = nullptr;
-        d.work_cap = 0;
-        std::size_t got = 0;
-        bool fresh = true;
-        d.work = static_cast<unsigned char*>(zeroPool().take(need, got, fresh));
-        d.work_cap = got;
-        d.work_dirty = fresh;  // (fresh memory: whatever it holds)
+        else zeroPool().give(d.work);
+        d.work = zeroPool().take(need, d.work_dirty);  // (fresh memory: whatever it holds)
     }
     const int use = ws_sample_batch_workspace_use(&b);
     if (use == WS_WORK_MEETING && d.work_dirty) {
-        checkHip(hipMemsetAsync(d.work, 0, d.work_cap, stream), "hipMemsetAsync");
+        checkHip(hipMemsetAsync(d.work.at, 0, d.work.bytes, stream), "hipMemsetAsync");
         d.work_dirty = false;
     } else if (use == WS_WORK_TABLES) {
         d.work_dirty = true;
     }
-    b.workspace = d.work;
-    b.workspace_bytes = d.work_cap;
+    b.workspace = d.work.at;
+    b.workspace_bytes = d.work.bytes;
     d.in_flight = true;
     check(ws_sample_batch_notify(stream_, &b, d.done, ++d.turn), "ws_sample_batch");
     waitForRows(n);  // results and kept sets are in host memory now
@@ -539,9 +484,9 @@ void DeviceRows::escalate(Sampler& s, std::uint32_t gr) {
     }
     if (!d.topk_ids) {
         d.topk_block.need(kBig * 8 + 256);
-        d.topk_ids = reinterpret_cast<std::int32_t*>(d.topk_block.at);
-        d.topk_vals = reinterpret_cast<float*>(d.topk_block.at + kBig * 4);
-        d.topk_stats = reinterpret_cast<float*>(d.topk_block.at + kBig * 8);
+        d.topk_ids = reinterpret_cast<std::int32_t*>(d.topk_block.at());
+        d.topk_vals = reinterpret_cast<float*>(d.topk_block.at() + kBig * 4);
+        d.topk_stats = reinterpret_cast<float*>(d.topk_block.at() + kBig * 8);
     }
     Cand* c = room(s, std::min(kBig, vocab_));
     bool first = true;
@@ -579,7 +524,7 @@ const float* DeviceRows::loadFullRow(std::uint32_t gr) {
     if (gr >= rows_) throw DeviceError("loadFullRow", WS_E_INVALID, "loadFullRow: row out of range");
     if (!dev_->row_host) {
         dev_->row_block.need(vocab_ * sizeof(float));
-        dev_->row_host = reinterpret_cast<float*>(dev_->row_block.at);
+        dev_->row_host = reinterpret_cast<float*>(dev_->row_block.at());
     }
     auto stream = static_cast<hipStream_t>(stream_);
     const bool penalised = adj_.n_history || adj_.n_bias;
