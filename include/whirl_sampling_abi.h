@@ -78,6 +78,16 @@ int ws_argmax(void* stream, const float* x, int n, int* out, int* ids, int* pos,
 int ws_argmax_rows(void* stream, const float* x, int n, int* out, unsigned rows);
 /* argmax_rows_to(x, n, out, dst): sample_pick_set_tokens.h:47-53. Row b goes to out[dst->v[b]]; rows <= 32. */
 int ws_argmax_rows_to(void* stream, const float* x, int n, int* out, const ws_row_idx* dst, unsigned rows);
+/* The three with a workspace: few rows are then shared by 2 to 16 workgroups each (the reference, and the three above, give a row
+ * to one, which leaves most of a large GPU idle). Same picks. workspace: device memory of ws_argmax_workspace() bytes (16 a
+ * workgroup, which makes 4096 at most; 0: this shape is not shared), 8-byte aligned, of any contents, nobody else's until the launch is done: memory an
+ * allocator has just handed out will do, and a captured launch may be replayed. Without one, or for shapes that are not
+ * shared, these are the three above. */
+uint64_t ws_argmax_workspace(int n, unsigned rows);
+int ws_argmax_ws(void* stream, const float* x, int n, int* out, int* ids, int* pos, int advance, void* workspace, uint64_t workspace_bytes);
+int ws_argmax_rows_ws(void* stream, const float* x, int n, int* out, unsigned rows, void* workspace, uint64_t workspace_bytes);
+int ws_argmax_rows_to_ws(void* stream, const float* x, int n, int* out, const ws_row_idx* dst, unsigned rows, void* workspace,
+                         uint64_t workspace_bytes);
 /* argmax_prob(x, n, out_tok, out_prob): sample_pick_set_tokens.h:96-105. out_prob[0] = 1 / sum exp(x - max). */
 int ws_argmax_prob(void* stream, const float* x, int n, int* out_tok, float* out_prob);
 /* draft_pick(x, n, tok, prob, ctl, r, n_min, p_min, map): sample_pick_set_tokens.h:60-86. tok[r] = map ? map[top] : top,

@@ -182,3 +182,57 @@ def test_greedy_picks_shared_between_workgroups(rows, n):
                 assert np.array_equal(got.cpu().numpy(), want)
                 assert rows > 32 or np.array_equal(to.cpu().numpy()[1:rows + 1][::-1], want)
                 assert one.item() == ids.item() == want[rows - 1] and pos.item() == 7
+
+
+def test_greedy_picks_over_any_workspace_and_under_capture():
+    """The picks' workspace may hold anything when a launch begins - what the allocator left there, a launch of another shape, the
+    launch's own words of an earlier replay -, a stream beyond the 64th has the same kernel as the first, and so has a captured
+    one: replays over other logits, with other work on the memory between them, give every replay's picks."""
+    m = gc.pkg()
+    L = m.lib()
+    rng = np.random.default_rng(5)
+    rows, n = 8, 50257
+    xs = [torch.from_numpy((rng.standard_normal((rows, n)) * 2).astype(np.float32)).cuda() for _ in range(3)]
+    want = [x.argmax(dim=1).to(torch.int32) for x in xs]
+    need = int(L.ws_argmax_workspace(n, rows))
+    assert 0 < need <= 4096 and int(L.ws_argmax_workspace(4096, rows)) == 0
+    out = torch.empty(rows, dtype=torch.int32, device="cuda")
+    work = torch.empty(need // 8, dtype=torch.int64, device="cuda")
+
+    def pick(x, out, work, stream):
+        m.check(L.ws_argmax_rows_ws(stream, x.data_ptr(), n, out.data_ptr(), rows, work.data_ptr(), need), "ws_argmax_rows_ws")
+
+    here = torch.cuda.current_stream().cuda_stream
+    for k, fill in enumerate([0, -1, 0x7fffffffffffffff, None, None]):
+        if fill is not None:
+            work.fill_(fill)
+        elif k == 3:
+            work.copy_(torch.from_numpy(rng.integers(-2**62, 2**62, need // 8)))
+        pick(xs[k % 3], out, work, here)
+        assert torch.equal(out, want[k % 3]), k
+    for k in range(70):
+        s = torch.cuda.Stream()
+        with torch.cuda.stream(s):
+            got = m.argmax_rows(xs[k % 3])
+        s.synchronize()
+        assert torch.equal(got, want[k % 3])
+
+    x = xs[0].clone()
+    ids, pos = torch.zeros(1, dtype=torch.int32, device="cuda"), torch.zeros(1, dtype=torch.int32, device="cuda")
+    side = torch.cuda.Stream()
+    g = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        g.capture_begin()
+        got, one = m.argmax_rows(x), m.argmax(x[3], ids, pos, 1)
+        g.capture_end()
+        for k in range(6):
+            x.copy_(xs[k % 3])
+            g.replay()
+            side.synchronize()
+            assert torch.equal(got, want[k % 3]) and one.item() == ids.item() == want[k % 3][3].item() and pos.item() == k + 1, k
+    # without a workspace, or with too little of it: the kernel that gives a row to one workgroup
+    for w, b in ((None, 0), (work.data_ptr(), need - 1), (work.data_ptr() + 4, need)):
+        out.fill_(-1)
+        m.check(L.ws_argmax_rows_ws(here, xs[1].data_ptr(), n, out.data_ptr(), rows, w, b), "ws_argmax_rows_ws")
+        assert torch.equal(out, want[1])

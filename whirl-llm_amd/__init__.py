@@ -116,6 +116,10 @@ ABI = {
     "ws_argmax": (C.c_int, [C.c_void_p, C.c_void_p, C.c_int, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int]),
     "ws_argmax_rows": (C.c_int, [C.c_void_p, C.c_void_p, C.c_int, C.c_void_p, C.c_uint]),
     "ws_argmax_rows_to": (C.c_int, [C.c_void_p, C.c_void_p, C.c_int, C.c_void_p, C.POINTER(RowIdx), C.c_uint]),
+    "ws_argmax_workspace": (C.c_uint64, [C.c_int, C.c_uint]),
+    "ws_argmax_ws": (C.c_int, [C.c_void_p, C.c_void_p, C.c_int, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, C.c_void_p, C.c_uint64]),
+    "ws_argmax_rows_ws": (C.c_int, [C.c_void_p, C.c_void_p, C.c_int, C.c_void_p, C.c_uint, C.c_void_p, C.c_uint64]),
+    "ws_argmax_rows_to_ws": (C.c_int, [C.c_void_p, C.c_void_p, C.c_int, C.c_void_p, C.POINTER(RowIdx), C.c_uint, C.c_void_p, C.c_uint64]),
     "ws_argmax_prob": (C.c_int, [C.c_void_p, C.c_void_p, C.c_int, C.c_void_p, C.c_void_p]),
     "ws_draft_pick": (C.c_int, [C.c_void_p, C.c_void_p, C.c_int, C.c_void_p, C.c_void_p, C.c_void_p, C.c_int, C.c_int,
                                 C.c_float, C.c_void_p]),
@@ -212,26 +216,38 @@ def _row_idx(values):
     return ri
 
 
+# Workspace of a greedy pick (ws_argmax_workspace: 4096 bytes at most, of any contents). It is asked for with every call, in one
+# piece with the result where that is the call's own: torch's allocator hands memory out and takes it back in the order of the
+# stream, so that every stream, thread and captured graph has its own. (A piece of its own takes the host 0.8 us longer.)
+_PICK_WORDS, _PICK_BYTES = 1024, 4096
+
+
 def argmax_rows(x):
     """x: [rows, n] float32 device -> int32 [rows] (first index of each row's maximum)."""
     _dev_f32(x)
-    out = torch.empty(x.shape[0], dtype=torch.int32, device=x.device)
-    check(lib().ws_argmax_rows(_stream(), _p(x), x.shape[1], _p(out), x.shape[0]), "ws_argmax_rows")
-    return out
+    rows, n = x.shape
+    first = rows + (rows & 1)
+    out = torch.empty(first + _PICK_WORDS, dtype=torch.int32, device=x.device)  # the picks, and behind them the workspace
+    at = out.data_ptr()
+    check(lib().ws_argmax_rows_ws(_stream(), _p(x), n, at, rows, at + 4 * first, _PICK_BYTES), "ws_argmax_rows_ws")
+    return out.resize_(rows)
 
 
 def argmax(x, ids, pos, advance=1):
     """x: [n] row; ids, pos: int32 [1] device (next-step token / position, updated in place) -> int32 [1]."""
     _dev_f32(x)
-    out = torch.empty(1, dtype=torch.int32, device=x.device)
-    check(lib().ws_argmax(_stream(), _p(x), x.numel(), _p(out), _p(ids), _p(pos), advance), "ws_argmax")
-    return out
+    out = torch.empty(2 + _PICK_WORDS, dtype=torch.int32, device=x.device)
+    at = out.data_ptr()
+    check(lib().ws_argmax_ws(_stream(), _p(x), x.numel(), at, _p(ids), _p(pos), advance, at + 8, _PICK_BYTES), "ws_argmax_ws")
+    return out.resize_(1)
 
 
 def argmax_rows_to(x, out, dst):
     _dev_f32(x)
     ri = _row_idx(dst)
-    check(lib().ws_argmax_rows_to(_stream(), _p(x), x.shape[1], _p(out), C.byref(ri), x.shape[0]), "ws_argmax_rows_to")
+    rows, n = x.shape
+    work = torch.empty(_PICK_WORDS, dtype=torch.int32, device=x.device)
+    check(lib().ws_argmax_rows_to_ws(_stream(), _p(x), n, _p(out), C.byref(ri), rows, _p(work), _PICK_BYTES), "ws_argmax_rows_to_ws")
     return out
 
 

@@ -48,7 +48,7 @@ int launch_dflash_shared(hipStream_t stream, const float* x, int n, int ld, int 
 int launch_draft_shared(hipStream_t stream, const float* x, int n, int* ctl_all, const void* area, int r, const int* map, const void* args, int* qbuf,
                         unsigned rows, unsigned parts, unsigned chunk_log2, unsigned char* work);
 int launch_argmax_shared(hipStream_t stream, int mode, const float* x, int n, int* out, const void* dst, int* ids, int* pos, int advance, unsigned rows,
-                         unsigned parts, unsigned long long* scratch);
+                         unsigned parts, unsigned long long* scratch, unsigned long long tag);
 int prepare_top();
 }  // namespace ws
 
@@ -294,51 +294,26 @@ int scratch_address(unsigned char** out) {
     return WS_OK;
 }
 
-// Scratch of the greedy picks, whose entry points take no workspace: kPickStreams blocks of it in every GPU's copy of the code
-// object, each given to the first stream that asks and kept by it. Launches on one stream follow one another, so a block is
-// never in two launches at once; the streams beyond the first kPickStreams, the handle that names a stream per thread, and a
-// stream under capture (whose graph may be replayed on another) get none and take the kernels that need none.
-constexpr uint32_t kPickStreams = 64, kPickRows = 128;
-static __device__ __align__(256) unsigned char pick_scratch[kPickStreams * kPickRows * ws::kPickSplitRowBytes];
-std::atomic<unsigned char*> pick_scratch_at[64];
-std::atomic<uintptr_t> pick_owner[64][kPickStreams];  // [device][block]: the stream's handle, 1 for the null stream
-
-unsigned long long* pick_block(void* stream, unsigned rows) {
-    int dev = 0;
-    if (rows > kPickRows || stream == static_cast<void*>(hipStreamPerThread) || hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return nullptr;
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(S(stream), &cap) != hipSuccess) {
-        (void)hipGetLastError();
-        return nullptr;
-    }
-    if (cap != hipStreamCaptureStatusNone) return nullptr;
-    unsigned char* at = pick_scratch_at[dev].load(std::memory_order_acquire);
-    if (!at) {
-        void* sym = nullptr;
-        if (hipGetSymbolAddress(&sym, HIP_SYMBOL(pick_scratch)) != hipSuccess) {
-            (void)hipGetLastError();
-            return nullptr;
-        }
-        at = static_cast<unsigned char*>(sym);
-        pick_scratch_at[dev].store(at, std::memory_order_release);
-    }
-    const uintptr_t key = stream ? reinterpret_cast<uintptr_t>(stream) : 1u;
-    const uint32_t first = static_cast<uint32_t>((key >> 4) * 0x9E3779B1u) >> 26;
-    for (uint32_t i = 0; i < kPickStreams; ++i) {
-        const uint32_t b = (first + i) % kPickStreams;
-        uintptr_t owner = pick_owner[dev][b].load(std::memory_order_relaxed);
-        if (owner == 0 && pick_owner[dev][b].compare_exchange_strong(owner, key)) owner = key;
-        if (owner == key) return reinterpret_cast<unsigned long long*>(at + size_t{b} * kPickRows * ws::kPickSplitRowBytes);
-    }
-    return nullptr;
-}
-
 // workgroups a row of a greedy pick: within the compute units, at least 4096 tokens each
 unsigned argmax_parts(int n, unsigned rows) {
-    unsigned parts = rows ? static_cast<unsigned>(compute_units()) / rows : 0u;
+    if (rows == 0) return 0u;
+    unsigned parts = static_cast<unsigned>(compute_units()) / rows;
     if (parts > 16u) parts = 16u;
     if (parts > static_cast<unsigned>(n) / 4096u) parts = static_cast<unsigned>(n) / 4096u;
     return parts < 2u ? 0u : parts;
+}
+bool argmax_workspace_ok(const void* w, uint64_t bytes, int n, unsigned rows) {
+    return w && bytes >= ws_argmax_workspace(n, rows) && reinterpret_cast<uintptr_t>(w) % 8u == 0;
+}
+// another one for every launch of the process: the n-th output of the splitmix64 generator (a bijection of n), zero left out
+unsigned long long launch_tag() {
+    static std::atomic<uint64_t> launches{0};
+    for (;;) {
+        uint64_t z = (launches.fetch_add(1, std::memory_order_relaxed) + 1u) * 0x9E3779B97F4A7C15ull;
+        z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+        z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
+        if (z ^= z >> 31; z != 0) return z;
+    }
 }
 
 // the kernels launched from this file whose dynamic LDS goes beyond the default limit
@@ -402,26 +377,38 @@ int ws_probe(void) {
     return WS_OK;
 }
 
+uint64_t ws_argmax_workspace(int n, unsigned rows) { return n > 0 ? uint64_t{rows} * argmax_parts(n, rows) * 16u : 0ull; }
+
 int ws_argmax(void* stream, const float* x, int n, int* out, int* ids, int* pos, int advance) {
+    return ws_argmax_ws(stream, x, n, out, ids, pos, advance, nullptr, 0);
+}
+
+int ws_argmax_ws(void* stream, const float* x, int n, int* out, int* ids, int* pos, int advance, void* workspace, uint64_t workspace_bytes) {
     if (!x || !out || !ids || !pos || n <= 0) return WS_E_INVALID;
-    if (const unsigned parts = argmax_parts(n, 1u))
-        if (unsigned long long* scratch = pick_block(stream, 1u)) return ws::launch_argmax_shared(S(stream), 2, x, n, out, nullptr, ids, pos, advance, 1u, parts, scratch);
+    if (const unsigned parts = argmax_parts(n, 1u); parts && argmax_workspace_ok(workspace, workspace_bytes, n, 1u))
+        return ws::launch_argmax_shared(S(stream), 2, x, n, out, nullptr, ids, pos, advance, 1u, parts, static_cast<unsigned long long*>(workspace), launch_tag());
     hipLaunchKernelGGL(argmax, dim3(1), dim3(WS_BLOCK), 0, S(stream), x, n, out, ids, pos, advance);
     return done();
 }
 
-int ws_argmax_rows(void* stream, const float* x, int n, int* out, unsigned rows) {
+int ws_argmax_rows(void* stream, const float* x, int n, int* out, unsigned rows) { return ws_argmax_rows_ws(stream, x, n, out, rows, nullptr, 0); }
+
+int ws_argmax_rows_ws(void* stream, const float* x, int n, int* out, unsigned rows, void* workspace, uint64_t workspace_bytes) {
     if (!x || !out || n <= 0 || rows == 0) return WS_E_INVALID;
-    if (const unsigned parts = argmax_parts(n, rows))
-        if (unsigned long long* scratch = pick_block(stream, rows)) return ws::launch_argmax_shared(S(stream), 0, x, n, out, nullptr, nullptr, nullptr, 0, rows, parts, scratch);
+    if (const unsigned parts = argmax_parts(n, rows); parts && argmax_workspace_ok(workspace, workspace_bytes, n, rows))
+        return ws::launch_argmax_shared(S(stream), 0, x, n, out, nullptr, nullptr, nullptr, 0, rows, parts, static_cast<unsigned long long*>(workspace), launch_tag());
     hipLaunchKernelGGL(argmax_rows, dim3(rows), dim3(WS_BLOCK), 0, S(stream), x, n, out);
     return done();
 }
 
 int ws_argmax_rows_to(void* stream, const float* x, int n, int* out, const ws_row_idx* dst, unsigned rows) {
+    return ws_argmax_rows_to_ws(stream, x, n, out, dst, rows, nullptr, 0);
+}
+
+int ws_argmax_rows_to_ws(void* stream, const float* x, int n, int* out, const ws_row_idx* dst, unsigned rows, void* workspace, uint64_t workspace_bytes) {
     if (!x || !out || !dst || n <= 0 || rows == 0 || rows > WS_MAX_TABLE_ROWS) return WS_E_INVALID;
-    if (const unsigned parts = argmax_parts(n, rows))
-        if (unsigned long long* scratch = pick_block(stream, rows)) return ws::launch_argmax_shared(S(stream), 1, x, n, out, dst, nullptr, nullptr, 0, rows, parts, scratch);
+    if (const unsigned parts = argmax_parts(n, rows); parts && argmax_workspace_ok(workspace, workspace_bytes, n, rows))
+        return ws::launch_argmax_shared(S(stream), 1, x, n, out, dst, nullptr, nullptr, 0, rows, parts, static_cast<unsigned long long*>(workspace), launch_tag());
     RowIdx d;
     std::memcpy(&d, dst, sizeof d);
     hipLaunchKernelGGL(argmax_rows_to, dim3(rows), dim3(WS_BLOCK), 0, S(stream), x, n, out, d);

@@ -161,21 +161,34 @@ __global__ void __launch_bounds__(WS_BLOCK)
 #endif
 }
 
-// ---- greedy picks of few rows: every part leaves the largest {logit, lowest index} of its stretch as an order key (never
-// zero) in the row's 256 bytes of scratch, and the part that arrives last picks among them (a key still on its way reads as zero
-// and is read again) and puts the scratch back to zero. What bounds it: the stretch's loads (76 KB a compute unit at 32 rows of
-// 151936) and three trips to memory; 32 rows took 10.4 us with a compute unit a row.
-struct PickTable {
+// ---- greedy picks of few rows: every part leaves the largest {logit, lowest index} of its stretch as an order key in the row's
+// scratch, once as it is and once mixed with a tag that no other launch has, waits until both have arrived and looks at all
+// parts' places: where the two words of every part differ by the tag, everybody is there, and whoever sees that picks. The one
+// whose words come last sees it, others may as well and write the same. So the scratch may hold anything when the launch
+// begins, a caller need not clear or keep it, and no counter has to be reset. (What it holds by chance makes a pair of this tag
+// once in 2^64; the picker breaks the row's pairs, for a captured launch has its tag again at every replay.) What bounds it: the
+// stretch's loads (76 KB a compute unit at 32 rows of 151936) and two trips to memory; 32 rows took 10.4 us with a compute unit a
+// row, and take 6.5.
+struct PickArgs {  // (one argument of the launch: ten of them take the host 0.7 us longer)
+    const float* x;
+    int* out;
+    unsigned long long* scratch;
+    unsigned long long tag;
+    unsigned n, parts;
+    int* ids;
+    int* pos;
+    int advance;
+};
+struct PickArgsTo : PickArgs {
     RowIdx dst;  // argmax_rows_to: where each row's pick goes
 };
 template <int MODE>  // 0: out[row]; 1: out[dst.v[row]]; 2: one row, out[0], ids[0] and pos[0] += advance
-__global__ void __launch_bounds__(WS_BLOCK)
-    argmax_shared(const float* x, int n, int* out, PickTable table, int* ids, int* pos, int advance, unsigned parts, unsigned long long* scratch) {
+__global__ void __launch_bounds__(WS_BLOCK) argmax_shared(std::conditional_t<MODE == 1, PickArgsTo, PickArgs> A) {
     __shared__ unsigned long long red[WS_WAVES];
-    __shared__ uint32_t s_ticket;
-    const uint32_t row = blockIdx.y, part = blockIdx.x, t = threadIdx.x, lane = t & 63u, V = static_cast<uint32_t>(n);
-    const unsigned char* base = reinterpret_cast<const unsigned char*>(x + static_cast<size_t>(row) * V);
-    scratch += static_cast<size_t>(row) * (kPickSplitRowBytes / 8u);
+    const uint32_t row = blockIdx.y, part = blockIdx.x, t = threadIdx.x, lane = t & 63u, V = A.n, parts = A.parts;
+    const unsigned long long tag = A.tag;
+    const unsigned char* base = reinterpret_cast<const unsigned char*>(A.x + static_cast<size_t>(row) * V);
+    unsigned long long* scratch = A.scratch + static_cast<size_t>(row) * (2u * parts);
     const uint32_t nv = (V + 3u) / 4u, per = (nv + parts - 1u) / parts, j0 = min(part * per, nv), j1 = min(j0 + per, nv);
     float best = -INFINITY;
     uint32_t at = 0xffffffffu;
@@ -204,33 +217,44 @@ __global__ void __launch_bounds__(WS_BLOCK)
     const unsigned long long mine = wave_pick(best, at);
     if (lane == 0u) red[t >> 6] = mine;
     __syncthreads();
-    auto key_max = [](unsigned long long a, unsigned long long b) { return a > b ? a : b; };
+    if (t >= 64u) return;
+    auto word = [&](uint32_t p, uint32_t second) { return &scratch[2u * p + second]; };
     if (t == 0) {
         unsigned long long k = red[0];
 #pragma unroll
-        for (uint32_t w = 1; w < WS_WAVES; ++w) k = key_max(k, red[w]);
-        __hip_atomic_store(&scratch[part], k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        s_ticket = __hip_atomic_fetch_add(reinterpret_cast<uint32_t*>(scratch + 16), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        for (uint32_t w = 1; w < WS_WAVES; ++w) k = k > red[w] ? k : red[w];
+        __hip_atomic_store(word(part, 0u), k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(word(part, 1u), k ^ tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    __syncthreads();
-    if (s_ticket != parts - 1u || t >= 64u) return;
-    unsigned long long k = 1ull;
-    for (uint32_t tries = 0; tries < 4096u; ++tries) {
-        k = lane < parts ? __hip_atomic_load(&scratch[lane], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 1ull;
-        if (__ballot(k == 0ull) == 0ull) break;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (the wave's: both words have arrived before it looks at the others')
+    unsigned long long k = 0ull, k2 = tag;
+    if (lane < parts) {
+        k = __hip_atomic_load(word(lane, 0u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        k2 = __hip_atomic_load(word(lane, 1u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    if (lane < parts) __hip_atomic_store(&scratch[lane], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (lane == 16u) __hip_atomic_store(&scratch[16], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (__ballot((k ^ k2) != tag) != 0ull) return;  // somebody is still to come
+    if (MODE == 2) {  // (pos moves once: of several who see everybody, the one who takes the first pair apart)
+        bool mine_to_do = false;
+        if (lane == 0u) {
+            unsigned long long was = k2;
+            mine_to_do = __hip_atomic_compare_exchange_strong(word(0u, 1u), &was, 0ull, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        if (__ballot(mine_to_do) == 0ull) return;
+    }
+    if (lane < parts) {  // no pair of this tag is left behind
+        __hip_atomic_store(word(lane, 0u), 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(word(lane, 1u), 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
     const bool some = lane < parts;
     const unsigned long long r = wave_pick(some ? unkey32(static_cast<uint32_t>(k >> 32)) : -INFINITY, some ? 0xffffffffu - static_cast<uint32_t>(k) : 0xffffffffu);
     if (lane == 0u) {
         const uint32_t i = 0xffffffffu - static_cast<uint32_t>(r);
         const int id = i == 0xffffffffu ? 0 : static_cast<int>(i);  // (a row without a number: the first index)
-        if (MODE == 1) out[table.dst.v[row]] = id;
-        else out[row] = id;
+        if constexpr (MODE == 1) A.out[A.dst.v[row]] = id;
+        else A.out[row] = id;
         if (MODE == 2) {
-            ids[0] = id;
-            pos[0] += advance;
+            A.ids[0] = id;
+            A.pos[0] += A.advance;
         }
     }
 }

@@ -66,11 +66,16 @@ int launch_draft_shared(hipStream_t stream, const float* x, int n, int* ctl_all,
 }
 
 int launch_argmax_shared(hipStream_t stream, int mode, const float* x, int n, int* out, const void* dst, int* ids, int* pos, int advance, unsigned rows,
-                         unsigned parts, unsigned long long* scratch) {
-    PickTable t{};
-    if (mode == 1) __builtin_memcpy(&t.dst, dst, sizeof t.dst);
-    const auto f = mode == 0 ? argmax_shared<0> : (mode == 1 ? argmax_shared<1> : argmax_shared<2>);
-    hipLaunchKernelGGL(f, dim3(parts, rows), dim3(WS_BLOCK), 0, stream, x, n, out, t, ids, pos, advance, parts, scratch);
+                         unsigned parts, unsigned long long* scratch, unsigned long long tag) {
+    const PickArgs a{x, out, scratch, tag, static_cast<unsigned>(n), parts, ids, pos, advance};
+    const dim3 grid(parts, rows);
+    if (mode == 1) {
+        PickArgsTo to{a, {}};
+        __builtin_memcpy(&to.dst, dst, sizeof to.dst);
+        hipLaunchKernelGGL(argmax_shared<1>, grid, dim3(WS_BLOCK), 0, stream, to);
+    } else {
+        hipLaunchKernelGGL(mode == 0 ? argmax_shared<0> : argmax_shared<2>, grid, dim3(WS_BLOCK), 0, stream, a);
+    }
     return static_cast<int>(hipGetLastError());
 }
 
