@@ -236,3 +236,15 @@ def test_greedy_picks_over_any_workspace_and_under_capture():
         out.fill_(-1)
         m.check(L.ws_argmax_rows_ws(here, xs[1].data_ptr(), n, out.data_ptr(), rows, w, b), "ws_argmax_rows_ws")
         assert torch.equal(out, want[1])
+
+
+def test_greedy_pick_of_a_row_beyond_32_bit_offsets():
+    """2^30 + 12 tokens, the largest of them behind byte 2^32 of the row."""
+    m = gc.pkg()
+    n = (1 << 30) + 12
+    x = torch.zeros(n, dtype=torch.float32, device="cuda")
+    x[n - 5] = 1.0
+    x[7] = 0.5  # (where an offset that lost its 33rd bit would look)
+    ids, pos = torch.zeros(1, dtype=torch.int32, device="cuda"), torch.zeros(1, dtype=torch.int32, device="cuda")
+    assert m.argmax(x, ids, pos).item() == ids.item() == n - 5
+    assert m.argmax_rows(x.view(1, n)).item() == n - 5

@@ -294,9 +294,9 @@ int scratch_address(unsigned char** out) {
     return WS_OK;
 }
 
-// workgroups a row of a greedy pick: within the compute units, at least 4096 tokens each
+// workgroups a row of a greedy pick: within the compute units, at least 4096 tokens each (and byte offsets of 32 bits)
 unsigned argmax_parts(int n, unsigned rows) {
-    if (rows == 0) return 0u;
+    if (n >= (1 << 30) || rows == 0) return 0u;
     unsigned parts = static_cast<unsigned>(compute_units()) / rows;
     if (parts > 16u) parts = 16u;
     if (parts > static_cast<unsigned>(n) / 4096u) parts = static_cast<unsigned>(n) / 4096u;
