@@ -210,6 +210,26 @@ def _dsamp_struct(n):
     return st
 
 
+def _dsamp_args(args):
+    """DSampArgs of the rows' dicts, in one go; what a struct refuses and ctypes takes (integers that wrap, numbers beyond float32's
+    range) one by one."""
+    da = DSampArgs()
+    if not isinstance(args, (list, tuple)):
+        args = list(args)
+    if not args:
+        return da
+    try:
+        top_k, qoff, inv_t, top_p, min_p, key = zip(*map(_DSAMP_FIELDS, args))
+        _dsamp_struct(len(args)).pack_into(da, 0, *[a.get("on", 1) for a in args], *top_k, *qoff, *inv_t, *top_p, *min_p,
+                                           *[k & 0xFFFFFFFF for k in key], *[(k >> 32) & 0xFFFFFFFF for k in key])
+    except (struct.error, OverflowError):
+        for i, a in enumerate(args):
+            da.on[i], da.top_k[i], da.qoff[i] = a.get("on", 1), a["top_k"], a["qoff"]
+            da.inv_t[i], da.top_p[i], da.min_p[i] = a["inv_t"], a["top_p"], a["min_p"]
+            da.key_lo[i], da.key_hi[i] = a["key"] & 0xFFFFFFFF, (a["key"] >> 32) & 0xFFFFFFFF
+    return da
+
+
 def _row_idx(values):
     ri = RowIdx()
     ri.v[:len(values)] = values
@@ -288,11 +308,7 @@ def draft_pick_rows(x, ctl_all, area, r, n_min, p_min, vmap=None, workspace=None
 def draft_sample_rows(x, ctl_all, area, r, args, qbuf, vmap=None, workspace=None):
     """args: list of per-row dicts (on, top_k, qoff, inv_t, top_p, min_p, key). workspace: as for topk_rows (K = 32)."""
     _dev_f32(x)
-    ri, da = _row_idx(area), DSampArgs()
-    if args:
-        top_k, qoff, inv_t, top_p, min_p, key = zip(*map(_DSAMP_FIELDS, args))
-        _dsamp_struct(len(args)).pack_into(da, 0, *[a.get("on", 1) for a in args], *top_k, *qoff, *inv_t, *top_p, *min_p,
-                                           *[k & 0xFFFFFFFF for k in key], *[k >> 32 for k in key])
+    ri, da = _row_idx(area), _dsamp_args(args)
     if workspace is not None:
         check(lib().ws_draft_sample_rows_ws(_stream(), _p(x), x.shape[1], _p(ctl_all), C.byref(ri), r, _p(vmap), C.byref(da),
                                             _p(qbuf), x.shape[0], _p(workspace), workspace.numel()), "ws_draft_sample_rows_ws")
