@@ -39,3 +39,13 @@ def test_draft_arguments_that_are_refused():
         m._dsamp_args([dict(ROW), {k: v for k, v in ROW.items() if k != "min_p"}])
     with pytest.raises(TypeError):
         m._dsamp_args([dict(ROW, top_k=1.5)])
+
+
+def test_row_tables_from_any_iterable():
+    m = gpu_cases.pkg()
+    want = (C.c_int32 * 32)(*range(5, 25))
+    for values in (list(range(5, 25)), tuple(range(5, 25)), range(5, 25), iter(range(5, 25)), {v: 0 for v in range(5, 25)}):
+        assert list(m._row_idx(values).v) == list(want)
+    for values in (list(range(33)), iter(range(33))):
+        with pytest.raises(IndexError):
+            m._row_idx(values)

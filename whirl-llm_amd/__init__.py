@@ -232,7 +232,11 @@ def _dsamp_args(args):
 
 def _row_idx(values):
     ri = RowIdx()
-    ri.v[:len(values)] = values
+    if type(values) is list and len(values) <= 32:
+        ri.v[:len(values)] = values
+    else:
+        for i, v in enumerate(values):
+            ri.v[i] = v
     return ri
 
 
