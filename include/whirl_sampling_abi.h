@@ -323,7 +323,12 @@ typedef struct ws_batch {
                                    set as a top-k does: what passes lies within -ln(min_p) / inv_t of the row's maximum).
                                    With it - alone, or together with top_k_max for the rows that do have a top_k - the
                                    batch takes the short-list kernel. Useful from about 1e-3 upwards: a row whose floor
-                                   lets more than 4096 tokens through is handed back like one that breaks the word */
+                                   lets more than 4096 tokens through is handed back like one that breaks the word. A row
+                                   shared by n workgroups (few rows, see workspace) is dealt out to their 8 n waves, 32
+                                   neighbouring fp32 or 64 bf16 tokens at a time (128 or 256 where rows lie off the 16-byte
+                                   boundaries), and a wave lists at most 7648 / (8 n) tokens, rounded down: 59 of sixteen
+                                   workgroups, 478 of two. The row is handed back as soon as the floor - or the lower one that
+                                   goes by the largest logit a workgroup knows of when it lists - lets more through in one of them */
 } ws_batch;
 
 /* Bytes of device scratch ws_sample_batch needs for this batch shape (host-only computation). */

@@ -74,6 +74,34 @@ def test_min_p_without_a_top_k(min_p):
     run(case(4, 60001, top_k=0, min_p=min_p), max_differ=1, handed_back=1 if min_p < 0.1 else 0)
 
 
+@pytest.mark.parametrize("dtype,rows,V,slots,chunk", [("f32", 16, 32768, 59, 32), ("bf16", 16, 32768, 59, 64), ("f32", 127, 16384, 478, 32), ("f32", 16, 32769, 59, 128)])
+def test_a_waves_list_holds_what_the_header_says(dtype, rows, V, slots, chunk):
+    """Min-p rows of sixteen and of two parts whose floor lets through tokens of one wave's share alone: as many as the wave lists
+    at most, and one more, which hands the row back. Answers are the oracle's either way."""
+    m = gc.pkg()
+    rng = np.random.default_rng(slots)
+    c = case(rows, V, top_k=0, min_p=0.5, n_hist=0, n_bias=0)
+    waves = 8 * (16 if rows == 16 else 2)
+    ids = np.concatenate([np.arange(chunk) + chunk * (5 + waves * k) for k in range(1 + (slots + 1) // chunk)])  # of the wave 5 of the row
+    c["logits"][:] = -50.0 - 1e4 * rng.random((rows, V), dtype=np.float32)  # (far apart: no part lists more than a few of these)
+    c["inv_t"][:] = 1.0
+    c["top_p"][:] = 1.0
+    for r in range(rows):
+        n = slots + (r & 1)
+        c["logits"][r, rng.permutation(ids)[:n]] = rng.permutation(n).astype(np.float32) / (2 * n)  # (a floor of half lets 0.69 units through)
+    if dtype == "bf16":
+        c["logits"], c["dtype"] = gc.f32_to_bf16_bits(c["logits"]), "bf16"
+    d = gc.upload(c, hints=True, min_p_hint=True)
+    smp = gc.sampler_for(c, d, 1, kept_cap=1024)
+    for _ in range(2):
+        smp.run()
+    res = gc.compare_rows(c, smp, range(0, rows, 1 if rows == 16 else 9), 1)
+    assert res["differ"] == 0, res
+    back = (smp.flags.cpu().numpy() & m.FLAG_ROUTE_HANDED_BACK) != 0
+    assert np.array_equal(back, np.arange(rows) % 2 == 1), back
+    assert not smp.workspace.any().item()
+
+
 def test_long_histories_and_repeated_bias_entries():
     """9000 ids of few tokens, so that counts are in the hundreds, and bias lists that name tokens of the history, some of
     them three times (their values are added in the order of the list)."""
