@@ -423,17 +423,20 @@ __device__ __forceinline__ bool short_row(const BatchArgs& A, const uint32_t row
     uint32_t* cnt = reinterpret_cast<uint32_t*>(lds + A.lds_cnt);
     uint16_t* first = reinterpret_cast<uint16_t*>(cnt + A.patch_cap);
 
-    // The row in vectors. Without a mask the whole ones, and the few tokens behind them (none, of most vocabularies) one by one
-    // after the sweep; with one all of them, the last read where it ends with the row and moved down. (Either way for the registers'
-    // sake: moved vectors spill them in the unmasked bf16 kernel - 1000 rows of 24896: 118 us, now 72 -, clamped whole ones in
-    // the masked fp32 kernel - 1024 rows of 262144: 430 us and more against 390.)
-    const uint32_t nv = MASKED ? (V + TPV - 1u) / TPV : V / TPV, n_odd = MASKED ? 0u : V % TPV;
-    const uint32_t j_part = MASKED && V % TPV ? nv - 1u : 0xffffffffu;
+    // The row in vectors: the whole ones, and the few tokens behind them (none, of most vocabularies) one by one after the sweep.
+    // Masked fp32 rows: all of them, the last read where it ends with the row and moved down. (Either way for the registers'
+    // sake: moved vectors spill them in the bf16 kernels - unmasked, 1000 rows of 24896: 118 us against 72; masked, 300 rows of
+    // 151936: 102 against 89, 1024 of 262144: 445 against 411 -, clamped whole ones in the masked fp32 kernel - 300 rows of
+    // 151936: 99 us against 81, 1024 of 262144: 430 against 390.)
+    constexpr bool MOVED = MASKED && DT == 0;
+    const uint32_t nv = MOVED ? (V + TPV - 1u) / TPV : V / TPV, n_odd = MOVED ? 0u : V % TPV;
+    const uint32_t j_part = MOVED && V % TPV ? nv - 1u : 0xffffffffu;
     auto vector_at = [&](uint32_t j) __attribute__((always_inline)) {
-        if (MASKED) return row_vector<DT>(base, j, V);
+        if (MOVED) return row_vector<DT>(base, j, V);
         const LooseVec v = *reinterpret_cast<const LooseVec*>(base + min(j, nv - 1u) * 16u);
         return make_uint4(v.x, v.y, v.z, v.w);
     };
+    auto word_at = [&](uint32_t j) __attribute__((always_inline)) { return MOVED ? min(j * TPV, V - 1u) >> 5 : (min(j, nv - 1u) * TPV) >> 5; };
 
     // the head of the row is asked for before anything else
     // (every load of the row is unconditional, its index clamped to the row, and brings the vector's word of the allow
@@ -444,7 +447,7 @@ __device__ __forceinline__ bool short_row(const BatchArgs& A, const uint32_t row
     for (uint32_t k = 0; k < kShortHead; ++k) {
         const uint32_t j = k * WS_BLOCK + t;
         hq[k] = vector_at(j);
-        hna[k] = MASKED ? allow[min(j * TPV, V - 1u) >> 5] : 0xffffffffu;
+        hna[k] = MASKED ? allow[word_at(j)] : 0xffffffffu;
     }
     for (uint32_t b = t; b < 4096u; b += WS_BLOCK) head_cnt[b] = 0u;
     // (the tables of the touched tokens as well, while the parameters travel: their sizes are the launch's, not the row's)
@@ -569,7 +572,7 @@ __device__ __forceinline__ bool short_row(const BatchArgs& A, const uint32_t row
     // one vector: its tokens as floats, masked-out / touched / NaN ones as -inf
     auto unpack = [&](uint4 q, uint32_t na, uint32_t j, float (&x)[TPV]) {
         const uint32_t i0 = j * TPV;
-        if (MASKED && j_part != 0xffffffffu && j == j_part) q = part_vector<DT>(q, TPV - V % TPV);  // (uniform before per lane)
+        if (MOVED && j_part != 0xffffffffu && j == j_part) q = part_vector<DT>(q, TPV - V % TPV);  // (uniform before per lane)
         uint32_t invalid = 0u;  // bit e: token e does not count here
         if (MASKED) invalid = ~(na >> (i0 & 31u));
         if (n_touched) invalid |= touched[i0 >> 5] >> (i0 & 31u);
@@ -592,7 +595,7 @@ __device__ __forceinline__ bool short_row(const BatchArgs& A, const uint32_t row
         for (uint32_t k = 0; k < KB; ++k) {
             const uint32_t j = jbase + k * WS_BLOCK + t;
             q[k] = vector_at(j);
-            na[k] = MASKED ? allow[min(j * TPV, V - 1u) >> 5] : 0xffffffffu;
+            na[k] = MASKED ? allow[word_at(j)] : 0xffffffffu;
         }
     };
     load(qa, naa, jb);
@@ -733,7 +736,7 @@ __device__ __forceinline__ bool short_row(const BatchArgs& A, const uint32_t row
     if (n_odd && !not_mine && ref > -INFINITY) {  // uniform: the tokens behind the last whole vector
         float x = -INFINITY;
         const uint32_t id = nv * TPV + t;
-        if (t < n_odd && !(n_touched && ((touched[id >> 5] >> (id & 31u)) & 1u)))
+        if (t < n_odd && (!MASKED || ((allow[id >> 5] >> (id & 31u)) & 1u)) && !(n_touched && ((touched[id >> 5] >> (id & 31u)) & 1u)))
             x = fmaxf(DT == 0 ? reinterpret_cast<const float*>(base)[id] : bf16_to_f32(reinterpret_cast<const uint16_t*>(base)[id]), -INFINITY);
         if (t < n_odd) {
             const float a = fmaxf(__fsub_rn(x, ref), -1e30f);
