@@ -275,7 +275,8 @@ typedef struct ws_batch {
                                first use and leaves it alone afterwards: every launch leaves all of it zero-filled again,
                                so batches of any shape may follow each other on it (with kept_ids set the size asked for
                                includes a staging area per row; memory that holds only the rows' meeting places, 65792
-                               bytes a row, still lets them be shared);
+                               bytes a row, still lets them be shared; short-list rows ask for 65536 bytes, which the
+                               kernel that holds them in registers needs, and are shared with 33536 as well);
                                (b) rows of the kernels that sweep the row twice (long or unaligned vocabularies)
                                that have a history or a bias: the first sweep leaves the raw logits of those tokens
                                here (8 bytes per history / bias entry) instead of gathering them one by one, and
@@ -353,9 +354,10 @@ int ws_sample_batch_notify(void* stream, const ws_batch* b, uint32_t* done, uint
 /* ws_sample_batch for callers that cannot allocate device memory - code under HIP graph capture, tight serving loops,
  * harnesses that forbid it; it has no counterpart in the reference. The split rows of a small batch meet in memory that is
  * part of the library's code object on every GPU (WS_STATIC_SPLIT_ROWS rows of it, about 4 MiB, held until the process
- * ends) instead of b->workspace, which is ignored. Nothing is allocated or freed, here or in the kernels. Every batch the
- * library splits on its own fits (at most 64 rows are split); one that the caller's max_split would split into more rows
- * than that (65 to 128 rows in two parts each) is refused with WS_E_STATIC_LIMIT. The memory's address on a device is
+ * ends) instead of b->workspace, which is ignored. Nothing is allocated or freed, here or in the kernels. A batch the
+ * library would split on its own always goes through (rows that do not fit are not split: 64 do, of the short-list kinds
+ * - top_k_max, min_p_min - 125); one that the caller's max_split would split into more rows than fit (65 to 128 rows in two
+ * parts each, short-list rows from 126) is refused with WS_E_STATIC_LIMIT. The memory's address on a device is
  * looked up on the first call there (or by ws_probe): make that call before capturing a graph. All calls on one GPU
  * share this memory: two of them that run at the same time (different streams) race; on one stream they are safe, each
  * launch leaves the memory as the next needs it. (Only split rows use it: use (b) of b->workspace is off here. The

@@ -204,3 +204,105 @@ def test_unshared_rows_that_end_inside_a_vector(V, allowed, dtype):
     smp = gc.sampler_for(c, d, 1, kept_cap=1024, max_split=1).run()
     res = gc.compare_rows(c, smp, range(6), 1)
     assert res["differ"] <= (1 if dtype == "bf16" else 0) and res["exact"] + res["differ"] == 6, res
+
+
+def _odd(rows, V, dtype="f32", top_k=40, min_p=0.0, n_hist=700, n_bias=20, allowed=None):
+    c = gc.make_cfg2(rows=rows, V=V, n_hist=n_hist, n_bias=n_bias)
+    c["top_k"][:] = top_k
+    c["min_p"][:] = min_p
+    if dtype == "bf16":
+        c["logits"], c["dtype"] = gc.f32_to_bf16_bits(c["logits"]), "bf16"
+    if allowed is not None:
+        words = (V + 31) // 32
+        rng = np.random.default_rng(V)
+        c["allow"] = np.ascontiguousarray(np.packbits(rng.random((rows, words * 32)) < allowed, axis=1, bitorder="little").view(np.uint32))
+    return c
+
+
+# bytes a row of the short-list kernel's own shared rows (a workspace of this size holds nothing else)
+SHORT_ROW_BYTES = 4096 * 8 + 768
+
+
+@pytest.mark.parametrize("dtype,allowed", [("f32", None), ("f32", 0.3), ("bf16", None), ("bf16", 0.6)])
+@pytest.mark.parametrize("V,max_split", [(16384, 2), (20001, 2), (32770, 4), (65531, 4), (65543, 8), (131079, 16), (151937, 0)])
+def test_rows_shared_by_the_short_list_kernel(V, max_split, dtype, allowed):
+    """Slices that end inside a vector, a chunk, a mask word; two to sixteen parts; the workspace is one of these rows' alone, so
+    the kernel that holds shares in registers does not take them. Twice on one workspace, which is zero again afterwards."""
+    m = gc.pkg()
+    c = _odd(3, V, dtype, allowed=allowed)
+    d = gc.upload(c, hints=True)
+    smp = gc.sampler_for(c, d, 1, kept_cap=1024, max_split=max_split)
+    smp.workspace = torch.zeros(3 * SHORT_ROW_BYTES, dtype=torch.uint8, device="cuda")
+    assert int(m.lib().ws_sample_batch_workspace(smp.desc)) > smp.workspace.numel()
+    smp.desc.workspace, smp.desc.workspace_bytes = smp.workspace.data_ptr(), smp.workspace.numel()
+    for _ in range(2):
+        smp.run()
+        assert not smp.workspace.any().item()
+    res = gc.compare_rows(c, smp, range(3), 1)
+    assert res["exact"] == 3 and ((smp.flags.cpu().numpy() & m.FLAG_ROUTE_MASK) == m.FLAG_ROUTE_SHORT).all(), res
+
+
+@pytest.mark.parametrize("rows,V,parts", [(90, 151936, 2), (60, 262144, 4), (128, 131072, 2), (129, 131072, 1)])
+def test_rows_too_long_for_the_registers_are_shared_all_the_same(rows, V, parts):
+    """Row counts at which the compute units allow too few workgroups a row to hold it in registers."""
+    m = gc.pkg()
+    c = _odd(rows, V, top_k=50, n_hist=64, n_bias=0)
+    d = gc.upload(c, hints=True)
+    smp = gc.sampler_for(c, d, 1, kept_cap=64)
+    need = int(m.lib().ws_sample_batch_workspace(smp.desc))
+    assert need == (rows * SHORT_ROW_BYTES if parts > 1 else 0)
+    for _ in range(2):
+        smp.run()
+    res = gc.compare_rows(c, smp, range(0, rows, 17), 1)
+    assert res["differ"] == 0 and ((smp.flags.cpu().numpy() & m.FLAG_ROUTE_MASK) == m.FLAG_ROUTE_SHORT).all(), res
+    assert not smp.workspace.any().item()
+
+
+def test_shared_rows_with_histories_too_long_for_the_registers_kernel():
+    m = gc.pkg()
+    c = _odd(2, 100003, n_hist=10300, n_bias=50)
+    d = gc.upload(c, hints=True)
+    smp = gc.sampler_for(c, d, 1, kept_cap=1024)
+    assert int(m.lib().ws_sample_batch_workspace(smp.desc)) == 2 * SHORT_ROW_BYTES
+    for _ in range(2):
+        smp.run()
+    assert gc.compare_rows(c, smp, range(2), 1)["exact"] == 2 and not smp.workspace.any().item()
+
+
+def test_shared_rows_that_are_handed_back_leave_the_workspace_zero():
+    """Parts whose lists run over beside parts that have listed theirs, a slice without a token, a row that breaks the word: handed
+    back, answered as the oracle does, and the workspace is zero for the rows of the next launch."""
+    m = gc.pkg()
+    c = _odd(100, 131072, top_k=30, n_hist=0, n_bias=0)
+    c["logits"][1, 65536:] = 3.0                  # the second part's tokens are all equal: its list runs over
+    c["logits"][2, :] = -7.5
+    c["logits"][3, 65536:] = -np.inf
+    c["top_k"][4], c["min_p"][4] = 0, 0.0
+    d = gc.upload(c, hints=True)
+    d["top_k_max"] = 30
+    smp = gc.sampler_for(c, d, 1, kept_cap=1024)
+    assert int(m.lib().ws_sample_batch_workspace(smp.desc)) == 100 * SHORT_ROW_BYTES
+    for _ in range(2):
+        smp.run()
+        assert not smp.workspace.any().item()
+    res = gc.compare_rows(c, smp, list(range(8)) + [99], 1)
+    assert res["differ"] <= 1, res
+    back = (smp.flags.cpu().numpy() & m.FLAG_ROUTE_HANDED_BACK) != 0
+    assert back[1] and back[2] and back[3] and back[4] and not back[5:].any(), np.nonzero(back)
+
+
+@pytest.mark.parametrize("rows", [65, 125, 126])
+def test_static_entry_point_with_two_parts_a_row(rows):
+    """A caller's max_split of 2: up to 125 short-list rows fit the library's own workspace (33 536 bytes each), more are refused."""
+    m = gc.pkg()
+    c = _odd(rows, 65536, n_hist=64, n_bias=0)
+    d = gc.upload(c, hints=True)
+    smp = gc.sampler_for(c, d, 1, kept_cap=64, max_split=2)
+    if rows > 125:
+        with pytest.raises(m.WsError, match="own workspace"):
+            smp.run_static()
+        smp.desc.max_split = 0  # the library's own choice always goes through
+    for _ in range(2):
+        smp.run_static()
+    res = gc.compare_rows(c, smp, range(0, rows, 13), 1)
+    assert res["differ"] == 0, res

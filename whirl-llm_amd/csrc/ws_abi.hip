@@ -35,7 +35,7 @@ int prepare_fused_kept(unsigned lds_limit);
 int prepare_split_kept(unsigned lds_limit);
 int prepare_lean(unsigned lds_limit);
 // ws_short.hip: the short-list kernel for batches whose rows all have a bounded top-k
-int launch_short(hipStream_t stream, const BatchArgs& a, unsigned blocks, unsigned lds_bytes, unsigned lds_limit);
+int launch_short(hipStream_t stream, const BatchArgs& a, unsigned lds_bytes, unsigned lds_limit);
 int prepare_short(unsigned lds_limit);
 // ws_few.hip: the same rows shared between workgroups that hold them in registers
 int launch_few(hipStream_t stream, const BatchArgs& a, unsigned lds_bytes, unsigned lds_limit);
@@ -109,13 +109,29 @@ int compute_units() {
     return n > 0 ? n : 0;
 }
 
+// Short-list rows that ws_few.h does not take - too long for the registers of as many workgroups as there are compute units
+// for, or with histories too long for its lists - shared by the short-list kernel's own workgroups, which sweep a slice each: 2^n
+// of them, 16 at most, of at least 8192 tokens, within the compute units (a second round of workgroups is not worth it).
+// Unshared and shared microseconds, top-k 50 with 1000-id histories: 60 rows of 262144 fp32 47.0 / 35.0, 90 of 151936 36.7 /
+// 33.4, 120 of 262144 48.9 / 44.0; min-p alone: 90 of 262144 65.7 / 48.0; 64 of 151936 with 8192 ids each 42.3 / 34.1.
+uint32_t short_split_log2(const ws_batch* b) {
+    if (b->max_split == 1u) return 0u;
+    const uint32_t cus = static_cast<uint32_t>(compute_units()), most = b->max_split ? b->max_split : 16u;
+    uint32_t lg = 0;
+    while (lg < 4u && (2u << lg) <= most && uint64_t{b->rows} * (2u << lg) <= cus && b->vocab / (2u << lg) >= 8192u) ++lg;
+    return lg;
+}
+
 // Few rows of the short-list kind: how many workgroups share a row. A share fits the registers of 512 threads (80 tokens
 // each) and has 2048 tokens at least; as many parts as the compute units allow, up to 16 - a wide top-k gets 8 at most, its
 // waves' lists need the room. Where the compute units allow fewer parts than that takes, shares of 112 tokens a thread are
 // tried (two parts hold 114688 tokens, three 172032: unshared and shared microseconds, top-k 40: 90 rows of 82000 fp32
 // 23.3 / 18.9, 70 of 151936 33.2 / 25.3, 90 of 92736 bf16 32 / 17). More workgroups than compute units: nobody waits for
 // anybody, but the second round of them costs more than it saves (181 rows of 44992 fp32 22.4 / 32.7, 160 of 82000 bf16
-// 29 / 32), bf16 rows of 130000 tokens and more aside (90 rows of 151936 38.8 / 32.7, 60 of 220032 44.7 / 29.0).
+// 29 / 32), bf16 rows aside whose slices in the short-list kernel would be longer than 90000 tokens: two rounds take 35 to 39 us
+// whatever the length, such a slice more and more (bf16, top-k 50, its slices and two rounds here: 86 rows of 131072 30.3 / 37.3, 86
+// of 151936 35.4 / 36.3, 66 of 200000 38.5 / 34.5, 86 of 200000 38.9 / 38.2, 64 of 262144 - slices of 65536 - 32.0 / 37.3, 73
+// of 262144 42.7 / 39.2).
 void few_plan(const ws_batch* b, uint64_t cap, uint64_t maps, BatchPlan& p) {
     p.few_parts = 0;
     if (b->max_split == 1u || cap > ws::kFewLists) return;
@@ -129,7 +145,7 @@ void few_plan(const ws_batch* b, uint64_t cap, uint64_t maps, BatchPlan& p) {
     if (parts > b->vocab / 2048u) parts = b->vocab / 2048u;
     if (parts < least && (parts < 2u || uint64_t{parts} * ws::kFewWide < b->vocab)) parts = least;
     if (cap > uint64_t{parts} * 1600u) return;  // (touched tokens of a share: room for 2048)
-    const bool twice = b->dtype == WS_DTYPE_BF16 && b->vocab >= 130000u;
+    const bool twice = b->dtype == WS_DTYPE_BF16 && b->vocab >> short_split_log2(b) > 90000u;
     if (parts < 2u || parts > most || static_cast<uint64_t>(b->rows) * parts > (twice ? 2ull : 1ull) * cus) return;
     const uint64_t three = (cap * 8u > 65536u ? ((cap * 8u + 15u) & ~uint64_t{15}) : 65536u) + maps;
     const uint64_t own = 32768u + (parts < least ? ws::kFewWide : ws::kFewShare) * 2u;
@@ -140,7 +156,8 @@ void few_plan(const ws_batch* b, uint64_t cap, uint64_t maps, BatchPlan& p) {
     p.workspace = p.workspace_min = uint64_t{b->rows} * ws::kFewRowBytes;
 }
 
-BatchPlan plan_batch(const ws_batch* b) {
+// few: whether ws_few.h is considered
+BatchPlan plan_batch(const ws_batch* b, bool few = true) {
     BatchPlan p{};
     p.err = WS_E_INVALID;
     if (!b || !b->logits || !b->inv_t || !b->seed || !b->step || !b->token || !b->flags) return p;
@@ -241,7 +258,8 @@ BatchPlan plan_batch(const ws_batch* b) {
         p.lean = false;
         p.split_log2 = 0;
         p.workspace = p.workspace_min = 0;
-        few_plan(b, cap, maps, p);
+        if (few) few_plan(b, cap, maps, p);
+        if (!p.few_parts && (p.split_log2 = short_split_log2(b)) != 0u) p.workspace = p.workspace_min = uint64_t{b->rows} * ws::kShortSplitRowBytes;
         p.err = WS_OK;
         return p;
     }
@@ -593,6 +611,12 @@ bool split_fits(const BatchPlan& p, const unsigned char* work, uint64_t work_byt
     return p.workspace_min && work && work_bytes >= p.workspace_min && reinterpret_cast<uintptr_t>(work) % 8u == 0;
 }
 
+// the plan for a workspace of this size: rows of ws_few.h need twice the memory of the short-list kernel's own shared rows
+BatchPlan plan_for(const ws_batch* b, uint64_t work_bytes) {
+    const BatchPlan p = plan_batch(b);
+    return p.err == WS_OK && p.few_parts && work_bytes < p.workspace_min ? plan_batch(b, false) : p;
+}
+
 // done: a word per row that gets `value` once the row's results are visible to the host, or nullptr (ws_sample_batch_notify)
 int sample_batch_on(void* stream, const ws_batch* b, const BatchPlan& p, unsigned char* work, uint64_t work_bytes, uint32_t* done_at = nullptr,
                     uint32_t done_value = 0u) {
@@ -663,8 +687,8 @@ int sample_batch_on(void* stream, const ws_batch* b, const BatchPlan& p, unsigne
         a.lds_cnt = p.short_cnt;
         a.fb_lds_tie = p.short_fb_tie;
         a.fb_lds_ab = p.short_fb_ab;
-        a.work = nullptr;
-        return ws::launch_short(S(stream), a, b->rows, p.short_total, kMaxLds - kStaticShort);
+        a.work = a.split_log2 ? work : nullptr;
+        return ws::launch_short(S(stream), a, p.short_total, kMaxLds - kStaticShort);
     }
     if (p.fused && a.split_log2)
         return (a.kept_ids ? ws::launch_split_kept : ws::launch_split)(S(stream), a, b->rows << a.split_log2, p.lds_total, kMaxLds - kStaticLds);
@@ -683,14 +707,14 @@ int sample_batch_on(void* stream, const ws_batch* b, const BatchPlan& p, unsigne
 }  // namespace
 
 int ws_sample_batch(void* stream, const ws_batch* b) {
-    const BatchPlan p = plan_batch(b);
+    const BatchPlan p = plan_for(b, b ? b->workspace_bytes : 0);
     if (p.err != WS_OK) return p.err;
     return sample_batch_on(stream, b, p, static_cast<unsigned char*>(b->workspace), b->workspace_bytes);
 }
 
 int ws_sample_batch_notify(void* stream, const ws_batch* b, uint32_t* done, uint32_t value) {
     if (!done) return WS_E_INVALID;
-    const BatchPlan p = plan_batch(b);
+    const BatchPlan p = plan_for(b, b ? b->workspace_bytes : 0);
     if (p.err != WS_OK) return p.err;
     unsigned char* work = static_cast<unsigned char*>(b->workspace);
     if (const int e = sample_batch_on(stream, b, p, work, b->workspace_bytes, done, value); e != WS_OK) return e;
@@ -701,11 +725,11 @@ int ws_sample_batch_notify(void* stream, const ws_batch* b, uint32_t* done, uint
 }
 
 int ws_sample_batch_static(void* stream, const ws_batch* b) {
-    const BatchPlan p = plan_batch(b);
+    const BatchPlan p = plan_for(b, sizeof(scratch));
     if (p.err != WS_OK) return p.err;
     if (!p.fused && !p.shortlist) return sample_batch_on(stream, b, p, nullptr, 0);  // (nothing may be left in the split rows' memory)
     if (p.workspace_min > sizeof(scratch)) {  // more split rows than the library's own memory holds
-        if (p.few_parts && b->max_split == 0u) return sample_batch_on(stream, b, p, nullptr, 0);  // (split by the library's own choice: not here)
+        if (p.shortlist && b->max_split == 0u) return sample_batch_on(stream, b, p, nullptr, 0);  // (split by the library's own choice: not here)
         return WS_E_STATIC_LIMIT;
     }
     unsigned char* at = nullptr;

@@ -402,8 +402,8 @@ __device__ __forceinline__ void short_rules(uint64_t* list, const uint32_t row, 
 // tokens, its 16-bit popcount prefixes, and at lds_cnt the per-rank words {history count | bias entries << 20 | claimed}
 // and 16-bit indices of each rank's first bias entry.
 // Returns false when the row has to go to the three-pass code (uniform over the workgroup; nothing has been written for it).
-template <int DT, bool MASKED>
-__device__ __forceinline__ bool short_row(const BatchArgs& A, const uint32_t row, ShortShared& S) {
+template <int DT, bool MASKED, bool SHARED>
+__device__ __forceinline__ bool short_row(const BatchArgs& A, const uint32_t row, const uint32_t part, const uint32_t n_parts, ShortShared& S, bool& finisher) {
 #ifdef WS_SHORT_TIMERS
     const long long wss_t0 = clock64();
     if (threadIdx.x == 0) S.marks[13] = 0.f;
@@ -431,21 +431,27 @@ __device__ __forceinline__ bool short_row(const BatchArgs& A, const uint32_t row
     constexpr bool MOVED = MASKED && DT == 0;
     const uint32_t nv = MOVED ? (V + TPV - 1u) / TPV : V / TPV, n_odd = MOVED ? 0u : V % TPV;
     const uint32_t j_part = MOVED && V % TPV ? nv - 1u : 0xffffffffu;
+    // the vectors [j0, j1) and the tokens of this workgroup: the row, or a shared row's slice
+    const uint32_t nvp = SHARED ? (nv + n_parts - 1u) / n_parts : nv, j0 = SHARED ? min(part * nvp, nv) : 0u, j1 = SHARED ? min(j0 + nvp, nv) : nv;
+    const uint32_t tok0 = j0 * TPV, tok1 = SHARED && part != n_parts - 1u ? j1 * TPV : V, n_tok = tok1 - tok0;
+    finisher = !SHARED;
     auto vector_at = [&](uint32_t j) __attribute__((always_inline)) {
-        if (MOVED) return row_vector<DT>(base, j, V);
-        const LooseVec v = *reinterpret_cast<const LooseVec*>(base + min(j, nv - 1u) * 16u);
+        if (MOVED) return row_vector<DT>(base, SHARED ? min(j, j1 - 1u) : j, V);
+        const LooseVec v = *reinterpret_cast<const LooseVec*>(base + min(j, j1 - 1u) * 16u);
         return make_uint4(v.x, v.y, v.z, v.w);
     };
-    auto word_at = [&](uint32_t j) __attribute__((always_inline)) { return MOVED ? min(j * TPV, V - 1u) >> 5 : (min(j, nv - 1u) * TPV) >> 5; };
+    auto word_at = [&](uint32_t j) __attribute__((always_inline)) {
+        return MOVED ? min((SHARED ? min(j, j1 - 1u) : j) * TPV, V - 1u) >> 5 : (min(j, j1 - 1u) * TPV) >> 5;
+    };
 
-    // the head of the row is asked for before anything else
-    // (every load of the row is unconditional, its index clamped to the row, and brings the vector's word of the allow
+    // the head of the slice is asked for before anything else
+    // (every load of the row is unconditional, its index clamped to the slice, and brings the vector's word of the allow
     // mask with it: a load behind a branch makes the compiler wait for every load before it)
     uint4 hq[kShortHead];
     uint32_t hna[kShortHead];
 #pragma unroll
     for (uint32_t k = 0; k < kShortHead; ++k) {
-        const uint32_t j = k * WS_BLOCK + t;
+        const uint32_t j = j0 + k * WS_BLOCK + t;
         hq[k] = vector_at(j);
         hna[k] = MASKED ? allow[word_at(j)] : 0xffffffffu;
     }
@@ -589,7 +595,7 @@ __device__ __forceinline__ bool short_row(const BatchArgs& A, const uint32_t row
     constexpr uint32_t KB = 4;  // vectors a thread and batch, two batches in flight
     uint4 qa[KB], qb[KB];
     uint32_t naa[KB], nab[KB];
-    const uint32_t jb = kShortHead * WS_BLOCK;
+    const uint32_t jb = j0 + kShortHead * WS_BLOCK;
     auto load = [&](uint4 (&q)[KB], uint32_t (&na)[KB], uint32_t jbase) __attribute__((always_inline)) {
 #pragma unroll
         for (uint32_t k = 0; k < KB; ++k) {
@@ -603,13 +609,13 @@ __device__ __forceinline__ bool short_row(const BatchArgs& A, const uint32_t row
 
     // ---- the threshold: the head's logits counted in 4096 bins of 1/64 e-fold below the head's maximum
     float ref = -INFINITY;
-    const uint32_t n_head_vec = min(nv, kShortSample * WS_BLOCK);
+    const uint32_t n_head_vec = min(j1 - j0, kShortSample * WS_BLOCK);
     {
         float x[TPV];
 #pragma unroll
         for (uint32_t k = 0; k < kShortSample; ++k) {
-            const uint32_t j = k * WS_BLOCK + t;
-            if (j < nv) {
+            const uint32_t j = j0 + k * WS_BLOCK + t;
+            if (j < j1) {
                 unpack(hq[k], hna[k], j, x);
 #pragma unroll
                 for (uint32_t e = 0; e < TPV; ++e) ref = fmaxf(ref, x[e]);
@@ -620,16 +626,19 @@ __device__ __forceinline__ bool short_row(const BatchArgs& A, const uint32_t row
     const float c64 = inv_t * 64.f;
     float thr = -INFINITY;  // tokens above it are listed
     // tokens to list: the count above a threshold fitted to a sample of the row scatters like the square root of the
-    // sample's rank: half of top_k on top, 150 at least
-    const uint32_t n_head = n_head_vec == nv ? V : min(n_head_vec * TPV, V);
+    // sample's rank: half of top_k on top, 150 at least; of a slice its share of those. (A slice that is the sample itself: the
+    // count is exact but for a bin's tokens, and what matters is that no part holds more of the row's top_k than it lists.)
+    const uint32_t n_head = n_head_vec == j1 - j0 ? n_tok : min(n_head_vec * TPV, n_tok);
     // (a head that is the whole row: the count is exact but for the tokens of a bin, and twice top_k will do. 156 rows of
     // 24896, Zipfian, top-k 25: 30.6 us with 191 tokens to list, most of them in a second round of counting, 21 with 56)
-    const uint32_t want = min(n_head >= V ? 2u * top_k + 6u : 0xffffffffu, top_k + max(top_k >> 1, 150u) + 16u);
-    bool list_all = by_k && n_head >= V && want >= V;
+    const uint32_t want = !SHARED ? min(n_head >= V ? 2u * top_k + 6u : 0xffffffffu, top_k + max(top_k >> 1, 150u) + 16u)
+                          : n_head >= n_tok ? 2u * ((top_k + n_parts - 1u) / n_parts) + 6u
+                                            : (top_k + max(top_k >> 1, 150u) + n_parts - 1u) / n_parts + 16u;
+    bool list_all = by_k && n_head >= n_tok && want >= n_tok;
     if (by_p && ref > -INFINITY) thr = __fadd_rn(ref, __fdiv_rn(static_cast<float>(log(min_p)) - 0.02f, inv_t));  // (0.02 e-folds below the floor: roundings)
     if (!not_mine && by_k && ref > -INFINITY && !list_all) {
-        // rank in the head that about `want` tokens of the row lie above
-        const uint64_t r_star64 = (static_cast<uint64_t>(n_head) * want + V - 1u) / V;
+        // rank in the head that about `want` tokens of the slice lie above
+        const uint64_t r_star64 = (static_cast<uint64_t>(n_head) * want + n_tok - 1u) / n_tok;
         const uint32_t r_star = static_cast<uint32_t>(r_star64 < 4u ? 4u : r_star64);
         // The bins near the top are all that matters (the r_star-th largest of the head is one of its largest per cent
         // or so): first only the tokens within 8 e-folds of the head's maximum are counted - an LDS atomic each, and a
@@ -641,8 +650,8 @@ __device__ __forceinline__ bool short_row(const BatchArgs& A, const uint32_t row
             float x[TPV];
 #pragma unroll
             for (uint32_t k = 0; k < kShortSample; ++k) {
-                const uint32_t j = k * WS_BLOCK + t;
-                if (j < nv) {
+                const uint32_t j = j0 + k * WS_BLOCK + t;
+                if (j < j1) {
                     unpack(hq[k], hna[k], j, x);
 #pragma unroll
                     for (uint32_t e = 0; e < TPV; ++e) {
@@ -713,18 +722,18 @@ __device__ __forceinline__ bool short_row(const BatchArgs& A, const uint32_t row
     if (!not_mine && ref > -INFINITY) {  // (a head without any token: the row goes the other way)
 #pragma unroll
         for (uint32_t k = 0; k < kShortHead; ++k) {
-            const uint32_t j = k * WS_BLOCK + t;
-            if (j < nv) take(hq[k], hna[k], j);
+            const uint32_t j = j0 + k * WS_BLOCK + t;
+            if (j < j1) take(hq[k], hna[k], j);
         }
         auto eat = [&](const uint4 (&q)[KB], const uint32_t (&na)[KB], uint32_t jbase) __attribute__((always_inline)) {
 #pragma unroll
             for (uint32_t k = 0; k < KB; ++k) {
                 const uint32_t j = jbase + k * WS_BLOCK + t;
-                if (j < nv) take(q[k], na[k], j);
+                if (j < j1) take(q[k], na[k], j);
             }
         };
-        if (jb < nv) {
-            for (uint32_t jc = jb; jc < nv; jc += 2u * KB * WS_BLOCK) {
+        if (jb < j1) {
+            for (uint32_t jc = jb; jc < j1; jc += 2u * KB * WS_BLOCK) {
                 eat(qa, naa, jc);
                 load(qa, naa, jc + 2u * KB * WS_BLOCK);
                 eat(qb, nab, jc + KB * WS_BLOCK);
@@ -733,7 +742,7 @@ __device__ __forceinline__ bool short_row(const BatchArgs& A, const uint32_t row
         }
     }
 
-    if (n_odd && !not_mine && ref > -INFINITY) {  // uniform: the tokens behind the last whole vector
+    if (n_odd && tok1 == V && !not_mine && ref > -INFINITY) {  // uniform: the tokens behind the last whole vector
         float x = -INFINITY;
         const uint32_t id = nv * TPV + t;
         if (t < n_odd && (!MASKED || ((allow[id >> 5] >> (id & 31u)) & 1u)) && !(n_touched && ((touched[id >> 5] >> (id & 31u)) & 1u)))
@@ -774,7 +783,7 @@ __device__ __forceinline__ bool short_row(const BatchArgs& A, const uint32_t row
             for (uint32_t k = 0; k < KS; ++k) {
                 old[k] = kClaim;
                 r[k] = 0u;
-                if (k * WS_BLOCK < n_live && id[k] < V) {
+                if (k * WS_BLOCK < n_live && id[k] < tok1 && (!SHARED || id[k] >= tok0)) {
                     r[k] = rank(id[k]);
                     old[k] = atomicOr(&cnt[r[k]], kClaim);
                 }
@@ -847,15 +856,100 @@ __device__ __forceinline__ bool short_row(const BatchArgs& A, const uint32_t row
     WSS_MARK(9);
     uint32_t n_list = S.s_w[1];
     bool bad = not_mine || S.s_w[2] != 0u || n_list > kShortCap || !(ref > -INFINITY) || !(m > -INFINITY) || !(__fsub_rn(m, ref) * inv_t < 80.f);
-    WSS_MARK(5);
+    float thr_max = thr;
+
+    // ---- a shared row: the parts' lists, maxima and sums meet in the row's workspace; the last one to arrive goes on
+    if constexpr (SHARED) {
+        unsigned char* work = A.work + static_cast<size_t>(row) * kShortSplitRowBytes;
+        unsigned long long* glist = reinterpret_cast<unsigned long long*>(work);
+        uint32_t* ctrl = reinterpret_cast<uint32_t*>(work + kShortSplitCtrl);
+        const uint32_t region = kShortCap / n_parts;  // every part has its own stretch of the list: nothing to reserve
+        if (n_list > region) bad = true;
+        if (t == 0) {
+            uint32_t* mine = ctrl + 64u + 8u * part;
+            __hip_atomic_store(&mine[0], key32(m), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(&mine[1], key32(thr), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            // the sum as it is, against the part's `ref`, and `ref` with it (against the `ref` of a bad part it may not be a number)
+            __hip_atomic_store(reinterpret_cast<unsigned long long*>(&mine[2]), static_cast<unsigned long long>(__double_as_longlong(bad ? 0.0 : z)), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(&mine[4], bad ? 0xffffffffu : n_list, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(&mine[5], key32(ref), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        if (!bad)
+            for (uint32_t k = t; k < n_list; k += WS_BLOCK)
+                __hip_atomic_store(&glist[part * region + k], static_cast<unsigned long long>(list[k]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        // (device-scope accesses and this wait make the meeting sound without a release or an acquire, which would write back and
+        // invalidate whole caches: as in ws_few.h)
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();  // every wave's stores have arrived
+        if (t == 0) S.s_w[5] = __hip_atomic_fetch_add(&ctrl[0], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        if (S.s_w[5] != n_parts - 1u) return true;  // not the last: done
+        finisher = true;
+        // The keys are asked for right away, every place of every stretch: which of them count is known when the parts' words
+        // are in. Lane p of the first wave reads part p's.
+        constexpr uint32_t kSlots = kShortCap / WS_BLOCK;
+        uint64_t got[kSlots];
+#pragma unroll
+        for (uint32_t i = 0; i < kSlots; ++i) got[i] = __hip_atomic_load(&glist[i * WS_BLOCK + t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();  // (everybody is done with its own list)
+        if (wv == 0u) {   // (one wave: sixteen doing the same arithmetic side by side take four times as long)
+            float mp = -INFINITY, tp = -INFINITY, rp = -INFINITY;
+            double zp = 0.0;
+            uint32_t np = 0u;
+            if (lane < n_parts) {
+                const uint32_t* words = ctrl + 64u + 8u * lane;
+                mp = unkey32(__hip_atomic_load(&words[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+                tp = unkey32(__hip_atomic_load(&words[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+                zp = __longlong_as_double(static_cast<long long>(__hip_atomic_load(reinterpret_cast<const unsigned long long*>(&words[2]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)));
+                np = __hip_atomic_load(&words[4], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                rp = unkey32(__hip_atomic_load(&words[5], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+            }
+            const bool any_bad = __ballot(np == 0xffffffffu) != 0ull;
+            if (np == 0xffffffffu) np = 0u;
+            const float mm = wave_max(mp), tt = wave_max(tp);
+            const double zz = wave_sum(zp > 0.0 ? zp * exp(static_cast<double>(__fsub_rn(rp, mm)) * static_cast<double>(inv_t)) : 0.0);
+            const uint32_t upto = wave_incl_scan(np);  // where the part's keys end in the merged list
+            if (lane < n_parts) {
+                S.red_u[lane] = np;
+                S.bcnt[lane] = upto - np;
+            }
+            if (lane == 63u) {
+                S.red_f[0] = mm;
+                S.red_f[1] = tt;
+                S.s_d[0] = zz;
+                S.bstart[0] = upto;
+                S.bstart[1] = any_bad ? 1u : 0u;
+            }
+        }
+        __syncthreads();
+        m = S.red_f[0];
+        thr_max = S.red_f[1];
+        z = S.s_d[0];  // against the row's maximum from here on
+        ref = m;
+        n_list = S.bstart[0];
+        bad = S.bstart[1] != 0u || !(m > -INFINITY);
+        const uint32_t region_log2 = static_cast<uint32_t>(__ffs(region)) - 1u;  // (a power of two, as the number of parts is)
+#pragma unroll
+        for (uint32_t i = 0; i < kSlots; ++i) {
+            const uint32_t slot = i * WS_BLOCK + t, p = slot >> region_log2, k = slot - (p << region_log2);
+            if (k < S.red_u[p]) {
+                list[S.bcnt[p] + k] = got[i];
+                __hip_atomic_store(&glist[slot], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // the workspace as the next launch needs it
+            }
+        }
+        if (t < 64u + 8u * n_parts) __hip_atomic_store(&ctrl[t], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+    }
+    WSS_MARK(5);  // parts met
     const uint32_t n_cand = by_k ? top_k : n_list;  // candidates the rules look at
     if (bad || n_list < n_cand || n_cand == 0u || n_cand > kShortCap) return false;
     short_sort(list, n_list, m, S);
     WSS_MARK(6);  // sorted
-    // the k-th largest has to lie above the threshold (below it, the sweep has left out tokens that rank before it);
+    // the k-th largest has to lie above the threshold, every part's (below one, the sweep has left out tokens that rank before it);
     // a min-p row's threshold lies below its floor by construction
     const float x_k = unkey32(static_cast<uint32_t>(list[n_cand - 1u] >> 32));
-    if ((by_k && !(x_k > thr)) || !(x_k > -INFINITY)) return false;
+    if ((by_k && !(x_k > thr_max)) || !(x_k > -INFINITY)) return false;
     ShortRow R;
     R.top_p = top_p;
     R.min_p = min_p;
@@ -874,11 +968,12 @@ __device__ __forceinline__ bool short_row(const BatchArgs& A, const uint32_t row
     return true;
 }
 
-template <int DT, bool MASKED>
+template <int DT, bool MASKED, bool SHARED>
 __global__ void __launch_bounds__(WS_BLOCK) short_batch_kernel(BatchArgs A) {
     __shared__ ShortShared shared;
-    const uint32_t row = blockIdx.x;
-    if (!short_row<DT, MASKED>(A, row, shared)) {
+    const uint32_t lg = SHARED ? A.split_log2 : 0u, row = blockIdx.x >> lg, part = blockIdx.x & ((1u << lg) - 1u);
+    bool finisher;
+    if (!short_row<DT, MASKED, SHARED>(A, row, part, 1u << lg, shared, finisher) && finisher) {
         __syncthreads();
         LeanArgPtr Ap = (LeanArgPtr)__builtin_amdgcn_kernarg_segment_ptr();
         asm volatile("" : "+s"(Ap));
