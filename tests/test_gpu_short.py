@@ -306,3 +306,20 @@ def test_static_entry_point_with_two_parts_a_row(rows):
         smp.run_static()
     res = gc.compare_rows(c, smp, range(0, rows, 13), 1)
     assert res["differ"] == 0, res
+
+
+@pytest.mark.parametrize("dtype,V,rows", [("f32", 151936, 140), ("f32", 100003, 140), ("bf16", 151936, 140), ("f32", 151936, 90)])
+def test_normaliser_of_rows_whose_maximum_lies_far_above_their_head(dtype, V, rows):
+    """Cold rows (inv_t 20) with a few tokens 45 to 75 units of the exponent above the largest of the head the sweep's sum starts
+    from, some of them in the history or behind the last whole vector: the normaliser is held to 1e-6 of the oracle's all the same."""
+    c = _odd(rows, V, dtype, top_k=50, n_hist=64, n_bias=0, allowed=0.8 if V % 2 else None)
+    rng = np.random.default_rng(rows)
+    c["inv_t"][:] = 20.0
+    x = (rng.standard_normal((rows, V)) * 0.5).astype(np.float32)
+    for r in range(rows):
+        ids = rng.integers(110000 if V > 120000 else 70000, V, 4)  # (behind the head of the row, and of a second slice)
+        x[r, ids] = (5.0 + 0.7 * rng.random()) + np.array([0.0, 0.013, 0.04, 0.11], np.float32)
+        x[r, V - 1] = x[r, ids[0]]
+        c["hist"][r, 0] = ids[1]
+    c["logits"] = gc.f32_to_bf16_bits(x) if dtype == "bf16" else x
+    run_short(c, 1, rows=range(0, rows, 6), kept_cap=64, handed_back=rows // 8, top_k_max=50)

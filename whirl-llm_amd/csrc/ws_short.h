@@ -856,6 +856,17 @@ __device__ __forceinline__ bool short_row(const BatchArgs& A, const uint32_t row
     WSS_MARK(9);
     uint32_t n_list = S.s_w[1];
     bool bad = not_mine || S.s_w[2] != 0u || n_list > kShortCap || !(ref > -INFINITY) || !(m > -INFINITY) || !(__fsub_rn(m, ref) * inv_t < 80.f);
+    // Tokens above `ref` can be most of the sum, and the larger the exponent, the less of a fraction 32 bits leave it (1.2e-6 of
+    // the normaliser where the maximum lies 60 units above the head's; 2e-7 up to the four units below which nothing is done):
+    // they are all on the list, and their terms are taken out and put back in 64 bits.
+    if (!bad && __fsub_rn(m, ref) * inv_t > 4.f) {  // uniform
+        double more = 0.0;
+        for (uint32_t k = t; k < n_list; k += WS_BLOCK) {
+            const float x = unkey32(static_cast<uint32_t>(list[k] >> 32)), a = __fsub_rn(x, ref);
+            if (a > 0.f) more += exp((static_cast<double>(x) - static_cast<double>(ref)) * static_cast<double>(inv_t)) - static_cast<double>(__builtin_amdgcn_exp2f(fmaf(a, k2lo, a * k2)));
+        }
+        z += block_sum(more, S.red_d);
+    }
     float thr_max = thr;
 
     // ---- a shared row: the parts' lists, maxima and sums meet in the row's workspace; the last one to arrive goes on
@@ -908,7 +919,7 @@ __device__ __forceinline__ bool short_row(const BatchArgs& A, const uint32_t row
             const bool any_bad = __ballot(np == 0xffffffffu) != 0ull;
             if (np == 0xffffffffu) np = 0u;
             const float mm = wave_max(mp), tt = wave_max(tp);
-            const double zz = wave_sum(zp > 0.0 ? zp * exp(static_cast<double>(__fsub_rn(rp, mm)) * static_cast<double>(inv_t)) : 0.0);
+            const double zz = wave_sum(zp > 0.0 ? zp * exp((static_cast<double>(rp) - static_cast<double>(mm)) * static_cast<double>(inv_t)) : 0.0);
             const uint32_t upto = wave_incl_scan(np);  // where the part's keys end in the merged list
             if (lane < n_parts) {
                 S.red_u[lane] = np;
@@ -954,7 +965,7 @@ __device__ __forceinline__ bool short_row(const BatchArgs& A, const uint32_t row
     R.top_p = top_p;
     R.min_p = min_p;
     R.u = batch_uniform(A.rng, P.seed, row, P.step, 0);
-    R.z = z * exp(static_cast<double>(__fsub_rn(ref, m)) * static_cast<double>(inv_t));
+    R.z = z * exp((static_cast<double>(ref) - static_cast<double>(m)) * static_cast<double>(inv_t));
     R.inv_t = inv_t;
     R.m = m;
     R.n_cand = n_cand;
