@@ -86,7 +86,6 @@ struct BatchPlan {
     uint32_t lean_tie;    // its second histogram copy (0: none), its dynamic LDS, and the spare LDS of the three-pass code it calls
     uint32_t lean_total;
     uint32_t lean_fb_tie;
-    bool vec_rows;        // rows of whole aligned 128-bit vectors
     bool shortlist;       // the short-list kernel takes the batch: every row has a top-k of at most top_k_max (the caller's word)
     uint32_t short_ab, short_cnt, short_total, short_fb_tie, short_fb_ab;  // its LDS: bitmap at short_ab, rank words at short_cnt
     uint32_t few_parts, few_total;  // short-list rows shared between this many workgroups each (0: not), and the dynamic LDS of those
@@ -176,7 +175,7 @@ BatchPlan plan_batch(const ws_batch* b, bool few = true) {
     // fused sweep: rows of whole 128-bit vectors that fit the register cache, and LDS room for the per-rank counters
     // next to the histogram (the exact path reuses the histogram's LDS for them)
     const uint64_t esz = b->dtype == WS_DTYPE_F32 ? 4 : 2;
-    const bool vec_rows = p.vec_rows = b->vocab % 8u == 0 && (b->row_stride * esz) % 16u == 0 && reinterpret_cast<uintptr_t>(b->logits) % 16u == 0;
+    const bool vec_rows = b->vocab % 8u == 0 && (b->row_stride * esz) % 16u == 0 && reinterpret_cast<uintptr_t>(b->logits) % 16u == 0;
     const uint64_t fused_total = 65536u + maps + cap * 8u;
     // (a token's bias entries are counted in 11 bits of its rank word)
     const bool can_fuse = vec_rows && b->vocab <= 163840u && fused_total + kStaticLds <= kMaxLds && (!b->bias_ids || b->max_bias <= 2047u);

@@ -470,7 +470,6 @@ __device__ __forceinline__ bool short_row(const BatchArgs& A, const uint32_t row
     const float inv_t = P.inv_t;
     const uint32_t top_k = P.top_k, nh = P.nh, nb = P.nb;
     const double top_p = P.top_p, min_p = P.min_p;
-    const bool use_top_p = top_p < 1.0, use_min_p = min_p > 0.0;
     // rows this code does not take
     const bool by_k = top_k >= 1u && top_k <= kShortMaxK && top_k <= V;  // the top_k largest decide
     const bool by_p = top_k == 0u && min_p > 0.0 && min_p <= 1.0;      // no top-k: what the min-p floor lets through decides
