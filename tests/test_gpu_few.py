@@ -276,3 +276,54 @@ def test_greedy_pick_of_a_row_beyond_32_bit_offsets():
     ids, pos = torch.zeros(1, dtype=torch.int32, device="cuda"), torch.zeros(1, dtype=torch.int32, device="cuda")
     assert m.argmax(x, ids, pos).item() == ids.item() == n - 5
     assert m.argmax_rows(x.view(1, n)).item() == n - 5
+
+
+@pytest.mark.parametrize("rows,top_k", [(1, 40), (5, 40), (200, 40), (3, 0)])
+def test_notify_writes_its_words_once_the_results_are_in_host_memory(rows, top_k):
+    """ws_sample_batch_notify on rows the registers kernel takes (it writes the words itself), on rows with a workgroup each and on
+    rows without a top-k (the stream does): all words come, and then tokens and kept sets in pinned memory are the eager call's."""
+    import time
+    m = gc.pkg()
+    c = case(rows, 40003 if top_k else 40000, top_k=top_k)
+    d = gc.upload(c, hints=top_k > 0)
+    want = gc.sampler_for(c, d, 1, kept_cap=64).run()
+    torch.cuda.synchronize()
+    smp = gc.sampler_for(c, d, 1, kept_cap=64)
+    host = dict(token=torch.zeros(rows, dtype=torch.int32, pin_memory=True), n_kept=torch.zeros(rows, dtype=torch.int32, pin_memory=True),
+                kept_ids=torch.full((rows, 64), -1, dtype=torch.int32, pin_memory=True))
+    smp.desc.token, smp.desc.n_kept, smp.desc.kept_ids = (host[k].data_ptr() for k in ("token", "n_kept", "kept_ids"))
+    done = torch.zeros(rows, dtype=torch.int32, pin_memory=True)
+    words = done.numpy()
+    for turn in (1, 2, 7):
+        host["token"].fill_(-5)
+        m.check(m.lib().ws_sample_batch_notify(torch.cuda.current_stream().cuda_stream, m.C.byref(smp.desc), done.data_ptr(), turn), "ws_sample_batch_notify")
+        until = time.monotonic() + 20.0
+        while not (words == turn).all() and time.monotonic() < until:
+            pass
+        assert (words == turn).all(), words
+        assert torch.equal(host["token"], want.token.cpu()) and torch.equal(host["n_kept"], want.n_kept.cpu())
+        assert torch.equal(host["kept_ids"], want.kept_ids.cpu())
+    torch.cuda.synchronize()
+    assert m.lib().ws_sample_batch_notify(None, m.C.byref(smp.desc), None, 1) == -1
+
+
+def test_one_workspace_for_batches_of_any_shape():
+    """Small and large vocabularies, many and few parts, the kernel that holds rows in registers, the short-list kernel's slices and
+    the single sweep's parts, one after the other on one workspace that was cleared once: answers as on one of their own."""
+    m = gc.pkg()
+    work = torch.zeros(128 * 65792, dtype=torch.uint8, device="cuda")
+    shapes = [(2, 4097, 5, "f32"), (1, 151936, 40, "f32"), (90, 131072, 30, "f32"), (3, 8192, 1000, "bf16"), (3, 65536, 0, "f32"), (60, 20000, 20, "bf16"),
+              (1, 262144, 64, "bf16"), (16, 151936, 0, "f32"), (2, 100003, 513, "f32")]
+    for rows, V, top_k, dtype in shapes + shapes[::-1]:
+        c = case(rows, V, dtype, top_k=top_k)
+        d = gc.upload(c, hints=top_k > 0)
+        smp = gc.sampler_for(c, d, 1, kept_cap=0)
+        assert smp.workspace.numel() <= work.numel()
+        want = smp.run()
+        got = gc.sampler_for(c, d, 1, kept_cap=0)
+        got.desc.workspace, got.desc.workspace_bytes = work.data_ptr(), work.numel()
+        got.run()
+        torch.cuda.synchronize()
+        assert torch.equal(got.token, want.token) and torch.equal(got.n_kept, want.n_kept) and torch.equal(got.flags, want.flags), (rows, V, top_k)
+        assert torch.allclose(got.stats, want.stats, rtol=1e-6, atol=0)  # (a shared row's sum is taken in the order its parts arrive)
+        assert not work.any().item(), (rows, V, top_k)
