@@ -29,7 +29,7 @@ sys.path.insert(0, ROOT)
 HBM_PEAK_GBS = 8000.0
 MODE = 0
 KEPT_CAP = 0  # entries a row of the kept-set dump (--kept-cap), 0: no dump
-# HBM bytes per launch of ws::sample_batch_kernel: rocprofv3 FETCH_SIZE + WRITE_SIZE, each scaled by what the same counter
+# HBM bytes per launch of the kernel a workload takes: rocprofv3 FETCH_SIZE + WRITE_SIZE, each scaled by what the same counter
 # reads for a 256 MiB device copy; measured for one build of the kernel and only reported for that build (the digest
 # of the kernel sources the counters were taken with), otherwise null. File names are relative to profiles/.
 TRAFFIC = {
@@ -58,10 +58,10 @@ def checker():
 
 
 def kernel_digest():
-    """sha256[:16] over the sources of the sampler kernels (ws_sample.h, ws_lean.h, ws_short.h, in this order)."""
+    """sha256[:16] over the sources of the sampler kernels (ws_common.h, ws_sample.h, ws_lean.h, ws_short.h, ws_few.h, in this order)."""
     import hashlib
     h = hashlib.sha256()
-    for name in ("ws_sample.h", "ws_lean.h", "ws_short.h"):
+    for name in ("ws_common.h", "ws_sample.h", "ws_lean.h", "ws_short.h", "ws_few.h"):
         with open(os.path.join(ROOT, "whirl-llm_amd", "csrc", name), "rb") as f:
             h.update(f.read())
     return h.hexdigest()[:16]
@@ -232,6 +232,18 @@ def cpu_model():
     return platform.processor() or "unknown"
 
 
+def kernel_name(smp, routes):
+    """The kernel that took the launch's rows: the short-list kinds by the workspace they ask for (65536 bytes a row: the kernel whose
+    workgroups hold their share of a row in registers)."""
+    from __graft_entry__ import load_package
+    m = load_package()
+    if routes["one_sweep_no_top_k"]:
+        return "ws::lean_batch_kernel"
+    if routes["short_list_top_k"]:
+        return "ws::few_batch_kernel" if m.lib().ws_sample_batch_workspace(m.C.byref(smp.desc)) == 65536 * smp.desc.rows else "ws::short_batch_kernel"
+    return "ws::sample_batch_kernel"
+
+
 def run_workload(name, steps, warmup, check_rows, top_k_array=False):
     gc = workloads()
     make = dict(tile=gc.make_tile, cfg1=gc.make_cfg1, cfg2=gc.make_cfg2, cfg3=gc.make_cfg3, cfg5=gc.make_cfg5)[name]
@@ -239,10 +251,8 @@ def run_workload(name, steps, warmup, check_rows, top_k_array=False):
     smp, wall_ms, kern_ms, warm_ms, n_rot = time_gpu(c, steps, warmup, top_k_array=top_k_array)
     par = parity_sample(c, smp, check_rows) if check_rows else device_report(smp)
     ab = algorithmic_bytes(c)
-    lean = par["routes"]["one_sweep_no_top_k"] > 0
-    short = par["routes"]["short_list_top_k"] > 0
     return c, dict(workload=name + (" (top_k: an array of zeros)" if top_k_array else ""), rows=c["rows"], vocab=c["V"], dtype=c["dtype"],
-                   kernel="ws::lean_batch_kernel" if lean else ("ws::short_batch_kernel" if short else "ws::sample_batch_kernel"), ms_per_step=wall_ms, kernel_ms=kern_ms,
+                   kernel=kernel_name(smp, par["routes"]), ms_per_step=wall_ms, kernel_ms=kern_ms,
                    kernel_ms_warm=warm_ms, logits_copies_rotated=n_rot,
                    rows_per_s=c["rows"] / (wall_ms * 1e-3), algorithmic_MB=ab / 1e6, achieved_GBs=ab / (kern_ms * 1e-3) / 1e9,
                    achieved_GBs_warm=ab / (warm_ms * 1e-3) / 1e9,
@@ -277,6 +287,9 @@ def reference_kernels(steps):
         x = torch.randn(rows, V, device="cuda:0") * 2
         o = torch.empty(rows, dtype=torch.int32, device="cuda:0")
         timed("argmax_rows", rows, lambda: L.ws_argmax_rows(S(), P(x), V, P(o), rows), rows * V * 4)
+        if need := int(L.ws_argmax_workspace(V, rows)):
+            work = torch.empty(need, dtype=torch.uint8, device="cuda:0")
+            timed("argmax_rows_ws", rows, lambda: L.ws_argmax_rows_ws(S(), P(x), V, P(o), rows, P(work), need), rows * V * 4)
         if rows == 256:  # the same with each launch on another copy of the rows (beyond the memory-side cache): HBM reads
             xs = [x] + [x.clone() for _ in range(rotation_for(x.numel() * 4) - 1)]
             turn = [0]
