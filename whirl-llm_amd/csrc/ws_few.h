@@ -15,12 +15,12 @@
 //   * the part that arrives last - a ticket, nobody waits - reads the waves' headers and lists. With top_k at most the
 //     number of waves, the top_k-th largest of the waves' maxima bounds the row's top_k-th largest logit from below, so
 //     that about as many keys as top_k are left to sort.
-// What bounds it is that chain: parameters, ids, their tokens' logits, headers, keys are five trips to memory of about
-// 0.7 us, between them some 2500 instructions of the slowest wave. 512 threads rather than 1024: the cost of a wave's own
+// What bounds it is that chain: parameters, ids, their tokens' logits, the stores of the keys, headers and keys are six trips to
+// memory of about 0.7 us, between them some 2500 instructions of the slowest wave. 512 threads rather than 1024: the cost of a wave's own
 // work (threshold, sums, publishing) is paid half as often, and a share still fits the registers. Measured against the
-// short-list kernel's shared rows (151936 fp32, microseconds a launch): one row, top-k 40: 20.6 -> 11.5; 64 rows of mixed
-// filters with 4096-id histories: 50 (126 when a row's min-p list ran over) -> 33; 32 rows of 50257, which went through
-// the three-pass kernel: 55.6 -> 15.0.
+// short-list kernel's shared rows (151936 fp32, microseconds a launch): one row, top-k 40: 20.6 -> 11.9; 64 rows of mixed
+// filters with 4096-id histories: 50 (126 when a row's min-p list ran over) -> 32.5; 32 rows of 50257, which went through
+// the three-pass kernel: 55.6 -> 15.4.
 #pragma once
 #include "ws_short.h"
 

@@ -1,5 +1,5 @@
 // The sampler for few rows (ws_few.h), a translation unit of its own: 512 threads per workgroup (256 registers each); fp32 and bf16 rows, with
-// and without an allow mask, shares of up to 20 (24), 40 and 80 tokens a thread; the three-pass code of ws_sample.h as a
+// and without an allow mask, shares of up to 20 (bf16: 24), 40, 80 and 112 tokens a thread; the three-pass code of ws_sample.h as a
 // function for the rows it hands back.
 #define WS_BLOCK 512
 #include "ws_lds_limit.h"

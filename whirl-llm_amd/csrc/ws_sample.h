@@ -94,7 +94,7 @@ struct BatchArgs {
     const int32_t* query;      // per row or nullptr: a token whose probability is asked for (< 0: none)
     double* query_prob;        // out per row or nullptr
     double* entropy;           // out per row or nullptr: entropy of the kept set
-    uint32_t split_log2;       // single-sweep kernel: a row is worked on by 2^split_log2 workgroups (0: one), block = row * parts + part
+    uint32_t split_log2;       // single-sweep and short-list kernels: a row is worked on by 2^split_log2 workgroups (0: one), block = row * parts + part
     unsigned char* work;       // split rows: split_row_bytes of zero-filled global memory per row, left zero-filled
     uint32_t split_spins;      // split rows: looks at the arrival counter before a part gives up on the others (0: about a second's worth)
     uint32_t split_row_bytes;  // kSplitRowBytes, or kSplitRowBytesKept when the rows have a staging area

@@ -3,8 +3,8 @@
 //
 // What src/sampling/sampler.cpp:15-78 keeps of such a row is decided among its top_k largest logits alone, so the row
 // needs no histogram of every token. One sweep at the speed of the loads:
-//   * from the head of the row a threshold is read off a 4096-bin count of the head's
-//     logits, such that about 3 top_k + 64 tokens of the row lie above it;
+//   * from the head of the row (of the slice, for a shared row) a threshold is read off a 4096-bin count of the head's
+//     logits, such that about top_k + max(top_k / 2, 150) tokens of the row lie above it;
 //   * the sweep keeps the maximum and the sum of exp((x - ref) inv_t) (Sampler::m and Sampler::sum, src/sampling/sampler.h:37-38)
 //     and puts every token above the threshold on a list in LDS, as its 64-bit order key (logit, then id);
 //   * tokens the history or the bias list touch are left out by the sweep (a bitmap in LDS, built as in ws_sample.h's
@@ -12,8 +12,11 @@
 //   * the list is sorted, and the reference's rules run on the sorted candidates: top-k, top-p on the mass of those, min-p
 //     against the largest, the draw by inverse CDF with the row's uniform.
 // A row for which a check fails, whose list runs over, or that has neither a top-k nor a min-p after all, is handed to the
-// three-pass code of ws_sample.h inside the same launch (WS_FLAG_ROUTE_HANDED_BACK). Few rows are shared between workgroups
-// by the kernel of ws_few.h, which ends with the same sort and rules.
+// three-pass code of ws_sample.h inside the same launch (WS_FLAG_ROUTE_HANDED_BACK).
+// Few rows are shared between workgroups by the kernel of ws_few.h, which ends with the same sort and rules; those it has no
+// registers or lists for are shared here: each part lists its slice against its own threshold and leaves list, maximum and sum in
+// the row's workspace, and the part that arrives last - a ticket, nobody waits - takes them all and finishes the row. The
+// top_k largest of the merged list are the row's when the k-th of them lies above every part's threshold.
 // A row without a top-k but with a min-p: what the floor min_p * p(max) lets through lies within -ln(min_p) / inv_t of the
 // row's maximum, so the threshold needs no fitting - the head's maximum (never above the row's) minus that distance and
 // a little more; the candidates are the whole list, the top-p cut compares with the row's normaliser (the sweep's sum,
@@ -401,7 +404,8 @@ __device__ __forceinline__ void short_rules(uint64_t* list, const uint32_t row, 
 // LDS of a row: [0, 32 KiB) the list (before the sweep: the head's bin counts), then at lds_ab the bitmap of the touched
 // tokens, its 16-bit popcount prefixes, and at lds_cnt the per-rank words {history count | bias entries << 20 | claimed}
 // and 16-bit indices of each rank's first bias entry.
-// Returns false when the row has to go to the three-pass code (uniform over the workgroup; nothing has been written for it).
+// Returns false when the row has to go to the three-pass code (uniform over the workgroup; nothing has been written for it, and a
+// shared row's workspace is as the launch found it); finisher: this workgroup is the one that would do that.
 template <int DT, bool MASKED, bool SHARED>
 __device__ __forceinline__ bool short_row(const BatchArgs& A, const uint32_t row, const uint32_t part, const uint32_t n_parts, ShortShared& S, bool& finisher) {
 #ifdef WS_SHORT_TIMERS

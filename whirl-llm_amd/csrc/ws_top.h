@@ -2,8 +2,8 @@
 // it in registers: the waves list and sum as in ws_few.h (no history, no mask), the part that arrives last sorts about as many
 // keys as are asked for. No counterpart in the reference, whose kernels give a row to one workgroup. What bounds it is the
 // chain of dependent steps (see ws_few.h). Against shared rows whose parts fitted a histogram to the head of the row and
-// whose last part counted the merged list once more (151936 fp32, microseconds a launch): 8 rows, K = 256: 19.6 -> 13.0;
-// a draft draw of 8 rows: 26.0 -> 12.5, of which the draw's one wave took 7 and takes 2.5.
+// whose last part counted the merged list once more (151936 fp32, microseconds a launch): 8 rows, K = 256: 19.6 -> 13.3;
+// a draft draw of 8 rows: 26.0 -> 11.6, of which the draw's one wave took 7 and takes 2.5.
 #pragma once
 #include "ws_draft.h"
 #include "ws_few.h"
