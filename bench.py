@@ -5,7 +5,7 @@
     python bench.py --reference-kernels      (greedy picks and topk_rows at the engine's shapes)
 
 A step = one launch of the fused batched sampler (ws_sample_batch) over one batch of synthetic logits that already
-sit in HBM. The default workload is the north-star tile: 256 rows x 151,936 fp32 logits ~ N(0, sigma 2), repetition /
+sit in HBM. The default workload is the tile: 256 rows x 151,936 fp32 logits ~ N(0, sigma 2), repetition /
 presence / frequency penalties over a 2048-id history per row, temperature in [0.7, 1.0], top-p 0.9 (top-k and min-p
 off, so every row needs a full-vocabulary mass select), seeded Philox draws. One JSON line goes to stdout.
 
@@ -352,7 +352,7 @@ def reference_kernels(steps):
 
 
 def spec_verify_workload(steps, warmup):
-    """classic speculative verification, 32 sequences x 9 positions x 151936 fp32 probabilities (target =
+    """cfg4: classic speculative verification, 32 sequences x 9 positions x 151936 fp32 probabilities (target =
     softmax of N(0, sigma 2) logits, draft = softmax of the same logits mixed 70 / 30 with fresh ones, draft ids drawn from
     the draft distribution), one ws_spec_verify_classic call per step. Necessary bytes: the two gathers per tested draft
     and, per sequence, the rejected position's p and q rows (or the last position's p row when every draft passed)."""
@@ -400,9 +400,9 @@ def spec_verify_workload(steps, warmup):
 
 
 def host_decode_step(steps):
-    """Wall clock of the C++ host API's decode step on configs[0]'s row (151936 fp32 logits on the device, temperature 0.8,
+    """Wall clock of the C++ host API's decode step on cfg1's row (151936 fp32 logits on the device, temperature 0.8,
     256-id history with repetition 1.1): sampling::DeviceRows::newCycle + prepareRow + sampling::sampleRow, one object serving
-    every step, as the engine's decode loop calls it - with configs[0]'s own filters (top-k 40 + top-p 0.95), with top-p 0.9
+    every step, as the engine's decode loop calls it - with cfg1's own filters (top-k 40 + top-p 0.95), with top-p 0.9
     alone and without any filter."""
     from __graft_entry__ import load_package
     m = load_package()

@@ -1,5 +1,5 @@
-"""Synthetic workloads of the sampling path: the five benchmark configurations (configs[0] .. configs[4]: a lone decode
-row, a mixed batch, bf16 Zipfian rows, classic verification, long masked rows) and the north-star tile, as seeded
+"""Synthetic workloads of the sampling path: the five benchmark configurations (cfg1 .. cfg5: a lone decode
+row, a mixed batch, bf16 Zipfian rows, classic verification, long masked rows) and the tile, as seeded
 numpy arrays, their upload into the device layouts ws_batch expects, and a BatchSampler over them. Used by bench.py,
 the GPU tests and the smoke run; nothing here touches a CPU sampler."""
 import numpy as np
@@ -39,7 +39,7 @@ def _common(rows, rng, V, n_hist, n_bias):
 
 
 def make_cfg1(V=151936):
-    """batch 1, N(0, sigma 2) with 5 tokens at +12, 256-id history, repetition 1.1, T 0.8, top-k 40, top-p 0.95."""
+    """cfg1: batch 1, N(0, sigma 2) with 5 tokens at +12, 256-id history, repetition 1.1, T 0.8, top-k 40, top-p 0.95."""
     rng = np.random.default_rng(DATA_SEED + 1)
     c = _common(1, rng, V, 256, 0)
     x = (rng.standard_normal((1, V)) * 2).astype(np.float32)
@@ -51,7 +51,7 @@ def make_cfg1(V=151936):
 
 
 def make_cfg2(rows=64, V=151936, n_hist=4096, n_bias=300):
-    """N(0, sigma 2) fp32, T in [0.5, 1.2], top-k in {0, 20, 50}, top-p in [0.8, 1], min-p 0.05, repetition /
+    """cfg2: N(0, sigma 2) fp32, T in [0.5, 1.2], top-k in {0, 20, 50}, top-p in [0.8, 1], min-p 0.05, repetition /
     presence / frequency penalties over a 4096-id history, 300 bias entries in [-5, 5]."""
     rng = np.random.default_rng(DATA_SEED + 2)
     c = _common(rows, rng, V, n_hist, n_bias)
@@ -64,7 +64,7 @@ def make_cfg2(rows=64, V=151936, n_hist=4096, n_bias=300):
 
 
 def make_cfg3(rows=256, V=151936, n_hist=2048):
-    """bf16 Zipfian logits -1.1 ln(rank) + N(0, 0.3) over a random permutation, top-k off, top-p 0.9,
+    """cfg3: bf16 Zipfian logits -1.1 ln(rank) + N(0, 0.3) over a random permutation, top-k off, top-p 0.9,
     penalties over a 2048-id history."""
     rng = np.random.default_rng(DATA_SEED + 3)
     c = _common(rows, rng, V, n_hist, 0)
@@ -80,7 +80,7 @@ def make_cfg3(rows=256, V=151936, n_hist=2048):
 
 
 def make_tile(rows=256, V=151936, n_hist=2048):
-    """The north-star tile: fp32 N(0, sigma 2), repetition / presence / frequency penalties over a 2048-id history,
+    """The tile: fp32 N(0, sigma 2), repetition / presence / frequency penalties over a 2048-id history,
     T in [0.7, 1.0], top-p 0.9, top-k and min-p off (a full-vocabulary mass select on every row)."""
     rng = np.random.default_rng(DATA_SEED + 6)
     c = _common(rows, rng, V, n_hist, 0)
@@ -92,7 +92,7 @@ def make_tile(rows=256, V=151936, n_hist=2048):
 
 
 def make_cfg5(rows=1024, V=262144, n_hist=8192, n_bias=500):
-    """fp32 N(0, sigma 3), allow-mask with 90 % of the tokens at -inf, 500 bias entries, 8192-id history,
+    """cfg5: fp32 N(0, sigma 3), allow-mask with 90 % of the tokens at -inf, 500 bias entries, 8192-id history,
     top-k 1000, top-p 0.95, T 1."""
     rng = np.random.default_rng(DATA_SEED + 5)
     c = _common(rows, rng, V, n_hist, n_bias)
@@ -112,7 +112,7 @@ def upload(c, device="cuda:0", hints=True, min_p_hint=True):
     """numpy case -> dict of device tensors in the layouts ws_batch expects. hints: say what is known about the rows
     (top_k left out when no row has one, top_k_max), as a caller that wants the fastest kernel would; without them
     every batch goes the way a descriptor that says nothing goes. min_p_hint: also say min_p_min, which sends rows
-    without a top-k but with a min-p to the short-list kernel (measured on configs[1]: 45 against 48 us of the split
+    without a top-k but with a min-p to the short-list kernel (measured on cfg2: 45 against 48 us of the split
     single-sweep kernel)."""
     import torch
     d = {}
