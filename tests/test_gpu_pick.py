@@ -426,3 +426,14 @@ def test_topk_rows_off_the_vector_boundaries(n, K):
         assert stats[r, 0] == xr.max()
         truth = np.exp((xr - xr.max()) * 1.25).sum()
         assert abs(stats[r, 1] - truth) <= 2e-6 * truth  # (the bar of the aligned rows)
+
+
+def test_rows_with_trailing_dimensions_of_one():
+    """[rows, n, 1] is taken like [rows, n]: only the first two dimensions are looked at."""
+    m = gpu_cases.pkg()
+    x = torch.from_numpy(np.random.default_rng(4).standard_normal((3, 9001)).astype(np.float32)).to(DEV)
+    assert torch.equal(m.argmax_rows(x[:, :, None]), m.argmax_rows(x))
+    a, b = (torch.zeros(3, dtype=torch.int32, device=DEV) for _ in range(2))
+    assert torch.equal(m.argmax_rows_to(x[:, :, None], a, [2, 0, 1]), m.argmax_rows_to(x, b, [2, 0, 1]))
+    for p, q in zip(m.topk_rows(x[:, :, None], 20, 1.0), m.topk_rows(x, 20, 1.0)):
+        assert torch.equal(p, q)

@@ -249,7 +249,7 @@ _PICK_WORDS, _PICK_BYTES = 1024, 4096
 def argmax_rows(x):
     """x: [rows, n] float32 device -> int32 [rows] (first index of each row's maximum)."""
     _dev_f32(x)
-    rows, n = x.shape
+    rows, n = x.shape[0], x.shape[1]
     first = rows + (rows & 1)
     out = torch.empty(first + _PICK_WORDS, dtype=torch.int32, device=x.device)  # the picks, and behind them the workspace
     at = out.data_ptr()
@@ -269,7 +269,7 @@ def argmax(x, ids, pos, advance=1):
 def argmax_rows_to(x, out, dst):
     _dev_f32(x)
     ri = _row_idx(dst)
-    rows, n = x.shape
+    rows, n = x.shape[0], x.shape[1]
     work = torch.empty(_PICK_WORDS, dtype=torch.int32, device=x.device)
     check(lib().ws_argmax_rows_to_ws(_stream(), _p(x), n, _p(out), C.byref(ri), rows, _p(work), _PICK_BYTES), "ws_argmax_rows_to_ws")
     return out
@@ -326,7 +326,7 @@ def topk_rows(x, K, inv_t, workspace=None):
     workspace: a zero-filled uint8 device tensor of ws_topk_rows_workspace bytes kept between calls - small batches then
     share each row between several workgroups (ws_topk_rows_ws)."""
     _dev_f32(x)
-    rows, n = x.shape
+    rows, n = x.shape[0], x.shape[1]
     if K <= n:  # (every entry is written)
         ids = torch.empty((rows, K), dtype=torch.int32, device=x.device)
         vals = torch.empty((rows, K), dtype=torch.float32, device=x.device)
