@@ -37,6 +37,10 @@ int prepare_lean(unsigned lds_limit);
 // ws_short.hip: the short-list kernel for batches whose rows all have a bounded top-k
 int launch_short(hipStream_t stream, const BatchArgs& a, unsigned lds_bytes, unsigned lds_limit);
 int prepare_short(unsigned lds_limit);
+// ws_code.hip: bf16 rows, held in registers and counted by value
+int launch_code(hipStream_t stream, const BatchArgs& a, unsigned rows, unsigned lds_bytes, unsigned lds_limit);
+int prepare_code(unsigned lds_limit);
+uint64_t code_lds_bytes(uint32_t vocab, uint32_t cap, uint32_t copies);
 // ws_few.hip: the same rows shared between workgroups that hold them in registers
 int launch_few(hipStream_t stream, const BatchArgs& a, unsigned lds_bytes, unsigned lds_limit);
 int prepare_few(unsigned lds_limit);
@@ -68,6 +72,8 @@ constexpr uint32_t kStaticLds = 4096u;
 constexpr uint32_t kStaticShort = 9216u;
 // the same for the kernel of few rows
 constexpr uint32_t kStaticFew = 10240u;
+// the same for the kernel of bf16 rows
+constexpr uint32_t kStaticCode = 14336u;
 // the lean kernel's own tables and those of the three-pass code it calls
 #ifdef WS_PHASE_TIMERS
 constexpr uint32_t kStaticLean = 11776u + 768u;
@@ -89,6 +95,10 @@ struct BatchPlan {
     bool shortlist;       // the short-list kernel takes the batch: every row has a top-k of at most top_k_max (the caller's word)
     uint32_t short_ab, short_cnt, short_total, short_fb_tie, short_fb_ab;  // its LDS: bitmap at short_ab, rank words at short_cnt
     uint32_t few_parts, few_total;  // short-list rows shared between this many workgroups each (0: not), and the dynamic LDS of those
+    bool code;            // the kernel of bf16 rows takes the batch
+    uint32_t code_head;   // its masses (BatchArgs)
+    float code_above;
+    uint32_t code_cap, code_copies, code_total, code_fb_tie, code_fb_ab;  // entries its tables take, copies of its counts, its dynamic LDS, and the three-pass code's layout in it
     uint32_t split_log2;  // the most parts per row that pay for this batch
     uint64_t workspace_min;  // split rows: the least that lets them split (no staging areas), 0 when nothing is split
     uint64_t workspace;   // bytes for that
@@ -155,6 +165,54 @@ void few_plan(const ws_batch* b, uint64_t cap, uint64_t maps, BatchPlan& p) {
     p.workspace = p.workspace_min = uint64_t{b->rows} * ws::kFewRowBytes;
 }
 
+// bf16 rows of ws_code.h: any filters, any alignment; no optional outputs and no race. Two copies of the counts where there is room for
+// them beside the tables of the history and bias entries: with one, rows of tied logits queue up at its words.
+void code_plan(const ws_batch* b, uint64_t cap, uint64_t maps, uint64_t spare_bytes, BatchPlan& p) {
+    p.code = false;
+    if (b->dtype != WS_DTYPE_BF16 || b->mode != WS_MODE_AUTO || b->vocab < 8u || b->kept_ids || b->query_prob || b->entropy || b->race ||
+        (b->bias_ids && b->max_bias > 2047u))
+        return;
+    p.code_cap = (static_cast<uint32_t>(cap) + 3u) & ~3u;
+    // The masses of rows that are not of the short-list kind go by the bins of the other kernels such rows can get - with another dump, draw
+    // or address - so that a cut among thousands of tokens falls on the same one: ws_sample.h's anchor, or for unshared rows without a top-k
+    // ws_lean.h's.
+    const bool shared = b->max_split != 1u && uint64_t{b->rows} * 4u <= static_cast<uint64_t>(compute_units()) && b->vocab >= 65536u;
+    p.code_head = p.shortlist ? 0u : (p.fused ? 2u : 1u);
+    p.code_above = p.fused && !b->top_k && !shared ? 12.f : 8.f;
+    const uint64_t three = (cap * 8u > 65536u ? ((cap * 8u + 15u) & ~uint64_t{15}) : 65536u) + maps;
+    for (p.code_copies = 2; p.code_copies > 0; --p.code_copies) {
+        uint64_t total = ws::code_lds_bytes(b->vocab, p.code_cap, p.code_copies);
+        if (total < three) total = three;
+        if (total + kStaticCode > kMaxLds) continue;
+        p.code = true;
+        p.code_fb_ab = static_cast<uint32_t>(three - maps);
+        p.code_fb_tie = three + spare_bytes <= total ? static_cast<uint32_t>((three + 15u) & ~uint64_t{15}) : 0u;
+        p.code_total = static_cast<uint32_t>(total);
+        return;
+    }
+}
+
+// bf16 rows of the short-list kind: ws_code.h, ws_few.h or ws_short.h. Few rows are ws_few.h's: it shares them, and its lists are short -
+// but a list of some hundred keys has to be sorted, which costs more than counting a row that is not long, and two workgroups a row
+// are not much of a share. Microseconds, ws_few.h and ws_code.h (1000-id histories): top-k 50: 64 rows of 50257 16.0 / 18.4, 100 rows 19.9 /
+// 17.9, 100 of 80000 21.2 / 18.9, 100 of 32000 16.1 / 16.4, 64 of 151936 21.5 / 24.2; top-k 300: 1 of 32000 16.9 / 14.8, 8 of 151936 18.6 / 23.7;
+// top-k 600 and 1000: 8 of 32000 20.5 / 16.3 and 22.2 / 16.6, 8 of 151936 24.8 / 24.7 and 29.2 / 24.6, 16 of 262144 29.5 / 35.5 and 34.8 / 35.9;
+// min-p alone: 100 of 50257 18.2 / 18.5, 128 of 60000 18.9 / 19.5. What ws_few.h does not take: top-k 50, ws_short.h and ws_code.h: 200 of 32000 24.9 /
+// 16.5, 1000 of 8000 with a min-p 62.2 / 59.1, 256 of 151936 52.2 / 29.4, 400 of 262144 118.6 / 90.0. Rows without a top-k have a short list and nothing to
+// estimate: 150 of 20000 14.3 / 16.5, 1000 of 8000 46.2 / 56.3, 300 of 40000 31.9 / 31.2, 256 of 50257 22.5 / 20.0, 256 of 151936 45.1 / 30.4; longer than the
+// registers hold and in four slices or more: 60 of 262144 32.0 / 37.9, in two: 100 of 262144 44.7 / 38.2.
+void code_or_short(const ws_batch* b, BatchPlan& p) {
+    const bool by_k = b->top_k && b->top_k_max >= 1u;
+    if (p.few_parts) {
+        const bool long_lists = b->top_k_max > 512u ? b->vocab <= 163840u : b->top_k_max > 256u && b->vocab <= 40960u;
+        p.code = by_k && (long_lists || (p.few_parts <= 2u && b->vocab > 32768u));
+        if (p.code) p.few_parts = 0;
+    } else if (!by_k) {
+        p.code = b->vocab > 40960u && !(b->vocab > 163840u && short_split_log2(b) >= 2u);
+    }
+    if (p.code) p.workspace = p.workspace_min = 0;
+}
+
 // few: whether ws_few.h is considered
 BatchPlan plan_batch(const ws_batch* b, bool few = true) {
     BatchPlan p{};
@@ -214,7 +272,7 @@ BatchPlan plan_batch(const ws_batch* b, bool few = true) {
 #endif
     // Its rows are those without a top-k, and a batch says so by leaving `top_k` out: a row with one would be handed
     // back to the three-pass code inside the launch, at twice the time of the kernel that takes a top-k in its stride.
-    p.lean = p.fused && b->mode == WS_MODE_AUTO && !b->top_k && !b->kept_ids && !b->query_prob && !wants_entropy && !b->race &&
+    p.lean = p.fused && b->dtype == WS_DTYPE_F32 && b->mode == WS_MODE_AUTO && !b->top_k && !b->kept_ids && !b->query_prob && !wants_entropy && !b->race &&
              fused_total + kStaticLean <= kMaxLds;
     if (p.lean) {
         uint64_t lt = fused_total;
@@ -253,12 +311,20 @@ BatchPlan plan_batch(const ws_batch* b, bool few = true) {
             p.short_total = static_cast<uint32_t>(st);
         }
     }
+    code_plan(b, cap, maps, spare_bytes, p);
     if (p.shortlist) {
         p.lean = false;
         p.split_log2 = 0;
         p.workspace = p.workspace_min = 0;
         if (few) few_plan(b, cap, maps, p);
-        if (!p.few_parts && (p.split_log2 = short_split_log2(b)) != 0u) p.workspace = p.workspace_min = uint64_t{b->rows} * ws::kShortSplitRowBytes;
+        if (p.code) code_or_short(b, p);
+        if (!p.code && !p.few_parts && (p.split_log2 = short_split_log2(b)) != 0u) p.workspace = p.workspace_min = uint64_t{b->rows} * ws::kShortSplitRowBytes;
+        p.err = WS_OK;
+        return p;
+    }
+    if (p.code) {
+        p.split_log2 = 0;
+        p.workspace = p.workspace_min = 0;
         p.err = WS_OK;
         return p;
     }
@@ -351,6 +417,7 @@ int prepare_all() {
     if (const int e = ws::prepare_fused_kept(kMaxLds - kStaticLds); e != 0) return e;
     if (const int e = ws::prepare_split_kept(kMaxLds - kStaticLds); e != 0) return e;
     if (const int e = ws::prepare_lean(kMaxLds - kStaticLean); e != 0) return e;
+    if (const int e = ws::prepare_code(kMaxLds - kStaticCode); e != 0) return e;
     if (const int e = ws::prepare_few(kMaxLds - kStaticFew); e != 0) return e;
     if (const int e = ws::prepare_top(); e != 0) return e;
     return ws::prepare_short(kMaxLds - kStaticShort);
@@ -681,6 +748,16 @@ int sample_batch_on(void* stream, const ws_batch* b, const BatchPlan& p, unsigne
         a.fb_lds_ab = p.short_fb_ab;
         return ws::launch_few(S(stream), a, p.few_total, kMaxLds - kStaticFew);
     }
+    if (p.code) {
+        a.lds_tie = p.code_copies > 1u;
+        a.fb_lds_tie = p.code_fb_tie;
+        a.fb_lds_ab = p.code_fb_ab;
+        a.code_cap = p.code_cap;
+        a.code_route = p.shortlist ? WS_FLAG_ROUTE_SHORT : (b->top_k ? 0u : WS_FLAG_ROUTE_LEAN);
+        a.code_head = p.code_head;
+        a.code_above = p.code_above;
+        return ws::launch_code(S(stream), a, b->rows, p.code_total, kMaxLds - kStaticCode);
+    }
     if (p.shortlist) {
         a.lds_ab = p.short_ab;
         a.lds_cnt = p.short_cnt;
@@ -726,7 +803,7 @@ int ws_sample_batch_notify(void* stream, const ws_batch* b, uint32_t* done, uint
 int ws_sample_batch_static(void* stream, const ws_batch* b) {
     const BatchPlan p = plan_for(b, sizeof(scratch));
     if (p.err != WS_OK) return p.err;
-    if (!p.fused && !p.shortlist) return sample_batch_on(stream, b, p, nullptr, 0);  // (nothing may be left in the split rows' memory)
+    if (p.code || (!p.fused && !p.shortlist)) return sample_batch_on(stream, b, p, nullptr, 0);  // (nothing may be left in the split rows' memory)
     if (p.workspace_min > sizeof(scratch)) {  // more split rows than the library's own memory holds
         if (p.shortlist && b->max_split == 0u) return sample_batch_on(stream, b, p, nullptr, 0);  // (split by the library's own choice: not here)
         return WS_E_STATIC_LIMIT;

@@ -104,6 +104,9 @@ struct BatchArgs {
     uint32_t* done;       // ws_few.h: a word per row for a host that waits (or nullptr), and what goes there
     uint32_t done_value;
     uint32_t few_parts, few_magic, few_chunk_log2;  // ws_few.h: parts a row, 2^32 / waves a row rounded up, log2 of the lanes a chunk
+    uint32_t code_cap, code_route;  // ws_code.h: history and bias entries its tables have room for, and the route bit of its rows
+    uint32_t code_head;           // its masses: 0 in 64 bits; else by the single-sweep kernels' bins, the anchor above the first 8192 tokens that nothing touches (1), or the first 16384 (2)
+    float code_above;             // .. by so many units of the exponent
 };
 
 // Global memory of a split row: the merged histogram, the merged candidate list, and four control words (parts that
