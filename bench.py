@@ -58,10 +58,10 @@ def checker():
 
 
 def kernel_digest():
-    """sha256[:16] over the sources of the sampler kernels (ws_common.h, ws_sample.h, ws_lean.h, ws_short.h, ws_few.h, in this order)."""
+    """sha256[:16] over the sources of the sampler kernels (ws_common.h, ws_sample.h, ws_lean.h, ws_code.h, ws_short.h, ws_few.h, in this order)."""
     import hashlib
     h = hashlib.sha256()
-    for name in ("ws_common.h", "ws_sample.h", "ws_lean.h", "ws_short.h", "ws_few.h"):
+    for name in ("ws_common.h", "ws_sample.h", "ws_lean.h", "ws_code.h", "ws_short.h", "ws_few.h"):
         with open(os.path.join(ROOT, "whirl-llm_amd", "csrc", name), "rb") as f:
             h.update(f.read())
     return h.hexdigest()[:16]
@@ -238,7 +238,7 @@ def kernel_name(smp, routes):
     from __graft_entry__ import load_package
     m = load_package()
     if routes["one_sweep_no_top_k"]:
-        return "ws::lean_batch_kernel"
+        return "ws::code_batch_kernel" if smp.desc.dtype == m.DTYPE_BF16 else "ws::lean_batch_kernel"
     if routes["short_list_top_k"]:
         return "ws::few_batch_kernel" if m.lib().ws_sample_batch_workspace(m.C.byref(smp.desc)) == 65536 * smp.desc.rows else "ws::short_batch_kernel"
     return "ws::sample_batch_kernel"

@@ -1,5 +1,5 @@
 // The lean single-sweep sampler for gfx950: one workgroup of 1024 threads (sixteen wave64s, four per SIMD) per row,
-// for batches with at least one row per compute unit. It answers the rows most requests are made of - fp32 or bf16
+// for batches with at least one row per compute unit. It answers the rows most requests are made of - fp32
 // logits in whole 128-bit vectors, a closed filter without a top-k (top-p and / or min-p), the inverse-CDF draw - and
 // hands every other row (and every row on which one of its own checks fails) to the three-pass code of ws_sample.h
 // inside the same launch. Results are those of ws_sample.h's single-sweep kernel: the same bins, the same histogram
@@ -31,8 +31,7 @@ constexpr int kLeanRegs = 40;   // bin-cache registers per thread: 160 tokens, r
 constexpr int kLeanBatch = 2;   // 128-bit loads per thread and batch
 constexpr uint32_t kLeanBuckets = 128u;   // words of the finish's tables in LeanShared
 constexpr uint32_t kLeanMaxList = 4096u;  // candidates of a row's ranges together: what the sort's 32 KiB hold
-// The bins the cut and the draw can fall in: sixteen at most, with eight different cache bytes at most among them (fp32
-// rows: eight bins; bf16 rows, where four neighbours share a byte: all sixteen).
+// The bins the cut and the draw can fall in: as many as have eight different cache bytes, sixteen at most.
 constexpr uint32_t kLeanMaxBins = 16u;
 // Bins are counted down from an anchor this many units of the exponent above the largest of the row's first tokens
 // (the row's maximum may lie up to 16 above it before the row is handed back). Eight were too few for peaked rows: with
@@ -91,37 +90,34 @@ struct LeanHits {
 };
 
 // A third token of a group and beyond goes to list[] as (token | kListNeedsLoad, 0), one LDS atomic each (rare). With
-// TO_LIST every find goes there (a second round of bytes). DT: 0 fp32 rows (a 128-bit vector is four tokens, one
-// register of the cache), 1 bf16 rows (eight tokens, two registers); nv: the row's vectors.
-template <int NT, bool TO_LIST, int DT>
+// TO_LIST every find goes there (a second round of bytes). nv: the row's vectors.
+template <int NT, bool TO_LIST>
 __device__ __forceinline__ void lean_scan(const uint32_t (&cache)[kLeanRegs], const uint32_t (&c4)[4], const void* __restrict__ xg, LeanHits& H,
                                           uint2* list, uint32_t* n_list, uint32_t cap, uint32_t nv) {
     const uint32_t t = threadIdx.x;
-    constexpr int kRegsPerVec = DT == 0 ? 1 : 2;
     auto logit_bits = [&](uint32_t i) {
-        return DT == 0 ? static_cast<const uint32_t*>(xg)[i] : static_cast<uint32_t>(static_cast<const uint16_t*>(xg)[i]) << 16;
+        return static_cast<const uint32_t*>(xg)[i];
     };
 #pragma unroll
     for (int g = 0; g < kLeanGroups; ++g) {
         // where the row ends is looked at per group, uniformly: a group past the row is skipped, the one group the end
         // falls in masks its finds, the others need no test
         uint32_t acc = 0;
-        const uint32_t g_lo = static_cast<uint32_t>(g * 8 / kRegsPerVec) * WS_BLOCK;
-        if (g_lo + static_cast<uint32_t>(8 / kRegsPerVec) * WS_BLOCK <= nv) {
+        const uint32_t g_lo = static_cast<uint32_t>(g * 8) * WS_BLOCK;
+        if (g_lo + 8u * WS_BLOCK <= nv) {
 #pragma unroll
             for (int r = 0; r < 8; ++r)  // bit 8 e + r: token e of register r
                 acc = ((lean_flags<NT>(cache[g * 8 + r], c4) >> (7 - r)) & (0x01010101u << r)) | acc;
         } else if (g_lo < nv) {
 #pragma unroll
             for (int r = 0; r < 8; ++r) {
-                const uint32_t keep = g_lo + static_cast<uint32_t>(r / kRegsPerVec) * WS_BLOCK + t < nv ? 0x01010101u << r : 0u;
+                const uint32_t keep = g_lo + static_cast<uint32_t>(r) * WS_BLOCK + t < nv ? 0x01010101u << r : 0u;
                 acc = ((lean_flags<NT>(cache[g * 8 + r], c4) >> (7 - r)) & keep) | acc;
             }
         }
         auto token_of = [&](uint32_t bit) {
             const uint32_t reg = static_cast<uint32_t>(g * 8) + (bit & 7u);
-            if (DT == 0) return ((reg * WS_BLOCK + t) << 2) + (bit >> 3);
-            return (((reg >> 1) * WS_BLOCK + t) << 3) + ((reg & 1u) << 2) + (bit >> 3);
+            return ((reg * WS_BLOCK + t) << 2) + (bit >> 3);
         };
         if (!TO_LIST) {
             H.idx[g] = H.idx[kLeanGroups + g] = 0xffffffffu;
@@ -333,16 +329,10 @@ struct LeanShared {
 __device__ __forceinline__ double sel_dbg(const LeanShared& S) { return S.sel.n_r0 + 1e5 * S.sel.n_r1 + 1e10 * (S.sel.r0hi - S.sel.r0lo + 1) + 1e12 * (S.sel.r1hi - S.sel.r1lo + 1); }
 #endif
 // One row. Returns false when the row is left to the three-pass code (nothing has been written for it then).
-template <bool MASKED, int DT>  // DT: 0 fp32 rows, 1 bf16 rows
+template <bool MASKED>
 __device__ __forceinline__ bool lean_row(const BatchArgs& A, const uint32_t row, LeanShared& S) {
-    constexpr uint32_t kTok = DT == 0 ? 4u : 8u, kTokLog = DT == 0 ? 2u : 3u;  // tokens in a 128-bit vector
-    constexpr int kRegsPerVec = DT == 0 ? 1 : 2;                                // and its registers in the bin cache
-    // What the cache remembers of a token's bin: bits kCacheShift .. kCacheShift + 7. A scan for a bin also finds the
-    // tokens of the bins that share those bits and drops them afterwards. fp32 rows: the bins 256 apart, which hold some
-    // hundreds of tokens each. bf16 rows have their tokens on few values, four bins apart and more where the tokens are
-    // many, thousands to a value in the row's tail: there a bin's three neighbours (mostly empty) are found with it, and
-    // the bins that alias are 1024 apart, beyond the span of any row.
-    constexpr uint32_t kCacheShift = DT == 0 ? 0u : 2u;
+    constexpr uint32_t kTok = 4u, kTokLog = 2u;  // tokens in a 128-bit vector, which is one register of the bin cache: the low eight bits of each bin
+    // (a scan for a bin also finds the tokens of the bins 256 apart, some hundreds each, and drops them afterwards)
 #ifdef WS_PHASE_TIMERS
     const long long wsl_t0 = clock64();  // debug builds: the marks go to LDS, and at the end to `entropy`, 16 doubles a row
     if (threadIdx.x < 32) S.marks[threadIdx.x] = 0;
@@ -367,8 +357,8 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const uint32_t row,
 
     RowView rv;
     rv.V = V;
-    rv.dtype = DT;
-    rv.base = static_cast<const unsigned char*>(A.logits) + static_cast<size_t>(row) * A.row_stride * (DT == 0 ? 4u : 2u);
+    rv.dtype = 0;
+    rv.base = static_cast<const unsigned char*>(A.logits) + static_cast<size_t>(row) * A.row_stride * 4u;
     rv.vec = true;
     rv.allow = MASKED ? A.allow + static_cast<size_t>(row) * A.allow_stride : nullptr;
     rv.touched = nullptr;
@@ -379,8 +369,8 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const uint32_t row,
     // anything else - their address needs the kernel's arguments only - and travel while the row's parameters and then
     // the history ids are fetched, two dependent trips to memory; the first kEarly batches are binned before those ids
     // are looked at (what the ids touch there is put right afterwards), so that phase 0 costs its LDS work and no wait.
-    constexpr int kRing = 3, kEarly = WS_LEAN_EARLY / kRegsPerVec;  // (as many tokens either way)
-    constexpr int NB = kLeanRegs / (kLeanBatch * kRegsPerVec);
+    constexpr int kRing = 3, kEarly = WS_LEAN_EARLY;
+    constexpr int NB = kLeanRegs / kLeanBatch;
     uint4 q[kRing][kLeanBatch];
     uint32_t na[kRing][kLeanBatch];
     auto load = [&](int bt, int slot) __attribute__((always_inline)) {
@@ -460,8 +450,7 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const uint32_t row,
             const uint32_t w[4] = {q[0][u].x, q[0][u].y, q[0][u].z, q[0][u].w};
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                if (DT == 0) s = fmaxf(s, __uint_as_float(w[e]));
-                else s = fmaxf(s, fmaxf(__uint_as_float(w[e] << 16), __uint_as_float(w[e] & 0xffff0000u)));
+                s = fmaxf(s, __uint_as_float(w[e]));
             }
         }
         s = block_max(s, red_f);  // its barriers also publish the zeroed histogram
@@ -476,15 +465,6 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const uint32_t row,
     float vm_early[kEarly * kLeanBatch];  // maxima of the early batches' vectors, until the bitmap says which hold a touched token
     const float tail_f = static_cast<float>(kLeanTail + static_cast<int>(t));  // this thread's own tail bin
     uint64_t* myhist = (hist2 && (t & 1u)) ? hist2 : hist;
-    // Where a bin's word lies in the histogram. bf16 rows: the words of four neighbouring bins change places by bits 4
-    // and 5 of the bin. Such a row's tokens sit on few values four bins apart and more - in the tail of a long row two
-    // thirds of all tokens on some twenty - and in their natural places those words share four of the sixteen pairs of
-    // LDS banks: the additions of a wave would queue up there four times as long.
-#ifdef WS_NO_SWZ
-    auto hist_word = [&](uint32_t b) { return b; };
-#else
-    auto hist_word = [&](uint32_t b) { return DT == 0 ? b : b ^ ((b >> 4) & 3u); };
-#endif
     const uint32_t stage_cap = 2047u;
     const uint32_t n_full = nv / WS_BLOCK;  // vector rounds that are inside the row for every thread
     bool any_touched = false;               // uniform
@@ -520,29 +500,20 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const uint32_t row,
             const uint32_t w[4] = {q[slot][u].x, q[slot][u].y, q[slot][u].z, q[slot][u].w};                                          \
             const int32_t bw = MASKED ? static_cast<int32_t>(nal >> ((j * kTok) & 31u)) : 0;                                         \
             float vm = -INFINITY;                                                                                                    \
-            _Pragma("unroll") for (int h = 0; h < kRegsPerVec; ++h) { /* four tokens, one register of the cache */                   \
-                uint32_t bins[4];                                                                                                    \
-                _Pragma("unroll") for (int e = 0; e < 4; ++e) {                                                                      \
-                    uint32_t bits = w[e];                                                                                            \
-                    if (DT != 0) bits = (e & 1) ? w[2 * h + (e >> 1)] & 0xffff0000u : w[2 * h + (e >> 1)] << 16;                     \
-                    if (MASKED) bits |= static_cast<uint32_t>((bw << (31 - (4 * h + e))) >> 31);                                     \
-                    const float x = __uint_as_float(bits);                                                                           \
-                    vm = fmaxf(vm, x);                                                                                               \
-                    const float tc = bin_coord(aq, c64, x, tail_f);                                                                  \
-                    bins[e] = static_cast<uint32_t>(tc);                                                                             \
-                    WSL_HIST_ADD(bins[e], tc);                                                                                       \
-                }                                                                                                                    \
-                uint32_t packed;                                                                                                     \
-                if (kCacheShift == 0) {                                                                                              \
-                    const uint32_t lo2 = __builtin_amdgcn_perm(bins[1], bins[0], 0x0c0c0400u);                                       \
-                    packed = __builtin_amdgcn_perm(bins[3], bins[2], 0x04000c0cu) | lo2;                                             \
-                } else { /* bits kCacheShift .. kCacheShift + 7 of each bin: two bins to a word, shifted together */                  \
-                    const uint32_t p01 = ((bins[1] << 16) | bins[0]) >> kCacheShift, p23 = ((bins[3] << 16) | bins[2]) >> kCacheShift; \
-                    packed = __builtin_amdgcn_perm(p23, p01, 0x06040200u);                                                           \
-                }                                                                                                                    \
-                asm volatile("" : "+v"(packed)); /* (packed here, not where the tail first looks at it: four bins would stay live) */ \
-                cache[c * kRegsPerVec + h] = packed;                                                                                 \
-            }                                                                                                                        \
+            uint32_t bins[4];                                                                                                                \
+            _Pragma("unroll") for (int e = 0; e < 4; ++e) {                                                                                  \
+                uint32_t bits = w[e];                                                                                                        \
+                if (MASKED) bits |= static_cast<uint32_t>((bw << (31 - e)) >> 31);                                                           \
+                const float x = __uint_as_float(bits);                                                                                       \
+                vm = fmaxf(vm, x);                                                                                                           \
+                const float tc = bin_coord(aq, c64, x, tail_f);                                                                              \
+                bins[e] = static_cast<uint32_t>(tc);                                                                                         \
+                WSL_HIST_ADD(bins[e], tc);                                                                                                   \
+            }                                                                                                                                \
+            const uint32_t lo2 = __builtin_amdgcn_perm(bins[1], bins[0], 0x0c0c0400u);                                                       \
+            uint32_t packed = __builtin_amdgcn_perm(bins[3], bins[2], 0x04000c0cu) | lo2;                                                    \
+            asm volatile("" : "+v"(packed)); /* (packed here, not where the tail first looks at it: four bins would stay live) */            \
+            cache[c] = packed;                                                                                                               \
             if (early) {                                                                                                             \
                 vm_early[c < kEarly * kLeanBatch ? c : 0] = vm;                                                                      \
             } else {                                                                                                                 \
@@ -557,7 +528,7 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const uint32_t row,
         }                                                                                                                            \
     }
 #ifndef WS_EXP_NOATOMIC
-#define WSL_HIST_ADD(bin, tc) atomicAdd(reinterpret_cast<unsigned long long*>(&myhist[hist_word(bin)]), bin_word(tc))
+#define WSL_HIST_ADD(bin, tc) atomicAdd(reinterpret_cast<unsigned long long*>(&myhist[bin]), bin_word(tc))
 #else
 #define WSL_HIST_ADD(bin, tc) m = fmaxf(m, __uint_as_float(static_cast<uint32_t>(bin_word(tc))))
 #endif
@@ -659,7 +630,7 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const uint32_t row,
             WSL_SWEEP_BATCH(bt, false)
         } else {  // past the row (no way out of the loop here: with one, the cache no longer stays in registers)
 #pragma unroll
-            for (int u = 0; u < kLeanBatch * kRegsPerVec; ++u) cache[bt * kLeanBatch * kRegsPerVec + u] = 0u;
+            for (int u = 0; u < kLeanBatch; ++u) cache[bt * kLeanBatch + u] = 0u;
         }
         WSL_NEXT_LOAD(bt, bt % kRing);
     }
@@ -721,7 +692,7 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const uint32_t row,
                         if (rf < stage_cap && i >= early_end) vec[k] = stage[rf];
                         else vec[k] = xv[i >> kTokLog];
                     } else {  // (a token past the row's whole vectors, as the first token of a vector of its own)
-                        const uint32_t b = DT == 0 ? static_cast<const uint32_t*>(rv.base)[i] : static_cast<uint32_t>(static_cast<const uint16_t*>(rv.base)[i]);
+                        const uint32_t b = static_cast<const uint32_t*>(rv.base)[i];
                         vec[k] = make_uint4(b, b, b, b);
                     }
                 }
@@ -732,15 +703,13 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const uint32_t row,
                     const uint32_t w[4] = {vec[k].x, vec[k].y, vec[k].z, vec[k].w};
                     const bool whole = i < whole_end;
                     const uint32_t e_ = whole ? (i & (kTok - 1u)) : 0u;
-                    uint32_t bits = pick4(DT == 0 ? e_ : e_ >> 1, w[0], w[1], w[2], w[3]);
-                    if (DT != 0) bits = (e_ & 1u) ? bits & 0xffff0000u : bits << 16;
+                    const uint32_t bits = pick4(e_, w[0], w[1], w[2], w[3]);
                     const float raw = ((al[k] >> (i & 31u)) & 1u) ? fmaxf(__uint_as_float(bits), -INFINITY) : -INFINITY;
                     if (whole) {  // the vector's tokens that nothing touches count for the maximum here
                         const uint32_t free_bits = (al[k] & ~tw[k]) >> (i & (32u - kTok));
 #pragma unroll
                         for (uint32_t e = 0; e < kTok; ++e) {
-                            const uint32_t b_ = DT == 0 ? w[e & 3u] : ((e & 1u) ? w[(e >> 1) & 3u] & 0xffff0000u : w[(e >> 1) & 3u] << 16);
-                            if ((free_bits >> e) & 1u) mu = fmaxf(mu, __uint_as_float(b_));
+                            if ((free_bits >> e) & 1u) mu = fmaxf(mu, __uint_as_float(w[e]));
                         }
                     }
                     const uint32_t cw = old[k], c = cw & 0xfffffu, n_bias = (cw >> 20) & 0x7ffu;
@@ -760,8 +729,8 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const uint32_t row,
                     first[rk[k]] = i;  // the token id of the rank from here on
                     ma = fmaxf(ma, x);
                     const float t0 = bin_coord(aq, c64, raw, tail_own), t1 = bin_coord(aq, c64, x, tail_own);
-                    atomicAdd(reinterpret_cast<unsigned long long*>(&hist[hist_word(static_cast<uint32_t>(t0))]), 0ull - bin_word(t0));
-                    atomicAdd(reinterpret_cast<unsigned long long*>(&hist[hist_word(static_cast<uint32_t>(t1))]), bin_word(t1));
+                    atomicAdd(reinterpret_cast<unsigned long long*>(&hist[static_cast<uint32_t>(t0)]), 0ull - bin_word(t0));
+                    atomicAdd(reinterpret_cast<unsigned long long*>(&hist[static_cast<uint32_t>(t1)]), bin_word(t1));
                 }
             }
         };
@@ -804,19 +773,6 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const uint32_t row,
             if (hist2) {
                 const ulonglong2 g01 = *reinterpret_cast<const ulonglong2*>(&hist2[bb]), g23 = *reinterpret_cast<const ulonglong2*>(&hist2[bb + 2u]);
                 h[0] += g01.x, h[1] += g01.y, h[2] += g23.x, h[3] += g23.y;
-            }
-#ifndef WS_NO_SWZ
-            if (DT != 0)
-#else
-            if (false)
-#endif
-            {  // (the four words are the four bins' own, in the places hist_word gives them)
-                const uint32_t sw = (bb >> 4) & 3u;
-                const uint64_t w0_ = h[0], w1_ = h[1], w2_ = h[2], w3_ = h[3];
-                h[0] = pick4(sw, w0_, w1_, w2_, w3_);
-                h[1] = pick4(1u ^ sw, w0_, w1_, w2_, w3_);
-                h[2] = pick4(2u ^ sw, w0_, w1_, w2_, w3_);
-                h[3] = pick4(3u ^ sw, w0_, w1_, w2_, w3_);
             }
         }
         double ms[4];
@@ -1062,7 +1018,7 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const uint32_t row,
         {  // the bytes to scan the cache for: lane k looks at the k-th bin of the ranges, the first of a kind is listed
             uint32_t my_bin = lane < nb0 ? static_cast<uint32_t>(r0lo) + lane : static_cast<uint32_t>(r1lo) + (lane - nb0);
             uint32_t n_bins = nb0 + nb1;
-            if (ok && n_bins > (kCacheShift == 0u ? 8u : kLeanMaxBins)) {  // (more bins than the scan takes bytes)
+            if (ok && n_bins > 8u) {  // (more bins than the scan takes bytes)
                 // (uniform, rare) A peaked row: a handful of tokens, dozens of bins apart, where the draw may land. Only
                 // the bins that hold a token count: the lanes look them up in the histogram, 64 bins a round, and those
                 // with a token move up to the first lanes in order.
@@ -1071,7 +1027,7 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const uint32_t row,
                     const uint32_t k = base + lane;
                     const uint32_t b = k < nb0 ? static_cast<uint32_t>(r0lo) + k : static_cast<uint32_t>(r1lo) + (k - nb0);
                     uint64_t word = 0ull;
-                    if (k < nb0 + nb1) word = hist[hist_word(b)] + (hist2 ? hist2[hist_word(b)] : 0ull);
+                    if (k < nb0 + nb1) word = hist[b] + (hist2 ? hist2[b] : 0ull);
                     const uint64_t has = __ballot((word >> kCountShift) != 0ull);
                     // lane n_found + j takes the j-th bin of this round that holds a token
                     const uint32_t want_j = lane - n_found;
@@ -1089,7 +1045,7 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const uint32_t row,
                 n_bins = n_found;
                 ok = ok && n_found <= kLeanMaxBins;
             }
-            const uint32_t my_byte = (my_bin >> kCacheShift) & 0xffu;
+            const uint32_t my_byte = my_bin & 0xffu;
             bool is_first = lane < n_bins && lane < kLeanMaxBins;
 #pragma unroll
             for (uint32_t j = 0; j + 1u < kLeanMaxBins; ++j) {
@@ -1146,15 +1102,15 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const uint32_t row,
         {
             const uint32_t c4[4] = {by0.x, by0.y, by0.z, by0.w};
             const uint32_t n = min(4u, nt);
-            if (n == 1u) lean_scan<1, false, DT>(cache, c4, xg, H, list, &s_w[0], kListCap, nv);
-            else if (n == 2u) lean_scan<2, false, DT>(cache, c4, xg, H, list, &s_w[0], kListCap, nv);
-            else if (n == 3u) lean_scan<3, false, DT>(cache, c4, xg, H, list, &s_w[0], kListCap, nv);
-            else lean_scan<4, false, DT>(cache, c4, xg, H, list, &s_w[0], kListCap, nv);
+            if (n == 1u) lean_scan<1, false>(cache, c4, xg, H, list, &s_w[0], kListCap, nv);
+            else if (n == 2u) lean_scan<2, false>(cache, c4, xg, H, list, &s_w[0], kListCap, nv);
+            else if (n == 3u) lean_scan<3, false>(cache, c4, xg, H, list, &s_w[0], kListCap, nv);
+            else lean_scan<4, false>(cache, c4, xg, H, list, &s_w[0], kListCap, nv);
         }
         if (nt > 4u) {  // uniform, rare: a second round for the other bytes, every find through the list
             const uint4 by1 = *reinterpret_cast<const uint4*>(&sel.bytes[4]);
             const uint32_t c4[4] = {by1.x, nt > 5u ? by1.y : by1.x, nt > 6u ? by1.z : by1.x, nt > 7u ? by1.w : by1.x};
-            lean_scan<4, true, DT>(cache, c4, xg, H, list, &s_w[0], kListCap, nv);
+            lean_scan<4, true>(cache, c4, xg, H, list, &s_w[0], kListCap, nv);
         }
         WSL_MARK(20);
         // touched tokens whose adjusted logit lies in the ranges
@@ -1232,7 +1188,7 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const uint32_t row,
             bool ok = live;
             if (!(en[r].x & kListAdjusted)) {
                 if (en[r].x & kListNeedsLoad)
-                    x = __uint_as_float(DT == 0 ? static_cast<const uint32_t*>(rv.base)[id] : static_cast<uint32_t>(static_cast<const uint16_t*>(rv.base)[id]) << 16);
+                    x = __uint_as_float(static_cast<const uint32_t*>(rv.base)[id]);
                 x = fmaxf(x, -INFINITY);
                 ok = ok && (!MASKED || is_allowed(rv, id)) && !is_touched(rv, id) && in_ranges(x);
             }
@@ -1262,7 +1218,7 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const uint32_t row,
     if (s_w[5] != n_list) WSL_FAIL(7);  // the histogram and the gather disagree
     // ---- the candidates in order (logit descending, id ascending): their 64-bit keys sorted by buckets. A bucket is
     // a bin of the ranges (eight at most) and, inside the bin, a 32nd of the span of the bin's logits - or, when all
-    // its candidates tie, as bf16 rows have them by the hundred, a 32nd of the vocabulary's ids: either way some dozens
+    // its candidates tie, a 32nd of the vocabulary's ids: either way some dozens
     // of keys to compare with, and no limit on ties. A key's place is the start of its bucket plus the number of larger
     // keys among the bucket's members, which it reads once all keys lie bucket by bucket.
     constexpr int kRounds = kLeanMaxList / WS_BLOCK;  // the candidates at places kRounds t .. kRounds t + kRounds - 1 of the order
@@ -1560,11 +1516,11 @@ __device__ __noinline__ void three_pass_row(LeanArgPtr Ap, const uint32_t row) {
 }
 
 // MASKED: the batch has an allow mask (a kernel of its own: one build carrying both paths spilled far more registers)
-template <bool MASKED, int DT>
+template <bool MASKED>
 __global__ void __launch_bounds__(WS_BLOCK) lean_batch_kernel(BatchArgs A) {
     __shared__ LeanShared shared;
     const uint32_t row = blockIdx.x;
-    const bool done = lean_row<MASKED, DT>(A, row, shared);
+    const bool done = lean_row<MASKED>(A, row, shared);
 #ifndef WS_LEAN_NO_FALLBACK
     if (done) return;
     __syncthreads();  // whatever the lean path left in LDS is dead
