@@ -91,6 +91,7 @@ __device__ __forceinline__ void short_sort(uint64_t* list, const uint32_t n_list
         }
         dmax = wave_max(dmax);
         dsum = wave_sum(dsum);
+        __syncthreads();  // (the row's maximum and sum were read from these words, and not every wave need have come by)
         if ((t & 63u) == 0u) {
             S.red_f[t >> 6] = dmax;
             S.red_d[t >> 6] = static_cast<double>(dsum);
