@@ -1,0 +1,121 @@
+"""GPU: short-list rows two a compute unit (ws_twin.h), which batches of more rows than compute units get, through the C ABI against the
+CPU oracle on identical seeded inputs: vocabularies either side of a vector, of a chunk and of the sample, the tables behind the bitmap and
+in the list's place, ids at hand and behind those, repeated bias entries, rows whose largest tokens lie far above the others, and the rows
+left to the three-pass code. Bars as in test_gpu_short.py."""
+import numpy as np
+import pytest
+import torch
+
+import gpu_cases as gc
+from test_gpu_short import _odd, run_short
+
+pytestmark = pytest.mark.gpu
+
+
+def rows_of():
+    return torch.cuda.get_device_properties(0).multi_processor_count + 1
+
+
+def some(rows, step=31):
+    return sorted({0, 1, rows - 1, *range(0, rows, step)})
+
+
+def twice_biased(c):
+    """Every third row's first bias entries name one token three times, a token of its history."""
+    for r in range(0, c["rows"], 3):
+        c["bias_ids"][r, :3] = c["hist"][r, 0]
+    return c
+
+
+SIZES = [8, 9, 31, 2047, 2049, 8191, 16384, 16385, 16387, 18432, 18437, 20479, 50257]
+
+
+@pytest.mark.parametrize("dtype,allowed", [("f32", None), ("f32", 0.3), ("bf16", None), ("bf16", 0.6)])
+@pytest.mark.parametrize("V", SIZES)
+def test_vocabularies_off_every_boundary(V, dtype, allowed):
+    """Top-k rows and, every fourth, rows with a min-p alone (bf16: of the vocabularies that this kernel takes; ws_code.h has the others)."""
+    rows = rows_of()
+    c = _odd(rows, V, dtype, top_k=min(20, V), n_hist=min(300, V), n_bias=min(20, V), allowed=allowed)
+    c["top_k"][::4] = 0
+    c["min_p"][::4] = 0.02
+    c["top_p"][1::4] = 1.0
+    c["min_p"][2::4] = 0.1
+    if allowed is not None:
+        c["allow"][:, 0] |= 7  # (no row without a token)
+    run_short(c if V < 300 else twice_biased(c), 1, rows=some(rows), handed_back=rows if V < 64 else 2)
+
+
+@pytest.mark.parametrize("V,n_hist,n_bias,top_k,allowed", [(50257, 0, 0, 50, None), (50257, 0, 0, 50, 0.2), (50257, 1, 0, 3, None), (50257, 0, 1, 600, 0.5), (50257, 4608, 20, 50, None),
+                                                           (50257, 4609, 0, 50, None), (40000, 9000, 1000, 200, None), (151936, 7000, 500, 1000, None), (262144, 8192, 500, 1000, 0.1),
+                                                           (400000, 500, 20, 50, None)])
+def test_histories_bias_lists_and_wide_top_k(V, n_hist, n_bias, top_k, allowed):
+    """Tables of every size, a row's last ids at hand and the first behind them; one, two and eight candidates a thread."""
+    rows = rows_of()
+    c = _odd(rows, V, top_k=top_k, n_hist=max(n_hist, 1), n_bias=max(n_bias, 1), allowed=allowed)
+    if not n_hist:
+        c["hist"] = None
+    if not n_bias:
+        c["bias_ids"] = c["bias_vals"] = None
+    c["top_p"][::2] = 1.0
+    _, smp = run_short(c if n_hist == 0 or n_bias < 3 else twice_biased(c), 1, rows=some(rows, 67))
+    was = [x.clone() for x in (smp.token, smp.n_kept, smp.stats, smp.kept_ids)]
+    for _ in range(4):  # every row again: the same, whatever the two of a compute unit were at
+        smp.kept_ids.fill_(-7)
+        smp.run()
+        assert torch.equal(was[0], smp.token) and torch.equal(was[1], smp.n_kept) and torch.equal(was[3], smp.kept_ids)
+        assert torch.allclose(was[2], smp.stats, rtol=1e-6, atol=0)  # (the order of the sums differs)
+
+
+@pytest.mark.parametrize("V,allowed", [(50257, None), (50259, 0.9)])
+def test_min_p_rows_with_lists_of_thousands(V, allowed):
+    """Floors that 1000 to 7000 tokens pass; many a row's sample puts its own floor too low for the list, and the row is listed again.
+    Left to the three-pass code: rows whose list does not fit, and no others."""
+    rows = rows_of()
+    c = _odd(rows, V, top_k=0, min_p=0.0043, n_hist=200, n_bias=1, allowed=allowed)
+    c["bias_ids"] = c["bias_vals"] = None
+    c["logits"] = (np.random.default_rng(5).standard_normal((rows, V), dtype=np.float32) * 2).astype(np.float32)
+    c["inv_t"][:] = 1.0
+    c["hist"][:] = np.argpartition(c["logits"], 200, axis=1)[:, :200]  # (tokens that no list has)
+    _, smp = run_short(c, 1, rows=some(rows), kept_cap=4096, handed_back=rows)
+    x, m = c["logits"], gc.pkg()
+    if allowed is not None:
+        on = np.unpackbits(c["allow"].view(np.uint8), axis=1, bitorder="little")[:, :V].astype(bool)
+        x = np.where(on, x, -np.inf)
+    listed = (x > x.max(axis=1, keepdims=True) + np.log(0.0043)).sum(axis=1)
+    back = (smp.flags.cpu().numpy() & m.FLAG_ROUTE_HANDED_BACK) != 0
+    assert not back[listed < 3900].any() and back[listed > 4400].all()  # (0.02 e-folds more than the floor: a few per cent)
+    assert (listed < 3900).sum() > rows // 4 and back.any()
+
+
+@pytest.mark.parametrize("dtype,V", [("f32", 100003), ("bf16", 262144)])
+def test_rows_whose_largest_tokens_lie_far_above_the_others(dtype, V):
+    """Cold rows: a few tokens 58 to 76 units of the exponent above the rest; of most rows one or two are in the sample, of some none is."""
+    rows = rows_of()
+    c = _odd(rows, V, dtype, top_k=50, n_hist=64, n_bias=0)
+    c["inv_t"][:] = 20.0
+    rng = np.random.default_rng(rows)
+    x = (rng.standard_normal((rows, V), dtype=np.float32) * 0.5)
+    for r in range(rows):
+        x[r, rng.integers(0, V, 6)] = (5.0 + 0.5 * rng.random()) + np.array([0.0, 0.013, 0.04, 0.11, 0.3, 0.4], np.float32)
+        c["hist"][r, 0] = int(x[r].argmax())
+    c["logits"] = gc.f32_to_bf16_bits(x) if dtype == "bf16" else x
+    run_short(c, 1, rows=some(rows, 17), kept_cap=64, handed_back=rows // 50, top_k_max=50)
+
+
+def test_rows_left_to_the_three_pass_code():
+    """Rows that break the batch's word, rows of one value (more ties than the list holds), rows without a token, NaNs and infinities;
+    the rows between them are the kernel's own."""
+    rows, V = rows_of() + 300, 20001
+    c = _odd(rows, V, top_k=40, n_hist=100, n_bias=0)
+    c["top_k"][0] = 0
+    c["top_k"][1] = 1025
+    c["logits"][2:rows:50] = 1.5
+    c["logits"][3, :] = -np.inf
+    c["logits"][3, 77] = 0.25
+    c["logits"][4, 100:200] = np.nan
+    c["logits"][5, ::2] = -np.inf
+    res, smp = run_short(c, 1, rows=list(range(10)) + some(rows), handed_back=rows, top_k_max=40)
+    m = gc.pkg()
+    back = (smp.flags.cpu().numpy() & m.FLAG_ROUTE_HANDED_BACK) != 0
+    assert back[[0, 1, 3]].all() and back[2:rows:50].all()
+    assert int(back.sum()) <= 5 + len(range(2, rows, 50)), np.flatnonzero(back)

@@ -17,6 +17,7 @@ SRC_FUSED = os.path.join(HERE, "csrc", "ws_fused.hip")  # the single-sweep sampl
 SRC_SPLIT = os.path.join(HERE, "csrc", "ws_split.hip")  # the same kernel for rows split over several workgroups
 SRC_KEPT = [os.path.join(HERE, "csrc", f) for f in ("ws_fused_kept.hip", "ws_split_kept.hip")]  # both once more, with the kept-set dump
 SRC_SHORT = os.path.join(HERE, "csrc", "ws_short.hip")  # the short-list kernel for batches whose rows all have a bounded top-k
+SRC_TWIN = os.path.join(HERE, "csrc", "ws_twin.hip")  # the same for rows that are not shared, two of them a compute unit
 SRC_CODE = os.path.join(HERE, "csrc", "ws_code.hip")  # bf16 rows, held in registers and counted by value
 SRC_FEW = os.path.join(HERE, "csrc", "ws_few.hip")  # short-list rows shared between workgroups that hold them in registers
 SRC_TOP = os.path.join(HERE, "csrc", "ws_top.hip")  # top-k lists and draft draws of few rows, shared the same way
@@ -49,7 +50,7 @@ def build(verbose=True):
     # the translation units and the bare code object side by side (each takes a minute or two), then the link
     objdir = os.path.join(HERE, "csrc", "obj")
     os.makedirs(objdir, exist_ok=True)
-    srcs = (SRC, SRC_FUSED, SRC_SPLIT, *SRC_KEPT, SRC_LEAN, SRC_CODE, SRC_SHORT, SRC_FEW, SRC_TOP)
+    srcs = (SRC, SRC_FUSED, SRC_SPLIT, *SRC_KEPT, SRC_LEAN, SRC_CODE, SRC_SHORT, SRC_TWIN, SRC_FEW, SRC_TOP)
     objs = [os.path.join(objdir, os.path.basename(src)[:-4] + ".o") for src in srcs]
     jobs = [[hipcc, *FLAGS, "-fPIC", "-c", "-o", obj, src] for obj, src in zip(objs, srcs)]
     jobs.append([hipcc, *FLAGS, "--genco", "-o", co, SRC])

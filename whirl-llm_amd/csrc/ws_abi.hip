@@ -37,6 +37,10 @@ int prepare_lean(unsigned lds_limit);
 // ws_short.hip: the short-list kernel for batches whose rows all have a bounded top-k
 int launch_short(hipStream_t stream, const BatchArgs& a, unsigned lds_bytes, unsigned lds_limit);
 int prepare_short(unsigned lds_limit);
+int launch_short_rest(hipStream_t stream, const BatchArgs& a, unsigned blocks, unsigned lds_bytes, unsigned lds_limit);
+// ws_twin.hip: the same for rows that are not shared, two of them a compute unit
+int launch_twin(hipStream_t stream, const BatchArgs& a, unsigned lds_bytes, unsigned lds_limit);
+int prepare_twin(unsigned lds_limit);
 // ws_code.hip: bf16 rows, held in registers and counted by value
 int launch_code(hipStream_t stream, const BatchArgs& a, unsigned rows, unsigned lds_bytes, unsigned lds_limit);
 int prepare_code(unsigned lds_limit);
@@ -70,6 +74,8 @@ constexpr uint32_t kStaticLds = 4096u;
 #endif
 // the short-list kernel's own words and those of both builds of the three-pass code it calls (8.2 KiB)
 constexpr uint32_t kStaticShort = 9216u;
+// the same for the kernel of two rows a compute unit, which calls nothing
+constexpr uint32_t kStaticTwin = 1024u;
 // the same for the kernel of few rows
 constexpr uint32_t kStaticFew = 10240u;
 // the same for the kernel of bf16 rows
@@ -94,6 +100,8 @@ struct BatchPlan {
     uint32_t lean_fb_tie;
     bool shortlist;       // the short-list kernel takes the batch: every row has a top-k of at most top_k_max (the caller's word)
     uint32_t short_ab, short_cnt, short_total, short_fb_tie, short_fb_ab;  // its LDS: bitmap at short_ab, rank words at short_cnt
+    bool twin;            // its rows go two a compute unit (ws_twin.h)
+    uint32_t twin_ab, twin_tabs, twin_total;  // LDS of those: the bitmap, the tables, all
     uint32_t few_parts, few_total;  // short-list rows shared between this many workgroups each (0: not), and the dynamic LDS of those
     bool code;            // the kernel of bf16 rows takes the batch
     uint32_t code_head;   // its masses (BatchArgs)
@@ -192,6 +200,14 @@ void code_plan(const ws_batch* b, uint64_t cap, uint64_t maps, uint64_t spare_by
     }
 }
 
+// Rows of the short-list kind that go two a compute unit (ws_twin.h): more of them than compute units. Its sweep is no faster than ws_short.h's, one
+// row a unit, and the kernel behind it that looks for rows left over takes 3 us: 256 rows of 151936, ws_short.h and ws_twin.h, 44.7 / 48.6; 300 rows
+// 77.0 / 65.0, 512 82.2 / 73.2, 1000 of 8000 55.8 / 38.5.
+bool twin_rows(const ws_batch* b) {
+    const int cus = compute_units();
+    return cus > 0 && b->rows > static_cast<uint32_t>(cus);
+}
+
 // bf16 rows of the short-list kind: ws_code.h, ws_few.h or ws_short.h. Few rows are ws_few.h's: it shares them, and its lists are short -
 // but a list of some hundred keys has to be sorted, which costs more than counting a row that is not long, and two workgroups a row
 // are not much of a share. Microseconds, ws_few.h and ws_code.h (1000-id histories): top-k 50: 64 rows of 50257 16.0 / 18.4, 100 rows 19.9 /
@@ -200,17 +216,40 @@ void code_plan(const ws_batch* b, uint64_t cap, uint64_t maps, uint64_t spare_by
 // min-p alone: 100 of 50257 18.2 / 18.5, 128 of 60000 18.9 / 19.5. What ws_few.h does not take: top-k 50, ws_short.h and ws_code.h: 200 of 32000 24.9 /
 // 16.5, 1000 of 8000 with a min-p 62.2 / 59.1, 256 of 151936 52.2 / 29.4, 400 of 262144 118.6 / 90.0. Rows without a top-k have a short list and nothing to
 // estimate: 150 of 20000 14.3 / 16.5, 1000 of 8000 46.2 / 56.3, 300 of 40000 31.9 / 31.2, 256 of 50257 22.5 / 20.0, 256 of 151936 45.1 / 30.4; longer than the
-// registers hold and in four slices or more: 60 of 262144 32.0 / 37.9, in two: 100 of 262144 44.7 / 38.2.
+// registers hold and in four slices or more: 60 of 262144 32.0 / 37.9, in two: 100 of 262144 44.7 / 38.2. More rows than compute units are
+// ws_twin.h's where its sweep is a small part of the row or the row is longer than the registers hold, and the list is short: 1000 rows, top-k 50 (and
+// 300), ws_twin.h and ws_code.h: of 8000 36.3 / 54.4 (47.1 / 57.2), of 16000 44.7 / 55.4 (59.6 / 59.5), of 24000 52.5 / 56.4 (71.7 / 60.2); 400 of 16000,
+// top-k 50, 24.7 / 27.9; 400 of 180000 67.1 / 61.7, 700 of 200000, top-k 100, 118 / 104, 400 of 262144, top-k 50, 80.9 / 96.6, 1024 154 / 191, 512
+// with a top-k of 300 100.8 / 99.9.
 void code_or_short(const ws_batch* b, BatchPlan& p) {
     const bool by_k = b->top_k && b->top_k_max >= 1u;
     if (p.few_parts) {
         const bool long_lists = b->top_k_max > 512u ? b->vocab <= 163840u : b->top_k_max > 256u && b->vocab <= 40960u;
         p.code = by_k && (long_lists || (p.few_parts <= 2u && b->vocab > 32768u));
         if (p.code) p.few_parts = 0;
-    } else if (!by_k) {
+    } else if (by_k) {
+        p.code = !(twin_rows(b) && b->top_k_max <= 128u && (b->vocab <= 16384u || b->vocab >= 245760u));
+    } else {
         p.code = b->vocab > 40960u && !(b->vocab > 163840u && short_split_log2(b) >= 2u);
     }
     if (p.code) p.workspace = p.workspace_min = 0;
+}
+
+// LDS of a row of ws_twin.h: the list, the bitmap, the tables behind it; or, where that is more than half a compute unit's and the
+// other way is not, the tables below the bitmap, in the upper part of the list's place as far as they have to (8 KiB of it stay theirs alone: the
+// touched tokens above the threshold are listed while the tables are in use).
+void twin_plan(uint32_t nW, uint64_t cap, BatchPlan& p) {
+    const uint64_t map = uint64_t{nW} * 4u, tabs = ((uint64_t{nW} * 2u + 3u) & ~uint64_t{3}) + ((cap * 2u + 3u) & ~uint64_t{3});
+    const uint64_t half = kMaxLds / 2u - kStaticTwin, list = 32768u;
+    uint64_t ab = list, tabs_at = list + map, total = list + map + tabs;
+    if (total > half && map + list <= half && map + tabs + 8192u <= half) {
+        ab = (half - map) & ~uint64_t{15};
+        tabs_at = (ab - tabs) & ~uint64_t{3};
+        total = ab + map;
+    }
+    p.twin_ab = static_cast<uint32_t>(ab);
+    p.twin_tabs = static_cast<uint32_t>(tabs_at);
+    p.twin_total = static_cast<uint32_t>(total);
 }
 
 // few: whether ws_few.h is considered
@@ -309,6 +348,7 @@ BatchPlan plan_batch(const ws_batch* b, bool few = true) {
                 if (p.short_fb_tie + spare_bytes > st) st = p.short_fb_tie + spare_bytes;
             }
             p.short_total = static_cast<uint32_t>(st);
+            twin_plan(nW, cap, p);
         }
     }
     code_plan(b, cap, maps, spare_bytes, p);
@@ -319,6 +359,7 @@ BatchPlan plan_batch(const ws_batch* b, bool few = true) {
         if (few) few_plan(b, cap, maps, p);
         if (p.code) code_or_short(b, p);
         if (!p.code && !p.few_parts && (p.split_log2 = short_split_log2(b)) != 0u) p.workspace = p.workspace_min = uint64_t{b->rows} * ws::kShortSplitRowBytes;
+        p.twin = !p.code && !p.few_parts && !p.split_log2 && twin_rows(b);
         p.err = WS_OK;
         return p;
     }
@@ -418,6 +459,7 @@ int prepare_all() {
     if (const int e = ws::prepare_split_kept(kMaxLds - kStaticLds); e != 0) return e;
     if (const int e = ws::prepare_lean(kMaxLds - kStaticLean); e != 0) return e;
     if (const int e = ws::prepare_code(kMaxLds - kStaticCode); e != 0) return e;
+    if (const int e = ws::prepare_twin(kMaxLds - kStaticTwin); e != 0) return e;
     if (const int e = ws::prepare_few(kMaxLds - kStaticFew); e != 0) return e;
     if (const int e = ws::prepare_top(); e != 0) return e;
     return ws::prepare_short(kMaxLds - kStaticShort);
@@ -759,10 +801,17 @@ int sample_batch_on(void* stream, const ws_batch* b, const BatchPlan& p, unsigne
         return ws::launch_code(S(stream), a, b->rows, p.code_total, kMaxLds - kStaticCode);
     }
     if (p.shortlist) {
-        a.lds_ab = p.short_ab;
-        a.lds_cnt = p.short_cnt;
         a.fb_lds_tie = p.short_fb_tie;
         a.fb_lds_ab = p.short_fb_ab;
+        if (p.twin) {
+            a.work = nullptr;
+            a.lds_ab = p.twin_ab;
+            a.lds_cnt = p.twin_tabs;
+            if (const int e = ws::launch_twin(S(stream), a, p.twin_total, kMaxLds - kStaticTwin); e != 0) return e;
+            return ws::launch_short_rest(S(stream), a, static_cast<uint32_t>(compute_units()), p.short_total, kMaxLds - kStaticShort);
+        }
+        a.lds_ab = p.short_ab;
+        a.lds_cnt = p.short_cnt;
         a.work = a.split_log2 ? work : nullptr;
         return ws::launch_short(S(stream), a, p.short_total, kMaxLds - kStaticShort);
     }

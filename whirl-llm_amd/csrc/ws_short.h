@@ -13,7 +13,7 @@
 //     against the largest, the draw by inverse CDF with the row's uniform.
 // A row for which a check fails, whose list runs over, or that has neither a top-k nor a min-p after all, is handed to the
 // three-pass code of ws_sample.h inside the same launch (WS_FLAG_ROUTE_HANDED_BACK).
-// Few rows are shared between workgroups by the kernel of ws_few.h, which ends with the same sort and rules; those it has no
+// More rows than compute units are ws_twin.h's. Few rows are shared between workgroups by the kernel of ws_few.h, which ends with the same sort and rules; those it has no
 // registers or lists for are shared here: each part lists its slice against its own threshold and leaves list, maximum and sum in
 // the row's workspace, and the part that arrives last - a ticket, nobody waits - takes them all and finishes the row. The
 // top_k largest of the merged list are the row's when the k-th of them lies above every part's threshold.
@@ -30,6 +30,7 @@ constexpr uint32_t kShortMaxK = 1024u;  // largest top-k: one candidate a thread
 constexpr uint32_t kShortHead = 8u;     // head of a slice: vectors a thread asked for before anything else
 constexpr uint32_t kShortSample = 8u;   // of those, the vectors a thread whose tokens the threshold is fitted to (32768 tokens of fp32)
 constexpr uint32_t kRouteShort = 0x2000u;
+constexpr uint32_t kTwinRest = 0xffffffffu;  // in `flags`, between two kernels: a row of ws_twin.h's left to the three-pass code (no set of flags has every bit)
 
 
 #ifdef WS_SHORT_TIMERS
@@ -181,10 +182,10 @@ __device__ __forceinline__ void short_rules(uint64_t* list, const uint32_t row, 
         if (Ap->entropy) Ap->entropy[row] = log(Zk_) - e_ln_e / Zk_;
         if (Ap->query_prob) Ap->query_prob[row] = e_query / Zk_;
     };
-    constexpr uint32_t KC = kShortCap / WS_BLOCK;  // candidates a thread when there are more than one a thread (a wide min-p floor)
-    uint64_t wkey[KC];
-    if (n_cand > WS_BLOCK) {
-        // thread t has the candidates at places KC t .. KC t + KC - 1 of the order; the same rules
+    // more candidates than threads (a wide top-k, a wide min-p floor): thread t has those at places KC t .. KC t + KC - 1 of the order; the same rules
+    auto several = [&](auto kc) __attribute__((always_inline)) {
+        constexpr uint32_t KC = decltype(kc)::value;
+        uint64_t wkey[KC];
         double e[KC], cin[KC], cex[KC], tot = 0.0;
 #pragma unroll
         for (uint32_t j = 0; j < KC; ++j) {
@@ -277,6 +278,11 @@ __device__ __forceinline__ void short_rules(uint64_t* list, const uint32_t row, 
             sq = block_sum(sq, S.red_d);
             if (t == 0) write_more(se, sq, Zk);
         }
+    };
+    if (n_cand > 2u * WS_BLOCK) {
+        several(std::integral_constant<uint32_t, kShortCap / WS_BLOCK>{});
+    } else if (n_cand > WS_BLOCK) {
+        several(std::integral_constant<uint32_t, 2u>{});
     } else if (n_cand <= 64u) {
         // the usual case, a top-k of a few dozen: one wave, a candidate a lane, no barrier and no atomic
         if (wv == 0u) {
@@ -384,10 +390,10 @@ __device__ __forceinline__ void short_rules(uint64_t* list, const uint32_t row, 
         __syncthreads();
         if (n_cand <= 64u) n3 = S.s_w[7];
         if (n_cand > WS_BLOCK) {
-#pragma unroll
-            for (uint32_t j = 0; j < KC; ++j)
-                if (KC * t + j < n3)
-                    list[KC * t + j] = (static_cast<uint64_t>(static_cast<uint32_t>(wkey[j])) << 32) | static_cast<uint32_t>(__float_as_uint(unkey32(static_cast<uint32_t>(wkey[j] >> 32))));
+            for (uint32_t k = t; k < n3; k += WS_BLOCK) {
+                const uint64_t key_ = list[k];
+                list[k] = (static_cast<uint64_t>(static_cast<uint32_t>(key_)) << 32) | __float_as_uint(unkey32(static_cast<uint32_t>(key_ >> 32)));
+            }
         } else if (t < n3) {
             list[t] = (static_cast<uint64_t>(0xffffffffu - id) << 32) | __float_as_uint(x);
         }

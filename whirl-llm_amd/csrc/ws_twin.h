@@ -1,0 +1,565 @@
+// The short-list sampler (ws_short.h) for batches of more rows than compute units: 512 threads a row and tables small enough that a compute
+// unit holds two rows.
+//
+// What bounds it: memory while rows are swept, and nothing while they are not. 1024 threads with a unit to themselves took 177K clocks
+// for a row of 262144 tokens, a tenth of them allowed, with a history of 8192 and a top-k of 1000, 80K of them without a sweep: the tables, the
+// threshold, the sort, the rules. Here a unit's other row sweeps in the meantime, as far as the two are not at the same place (they start together);
+// a row of a small vocabulary is all such stretches, and two of them are at work instead of one. Microseconds, ws_short.h and this: 1024 rows as above 389 / 323,
+// the same without history 266 / 239; top-k 50, 1000-id histories: 512 of 151936 83.8 / 73.3, 300 of 151936 77.2 / 63.9, 1000 of 50257 108 / 72.9, 1000 of 8000
+// 55.9 / 38.1; min-p alone, 1000 of 151936 149 / 139. (1024 of 262144 with a top-k of 50: 195, 5.5 TB/s.)
+//
+// Against ws_short.h the touched tokens come before the sweep, not behind it: their tables are dead when it begins and can lie where the list
+// will be. A history entry's count, a token's bias marks and its claim are 16 bits, not 48: a token is claimed by clearing its word, and where a bias entry
+// names it only those claim it, so that nobody has to look the entry up. Rows for which a check fails are marked in `flags`, and a
+// kernel launched behind this one gives them to the three-pass code, which needs a unit's whole LDS.
+// Tried and dropped: the workgroups of half the rows started later (no faster at any delay up to 80K clocks); all batches asked for before the threshold, or
+// the ids before the sample (both within 1 %); the mask's words kept in registers for the second use (spills: 339 us against 330).
+#pragma once
+#include "ws_short.h"
+
+namespace ws {
+
+constexpr uint32_t kTwinBins = 2048u;  // of the sample's logits: 1/32 e-fold each
+constexpr uint32_t kTwinHead = 8u;  // vectors a thread of the sample that the threshold is fitted to
+
+// LDS: the list at 0 (32 KiB; first the sample's bin counts), the bitmap of the touched tokens at lds_ab, and at lds_cnt its 16-bit popcount
+// prefixes and a 16-bit word per rank: history count | kBias | kBiases. These two are dead when the sweep begins, and where a second
+// row would not fit beside them they lie in the upper part of the list's place.
+// Returns false when the row has to go to the three-pass code (uniform over the workgroup; nothing has been written for it).
+template <int DT, bool MASKED>
+__device__ __forceinline__ bool twin_row(const BatchArgs& A, const uint32_t row, ShortShared& S) {
+#ifdef WS_SHORT_TIMERS
+    const long long wss_t0 = clock64();
+    if (threadIdx.x == 0) S.marks[13] = 0.f;
+#endif
+    extern __shared__ __align__(16) unsigned char lds[];
+    constexpr uint32_t TPV = DT == 0 ? 4u : 8u;  // tokens in a 128-bit vector
+    const uint32_t t = threadIdx.x, lane = t & 63u;
+    const uint32_t wv = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(t >> 6)));
+    const uint32_t V = A.vocab, nW = (V + 31u) >> 5;
+    const unsigned char* base = static_cast<const unsigned char*>(A.logits) + static_cast<size_t>(row) * A.row_stride * (DT == 0 ? 4u : 2u);
+    const uint32_t* allow = MASKED ? A.allow + static_cast<size_t>(row) * A.allow_stride : nullptr;
+
+    uint64_t* list = reinterpret_cast<uint64_t*>(lds);
+    uint32_t* head_cnt = reinterpret_cast<uint32_t*>(lds);
+    uint32_t* touched = reinterpret_cast<uint32_t*>(lds + A.lds_ab);
+    uint32_t* invalid = touched;  // (what it holds from the sweep on)
+    uint16_t* wprefix = reinterpret_cast<uint16_t*>(lds + A.lds_cnt);
+    uint32_t* cnt = reinterpret_cast<uint32_t*>(lds + A.lds_cnt + ((nW * 2u + 3u) & ~3u));  // two ranks a word
+    const uint32_t early_slots = A.lds_cnt < A.lds_ab ? min(kShortCap, A.lds_cnt >> 3) : kShortCap;  // of the list, while the tables are needed
+
+    // The row: chunks of a vector a thread, whole ones and at most one that is not, and a few tokens behind the last vector
+    const uint32_t nv = V / TPV, n_odd = V % TPV, n_full = nv / WS_BLOCK;
+    auto vector_at = [&](uint32_t j) __attribute__((always_inline)) {
+        const LooseVec v = *reinterpret_cast<const LooseVec*>(base + min(j, nv - 1u) * 16u);
+        return make_uint4(v.x, v.y, v.z, v.w);
+    };
+    auto word_at = [&](uint32_t j) __attribute__((always_inline)) { return (min(j, nv - 1u) * TPV) >> 5; };
+
+    // The sample: 8 of the row's chunks of a vector a thread, evenly spread over it (a vocabulary's first ids are its frequent tokens).
+    const uint32_t spread = max(1u, n_full / kTwinHead);
+    uint4 hq[kTwinHead];
+    uint32_t hna[kTwinHead];
+#pragma unroll
+    for (uint32_t k = 0; k < kTwinHead; ++k) {
+        const uint32_t j = k * spread * WS_BLOCK + t;
+        hq[k] = vector_at(j);
+        hna[k] = MASKED ? allow[word_at(j)] : 0xffffffffu;
+    }
+    // the list's place takes the bin counts first; all tables are cleared while the parameters travel
+    reinterpret_cast<uint4*>(head_cnt)[t] = make_uint4(0u, 0u, 0u, 0u);
+    static_assert(kTwinBins == 4u * WS_BLOCK, "");
+    if (A.hist || A.bias_ids) {
+        for (uint32_t w = t; w < nW; w += WS_BLOCK) touched[w] = 0u;
+        for (uint32_t r = t; r < (A.patch_cap + 1u) >> 1; r += WS_BLOCK) cnt[r] = 0u;
+    }
+    const LeanRowParams P = load_row_params(A, row);
+    WSS_MARK(0);  // parameters in
+    const float inv_t = P.inv_t;
+    const uint32_t top_k = P.top_k, nh = P.nh, nb = P.nb, n_all = nh + nb;
+    const double top_p = P.top_p, min_p = P.min_p;
+    const bool by_k = top_k >= 1u && top_k <= kShortMaxK && top_k <= V;  // the top_k largest decide
+    const bool by_p = top_k == 0u && min_p > 0.0 && min_p <= 1.0;      // no top-k: what the min-p floor lets through decides
+    constexpr uint32_t kBias = 0x4000u, kBiases = 0x8000u;  // a bias entry names the token, a second one does
+    if (!(by_k || by_p) || !(inv_t > 0.f) || n_all > A.patch_cap || nh >= kBias) return false;
+    const int32_t* hist_ids = A.hist + P.h0;
+    const int32_t* bias_ids = A.bias_ids + P.b0;
+    const float* bias_vals = A.bias_vals + P.b0;
+
+    // Loads come back in order, and what is asked for behind the row's own vectors waits for them: the history and bias ids, one sequence, go first
+    // and stay in registers (9 rounds: 4608 of them), and all the tables are built from them while the vectors travel.
+    constexpr uint32_t kIds = 9u, kMore = 4u;
+    uint32_t ids[kIds];
+    auto entry = [&](uint32_t j) __attribute__((always_inline)) {  // (unconditional, as all these loads: one behind a branch makes the compiler wait for every load before it)
+        const int32_t* at = j < nh ? hist_ids + j : (j < n_all ? bias_ids + (j - nh) : reinterpret_cast<const int32_t*>(A.seed));
+        const uint32_t id = static_cast<uint32_t>(*at);
+        return j < n_all ? id : 0xffffffffu;
+    };
+#pragma unroll
+    for (uint32_t k = 0; k < kIds; ++k) {
+        ids[k] = 0xffffffffu;
+        if (k * WS_BLOCK < n_all) ids[k] = entry(k * WS_BLOCK + t);  // uniform
+    }
+    constexpr uint32_t kWords = 16u;  // words a thread of the allow mask (262144 tokens) in registers
+    uint32_t aw[kWords];
+    if (MASKED && n_all) {
+#pragma unroll
+        for (uint32_t k = 0; k < kWords; ++k) aw[k] = allow[min(k * WS_BLOCK + t, nW - 1u)];
+    }
+
+    // the other whole chunks in order
+    uint32_t c_next = spread == 1u ? kTwinHead : 1u, c_skip = spread == 1u ? 0xffffffffu : spread;
+    auto next_chunk = [&]() __attribute__((always_inline)) {
+        const uint32_t c = c_next++;
+        if (c_next == c_skip) {
+            ++c_next;
+            c_skip = c_skip + spread < kTwinHead * spread ? c_skip + spread : 0xffffffffu;
+        }
+        return c;
+    };
+
+    // ---- the bitmap of the touched tokens (of a masked row those that its mask allows: the others count nowhere), their ranks, history
+    // counts and bias entries
+    __syncthreads();  // (the tables are cleared)
+    // a touched token's rank, or none (an id outside of the vocabulary, a token that is masked out)
+    auto rank = [&](uint32_t id) __attribute__((always_inline)) {
+        if (id >= V) return 0xffffffffu;
+        const uint32_t w = touched[id >> 5], b = id & 31u;
+        if (MASKED && !((w >> b) & 1u)) return 0xffffffffu;
+        return static_cast<uint32_t>(wprefix[id >> 5]) + __popc(w & ((1u << b) - 1u));
+    };
+    if (n_all) {
+        auto mark = [&](uint32_t id) {
+            if (id < V) atomicOr(&touched[id >> 5], 1u << (id & 31u));
+        };
+        // entries beyond those in registers, some at a time
+        auto others = [&](auto&& what) {
+            for (uint32_t j0 = kIds * WS_BLOCK; j0 < n_all; j0 += kMore * WS_BLOCK) {
+                uint32_t id[kMore];
+#pragma unroll
+                for (uint32_t k = 0; k < kMore; ++k) id[k] = entry(j0 + k * WS_BLOCK + t);
+#pragma unroll
+                for (uint32_t k = 0; k < kMore; ++k) what(id[k], j0 + k * WS_BLOCK + t);
+            }
+        };
+#pragma unroll
+        for (uint32_t k = 0; k < kIds; ++k)
+            if (k * WS_BLOCK < n_all) mark(ids[k]);  // uniform
+        others([&](uint32_t id, uint32_t) { mark(id); });
+        __syncthreads();
+        if (MASKED) {
+#pragma unroll
+            for (uint32_t k = 0; k < kWords; ++k)
+                if (k * WS_BLOCK + t < nW) touched[k * WS_BLOCK + t] &= aw[k];
+            for (uint32_t w = kWords * WS_BLOCK + t; w < nW; w += WS_BLOCK) touched[w] &= allow[w];
+            __syncthreads();
+        }
+        {  // popcount prefixes: an odd number of consecutive words a thread (no two lanes of a read in one bank)
+            const uint32_t per = ((nW + WS_BLOCK - 1u) / WS_BLOCK) | 1u, w0 = min(t * per, nW), w1 = min(w0 + per, nW);
+            uint32_t local = 0, total;
+            for (uint32_t w = w0; w < w1; ++w) local += __popc(touched[w]);
+            uint32_t run = block_excl_scan(local, S.red_u, &total);
+            for (uint32_t w = w0; w < w1; ++w) {
+                wprefix[w] = static_cast<uint16_t>(run);
+                run += __popc(touched[w]);
+            }
+        }
+        __syncthreads();
+        auto count = [&](uint32_t id, uint32_t j) {
+            const uint32_t r = rank(id), sh = (r & 1u) * 16u;
+            if (r == 0xffffffffu) return;
+            if (j < nh) atomicAdd(&cnt[r >> 1], 1u << sh);
+            else if ((atomicOr(&cnt[r >> 1], kBias << sh) >> sh) & kBias) atomicOr(&cnt[r >> 1], kBiases << sh);
+        };
+#pragma unroll
+        for (uint32_t k = 0; k < kIds; ++k)
+            if (k * WS_BLOCK < n_all) count(ids[k], k * WS_BLOCK + t);  // uniform
+        others(count);
+    }
+    WSS_MARK(1);  // bitmap done
+    // one vector: its tokens as floats, masked-out / touched / NaN ones as -inf
+    auto unpack = [&](uint4 q, uint32_t na, uint32_t j, float (&x)[TPV]) {
+        const uint32_t i0 = j * TPV;
+        uint32_t invalid = 0u;  // bit e: token e does not count here
+        if (MASKED) invalid = ~(na >> (i0 & 31u));
+        if (n_all) invalid |= touched[i0 >> 5] >> (i0 & 31u);
+        const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+        for (uint32_t e = 0; e < TPV; ++e) {
+            uint32_t bits = DT == 0 ? w[e] : ((e & 1u) ? (w[e >> 1] & 0xffff0000u) : (w[e >> 1] << 16));
+            bits |= static_cast<uint32_t>(static_cast<int32_t>(invalid << (31u - e)) >> 31);  // -> NaN
+            x[e] = fmaxf(__uint_as_float(bits), -INFINITY);
+        }
+    };
+
+    // The first two batches behind the sample travel while the threshold is worked out. (A whole chunk's address is the
+    // same register for every thread and a lane's offset: nothing to add or to clamp a vector.)
+    constexpr uint32_t KB = 4;  // vectors a thread and batch, two batches in flight
+    uint4 qa[KB], qb[KB], q_part;
+    uint32_t ca[KB], cb[KB];
+    const uint32_t my_offset = (n_full ? t : min(t, nv - 1u)) * 16u;
+    auto load = [&](uint4 (&q)[KB], uint32_t (&c)[KB]) __attribute__((always_inline)) {
+#pragma unroll
+        for (uint32_t k = 0; k < KB; ++k) {
+            c[k] = next_chunk();
+            const LooseVec v = *reinterpret_cast<const LooseVec*>(base + static_cast<size_t>(min(c[k], max(n_full, 1u) - 1u)) * (WS_BLOCK * 16u) + my_offset);
+            q[k] = make_uint4(v.x, v.y, v.z, v.w);
+        }
+    };
+    load(qa, ca);
+
+    // ---- the threshold: the sample's logits counted in 2048 bins of 1/32 e-fold below the sample's maximum
+    float ref = -INFINITY;
+    {
+        float x[TPV];
+#pragma unroll
+        for (uint32_t k = 0; k < kTwinHead; ++k) {
+            const uint32_t j = k * spread * WS_BLOCK + t;
+            if (j < nv) {
+                unpack(hq[k], hna[k], j, x);
+#pragma unroll
+                for (uint32_t e = 0; e < TPV; ++e) ref = fmaxf(ref, x[e]);
+            }
+        }
+        ref = block_max(ref, S.red_f);
+    }
+    if (!(ref > -INFINITY)) return false;  // (a sample without any token)
+    const float c32 = inv_t * 32.f;
+    float thr = -INFINITY;  // tokens above it are listed
+    const bool whole = nv <= kTwinHead * WS_BLOCK;  // the sample is the row
+    const uint32_t n_sample = whole ? V : kTwinHead * WS_BLOCK * TPV;
+    // Tokens to list: of the row's top_k the sample holds about top_k * n_sample / V, give or take the root of that; the rank in the
+    // sample that the threshold is read off lies six such roots above, half of top_k and 150 tokens of the row at least. (A sample that
+    // is the row: the count is exact but for the tokens of a bin, and twice top_k will do.)
+    uint32_t want = 2u * top_k + 6u;
+    if (!whole) {
+        const float roots = 6.f * __builtin_sqrtf(static_cast<float>(top_k) * static_cast<float>(V) / static_cast<float>(n_sample));
+        want = top_k + max(max(top_k >> 1, 150u), static_cast<uint32_t>(roots)) + 16u;
+    }
+    bool list_all = by_k && whole && want >= V;
+    if (by_p) thr = __fadd_rn(ref, __fdiv_rn(static_cast<float>(log(min_p)) - 0.02f, inv_t));  // (0.02 e-folds below the floor: roundings)
+    if (by_k && !list_all) {
+        // rank in the sample that about `want` tokens of the row lie above
+        const uint64_t r_star64 = (static_cast<uint64_t>(n_sample) * want + V - 1u) / V;
+        const uint32_t r_star = static_cast<uint32_t>(r_star64 < 4u ? 4u : r_star64);
+        uint32_t still = r_star;
+        float top = ref;
+        if (t == 0) S.s_w[0] = 0xffffffffu;  // (the bin, once found; the barrier behind the counting publishes this)
+        // whether the bin is among those counted
+        auto found = [&]() __attribute__((always_inline)) {
+            __syncthreads();
+            constexpr uint32_t PER = kTwinBins / WS_BLOCK;
+            uint32_t c[PER], mine = 0;
+#pragma unroll
+            for (uint32_t k = 0; k < PER; k += 4u) {
+                const uint4 c4 = *reinterpret_cast<const uint4*>(&head_cnt[PER * t + k]);
+                c[k] = c4.x;
+                c[k + 1u] = c4.y;
+                c[k + 2u] = c4.z;
+                c[k + 3u] = c4.w;
+                mine += c4.x + c4.y + c4.z + c4.w;
+            }
+            uint32_t total;
+            const uint32_t before = block_excl_scan(mine, S.red_u, &total);
+            if (before < still && before + mine >= still) {  // the bin in which the sample's r_star-th largest lies
+                uint32_t run = before, b = PER * t;
+#pragma unroll
+                for (uint32_t k = 0; k < PER; ++k) {
+                    if (run < still && run + c[k] >= still) b = PER * t + k;
+                    run += c[k];
+                }
+                S.s_w[0] = b;
+            }
+            __syncthreads();
+            return total;
+        };
+        // The bins near the top are all that matters: first only the tokens within 8 e-folds of the sample's maximum are counted - an LDS
+        // atomic each, and a sixth of the tokens -, the others only when those turn out to be fewer than r_star.
+        // (what is 64 e-folds down - and masked-out tokens, nine in ten of some rows - is not counted: a wave's additions to one
+        // word would queue up sixty-four deep)
+        constexpr float kNear = 256.f, kFar = 2047.f;
+        uint32_t total = 0;
+        for (int round = 0; round < 2; ++round) {  // uniform
+            float x[TPV];
+#pragma unroll
+            for (uint32_t k = 0; k < kTwinHead; ++k) {
+                const uint32_t j = k * spread * WS_BLOCK + t;
+                if (j < nv) {
+                    unpack(hq[k], hna[k], j, x);
+#pragma unroll
+                    for (uint32_t e = 0; e < TPV; ++e) {
+                        const float d = fminf(__fmul_rn(__fsub_rn(top, x[e]), c32), kFar);
+                        if (round == 0 ? d < kNear : (d >= kNear && d < kFar)) atomicAdd(&head_cnt[static_cast<uint32_t>(d)], 1u);
+                    }
+                }
+            }
+            total = found();
+            if (S.s_w[0] != 0xffffffffu) break;
+        }
+        // A row whose largest tokens lie further above the others (a cold one): from the largest of those once more. (The sample is read again:
+        // there are no registers for another copy of the loop above.)
+        for (int more = 0; more < 4 && S.s_w[0] == 0xffffffffu; ++more) {  // uniform
+            still -= total;
+            float below = -INFINITY, x[TPV];
+#pragma unroll 1
+            for (uint32_t k = 0; k < kTwinHead; ++k) {
+                const uint32_t j = k * spread * WS_BLOCK + t;
+                if (j >= nv) break;
+                unpack(vector_at(j), MASKED ? allow[word_at(j)] : 0xffffffffu, j, x);
+#pragma unroll
+                for (uint32_t e = 0; e < TPV; ++e) below = __fmul_rn(__fsub_rn(top, x[e]), c32) >= kFar ? fmaxf(below, x[e]) : below;
+            }
+            reinterpret_cast<uint4*>(head_cnt)[t] = make_uint4(0u, 0u, 0u, 0u);
+            top = block_max(below, S.red_f);
+            if (!(top > -INFINITY)) break;
+#pragma unroll 1
+            for (uint32_t k = 0; k < kTwinHead; ++k) {
+                const uint32_t j = k * spread * WS_BLOCK + t;
+                if (j >= nv) break;
+                unpack(vector_at(j), MASKED ? allow[word_at(j)] : 0xffffffffu, j, x);
+#pragma unroll
+                for (uint32_t e = 0; e < TPV; ++e) {
+                    const float d = __fmul_rn(__fsub_rn(top, x[e]), c32);
+                    if (d >= 0.f && d < kFar) atomicAdd(&head_cnt[static_cast<uint32_t>(d)], 1u);
+                }
+            }
+            total = found();
+        }
+        const uint32_t b_star = S.s_w[0];
+        if (b_star == 0xffffffffu) list_all = true;  // (fewer than r_star tokens in the sample: everything is listed)
+        else thr = __fsub_rn(top, __fdiv_rn(static_cast<float>(b_star + 1u), c32));
+    }
+    if (list_all) thr = -INFINITY;
+    if (t == 0) {
+        S.s_w[1] = 0u;  // tokens listed
+        S.s_w[2] = 0u;  // the touched tokens did not fit
+        S.s_w[3] = 0u;  // how many they are
+    }
+    __syncthreads();  // (the counts and the bin have been read: the list takes the counts' place)
+    WSS_MARK(2);  // threshold known
+    load(qb, cb);
+    const double k2_d = static_cast<double>(inv_t) * 1.44269504088896340736;
+    const float k2 = static_cast<float>(k2_d), k2lo = static_cast<float>(k2_d - static_cast<double>(k2));
+    float m = -INFINITY, s0 = 0.f, s1 = 0.f;  // the largest token listed; two sums, of the tokens of even and of odd places (a thread has V / 512)
+    auto term = [&](float x) {
+        const float a = fmaxf(__fsub_rn(x, ref), -1e30f);
+        return __builtin_amdgcn_exp2f(fmaf(a, k2lo, a * k2));  // (v_exp_f32: arguments below -126 give 0, which is what they are worth)
+    };
+    auto push = [&](float x, uint32_t id, bool yes, bool early = false) {  // (one LDS atomic a listed token: they are few)
+        if (yes) {
+            m = fmaxf(m, x);
+            const uint32_t slot = atomicAdd(&S.s_w[1], 1u);
+            if (slot < (early ? early_slots : kShortCap)) list[slot] = key64(x, id);
+            else if (early) S.s_w[2] = 1u;
+            if (early) atomicAdd(&S.s_w[3], 1u);
+        }
+    };
+
+    // ---- the touched tokens: their adjusted logits (bias entries in list order, then repetition, then frequency / presence, as
+    // ws_sample.h applies them), into the sum and - above the threshold - the list. A token is taken by the entry that finds its word there
+    // and clears it: a bias entry where one names it, else one of its history.
+    if (n_all) {
+        auto take_touched = [&](auto n, auto&& id_of, uint32_t j0) __attribute__((always_inline)) {
+            constexpr uint32_t N = decltype(n)::value;
+            uint32_t word[N];
+            float raw[N];
+#pragma unroll
+            for (uint32_t k = 0; k < N; ++k) {
+                word[k] = 0u;
+                if (j0 + k * WS_BLOCK >= n_all) continue;  // uniform
+                const uint32_t r = rank(id_of(k)), sh = (r & 1u) * 16u;
+                if (r == 0xffffffffu) continue;
+                if (j0 + k * WS_BLOCK + t < nh && ((cnt[r >> 1] >> sh) & kBias)) continue;
+                word[k] = (atomicAnd(&cnt[r >> 1], ~(0xffffu << sh)) >> sh) & 0xffffu;
+            }
+#pragma unroll
+            for (uint32_t k = 0; k < N; ++k) {
+                raw[k] = -INFINITY;
+                if (word[k]) raw[k] = DT == 0 ? reinterpret_cast<const float*>(base)[id_of(k)] : bf16_to_f32(reinterpret_cast<const uint16_t*>(base)[id_of(k)]);
+            }
+#pragma unroll
+            for (uint32_t k = 0; k < N; ++k) {
+                if (j0 + k * WS_BLOCK >= n_all) continue;  // uniform
+                float x = -INFINITY;
+                if (word[k]) {
+                    const uint32_t c = word[k] & (kBias - 1u);
+                    x = fmaxf(raw[k], -INFINITY);
+                    if (word[k] & kBiases) {
+                        for (uint32_t j = 0; j < nb; ++j)
+                            if (static_cast<uint32_t>(bias_ids[j]) == id_of(k)) x = __fadd_rn(x, bias_vals[j]);
+                    } else if (word[k] & kBias) {
+                        x = __fadd_rn(x, bias_vals[j0 + k * WS_BLOCK + t - nh]);
+                    }
+                    if (c) {
+                        x = x > 0.f ? __fdiv_rn(x, P.rep) : __fmul_rn(x, P.rep);
+                        x = __fsub_rn(x, __fadd_rn(__fmul_rn(P.freq, static_cast<float>(c)), P.pres));
+                    }
+                    x = fmaxf(x, -INFINITY);
+                    s0 += term(x);
+                }
+                push(x, id_of(k), word[k] && x > thr, true);
+            }
+        };
+        constexpr uint32_t kThird = kIds / 3u;
+#pragma unroll
+        for (uint32_t h = 0; h < 3u; ++h)
+            if (h * kThird * WS_BLOCK < n_all) take_touched(std::integral_constant<uint32_t, kThird>{}, [&](uint32_t k) { return ids[h * kThird + k]; }, h * kThird * WS_BLOCK);
+        for (uint32_t j0 = kIds * WS_BLOCK; j0 < n_all; j0 += kMore * WS_BLOCK) {
+            uint32_t id[kMore];
+#pragma unroll
+            for (uint32_t k = 0; k < kMore; ++k) id[k] = entry(j0 + k * WS_BLOCK + t);
+            take_touched(std::integral_constant<uint32_t, kMore>{}, [&](uint32_t k) { return id[k]; }, j0);
+        }
+        __syncthreads();  // (the tables are done with: the list may take their place)
+    }
+    // from here on the bitmap says which tokens do not count
+    if (MASKED) {  // (the mask is read again: its words have no registers to stay in)
+        for (uint32_t w = t; w < nW; w += WS_BLOCK) invalid[w] = ~allow[w] | (n_all ? invalid[w] : 0u);
+        __syncthreads();
+    }
+    q_part = vector_at(n_full * WS_BLOCK + t);
+    // ---- the sweep: sum of exp, tokens above the threshold to the list
+    const bool mapped = MASKED || n_all != 0u;  // uniform
+    const float thr_a = __fsub_rn(thr, ref);  // (rounding is monotonous: x > thr makes x - ref, rounded, no smaller than this)
+    auto take = [&](const uint4& q, uint32_t word, uint32_t shift, uint32_t i0) __attribute__((always_inline)) {
+        const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+        float x[TPV], highest = -1e30f;
+        word >>= shift;
+#pragma unroll
+        for (uint32_t e = 0; e < TPV; ++e) {
+            uint32_t bits = DT == 0 ? w[e] : ((e & 1u) ? (w[e >> 1] & 0xffff0000u) : (w[e >> 1] << 16));
+            if (mapped) bits |= static_cast<uint32_t>(static_cast<int32_t>(word << (31u - e)) >> 31);  // -> NaN
+            x[e] = __uint_as_float(bits);
+            const float a = fmaxf(__fsub_rn(x[e], ref), -1e30f);  // (NaN as well: 0 in the sum; and never above `thr` below)
+            highest = fmaxf(highest, a);
+            (e & 1u ? s1 : s0) += __builtin_amdgcn_exp2f(fmaf(a, k2lo, a * k2));
+        }
+        if (__ballot(highest >= thr_a)) {  // uniform: a vector that may have a token for the list (a few per thousand)
+#pragma unroll
+            for (uint32_t e = 0; e < TPV; ++e) push(x[e], i0 + e, x[e] > thr);
+        }
+    };
+    auto take_at = [&](const uint4& q, uint32_t j) __attribute__((always_inline)) { take(q, mapped ? invalid[(j * TPV) >> 5] : 0u, (j * TPV) & 31u, j * TPV); };
+#pragma unroll
+    for (uint32_t k = 0; k < kTwinHead; ++k) {
+        const uint32_t j = k * spread * WS_BLOCK + t;
+        if (j < nv) take_at(hq[k], j);
+    }
+    const uint32_t my_word = (t * TPV) >> 5, my_shift = (t * TPV) & 31u;
+    auto eat = [&](const uint4 (&q)[KB], const uint32_t (&c)[KB]) __attribute__((always_inline)) {
+#pragma unroll
+        for (uint32_t k = 0; k < KB; ++k)
+            if (c[k] < n_full) take(q[k], mapped ? invalid[c[k] * (WS_BLOCK * TPV / 32u) + my_word] : 0u, my_shift, (c[k] * WS_BLOCK + t) * TPV);  // uniform
+    };
+    for (uint32_t i = kTwinHead; i < n_full; i += 2u * KB) {
+        eat(qa, ca);
+        load(qa, ca);
+        eat(qb, cb);
+        load(qb, cb);
+    }
+    if (!whole && n_full * WS_BLOCK + t < nv) take_at(q_part, n_full * WS_BLOCK + t);
+    if (n_odd) {  // uniform: the tokens behind the last whole vector
+        float x = -INFINITY;
+        const uint32_t id = nv * TPV + t;
+        if (t < n_odd && !(mapped && ((invalid[id >> 5] >> (id & 31u)) & 1u)))
+            x = fmaxf(DT == 0 ? reinterpret_cast<const float*>(base)[id] : bf16_to_f32(reinterpret_cast<const uint16_t*>(base)[id]), -INFINITY);
+        if (t < n_odd) s0 += term(x);
+        push(x, id, t < n_odd && x > thr);
+    }
+    WSS_MARK(4);  // sweep done
+#ifdef WS_SHORT_TIMERS
+    if (lane == 0u) atomicMax(reinterpret_cast<int*>(&S.marks[13]), __float_as_int(static_cast<float>(clock64() - wss_t0)));  // the slowest wave's
+#endif
+    double z;  // the sum against `ref`
+    {          // the block's maximum and sum with one barrier between them
+        const float wm_ = wave_max(m);
+        const double ws_ = wave_sum(static_cast<double>(s0) + static_cast<double>(s1));
+        __syncthreads();
+        if (lane == 0u) {
+            S.red_f[wv] = wm_;
+            S.red_d[wv] = ws_;
+        }
+        __syncthreads();
+        m = S.red_f[0];
+        z = S.red_d[0];
+#pragma unroll
+        for (uint32_t w = 1; w < WS_WAVES; ++w) {
+            m = fmaxf(m, S.red_f[w]);
+            z += S.red_d[w];
+        }
+    }
+    WSS_MARK(5);
+    uint32_t n_list = S.s_w[1];
+    if (by_p && n_list > kShortCap) {
+        // A min-p row whose sample's maximum lies well below its own: the floor is known now, and the row is read once more, for the list alone.
+        // (All of it, not what lies above the list's lowest: a row's sum has been taken. Of 65 rows of 50257 3 came this way.)
+        thr = fmaxf(thr, __fadd_rn(m, __fdiv_rn(static_cast<float>(log(min_p)) - 0.02f, inv_t)));
+        __syncthreads();
+        if (t == 0) S.s_w[1] = S.s_w[3];
+        __syncthreads();
+        auto list_from = [&](uint32_t id, uint32_t bits, bool there) {
+            const float x = fmaxf(__uint_as_float(bits), -INFINITY);
+            push(x, id, there && x > thr && !(mapped && ((invalid[id >> 5] >> (id & 31u)) & 1u)));
+        };
+        for (uint32_t j0 = t; j0 < nv; j0 += 4u * WS_BLOCK) {
+            uint4 q[4];
+#pragma unroll
+            for (uint32_t k = 0; k < 4u; ++k) q[k] = vector_at(j0 + k * WS_BLOCK);
+#pragma unroll
+            for (uint32_t k = 0; k < 4u; ++k) {
+                const uint32_t w[4] = {q[k].x, q[k].y, q[k].z, q[k].w}, j = j0 + k * WS_BLOCK;
+#pragma unroll
+                for (uint32_t e = 0; e < TPV; ++e)
+                    list_from(j * TPV + e, DT == 0 ? w[e] : ((e & 1u) ? (w[e >> 1] & 0xffff0000u) : (w[e >> 1] << 16)), j < nv);
+            }
+        }
+        if (t < n_odd)
+            list_from(nv * TPV + t, DT == 0 ? reinterpret_cast<const uint32_t*>(base)[nv * TPV + t] : static_cast<uint32_t>(reinterpret_cast<const uint16_t*>(base)[nv * TPV + t]) << 16, true);
+        __syncthreads();
+        n_list = S.s_w[1];
+    }
+    const uint32_t n_cand = by_k ? top_k : n_list;  // candidates the rules look at
+    if (S.s_w[2] != 0u || n_list > kShortCap || !(m > -INFINITY) || !(__fsub_rn(m, ref) * inv_t < 80.f) || n_list < n_cand || n_cand == 0u) return false;
+    // Tokens above `ref` can be most of the sum, and the larger the exponent, the less of a fraction 32 bits leave it (1.2e-6 of
+    // the normaliser where the maximum lies 60 units above the sample's; 2e-7 up to the four units below which nothing is done):
+    // they are all on the list, and their terms are taken out and put back in 64 bits.
+    if (__fsub_rn(m, ref) * inv_t > 4.f) {  // uniform
+        double more = 0.0;
+        for (uint32_t k = t; k < n_list; k += WS_BLOCK) {
+            const float x = unkey32(static_cast<uint32_t>(list[k] >> 32));
+            if (x > ref) more += exp((static_cast<double>(x) - static_cast<double>(ref)) * static_cast<double>(inv_t)) - static_cast<double>(term(x));
+        }
+        z += block_sum(more, S.red_d);
+    }
+    short_sort(list, n_list, m, S);
+    WSS_MARK(6);  // sorted
+    // the k-th largest has to lie above the threshold (below it, the sweep has left out tokens that rank before it); a min-p row's
+    // threshold lies below its floor by construction
+    const float x_k = unkey32(static_cast<uint32_t>(list[n_cand - 1u] >> 32));
+    if ((by_k && !(x_k > thr)) || !(x_k > -INFINITY)) return false;
+    ShortRow R;
+    R.top_p = top_p;
+    R.min_p = min_p;
+    R.u = batch_uniform(A.rng, P.seed, row, P.step, 0);
+    R.z = z * exp((static_cast<double>(ref) - static_cast<double>(m)) * static_cast<double>(inv_t));
+    R.inv_t = inv_t;
+    R.m = m;
+    R.n_cand = n_cand;
+    R.by_k = by_k;
+    short_rules(list, row, R, S);
+#ifdef WS_SHORT_TIMERS
+    WSS_MARK(8);
+    __syncthreads();
+    if (t < 16 && A.kept_logits) A.kept_logits[static_cast<size_t>(row) * A.kept_cap + 100u + t] = t == 15 ? static_cast<float>(n_list) : S.marks[t];
+#endif
+    return true;
+}
+
+// (two workgroups a compute unit are four waves a SIMD: 128 registers)
+template <int DT, bool MASKED>
+__global__ void __launch_bounds__(WS_BLOCK) __attribute__((amdgpu_waves_per_eu(4, 4))) twin_batch_kernel(BatchArgs A) {
+    __shared__ ShortShared shared;
+    if (!twin_row<DT, MASKED>(A, blockIdx.x, shared) && threadIdx.x == 0) A.flags[blockIdx.x] = kTwinRest;
+}
+
+}  // namespace ws
