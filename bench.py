@@ -34,11 +34,11 @@ KEPT_CAP = 0  # entries a row of the kept-set dump (--kept-cap), 0: no dump
 # of the kernel sources the counters were taken with), otherwise null. File names are relative to profiles/.
 TRAFFIC = {
     # (workload, mode): (bytes per launch, profiles/ file, kernel_digest() at the time)
-    ("tile", "auto"): (204944704, "lean_batch_kernel_tile_256x151936_f32.txt", "18280a84b5c2ef7e"),
-    ("cfg1", "auto"): (1033834, "few_batch_kernel_cfg1_1x151936_f32.txt", "18280a84b5c2ef7e"),
-    ("cfg2", "auto"): (55788602, "few_batch_kernel_cfg2_64x151936_f32.txt", "18280a84b5c2ef7e"),
-    ("cfg3", "auto"): (114211331, "lean_batch_kernel_cfg3_256x151936_bf16.txt", "18280a84b5c2ef7e"),
-    ("cfg5", "auto"): (1301521721, "short_batch_kernel_cfg5_1024x262144_f32.txt", "18280a84b5c2ef7e"),
+    ("tile", "auto"): (204919728, "lean_batch_kernel_tile_256x151936_f32.txt", "681fbc359644f608"),
+    ("cfg1", "auto"): (1044249, "few_batch_kernel_cfg1_1x151936_f32.txt", "681fbc359644f608"),
+    ("cfg2", "auto"): (55820626, "few_batch_kernel_cfg2_64x151936_f32.txt", "681fbc359644f608"),
+    ("cfg3", "auto"): (120634733, "code_batch_kernel_cfg3_256x151936_bf16.txt", "681fbc359644f608"),
+    ("cfg5", "auto"): (1306786906, "twin_batch_kernel_cfg5_1024x262144_f32.txt", "681fbc359644f608"),
 }
 
 
@@ -58,10 +58,10 @@ def checker():
 
 
 def kernel_digest():
-    """sha256[:16] over the sources of the sampler kernels (ws_common.h, ws_sample.h, ws_lean.h, ws_code.h, ws_short.h, ws_few.h, in this order)."""
+    """sha256[:16] over the sources of the sampler kernels (ws_common.h, ws_sample.h, ws_lean.h, ws_code.h, ws_short.h, ws_twin.h, ws_few.h, in this order)."""
     import hashlib
     h = hashlib.sha256()
-    for name in ("ws_common.h", "ws_sample.h", "ws_lean.h", "ws_code.h", "ws_short.h", "ws_few.h"):
+    for name in ("ws_common.h", "ws_sample.h", "ws_lean.h", "ws_code.h", "ws_short.h", "ws_twin.h", "ws_few.h"):
         with open(os.path.join(ROOT, "whirl-llm_amd", "csrc", name), "rb") as f:
             h.update(f.read())
     return h.hexdigest()[:16]
@@ -234,13 +234,17 @@ def cpu_model():
 
 def kernel_name(smp, routes):
     """The kernel that took the launch's rows: the short-list kinds by the workspace they ask for (65536 bytes a row: the kernel whose
-    workgroups hold their share of a row in registers)."""
+    workgroups hold their share of a row in registers) and by whether there are more rows than compute units."""
     from __graft_entry__ import load_package
     m = load_package()
     if routes["one_sweep_no_top_k"]:
         return "ws::code_batch_kernel" if smp.desc.dtype == m.DTYPE_BF16 else "ws::lean_batch_kernel"
     if routes["short_list_top_k"]:
-        return "ws::few_batch_kernel" if m.lib().ws_sample_batch_workspace(m.C.byref(smp.desc)) == 65536 * smp.desc.rows else "ws::short_batch_kernel"
+        if m.lib().ws_sample_batch_workspace(m.C.byref(smp.desc)) == 65536 * smp.desc.rows:
+            return "ws::few_batch_kernel"
+        import torch
+        many = smp.desc.rows > torch.cuda.get_device_properties(0).multi_processor_count
+        return "ws::twin_batch_kernel" if many else "ws::short_batch_kernel"
     return "ws::sample_batch_kernel"
 
 

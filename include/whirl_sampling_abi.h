@@ -201,8 +201,8 @@ enum {
                                             head of the row, or a masked-out outlier): the row was read again */
     WS_FLAG_ROUTE_SPLIT_ALONE = 1u << 11, /* a split row whose parts did not meet within split_spins looks: done by
                                             one workgroup. A caller that sees this often sets max_split = 1 */
-    WS_FLAG_ROUTE_LEAN = 1u << 12,       /* done by the one-sweep kernel for batches without a top-k (information only) */
-    WS_FLAG_ROUTE_SHORT = 1u << 13       /* done by the short-list kernel for batches with a bounded top-k or a min-p (information only) */
+    WS_FLAG_ROUTE_LEAN = 1u << 12,       /* done by the one-sweep kernel for batches without a top-k, or of bf16 rows by the kernel that counts them by value (information only) */
+    WS_FLAG_ROUTE_SHORT = 1u << 13       /* done by a short-list kernel for batches with a bounded top-k or a min-p, or so of bf16 rows by the kernel that counts them by value (information only) */
 };
 #define WS_FLAG_ROUTE_MASK 0x3f00u
 
@@ -230,8 +230,10 @@ typedef struct ws_batch {
     uint64_t row_stride; /* elements between rows (>= vocab) */
 
     const float* inv_t;     /* 1 / temperature, > 0 (Sampler::inv_t) */
-    const uint32_t* top_k;  /* 0 = off (NULL: off - and the caller's word that no row has one: fp32 and bf16 batches
-                               without optional outputs then take the one-sweep kernel written for such rows) */
+    const uint32_t* top_k;  /* 0 = off (NULL: off - and the caller's word that no row has one: fp32 batches
+                               without optional outputs then take the one-sweep kernel written for such rows. bf16
+                               batches without them take the kernel that counts a row's tokens by their value, which
+                               asks for no workspace, whether this is given or not) */
     const double* top_p;    /* 1 = off (NULL: off) */
     const double* min_p;    /* 0 = off (NULL: off) */
     const uint64_t* seed;   /* Sampler::seed */
@@ -318,7 +320,7 @@ typedef struct ws_batch {
                                    tokens that can be among a row's top_k largest instead of a histogram of all of them
                                    (fp32 and bf16, rows of any alignment, any vocabulary whose bitmap fits the LDS, kept-set
                                    dump, `query_prob` and `entropy` included; not with `race`). A row that breaks the word is still
-                                   answered correctly, by the three-pass code inside the launch (WS_FLAG_ROUTE_HANDED_BACK) */
+                                   answered correctly, by the three-pass code inside the call (WS_FLAG_ROUTE_HANDED_BACK) */
     double min_p_min;           /* 0: nothing is known about the rows without a top_k. Otherwise the caller's word that
                                    every row whose top_k is 0 has a min_p of at least this (a min-p floor bounds the kept
                                    set as a top-k does: what passes lies within -ln(min_p) / inv_t of the row's maximum).

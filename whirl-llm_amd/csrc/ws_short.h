@@ -12,7 +12,7 @@
 //   * the list is sorted, and the reference's rules run on the sorted candidates: top-k, top-p on the mass of those, min-p
 //     against the largest, the draw by inverse CDF with the row's uniform.
 // A row for which a check fails, whose list runs over, or that has neither a top-k nor a min-p after all, is handed to the
-// three-pass code of ws_sample.h inside the same launch (WS_FLAG_ROUTE_HANDED_BACK).
+// three-pass code of ws_sample.h inside the same call (WS_FLAG_ROUTE_HANDED_BACK).
 // More rows than compute units are ws_twin.h's. Few rows are shared between workgroups by the kernel of ws_few.h, which ends with the same sort and rules; those it has no
 // registers or lists for are shared here: each part lists its slice against its own threshold and leaves list, maximum and sum in
 // the row's workspace, and the part that arrives last - a ticket, nobody waits - takes them all and finishes the row. The
@@ -436,7 +436,7 @@ __device__ __forceinline__ bool short_row(const BatchArgs& A, const uint32_t row
 
     // The row in vectors: the whole ones, and the few tokens behind them (none, of most vocabularies) one by one after the sweep.
     // Masked fp32 rows: all of them, the last read where it ends with the row and moved down. (Either way for the registers'
-    // sake: moved vectors spill them in the bf16 kernels - unmasked, 1000 rows of 24896: 118 us against 72; masked, 300 rows of
+    // sake, measured when batches of any size came here: moved vectors spill them in the bf16 kernels - unmasked, 1000 rows of 24896: 118 us against 72; masked, 300 rows of
     // 151936: 102 against 89, 1024 of 262144: 445 against 411 -, clamped whole ones in the masked fp32 kernel - 300 rows of
     // 151936: 99 us against 81, 1024 of 262144: 430 against 390.)
     constexpr bool MOVED = MASKED && DT == 0;
