@@ -507,14 +507,10 @@ __device__ __forceinline__ bool code_row(const BatchArgs& A, const uint32_t row,
             float x = fmaxf(bf16_to_f32(raw[r]), -INFINITY);
             const uint32_t was = code_bin(x);  // (out of the raw logits' counts)
             if (was < kCodeTail) atomicSub(&count[was], 1u);
-            if (n_bias) {
-                uint32_t j = pos[r];
-                x = __fadd_rn(x, bias_vals[j]);
-                if (n_bias > 1u) {
-                    const int32_t id = static_cast<int32_t>(tid[r]);
-                    for (++j; j < nb; ++j)
-                        if (bias_ids[j] == id) x = __fadd_rn(x, bias_vals[j]);
-                }
+            if (__ballot(n_bias != 0u)) {  // uniform
+                const uint32_t j = n_bias ? pos[r] : 0u;
+                if (n_bias) x = __fadd_rn(x, bias_vals[j]);
+                if (__ballot(n_bias > 1u)) x = add_other_bias(n_bias > 1u, tid[r], j, x, bias_ids, bias_vals, nb);
             }
             if (c) {
                 x = x > 0.f ? __fdiv_rn(x, P.rep) : __fmul_rn(x, P.rep);

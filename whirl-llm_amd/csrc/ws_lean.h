@@ -714,12 +714,10 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const uint32_t row,
                     }
                     const uint32_t cw = old[k], c = cw & 0xfffffu, n_bias = (cw >> 20) & 0x7ffu;
                     float x = raw;
-                    if (n_bias) {
-                        uint32_t j = first[rk[k]];
-                        x = __fadd_rn(x, bias_vals2[j]);
-                        if (n_bias > 1u)
-                            for (++j; j < nb; ++j)
-                                if (static_cast<uint32_t>(bias_ids2[j]) == i) x = __fadd_rn(x, bias_vals2[j]);
+                    if (__ballot(n_bias != 0u)) {  // uniform
+                        const uint32_t j = n_bias ? first[rk[k]] : 0u;
+                        if (n_bias) x = __fadd_rn(x, bias_vals2[j]);
+                        x = add_other_bias(n_bias > 1u, i, j, x, bias_ids2, bias_vals2, nb);
                     }
                     if (c) {
                         x = x > 0.f ? __fdiv_rn(x, rep) : __fmul_rn(x, rep);

@@ -2064,14 +2064,12 @@ __device__ __forceinline__ void sample_row(const BatchArgs& A, const uint32_t bl
                 }
                 return x;
             };
-            // the bias values of an id, added one by one in listed order, starting at its first entry j
+            // the bias values of an id, added one by one in listed order: n of them (or none), starting at its first entry j
             auto add_bias = [&](float x, uint32_t j, uint32_t n) {
-                const int32_t id = bias_ids[j];
-                x = __fadd_rn(x, bias_vals[j]);
-                if (n > 1u)
-                    for (++j; j < nb; ++j)
-                        if (bias_ids[j] == id) x = __fadd_rn(x, bias_vals[j]);
-                return x;
+                if (!__ballot(n != 0u)) return x;  // uniform
+                const uint32_t id = n ? static_cast<uint32_t>(bias_ids[j]) : 0u;
+                if (n) x = __fadd_rn(x, bias_vals[j]);
+                return add_other_bias(n > 1u, id, j, x, bias_ids, bias_vals, nb);
             };
             if (saved_cnt) {
                 for (uint32_t r0 = 0; r0 < n_touched; r0 += 4u * WS_BLOCK) {  // four ranks a thread: their reads travel together
@@ -2089,7 +2087,7 @@ __device__ __forceinline__ void sample_row(const BatchArgs& A, const uint32_t bl
                         float x = pv[r];
                         const uint32_t n = cw[k] >> 20;
                         if (n == 1u) x = __fadd_rn(x, __uint_as_float(bw[k]));  // the one bias value itself
-                        else if (n) x = add_bias(x, bw[k], n);                   // its first entry
+                        x = add_bias(x, bw[k], n > 1u ? n : 0u);                 // its first entry
                         x = penalise(x, cw[k] & 0xfffffu);
                         pv[r] = x;
                         ma = fmaxf(ma, x);
@@ -2100,7 +2098,7 @@ __device__ __forceinline__ void sample_row(const BatchArgs& A, const uint32_t bl
                     const uint32_t cw = cnt[r], c = cw & 0xfffffu;
                     const float raw = pv[r];
                     float x = raw;
-                    if (cw >> 20) x = add_bias(x, first[r], cw >> 20);
+                    x = add_bias(x, first[r], cw >> 20);
                     x = penalise(x, c);
                     pv[r] = x;
                     cnt[r] = __float_as_uint(raw);
@@ -2217,11 +2215,9 @@ __device__ __forceinline__ void sample_row(const BatchArgs& A, const uint32_t bl
                     float x = raw;
                     if (n_bias) {
                         // the bias values of this id, added one by one in listed order, starting at its first entry
-                        uint32_t j = first[rk[k]];
+                        const uint32_t j = first[rk[k]];
                         x = __fadd_rn(x, bias_vals[j]);
-                        if (n_bias > 1u)
-                            for (++j; j < nb; ++j)
-                                if (static_cast<uint32_t>(bias_ids[j]) == i) x = __fadd_rn(x, bias_vals[j]);
+                        if (__ballot(n_bias > 1u)) x = add_other_bias(n_bias > 1u, i, j, x, bias_ids, bias_vals, nb);
                     }
                     if (c) {
                         x = x > 0.f ? __fdiv_rn(x, rep) : __fmul_rn(x, rep);

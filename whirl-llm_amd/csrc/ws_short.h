@@ -182,7 +182,9 @@ __device__ __forceinline__ void short_rules(uint64_t* list, const uint32_t row, 
         if (Ap->entropy) Ap->entropy[row] = log(Zk_) - e_ln_e / Zk_;
         if (Ap->query_prob) Ap->query_prob[row] = e_query / Zk_;
     };
-    // more candidates than threads (a wide top-k, a wide min-p floor): thread t has those at places KC t .. KC t + KC - 1 of the order; the same rules
+    // more candidates than threads (a wide top-k, a wide min-p floor): thread t has those at places KC t .. KC t + KC - 1 of the order; the same rules.
+    // (KC as small as will do: with eight a thread for all of them most waves had none. 512 threads: 8 rows of 32000, top-k 600, 18.5 us -> 16.3; 64 rows with
+    // min-p floors that let 600 to 2000 through 33.7 -> 32.2)
     auto several = [&](auto kc) __attribute__((always_inline)) {
         constexpr uint32_t KC = decltype(kc)::value;
         uint64_t wkey[KC];
@@ -279,11 +281,7 @@ __device__ __forceinline__ void short_rules(uint64_t* list, const uint32_t row, 
             if (t == 0) write_more(se, sq, Zk);
         }
     };
-    if (n_cand > 2u * WS_BLOCK) {
-        several(std::integral_constant<uint32_t, kShortCap / WS_BLOCK>{});
-    } else if (n_cand > WS_BLOCK) {
-        several(std::integral_constant<uint32_t, 2u>{});
-    } else if (n_cand <= 64u) {
+    if (n_cand <= 64u) {
         // the usual case, a top-k of a few dozen: one wave, a candidate a lane, no barrier and no atomic
         if (wv == 0u) {
             const double e = has ? exp(static_cast<double>(__fsub_rn(x, m)) * static_cast<double>(inv_t)) : 0.0;
@@ -327,7 +325,7 @@ __device__ __forceinline__ void short_rules(uint64_t* list, const uint32_t row, 
             }
             if (lane == 0u) S.s_w[7] = n3;
         }
-    } else {
+    } else if (n_cand <= WS_BLOCK) {
         double e = 0.0;
         if (wv * 64u < n_cand) e = has ? exp(static_cast<double>(__fsub_rn(x, m)) * static_cast<double>(inv_t)) : 0.0;  // (per wave: the exponential is a hundred instructions)
         double Zk1;
@@ -384,6 +382,12 @@ __device__ __forceinline__ void short_rules(uint64_t* list, const uint32_t row, 
             const double se = block_sum(kept && e > 0.0 ? e * log_mass(x) : 0.0, S.red_d), sq = block_sum(kept && id == query ? e : 0.0, S.red_d);
             if (t == 0) write_more(se, sq, Zk);
         }
+    } else if (n_cand <= 2u * WS_BLOCK) {
+        several(std::integral_constant<uint32_t, 2u>{});
+    } else if (WS_BLOCK < 1024 && n_cand <= 4u * WS_BLOCK) {
+        several(std::integral_constant<uint32_t, 4u>{});
+    } else {
+        several(std::integral_constant<uint32_t, kShortCap / WS_BLOCK>{});
     }
     // ---- the kept set in ascending id order (the first kept_cap of it): the same sort on (inverted id, logit) pairs
     if (Ap->kept_ids) {
@@ -817,12 +821,10 @@ __device__ __forceinline__ bool short_row(const BatchArgs& A, const uint32_t row
                 if (have) {
                     const uint32_t c = old[k] & 0xfffffu, n_bias = (old[k] >> 20) & 0x7ffu;
                     x = fmaxf(raw[k], -INFINITY);
-                    if (n_bias) {
-                        uint32_t j = first[r[k]];
-                        x = __fadd_rn(x, bias_vals[j]);
-                        if (n_bias > 1u)
-                            for (++j; j < nb; ++j)
-                                if (static_cast<uint32_t>(bias_ids[j]) == id[k]) x = __fadd_rn(x, bias_vals[j]);
+                    if (__ballot(n_bias != 0u)) {  // uniform
+                        const uint32_t j = n_bias ? first[r[k]] : 0u;
+                        if (n_bias) x = __fadd_rn(x, bias_vals[j]);
+                        x = add_other_bias(n_bias > 1u, id[k], j, x, bias_ids, bias_vals, nb);
                     }
                     if (c) {
                         x = x > 0.f ? __fdiv_rn(x, P.rep) : __fmul_rn(x, P.rep);

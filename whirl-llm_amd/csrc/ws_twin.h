@@ -384,12 +384,9 @@ __device__ __forceinline__ bool twin_row(const BatchArgs& A, const uint32_t row,
                 if (word[k]) {
                     const uint32_t c = word[k] & (kBias - 1u);
                     x = fmaxf(raw[k], -INFINITY);
-                    if (word[k] & kBiases) {
-                        for (uint32_t j = 0; j < nb; ++j)
-                            if (static_cast<uint32_t>(bias_ids[j]) == id_of(k)) x = __fadd_rn(x, bias_vals[j]);
-                    } else if (word[k] & kBias) {
-                        x = __fadd_rn(x, bias_vals[j0 + k * WS_BLOCK + t - nh]);
-                    }
+                    const bool several = (word[k] & kBiases) != 0u;
+                    if ((word[k] & kBias) && !several) x = __fadd_rn(x, bias_vals[j0 + k * WS_BLOCK + t - nh]);
+                    if (__ballot(several)) x = add_other_bias(several, id_of(k), 0xffffffffu, x, bias_ids, bias_vals, nb);  // (from the first of them)
                     if (c) {
                         x = x > 0.f ? __fdiv_rn(x, P.rep) : __fmul_rn(x, P.rep);
                         x = __fsub_rn(x, __fadd_rn(__fmul_rn(P.freq, static_cast<float>(c)), P.pres));
