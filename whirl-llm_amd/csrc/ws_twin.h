@@ -4,8 +4,8 @@
 // What bounds it: memory while rows are swept, and nothing while they are not. 1024 threads with a unit to themselves took 177K clocks
 // for a row of 262144 tokens, a tenth of them allowed, with a history of 8192 and a top-k of 1000, 80K of them without a sweep: the tables, the
 // threshold, the sort, the rules. Here a unit's other row sweeps in the meantime, as far as the two are not at the same place (they start together);
-// a row of a small vocabulary is all such stretches, and two of them are at work instead of one. Microseconds, ws_short.h and this: 1024 rows as above 389 / 323,
-// the same without history 266 / 239; top-k 50, 1000-id histories: 512 of 151936 83.8 / 73.3, 300 of 151936 77.2 / 63.9, 1000 of 50257 108 / 72.9, 1000 of 8000
+// a row of a small vocabulary is all such stretches, and two of them are at work instead of one. Microseconds, ws_short.h and this: 1024 rows as above 389 / 323
+// (280 since ws_common.h's search of bias lists), without history 266 / 239; top-k 50, 1000-id histories: 512 of 151936 83.8 / 73.3, 300 of 151936 77.2 / 63.9, 1000 of 50257 108 / 72.9, 1000 of 8000
 // 55.9 / 38.1; min-p alone, 1000 of 151936 149 / 139. (1024 of 262144 with a top-k of 50: 195, 5.5 TB/s.)
 //
 // Against ws_short.h the touched tokens come before the sweep, not behind it: their tables are dead when it begins and can lie where the list
@@ -86,8 +86,8 @@ __device__ __forceinline__ bool twin_row(const BatchArgs& A, const uint32_t row,
     const int32_t* bias_ids = A.bias_ids + P.b0;
     const float* bias_vals = A.bias_vals + P.b0;
 
-    // Loads come back in order, and what is asked for behind the row's own vectors waits for them: the history and bias ids, one sequence, go first
-    // and stay in registers (9 rounds: 4608 of them), and all the tables are built from them while the vectors travel.
+    // The history and bias ids, one sequence, stay in registers (9 rounds: 4608 of them) until their tokens have been taken. They are asked for behind
+    // the sample, which does not have to know the parameters first.
     constexpr uint32_t kIds = 9u, kMore = 4u;
     uint32_t ids[kIds];
     auto entry = [&](uint32_t j) __attribute__((always_inline)) {  // (unconditional, as all these loads: one behind a branch makes the compiler wait for every load before it)
