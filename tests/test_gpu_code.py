@@ -200,3 +200,51 @@ def test_rows_without_a_filter(V, allowed, n_hist):
     c["top_k"][:], c["top_p"][:], c["min_p"][:] = 0, 1.0, 0.0
     smp = run(c, max_differ=1)
     assert ((smp.flags & 64) != 0).all()  # (WS_FLAG_OPEN)
+
+
+# A row's largest tokens by their octave: at the low and at the high end of a group of eight values, and between.
+PEAKS = [9.0, 9.4375, 10.02, 16.0, 16.875, 17.05, 20.45, 24.05, 33.3, 38.0, 70.2, 301.0]
+TEMPERATURES = [0.03, 0.05, 0.1, 0.3]
+
+
+def cold_case(T, kind, hints, V=50001):
+    """Rows whose largest tokens lie a few e-folds apart at temperature T. kind "bias" and "history": tokens at any float, by a bias or by
+    penalties, untouched ones at the next values below them; "plain": no touched token at all; "beside": a touched token far below, the others on the grid."""
+    n = len(PEAKS)
+    c = case(2 * n, V, n_hist=0 if kind == "plain" else 40, n_bias=0 if kind == "plain" else 12)
+    rng = np.random.default_rng(int(T * 1000) + len(kind))
+    x = gc.bf16_bits_to_f32(c["logits"]).copy()
+    c["inv_t"][:] = np.float32(1.0) / np.float32(T)
+    c["rep"][:], c["pres"][:], c["freq"][:] = 1.1, 0.3, 0.02
+    for r in range(2 * n):
+        peak, at = np.float32(PEAKS[r // 2]), rng.permutation(V)
+        step = np.float32(2.0 ** (np.floor(np.log2(peak)) - 7))
+        low = np.float32(np.floor(peak / step) * step)  # the largest value at or below the peak
+        if kind in ("plain", "beside"):
+            x[r, at[:6]] = low - step * np.array([0, 0, 1, 1, 2, 5], np.float32)
+        else:
+            x[r, at[20:26]] = low - step * np.array([1, 1, 2, 3, 4, 9], np.float32)
+        if kind == "plain":
+            continue
+        c["bias_ids"][r], c["bias_vals"][r] = at[:12] if kind == "bias" else at[30:42], rng.uniform(-3, 0, 12)
+        c["hist"][r, :8] = at[50:58] if kind == "bias" else at[:8]
+        c["hist"][r, 8:] = at[60:92]
+        if kind == "bias":
+            c["bias_vals"][r] = peak - T * np.array([0, 0.2, 0.5, 0.9, 1.3, 2.1, 3.0, 4.2, 6.0, 9.0, 14.0, 20.0]) - x[r, at[:12]]
+        elif kind == "history":  # (raw values whose penalised ones lie around the peak)
+            x[r, at[:8]] = np.float32((peak + 0.32) * 1.1) - step * np.arange(8, dtype=np.float32)
+    c["logits"] = gc.f32_to_bf16_bits(x)
+    filters = [(0, 0.9, 0.0), (40, 1.0, 0.0), (0, 0.95, 0.05), (40, 0.7, 0.0), (0, 1.0, 0.02), (3, 1.0, 0.0), (1000, 0.99, 0.0), (0, 1.0, 0.0)]
+    if hints:
+        filters = [f for f in filters if f[0] or f[2]]
+    for r in range(2 * n):
+        c["top_k"][r], c["top_p"][r], c["min_p"][r] = filters[(r * 5 + r // len(filters)) % len(filters)]
+    return c
+
+
+@pytest.mark.parametrize("hints", [False, True])
+@pytest.mark.parametrize("T", TEMPERATURES)
+@pytest.mark.parametrize("kind", ["bias", "history", "beside"])
+def test_cold_rows(kind, T, hints):
+    """Octaves are many e-folds wide at low temperatures, and so are the groups of eight values that touched masses are added up in."""
+    run(cold_case(T, kind, hints), hints=hints)

@@ -15,7 +15,8 @@
 //   * The touched tokens (history, bias list) are counted like the others and taken out again afterwards. Their ids are ranked by a
 //     bitmap and its prefix sums, in four steps between the row's rounds, so that the trips to memory for the ids and for their
 //     logits pass meanwhile. Their adjusted logits are 32-bit floats: they are listed by the group of eight bins they fall in - count,
-//     and mass in fixed point -, and those of the bin that a cut or the draw falls in are put in order there.
+//     and mass in fixed point against the group's top or the row's maximum -, and those of the bin that a cut or the draw falls in are put in
+//     order there.
 //   * A thread has eight bins for the prefix sums; one wave then looks for the cuts and the draw, without a barrier.
 //
 // What bounds it: eight waves' worth of LDS additions at random words, some eight clocks an instruction of 64 lanes - 10 us for 151936
@@ -481,25 +482,8 @@ __device__ __forceinline__ bool code_row(const BatchArgs& A, const uint32_t row,
     const bool by_bins = A.code_head != 0u;
     const float c64 = inv_t * 64.f;
     const float anchor0 = code_value(min(S.head_bin, kCodeTail)) + A.code_above / inv_t;
-    const float aq0 = anchor_product(anchor0, c64);
     auto inside = [&](float tc) { return static_cast<double>(0x40000000u - static_cast<uint32_t>(bin_word(tc))); };  // of a bin's mass at its upper end, in units of 2^-30
     const double kFix = static_cast<double>(1ull << kCodeFixBits), kUnfix = 1.0 / kFix;
-    // a touched token's mass against that of its group's top (code_group_top), in fixed point, and the other way round: what comes to it
-    auto group_by_bins = [&](uint32_t g) {  // (none of them above the anchor, or too far below it)
-        return by_bins && code_group_top(g) <= static_cast<double>(anchor0) && (anchor0 - code_value(g * 8u + 7u)) * c64 < 4000.f;
-    };
-    auto top_bin_of = [&](uint32_t g) { return static_cast<uint32_t>(fmaxf(bin_coord(aq0, c64, static_cast<float>(code_group_top(g))), 0.f)); };
-    auto fix_of = [&](float x, uint32_t g) {
-        double e;
-        if (group_by_bins(g)) {
-            const float tc = bin_coord(aq0, c64, x);
-            const uint32_t d = min(static_cast<uint32_t>(tc) - top_bin_of(g), 4031u);
-            e = S.s_exp[d >> 6] * S.s_exp[64u + (d & 63u)] * (inside(tc) * kFixInv);
-        } else {
-            e = code_exp((code_group_top(g) - static_cast<double>(x)) * static_cast<double>(inv_t));
-        }
-        return static_cast<unsigned long long>(e * kFix + 0.5);
-    };
     if (TOUCHED) {
         uint32_t best = 0u;
         for (uint32_t r = t; r < n_touched; r += WS_BLOCK) {
@@ -522,7 +506,6 @@ __device__ __forceinline__ bool code_row(const BatchArgs& A, const uint32_t row,
             if (bin < kCodeTail && bin >= 8u) {
                 const uint32_t g = bin >> 3;
                 best = max(best, key32(x));
-                atomicAdd(&g_mass[g], fix_of(x, g));
                 pos[r] = static_cast<uint16_t>(atomicAdd(&g_cnt[g], 1u));
             }
         }
@@ -562,19 +545,45 @@ __device__ __forceinline__ bool code_row(const BatchArgs& A, const uint32_t row,
     WSC_MARK(5);
     if (S.bad || S.top_bin < 8u || !(m > -INFINITY) || !(__fsub_rn(m, code_value(kCodeTail)) * inv_t >= 50.f)) return false;
     // (an anchor that lies below the maximum, or wastefully far above it, gives way to the maximum itself)
-    const float aq = m <= anchor0 && (anchor0 - m) * c64 <= 1024.f ? aq0 : anchor_product(m, c64);
-    const double lift = static_cast<double>(aq) * (1.0 / 64.0) - static_cast<double>(m) * static_cast<double>(inv_t);
-    auto exact_mass = [&](float x) { return code_exp(static_cast<double>(__fsub_rn(m, x)) * static_cast<double>(inv_t)); };
+    // (the row's 64-bit values are kept in scalar registers: beside the row's vectors there is no room for them)
+    const float aq = anchor_product(m <= anchor0 && (anchor0 - m) * c64 <= 1024.f ? anchor0 : m, c64);
+    const double m_d = lane_value(static_cast<double>(m), 0u), inv_t_d = lane_value(static_cast<double>(inv_t), 0u);
+    const double lift = lane_value(static_cast<double>(aq) * (1.0 / 64.0) - m_d * inv_t_d, 0u);
+    auto exact_mass = [&](float x) { return code_exp(static_cast<double>(__fsub_rn(m, x)) * inv_t_d); };
     auto mass_of = [&](float x) {
         if (!by_bins) return exact_mass(x);  // uniform
         const float tc = bin_coord(aq, c64, x);
         return code_exp(static_cast<double>(static_cast<uint32_t>(tc)) * (1.0 / 64.0) - lift) * (inside(tc) * kFixInv);
     };
-    auto unfix_of = [&](unsigned long long sum, uint32_t g) {
-        const double top = group_by_bins(g) ? (static_cast<double>(top_bin_of(g)) - static_cast<double>(aq0)) * (1.0 / 64.0) + static_cast<double>(m) * static_cast<double>(inv_t)
-                                   : (static_cast<double>(m) - code_group_top(g)) * static_cast<double>(inv_t);
-        return static_cast<double>(sum) * kUnfix * code_exp(top);
+    // A touched token's mass in fixed point, and the other way round: what comes to it. It is taken against that of `top_of`, the group's top, but
+    // no more than the maximum: an octave's eighth is 0.5 from 8 to 16 and 2 from 32 to 64, 10 to 40 e-folds at a temperature of 0.05, and against a
+    // top so far above it the largest token of the row would weigh nothing. (So each is off by 2^-45 of the normaliser at most.)
+    auto top_of = [&](uint32_t g) { return fmin(code_group_top(g), m_d); };
+    auto group_by_bins = [&](uint32_t g) { return by_bins && bin_coord(aq, c64, code_value(g * 8u + 7u)) < 4000.f; };  // (none of them in the tail)
+    auto top_bin_of = [&](uint32_t g) { return static_cast<uint32_t>(bin_coord(aq, c64, static_cast<float>(top_of(g)))); };
+    auto fix_of = [&](float x, uint32_t g) {
+        double e;
+        if (group_by_bins(g)) {
+            const float tc = bin_coord(aq, c64, x);
+            const uint32_t d = static_cast<uint32_t>(tc) - top_bin_of(g);
+            e = S.s_exp[d >> 6] * S.s_exp[64u + (d & 63u)] * (inside(tc) * kFixInv);
+        } else {
+            e = code_exp((top_of(g) - static_cast<double>(x)) * inv_t_d);
+        }
+        return static_cast<unsigned long long>(e * kFix + 0.5);
     };
+    auto unfix_of = [&](unsigned long long sum, uint32_t g) {
+        const double down = group_by_bins(g) ? static_cast<double>(top_bin_of(g)) * (1.0 / 64.0) - lift : (m_d - top_of(g)) * inv_t_d;
+        return static_cast<double>(sum) * kUnfix * code_exp(down);
+    };
+    if (TOUCHED && n_touched) {
+        for (uint32_t r = t; r < n_touched; r += WS_BLOCK) {
+            const float x = adj[r];
+            const uint32_t bin = code_bin(x);
+            if (bin < kCodeTail) atomicAdd(&g_mass[bin >> 3], fix_of(x, bin >> 3));
+        }
+        __syncthreads();
+    }
     double Z;
     uint32_t n_all;
     {
@@ -589,7 +598,7 @@ __device__ __forceinline__ bool code_row(const BatchArgs& A, const uint32_t row,
                 }
                 mass *= kFixInv * code_exp(-lift);
             } else {  // equal steps: eight masses from the first one's and the factor of a step
-                const double f = code_exp(static_cast<double>(code_group_step(t)) * static_cast<double>(inv_t));
+                const double f = code_exp(static_cast<double>(code_group_step(t)) * inv_t_d);
                 mass = static_cast<double>(c8[7]);
 #pragma unroll
                 for (int k = 6; k >= 0; --k) mass = fma(mass, f, static_cast<double>(c8[k]));
