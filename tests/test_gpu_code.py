@@ -204,7 +204,7 @@ def test_rows_without_a_filter(V, allowed, n_hist):
 
 # A row's largest tokens by their octave: at the low and at the high end of a group of eight values, and between.
 PEAKS = [9.0, 9.4375, 10.02, 16.0, 16.875, 17.05, 20.45, 24.05, 33.3, 38.0, 70.2, 301.0]
-TEMPERATURES = [0.03, 0.05, 0.1, 0.3]
+TEMPERATURES = [2e-4, 2.5e-4, 1e-3, 0.01, 0.02, 0.03, 0.05, 0.1, 0.3]
 
 
 def cold_case(T, kind, hints, V=50001):
@@ -244,7 +244,9 @@ def cold_case(T, kind, hints, V=50001):
 
 @pytest.mark.parametrize("hints", [False, True])
 @pytest.mark.parametrize("T", TEMPERATURES)
-@pytest.mark.parametrize("kind", ["bias", "history", "beside"])
+@pytest.mark.parametrize("kind", ["bias", "history", "beside", "plain"])
 def test_cold_rows(kind, T, hints):
-    """Octaves are many e-folds wide at low temperatures, and so are the groups of eight values that touched masses are added up in."""
-    run(cold_case(T, kind, hints), hints=hints)
+    """Octaves are many e-folds wide at low temperatures, and so are the groups of eight values that masses are added up in: hundreds of e-folds, more
+    than 64 bits have room for. Below a temperature of 1/4096 the rows are the three-pass code's."""
+    c = cold_case(T, kind, hints)
+    run(c, hints=hints, handed_back=c["rows"] if T < 1 / 4096 else 0)

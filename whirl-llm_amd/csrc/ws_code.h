@@ -41,6 +41,9 @@ constexpr uint32_t kCodeGroups = kCodeBins / 8u;  // eight bins each, one group 
 constexpr uint32_t kCodeSub = 512u;               // touched tokens in one bin, where a cut or the draw falls in it
 constexpr uint32_t kCodeFixBits = 44u;            // fixed point of the groups' touched masses (65535 of them at most)
 constexpr uint32_t kCodeHeldVecs = 20u;           // vectors a thread holds
+// Up to here the anchor of a row of logits below 512 lies at most 64 of its bins further above the maximum than it was put (anchor_product's 2^-21): 2900
+// of them, 45 e-folds, are left below the maximum. Colder rows lose some to the tail.
+constexpr float kCodeMaxInvT = 4096.f;
 
 typedef uint16_t CodePair __attribute__((ext_vector_type(2)));
 typedef int16_t CodePairS __attribute__((ext_vector_type(2)));
@@ -248,9 +251,10 @@ __device__ __forceinline__ bool code_row(const BatchArgs& A, const uint32_t row,
     const float inv_t = P.inv_t;
     const double top_p = P.top_p, min_p = P.min_p;
     const bool use_top_p = top_p < 1.0, use_min_p = min_p > 0.0;
-    // rows this code does not take: a top-p that keeps nothing, a min-p above 1, the race draw, parameters the three-pass code reports
+    // rows this code does not take: a top-p that keeps nothing, a min-p above 1, the race draw, parameters the three-pass code reports, temperatures
+    // below kCodeMaxInvT's
     const bool open = P.top_k == 0u && !use_top_p && !use_min_p;
-    if (!(top_p > 0.0) || !(min_p <= 1.0) || P.race || !(inv_t > 0.f) || !(inv_t < INFINITY) ||
+    if (!(top_p > 0.0) || !(min_p <= 1.0) || P.race || !(inv_t > 0.f) || !(inv_t <= kCodeMaxInvT) ||
         P.nh + P.nb > cap)
         return false;
     if (wv == WS_WAVES - 1u) {  // (the seed by way of a vector register: as scalar arithmetic every wave would work the generator's rounds out)
@@ -598,11 +602,15 @@ __device__ __forceinline__ bool code_row(const BatchArgs& A, const uint32_t row,
                 }
                 mass *= kFixInv * code_exp(-lift);
             } else {  // equal steps: eight masses from the first one's and the factor of a step
+                // (the first that holds a token: a group may reach above the maximum, where masses have no bound)
                 const double f = code_exp(static_cast<double>(code_group_step(t)) * inv_t_d);
+                uint32_t k0 = 7u;
                 mass = static_cast<double>(c8[7]);
 #pragma unroll
-                for (int k = 6; k >= 0; --k) mass = fma(mass, f, static_cast<double>(c8[k]));
-                mass *= exact_mass(code_value(t * 8u));
+                for (int k = 6; k >= 0; --k) k0 = c8[k] ? static_cast<uint32_t>(k) : k0;
+#pragma unroll
+                for (int k = 6; k >= 0; --k) mass = static_cast<uint32_t>(k) >= k0 ? fma(mass, f, static_cast<double>(c8[k])) : mass;
+                mass *= exact_mass(code_value(t * 8u + k0));
             }
         }
         if (TOUCHED && ext) mass += unfix_of(g_mass[t], t);
@@ -625,6 +633,7 @@ __device__ __forceinline__ bool code_row(const BatchArgs& A, const uint32_t row,
         const uint32_t wn = row_incl_scan(S.red_u[lane & (WS_WAVES - 1u)]), we = TOUCHED ? row_incl_scan(S.red_v[lane & (WS_WAVES - 1u)]) : 0u;
         Z = lane_value(wm, WS_WAVES - 1u);
         n_all = lane_value(wn, WS_WAVES - 1u);
+        if (!(Z > 0.5 && Z < INFINITY)) return false;  // uniform (the maximum's own mass is 1: it has not been counted as it should)
         if (wave_has) {  // uniform
             const double base_m = wv ? lane_value(wm, wv - 1u) : 0.0;
             const uint32_t base_n = wv ? lane_value(wn, wv - 1u) : 0u;
@@ -726,14 +735,14 @@ __device__ __forceinline__ bool code_row(const BatchArgs& A, const uint32_t row,
                 if (lane < 8u) e = S.bin_cnt[lane];
             }
             const double w = mass_of(code_value(b_));
-            double mass = static_cast<double>(c) * w;
+            double mass = c ? static_cast<double>(c) * w : 0.0;  // (an empty bin may lie above the maximum: no bound to its w)
             if (e) mass += unfix_of(S.bin_mass[lane], g);
             if (lane >= 8u) c = 0u, mass = 0.0;
             const uint32_t ci = wave_incl_scan(c + e) + cpre;
             const double mi = wave_incl_scan(mass) + pre;
             uint32_t k = k_of;
             if (mode != kByPassing) {
-                const bool here = c + e != 0u;
+                const bool here = c + e != 0u && (mode == kByRank || mass > 0.0);
                 const uint64_t any = __ballot(here && (mode == kByRank ? ci >= K : (mode == kByMass ? mi >= X : mi > X))), some = __ballot(here);
                 if (some == 0ull) return R;
                 k = any ? static_cast<uint32_t>(__ffsll(static_cast<unsigned long long>(any)) - 1)
