@@ -119,3 +119,24 @@ def test_rows_left_to_the_three_pass_code():
     back = (smp.flags.cpu().numpy() & m.FLAG_ROUTE_HANDED_BACK) != 0
     assert back[[0, 1, 3]].all() and back[2:rows:50].all()
     assert int(back.sum()) <= 5 + len(range(2, rows, 50)), np.flatnonzero(back)
+
+
+def test_rows_with_bad_parameters_among_those_left_over():
+    """The kernel behind takes several rows a workgroup: one with a bad temperature writes its flags at once, the rows after it - of the same workgroup,
+    left over as well - are answered as ever."""
+    cus = rows_of() - 1
+    rows, V = 3 * cus, 20001
+    c = _odd(rows, V, top_k=40, n_hist=100, n_bias=0)
+    bad = np.arange(0, cus, 2)
+    c["inv_t"][bad] = np.where(bad % 4, np.float32(-1), np.float32(0))
+    c["top_k"][cus:] = 0  # (against the batch's word)
+    m = gc.pkg()
+    d = gc.upload(c, hints=True)
+    d["top_k_max"] = 40
+    for _ in range(3):
+        smp = gc.sampler_for(c, d, 1).run()
+        res = gc.compare_rows(c, smp, [1, 3, *range(cus, rows, 37), rows - 1], 1, check_kept=False)
+        assert res["differ"] == 0, res
+        fl = smp.flags.cpu().numpy()
+        assert ((fl[bad] & m.FLAG_BAD_PARAM) != 0).all() and (smp.token.cpu().numpy()[bad] == -1).all()
+        assert ((fl[cus:] & m.FLAG_ROUTE_HANDED_BACK) != 0).all() and not (fl[cus:] & m.FLAG_BAD_PARAM).any()

@@ -22,12 +22,13 @@ __global__ void __launch_bounds__(WS_BLOCK) short_rest_kernel(BatchArgs A) {
     for (uint32_t row = blockIdx.x + threadIdx.x * n; row < A.rows; row += WS_BLOCK * n) any |= A.flags[row] == kTwinRest;
     if (!__syncthreads_or(any)) return;
     for (uint32_t row = blockIdx.x; row < A.rows; row += n) {
-        if (A.flags[row] != kTwinRest) continue;  // uniform
+        const bool left = A.flags[row] == kTwinRest;
+        __syncthreads();  // (every wave has read the word before one of them writes the row's flags there; and the row before is done with LDS)
+        if (!left) continue;  // uniform
         LeanArgPtr Ap = (LeanArgPtr)__builtin_amdgcn_kernarg_segment_ptr();
         asm volatile("" : "+s"(Ap));
         if (Ap->kept_ids) three_pass_row<true>(Ap, row);
         else three_pass_row<false>(Ap, row);
-        __syncthreads();
     }
 }
 }  // namespace
