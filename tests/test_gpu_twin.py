@@ -87,16 +87,21 @@ def test_min_p_rows_with_lists_of_thousands(V, allowed):
     assert (listed < 3900).sum() > rows // 4 and back.any()
 
 
-@pytest.mark.parametrize("dtype,V", [("f32", 100003), ("bf16", 262144)])
-def test_rows_whose_largest_tokens_lie_far_above_the_others(dtype, V):
-    """Cold rows: a few tokens 58 to 76 units of the exponent above the rest; of most rows one or two are in the sample, of some none is."""
+@pytest.mark.parametrize("dtype,V,n_hist", [("f32", 100003, 64), ("bf16", 262144, 64), ("f32", 384961, 257), ("f32", 384930, 262), ("f32", 384930, 250)])
+def test_rows_whose_largest_tokens_lie_far_above_the_others(dtype, V, n_hist):
+    """Cold rows: a few tokens 58 to 76 units of the exponent above the rest; of most rows one or two are in the sample, of some none is. The counts of the
+    sample's tokens reach their last bin, and are cleared again: tables of the touched tokens that would just not, and just, lie behind them in the list's place."""
     rows = rows_of()
-    c = _odd(rows, V, dtype, top_k=50, n_hist=64, n_bias=0)
+    c = _odd(rows, V, dtype, top_k=50, n_hist=n_hist, n_bias=0)
     c["inv_t"][:] = 20.0
     rng = np.random.default_rng(rows)
     x = (rng.standard_normal((rows, V), dtype=np.float32) * 0.5)
     for r in range(rows):
-        x[r, rng.integers(0, V, 6)] = (5.0 + 0.5 * rng.random()) + np.array([0.0, 0.013, 0.04, 0.11, 0.3, 0.4], np.float32)
+        at = rng.integers(0, V, 6)
+        if n_hist > 64:  # (touched tokens of the bitmap's first words, the first of the ranks)
+            at[:3] = [31, 33, 70]
+            c["hist"][r, 1:91] = np.arange(90)
+        x[r, at] = (5.0 + 0.5 * rng.random()) + np.array([0.0, 0.013, 0.04, 0.11, 0.3, 0.4], np.float32)
         c["hist"][r, 0] = int(x[r].argmax())
     c["logits"] = gc.f32_to_bf16_bits(x) if dtype == "bf16" else x
     run_short(c, 1, rows=some(rows, 17), kept_cap=64, handed_back=rows // 50, top_k_max=50)

@@ -236,16 +236,19 @@ void code_or_short(const ws_batch* b, BatchPlan& p) {
 }
 
 // LDS of a row of ws_twin.h: the list, the bitmap, the tables behind it; or, where that is more than half a compute unit's and the
-// other way is not, the tables below the bitmap, in the upper part of the list's place as far as they have to (8 KiB of it stay theirs alone: the
-// touched tokens above the threshold are listed while the tables are in use).
+// other way is not, the tables below the bitmap, in the upper part of the list's place as far as they have to (not over the sample's bin
+// counts, which are in use with them; the touched tokens above the threshold are listed in what is left below the tables).
 void twin_plan(uint32_t nW, uint64_t cap, BatchPlan& p) {
     const uint64_t map = uint64_t{nW} * 4u, tabs = ((uint64_t{nW} * 2u + 3u) & ~uint64_t{3}) + ((cap * 2u + 3u) & ~uint64_t{3});
     const uint64_t half = kMaxLds / 2u - kStaticTwin, list = 32768u;
     uint64_t ab = list, tabs_at = list + map, total = list + map + tabs;
-    if (total > half && map + list <= half && map + tabs + 8192u <= half) {
-        ab = (half - map) & ~uint64_t{15};
-        tabs_at = (ab - tabs) & ~uint64_t{3};
-        total = ab + map;
+    if (total > half && map + list <= half) {
+        const uint64_t low_ab = (half - map) & ~uint64_t{15}, counts = ws::kTwinBins * 4u;
+        if (low_ab >= tabs + counts + 3u) {
+            ab = low_ab;
+            tabs_at = (ab - tabs) & ~uint64_t{3};
+            total = ab + map;
+        }
     }
     p.twin_ab = static_cast<uint32_t>(ab);
     p.twin_tabs = static_cast<uint32_t>(tabs_at);

@@ -121,6 +121,7 @@ constexpr uint32_t kSplitStage = kSplitRowBytes, kSplitStageCap = 8192u, kSplitR
 // entries its rows may have, workgroups a row at most, and the workspace of a row (its layout: ws_few.h)
 constexpr uint32_t kShortCap = 4096u;
 constexpr uint32_t kFewShare = 40960u, kFewWide = 57344u, kFewLists = 10240u, kFewMaxParts = 16u, kFewRowBytes = 65536u;
+constexpr uint32_t kTwinBins = 2048u;  // ws_twin.h: bins of the sample's logits, 1/32 e-fold each
 constexpr uint32_t kShortSplitCtrl = kShortCap * 8u, kShortSplitRowBytes = kShortSplitCtrl + 768u;  // the same of ws_short.h's shared rows
 // Workspace of one row of the three-pass kernel: per history / bias entry a word of each of phase 0's two rank
 // tables, which sit out the first sweep there. Whole memory lines, so that rows share none.

@@ -19,7 +19,6 @@
 
 namespace ws {
 
-constexpr uint32_t kTwinBins = 2048u;  // of the sample's logits: 1/32 e-fold each
 constexpr uint32_t kTwinHead = 8u;  // vectors a thread of the sample that the threshold is fitted to
 
 // LDS: the list at 0 (32 KiB; first the sample's bin counts), the bitmap of the touched tokens at lds_ab, and at lds_cnt its 16-bit popcount
