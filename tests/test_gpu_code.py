@@ -250,3 +250,25 @@ def test_cold_rows(kind, T, hints):
     than 64 bits have room for. Below a temperature of 1/4096 the rows are the three-pass code's."""
     c = cold_case(T, kind, hints)
     run(c, hints=hints, handed_back=c["rows"] if T < 1 / 4096 else 0)
+
+
+@pytest.mark.parametrize("allowed", [None, 0.5])
+@pytest.mark.parametrize("hints", [False, True])
+def test_hot_rows_and_floors_below_the_last_bin(hints, allowed):
+    """Temperatures at which the last bin is not 50 e-folds below the maximum, and min-p floors that lie below it: nothing is left out
+    as long as every token that is not masked out has a bin of its own."""
+    c = case(12, 50001, allowed=allowed)
+    c["inv_t"][:] = 1 / np.array([8.0, 10.0, 30.0, 1.0, 1.0, 0.7] * 2)
+    c["min_p"][:] = [0.05, 0.0, 0.3, 1e-200, 1e-300, 1e-250] * 2
+    c["top_k"][:] = [0, 50, 0, 0, 60000, 45000] * 2
+    c["top_p"][:] = [1.0, 0.9, 1.0, 1.0, 1.0, 1.0, 0.9, 1.0, 0.99, 0.9, 0.9, 1.0]
+    if hints:
+        c["top_k"][:] = [0, 50, 0, 0, 1000, 500] * 2
+        c["min_p"][3::6] = 1e-3
+    run(c, hints=hints)
+    x = gc.bf16_bits_to_f32(c["logits"]).copy()
+    x[:, 17] = -400.0  # (a token in the last bins: the rows are the three-pass code's, but for the one whose floor lies above it)
+    c["logits"] = gc.f32_to_bf16_bits(x)
+    if allowed is not None:
+        c["allow"][:, 0] |= 1 << 17
+    run(c, hints=hints, handed_back=10 if hints else 12)

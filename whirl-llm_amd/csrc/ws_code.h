@@ -144,6 +144,7 @@ struct CodeShared {
     uint32_t red_u[WS_WAVES], red_v[WS_WAVES];
     uint32_t head_bin;  // first bin of the row's head
     uint32_t top_bin, top_key, bad;  // the first bin that holds a token; the touched tokens' largest logit; a logit this kernel does not take
+    uint32_t n_out;  // masked-out tokens, where it matters
     // the drawn token, when it is one of a bin's tied tokens: their value (both halves), the place among them, the touched ones among
     // them (ids in ascending order in `sorted`), and the outcome
     uint32_t state, value2, place, n_eq, eq_at, token;  // state: 0 the row is handed back, 1 `token` it is, 2 it is to be found, 3 and 4 see walk
@@ -244,6 +245,7 @@ __device__ __forceinline__ bool code_row(const BatchArgs& A, const uint32_t row,
         S.head_bin = kCodeBins;
         S.top_key = 0u;
         S.bad = 0u;
+        S.n_out = 0u;
         S.state = 0u;
         S.g_first[0] = S.g_first[1] = S.g_draw = kCodeGroups;
     }
@@ -545,9 +547,19 @@ __device__ __forceinline__ bool code_row(const BatchArgs& A, const uint32_t row,
     if (lane == 0u && first < kCodeBins) atomicMin(&S.top_bin, first);
     __syncthreads();
     const float m = fmaxf(S.top_bin < kCodeTail ? code_value(S.top_bin) : -INFINITY, S.top_key ? unkey32(S.top_key) : -INFINITY);
-    // (a touched token that is not for this kernel, a token above the bins, none in them, or bins that end too near the maximum)
+    // (a touched token that is not for this kernel, a token above the bins, or none in them)
     WSC_MARK(5);
-    if (S.bad || S.top_bin < 8u || !(m > -INFINITY) || !(__fsub_rn(m, code_value(kCodeTail)) * inv_t >= 50.f)) return false;
+    if (S.bad || S.top_bin < 8u || !(m > -INFINITY)) return false;
+    // The last bins are not looked at. Where they do not lie 50 e-folds below the maximum, or not below the min-p floor, nothing but masked-out tokens
+    // may be in them: those are counted, and the row is handed back further down if there are others.
+    const bool tail_matters = !(__fsub_rn(m, code_value(kCodeTail)) * inv_t >= 50.f) ||
+                              (use_min_p && code_bin(static_cast<float>(static_cast<double>(m) - S.floor_below)) >= kCodeTail);  // uniform
+    if (MASKED && tail_matters) {
+        uint32_t out = 0;
+        for (uint32_t w = t; w < nW; w += WS_BLOCK) out += static_cast<uint32_t>(__popc(~allow[w] & (w + 1u < nW ? 0xffffffffu : 0xffffffffu >> (nW * 32u - V))));
+        out = wave_sum(out);
+        if (lane == 0u) atomicAdd(&S.n_out, out);
+    }
     // (an anchor that lies below the maximum, or wastefully far above it, gives way to the maximum itself)
     // (the row's 64-bit values are kept in scalar registers: beside the row's vectors there is no room for them)
     const float aq = anchor_product(m <= anchor0 && (anchor0 - m) * c64 <= 1024.f ? anchor0 : m, c64);
@@ -633,6 +645,7 @@ __device__ __forceinline__ bool code_row(const BatchArgs& A, const uint32_t row,
         const uint32_t wn = row_incl_scan(S.red_u[lane & (WS_WAVES - 1u)]), we = TOUCHED ? row_incl_scan(S.red_v[lane & (WS_WAVES - 1u)]) : 0u;
         Z = lane_value(wm, WS_WAVES - 1u);
         n_all = lane_value(wn, WS_WAVES - 1u);
+        if (tail_matters && n_all + S.n_out < V) return false;  // uniform
         if (!(Z > 0.5 && Z < INFINITY)) return false;  // uniform (the maximum's own mass is 1: it has not been counted as it should)
         if (wave_has) {  // uniform
             const double base_m = wv ? lane_value(wm, wv - 1u) : 0.0;
@@ -931,7 +944,7 @@ __device__ __forceinline__ bool code_row(const BatchArgs& A, const uint32_t row,
         if (ok && use_min_p) {
             const float fx = static_cast<float>(static_cast<double>(m) - S.floor_below);
             const uint32_t bin = code_bin(fx);
-            if (bin < kCodeTail) {  // (else everything that counts passes)
+            if (bin < kCodeTail) {  // (else all passes that is not masked out)
                 const CodeAt at = look(ByPassing{}, bin >> 3, 0u, min_p, bin & 7u);
                 ok = at.ok;
                 // (a floor within a rounding of the bin's ends may have a neighbour's token near it)
@@ -941,6 +954,8 @@ __device__ __forceinline__ bool code_row(const BatchArgs& A, const uint32_t row,
                     n = max(at.rank, 1u);
                     M = at.rank ? at.cex : 1.0;
                 }
+            } else {
+                n = min(n, n_all);
             }
         }
         if (ok) {
