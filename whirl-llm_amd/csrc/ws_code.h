@@ -40,7 +40,8 @@ constexpr uint32_t kCodeTail = kCodeBins - 64u;   // the last 64 bins, from -384
 constexpr uint32_t kCodeGroups = kCodeBins / 8u;  // eight bins each, one group to a thread
 constexpr uint32_t kCodeSub = 512u;               // touched tokens in one bin, where a cut or the draw falls in it
 constexpr uint32_t kCodeFixBits = 44u;            // fixed point of the groups' touched masses (65535 of them at most)
-constexpr uint32_t kCodeHeldVecs = 20u;           // vectors a thread holds
+constexpr float kCodeWide = 4.f;                  // e-folds a group spans from which its touched masses are not taken against its top
+constexpr uint32_t kCodeHeldVecs = 19u;           // vectors a thread holds
 // Up to here the anchor of a row of logits below 512 lies at most 64 of its bins further above the maximum than it was put (anchor_product's 2^-21): 2900
 // of them, 45 e-folds, are left below the maximum. Colder rows lose some to the tail.
 constexpr float kCodeMaxInvT = 4096.f;
@@ -144,7 +145,8 @@ struct CodeShared {
     uint32_t red_u[WS_WAVES], red_v[WS_WAVES];
     uint32_t head_bin;  // first bin of the row's head
     uint32_t top_bin, top_key, bad;  // the first bin that holds a token; the touched tokens' largest logit; a logit this kernel does not take
-    uint32_t n_out;  // masked-out tokens, where it matters
+    uint32_t n_out;    // masked-out tokens, where it matters
+    uint32_t waiting;  // whether a touched token's mass waits for the largest of them
     // the drawn token, when it is one of a bin's tied tokens: their value (both halves), the place among them, the touched ones among
     // them (ids in ascending order in `sorted`), and the outcome
     uint32_t state, value2, place, n_eq, eq_at, token;  // state: 0 the row is handed back, 1 `token` it is, 2 it is to be found, 3 and 4 see walk
@@ -246,6 +248,7 @@ __device__ __forceinline__ bool code_row(const BatchArgs& A, const uint32_t row,
         S.top_key = 0u;
         S.bad = 0u;
         S.n_out = 0u;
+        S.waiting = 0u;
         S.state = 0u;
         S.g_first[0] = S.g_first[1] = S.g_draw = kCodeGroups;
     }
@@ -338,11 +341,25 @@ __device__ __forceinline__ bool code_row(const BatchArgs& A, const uint32_t row,
         const uint32_t w = __shfl(aw[MASKED ? c >> 2 : 0], static_cast<int>((static_cast<uint32_t>(c & 3) << 4) + (lane >> 2)));
         return w >> ((lane & 3u) * 8u);
     };
-    auto load_again = [&](uint32_t j) {  // a vector as count_round leaves the held ones
-        uint4 v = row_vector<1>(base, j, V);
+    auto as_held = [&](uint4& v, uint32_t j) __attribute__((always_inline)) {  // what count_round makes of a held vector
         trim(v, j);
         if (MASKED) mask_out(v, allow[min(j >> 2, nW - 1u)] >> ((j * 8u) & 31u));
+    };
+    auto load_again = [&](uint32_t j) {
+        uint4 v = row_vector<1>(base, j, V);
+        as_held(v, j);
         return v;
+    };
+    // the row's vectors behind the held ones, one asked for while another is looked at (with every one waited for, rows of 262144 tokens took 1 us more)
+    auto behind_held = [&](auto&& what) __attribute__((always_inline)) {
+        if (NV != kCodeHeldVecs || NV * WS_BLOCK >= nv) return;  // uniform
+        uint4 next = row_vector<1>(base, NV * WS_BLOCK + t, V);
+        for (uint32_t j0 = NV * WS_BLOCK; j0 < nv; j0 += WS_BLOCK) {  // uniform
+            uint4 v = next;
+            next = row_vector<1>(base, j0 + WS_BLOCK + t, V);  // (past the row: its end)
+            as_held(v, j0 + t);
+            what(v, j0);
+        }
     };
     // the first bin of the row's head (S.head_bin): the anchor of the masses, see mass_of
     auto look_at_head = [&](const uint4& v) __attribute__((always_inline)) {
@@ -471,13 +488,11 @@ __device__ __forceinline__ bool code_row(const BatchArgs& A, const uint32_t row,
 #pragma unroll
     for (int c = 0; c < NV; ++c) {
         count_round(c);
-        if ((c + 1) % (NV / 5) == 0 && (c + 1) / (NV / 5) <= 4) touch((c + 1) / (NV / 5) - 1);
+        constexpr int kStep = (NV + 4) / 5;
+        if ((c + 1) % kStep == 0 && (c + 1) / kStep <= 4) touch((c + 1) / kStep - 1);
     }
     WSC_MARK(2);
-    if (NV == kCodeHeldVecs)
-        for (uint32_t j0 = NV * WS_BLOCK; j0 < nv; j0 += WS_BLOCK) {  // uniform
-            count_vector(load_again(j0 + t));
-        }
+    behind_held([&](const uint4& v, uint32_t) { count_vector(v); });
     __syncthreads();
 
     WSC_MARK(3);
@@ -488,8 +503,33 @@ __device__ __forceinline__ bool code_row(const BatchArgs& A, const uint32_t row,
     const bool by_bins = A.code_head != 0u;
     const float c64 = inv_t * 64.f;
     const float anchor0 = code_value(min(S.head_bin, kCodeTail)) + A.code_above / inv_t;
+    const float aq0 = anchor_product(anchor0, c64);
     auto inside = [&](float tc) { return static_cast<double>(0x40000000u - static_cast<uint32_t>(bin_word(tc))); };  // of a bin's mass at its upper end, in units of 2^-30
     const double kFix = static_cast<double>(1ull << kCodeFixBits), kUnfix = 1.0 / kFix;
+    // A touched token's mass in fixed point against that of `top`, and (unfix_of) the other way round. `top` is that of the token's group; in a wide
+    // one no more than the largest touched token: an octave's eighth is 0.5 from 8 to 16 and 2 from 32 to 64, 10 to 40 e-folds at a temperature of 0.05, and
+    // against a top so far above it the largest token of the row would weigh nothing. (Each is off by 2^-45 e^4 of the normaliser at most.)
+    // The largest is known behind a barrier, so those of wide groups wait for a loop of their own - and in the kernel whose vectors leave no registers for
+    // this code beside the bias search all of them (256 rows, 2048 ids, us, those of narrow groups at once and all of them later: of 50257 26.6 / 27.4, of 151936
+    // 41.7 with 63 registers spilled / 40.9).
+    // (The row's 64-bit values are kept in scalar registers for the same reason.)
+    const double inv_t_d = lane_value(static_cast<double>(inv_t), 0u);
+    auto group_waits = [&](uint32_t g) { return NV == kCodeHeldVecs || code_group_step(g) * inv_t > kCodeWide / 8.f; };
+    auto group_by_bins = [&](uint32_t g, double top) {  // (none of them above the anchor, or in the tail)
+        return by_bins && top <= static_cast<double>(anchor0) && bin_coord(aq0, c64, code_value(g * 8u + 7u)) < 4000.f;
+    };
+    auto top_bin_of = [&](double top) { return static_cast<uint32_t>(bin_coord(aq0, c64, static_cast<float>(top))); };
+    auto fix_of = [&](float x, uint32_t g, double top) {
+        double e;
+        if (group_by_bins(g, top)) {
+            const float tc = bin_coord(aq0, c64, x);
+            const uint32_t d = static_cast<uint32_t>(tc) - top_bin_of(top);
+            e = S.s_exp[d >> 6] * S.s_exp[64u + (d & 63u)] * (inside(tc) * kFixInv);
+        } else {
+            e = code_exp((top - static_cast<double>(x)) * inv_t_d);
+        }
+        return static_cast<unsigned long long>(e * kFix + 0.5);
+    };
     if (TOUCHED) {
         uint32_t best = 0u;
         for (uint32_t r = t; r < n_touched; r += WS_BLOCK) {
@@ -512,6 +552,8 @@ __device__ __forceinline__ bool code_row(const BatchArgs& A, const uint32_t row,
             if (bin < kCodeTail && bin >= 8u) {
                 const uint32_t g = bin >> 3;
                 best = max(best, key32(x));
+                if (group_waits(g)) S.waiting = 1u;
+                else atomicAdd(&g_mass[g], fix_of(x, g, code_group_top(g)));
                 pos[r] = static_cast<uint16_t>(atomicAdd(&g_cnt[g], 1u));
             }
         }
@@ -520,6 +562,14 @@ __device__ __forceinline__ bool code_row(const BatchArgs& A, const uint32_t row,
     }
     if (TOUCHED) __syncthreads();
     WSC_MARK(4);
+    const double touched_max = TOUCHED && S.top_key ? static_cast<double>(unkey32(S.top_key)) : -INFINITY;
+    auto top_of = [&](uint32_t g) { return group_waits(g) ? fmin(code_group_top(g), touched_max) : code_group_top(g); };
+    if (TOUCHED && S.waiting)  // uniform
+        for (uint32_t r = t; r < n_touched; r += WS_BLOCK) {
+            const float x = adj[r];
+            const uint32_t bin = code_bin(x), g = bin >> 3;
+            if (bin < kCodeTail && bin >= 8u && group_waits(g)) atomicAdd(&g_mass[g], fix_of(x, g, top_of(g)));
+        }
     // ------------------------------------------------------------------ this thread's eight bins, and the prefix sums over the groups: tokens,
     // mass, touched tokens
     uint32_t c8[8], own = 0, first = kCodeBins;
@@ -561,9 +611,8 @@ __device__ __forceinline__ bool code_row(const BatchArgs& A, const uint32_t row,
         if (lane == 0u) atomicAdd(&S.n_out, out);
     }
     // (an anchor that lies below the maximum, or wastefully far above it, gives way to the maximum itself)
-    // (the row's 64-bit values are kept in scalar registers: beside the row's vectors there is no room for them)
-    const float aq = anchor_product(m <= anchor0 && (anchor0 - m) * c64 <= 1024.f ? anchor0 : m, c64);
-    const double m_d = lane_value(static_cast<double>(m), 0u), inv_t_d = lane_value(static_cast<double>(inv_t), 0u);
+    const float aq = m <= anchor0 && (anchor0 - m) * c64 <= 1024.f ? aq0 : anchor_product(m, c64);
+    const double m_d = lane_value(static_cast<double>(m), 0u);
     const double lift = lane_value(static_cast<double>(aq) * (1.0 / 64.0) - m_d * inv_t_d, 0u);
     auto exact_mass = [&](float x) { return code_exp(static_cast<double>(__fsub_rn(m, x)) * inv_t_d); };
     auto mass_of = [&](float x) {
@@ -571,35 +620,11 @@ __device__ __forceinline__ bool code_row(const BatchArgs& A, const uint32_t row,
         const float tc = bin_coord(aq, c64, x);
         return code_exp(static_cast<double>(static_cast<uint32_t>(tc)) * (1.0 / 64.0) - lift) * (inside(tc) * kFixInv);
     };
-    // A touched token's mass in fixed point, and the other way round: what comes to it. It is taken against that of `top_of`, the group's top, but
-    // no more than the maximum: an octave's eighth is 0.5 from 8 to 16 and 2 from 32 to 64, 10 to 40 e-folds at a temperature of 0.05, and against a
-    // top so far above it the largest token of the row would weigh nothing. (So each is off by 2^-45 of the normaliser at most.)
-    auto top_of = [&](uint32_t g) { return fmin(code_group_top(g), m_d); };
-    auto group_by_bins = [&](uint32_t g) { return by_bins && bin_coord(aq, c64, code_value(g * 8u + 7u)) < 4000.f; };  // (none of them in the tail)
-    auto top_bin_of = [&](uint32_t g) { return static_cast<uint32_t>(bin_coord(aq, c64, static_cast<float>(top_of(g)))); };
-    auto fix_of = [&](float x, uint32_t g) {
-        double e;
-        if (group_by_bins(g)) {
-            const float tc = bin_coord(aq, c64, x);
-            const uint32_t d = static_cast<uint32_t>(tc) - top_bin_of(g);
-            e = S.s_exp[d >> 6] * S.s_exp[64u + (d & 63u)] * (inside(tc) * kFixInv);
-        } else {
-            e = code_exp((top_of(g) - static_cast<double>(x)) * inv_t_d);
-        }
-        return static_cast<unsigned long long>(e * kFix + 0.5);
-    };
     auto unfix_of = [&](unsigned long long sum, uint32_t g) {
-        const double down = group_by_bins(g) ? static_cast<double>(top_bin_of(g)) * (1.0 / 64.0) - lift : (m_d - top_of(g)) * inv_t_d;
+        const double top = top_of(g);
+        const double down = group_by_bins(g, top) ? (static_cast<double>(top_bin_of(top)) - static_cast<double>(aq0)) * (1.0 / 64.0) + m_d * inv_t_d : (m_d - top) * inv_t_d;
         return static_cast<double>(sum) * kUnfix * code_exp(down);
     };
-    if (TOUCHED && n_touched) {
-        for (uint32_t r = t; r < n_touched; r += WS_BLOCK) {
-            const float x = adj[r];
-            const uint32_t bin = code_bin(x);
-            if (bin < kCodeTail) atomicAdd(&g_mass[bin >> 3], fix_of(x, bin >> 3));
-        }
-        __syncthreads();
-    }
     double Z;
     uint32_t n_all;
     {
@@ -742,7 +767,7 @@ __device__ __forceinline__ bool code_row(const BatchArgs& A, const uint32_t row,
                     const float x = adj[order[list + i]];
                     const uint32_t k = code_bin(x) & 7u;
                     atomicAdd(&S.bin_cnt[k], 1u);
-                    atomicAdd(&S.bin_mass[k], fix_of(x, g));
+                    atomicAdd(&S.bin_mass[k], fix_of(x, g, top_of(g)));
                 }
                 lanes_meet();
                 if (lane < 8u) e = S.bin_cnt[lane];
@@ -1098,10 +1123,7 @@ __device__ __forceinline__ bool code_row(const BatchArgs& A, const uint32_t row,
             if (c < NV - 5 || static_cast<uint32_t>(c) * WS_BLOCK < nv) {  // uniform
                 tally(q[c], static_cast<uint32_t>(c) * WS_BLOCK);
             }
-        if (NV == kCodeHeldVecs)
-            for (uint32_t j0 = NV * WS_BLOCK; j0 < nv; j0 += WS_BLOCK) {
-                tally(load_again(j0 + t), j0);
-            }
+        behind_held(tally);
         if (wv == kSolver)
             for (uint32_t i = lane; i < S.n_eq; i += 64u) atomicAdd(&block[(0xffffffffu - static_cast<uint32_t>(S.sorted[S.eq_at + i])) >> 9], 1u);
         __syncthreads();

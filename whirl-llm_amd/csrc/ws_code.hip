@@ -1,5 +1,5 @@
 // The sampler for bf16 rows (ws_code.h), a translation unit of its own: with and without an allow mask, with and without touched
-// tokens, for rows of up to 5, 10, 15 and 20 vectors a thread. 1024 threads per workgroup, 128 registers a thread, and the three-pass
+// tokens, for rows of up to 5, 10, 15 and 19 vectors a thread and for longer ones. 1024 threads per workgroup, 128 registers a thread, and the three-pass
 // code of ws_sample.h as a function for the rows it hands back.
 #define WS_BLOCK 1024
 #include <vector>
@@ -10,10 +10,10 @@
 namespace ws {
 
 typedef void (*CodeKernel)(BatchArgs);
-// by number: vectors a thread (5, 10, 15, 20), + 4 with touched tokens, + 8 with an allow mask
+// by number: vectors a thread (5, 10, 15, 19), + 4 with touched tokens, + 8 with an allow mask
 template <bool MASKED, bool TOUCHED>
 static void add_kernels(std::vector<CodeKernel>& k) {
-    k.insert(k.end(), {&code_batch_kernel<MASKED, TOUCHED, 5>, &code_batch_kernel<MASKED, TOUCHED, 10>, &code_batch_kernel<MASKED, TOUCHED, 15>, &code_batch_kernel<MASKED, TOUCHED, 20>});
+    k.insert(k.end(), {&code_batch_kernel<MASKED, TOUCHED, 5>, &code_batch_kernel<MASKED, TOUCHED, 10>, &code_batch_kernel<MASKED, TOUCHED, 15>, &code_batch_kernel<MASKED, TOUCHED, kCodeHeldVecs>});
 }
 static const std::vector<CodeKernel>& code_kernels() {
     static const std::vector<CodeKernel> all = [] {
