@@ -2768,10 +2768,13 @@ __device__ __forceinline__ void sample_row(const BatchArgs& A, const uint32_t bl
 
     // bases of the two ranges
     const bool has_r1 = r1hi >= r1lo;
-    const uint32_t c0base = pc[r0lo], n_r0 = r0hi >= r0lo ? pc[r0hi + 1] - c0base : 0u;
-    const double m0base = pm[r0lo];
-    const uint32_t c1base = has_r1 ? pc[r1lo] : 0u, n_r1 = has_r1 ? pc[r1hi + 1] - c1base : 0u;
-    const double m1base = has_r1 ? pm[r1lo] : 0.0;
+    // (the same in every lane: in scalar registers where the bin cache leaves no others - as eight vector registers across the gather they spilled some of the
+    // cache, in both single-sweep kernels of unsplit rows 40 and 56 registers against 30; 256 rows of 151936, us, 55.4 / 54.4. A split row's kernel has the room.)
+    auto to_scalar = [](auto v) { return FUSED && !SPLIT ? lane_value(v, 0u) : v; };
+    const uint32_t c0base = to_scalar(pc[r0lo]), n_r0 = to_scalar(r0hi >= r0lo ? pc[r0hi + 1] - c0base : 0u);
+    const double m0base = to_scalar(pm[r0lo]);
+    const uint32_t c1base = to_scalar(has_r1 ? pc[r1lo] : 0u), n_r1 = to_scalar(has_r1 ? pc[r1hi + 1] - c1base : 0u);
+    const double m1base = to_scalar(has_r1 ? pm[r1lo] : 0.0);
     const uint32_t n_list = n_r0 + n_r1;
     if (n_list > kCap || n_list == 0) flags |= kOverflow;
     // The kept-set dump of a top-k row (and of an open row's list) needs no pass over the row: range 0 starts at the top
