@@ -38,7 +38,7 @@ def run(c, hints=False, handed_back=0, max_differ=0, rng_mode=1):
     return smp
 
 
-SIZES = [8, 9, 33, 1000, 8191, 8192, 8193, 40960, 40961, 81920, 81921, 122880, 122881, 151937, 163840, 163841, 200003, 262144]
+SIZES = [8, 9, 33, 1000, 8191, 8192, 8193, 40960, 40961, 81920, 81921, 122880, 122881, 151937, 155648, 155649, 163840, 163841, 200003, 262144]
 
 
 @pytest.mark.parametrize("V", SIZES)
@@ -272,3 +272,17 @@ def test_hot_rows_and_floors_below_the_last_bin(hints, allowed):
     if allowed is not None:
         c["allow"][:, 0] |= 1 << 17
     run(c, hints=hints, handed_back=10 if hints else 12)
+
+
+@pytest.mark.parametrize("n_hist,n_bias", [(29, 0), (30, 2), (0, 29)])
+def test_more_entries_than_the_batch_declares(n_hist, n_bias):
+    """The tables are rounded up to four entries: a row that has one to three more than max_hist and max_bias say is refused all the same."""
+    m = gc.pkg()
+    c = case(5, 50001, n_hist=n_hist, n_bias=n_bias)
+    smp = gc.sampler_for(c, gc.upload(c), 1, max_split=1)
+    if n_hist:
+        smp.desc.max_hist -= 1
+    else:
+        smp.desc.max_bias -= 1
+    smp.run()
+    assert ((smp.flags & m.FLAG_BAD_PARAM) != 0).all() and (smp.token == -1).all(), smp.flags

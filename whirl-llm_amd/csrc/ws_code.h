@@ -256,12 +256,10 @@ __device__ __forceinline__ bool code_row(const BatchArgs& A, const uint32_t row,
     const float inv_t = P.inv_t;
     const double top_p = P.top_p, min_p = P.min_p;
     const bool use_top_p = top_p < 1.0, use_min_p = min_p > 0.0;
-    // rows this code does not take: a top-p that keeps nothing, a min-p above 1, the race draw, parameters the three-pass code reports, temperatures
-    // below kCodeMaxInvT's
+    // rows this code does not take: a top-p that keeps nothing, a min-p above 1, the race draw, parameters the three-pass code reports (more entries than
+    // the batch declares: its tables may have room for up to three of them), temperatures below kCodeMaxInvT's
     const bool open = P.top_k == 0u && !use_top_p && !use_min_p;
-    if (!(top_p > 0.0) || !(min_p <= 1.0) || P.race || !(inv_t > 0.f) || !(inv_t <= kCodeMaxInvT) ||
-        P.nh + P.nb > cap)
-        return false;
+    if (!(top_p > 0.0) || !(min_p <= 1.0) || P.race || !(inv_t > 0.f) || !(inv_t <= kCodeMaxInvT) || P.nh + P.nb > (TOUCHED ? A.patch_cap : 0u)) return false;
     if (wv == WS_WAVES - 1u) {  // (the seed by way of a vector register: as scalar arithmetic every wave would work the generator's rounds out)
         uint32_t seed_lo = static_cast<uint32_t>(P.seed);
         asm volatile("" : "+v"(seed_lo));
