@@ -145,3 +145,19 @@ def test_rows_with_bad_parameters_among_those_left_over():
         fl = smp.flags.cpu().numpy()
         assert ((fl[bad] & m.FLAG_BAD_PARAM) != 0).all() and (smp.token.cpu().numpy()[bad] == -1).all()
         assert ((fl[cus:] & m.FLAG_ROUTE_HANDED_BACK) != 0).all() and not (fl[cus:] & m.FLAG_BAD_PARAM).any()
+
+
+@pytest.mark.parametrize("V,top_k,n_hist,allowed", [(8192, 64, 0, None), (8193, 64, 0, None), (24576, 64, 1, None), (24577, 64, 300, None), (24576, 65, 300, 0.5), (16384, 128, 300, None),
+                                                    (16385, 128, 1, 0.5), (12288, 256, 300, 0.5), (12289, 256, 300, None), (12288, 257, 300, None), (245760, 64, 300, None),
+                                                    (245759, 64, 300, None), (245760, 128, 300, 0.3), (245760, 128, 300, None), (400000, 64, 300, 0.3)])
+def test_bf16_rows_either_side_of_the_lines_between_the_kernels(V, top_k, n_hist, allowed):
+    """Rows that go to this kernel or to ws_code.h by vocabulary, top-k, touched tokens and room: the answers are the oracle's on both sides."""
+    rows = rows_of()
+    c = _odd(rows, V, "bf16", top_k=top_k, n_hist=max(n_hist, 1), n_bias=0, allowed=allowed)
+    if not n_hist:
+        c["hist"] = None
+    smp = gc.sampler_for(c, gc.upload(c, hints=True), 1).run()
+    res = gc.compare_rows(c, smp, some(rows, 67), 1, check_kept=False)
+    assert res["differ"] == 0 and res["exact"] == len(some(rows, 67)), res
+    fl, m = smp.flags.cpu().numpy(), gc.pkg()
+    assert (fl & m.FLAG_ROUTE_SHORT).all() and not (fl & m.FLAG_ROUTE_HANDED_BACK).any()

@@ -208,6 +208,26 @@ bool twin_rows(const ws_batch* b) {
     return cus > 0 && b->rows > static_cast<uint32_t>(cus);
 }
 
+// bf16 rows with a top-k, more of them than compute units: whether ws_twin.h takes them or ws_code.h. ws_twin.h sorts a list of some 1.5 top-k keys, the time of
+// which grows with the top-k, and its sweep costs more a token; touched tokens are cheaper in it. So it takes short rows with touched tokens and a list that is
+// not long, and rows so long that ws_code.h reads two fifths of them twice, where two of its own fit a compute unit. Microseconds, ws_twin.h and ws_code.h (N(0, 2) rows;
+// histories of 1000 ids but where it says so):
+//   1000 rows of    8000: top-k 50 37.8 / 62.6, 128 44.8 / 63.3, 300 49.6 / 64.6; without histories 30.5 / 36.4, 37.4 / 36.4, 41.5 / 36.4
+//               of 12288: 42.0 / 61.8, 50.5 / 65.4, 55.5 / 65.2
+//               of 16384: 45.6 / 61.6, 55.3 / 65.2, 61.2 / 66.6; 16 ids 43.3 / 54.0, 52.4 / 54.9, 59.8 / 54.8; no ids 37.2 / 38.2 (rows of raised tokens 44.1 / 37.9), 47.2 / 38.5
+//   512 rows of  24000: 29.3 / 33.3, 36.4 / 35.0, 41.5 / 36.6; 16 ids 28.3 / 29.5, 36.0 / 29.4; no ids 25.1 / 21.4
+//            of  28032: 32.3 / 33.6, 37.4 / 34.7; 16 ids 30.9 / 30.0; raised tokens (600 rows) 55.8 / 46.2
+//            of 151936: 63.0 / 56.7, 66.7 / 57.1       of 220032: 74.3 / 71.2, 80.2 / 70.5
+//            of 245760: 78.5 / 80.5, 82.6 / 80.2       of 262144: 84.2 / 88.1, 88.9 / 88.2; no ids (400 rows) 74.5 / 65.0
+//   400 masked rows (three tokens in ten) of 200000: 70.4 / 71.1, 73.4 / 71.8; of 262144 83.4 / 96.1, 87.6 / 96.0, top-k 300 97.1 / 97.1
+//   300 rows of 360000, two a unit: 91.6 / 99.2, 98.9 / 99.7; of 400000, one: 134.7 / 109.1
+bool twin_pays(const ws_batch* b, uint64_t cap, const BatchPlan& p) {
+    const uint32_t k = b->top_k_max, V = b->vocab;
+    if (cap == 0) return k <= 64u && V <= 8192u;
+    if (V >= 245760u) return p.twin_total <= kMaxLds / 2u - kStaticTwin && k <= (b->allow ? 128u : 64u);
+    return V <= (k <= 64u ? 24576u : k <= 128u ? 16384u : k <= 256u ? 12288u : 0u);
+}
+
 // bf16 rows of the short-list kind: ws_code.h, ws_few.h or ws_short.h. Few rows are ws_few.h's: it shares them, and its lists are short -
 // but a list of some hundred keys has to be sorted, which costs more than counting a row that is not long, and two workgroups a row
 // are not much of a share. Microseconds, ws_few.h and ws_code.h (1000-id histories): top-k 50: 64 rows of 50257 16.0 / 18.4, 100 rows 19.9 /
@@ -216,19 +236,15 @@ bool twin_rows(const ws_batch* b) {
 // min-p alone: 100 of 50257 18.2 / 18.5, 128 of 60000 18.9 / 19.5. What ws_few.h does not take: top-k 50, ws_short.h and ws_code.h: 200 of 32000 24.9 /
 // 16.5, 1000 of 8000 with a min-p 62.2 / 59.1, 256 of 151936 52.2 / 29.4, 400 of 262144 118.6 / 90.0. Rows without a top-k have a short list and nothing to
 // estimate: 150 of 20000 14.3 / 16.5, 1000 of 8000 46.2 / 56.3, 300 of 40000 31.9 / 31.2, 256 of 50257 22.5 / 20.0, 256 of 151936 45.1 / 30.4; longer than the
-// registers hold and in four slices or more: 60 of 262144 32.0 / 37.9, in two: 100 of 262144 44.7 / 38.2. More rows than compute units are
-// ws_twin.h's where its sweep is a small part of the row or the row is longer than the registers hold, and the list is short: 1000 rows, top-k 50 (and
-// 300), ws_twin.h and ws_code.h: of 8000 36.3 / 54.4 (47.1 / 57.2), of 16000 44.7 / 55.4 (59.6 / 59.5), of 24000 52.5 / 56.4 (71.7 / 60.2); 400 of 16000,
-// top-k 50, 24.7 / 27.9; 400 of 180000 67.1 / 61.7, 700 of 200000, top-k 100, 118 / 104, 400 of 262144, top-k 50, 80.9 / 96.6, 1024 154 / 191, 512
-// with a top-k of 300 100.8 / 99.9.
-void code_or_short(const ws_batch* b, BatchPlan& p) {
+// registers hold and in four slices or more: 60 of 262144 32.0 / 37.9, in two: 100 of 262144 44.7 / 38.2. More rows than compute units: see twin_pays.
+void code_or_short(const ws_batch* b, uint64_t cap, BatchPlan& p) {
     const bool by_k = b->top_k && b->top_k_max >= 1u;
     if (p.few_parts) {
         const bool long_lists = b->top_k_max > 512u ? b->vocab <= 163840u : b->top_k_max > 256u && b->vocab <= 40960u;
         p.code = by_k && (long_lists || (p.few_parts <= 2u && b->vocab > 32768u));
         if (p.code) p.few_parts = 0;
     } else if (by_k) {
-        p.code = !(twin_rows(b) && b->top_k_max <= 128u && (b->vocab <= 16384u || b->vocab >= 245760u));
+        p.code = !(twin_rows(b) && twin_pays(b, cap, p));
     } else {
         p.code = b->vocab > 40960u && !(b->vocab > 163840u && short_split_log2(b) >= 2u);
     }
@@ -360,7 +376,7 @@ BatchPlan plan_batch(const ws_batch* b, bool few = true) {
         p.split_log2 = 0;
         p.workspace = p.workspace_min = 0;
         if (few) few_plan(b, cap, maps, p);
-        if (p.code) code_or_short(b, p);
+        if (p.code) code_or_short(b, cap, p);
         if (!p.code && !p.few_parts && (p.split_log2 = short_split_log2(b)) != 0u) p.workspace = p.workspace_min = uint64_t{b->rows} * ws::kShortSplitRowBytes;
         p.twin = !p.code && !p.few_parts && !p.split_log2 && twin_rows(b);
         p.err = WS_OK;
