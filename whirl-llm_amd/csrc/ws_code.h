@@ -7,8 +7,8 @@
 // sorted, no bin is read again, and a row may have a top-k, a top-p and a min-p in any combination, or none: a top-k is a place in
 // the order like the others (src/sampling/sampler.cpp:15-78, :118-146).
 //
-//   * 20 vectors of 128 bits a thread hold 163840 tokens, six of them on their way at a time. Longer rows are read again behind the
-//     20th when the drawn token is looked for.
+//   * 19 vectors of 128 bits a thread hold 155648 tokens, six of them on their way at a time. Longer rows are read again behind the
+//     19th when the drawn token is looked for.
 //   * A token's bin by packed 16-bit integer instructions, two tokens each: saturating subtractions, a maximum and a minimum
 //     (code_pair), then one 32-bit LDS addition a token. Bins go from 512 down to 2^-23, one for everything nearer to zero, and from
 //     -2^-23 down to -512. Masked-out tokens become NaN in place: the last bins, one to a lane, where nothing is looked at.
@@ -78,10 +78,11 @@ __device__ __forceinline__ uint32_t code_bin(float x) {
 __device__ __forceinline__ float code_group_step(uint32_t g) { return __fsub_rn(code_value(g * 8u), code_value(g * 8u + 1u)); }
 __device__ __forceinline__ double code_group_top(uint32_t g) { return static_cast<double>(code_value(g * 8u)) + static_cast<double>(code_group_step(g)); }
 
-// e^-a, of either sign: 2^k e^r with |r| <= ln 2 / 2, the series to r^13 (two units in the last place; a quarter of the library's instructions)
+// e^-a, of either sign: 2^k e^r with |r| <= ln 2 / 2, the series to r^13 (two units in the last place; a quarter of the library's instructions).
+// The reduction is Cody and Waite's, with ln 2 in the two parts that Sun's public fdlibm (e_exp.c) gives it.
 __device__ __forceinline__ double code_exp(double a) {
     const double k = __builtin_rint(a * -1.44269504088896340736);
-    double r = fma(k, -6.93147180369123816490e-01, -a);  // (ln 2 in two parts)
+    double r = fma(k, -6.93147180369123816490e-01, -a);
     r = fma(k, -1.90821492927058770002e-10, r);
     double p = 1.0 / 6227020800.0;
     p = fma(p, r, 1.0 / 479001600.0);
