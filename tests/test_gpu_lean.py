@@ -110,7 +110,7 @@ def _as_bf16(c):
 
 
 def test_bf16_zipfian_rows_with_hundreds_of_ties_at_the_cut():
-    """configs[2]'s rows: bf16, -1.1 ln(rank) + noise, top-p 0.9 - some 17000 tokens kept, and the cut among the several
+    """cfg3's rows: bf16, -1.1 ln(rank) + noise, top-p 0.9 - some 17000 tokens kept, and the cut among the several
     hundred that share its bf16 value."""
     c = gc.make_cfg3(rows=64)
     # (two of these rows have their cut within 1e-7 of a token's edge and are reported as such, by every kernel here)

@@ -275,7 +275,7 @@ def test_bias_values_of_one_id_are_added_one_by_one(mode):
     print(res)
 
 
-@pytest.mark.parametrize("rng_mode", [1, 0])  # configs[0] names a Philox-seeded draw; the reference's own uniform as well
+@pytest.mark.parametrize("rng_mode", [1, 0])  # cfg1 is a Philox-seeded draw; the reference's own uniform as well
 @pytest.mark.parametrize("mode", MODES)
 def test_cfg1_shape(mode, rng_mode):
     res, _ = run_case(gc.make_cfg1(), rng_mode, mode=mode)
@@ -307,7 +307,7 @@ def test_cfg3_full_size(mode):
 
 
 def test_cfg5_full_size():
-    """configs[4] at its full size: 1024 rows x 262144 fp32 logits (1 GiB), 90 % masked, 8192-id histories, 500 bias entries,
+    """cfg5 at its full size: 1024 rows x 262144 fp32 logits (1 GiB), 90 % masked, 8192-id histories, 500 bias entries,
     top-k 1000 + top-p 0.95. The vocabulary is past what the single-sweep mode caches, so this is the two-sweep route.
     A sample of rows against the oracle, every row for the size-independent facts: a token that is allowed, a kept count
     within top-k, no failure flag."""

@@ -38,7 +38,7 @@ def run_short(c, rng_mode, rows=None, kept_cap=1024, max_differ=0, handed_back=0
 
 @pytest.mark.parametrize("rng_mode", [1, 0])
 def test_cfg1_one_row_shared_by_sixteen_workgroups(rng_mode):
-    """one row of 151936, 256-id history, repetition 1.1, T 0.8, top-k 40, top-p 0.95."""
+    """cfg1: one row of 151936, 256-id history, repetition 1.1, T 0.8, top-k 40, top-p 0.95."""
     c = gc.make_cfg1()
     res, smp = run_short(c, rng_mode, kept_cap=256)
     assert res["exact"] == 1 and res["short"] == 1, res
@@ -69,7 +69,7 @@ def test_all_features_top_k_from_1_to_1000(max_split):
 
 
 def test_long_masked_rows_top_k_1000():
-    """configs[4]'s shape: 262144 tokens, 90 % masked out, 8192-id histories, 500 bias entries, top-k 1000, top-p 0.95."""
+    """cfg5's shape: 262144 tokens, 90 % masked out, 8192-id histories, 500 bias entries, top-k 1000, top-p 0.95."""
     c = gc.make_cfg5(rows=32)
     res, _ = run_short(c, 1, rows=range(0, 32, 3))
     assert res["short"] == 32, res
@@ -140,7 +140,7 @@ def test_static_entry_point_and_the_workspace_one_agree():
 
 
 def test_cfg2_full_size_rows_with_a_top_k_and_rows_with_a_min_p_alone():
-    """configs[1] as it is: 64 rows, top-k in {0, 20, 50}, min-p 0.05 on every row, top-p 0.8 .. 1, bias, 4096-id
+    """cfg2 as it is: 64 rows, top-k in {0, 20, 50}, min-p 0.05 on every row, top-p 0.8 .. 1, bias, 4096-id
     histories; four workgroups a row."""
     c = gc.make_cfg2()
     res, smp = run_short(c, 1, kept_cap=1024)

@@ -232,7 +232,7 @@ def test_classic_verify_special_cases():
 
 
 def test_classic_verify_cfg4_shape():
-    """32 sequences x 9 positions x 151936, target / draft logits mixed 70 / 30 (acceptance near 0.6)."""
+    """cfg4: 32 sequences x 9 positions x 151936, target / draft logits mixed 70 / 30 (acceptance near 0.6)."""
     rng = np.random.default_rng(312)
     p, q, draft, seed, step0 = spec_case(rng, 32, 9, 151936)
     rate, near = check_spec(p, q, draft, seed, step0, 1)
