@@ -511,8 +511,10 @@ __device__ __forceinline__ bool code_row(const BatchArgs& A, const uint32_t row,
     // The largest is known behind a barrier, so those of wide groups wait for a loop of their own - and in the kernel whose vectors leave no registers for
     // this code beside the bias search all of them (256 rows, 2048 ids, us, those of narrow groups at once and all of them later: of 50257 26.6 / 27.4, of 151936
     // 41.7 with 63 registers spilled / 40.9).
-    // (The row's 64-bit values are kept in scalar registers for the same reason.)
-    const double inv_t_d = lane_value(static_cast<double>(inv_t), 0u);
+    // (The row's 64-bit values are kept in scalar registers there for the same reason; in the others, where vector registers are left, that only
+    // lengthens the chain: 250 rows with 500 ids, us, scalar / vector: of 80000 24.8 / 24.0, of 41000 21.3 / 21.0.)
+    auto row_value = [](double v) __attribute__((always_inline)) { return NV == kCodeHeldVecs ? lane_value(v, 0u) : v; };
+    const double inv_t_d = row_value(static_cast<double>(inv_t));
     auto group_waits = [&](uint32_t g) { return NV == kCodeHeldVecs || code_group_step(g) * inv_t > kCodeWide / 8.f; };
     auto group_by_bins = [&](uint32_t g, double top) {  // (none of them above the anchor, or in the tail)
         return by_bins && top <= static_cast<double>(anchor0) && bin_coord(aq0, c64, code_value(g * 8u + 7u)) < 4000.f;
@@ -611,8 +613,8 @@ __device__ __forceinline__ bool code_row(const BatchArgs& A, const uint32_t row,
     }
     // (an anchor that lies below the maximum, or wastefully far above it, gives way to the maximum itself)
     const float aq = m <= anchor0 && (anchor0 - m) * c64 <= 1024.f ? aq0 : anchor_product(m, c64);
-    const double m_d = lane_value(static_cast<double>(m), 0u);
-    const double lift = lane_value(static_cast<double>(aq) * (1.0 / 64.0) - m_d * inv_t_d, 0u);
+    const double m_d = row_value(static_cast<double>(m));
+    const double lift = row_value(static_cast<double>(aq) * (1.0 / 64.0) - m_d * inv_t_d);
     auto exact_mass = [&](float x) { return code_exp(static_cast<double>(__fsub_rn(m, x)) * inv_t_d); };
     auto mass_of = [&](float x) {
         if (!by_bins) return exact_mass(x);  // uniform
