@@ -327,3 +327,64 @@ def test_one_workspace_for_batches_of_any_shape():
         assert torch.equal(got.token, want.token) and torch.equal(got.n_kept, want.n_kept) and torch.equal(got.flags, want.flags), (rows, V, top_k)
         assert torch.allclose(got.stats, want.stats, rtol=1e-6, atol=0)  # (a shared row's sum is taken in the order its parts arrive)
         assert not work.any().item(), (rows, V, top_k)
+
+
+@pytest.mark.parametrize("rows", [1, 7, 8, 9, 16, 17, 33])
+def test_rows_whose_parts_share_a_chiplet_and_rows_whose_parts_do_not(rows):
+    """Up to 16 rows of 16 parts go a row to a chiplet, with workgroups that have no row where the rows are no multiple of eight; 17 and 33 do not."""
+    run(case(rows, 32771, n_hist=200, n_bias=5))
+    m = gc.pkg()
+    x = torch.from_numpy((np.random.default_rng(rows).standard_normal((rows, 32772)) * 2).astype(np.float32)).cuda()
+    work = m.topk_rows_workspace(32772, 64, rows)
+    for _ in range(2):
+        got = m.topk_rows(x, 64, 1.0, workspace=work)
+        assert torch.equal(got[0], m.topk_rows(x, 64, 1.0)[0]) and not work.any().item()
+
+
+@pytest.mark.parametrize("kind", ["normal", "steps", "halves", "far", "flat"])
+@pytest.mark.parametrize("K", [129, 300, 512])
+def test_top_lists_whose_last_bucket_alone_is_put_in_order(kind, K):
+    """Lists of more than 128 keys: distinct logits, many ties at the cut, most of the row tied, one token so far above the others that
+    they share a bucket, and a row of one value."""
+    m = gc.pkg()
+    x = (np.random.default_rng(K).standard_normal((3, 40000)) * 2).astype(np.float32)
+    if kind in ("steps", "halves"):
+        x = np.round(x * (32 if kind == "steps" else 2)) / np.float32(32 if kind == "steps" else 2)
+    if kind == "far":
+        x[:, 777] = 1e30
+    if kind == "flat":
+        x[:] = 0.25
+    dx = torch.from_numpy(x).cuda()
+    work = m.topk_rows_workspace(x.shape[1], K, x.shape[0])
+    for _ in range(2):
+        ids, vals, _ = m.topk_rows(dx, K, 1.25, workspace=work)
+        for r in range(x.shape[0]):
+            want = np.sort(np.lexsort((np.arange(x.shape[1]), -x[r].astype(np.float64)))[:K])
+            assert np.array_equal(ids[r].cpu().numpy(), want) and np.array_equal(vals[r].cpu().numpy(), x[r][want])
+    assert not work.any().item()
+
+
+@pytest.mark.parametrize("n", [4096, 8003, 24064, 34298])
+def test_draft_draws_of_rows_of_any_length_are_shared(n):
+    """ws_draft_sample_rows_ws against the kernel that gives a row to one workgroup, with and without a vocabulary map, for every number of
+    candidates a step of its sums can end at: same candidates, draws and probabilities (the normaliser: float sums in another order)."""
+    m = gc.pkg()
+    rng = np.random.default_rng(n)
+    tks = [1, 3, 4, 5, 20, 31, 32, 0, 40]
+    rows = len(tks)
+    x = torch.from_numpy((rng.standard_normal((rows, n)) * 3).astype(np.float32)).cuda()
+    vmap = torch.from_numpy(rng.permutation(n).astype(np.int32)).cuda()
+    work = torch.zeros(int(m.lib().ws_draft_sample_rows_workspace(n, rows)), dtype=torch.uint8, device="cuda")
+    assert work.numel() > 0
+    args = [dict(top_k=tks[b], qoff=b * m.Q_WORDS, inv_t=1.1, top_p=[1.0, 0.95, 0.6][b % 3], min_p=[0.0, 0.02][b % 2], key=int(rng.integers(1, 1 << 62))) for b in range(rows)]
+    for mp in (None, vmap):
+        got = []
+        for w in (None, work):
+            ctl = torch.zeros(rows * 64, dtype=torch.int32, device="cuda")
+            q = torch.zeros(rows * m.Q_WORDS, dtype=torch.int32, device="cuda")
+            m.draft_sample_rows(x, ctl, [64 * b for b in range(rows)], 2, args, q, vmap=mp, workspace=w)
+            got.append((ctl.cpu(), q.cpu().view(rows, m.Q_WORDS)))
+        (c0, q0), (c1, q1) = got
+        assert torch.equal(c0, c1) and torch.equal(q0[:, :33], q1[:, :33])
+        assert torch.allclose(q0[:, 33:65].contiguous().view(torch.float32), q1[:, 33:65].contiguous().view(torch.float32), rtol=1e-5, atol=1e-9)
+    assert not work.any().item()

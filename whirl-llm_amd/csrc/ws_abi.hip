@@ -50,11 +50,11 @@ int launch_few(hipStream_t stream, const BatchArgs& a, unsigned lds_bytes, unsig
 int prepare_few(unsigned lds_limit);
 // ws_top.hip: topk_rows, dflash_topk and draft_sample_rows with rows shared between workgroups
 int launch_topk_shared(hipStream_t stream, const float* x, int n, int K, float inv_t, int* ids, float* vals, float* stats, unsigned rows, unsigned parts,
-                       unsigned chunk_log2, unsigned char* work);
+                       unsigned chunk_log2, unsigned together, unsigned char* work);
 int launch_dflash_shared(hipStream_t stream, const float* x, int n, int ld, int k, int* ids, float* vals, unsigned rows, unsigned parts, unsigned chunk_log2,
-                         unsigned char* work);
+                         unsigned together, unsigned char* work);
 int launch_draft_shared(hipStream_t stream, const float* x, int n, int* ctl_all, const void* area, int r, const int* map, const void* args, int* qbuf,
-                        unsigned rows, unsigned parts, unsigned chunk_log2, unsigned char* work);
+                        unsigned rows, unsigned parts, unsigned chunk_log2, unsigned together, unsigned char* work);
 int launch_argmax_shared(hipStream_t stream, int mode, const float* x, int n, int* out, const void* dst, int* ids, int* pos, int advance, unsigned rows,
                          unsigned parts, unsigned long long* scratch, unsigned long long tag);
 int prepare_top();
@@ -77,7 +77,7 @@ constexpr uint32_t kStaticShort = 9216u;
 // the same for the kernel of two rows a compute unit, which calls nothing
 constexpr uint32_t kStaticTwin = 1024u;
 // the same for the kernel of few rows
-constexpr uint32_t kStaticFew = 10240u;
+constexpr uint32_t kStaticFew = 8192u;
 // the same for the kernel of bf16 rows
 constexpr uint32_t kStaticCode = 14336u;
 // the lean kernel's own tables and those of the three-pass code it calls
@@ -126,6 +126,13 @@ int compute_units() {
     return n > 0 ? n : 0;
 }
 
+// Whether a shared row's parts go to one chiplet: where its compute units take all parts of its rows at once. (What the parts leave for each other and
+// the ids and parameters they all read then come from one L2. Apart and together, us: one row of 20000 9.9 / 9.7, of 151936 10.6 / 10.2, of 262144 11.5 / 11.3, a
+// decode step with parameters in host memory 20.7 / 20.1; 5 rows level.)
+uint32_t parts_together(uint32_t parts, uint32_t rows) {
+    return (rows + ws::kChiplets - 1u) / ws::kChiplets * parts <= static_cast<uint32_t>(compute_units()) / ws::kChiplets ? 1u : 0u;
+}
+
 // Short-list rows that ws_few.h does not take - too long for the registers of as many workgroups as there are compute units
 // for, or with histories too long for its lists - shared by the short-list kernel's own workgroups, which sweep a slice each: 2^n
 // of them, 16 at most, of at least 8192 tokens, within the compute units (a second round of workgroups is not worth it).
@@ -165,7 +172,8 @@ void few_plan(const ws_batch* b, uint64_t cap, uint64_t maps, BatchPlan& p) {
     const bool twice = b->dtype == WS_DTYPE_BF16 && b->vocab >> short_split_log2(b) > 90000u;
     if (parts < 2u || parts > most || static_cast<uint64_t>(b->rows) * parts > (twice ? 2ull : 1ull) * cus) return;
     const uint64_t three = (cap * 8u > 65536u ? ((cap * 8u + 15u) & ~uint64_t{15}) : 65536u) + maps;
-    const uint64_t own = 32768u + (parts < least ? ws::kFewWide : ws::kFewShare) * 2u;
+    const uint32_t room = parts < least ? ws::kFewWide : ws::kFewShare;
+    const uint64_t own = 32768u + room * 2u + ws::few_bit_words(room / 512u) * 2048u;
     const uint64_t total = own > three ? own : three;
     if (total + kStaticFew > kMaxLds) return;
     p.few_parts = parts;
@@ -645,24 +653,22 @@ int ws_draft_sample_rows(void* stream, const float* x, int n, int* ctl_all, cons
 }
 
 namespace {
-unsigned top_parts(int n, int K, unsigned rows);
+unsigned shared_parts(int n, unsigned rows);
 unsigned chunk_log2(const void* x, uint64_t row_bytes);
 bool top_workspace_ok(const void* w, uint64_t bytes, unsigned rows);
 }
-uint64_t ws_topk_rows_workspace(int n, int K, unsigned rows);
-
-// (the draft sampler lists K <= 32 tokens: it splits like a topk_rows of 32)
-uint64_t ws_draft_sample_rows_workspace(int n, unsigned rows) { return ws_topk_rows_workspace(n, 32, rows); }
+// (a draft's row of any length and alignment is shared: with a workgroup a row and draw 7 rows of 24064 took 17 us, and take 9)
+uint64_t ws_draft_sample_rows_workspace(int n, unsigned rows) { return shared_parts(n, rows) ? uint64_t{rows} * ws::kFewRowBytes : 0ull; }
 
 int ws_draft_sample_rows_ws(void* stream, const float* x, int n, int* ctl_all, const ws_row_idx* area, int r, const int* map,
                             const ws_dsamp_args* a, int* qbuf, unsigned rows, void* workspace, uint64_t workspace_bytes) {
     if (!x || !ctl_all || !area || !a || !qbuf || n <= 0 || r < 0 || r >= 16 || rows == 0 || rows > WS_MAX_TABLE_ROWS)
         return WS_E_INVALID;
-    const unsigned parts = top_parts(n, 32, rows);
+    const unsigned parts = shared_parts(n, rows);
     if (!parts || !top_workspace_ok(workspace, workspace_bytes, rows))
         return ws_draft_sample_rows(stream, x, n, ctl_all, area, r, map, a, qbuf, rows);
     return ws::launch_draft_shared(S(stream), x, n, ctl_all, area, r, map, a, qbuf, rows, parts, chunk_log2(x, uint64_t{4} * static_cast<unsigned>(n)),
-                                   static_cast<unsigned char*>(workspace));
+                                   parts_together(parts, rows), static_cast<unsigned char*>(workspace));
 }
 
 int ws_topk_rows(void* stream, const float* x, int n, int K, float inv_t, int* ids, float* vals, float* stats, unsigned rows) {
@@ -672,10 +678,10 @@ int ws_topk_rows(void* stream, const float* x, int n, int K, float inv_t, int* i
 }
 
 namespace {
-// workgroups a row of the shared top-k kernels (0: rows are not shared): a short list, shares that fit the registers of 512
-// threads and have 2048 tokens at least, fewer rows than half the compute units
-unsigned top_parts(int n, int K, unsigned rows) {
-    if (n < 32768 || n % 4 != 0 || rows == 0 || K <= 0 || K > 512) return 0u;  // (the shapes the workspace functions have always named)
+// workgroups a row of the kernels of ws_top.h (0: rows are not shared): shares that fit the registers of 512 threads and have 2048
+// tokens at least, fewer rows than half the compute units
+unsigned shared_parts(int n, unsigned rows) {
+    if (n <= 0 || rows == 0) return 0u;
     const uint64_t cus = static_cast<uint64_t>(compute_units());
     const unsigned least = (static_cast<unsigned>(n) + ws::kFewShare - 1u) / ws::kFewShare;
     uint64_t parts = cus / rows;
@@ -683,6 +689,10 @@ unsigned top_parts(int n, int K, unsigned rows) {
     if (parts > static_cast<unsigned>(n) / 2048u) parts = static_cast<unsigned>(n) / 2048u;
     if (parts < least) parts = least;
     return parts < 2u || parts > ws::kFewMaxParts || rows * parts > 2u * cus || 2u * rows > cus ? 0u : static_cast<unsigned>(parts);
+}
+unsigned top_parts(int n, int K, unsigned rows) {
+    if (n < 32768 || n % 4 != 0 || K <= 0 || K > 512) return 0u;  // (a short list, and the shapes the workspace functions have always named)
+    return shared_parts(n, rows);
 }
 // chunks of eight lanes, a line of memory; where rows lie off the lines a chunk straddles two, and longer ones straddle fewer
 unsigned chunk_log2(const void* x, uint64_t row_bytes) { return reinterpret_cast<uintptr_t>(x) % 16u == 0 && row_bytes % 16u == 0 ? 3u : 5u; }
@@ -699,7 +709,7 @@ int ws_topk_rows_ws(void* stream, const float* x, int n, int K, float inv_t, int
     const unsigned parts = top_parts(n, K, rows);
     if (!parts || !top_workspace_ok(workspace, workspace_bytes, rows)) return ws_topk_rows(stream, x, n, K, inv_t, ids, vals, stats, rows);
     return ws::launch_topk_shared(S(stream), x, n, K, inv_t, ids, vals, stats, rows, parts, chunk_log2(x, uint64_t{4} * static_cast<unsigned>(n)),
-                                  static_cast<unsigned char*>(workspace));
+                                  parts_together(parts, rows), static_cast<unsigned char*>(workspace));
 }
 
 uint64_t ws_dflash_topk_workspace(int n, int ld, unsigned rows) {
@@ -712,7 +722,7 @@ int ws_dflash_topk_ws(void* stream, const float* x, int n, int ld, int k, int* i
     const unsigned parts = ld % 4 == 0 ? top_parts(n, k, rows) : 0u;
     if (!parts || !top_workspace_ok(workspace, workspace_bytes, rows)) return ws_dflash_topk(stream, x, n, ld, k, ids, vals, rows);
     return ws::launch_dflash_shared(S(stream), x, n, ld, k, ids, vals, rows, parts, chunk_log2(x, uint64_t{4} * static_cast<unsigned>(ld)),
-                                    static_cast<unsigned char*>(workspace));
+                                    parts_together(parts, rows), static_cast<unsigned char*>(workspace));
 }
 
 int ws_dflash_topk(void* stream, const float* x, int n, int ld, int k, int* ids, float* vals, unsigned rows) {
@@ -804,6 +814,7 @@ int sample_batch_on(void* stream, const ws_batch* b, const BatchPlan& p, unsigne
         const uint32_t waves = p.few_parts * 8u;  // (512 threads a workgroup)
         a.few_magic = static_cast<uint32_t>(((uint64_t{1} << 32) + waves - 1u) / waves);
         a.few_chunk_log2 = chunk_log2(b->logits, b->row_stride * (b->dtype == WS_DTYPE_F32 ? 4u : 2u));
+        a.few_together = parts_together(p.few_parts, b->rows);
         a.work = work;
         a.fb_lds_tie = 0u;
         a.fb_lds_ab = p.short_fb_ab;

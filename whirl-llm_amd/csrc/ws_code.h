@@ -78,29 +78,6 @@ __device__ __forceinline__ uint32_t code_bin(float x) {
 __device__ __forceinline__ float code_group_step(uint32_t g) { return __fsub_rn(code_value(g * 8u), code_value(g * 8u + 1u)); }
 __device__ __forceinline__ double code_group_top(uint32_t g) { return static_cast<double>(code_value(g * 8u)) + static_cast<double>(code_group_step(g)); }
 
-// e^-a, of either sign: 2^k e^r with |r| <= ln 2 / 2, the series to r^13 (two units in the last place; a quarter of the library's instructions).
-// The reduction is Cody and Waite's, with ln 2 in the two parts that Sun's public fdlibm (e_exp.c) gives it.
-__device__ __forceinline__ double code_exp(double a) {
-    const double k = __builtin_rint(a * -1.44269504088896340736);
-    double r = fma(k, -6.93147180369123816490e-01, -a);
-    r = fma(k, -1.90821492927058770002e-10, r);
-    double p = 1.0 / 6227020800.0;
-    p = fma(p, r, 1.0 / 479001600.0);
-    p = fma(p, r, 1.0 / 39916800.0);
-    p = fma(p, r, 1.0 / 3628800.0);
-    p = fma(p, r, 1.0 / 362880.0);
-    p = fma(p, r, 1.0 / 40320.0);
-    p = fma(p, r, 1.0 / 5040.0);
-    p = fma(p, r, 1.0 / 720.0);
-    p = fma(p, r, 1.0 / 120.0);
-    p = fma(p, r, 1.0 / 24.0);
-    p = fma(p, r, 1.0 / 6.0);
-    p = fma(p, r, 0.5);
-    p = fma(p, r, 1.0);
-    p = fma(p, r, 1.0);
-    return __builtin_amdgcn_ldexp(p, static_cast<int>(k));
-}
-
 // each half: zero stays zero, everything else is one
 __device__ __forceinline__ CodePair code_one(uint32_t y) {
     CodePair d;  // (written out: the compiler makes two comparisons and a permutation of it)

@@ -113,30 +113,39 @@ __device__ __forceinline__ double last_lane(double v) {
     return __longlong_as_double(static_cast<long long>(r));
 }
 
-// ---- wave reductions (every lane gets the result)
-__device__ __forceinline__ float wave_max(float v) {
-    v = fmaxf(v, dpp_or_self<0x111, 0xf>(v));
-    v = fmaxf(v, dpp_or_self<0x112, 0xf>(v));
-    v = fmaxf(v, dpp_or_self<0x114, 0xf>(v));
-    v = fmaxf(v, dpp_or_self<0x118, 0xf>(v));
-    v = fmaxf(v, dpp_or_self<0x142, 0xa>(v));
-    v = fmaxf(v, dpp_or_self<0x143, 0xc>(v));
-    return last_lane(v);
+// adds to a word in LDS and returns what it was. (Written out for the one lane that does so for its wave: the compiler makes a reduction over the active lanes
+// of it first.)
+__device__ __forceinline__ uint32_t lds_add(uint32_t* word, uint32_t v) {
+    typedef __attribute__((address_space(3))) uint32_t* LdsWord;
+    uint32_t was;
+    asm volatile("ds_add_rtn_u32 %0, %1, %2\n\ts_waitcnt lgkmcnt(0)" : "=&v"(was) : "v"(static_cast<uint32_t>((uintptr_t)(LdsWord)word)), "v"(v) : "memory");
+    return was;
 }
-template <int CTRL, int ROW_MASK>
-__device__ __forceinline__ uint32_t dpp_or_self(uint32_t v) {
-    return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(static_cast<int>(v), static_cast<int>(v), CTRL, ROW_MASK, 0xf, false));
+
+// ---- wave reductions (every lane gets the result)
+// (The steps written out: of a maximum with a lane's neighbour the compiler makes five instructions, each waiting for the one before.
+// A lane without a source keeps its own value; the pauses are what a neighbour's register needs after it has been written.)
+#define WS_WAVE_FOLD(op)                                                \
+    "s_nop 1\n\t" op " %0, %0, %0 row_shr:1 row_mask:0xf bank_mask:0xf\n\t" \
+    "s_nop 1\n\t" op " %0, %0, %0 row_shr:2 row_mask:0xf bank_mask:0xf\n\t" \
+    "s_nop 1\n\t" op " %0, %0, %0 row_shr:4 row_mask:0xf bank_mask:0xf\n\t" \
+    "s_nop 1\n\t" op " %0, %0, %0 row_shr:8 row_mask:0xf bank_mask:0xf\n\t" \
+    "s_nop 1\n\t" op " %0, %0, %0 row_bcast:15 row_mask:0xa bank_mask:0xf\n\t" \
+    "s_nop 1\n\t" op " %0, %0, %0 row_bcast:31 row_mask:0xc bank_mask:0xf\n\t" \
+    "s_nop 1"
+__device__ __forceinline__ float wave_max(float v) {
+    asm volatile(WS_WAVE_FOLD("v_max_f32_dpp") : "+v"(v));
+    return last_lane(v);
 }
 __device__ __forceinline__ uint32_t wave_min_u32(uint32_t v) {
-    v = min(v, dpp_or_self<0x111, 0xf>(v));
-    v = min(v, dpp_or_self<0x112, 0xf>(v));
-    v = min(v, dpp_or_self<0x114, 0xf>(v));
-    v = min(v, dpp_or_self<0x118, 0xf>(v));
-    v = min(v, dpp_or_self<0x142, 0xa>(v));
-    v = min(v, dpp_or_self<0x143, 0xc>(v));
+    asm volatile(WS_WAVE_FOLD("v_min_u32_dpp") : "+v"(v));
     return last_lane(v);
 }
-__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) { return ~wave_min_u32(~v); }
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
+    asm volatile(WS_WAVE_FOLD("v_max_u32_dpp") : "+v"(v));
+    return last_lane(v);
+}
+#undef WS_WAVE_FOLD
 __device__ __forceinline__ float wave_sum(float v) { return last_lane(wave_incl_scan(v)); }
 __device__ __forceinline__ double wave_sum(double v) { return last_lane(wave_incl_scan(v)); }
 __device__ __forceinline__ uint32_t wave_sum(uint32_t v) { return last_lane(wave_incl_scan(v)); }

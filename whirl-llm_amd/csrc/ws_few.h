@@ -15,12 +15,16 @@
 //   * the part that arrives last - a ticket, nobody waits - reads the waves' headers and lists. With top_k at most the
 //     number of waves, the top_k-th largest of the waves' maxima bounds the row's top_k-th largest logit from below, so
 //     that about as many keys as top_k are left to sort.
+//   * a row's parts are on one chiplet where its compute units take all parts of its rows at once (few_place).
 // What bounds it is that chain: parameters, ids, their tokens' logits, the stores of the keys, headers and keys are six trips to
-// memory of about 0.7 us, between them some 2500 instructions of the slowest wave. 512 threads rather than 1024: the cost of a wave's own
+// memory, between them some 2000 instructions of the slowest wave; with 64 rows and more the instructions a token, which two waves a SIMD
+// issue one after the other. 512 threads rather than 1024: the cost of a wave's own
 // work (threshold, sums, publishing) is paid half as often, and a share still fits the registers. Measured against the
 // short-list kernel's shared rows (151936 fp32, microseconds a launch): one row, top-k 40: 20.6 -> 11.9; 64 rows of mixed
 // filters with 4096-id histories: 50 (126 when a row's min-p list ran over) -> 32.5; 32 rows of 50257, which went through
-// the three-pass kernel: 55.6 -> 15.4.
+// the three-pass kernel: 55.6 -> 15.4. Since then 11.8 -> 10.3, 30.8 -> 26.8 and 15.6 -> 14.5: a bit a token for those that lists name and a look a vector
+// for those to list (64 rows 8 %, 40 rows 12 %), the waves' maxima and thresholds by a third of the instructions, the last part's exponentials by a quarter,
+// its places in the list by one addition a wave (one row 9 %), and a row's parts on one chiplet (1 to 2 %; 6 % of a row whose parameters come over the bus).
 #pragma once
 #include "ws_short.h"
 
@@ -48,7 +52,7 @@ struct FewShared {
     long long t0;
 #endif
     ShortShared sh;
-    uint32_t dup_at[kFewDups], dup_j[kFewDups];
+    uint16_t dup_at[kFewDups], dup_j[kFewDups];  // (places of a share and entries of a bias list: below 2^16)
     float dup_v[kFewDups];
     float red_f[WS_WAVES];  // (few_collect: the row's maximum, and the lowest logit looked at)
     uint32_t w[16];
@@ -61,15 +65,14 @@ struct FewShared {
     }
 };
 
-// the largest prefix (bits 31 .. 14) of an order key that at least d lanes of the wave reach, two bits a step
+// the largest prefix (bits 31 .. 14) of an order key that at least d lanes of the wave reach: five instructions a bit (two bits a step are
+// fifteen, and no shorter a chain)
 __device__ __forceinline__ uint32_t few_lane_threshold(uint32_t k32, uint32_t d) {
     uint32_t at = 0u;
-#pragma unroll 1
-    for (int b = 30; b >= 14; b -= 2) {
-        const uint32_t c1 = at | (1u << b), c2 = at | (2u << b), c3 = at | (3u << b);
-        const uint32_t n1 = static_cast<uint32_t>(__popcll(__ballot(k32 >= c1))), n2 = static_cast<uint32_t>(__popcll(__ballot(k32 >= c2))),
-                       n3 = static_cast<uint32_t>(__popcll(__ballot(k32 >= c3)));
-        at = n3 >= d ? c3 : (n2 >= d ? c2 : (n1 >= d ? c1 : at));
+#pragma unroll
+    for (int b = 31; b >= 14; --b) {
+        const uint32_t c = at | (1u << b);
+        at = static_cast<uint32_t>(__popcll(__ballot(k32 >= c))) >= d ? c : at;
     }
     return at;
 }
@@ -77,6 +80,17 @@ __device__ __forceinline__ uint32_t lanes_before(uint64_t m) {  // set bits of m
     return __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(m >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(m), 0u));
 }
 
+// Which row a workgroup has, and which part of it; false: none. Workgroups go to the chiplets in turn, so parts whose numbers lie
+// kChiplets apart share one, and its L2: what they leave for each other need not go through memory.
+__device__ __forceinline__ bool few_place(uint32_t together, uint32_t rows, uint32_t& row, uint32_t& part) {
+    row = blockIdx.y;
+    part = blockIdx.x;
+    if (together) {
+        row = row * kChiplets + part % kChiplets;
+        part /= kChiplets;
+    }
+    return row < rows;
+}
 // What a workgroup of a shared row is given: which share of the row is its own, and how the row is dealt out. Chunk c of the
 // row (2^cl vectors) is wave c mod G's; vector k of a lane lies in its wave's chunk number k * (chunks a load) + lane / (lanes a
 // chunk).
@@ -113,11 +127,31 @@ __device__ __forceinline__ void few_exp_scale(float inv_t, float& k2, float& k2l
     k2lo = static_cast<float>(static_cast<double>(inv_t) * 1.44269504088896340736 - static_cast<double>(k2));
 }
 
-// Threshold, list and sum of every wave of this workgroup, published in the row's workspace. x: the share in registers (-inf:
-// no token), lm: this thread's largest logit, ext: n_ext more tokens {id, logit}; ok false: the share cannot be listed. SUM
+// A logit as it stands in a row, a signalling NaN made a quiet one; the largest of three such (NaN: not among them). Written out: of bits that
+// could be a signalling NaN the compiler would quiet every operand of every maximum.
+__device__ __forceinline__ float few_logit(uint32_t bits) {
+    float v;
+    asm("v_max_f32 %0, %1, %1" : "=v"(v) : "v"(bits));
+    return v;
+}
+__device__ __forceinline__ float few_max3(float a, float b, float c) {
+    float v;
+    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(v) : "v"(a), "v"(b), "v"(c));
+    return v;
+}
+template <uint32_t TPV>
+__device__ __forceinline__ float few_max_of(const float (&x)[TPV]) {
+    float v = few_max3(x[0], x[1], x[2]);
+#pragma unroll
+    for (uint32_t e = 3; e + 1u < TPV; e += 2u) v = few_max3(v, x[e], x[e + 1u]);
+    return few_max3(v, x[TPV - 1u], x[TPV - 1u]);
+}
+
+// Threshold, list and sum of every wave of this workgroup, published in the row's workspace. x: the share in registers (NaN or -inf:
+// no token), vm: the largest of each vector, lm: this thread's largest logit, ext: n_ext more tokens {id, logit}; ok false: the share cannot be listed. SUM
 // false: nobody asks for the normaliser. Returns whether this workgroup is the last of the row's: it has everything to go on.
 template <int DT, int NV, bool SUM>
-__device__ __forceinline__ bool few_publish(const FewShare& L, const FewWant& W, const float (&x)[NV][DT == 0 ? 4 : 8], float lm, const uint4* ext, uint32_t n_ext,
+__device__ __forceinline__ bool few_publish(const FewShare& L, const FewWant& W, const float (&x)[NV][DT == 0 ? 4 : 8], const float (&vm)[NV], float lm, const uint4* ext, uint32_t n_ext,
                                             bool ok, unsigned char* work, FewShared& F) {
     constexpr uint32_t TPV = DT == 0 ? 4u : 8u;
     const uint32_t t = threadIdx.x, lane = t & 63u;
@@ -179,11 +213,14 @@ __device__ __forceinline__ bool few_publish(const FewShare& L, const FewWant& W,
         }
     };
     if (ok && wm < INFINITY) {
+        // (a look a vector, and at its tokens only where one of them is listed)
 #pragma unroll
         for (uint32_t k = 0; k < NV; ++k)
+            if (k < L.n_vec && __ballot(vm[k] >= thr_list)) {  // uniform
+                const uint32_t id0 = L.vec_of(k) * TPV;
 #pragma unroll
-            for (uint32_t e = 0; e < TPV; ++e)
-                if (k < L.n_vec) push(x[k][e], L.vec_of(k) * TPV + e);
+                for (uint32_t e = 0; e < TPV; ++e) push(x[k][e], id0 + e);
+            }
         for (uint32_t i0 = 0; i0 < n_ext; i0 += WS_BLOCK) {  // uniform
             uint2 en = make_uint2(0u, 0xff800000u);
             if (i0 + t < n_ext) en = *reinterpret_cast<const uint2*>(&ext[i0 + t]);
@@ -193,9 +230,11 @@ __device__ __forceinline__ bool few_publish(const FewShare& L, const FewWant& W,
         if (SUM)
 #pragma unroll
             for (uint32_t k = 0; k < NV; ++k)
+                if (k < L.n_vec) {  // uniform
+                    asm volatile("");  // (a branch: else the vectors a share does not have are summed and dropped)
 #pragma unroll
-                for (uint32_t e = 0; e < TPV; ++e)
-                    if (k < L.n_vec) add(x[k][e]);
+                    for (uint32_t e = 0; e < TPV; ++e) add(x[k][e]);
+                }
     }
     {
         const double z = wm > -INFINITY && wm < INFINITY ? wave_sum(static_cast<double>(s)) : 0.0;
@@ -233,10 +272,24 @@ __device__ __forceinline__ uint32_t few_collect(const FewShare& L, const FewWant
     uint32_t* gcount = reinterpret_cast<uint32_t*>(work + kFewCount);
     uint32_t* ctrl = reinterpret_cast<uint32_t*>(work + kFewCtrl);
     const uint32_t G = L.G, slots = kFewKeys / G;
-    // everybody's keys asked for (those of the first slots right away), then the headers. Five waves read them side by side, each
+    // Headers and everybody's keys asked for (those of the first slots right away). Five waves read the headers side by side, each
     // for what it works out: the threshold, the normaliser (two of them: the exponentials are the longest chain here, and one a
     // lane is 0.1 us shorter than two), how many slots hold keys; and one the uniform.
     constexpr uint32_t kBlind = 4096u / WS_BLOCK, kHL = kFewWaves / 64u;
+    static_assert(kHL == 2u, "a wave of this part for every 64 of the row");
+    const uint32_t w0 = min(lane, G - 1u), w1 = min(64u + lane, G - 1u);
+    const bool on0 = lane < G, on1 = 64u + lane < G;
+    uint64_t h0 = 0ull, h1 = 0ull, zs = 0ull;
+    uint32_t n0 = 0u, n1 = 0u;
+    if (wv < 5u) {
+        h0 = __hip_atomic_load(&ghead[w0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        h1 = __hip_atomic_load(&ghead[w1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (SUM && (wv == 1u || wv == 4u)) zs = __hip_atomic_load(&ghead[kFewWaves + (wv == 4u ? w1 : w0)], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (wv == 2u) {
+            n0 = __hip_atomic_load(&gcount[w0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            n1 = __hip_atomic_load(&gcount[w1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
     uint64_t got[kBlind];
 #pragma unroll
     for (uint32_t i = 0; i < kBlind; ++i) got[i] = __hip_atomic_load(&gkeys[i * WS_BLOCK + t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -244,47 +297,22 @@ __device__ __forceinline__ uint32_t few_collect(const FewShare& L, const FewWant
     if (wv == 3u) {
         fourth();
     } else if (wv < 5u) {
-        const bool sums = wv == 1u || wv == 4u;
-        const uint32_t half = wv == 4u ? 1u : 0u;  // of the waves: the first 64, or the others
-        static_assert(kHL == 2u, "a wave of this part for every 64 of the row");
-        uint64_t h0[kHL], zs = 0ull;
-        uint32_t ns[kHL];
-#pragma unroll
-        for (uint32_t i = 0; i < kHL; ++i) {
-            const uint32_t w = min(i * 64u + lane, G - 1u);
-            h0[i] = __hip_atomic_load(&ghead[w], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (SUM && sums && i == half) zs = __hip_atomic_load(&ghead[kFewWaves + w], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (wv == 2u) ns[i] = __hip_atomic_load(&gcount[w], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-        float m4[kHL], mx = -INFINITY;
-#pragma unroll
-        for (uint32_t i = 0; i < kHL; ++i) {
-            m4[i] = i * 64u + lane < G ? unkey32(static_cast<uint32_t>(h0[i] >> 32)) : -INFINITY;
-            mx = fmaxf(mx, m4[i]);
-        }
-        mx = wave_max(mx);
+        const float m0 = on0 ? unkey32(static_cast<uint32_t>(h0 >> 32)) : -INFINITY, m1 = on1 ? unkey32(static_cast<uint32_t>(h1 >> 32)) : -INFINITY;
+        const float mx = wave_max(fmaxf(m0, m1));
         if (wv == 0u) {
-            float tx = -INFINITY;
-#pragma unroll
-            for (uint32_t i = 0; i < kHL; ++i) tx = fmaxf(tx, unkey32(static_cast<uint32_t>(h0[i])));
-            tx = wave_max(tx);
             // the keys that are looked at: from the largest of the waves' thresholds up (every wave has listed what it has
             // there), or - higher - from the top_k-th largest of the waves' maxima
-            float floor_v = tx;
+            float floor_v = wave_max(fmaxf(unkey32(static_cast<uint32_t>(h0)), unkey32(static_cast<uint32_t>(h1))));
             if (W.by_k && W.top_k <= G) {
-                float lo = tx, hi = mx;
-                auto reach = [&](float v) {
-                    uint32_t n = 0;
-#pragma unroll
-                    for (uint32_t i = 0; i < kHL; ++i) n += static_cast<uint32_t>(__popcll(__ballot(m4[i] >= v)));
-                    return n;
-                };
+                float lo = floor_v, hi = mx;
+                auto reach = [&](float v) { return static_cast<uint32_t>(__popcll(__ballot(m0 >= v)) + __popcll(__ballot(m1 >= v))); };
                 if (lo > -INFINITY && reach(lo) >= W.top_k)
-                    for (int i = 0; i < 5; ++i) {  // two halvings a step
-                        const float m2 = 0.5f * lo + 0.5f * hi, m1 = 0.5f * lo + 0.5f * m2, m3 = 0.5f * m2 + 0.5f * hi;
-                        const uint32_t n1 = reach(m1), n2 = reach(m2), n3 = reach(m3);
-                        hi = n1 < W.top_k ? m1 : (n2 < W.top_k ? m2 : (n3 < W.top_k ? m3 : hi));
-                        lo = n3 >= W.top_k ? m3 : (n2 >= W.top_k ? m2 : (n1 >= W.top_k ? m1 : lo));
+#pragma unroll
+                    for (int i = 0; i < 9; ++i) {
+                        const float mid = 0.5f * lo + 0.5f * hi;
+                        const bool enough = reach(mid) >= W.top_k;
+                        lo = enough ? mid : lo;
+                        hi = enough ? hi : mid;
                     }
                 floor_v = lo;
             }
@@ -293,53 +321,58 @@ __device__ __forceinline__ uint32_t few_collect(const FewShare& L, const FewWant
                 F.red_f[0] = mx;
                 F.red_f[1] = floor_v;
             }
-        } else if (sums) {
-            double z = 0.0;
-            if (SUM) {  // (the factors in 64 bits, as the rules work out the candidates' masses)
-                const float own = half ? m4[1] : m4[0];
-                if (own > -INFINITY) z = __longlong_as_double(static_cast<long long>(zs)) * exp(static_cast<double>(__fsub_rn(own, mx)) * static_cast<double>(W.inv_t));
-                z = wave_sum(z);
-            }
-            if (lane == 0u) F.z[half] = z;
-        } else {
-            uint32_t most = 0;
-            bool bad = !(mx > -INFINITY);
-#pragma unroll
-            for (uint32_t i = 0; i < kHL; ++i)
-                if (i * 64u + lane < G) {
-                    bad = bad || ns[i] == kFewBad;
-                    most = max(most, ns[i]);
-                }
-            most = wave_max_u32(most);
-            bad = __ballot(bad) != 0ull;
+        } else if (wv == 2u) {
+            const bool bad = __ballot((on0 && n0 == kFewBad) || (on1 && n1 == kFewBad)) != 0ull || !(mx > -INFINITY);
+            const uint32_t most = wave_max_u32(max(on0 ? n0 : 0u, on1 ? n1 : 0u));
             if (lane == 0u) {
                 F.w[3] = bad ? slots : most;  // (a wave that could not list its share may have left keys in every slot)
                 F.w[4] = bad ? 1u : 0u;
             }
+        } else {
+            double z = 0.0;
+            if (SUM) {  // (the factors in 64 bits, as the rules work out the candidates' masses)
+                const float own = wv == 4u ? m1 : m0;
+                if (own > -INFINITY) z = __longlong_as_double(static_cast<long long>(zs)) * exp_down(static_cast<double>(__fsub_rn(mx, own)) * static_cast<double>(W.inv_t));
+                z = wave_sum(z);
+            }
+            if (lane == 0u) F.z[wv == 4u ? 1u : 0u] = z;
         }
     }
     __syncthreads();
     WSF_MARK(6);
-    const uint32_t floor_key = key32(F.red_f[1]);
+    const uint32_t floor_key = max(key32(F.red_f[1]), 1u);  // (no key: zeros)
     const uint32_t n_read = F.w[3] * G;
     const bool bad = F.w[4] != 0u;
-    auto keep = [&](uint64_t key, uint32_t at) {
-        if (key != 0ull) __hip_atomic_store(&gkeys[at], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // the workspace as the next launch needs it
-        const bool yes = static_cast<uint32_t>(key >> 32) >= floor_key && key != 0ull;
-        const uint64_t mk = __ballot(yes);
-        if (mk) {  // uniform
-            uint32_t at0 = 0;
-            if (lane == 0u) at0 = atomicAdd(&F.w[5], static_cast<uint32_t>(__popcll(mk)));
-            const uint32_t slot = lane_value(at0, 0u) + lanes_before(mk);
-            if (yes && slot < kShortCap) list[slot] = key;
-        }
-    };
+    // (a wave's places in the list by one addition for all the slots it has read)
+    auto keep = [&](const uint64_t (&key)[kBlind], uint32_t i0) __attribute__((always_inline)) {
+        uint32_t mine = 0;
 #pragma unroll
-    for (uint32_t i = 0; i < kBlind; ++i)
-        if (i * WS_BLOCK < n_read) keep(got[i], i * WS_BLOCK + t);  // uniform
-    for (uint32_t i0 = kBlind * WS_BLOCK; i0 < n_read; i0 += WS_BLOCK) {
-        const uint32_t at = i0 + t;
-        keep(at < n_read ? __hip_atomic_load(&gkeys[at], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0ull, at);
+        for (uint32_t i = 0; i < kBlind; ++i) mine += i0 + i * WS_BLOCK < n_read && static_cast<uint32_t>(key[i] >> 32) >= floor_key ? 1u : 0u;
+        const uint32_t inc = wave_incl_scan(mine), all = lane_value(inc, 63u);
+        if (all) {  // uniform
+            uint32_t slot = 0;
+            if (lane == 0u) slot = lds_add(&F.w[5], all);
+            slot = lane_value(slot, 0u) + inc - mine;
+#pragma unroll
+            for (uint32_t i = 0; i < kBlind; ++i)
+                if (i0 + i * WS_BLOCK < n_read && static_cast<uint32_t>(key[i] >> 32) >= floor_key) {
+                    if (slot < kShortCap) list[slot] = key[i];
+                    ++slot;
+                }
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < kBlind; ++i)  // the workspace as the next launch needs it
+            if (i0 + i * WS_BLOCK < n_read && key[i] != 0ull) __hip_atomic_store(&gkeys[i0 + i * WS_BLOCK + t], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    keep(got, 0u);
+    for (uint32_t i0 = kBlind * WS_BLOCK; i0 < n_read; i0 += kBlind * WS_BLOCK) {  // uniform
+        uint64_t more[kBlind];
+#pragma unroll
+        for (uint32_t i = 0; i < kBlind; ++i) {
+            const uint32_t at = i0 + i * WS_BLOCK + t;
+            more[i] = at < n_read ? __hip_atomic_load(&gkeys[at], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0ull;
+        }
+        keep(more, i0);
     }
     if (t < G) {
         __hip_atomic_store(&ghead[t], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -414,10 +447,17 @@ __device__ __forceinline__ bool few_row(const BatchArgs& A, const uint32_t row, 
         na[k] = MASKED ? allow[min(j * TPV, V - 1u) >> 5] : 0xffffffffu;
     }
     uint32_t* cnt = reinterpret_cast<uint32_t*>(lds + 32768);  // two 16-bit counts a word; bit 15 of a count: somebody takes the token
+    // and a bit for each of a thread's tokens that a list names: [word][thread]. (The counts alone took a thread two LDS words and ten
+    // instructions a vector to find out that none of its four is named.)
+    constexpr uint32_t kBits = few_bit_words(NV * TPV);
+    uint32_t* named = cnt + NV * TPV * WS_BLOCK / 2u;
     const bool lists = A.hist || A.bias_ids;
-    if (lists)
+    if (lists) {
 #pragma unroll
         for (uint32_t k = 0; k < NV * TPV / 8u + (NV * TPV % 8u ? 1u : 0u); ++k) reinterpret_cast<uint4*>(cnt)[k * WS_BLOCK + t] = make_uint4(0u, 0u, 0u, 0u);
+#pragma unroll
+        for (uint32_t w = 0; w < kBits; ++w) named[w * WS_BLOCK + t] = 0u;
+    }
 
     // ---- the row's parameters
     const LeanRowParams P = load_row_params(A, row);
@@ -441,6 +481,10 @@ __device__ __forceinline__ bool few_row(const BatchArgs& A, const uint32_t row, 
         const uint32_t cq = static_cast<uint32_t>((static_cast<uint64_t>(c) * A.few_magic) >> 32), cg = c - cq * G;  // c / G, c mod G
         const uint32_t at = (((cg % WS_WAVES) * (NV * 64u) + (cq << cl) + (v & ((1u << cl) - 1u))) * TPV) + id % TPV;
         return id < V && cg / WS_WAVES == part ? at : 0xffffffffu;
+    };
+    auto name = [&](uint32_t li) {  // its bit: a wave's places are [vector][lane][token]
+        const uint32_t w = li / (NV * 64u * TPV), r = li % (NV * 64u * TPV), b = r / (64u * TPV) * TPV + li % TPV;
+        atomicOr(&named[(b >> 5) * WS_BLOCK + w * 64u + r / TPV % 64u], 1u << (b & 31u));
     };
     if (any_ext) {
         const int32_t* hist_ids = A.hist + P.h0;
@@ -480,14 +524,15 @@ __device__ __forceinline__ bool few_row(const BatchArgs& A, const uint32_t row, 
                         atomicOr(&cnt[li[r] >> 1], kFewDup << sh);
                         const uint32_t at = atomicAdd(&F.w[0], 1u);
                         if (at < kFewDups) {
-                            F.dup_at[at] = li[r];
-                            F.dup_j[at] = j0 + r * WS_BLOCK + t;
+                            F.dup_at[at] = static_cast<uint16_t>(li[r]);
+                            F.dup_j[at] = static_cast<uint16_t>(j0 + r * WS_BLOCK + t);
                             F.dup_v[at] = bv[r];
                         }
                     } else {
                         takes = true;
                     }
                 }
+                if (takes) name(li[r]);
                 const uint64_t mk = __ballot(takes);
                 if (mk) {  // uniform
                     uint32_t at0 = 0;
@@ -505,42 +550,36 @@ __device__ __forceinline__ bool few_row(const BatchArgs& A, const uint32_t row, 
     __syncthreads();
     WSS_MARK(1);  // history and bias entries counted
 
-    // ---- the share: tokens that do not count - masked out, NaN, past the row, touched - become -inf
-    float x[NV][TPV];
+    // ---- the share: tokens that do not count - masked out, past the row, named by a list - become NaN
+    uint32_t out[kBits];
+#pragma unroll
+    for (uint32_t w = 0; w < kBits; ++w) out[w] = any_ext ? named[w * WS_BLOCK + t] : 0u;
+    if (MASKED)
+#pragma unroll
+        for (uint32_t k = 0; k < NV; ++k) out[k * TPV / 32u] |= (~(na[k] >> ((L.vec_of(k) * TPV) & 31u)) & ((1u << TPV) - 1u)) << (k * TPV % 32u);
+    float x[NV][TPV], vm[NV];
     float lm = -INFINITY;
 #pragma unroll
     for (uint32_t k = 0; k < NV; ++k) {
         if (k >= n_vec) {  // uniform
 #pragma unroll
             for (uint32_t e = 0; e < TPV; ++e) x[k][e] = -INFINITY;
+            vm[k] = -INFINITY;
             continue;
         }
-        const uint32_t j = L.vec_of(k);
-        uint4 qq = q[k];
-        if (j_part != 0xffffffffu && j == j_part) qq = part_vector<DT>(qq, TPV - V % TPV);
-        const uint32_t w[4] = {qq.x, qq.y, qq.z, qq.w};
-        uint32_t invalid = j < nv ? 0u : ~0u;  // bit e: token e does not count
-        if (MASKED) invalid |= ~(na[k] >> ((j * TPV) & 31u));
-        uint32_t c2[TPV / 2u];
-#pragma unroll
-        for (uint32_t e = 0; e < TPV / 2u; ++e) c2[e] = 0u;
-        if (any_ext) {  // uniform
-            const uint32_t at = (wv * (NV * 64u) + k * 64u + lane) * (TPV / 2u);
-#pragma unroll
-            for (uint32_t e = 0; e < TPV / 2u; e += 2u) {
-                const uint2 two = *reinterpret_cast<const uint2*>(&cnt[at + e]);
-                c2[e] = two.x;
-                c2[e + 1u] = two.y;
-            }
+        if (k + 1u == n_vec) {  // uniform: the round the row ends in
+            const uint32_t j = L.vec_of(k);
+            if (j == j_part) q[k] = part_vector<DT>(q[k], TPV - V % TPV);
+            if (j >= nv) q[k] = make_uint4(0xffffffffu, 0xffffffffu, 0xffffffffu, 0xffffffffu);
         }
+        const uint32_t w[4] = {q[k].x, q[k].y, q[k].z, q[k].w};
 #pragma unroll
         for (uint32_t e = 0; e < TPV; ++e) {
             const uint32_t bits = DT == 0 ? w[e] : ((e & 1u) ? (w[e >> 1] & 0xffff0000u) : (w[e >> 1] << 16));
-            const uint32_t c = (e & 1u) ? c2[e >> 1] & 0xffff0000u : c2[e >> 1] & 0xffffu;
-            const bool out = ((invalid >> e) & 1u) || c;
-            x[k][e] = out ? -INFINITY : fmaxf(__uint_as_float(bits), -INFINITY);
-            lm = fmaxf(lm, x[k][e]);
+            x[k][e] = few_logit(bits | static_cast<uint32_t>(static_cast<int32_t>(out[k * TPV / 32u] << (31u - (k * TPV + e) % 32u)) >> 31));
         }
+        vm[k] = few_max_of<TPV>(x[k]);
+        lm = fmaxf(lm, vm[k]);
     }
     WSS_MARK(2);  // share in registers
 
@@ -592,7 +631,7 @@ __device__ __forceinline__ bool few_row(const BatchArgs& A, const uint32_t row, 
     W.top_k = top_k;
     W.inv_t = inv_t;
     W.min_p = min_p;
-    if (!few_publish<DT, NV, true>(L, W, x, lm, ext, n_ext, !not_mine && n_ext_all <= kFewExt, work, F)) return true;  // not the last: done
+    if (!few_publish<DT, NV, true>(L, W, x, vm, lm, ext, n_ext, !not_mine && n_ext_all <= kFewExt, work, F)) return true;  // not the last: done
     finisher = true;
     WSS_MARK(6);  // ticket
     uint64_t* list = reinterpret_cast<uint64_t*>(lds);
@@ -631,7 +670,8 @@ __device__ __forceinline__ bool few_row(const BatchArgs& A, const uint32_t row, 
 template <int DT, bool MASKED, int NV>
 __global__ void __launch_bounds__(WS_BLOCK) few_batch_kernel(BatchArgs A) {
     __shared__ FewShared shared;
-    const uint32_t row = blockIdx.y, part = blockIdx.x;
+    uint32_t row, part;
+    if (!few_place(A.few_together, A.rows, row, part)) return;
     bool finisher;
     if (!few_row<DT, MASKED, NV>(A, row, part, shared, finisher) && finisher) {
         __syncthreads();

@@ -31,7 +31,7 @@ int launch_few(hipStream_t stream, const BatchArgs& a, unsigned lds_bytes, unsig
     const uint32_t each = (vectors + load - 1u) / load;
     int size = 0;
     while (size < 3 && each > kFewVectors[a.dtype][size]) ++size;
-    hipLaunchKernelGGL(kFewKernels[a.dtype][a.allow ? 1 : 0][size], dim3(a.few_parts, a.rows), dim3(WS_BLOCK), lds_bytes, stream, a);
+    hipLaunchKernelGGL(kFewKernels[a.dtype][a.allow ? 1 : 0][size], few_grid(a.few_parts, a.rows, a.few_together), dim3(WS_BLOCK), lds_bytes, stream, a);
     return static_cast<int>(hipGetLastError());
 }
 

@@ -193,7 +193,7 @@ __device__ __forceinline__ void short_rules(uint64_t* list, const uint32_t row, 
         for (uint32_t j = 0; j < KC; ++j) {
             const uint32_t pos = KC * t + j;
             wkey[j] = pos < n_cand ? list[pos] : 0ull;
-            e[j] = pos < n_cand ? exp(static_cast<double>(__fsub_rn(unkey32(static_cast<uint32_t>(wkey[j] >> 32)), m)) * static_cast<double>(inv_t)) : 0.0;
+            e[j] = pos < n_cand ? exp_down(static_cast<double>(__fsub_rn(m, unkey32(static_cast<uint32_t>(wkey[j] >> 32)))) * static_cast<double>(inv_t)) : 0.0;
             tot += e[j];
         }
         double Zk1;
@@ -284,7 +284,7 @@ __device__ __forceinline__ void short_rules(uint64_t* list, const uint32_t row, 
     if (n_cand <= 64u) {
         // the usual case, a top-k of a few dozen: one wave, a candidate a lane, no barrier and no atomic
         if (wv == 0u) {
-            const double e = has ? exp(static_cast<double>(__fsub_rn(x, m)) * static_cast<double>(inv_t)) : 0.0;
+            const double e = has ? exp_down(static_cast<double>(__fsub_rn(m, x)) * static_cast<double>(inv_t)) : 0.0;
             const double cin = wave_incl_scan(e);
             const double up = __shfl_up(cin, 1);
             const double cex = lane ? up : 0.0;
@@ -323,11 +323,10 @@ __device__ __forceinline__ void short_rules(uint64_t* list, const uint32_t row, 
                 const double se = wave_sum(kept && e > 0.0 ? e * log_mass(x) : 0.0), sq = wave_sum(kept && id == query ? e : 0.0);
                 if (lane == 0u) write_more(se, sq, Zk);
             }
-            if (lane == 0u) S.s_w[7] = n3;
         }
     } else if (n_cand <= WS_BLOCK) {
         double e = 0.0;
-        if (wv * 64u < n_cand) e = has ? exp(static_cast<double>(__fsub_rn(x, m)) * static_cast<double>(inv_t)) : 0.0;  // (per wave: the exponential is a hundred instructions)
+        if (wv * 64u < n_cand) e = has ? exp_down(static_cast<double>(__fsub_rn(m, x)) * static_cast<double>(inv_t)) : 0.0;  // (per wave)
         double Zk1;
         const double cex = block_excl_scan(e, S.red_d, &Zk1);  // mass ranked before this candidate; Zk1: of all top_k
         const double cin = cex + e;
@@ -389,10 +388,19 @@ __device__ __forceinline__ void short_rules(uint64_t* list, const uint32_t row, 
     } else {
         several(std::integral_constant<uint32_t, kShortCap / WS_BLOCK>{});
     }
-    // ---- the kept set in ascending id order (the first kept_cap of it): the same sort on (inverted id, logit) pairs
-    if (Ap->kept_ids) {
+    // ---- the kept set in ascending id order (the first kept_cap of it): of up to 64 by the wave that has them, else the same sort on (inverted
+    // id, logit) pairs
+    if (Ap->kept_ids && n_cand <= 64u) {
+        if (wv == 0u) {
+            uint32_t place = 0;
+            for (uint32_t j = 0; j < n3; ++j) place += lane_value(id, j) < id ? 1u : 0u;  // uniform
+            if (lane < n3 && place < Ap->kept_cap) {
+                Ap->kept_ids[static_cast<size_t>(row) * Ap->kept_cap + place] = static_cast<int32_t>(id);
+                if (Ap->kept_logits) Ap->kept_logits[static_cast<size_t>(row) * Ap->kept_cap + place] = x;
+            }
+        }
+    } else if (Ap->kept_ids) {
         __syncthreads();
-        if (n_cand <= 64u) n3 = S.s_w[7];
         if (n_cand > WS_BLOCK) {
             for (uint32_t k = t; k < n3; k += WS_BLOCK) {
                 const uint64_t key_ = list[k];

@@ -3,7 +3,9 @@
 // keys as are asked for. No counterpart in the reference, whose kernels give a row to one workgroup. What bounds it is the
 // chain of dependent steps (see ws_few.h). Against shared rows whose parts fitted a histogram to the head of the row and
 // whose last part counted the merged list once more (151936 fp32, microseconds a launch): 8 rows, K = 256: 19.6 -> 13.3;
-// a draft draw of 8 rows: 26.0 -> 11.6, of which the draw's one wave took 7 and takes 2.5.
+// a draft draw of 8 rows: 26.0 -> 11.6, of which the draw's one wave took 7 and takes 2.5. Since then 13.3 -> 11.8 (top_select, and what ws_few.h names), and of
+// the draw's one wave 6.5 K clocks -> 4.4 K: its parameters are asked for at the start, its sums end with the candidates, and the logarithms of the race
+// keys are another wave's. (A cycle of 8 sequences and 4 drafts, with its verification: 81.1 us -> 68.3.)
 #pragma once
 #include "ws_draft.h"
 #include "ws_few.h"
@@ -11,36 +13,41 @@
 namespace ws {
 
 struct TopSplit {
-    uint32_t parts, chunk_log2;
+    uint32_t parts, chunk_log2, rows, together;  // (together: few_place)
     unsigned char* work;  // kFewRowBytes a row
 };
 
 // The K largest logits of this row, by the part of it that arrives last: `list` in descending order (value desc, id asc), F.sum()
-// the normaliser. Returns 0: another part's business; 1: listed; 2: this part has to do the row without the list.
-template <int NV, bool SUM>
-__device__ __forceinline__ int top_share(const float* x, int n, int K, float inv_t, const TopSplit& sp, uint32_t row, FewShared& F, uint64_t*& list) {
+// the normaliser. K_of() says how many, once the share is on its way (0: the row is not looked at). Returns 0: another part's business; 1: listed;
+// 2: this part has to do the row without the list; and with ORDER false 3: more keys are listed than are sorted by comparing all, n_keys of them, in no order.
+template <int NV, bool SUM, bool ORDER, class KOF>
+__device__ __forceinline__ int top_share(const float* x, int n, KOF&& K_of, float inv_t, const TopSplit& sp, uint32_t row, uint32_t part, FewShared& F, uint64_t*& list, uint32_t& n_keys) {
     extern __shared__ __align__(16) unsigned char lds[];
     const uint32_t V = static_cast<uint32_t>(n);
 #ifdef WS_SHORT_TIMERS
     if (threadIdx.x == 0) F.t0 = clock64();
 #endif
-    const FewShare L = FewShare::of<0>(V, sp.parts, blockIdx.x, sp.chunk_log2);
+    const FewShare L = FewShare::of<0>(V, sp.parts, part, sp.chunk_log2);
     const uint32_t j_part = V % 4u ? L.nv - 1u : 0xffffffffu;
     const unsigned char* base = reinterpret_cast<const unsigned char*>(x);
     uint4 q[NV];
 #pragma unroll
     for (uint32_t k = 0; k < NV; ++k) q[k] = row_vector<0>(base, L.vec_of(k), V);
-    float v[NV][4], lm = -INFINITY;
+    const int K = K_of();
+    if (K == 0) return 0;  // (every part of the row sees the same words)
+    float v[NV][4], vm[NV], lm = -INFINITY;
 #pragma unroll
     for (uint32_t k = 0; k < NV; ++k) {
-        const uint32_t j = L.vec_of(k);
-        if (j_part != 0xffffffffu && j == j_part) q[k] = part_vector<0>(q[k], 4u - V % 4u);
+        if (k + 1u >= L.n_vec) {  // uniform: the round the row ends in, and those behind it
+            const uint32_t j = L.vec_of(k);
+            if (j == j_part) q[k] = part_vector<0>(q[k], 4u - V % 4u);
+            if (j >= L.nv) q[k] = make_uint4(0xffffffffu, 0xffffffffu, 0xffffffffu, 0xffffffffu);
+        }
         const uint32_t w[4] = {q[k].x, q[k].y, q[k].z, q[k].w};
 #pragma unroll
-        for (uint32_t e = 0; e < 4u; ++e) {
-            v[k][e] = j < L.nv ? fmaxf(__uint_as_float(w[e]), -INFINITY) : -INFINITY;
-            lm = fmaxf(lm, v[k][e]);
-        }
+        for (uint32_t e = 0; e < 4u; ++e) v[k][e] = few_logit(w[e]);
+        vm[k] = few_max_of<4u>(v[k]);
+        lm = fmaxf(lm, vm[k]);
     }
     FewWant W;
     W.by_k = true;
@@ -49,10 +56,11 @@ __device__ __forceinline__ int top_share(const float* x, int n, int K, float inv
     W.inv_t = inv_t;
     W.min_p = 0.0;
     unsigned char* work = sp.work + static_cast<size_t>(row) * kFewRowBytes;
-    if (!few_publish<0, NV, SUM>(L, W, v, lm, nullptr, 0u, !SUM || inv_t > 0.f, work, F)) return 0;
+    if (!few_publish<0, NV, SUM>(L, W, v, vm, lm, nullptr, 0u, !SUM || inv_t > 0.f, work, F)) return 0;
     list = reinterpret_cast<uint64_t*>(lds);
-    const uint32_t n_keys = few_collect<SUM>(L, W, work, F, list, []() {});
+    n_keys = few_collect<SUM>(L, W, work, F, list, []() {});
     if (n_keys < W.top_k || n_keys > kShortCap) return 2;
+    if (!ORDER && n_keys > WS_BLOCK / 4u) return 3;
     list = few_sort(list, n_keys, F);
 #ifdef WS_SHORT_TIMERS
     if (threadIdx.x == 0) reinterpret_cast<long long*>(work + 64512)[10] = n_keys;
@@ -61,15 +69,104 @@ __device__ __forceinline__ int top_share(const float* x, int n, int K, float inv
     return 1;
 }
 
+// The ids of the K largest of the n listed keys (n > K, n <= kShortCap), in no order, to `ids`: the buckets of short_sort, of which only the one that the
+// K-th falls in has to be put in order. (8 rows of 151936, K = 256, some 700 keys: the whole list sorted took 7.5 K clocks.)
+__device__ __forceinline__ void top_select(uint64_t* list, uint32_t n, uint32_t K, uint32_t* ids, FewShared& F) {
+    constexpr uint32_t KPT = kShortCap / WS_BLOCK, NBK = 512u;
+    static_assert(NBK == WS_BLOCK, "a bucket a thread");
+    const uint32_t t = threadIdx.x, lane = t & 63u;
+    const uint32_t wv = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(t >> 6)));
+    uint32_t* bc = reinterpret_cast<uint32_t*>(list + kShortCap);  // (behind the list: its sorted copy's place)
+    uint32_t* bs = bc + NBK;
+    const float m = F.red_f[0];
+    uint64_t key[KPT];
+    uint32_t bk[KPT], pos[KPT];
+    float dmax = 0.f, dsum = 0.f;
+    auto down = [&](uint64_t k) { return fminf(__fsub_rn(m, unkey32(static_cast<uint32_t>(k >> 32))), 3e38f); };
+#pragma unroll
+    for (uint32_t k = 0; k < KPT; ++k)
+        if (k * WS_BLOCK < n) {  // uniform
+            key[k] = k * WS_BLOCK + t < n ? list[k * WS_BLOCK + t] : 0ull;
+            const float d = key[k] ? down(key[k]) : 0.f;
+            dmax = fmaxf(dmax, d);
+            dsum += d;
+        }
+    dmax = wave_max(dmax);
+    dsum = wave_sum(dsum);
+    if (lane == 0u) {
+        F.sh.red_f[wv] = dmax;
+        F.sh.red_d[wv] = static_cast<double>(dsum);
+    }
+    bc[t] = 0u;
+    __syncthreads();
+    dmax = F.sh.red_f[0];
+    double total = F.sh.red_d[0];
+#pragma unroll
+    for (uint32_t w = 1; w < WS_WAVES; ++w) {
+        dmax = fmaxf(dmax, F.sh.red_f[w]);
+        total += F.sh.red_d[w];
+    }
+    // (short_sort's logarithmic scale)
+    const float mean = fmaxf(dmax - static_cast<float>(total) / static_cast<float>(n), dmax * 1e-6f + 1e-30f), per = 1.f / mean;
+    auto level = [&](float d) { return static_cast<float>(__float_as_uint(__fadd_rn(1.f, __fmul_rn(fmaxf(__fsub_rn(dmax, d), 0.f), per))) - 0x3f800000u); };
+    const float scale = static_cast<float>(NBK) / (level(0.f) + 1.f);
+#pragma unroll
+    for (uint32_t k = 0; k < KPT; ++k)
+        if (k * WS_BLOCK + t < n) {
+            bk[k] = NBK - 1u - min(NBK - 1u, static_cast<uint32_t>(level(down(key[k])) * scale));
+            pos[k] = atomicAdd(&bc[bk[k]], 1u);
+        }
+    __syncthreads();
+    if (wv == 0u) {  // eight consecutive counts a lane
+        const uint4 a = *reinterpret_cast<const uint4*>(&bc[lane * 8u]), b = *reinterpret_cast<const uint4*>(&bc[lane * 8u + 4u]);
+        const uint32_t c[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+        uint32_t own = 0u;
+#pragma unroll
+        for (uint32_t i = 0; i < 8u; ++i) own += c[i];
+        uint32_t run = wave_incl_scan(own) - own;
+#pragma unroll
+        for (uint32_t i = 0; i < 8u; ++i) {
+            bs[lane * 8u + i] = run;
+            if (run < K && run + c[i] >= K) F.w[6] = lane * 8u + i;  // the K-th falls in this one
+            run += c[i];
+        }
+    }
+    __syncthreads();
+    const uint32_t last = F.w[6], b0 = bs[last], c0 = bc[last];
+#pragma unroll
+    for (uint32_t k = 0; k < KPT; ++k)
+        if (k * WS_BLOCK + t < n) {
+            if (bk[k] < last) ids[bs[bk[k]] + pos[k]] = 0xffffffffu - static_cast<uint32_t>(key[k]);
+            else if (bk[k] == last) list[pos[k]] = key[k];  // (every key is in a register)
+        }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t k = 0; k < KPT; ++k)
+        if (k * WS_BLOCK + t < n && bk[k] == last) {
+            uint32_t place = b0;
+            for (uint32_t i = 0; i < c0; i += 4u) {  // four reads on their way together
+                uint64_t o[4];
+#pragma unroll
+                for (uint32_t q = 0; q < 4u; ++q) o[q] = list[min(i + q, c0 - 1u)];
+#pragma unroll
+                for (uint32_t q = 0; q < 4u; ++q) place += (i + q < c0 && o[q] > key[k]) ? 1u : 0u;
+            }
+            if (place < K) ids[place] = 0xffffffffu - static_cast<uint32_t>(key[k]);
+        }
+}
+
 template <int NV>
 __global__ void __launch_bounds__(WS_BLOCK) topk_rows_shared(const float* x, int n, int K, float inv_t, int* ids, float* vals, float* stats, TopSplit sp) {
     __shared__ FewShared F;
-    const size_t row = blockIdx.y;
+    uint32_t row_, part;
+    if (!few_place(sp.together, sp.rows, row_, part)) return;
+    const size_t row = row_;
     x += row * n;
     ids += row * K;
     vals += row * K;
     uint64_t* list;
-    const int how = top_share<NV, true>(x, n, K, inv_t, sp, static_cast<uint32_t>(row), F, list);
+    uint32_t n_keys;
+    const int how = top_share<NV, true, false>(x, n, [&]() { return K; }, inv_t, sp, row_, part, F, list, n_keys);
     if (how == 0) return;
     if (how == 2) {
         __syncthreads();
@@ -79,7 +176,11 @@ __global__ void __launch_bounds__(WS_BLOCK) topk_rows_shared(const float* x, int
     // ascending id: every kept entry counts the kept ids below its own, two threads an entry
     const uint32_t t = threadIdx.x, kk = static_cast<uint32_t>(K);
     __shared__ __align__(16) uint32_t kid[512];
-    for (uint32_t i = t; i < ((kk + 15u) & ~15u); i += WS_BLOCK) kid[i] = i < kk ? 0xffffffffu - static_cast<uint32_t>(list[i]) : 0xffffffffu;
+    for (uint32_t i = t; i < ((kk + 15u) & ~15u); i += WS_BLOCK) kid[i] = how == 1 && i < kk ? 0xffffffffu - static_cast<uint32_t>(list[i]) : 0xffffffffu;
+    if (how == 3) {
+        if (n_keys > kk) top_select(list, n_keys, kk, kid, F);
+        else if (t < n_keys) kid[t] = 0xffffffffu - static_cast<uint32_t>(list[t]);
+    }
     __syncthreads();
     if (t == 0) {
         stats[2 * row] = F.red_f[0];
@@ -111,12 +212,15 @@ __global__ void __launch_bounds__(WS_BLOCK) topk_rows_shared(const float* x, int
 template <int NV>
 __global__ void __launch_bounds__(WS_BLOCK) dflash_topk_shared(const float* x, int n, int ld, int k, int* ids, float* vals, TopSplit sp) {
     __shared__ FewShared F;
-    const size_t row = blockIdx.y;
+    uint32_t row_, part;
+    if (!few_place(sp.together, sp.rows, row_, part)) return;
+    const size_t row = row_;
     x += row * ld;
     ids += row * k;
     vals += row * k;
     uint64_t* list;
-    const int how = top_share<NV, false>(x, n, k, 1.f, sp, static_cast<uint32_t>(row), F, list);
+    uint32_t n_keys;
+    const int how = top_share<NV, false, true>(x, n, [&]() { return k; }, 1.f, sp, row_, part, F, list, n_keys);
     if (how == 0) return;
     if (how == 2) {
         __syncthreads();
@@ -135,10 +239,20 @@ template <int NV>
 __global__ void __launch_bounds__(WS_BLOCK)
     draft_sample_rows_shared(const float* x, int n, int* ctl_all, RowIdx area, int r, const int* map, DSampArgs a, int* qbuf, TopSplit sp) {
     __shared__ FewShared F;
-    const int b = static_cast<int>(blockIdx.y), K = draft_candidates(ctl_all, area, r, a, n, b);
-    if (K == 0) return;  // (every part of the row sees the same words)
+    uint32_t row, part;
+    if (!few_place(sp.together, sp.rows, row, part)) return;
+    const int b = static_cast<int>(row);
+    if (a.on[b] == 0) return;
+    // (all of the row's parameters now: at the end each would be a trip of its own)
+    DraftRow D = DraftRow::of(a, b);
+    int at = area.v[b];
+    asm volatile("" : "+s"(D.top_k), "+s"(D.qoff), "+s"(D.inv_t), "+s"(D.top_p), "+s"(D.min_p), "+s"(D.key), "+s"(at));
+    int* c = ctl_all + at;
     uint64_t* list;
-    const int how = top_share<NV, true>(x + static_cast<size_t>(b) * n, n, K, a.inv_t[b], sp, static_cast<uint32_t>(b), F, list);
+    uint32_t n_keys;
+    int K = 0;
+    const int how = top_share<NV, true, true>(x + static_cast<size_t>(b) * n, n, [&]() { return K = draft_candidates(c, r, D.top_k, n); }, D.inv_t, sp, row, part, F,
+                                              list, n_keys);
     if (how == 0) return;
     if (how == 2) {
         __syncthreads();
@@ -147,14 +261,26 @@ __global__ void __launch_bounds__(WS_BLOCK)
     }
     __shared__ int s_id[kDraftMax];
     __shared__ float s_lg[kDraftMax];
+    __shared__ double s_race[kDraftMax];
     const int t = static_cast<int>(threadIdx.x);
-    if (t >= 64) return;
+    if (t >= 64) {  // another wave works out the logarithms of the candidates' race keys, which depend on nothing that this one does
+        const int i = t - 64;
+        if (i < K) {
+            const int id = static_cast<int>(0xffffffffu - static_cast<uint32_t>(list[i]));
+            s_race[i] = draft_race(D.key, map ? map[id] : id);
+        }
+        __syncthreads();
+        return;
+    }
     if (t < K) {
         s_id[t] = static_cast<int>(0xffffffffu - static_cast<uint32_t>(list[t]));
         s_lg[t] = unkey32(static_cast<uint32_t>(list[t] >> 32));
     }
     __builtin_amdgcn_wave_barrier();  // (one wave: its LDS stores are done before its loads)
-    draft_finish<true>(ctl_all, area, r, map, a, qbuf, b, K, s_id, s_lg, F.red_f[0], static_cast<float>(F.sum()));
+    draft_finish<true>(c, D, r, map, qbuf, K, s_id, s_lg, F.red_f[0], static_cast<float>(F.sum()), [&](int, int from) {
+        __syncthreads();
+        return s_race[from < K ? from : 0];
+    });
 #ifdef WS_SHORT_TIMERS
     unsigned char* work = sp.work + static_cast<size_t>(b) * kFewRowBytes;
     WSF_MARK(9);

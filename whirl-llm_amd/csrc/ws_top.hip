@@ -14,9 +14,9 @@ struct Sizes {
     TopSplit sp;
     int size;  // 0: 5 vectors a thread, 1: 10, 2: 20
 };
-Sizes sizes(int n, unsigned rows, unsigned parts, unsigned chunk_log2, unsigned char* work) {
+Sizes sizes(int n, unsigned rows, unsigned parts, unsigned chunk_log2, unsigned together, unsigned char* work) {
     const unsigned vectors = (static_cast<unsigned>(n) + 3u) / 4u, load = 64u * WS_WAVES * parts, each = (vectors + load - 1u) / load;
-    return {dim3(parts, rows), TopSplit{parts, chunk_log2, work}, each <= 5u ? 0 : (each <= 10u ? 1 : 2)};
+    return {few_grid(parts, rows, together), TopSplit{parts, chunk_log2, rows, together, work}, each <= 5u ? 0 : (each <= 10u ? 1 : 2)};
 }
 using TopkFn = void (*)(const float*, int, int, float, int*, float*, float*, TopSplit);
 using DflashFn = void (*)(const float*, int, int, int, int*, float*, TopSplit);
@@ -38,25 +38,25 @@ int prepare_top() {
 }
 
 int launch_topk_shared(hipStream_t stream, const float* x, int n, int K, float inv_t, int* ids, float* vals, float* stats, unsigned rows, unsigned parts,
-                       unsigned chunk_log2, unsigned char* work) {
+                       unsigned chunk_log2, unsigned together, unsigned char* work) {
     if (const int e = prepare_top(); e != 0) return e;
-    const Sizes z = sizes(n, rows, parts, chunk_log2, work);
+    const Sizes z = sizes(n, rows, parts, chunk_log2, together, work);
     hipLaunchKernelGGL(kTopk[z.size], z.grid, dim3(WS_BLOCK), kTopLds, stream, x, n, K, inv_t, ids, vals, stats, z.sp);
     return static_cast<int>(hipGetLastError());
 }
 
-int launch_dflash_shared(hipStream_t stream, const float* x, int n, int ld, int k, int* ids, float* vals, unsigned rows, unsigned parts, unsigned chunk_log2,
+int launch_dflash_shared(hipStream_t stream, const float* x, int n, int ld, int k, int* ids, float* vals, unsigned rows, unsigned parts, unsigned chunk_log2, unsigned together,
                          unsigned char* work) {
     if (const int e = prepare_top(); e != 0) return e;
-    const Sizes z = sizes(n, rows, parts, chunk_log2, work);
+    const Sizes z = sizes(n, rows, parts, chunk_log2, together, work);
     hipLaunchKernelGGL(kDflash[z.size], z.grid, dim3(WS_BLOCK), kTopLds, stream, x, n, ld, k, ids, vals, z.sp);
     return static_cast<int>(hipGetLastError());
 }
 
 int launch_draft_shared(hipStream_t stream, const float* x, int n, int* ctl_all, const void* area, int r, const int* map, const void* args, int* qbuf,
-                        unsigned rows, unsigned parts, unsigned chunk_log2, unsigned char* work) {
+                        unsigned rows, unsigned parts, unsigned chunk_log2, unsigned together, unsigned char* work) {
     if (const int e = prepare_top(); e != 0) return e;
-    const Sizes z = sizes(n, rows, parts, chunk_log2, work);
+    const Sizes z = sizes(n, rows, parts, chunk_log2, together, work);
     RowIdx ri;
     DSampArgs da;
     __builtin_memcpy(&ri, area, sizeof ri);
