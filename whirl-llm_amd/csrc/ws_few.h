@@ -34,7 +34,7 @@ constexpr uint32_t kFewWaves = kFewMaxParts * WS_WAVES;
 // Workspace of a row: kFewKeys keys, slot by slot with one key a wave in each, then what every wave says of its share -
 // {maximum, threshold} as order keys; the sum of exp against the maximum; how many keys it has listed, kFewBad when it could not
 // list them -, then {parts arrived, largest logit so far as an order key}. Zero-filled between launches.
-constexpr uint32_t kFewKeys = 7648u, kFewHead = kFewKeys * 8u, kFewCount = kFewHead + kFewWaves * 16u, kFewCtrl = kFewCount + kFewWaves * 4u;
+constexpr uint32_t kFewHead = kFewKeys * 8u, kFewCount = kFewHead + kFewWaves * 16u, kFewCtrl = kFewCount + kFewWaves * 4u;
 static_assert(kFewCtrl + 256u <= 64512u && 64512u < kFewRowBytes, "a row's workspace (debug builds put their clocks at 64512)");
 constexpr uint32_t kFewBad = 0xffffffffu;
 constexpr uint32_t kFewExt = 2048u;  // touched tokens of a share
@@ -65,15 +65,20 @@ struct FewShared {
     }
 };
 
-// the largest prefix (bits 31 .. 14) of an order key that at least d lanes of the wave reach: five instructions a bit (two bits a step are
-// fifteen, and no shorter a chain)
-__device__ __forceinline__ uint32_t few_lane_threshold(uint32_t k32, uint32_t d) {
+// the largest prefix (bits 31 .. 14) of an order key that at least d lanes of the wave reach; top: the largest key. Five instructions a bit (two bits a step
+// are fifteen, and no shorter a chain); the first eight bits are those of the top, or one octave below, as a rule.
+__device__ __forceinline__ uint32_t few_lane_threshold(uint32_t k32, uint32_t top, uint32_t d) {
+    auto reached = [&](uint32_t c) { return static_cast<uint32_t>(__popcll(__ballot(k32 >= c))) >= d; };
+    const uint32_t near = (top & 0xff000000u);
     uint32_t at = 0u;
+    if (reached(near)) {  // uniform
+        at = near;
+    } else {
 #pragma unroll
-    for (int b = 31; b >= 14; --b) {
-        const uint32_t c = at | (1u << b);
-        at = static_cast<uint32_t>(__popcll(__ballot(k32 >= c))) >= d ? c : at;
+        for (int b = 31; b >= 24; --b) at = reached(at | (1u << b)) ? at | (1u << b) : at;
     }
+#pragma unroll
+    for (int b = 23; b >= 14; --b) at = reached(at | (1u << b)) ? at | (1u << b) : at;
     return at;
 }
 __device__ __forceinline__ uint32_t lanes_before(uint64_t m) {  // set bits of m below this lane
@@ -95,9 +100,9 @@ __device__ __forceinline__ bool few_place(uint32_t together, uint32_t rows, uint
 // row (2^cl vectors) is wave c mod G's; vector k of a lane lies in its wave's chunk number k * (chunks a load) + lane / (lanes a
 // chunk).
 struct FewShare {
-    uint32_t parts, part, G, g, cl, V, nv, n_vec;  // G: waves a row, g: this one, nv: vectors of the row, n_vec: of a lane
+    uint32_t parts, part, G, g, cl, V, nv, n_vec, slots;  // G: waves a row, g: this one, nv: vectors of the row, n_vec: of a lane, slots: keys a wave can list
     template <int DT>
-    __device__ __forceinline__ static FewShare of(uint32_t V, uint32_t parts, uint32_t part, uint32_t cl) {
+    __device__ __forceinline__ static FewShare of(uint32_t V, uint32_t parts, uint32_t part, uint32_t cl, uint32_t n_vec, uint32_t slots) {
         constexpr uint32_t TPV = DT == 0 ? 4u : 8u;
         FewShare L;
         L.parts = parts;
@@ -107,7 +112,8 @@ struct FewShare {
         L.cl = cl;
         L.V = V;
         L.nv = (V + TPV - 1u) / TPV;
-        L.n_vec = (L.nv + 64u * L.G - 1u) / (64u * L.G);
+        L.slots = slots;
+        L.n_vec = n_vec;
         return L;
     }
     __device__ __forceinline__ uint32_t vec_of(uint32_t k) const {
@@ -156,7 +162,7 @@ __device__ __forceinline__ bool few_publish(const FewShare& L, const FewWant& W,
     constexpr uint32_t TPV = DT == 0 ? 4u : 8u;
     const uint32_t t = threadIdx.x, lane = t & 63u;
     const uint32_t wv = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(t >> 6)));
-    const uint32_t slots = kFewKeys / L.G;
+    const uint32_t slots = L.slots;
     const float wm = wave_max(lm);
     unsigned long long* gkeys = reinterpret_cast<unsigned long long*>(work);
     unsigned long long* ghead = reinterpret_cast<unsigned long long*>(work + kFewHead);
@@ -169,10 +175,10 @@ __device__ __forceinline__ bool few_publish(const FewShare& L, const FewWant& W,
     if (W.by_k) {
         // A wave has top_k / G of the row's top_k largest on average; two more and five times the scatter of that number
         // are listed, d of them in different lanes.
-        const float lambda = static_cast<float>(W.top_k) / static_cast<float>(L.G);
-        const uint32_t want = static_cast<uint32_t>(lambda + 5.f * __builtin_sqrtf(lambda) + 2.f) + 1u;
+        const float lambda = static_cast<float>(W.top_k) * __builtin_amdgcn_rcpf(static_cast<float>(L.G));
+        const uint32_t want = static_cast<uint32_t>(lambda + 5.f * __builtin_amdgcn_sqrtf(lambda) + 2.f) + 1u;
         const uint32_t d = min(60u, want <= 20u ? want : 20u + (want - 20u) / 2u);
-        const uint32_t at = few_lane_threshold(key32(lm), d);
+        const uint32_t at = few_lane_threshold(key32(lm), key32(wm), d);
         thr = at > 0x007fffffu ? unkey32(at) : -INFINITY;  // (below that prefix: -inf and the NaN patterns under it)
     } else if (W.by_p) {
         // what the floor lets through lies within -ln(min_p) / W.inv_t of the row's maximum: of the largest logit any part
@@ -271,7 +277,7 @@ __device__ __forceinline__ uint32_t few_collect(const FewShare& L, const FewWant
     unsigned long long* ghead = reinterpret_cast<unsigned long long*>(work + kFewHead);
     uint32_t* gcount = reinterpret_cast<uint32_t*>(work + kFewCount);
     uint32_t* ctrl = reinterpret_cast<uint32_t*>(work + kFewCtrl);
-    const uint32_t G = L.G, slots = kFewKeys / G;
+    const uint32_t G = L.G, slots = L.slots;
     // Headers and everybody's keys asked for (those of the first slots right away). Five waves read the headers side by side, each
     // for what it works out: the threshold, the normaliser (two of them: the exponentials are the longest chain here, and one a
     // lane is 0.1 us shorter than two), how many slots hold keys; and one the uniform.
@@ -360,9 +366,6 @@ __device__ __forceinline__ uint32_t few_collect(const FewShare& L, const FewWant
                     ++slot;
                 }
         }
-#pragma unroll
-        for (uint32_t i = 0; i < kBlind; ++i)  // the workspace as the next launch needs it
-            if (i0 + i * WS_BLOCK < n_read && key[i] != 0ull) __hip_atomic_store(&gkeys[i0 + i * WS_BLOCK + t], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     };
     keep(got, 0u);
     for (uint32_t i0 = kBlind * WS_BLOCK; i0 < n_read; i0 += kBlind * WS_BLOCK) {  // uniform
@@ -373,7 +376,14 @@ __device__ __forceinline__ uint32_t few_collect(const FewShare& L, const FewWant
             more[i] = at < n_read ? __hip_atomic_load(&gkeys[at], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0ull;
         }
         keep(more, i0);
+#pragma unroll
+        for (uint32_t i = 0; i < kBlind; ++i)
+            if (more[i] != 0ull) __hip_atomic_store(&gkeys[i0 + i * WS_BLOCK + t], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
+    // the workspace as the next launch needs it, all zeros (cleared behind the sort instead, rows with long lists took 2 % longer and lone rows 1 % less)
+#pragma unroll
+    for (uint32_t i = 0; i < kBlind; ++i)
+        if (i * WS_BLOCK < n_read && got[i] != 0ull) __hip_atomic_store(&gkeys[i * WS_BLOCK + t], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (t < G) {
         __hip_atomic_store(&ghead[t], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __hip_atomic_store(&ghead[kFewWaves + t], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -435,7 +445,7 @@ __device__ __forceinline__ bool few_row(const BatchArgs& A, const uint32_t row, 
     const long long wss_t0 = clock64();
 #endif
 
-    const FewShare L = FewShare::of<DT>(V, A.few_parts, part, A.few_chunk_log2);
+    const FewShare L = FewShare::of<DT>(V, A.few_parts, part, A.few_chunk_log2, A.few_vecs, A.few_slots);
     const uint32_t G = L.G, cl = L.cl, nv = L.nv, n_vec = L.n_vec;
     const uint32_t j_part = V % TPV ? nv - 1u : 0xffffffffu;
     uint4 q[NV];

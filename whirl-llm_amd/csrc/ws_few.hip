@@ -29,9 +29,12 @@ int launch_few(hipStream_t stream, const BatchArgs& a, unsigned lds_bytes, unsig
     if (const int e = prepare_few(lds_limit); e != 0) return e;
     const uint32_t per = a.dtype == 0 ? 4u : 8u, vectors = (a.vocab + per - 1u) / per, load = 64u * WS_WAVES * a.few_parts;
     const uint32_t each = (vectors + load - 1u) / load;
+    BatchArgs b = a;
+    b.few_vecs = each;
+    b.few_slots = kFewKeys / (WS_WAVES * a.few_parts);
     int size = 0;
     while (size < 3 && each > kFewVectors[a.dtype][size]) ++size;
-    hipLaunchKernelGGL(kFewKernels[a.dtype][a.allow ? 1 : 0][size], few_grid(a.few_parts, a.rows, a.few_together), dim3(WS_BLOCK), lds_bytes, stream, a);
+    hipLaunchKernelGGL(kFewKernels[a.dtype][a.allow ? 1 : 0][size], few_grid(a.few_parts, a.rows, a.few_together), dim3(WS_BLOCK), lds_bytes, stream, b);
     return static_cast<int>(hipGetLastError());
 }
 

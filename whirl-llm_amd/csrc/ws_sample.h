@@ -103,7 +103,7 @@ struct BatchArgs {
     uint32_t fb_lds_ab;
     uint32_t* done;       // ws_few.h: a word per row for a host that waits (or nullptr), and what goes there
     uint32_t done_value;
-    uint32_t few_parts, few_magic, few_chunk_log2;  // ws_few.h: parts a row, 2^32 / waves a row rounded up, log2 of the lanes a chunk
+    uint32_t few_parts, few_magic, few_chunk_log2, few_vecs, few_slots;  // ws_few.h: parts a row, 2^32 / waves a row rounded up, log2 of the lanes a chunk, vectors a lane, keys a wave can list
     uint32_t few_together;  // ws_few.h: whether a row's parts go to one chiplet (few_place)
     uint32_t code_cap, code_route;  // ws_code.h: history and bias entries its tables have room for, and the route bit of its rows
     uint32_t code_head;           // its masses: 0 in 64 bits; else by the single-sweep kernels' bins, the anchor above the first 8192 tokens that nothing touches (1), or the first 16384 (2)
@@ -128,6 +128,7 @@ constexpr uint32_t kChiplets = 8u;  // XCDs of the device
 __host__ inline dim3 few_grid(uint32_t parts, uint32_t rows, uint32_t together) {
     return together ? dim3(parts * kChiplets, (rows + kChiplets - 1u) / kChiplets) : dim3(parts, rows);
 }
+constexpr uint32_t kFewKeys = 7648u;  // keys of a row in its workspace (ws_few.h)
 constexpr uint32_t kTwinBins = 2048u;  // ws_twin.h: bins of the sample's logits, 1/32 e-fold each
 constexpr uint32_t kShortSplitCtrl = kShortCap * 8u, kShortSplitRowBytes = kShortSplitCtrl + 768u;  // the same of ws_short.h's shared rows
 // Workspace of one row of the three-pass kernel: per history / bias entry a word of each of phase 0's two rank

@@ -152,13 +152,17 @@ __device__ __forceinline__ void short_rules(uint64_t* list, const uint32_t row, 
     typedef const __attribute__((address_space(4))) BatchArgs* ArgPtr;
     ArgPtr Ap = (ArgPtr)__builtin_amdgcn_kernarg_segment_ptr();
     uint32_t n3;
-    auto write_out = [&](uint32_t id_, double e_, double cin_, double cex_, double Zk_, double target_, bool drawn, double mg_top_p_, double mg_min_p_, uint32_t pos) {
-        const double mg = drawn ? fmin(cin_ - target_, pos > 0u ? target_ - cex_ : 1e300) / Zk_ : 0.0;
+    // a distance to a decision, and what it is measured in (divided only where somebody asks for the quotient: a division is some 200 clocks of the chain)
+    struct Margin {
+        double d, of;
+    };
+    auto write_out = [&](uint32_t id_, double e_, double cin_, double cex_, double Zk_, double target_, bool drawn, Margin mg_top_p_, Margin mg_min_p_, uint32_t pos) {
+        const Margin mg = {drawn ? fmin(cin_ - target_, pos > 0u ? target_ - cex_ : 1e300) : 0.0, Zk_};
         const double tol = Ap->tol;
         uint32_t flags = kRouteShort;
-        if (mg_top_p_ < tol) flags |= kNearTopP;
-        if (mg_min_p_ < tol) flags |= kNearMinP;
-        if (mg < tol) flags |= kNearDraw;
+        if (mg_top_p_.d < tol * mg_top_p_.of) flags |= kNearTopP;
+        if (mg_min_p_.d < tol * mg_min_p_.of) flags |= kNearMinP;
+        if (mg.d < tol * mg.of) flags |= kNearDraw;
         Ap->token[row] = static_cast<int32_t>(id_);
         Ap->flags[row] = flags;
         if (Ap->prob) Ap->prob[row] = static_cast<float>(e_ / Zk_);
@@ -168,9 +172,9 @@ __device__ __forceinline__ void short_rules(uint64_t* list, const uint32_t row, 
             Ap->stats[2 * row + 1] = static_cast<float>(R.z);
         }
         if (Ap->margin) {
-            Ap->margin[3 * row] = mg_top_p_;
-            Ap->margin[3 * row + 1] = mg_min_p_;
-            Ap->margin[3 * row + 2] = mg;
+            Ap->margin[3 * row] = mg_top_p_.d / mg_top_p_.of;
+            Ap->margin[3 * row + 1] = mg_min_p_.d / mg_min_p_.of;
+            Ap->margin[3 * row + 2] = mg.d / mg.of;
         }
     };
     // optional outputs: -sum p ln p over the kept set with p = e / Zk and ln e = (x - m) / temperature, which is
@@ -267,7 +271,7 @@ __device__ __forceinline__ void short_rules(uint64_t* list, const uint32_t row, 
 #pragma unroll
         for (uint32_t j = 0; j < KC; ++j)
             if (KC * t + j == d_pos)
-                write_out(0xffffffffu - static_cast<uint32_t>(wkey[j]), e[j], cin[j], cex[j], Zk, target, dq != ~0ull, mg_top_p, mg_min_p, d_pos);
+                write_out(0xffffffffu - static_cast<uint32_t>(wkey[j]), e[j], cin[j], cex[j], Zk, target, dq != ~0ull, {mg_top_p, 1.0}, {mg_min_p, 1.0}, d_pos);
         if (more) {
             double se = 0.0, sq = 0.0;
 #pragma unroll
@@ -291,17 +295,17 @@ __device__ __forceinline__ void short_rules(uint64_t* list, const uint32_t row, 
             const double Zk1 = lane_value(cin, n_cand - 1u);
             const double X = top_p * (by_k ? Zk1 : z_row);
             uint32_t n2 = n_cand;
-            double mg_top_p = 1.0, mg_min_p = 1.0;
+            Margin mg_top_p = {1.0, 1.0}, mg_min_p = {1.0, 1.0};
             if (use_top_p) {
                 const uint64_t cm = __ballot(has && cin >= X && !(cex >= X));
                 if (cm) {
                     const uint32_t jc = static_cast<uint32_t>(__ffsll(static_cast<unsigned long long>(cm)) - 1);
                     n2 = jc + 1u;
                     const double ci = lane_value(cin, jc), ce = lane_value(cex, jc);
-                    mg_top_p = fmin(ci - X, jc > 0u ? X - ce : X) / X;
+                    mg_top_p = {fmin(ci - X, jc > 0u ? X - ce : X), X};
                 } else {
                     // a top-k row: rounding, the running mass never reaches top_p of itself. Else: the cut lies behind the list
-                    mg_top_p = by_k ? 0.0 : (X - Zk1) / X;
+                    mg_top_p = {by_k ? 0.0 : X - Zk1, X};
                 }
             }
             n3 = n2;
@@ -309,9 +313,10 @@ __device__ __forceinline__ void short_rules(uint64_t* list, const uint32_t row, 
                 const uint32_t passed = static_cast<uint32_t>(__popcll(__ballot(has && e >= min_p)));  // (a prefix of the order: masses do not rise along it)
                 n3 = min(n2, passed);
                 if (n3 < 1u) n3 = 1u;
-                const double near = fabs(e - min_p) / min_p;
-                if (passed > 0u) mg_min_p = fmin(mg_min_p, lane_value(near, passed - 1u));
-                if (passed < n_cand) mg_min_p = fmin(mg_min_p, lane_value(near, passed));
+                const double near = fabs(e - min_p);
+                mg_min_p = {min_p, min_p};
+                if (passed > 0u) mg_min_p.d = fmin(mg_min_p.d, lane_value(near, passed - 1u));
+                if (passed < n_cand) mg_min_p.d = fmin(mg_min_p.d, lane_value(near, passed));
             }
             const double Zk = lane_value(cin, n3 - 1u);
             const double target = u * Zk;
@@ -375,7 +380,7 @@ __device__ __forceinline__ void short_rules(uint64_t* list, const uint32_t row, 
         __syncthreads();
         const unsigned long long dq = S.s_q[1];
         const uint32_t d_pos = dq != ~0ull ? static_cast<uint32_t>(dq) : n3 - 1u;  // (src/sampling/sampler.cpp:131: the walk falls through to the last kept)
-        if (has && t == d_pos) write_out(id, e, cin, cex, Zk, target, dq != ~0ull, mg_top_p, mg_min_p, d_pos);
+        if (has && t == d_pos) write_out(id, e, cin, cex, Zk, target, dq != ~0ull, {mg_top_p, 1.0}, {mg_min_p, 1.0}, d_pos);
         if (more) {
             const bool kept = has && t < n3;
             const double se = block_sum(kept && e > 0.0 ? e * log_mass(x) : 0.0, S.red_d), sq = block_sum(kept && id == query ? e : 0.0, S.red_d);

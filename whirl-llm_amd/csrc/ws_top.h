@@ -13,7 +13,7 @@
 namespace ws {
 
 struct TopSplit {
-    uint32_t parts, chunk_log2, rows, together;  // (together: few_place)
+    uint32_t parts, chunk_log2, rows, together, vecs, slots;  // (together: few_place)
     unsigned char* work;  // kFewRowBytes a row
 };
 
@@ -27,7 +27,7 @@ __device__ __forceinline__ int top_share(const float* x, int n, KOF&& K_of, floa
 #ifdef WS_SHORT_TIMERS
     if (threadIdx.x == 0) F.t0 = clock64();
 #endif
-    const FewShare L = FewShare::of<0>(V, sp.parts, part, sp.chunk_log2);
+    const FewShare L = FewShare::of<0>(V, sp.parts, part, sp.chunk_log2, sp.vecs, sp.slots);
     const uint32_t j_part = V % 4u ? L.nv - 1u : 0xffffffffu;
     const unsigned char* base = reinterpret_cast<const unsigned char*>(x);
     uint4 q[NV];
@@ -60,13 +60,13 @@ __device__ __forceinline__ int top_share(const float* x, int n, KOF&& K_of, floa
     list = reinterpret_cast<uint64_t*>(lds);
     n_keys = few_collect<SUM>(L, W, work, F, list, []() {});
     if (n_keys < W.top_k || n_keys > kShortCap) return 2;
-    if (!ORDER && n_keys > WS_BLOCK / 4u) return 3;
-    list = few_sort(list, n_keys, F);
+    const bool sorts = ORDER || n_keys <= WS_BLOCK / 4u;
+    if (sorts) list = few_sort(list, n_keys, F);
 #ifdef WS_SHORT_TIMERS
     if (threadIdx.x == 0) reinterpret_cast<long long*>(work + 64512)[10] = n_keys;
 #endif
     WSF_MARK(8);
-    return 1;
+    return sorts ? 1 : 3;
 }
 
 // The ids of the K largest of the n listed keys (n > K, n <= kShortCap), in no order, to `ids`: the buckets of short_sort, of which only the one that the

@@ -16,7 +16,7 @@ struct Sizes {
 };
 Sizes sizes(int n, unsigned rows, unsigned parts, unsigned chunk_log2, unsigned together, unsigned char* work) {
     const unsigned vectors = (static_cast<unsigned>(n) + 3u) / 4u, load = 64u * WS_WAVES * parts, each = (vectors + load - 1u) / load;
-    return {few_grid(parts, rows, together), TopSplit{parts, chunk_log2, rows, together, work}, each <= 5u ? 0 : (each <= 10u ? 1 : 2)};
+    return {few_grid(parts, rows, together), TopSplit{parts, chunk_log2, rows, together, each, kFewKeys / (parts * WS_WAVES), work}, each <= 5u ? 0 : (each <= 10u ? 1 : 2)};
 }
 using TopkFn = void (*)(const float*, int, int, float, int*, float*, float*, TopSplit);
 using DflashFn = void (*)(const float*, int, int, int, int*, float*, TopSplit);
