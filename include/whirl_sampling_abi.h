@@ -472,6 +472,8 @@ int ws_accept_sampled(void* stream, const ws_accept* a);
 /* Acceptor::greedy on the device (src/sampling/acceptor.cpp:30-61). Per sequence: c[WS_CTL_ROWS + j] holds the argmax of
  * verify row j (argmax_rows_to), the drafts are kept while they equal it; with `relax` a draft that differs is still kept
  * when it is among the row's relax_k largest logits - fewer than relax_k candidates before it in (logit desc, id asc)
+/* The same with `relaxed` written, not added to: a caller that starts each cycle's counts at zero need not clear them first. */
+int ws_accept_sampled_fresh(void* stream, const ws_accept* a);
  * order - with exp(logit - max) >= alpha (include/whirl/relax_accept.h:55-70) and does not close a repeated 6-gram.
  * The rows' largest logits come from ws_topk_rows(K = k, inv_t = 1) in its [ids | vals | stats] layout
  * (src/sampling/acceptor.h:42-48): row of position j of sequence s = row0[s] + j. chosen = the argmax at the stop.

@@ -153,6 +153,7 @@ ABI = {
     "ws_adjust_rows": (C.c_int, [C.c_void_p, C.POINTER(Adjust)]),
     "ws_accept_sampled": (C.c_int, [C.c_void_p, C.POINTER(Accept)]),
     "ws_accept_greedy": (C.c_int, [C.c_void_p, C.POINTER(AcceptGreedy)]),
+    "ws_accept_sampled_fresh": (C.c_int, [C.c_void_p, C.POINTER(Accept)]),
     "ws_history_stage": (C.c_int, [C.c_void_p, C.POINTER(HistoryStage)]),
     "ws_spec_verify_workspace": (C.c_uint64, [C.POINTER(SpecVerify)]),
     "ws_spec_verify_classic": (C.c_int, [C.c_void_p, C.POINTER(SpecVerify)]),
@@ -405,7 +406,7 @@ def history_stage(hist, slot, ctl_all, area, row0, hist_off, hist_len, query=Non
 
 
 def accept_sampled(token, flags, row0, ctl_all, area, typical=None, hist=None, slot=None):
-    """Accepted draft count and chosen token per sequence from the sampled tokens of its verify rows (ws_accept_sampled).
+    """Accepted draft count and chosen token per sequence from the sampled tokens of its verify rows (ws_accept_sampled_fresh).
     token int32 [rows], flags uint32-as-int32 [rows], row0 int32 [n_seq], ctl_all int32 control areas, area int32 [n_seq]
     word offsets; all device tensors. typical: dict(query_prob, entropy, eps, delta) for the relaxacc_typical rule.
     hist / slot: a DeviceHistory and the sequences' slots. Returns (n_accepted, chosen, status, relaxed) int32 device
@@ -414,7 +415,7 @@ def accept_sampled(token, flags, row0, ctl_all, area, typical=None, hist=None, s
         if not v.is_cuda or v.dtype != torch.int32 or not v.is_contiguous():
             raise WsError(f"{name}: contiguous int32 device tensor")
     n_seq = row0.numel()
-    n_acc, chosen, status, relaxed = torch.zeros((4, n_seq), dtype=torch.int32, device=token.device).unbind()
+    n_acc, chosen, status, relaxed = torch.empty((4, n_seq), dtype=torch.int32, device=token.device).unbind()  # (all four are written)
     a = Accept(token=_p(token), flags=_p(flags), row0=_p(row0), ctl_all=_p(ctl_all), area=_p(area), n_seq=n_seq,
                n_accepted=_p(n_acc), chosen=_p(chosen), status=_p(status), relaxed=_p(relaxed))
     if typical is not None:
@@ -423,7 +424,7 @@ def accept_sampled(token, flags, row0, ctl_all, area, typical=None, hist=None, s
         a.eps, a.delta = typical["eps"], typical["delta"]
     if hist is not None:
         a.hist = hist.ref(slot)
-    check(lib().ws_accept_sampled(_stream(), C.byref(a)), "ws_accept_sampled")
+    check(lib().ws_accept_sampled_fresh(_stream(), C.byref(a)), "ws_accept_sampled_fresh")
     return n_acc, chosen, status, relaxed
 
 

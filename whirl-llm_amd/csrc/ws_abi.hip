@@ -929,7 +929,8 @@ ws::HistoryRef history_ref(const ws_history& h) { return ws::HistoryRef{h.tokens
 bool history_ok(const ws_history& h) { return !h.tokens || (h.len && h.slot && h.cap >= 2u); }
 }  // namespace
 
-int ws_accept_sampled(void* stream, const ws_accept* b) {
+namespace {
+int accept_sampled_on(void* stream, const ws_accept* b, bool fresh) {
     if (!b || !b->token || !b->flags || !b->row0 || !b->ctl_all || !b->area || !b->n_accepted || !b->chosen || !b->status)
         return WS_E_INVALID;
     if (b->n_seq == 0 || !history_ok(b->hist)) return WS_E_INVALID;
@@ -953,7 +954,7 @@ int ws_accept_sampled(void* stream, const ws_accept* b) {
     a.approx_mask = WS_FLAG_APPROX_ENTROPY;
     a.relaxed = b->relaxed;
     a.hist = history_ref(b->hist);
-    hipLaunchKernelGGL(ws::accept_sampled_kernel, dim3(b->n_seq), dim3(64), 0, S(stream), a);
+    hipLaunchKernelGGL(fresh ? ws::accept_sampled_kernel<true> : ws::accept_sampled_kernel<false>, dim3(b->n_seq), dim3(64), 0, S(stream), a);
     return done();
 }
 
@@ -986,6 +987,11 @@ int ws_accept_greedy(void* stream, const ws_accept_greedy_args* b) {
 int ws_history_stage(void* stream, const ws_history_stage_args* b) {
     if (!b || !b->hist.tokens || !history_ok(b->hist) || !b->ctl_all || !b->area || !b->row0 || !b->hist_off || !b->hist_len || !b->status ||
         b->n_seq == 0)
+}  // namespace
+
+int ws_accept_sampled(void* stream, const ws_accept* b) { return accept_sampled_on(stream, b, false); }
+
+int ws_accept_sampled_fresh(void* stream, const ws_accept* b) { return accept_sampled_on(stream, b, true); }
         return WS_E_INVALID;
     if (b->step && !b->hist.n_gen) return WS_E_INVALID;
     ws::StageArgs a{};
@@ -999,7 +1005,7 @@ int ws_history_stage(void* stream, const ws_history_stage_args* b) {
     a.query = b->query;
     a.step = b->step;
     a.status = b->status;
-    hipLaunchKernelGGL(ws::history_stage_kernel, dim3((b->n_seq + 63u) / 64u), dim3(64), 0, S(stream), a);
+    hipLaunchKernelGGL(ws::history_stage_kernel, dim3((b->n_seq + ws::kStageSeqs - 1u) / ws::kStageSeqs), dim3(64), 0, S(stream), a);
     return done();
 }
 

@@ -83,63 +83,86 @@ __device__ __forceinline__ bool history_append(const HistoryRef& h, uint32_t seq
     return true;
 }
 
-// One wave per sequence: at most 16 positions, a few dozen bytes; the wave is there for the repeat guard.
+// One wave per sequence, a lane per position: a cycle has at most 16. What the positions say is read by all lanes at once - the area's words, the rows' answers, two
+// trips to memory behind the offsets - and the walk below goes over registers. (A lane that walked from position to position made a trip of each: 8
+// sequences of 4 drafts took 6.2 us and the fill before it, which cleared `relaxed`, 3.9; the kernel takes 3.8 now, without a fill.) FRESH: `relaxed` is written, not added to.
+template <bool FRESH>
 __global__ void __launch_bounds__(64) accept_sampled_kernel(AcceptArgs A) {
-    const uint32_t s = blockIdx.x;
+    const uint32_t s = blockIdx.x, lane = threadIdx.x;
     if (s >= A.n_seq) return;
     int32_t* c = A.ctl_all + A.area[s];
-    int32_t nd = c[48];
-    nd = nd < 0 ? 0 : (nd > 15 ? 15 : nd);
     const uint32_t r0 = A.row0[s];
-    const int32_t* text = nullptr;
+    const uint32_t slot = A.hist.tokens ? A.hist.slot[s] : 0u;
+    int32_t nd = c[48];
+    const int32_t draft = c[16 + (lane & 15u)];
+    int32_t* text = nullptr;
     uint32_t n_hist = 0;
+    uint64_t n_gen = 0;
     if (A.hist.tokens) {
-        const uint32_t slot = A.hist.slot[s];
         text = A.hist.tokens + static_cast<size_t>(slot) * A.hist.cap;
         n_hist = A.hist.len[slot];
+        if (A.hist.n_gen) n_gen = A.hist.n_gen[slot];
     }
-    int32_t acc = 0;
-    uint32_t st = 0, n_relaxed = 0;
-    int32_t tok = -1;
+    nd = nd < 0 ? 0 : (nd > 15 ? 15 : nd);
+    const uint32_t was_relaxed = !FRESH && A.relaxed ? A.relaxed[s] : 0u;
     if (text && n_hist + 2u + static_cast<uint32_t>(nd) > A.hist.cap) {
         // no room for next and the drafts behind the text: the guard would read past the slot. The host takes the sequence.
-        if (threadIdx.x == 0) {
+        if (lane == 0u) {
             A.n_accepted[s] = 0;
             A.chosen[s] = -1;
             A.status[s] = kAcceptHistoryFull | kAcceptHost;
+            if (FRESH && A.relaxed) A.relaxed[s] = 0u;
         }
         return;
     }
-    for (;;) {  // position acc: its token is the output; it is accepted when it is a draft position and equals the draft
-        tok = A.token[r0 + acc];
-        const uint32_t fl = A.flags[r0 + acc];
-        if (tok < 0 || (fl & A.host_mask) != 0u) {
+    // every lane's position (those behind the last stand for it once more, and are not looked at)
+    const uint32_t row = r0 + min(lane, static_cast<uint32_t>(nd));
+    const bool drafted = lane < static_cast<uint32_t>(nd);
+    const int32_t tok_ = A.token[row];
+    const uint32_t fl = A.flags[row];
+    bool typical = false, near = false;
+    if (A.typical) {
+        // p(draft) >= min(eps, delta * exp(-entropy)), and the draft does not close a repeated 6-gram
+        const double pd = A.query_prob[row];
+        const double thr = fmin(static_cast<double>(A.eps), static_cast<double>(A.delta) * exp(-A.entropy[row]));
+        typical = drafted && pd >= thr;
+        near = drafted && (fl & A.approx_mask) && fabs(pd - thr) < 0.02 * thr;
+    }
+    const uint32_t gone = static_cast<uint32_t>(__ballot(tok_ < 0 || (fl & A.host_mask) != 0u)), nears = static_cast<uint32_t>(__ballot(near)),
+                   typicals = static_cast<uint32_t>(__ballot(typical)), equals = static_cast<uint32_t>(__ballot(drafted && tok_ == draft));
+    uint32_t acc = 0, st = 0, n_relaxed = 0;
+    for (;; ++acc) {  // position acc: its token is the output; it is accepted when it is a draft position and equals the draft
+        const uint32_t bit = 1u << acc;
+        if (gone & bit) {
             st |= kAcceptHost;
             break;
         }
-        if (A.typical && acc < nd) {
-            // p(draft) >= min(eps, delta * exp(-entropy)), and the draft does not close a repeated 6-gram
-            const double pd = A.query_prob[r0 + acc];
-            const double thr = fmin(static_cast<double>(A.eps), static_cast<double>(A.delta) * exp(-A.entropy[r0 + acc]));
-            if ((fl & A.approx_mask) && fabs(pd - thr) < 0.02 * thr) st |= kAcceptNearTypical;
-            // tail of the guard: next, dr[0 .. acc] - they sit behind the history when the cycle was staged
-            if (pd >= thr && !(text && extends_repeat(text, n_hist, static_cast<uint32_t>(acc) + 2u))) {
-                c[acc] = c[16 + acc];
-                ++acc;
-                ++n_relaxed;
-                continue;
-            }
+        if (nears & bit) st |= kAcceptNearTypical;
+        // tail of the guard: next, dr[0 .. acc] - they sit behind the history when the cycle was staged
+        if ((typicals & bit) && !(text && extends_repeat(text, n_hist, acc + 2u))) {
+            ++n_relaxed;
+            continue;
         }
-        c[acc] = tok;  // where the greedy path keeps the row's argmax
-        if (acc == nd || tok != c[16 + acc]) break;
-        ++acc;
+        if (!(equals & bit)) break;  // (none behind the last draft)
     }
-    if (threadIdx.x == 0) {
-        if (!(st & kAcceptHost) && !history_append(A.hist, s, c, acc, tok)) st |= kAcceptHistoryFull | kAcceptHost;
-        A.n_accepted[s] = acc;
+    const int32_t tok = __builtin_amdgcn_readlane(tok_, acc);
+    if (lane < acc) c[lane] = draft;  // where the greedy path keeps the row's argmax
+    if (lane == acc && !(st & kAcceptHost)) c[lane] = tok;
+    if (text && !(st & kAcceptHost)) {  // what was accepted goes behind the sequence's text: next, the kept drafts; the chosen token becomes the new `next`
+        // (there is room: less than next and the drafts. The drafts are there already when the cycle was staged; written again for callers that did not)
+        const uint32_t new_len = n_hist + 1u + acc;
+        if (lane < acc) text[n_hist + 1u + lane] = draft;
+        if (lane == 0u) {
+            text[new_len] = tok;
+            A.hist.len[slot] = new_len;
+            if (A.hist.n_gen) A.hist.n_gen[slot] = n_gen + acc + 1ull;
+        }
+    }
+    if (lane == 0u) {
+        A.n_accepted[s] = static_cast<int32_t>(acc);
         A.chosen[s] = tok;
         A.status[s] = st;
-        if (A.relaxed) A.relaxed[s] += n_relaxed;
+        if (A.relaxed) A.relaxed[s] = was_relaxed + n_relaxed;
     }
 }
 
@@ -243,26 +266,28 @@ struct StageArgs {
     uint32_t* status;     // out per sequence: kAcceptHistoryFull when the slot has no room
 };
 
-__global__ void history_stage_kernel(StageArgs A) {
-    const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
+// Sixteen lanes a sequence, one a position: the words they need are two trips to memory behind the offsets. (One lane that went from position to position, each
+// waiting for its draft, took 4.3 us for 8 sequences of 4 drafts; these take 2.5.)
+constexpr uint32_t kStageLanes = 16u, kStageSeqs = 64u / kStageLanes;
+__global__ void __launch_bounds__(64) history_stage_kernel(StageArgs A) {
+    const uint32_t s = blockIdx.x * kStageSeqs + threadIdx.x / kStageLanes, j = threadIdx.x % kStageLanes;
     if (s >= A.n_seq) return;
     const int32_t* c = A.ctl_all + A.area[s];
+    const uint32_t slot = A.hist.slot[s], row = A.row0[s] + j;
     int32_t nd = c[48];
-    nd = nd < 0 ? 0 : (nd > 15 ? 15 : nd);
-    const uint32_t slot = A.hist.slot[s];
-    int32_t* text = A.hist.tokens + static_cast<size_t>(slot) * A.hist.cap;
+    const int32_t draft = c[16u + j];
     const uint32_t len = A.hist.len[slot];
-    const bool room = len + 2u + static_cast<uint32_t>(nd) <= A.hist.cap;
-    A.status[s] = room ? 0u : kAcceptHistoryFull;
-    const uint32_t r0 = A.row0[s];
-    for (int32_t j = 0; j <= nd; ++j) {
-        if (room && j < nd) text[len + 1u + j] = c[16 + j];
-        const uint32_t row = r0 + static_cast<uint32_t>(j);
-        A.hist_off[row] = slot * A.hist.cap;
-        A.hist_len[row] = room ? len + 1u + static_cast<uint32_t>(j) : 0u;
-        if (A.query) A.query[row] = j < nd ? c[16 + j] : -1;
-        if (A.step && A.hist.n_gen) A.step[row] = A.hist.n_gen[slot] + static_cast<uint64_t>(j);
-    }
+    const uint64_t n_gen = A.step && A.hist.n_gen ? A.hist.n_gen[slot] : 0ull;
+    nd = nd < 0 ? 0 : (nd > 15 ? 15 : nd);
+    const uint32_t n = static_cast<uint32_t>(nd);
+    const bool room = len + 2u + n <= A.hist.cap;
+    if (j == 0u) A.status[s] = room ? 0u : kAcceptHistoryFull;
+    if (j > n) return;
+    if (room && j < n) A.hist.tokens[static_cast<size_t>(slot) * A.hist.cap + len + 1u + j] = draft;
+    A.hist_off[row] = slot * A.hist.cap;
+    A.hist_len[row] = room ? len + 1u + j : 0u;
+    if (A.query) A.query[row] = j < n ? draft : -1;
+    if (A.step && A.hist.n_gen) A.step[row] = n_gen + j;
 }
 
 }  // namespace ws
