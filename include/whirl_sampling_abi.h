@@ -353,6 +353,10 @@ int ws_sample_batch(void* stream, const ws_batch* b);
  * once everything the launch writes is visible to the host. Looking at those words costs some 5 us less than a stream wait;
  * a caller that looks in vain asks the stream (hipStreamQuery) for an error. */
 int ws_sample_batch_notify(void* stream, const ws_batch* b, uint32_t* done, uint32_t value);
+/* The same for a caller whose parameters and lists (inv_t .. freq, hist, bias_*, their offsets) lie in host memory that the device reads in place
+ * (hipHostMalloc) and are as they should be when the call is made: the call may read them too, and send a lone row's along with the
+ * launch. They stay as they are until the words have come. */
+int ws_sample_batch_notify_host(void* stream, const ws_batch* b, uint32_t* done, uint32_t value);
 /* ws_sample_batch for callers that cannot allocate device memory - code under HIP graph capture, tight serving loops,
  * harnesses that forbid it; it has no counterpart in the reference. The split rows of a small batch meet in memory that is
  * part of the library's code object on every GPU (WS_STATIC_SPLIT_ROWS rows of it, about 4 MiB, held until the process
@@ -468,12 +472,12 @@ typedef struct ws_accept {
 } ws_accept;
 
 int ws_accept_sampled(void* stream, const ws_accept* a);
+/* The same with `relaxed` written, not added to: a caller that starts each cycle's counts at zero need not clear them first. */
+int ws_accept_sampled_fresh(void* stream, const ws_accept* a);
 
 /* Acceptor::greedy on the device (src/sampling/acceptor.cpp:30-61). Per sequence: c[WS_CTL_ROWS + j] holds the argmax of
  * verify row j (argmax_rows_to), the drafts are kept while they equal it; with `relax` a draft that differs is still kept
  * when it is among the row's relax_k largest logits - fewer than relax_k candidates before it in (logit desc, id asc)
-/* The same with `relaxed` written, not added to: a caller that starts each cycle's counts at zero need not clear them first. */
-int ws_accept_sampled_fresh(void* stream, const ws_accept* a);
  * order - with exp(logit - max) >= alpha (include/whirl/relax_accept.h:55-70) and does not close a repeated 6-gram.
  * The rows' largest logits come from ws_topk_rows(K = k, inv_t = 1) in its [ids | vals | stats] layout
  * (src/sampling/acceptor.h:42-48): row of position j of sequence s = row0[s] + j. chosen = the argmax at the stop.

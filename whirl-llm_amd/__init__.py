@@ -149,11 +149,12 @@ ABI = {
     "ws_sample_batch_workspace_use": (C.c_int, [C.POINTER(Batch)]),
     "ws_sample_batch": (C.c_int, [C.c_void_p, C.POINTER(Batch)]),
     "ws_sample_batch_notify": (C.c_int, [C.c_void_p, C.POINTER(Batch), C.c_void_p, C.c_uint32]),
+    "ws_sample_batch_notify_host": (C.c_int, [C.c_void_p, C.POINTER(Batch), C.c_void_p, C.c_uint32]),
     "ws_sample_batch_static": (C.c_int, [C.c_void_p, C.POINTER(Batch)]),
     "ws_adjust_rows": (C.c_int, [C.c_void_p, C.POINTER(Adjust)]),
     "ws_accept_sampled": (C.c_int, [C.c_void_p, C.POINTER(Accept)]),
-    "ws_accept_greedy": (C.c_int, [C.c_void_p, C.POINTER(AcceptGreedy)]),
     "ws_accept_sampled_fresh": (C.c_int, [C.c_void_p, C.POINTER(Accept)]),
+    "ws_accept_greedy": (C.c_int, [C.c_void_p, C.POINTER(AcceptGreedy)]),
     "ws_history_stage": (C.c_int, [C.c_void_p, C.POINTER(HistoryStage)]),
     "ws_spec_verify_workspace": (C.c_uint64, [C.POINTER(SpecVerify)]),
     "ws_spec_verify_classic": (C.c_int, [C.c_void_p, C.POINTER(SpecVerify)]),

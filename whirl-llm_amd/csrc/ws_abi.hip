@@ -46,7 +46,7 @@ int launch_code(hipStream_t stream, const BatchArgs& a, unsigned rows, unsigned 
 int prepare_code(unsigned lds_limit);
 uint64_t code_lds_bytes(uint32_t vocab, uint32_t cap, uint32_t copies);
 // ws_few.hip: the same rows shared between workgroups that hold them in registers
-int launch_few(hipStream_t stream, const BatchArgs& a, unsigned lds_bytes, unsigned lds_limit);
+int launch_few(hipStream_t stream, const BatchArgs& a, unsigned lds_bytes, unsigned lds_limit, const OwnRow* own);
 int prepare_few(unsigned lds_limit);
 // ws_top.hip: topk_rows, dflash_topk and draft_sample_rows with rows shared between workgroups
 int launch_topk_shared(hipStream_t stream, const float* x, int n, int K, float inv_t, int* ids, float* vals, float* stats, unsigned rows, unsigned parts,
@@ -756,7 +756,7 @@ BatchPlan plan_for(const ws_batch* b, uint64_t work_bytes) {
 
 // done: a word per row that gets `value` once the row's results are visible to the host, or nullptr (ws_sample_batch_notify)
 int sample_batch_on(void* stream, const ws_batch* b, const BatchPlan& p, unsigned char* work, uint64_t work_bytes, uint32_t* done_at = nullptr,
-                    uint32_t done_value = 0u) {
+                    uint32_t done_value = 0u, const ws::OwnRow* own = nullptr) {
     const bool can_split = split_fits(p, work, work_bytes);
     const bool staged = can_split && work_bytes >= p.workspace && p.workspace > p.workspace_min;
     ws::BatchArgs a{};
@@ -818,7 +818,7 @@ int sample_batch_on(void* stream, const ws_batch* b, const BatchPlan& p, unsigne
         a.work = work;
         a.fb_lds_tie = 0u;
         a.fb_lds_ab = p.short_fb_ab;
-        return ws::launch_few(S(stream), a, p.few_total, kMaxLds - kStaticFew);
+        return ws::launch_few(S(stream), a, p.few_total, kMaxLds - kStaticFew, own);
     }
     if (p.code) {
         a.lds_tie = p.code_copies > 1u;
@@ -867,17 +867,47 @@ int ws_sample_batch(void* stream, const ws_batch* b) {
     return sample_batch_on(stream, b, p, static_cast<unsigned char*>(b->workspace), b->workspace_bytes);
 }
 
-int ws_sample_batch_notify(void* stream, const ws_batch* b, uint32_t* done, uint32_t value) {
+namespace {
+// what load_row_params makes of the first row's parameters, read by the host
+void own_row(const ws_batch* b, ws::OwnRow& o) {
+    ws::LeanRowParams& P = o.P;
+    P.inv_t = b->inv_t[0];
+    P.top_k = b->top_k ? b->top_k[0] : 0u;
+    P.race = b->race && b->race[0];
+    P.top_p = b->top_p ? b->top_p[0] : 1.0;
+    P.min_p = b->min_p ? b->min_p[0] : 0.0;
+    P.h0 = b->hist ? b->hist_off[0] : 0u;
+    P.nh = b->hist ? (b->hist_len ? b->hist_len[0] : b->hist_off[1] - P.h0) : 0u;
+    P.b0 = b->bias_ids ? b->bias_off[0] : 0u;
+    P.nb = b->bias_ids ? b->bias_off[1] - P.b0 : 0u;
+    P.seed = b->seed[0];
+    P.step = b->step[0];
+    P.rep = b->rep ? b->rep[0] : 1.f;
+    P.pres = b->pres ? b->pres[0] : 0.f;
+    P.freq = b->freq ? b->freq[0] : 0.f;
+    o.n_ids = P.nh <= ws::kOwnIds && P.nh <= b->max_hist ? P.nh : 0u;  // (a row with more than the batch declares: its ids are not read)
+    if (o.n_ids) std::memcpy(o.ids, b->hist + P.h0, o.n_ids * sizeof(int32_t));
+}
+
+int notify_on(void* stream, const ws_batch* b, uint32_t* done, uint32_t value, bool host_inputs) {
     if (!done) return WS_E_INVALID;
     const BatchPlan p = plan_for(b, b ? b->workspace_bytes : 0);
     if (p.err != WS_OK) return p.err;
     unsigned char* work = static_cast<unsigned char*>(b->workspace);
-    if (const int e = sample_batch_on(stream, b, p, work, b->workspace_bytes, done, value); e != WS_OK) return e;
-    if (p.few_parts && split_fits(p, work, b->workspace_bytes)) return WS_OK;  // (that kernel writes the words itself)
+    const bool few = p.few_parts && split_fits(p, work, b->workspace_bytes), with_row = host_inputs && few && b->rows == 1u;
+    ws::OwnRow own;
+    if (with_row) own_row(b, own);
+    if (const int e = sample_batch_on(stream, b, p, work, b->workspace_bytes, done, value, with_row ? &own : nullptr); e != WS_OK) return e;
+    if (few) return WS_OK;  // (that kernel writes the words itself)
     if (!b->rows) return WS_OK;
     for (uint32_t r = 0; r + 1u < b->rows; ++r) done[r] = value;
     return static_cast<int>(hipStreamWriteValue32(S(stream), done + b->rows - 1u, value, 0));
 }
+}  // namespace
+
+int ws_sample_batch_notify(void* stream, const ws_batch* b, uint32_t* done, uint32_t value) { return notify_on(stream, b, done, value, false); }
+
+int ws_sample_batch_notify_host(void* stream, const ws_batch* b, uint32_t* done, uint32_t value) { return notify_on(stream, b, done, value, true); }
 
 int ws_sample_batch_static(void* stream, const ws_batch* b) {
     const BatchPlan p = plan_for(b, sizeof(scratch));
@@ -957,6 +987,11 @@ int accept_sampled_on(void* stream, const ws_accept* b, bool fresh) {
     hipLaunchKernelGGL(fresh ? ws::accept_sampled_kernel<true> : ws::accept_sampled_kernel<false>, dim3(b->n_seq), dim3(64), 0, S(stream), a);
     return done();
 }
+}  // namespace
+
+int ws_accept_sampled(void* stream, const ws_accept* b) { return accept_sampled_on(stream, b, false); }
+
+int ws_accept_sampled_fresh(void* stream, const ws_accept* b) { return accept_sampled_on(stream, b, true); }
 
 int ws_accept_greedy(void* stream, const ws_accept_greedy_args* b) {
     if (!b || !b->ctl_all || !b->area || !b->row0 || !b->n_accepted || !b->chosen || !b->status || b->n_seq == 0) return WS_E_INVALID;
@@ -987,11 +1022,6 @@ int ws_accept_greedy(void* stream, const ws_accept_greedy_args* b) {
 int ws_history_stage(void* stream, const ws_history_stage_args* b) {
     if (!b || !b->hist.tokens || !history_ok(b->hist) || !b->ctl_all || !b->area || !b->row0 || !b->hist_off || !b->hist_len || !b->status ||
         b->n_seq == 0)
-}  // namespace
-
-int ws_accept_sampled(void* stream, const ws_accept* b) { return accept_sampled_on(stream, b, false); }
-
-int ws_accept_sampled_fresh(void* stream, const ws_accept* b) { return accept_sampled_on(stream, b, true); }
         return WS_E_INVALID;
     if (b->step && !b->hist.n_gen) return WS_E_INVALID;
     ws::StageArgs a{};

@@ -428,8 +428,9 @@ __device__ __forceinline__ uint64_t* few_sort(uint64_t* list, uint32_t n_keys, F
 
 // LDS: [0, 32 KiB) the list, [32 KiB, 64 KiB) its sorted copy while it is short; the history counts from 32 KiB on (they are
 // dead by then).
-template <int DT, bool MASKED, int NV>
-__device__ __forceinline__ bool few_row(const BatchArgs& A, const uint32_t row, const uint32_t part, FewShared& F, bool& finisher) {
+// OWN: the row's parameters are those of `own` (kernel arguments behind the batch's).
+template <int DT, bool MASKED, int NV, bool OWN>
+__device__ __forceinline__ bool few_row(const BatchArgs& A, const OwnRow* own, const uint32_t row, const uint32_t part, FewShared& F, bool& finisher) {
     extern __shared__ __align__(16) unsigned char lds[];
     constexpr uint32_t TPV = DT == 0 ? 4u : 8u;  // tokens in a 128-bit vector
     static_assert(NV * TPV * WS_BLOCK <= kFewWide, "tokens a share");
@@ -470,7 +471,7 @@ __device__ __forceinline__ bool few_row(const BatchArgs& A, const uint32_t row, 
     }
 
     // ---- the row's parameters
-    const LeanRowParams P = load_row_params(A, row);
+    const LeanRowParams P = OWN ? own->P : load_row_params(A, row);
     WSS_MARK(0);  // parameters in
     const float inv_t = P.inv_t;
     const uint32_t top_k = P.top_k, nh = P.nh, nb = P.nb, n_all = nh + nb;
@@ -497,7 +498,10 @@ __device__ __forceinline__ bool few_row(const BatchArgs& A, const uint32_t row, 
         atomicOr(&named[(b >> 5) * WS_BLOCK + w * 64u + r / TPV % 64u], 1u << (b & 31u));
     };
     if (any_ext) {
-        const int32_t* hist_ids = A.hist + P.h0;
+        typedef const __attribute__((address_space(1))) int32_t* Ids;
+        Ids hist_ids = (Ids)(A.hist + P.h0);
+        if (OWN && own->n_ids)  // uniform
+            hist_ids = (Ids)((uintptr_t)(const __attribute__((address_space(4))) void*)__builtin_amdgcn_kernarg_segment_ptr() + sizeof(BatchArgs) + offsetof(OwnRow, ids));
         const int32_t* bias_ids = A.bias_ids + P.b0;
         const float* bias_vals = A.bias_vals + P.b0;
         constexpr uint32_t kR = 4u;  // entries a thread at a time, their loads together
@@ -509,7 +513,7 @@ __device__ __forceinline__ bool few_row(const BatchArgs& A, const uint32_t row, 
             for (uint32_t r = 0; r < kR; ++r) {
                 const uint32_t j = j0 + r * WS_BLOCK + t;
                 id[r] = 0xffffffffu;
-                if (j0 + r * WS_BLOCK < n && j < n) id[r] = static_cast<uint32_t>((BIAS ? bias_ids : hist_ids)[j]);
+                if (j0 + r * WS_BLOCK < n && j < n) id[r] = static_cast<uint32_t>(BIAS ? bias_ids[j] : hist_ids[j]);
             }
             if (first) __syncthreads();  // the counts are clear
 #pragma unroll
@@ -677,13 +681,13 @@ __device__ __forceinline__ bool few_row(const BatchArgs& A, const uint32_t row, 
     return true;
 }
 
-template <int DT, bool MASKED, int NV>
-__global__ void __launch_bounds__(WS_BLOCK) few_batch_kernel(BatchArgs A) {
+template <int DT, bool MASKED, int NV, bool OWN>
+__device__ __forceinline__ void few_batch(const BatchArgs& A, const OwnRow* own) {
     __shared__ FewShared shared;
     uint32_t row, part;
     if (!few_place(A.few_together, A.rows, row, part)) return;
     bool finisher;
-    if (!few_row<DT, MASKED, NV>(A, row, part, shared, finisher) && finisher) {
+    if (!few_row<DT, MASKED, NV, OWN>(A, own, row, part, shared, finisher) && finisher) {
         __syncthreads();
         LeanArgPtr Ap = (LeanArgPtr)__builtin_amdgcn_kernarg_segment_ptr();
         asm volatile("" : "+s"(Ap));
@@ -695,6 +699,16 @@ __global__ void __launch_bounds__(WS_BLOCK) few_batch_kernel(BatchArgs A) {
         __syncthreads();
         if (threadIdx.x == 0) __hip_atomic_store(&A.done[row], A.done_value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
     }
+}
+template <int DT, bool MASKED, int NV>
+__global__ void __launch_bounds__(WS_BLOCK) few_batch_kernel(BatchArgs A) {
+    few_batch<DT, MASKED, NV, false>(A, nullptr);
+}
+// A lone row whose parameters and ids lie in host memory: as arguments they come with the launch, where the kernel above makes two trips over the bus, one behind
+// the other, before it knows its touched tokens (a decode step of 151936 tokens and 256 ids through the host API: 19.4 -> 16.6 us, of 19471 and 958 19.8 -> 17.2).
+template <int DT, int NV>
+__global__ void __launch_bounds__(WS_BLOCK) few_own_kernel(BatchArgs A, OwnRow own) {
+    few_batch<DT, false, NV, true>(A, &own);
 }
 
 }  // namespace ws

@@ -254,15 +254,6 @@ __device__ __forceinline__ void bucket_sort_desc(uint64_t* keys, uint32_t n, uin
     __syncthreads();
 }
 
-// a row's parameters as the scalar loads at the top of lean_row leave them
-struct LeanRowParams {
-    double top_p, min_p;
-    uint64_t seed, step;
-    float inv_t, rep, pres, freq;
-    uint32_t top_k, h0, nh, b0, nb;
-    bool race;
-};
-
 // Every one of a row's parameters with one scalar load, all asked for together and waited for once. (Written as plain reads
 // they become vector loads, each behind the test of its pointer and each waited for on its own: a dozen trips to memory one
 // after the other.) An absent array is read at the kernel's argument segment instead and the value dropped.

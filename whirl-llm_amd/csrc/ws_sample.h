@@ -110,6 +110,24 @@ struct BatchArgs {
     float code_above;             // .. by so many units of the exponent
 };
 
+// a row's parameters as load_row_params (ws_lean.h) leaves them
+struct LeanRowParams {
+    double top_p, min_p;
+    uint64_t seed, step;
+    float inv_t, rep, pres, freq;
+    uint32_t top_k, h0, nh, b0, nb;
+    bool race;
+};
+// A lone row whose parameters the host knows, as they travel with the launch (ws_few.h): and its history ids, if they fit (n_ids of them; else 0, and they
+// are read where the batch has them). Arguments of 4 KB in all at most.
+constexpr uint32_t kOwnIds = 768u;
+struct OwnRow {
+    LeanRowParams P;
+    uint32_t n_ids;
+    int32_t ids[kOwnIds];
+};
+static_assert(sizeof(BatchArgs) + sizeof(OwnRow) <= 4096u && sizeof(BatchArgs) % alignof(OwnRow) == 0u, "kernel arguments");
+
 // Global memory of a split row: the merged histogram, the merged candidate list, and four control words (parts that
 // have merged their histogram, parts that are done with the shared state, candidates listed, the row maximum as an
 // ordered integer).

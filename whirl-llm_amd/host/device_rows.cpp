@@ -3,8 +3,8 @@
 // a sort of the kept candidates on the host; prefetchRows does the launch for several rows at once.
 // No vocabulary-sized work happens here unless the device flags the row.
 // Parameters, penalty lists, results and kept sets live in pinned host memory that the device addresses directly
-// (hipHostMalloc): the host writes the few hundred bytes a row needs, the kernel reads them over the bus, writes what
-// it kept straight back and then a word the host looks at (ws_sample_batch_notify), and no copy command sits before or after
+// (hipHostMalloc): the host writes the few hundred bytes a row needs, the kernel reads them over the bus (a lone row's come with the
+// launch), writes what it kept straight back and then a word the host looks at (ws_sample_batch_notify_host), and no copy command sits before or after
 // the launch - a decode step is one launch and one wait for that word, which comes some 5 us before a stream wait would end.
 // Everything here has waited for what it launched before it returns, so the host never rewrites a block that a launch
 // still reads.
@@ -336,7 +336,7 @@ void DeviceRows::filterOnDevice(const Sampler& s, std::uint32_t gr0, std::uint32
     b.workspace = d.work.at;
     b.workspace_bytes = d.work.bytes;
     d.in_flight = true;
-    check(ws_sample_batch_notify(stream_, &b, d.done, ++d.turn), "ws_sample_batch");
+    check(ws_sample_batch_notify_host(stream_, &b, d.done, ++d.turn), "ws_sample_batch");
     waitForRows(n);  // results and kept sets are in host memory now
     d.in_flight = false;
     const Dev::ResultView& h = o;
