@@ -86,6 +86,26 @@ def test_other_vocabularies(V):
     print(res)
 
 
+@pytest.mark.parametrize("V,masked,lists", [(V, masked, lists) for V in (8193, 8195, 16386, 20481, 32771, 50257, 71348, 102397, 102398, 102399, 151937, 163837, 163839)
+                                            for masked in (False, True) for lists in (False, True)
+                                            if lists or V >= (32768 if masked else 20480)])  # (shorter rows without lists are swept three times)
+def test_rows_off_every_boundary(V, masked, lists):
+    """Rows of any length, which begin at any address: those that end inside a vector, one token either side of a round; with touched tokens, the largest
+    logits and masked-out tokens in the last vector, and mask bits set behind the row's end."""
+    c = _no_top_k(gc.make_cfg2(rows=6, V=V, n_hist=700 if lists else 0, n_bias=50 if lists else 0))
+    c["top_p"] = np.minimum(c["top_p"], 0.95)
+    rng = np.random.default_rng(V)
+    for r in range(6):
+        if lists:
+            c["hist"][r][:2] = [V - 1, V - 1 - r % 4]
+        c["logits"][r, V - 1 - (r * 3) % 8] = 9.0 + r
+    if masked:
+        c["allow"] = rng.integers(0, 1 << 32, (6, (V + 31) // 32), dtype=np.uint64).astype(np.uint32) | np.uint32(0x10000001)
+        c["logits"][:2, :500:40] = 14.0  # (some of them masked out: far above the others)
+    res, _ = run_lean(c, 1, handed_back=2 if masked else 1)
+    assert res["exact"] == 6, res
+
+
 def test_no_history_no_bias_no_penalties():
     c = _no_top_k(gc.make_cfg2(rows=8, V=151936, n_hist=0, n_bias=0))
     res, _ = run_lean(c, 0, handed_back=1)

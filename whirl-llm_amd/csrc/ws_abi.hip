@@ -338,9 +338,18 @@ BatchPlan plan_batch(const ws_batch* b, bool few = true) {
 #endif
     // Its rows are those without a top-k, and a batch says so by leaving `top_k` out: a row with one would be handed
     // back to the three-pass code inside the launch, at twice the time of the kernel that takes a top-k in its stride.
-    p.lean = p.fused && b->dtype == WS_DTYPE_F32 && b->mode == WS_MODE_AUTO && !b->top_k && !b->kept_ids && !b->query_prob && !wants_entropy && !b->race &&
-             fused_total + kStaticLean <= kMaxLds;
+    // It reads rows at any address. Rows that are not whole aligned vectors, which the other single-sweep kernels do not take, are swept three times otherwise, and
+    // that is the faster way only for short ones (us, three sweeps and this kernel; N(0, 2) and rows of raised tokens):
+    //   without lists, 1 row:  of 9001 17.6 / 19.4, 16387 19.1 / 19.5, 20011 21.0 / 19.6 and 19.7 / 19.7, 50257 28.7 / 22.0, 151937 49.1 / 32.1
+    //                256 rows: of 9001 19.7 / 20.3, 16387 23.3 / 20.7 and 21.7 / 20.7, 50257 37.9 / 25.2, 151937 67.1 / 40.0
+    //     masked,      1 row:  of 20011 21.1 / 22.4, 32003 23.5 / 23.0 and 23.0 / 23.9;  256 rows of 20011 24.0 / 26.3, 32003 29.5 / 25.4
+    //   with histories of 16 to 3400 ids: 1 row of 9001 22.2 / 22.2 and 21.3 / 22.0, 50257 38.7 / 24.5; 256 rows of 8003 27.0 / 23.0, 151937 77.9 / 42.8
+    const uint32_t lean_least = vec_rows ? 8u : (cap ? 8192u : (b->allow ? 32768u : 20480u));
+    p.lean = (p.fused || !vec_rows) && b->dtype == WS_DTYPE_F32 && b->mode == WS_MODE_AUTO && !b->top_k && !b->kept_ids && !b->query_prob && !wants_entropy && !b->race &&
+             b->vocab >= lean_least && b->vocab <= 163840u && (!b->bias_ids || b->max_bias <= 2047u) && fused_total + kStaticLean <= kMaxLds;
     if (p.lean) {
+        p.lds_ab = 65536u;
+        p.lds_cnt = static_cast<uint32_t>(65536u + maps);
         uint64_t lt = fused_total;
         p.lean_tie = 0;
         if (lt + 32768u + kStaticLean <= kMaxLds) {
@@ -418,7 +427,7 @@ BatchPlan plan_batch(const ws_batch* b, bool few = true) {
     }
     // The kernels without a bin cache (long vocabularies, unaligned rows) take the touched tokens' raw logits from
     // their first sweep when they have somewhere to put them: 8 bytes per history / bias entry and row.
-    if (!p.fused && cap > 0 && b->mode == WS_MODE_AUTO) p.workspace = uint64_t{b->rows} * ws::capture_row_bytes(p.patch_cap);
+    if (!p.fused && !p.lean && cap > 0 && b->mode == WS_MODE_AUTO) p.workspace = uint64_t{b->rows} * ws::capture_row_bytes(p.patch_cap);
     p.err = WS_OK;
     return p;
 }
