@@ -341,7 +341,7 @@ __device__ __forceinline__ bool code_row(const BatchArgs& A, const uint32_t row,
     auto look_at_head = [&](const uint4& v) __attribute__((always_inline)) {
         const CodePair a = __builtin_elementwise_min(code_pair(v.x, last), code_pair(v.y, last)), b = __builtin_elementwise_min(code_pair(v.z, last), code_pair(v.w, last));
         const CodePair c = __builtin_elementwise_min(a, b);
-        const uint32_t first = wave_min_u32(min(static_cast<uint32_t>(c.x), static_cast<uint32_t>(c.y)));
+        const uint32_t first = wave_min_u32_apart(min(static_cast<uint32_t>(c.x), static_cast<uint32_t>(c.y)));
         if (lane == 0u) atomicMin(&S.head_bin, first);
     };
     auto count_round = [&](const int c) __attribute__((always_inline)) {
@@ -535,7 +535,7 @@ __device__ __forceinline__ bool code_row(const BatchArgs& A, const uint32_t row,
                 pos[r] = static_cast<uint16_t>(atomicAdd(&g_cnt[g], 1u));
             }
         }
-        best = wave_max_u32(best);
+        best = ~wave_min_u32_apart(~best);
         if (lane == 0u && best) atomicMax(&S.top_key, best);
     }
     if (TOUCHED) __syncthreads();
@@ -571,7 +571,7 @@ __device__ __forceinline__ bool code_row(const BatchArgs& A, const uint32_t row,
     }
     const uint32_t ext = TOUCHED ? g_cnt[t] : 0u;
     const bool wave_has = __ballot(own + ext != 0u) != 0ull;
-    first = wave_has ? wave_min_u32(first) : kCodeBins;
+    first = wave_has ? wave_min_u32_apart(first) : kCodeBins;
     if (lane == 0u && first < kCodeBins) atomicMin(&S.top_bin, first);
     __syncthreads();
     const float m = fmaxf(S.top_bin < kCodeTail ? code_value(S.top_bin) : -INFINITY, S.top_key ? unkey32(S.top_key) : -INFINITY);

@@ -146,6 +146,21 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
     return last_lane(v);
 }
 #undef WS_WAVE_FOLD
+// The same in steps between which the compiler puts other work: where a wave has some (ws_code.h's, whose row is on its way: 256 rows of 151936, Zipfian, with the
+// folds above 40.0 us and with these 39.5).
+template <int CTRL, int ROW_MASK>
+__device__ __forceinline__ uint32_t dpp_or_self(uint32_t v) {
+    return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(static_cast<int>(v), static_cast<int>(v), CTRL, ROW_MASK, 0xf, false));
+}
+__device__ __forceinline__ uint32_t wave_min_u32_apart(uint32_t v) {
+    v = min(v, dpp_or_self<0x111, 0xf>(v));
+    v = min(v, dpp_or_self<0x112, 0xf>(v));
+    v = min(v, dpp_or_self<0x114, 0xf>(v));
+    v = min(v, dpp_or_self<0x118, 0xf>(v));
+    v = min(v, dpp_or_self<0x142, 0xa>(v));
+    v = min(v, dpp_or_self<0x143, 0xc>(v));
+    return last_lane(v);
+}
 __device__ __forceinline__ float wave_sum(float v) { return last_lane(wave_incl_scan(v)); }
 __device__ __forceinline__ double wave_sum(double v) { return last_lane(wave_incl_scan(v)); }
 __device__ __forceinline__ uint32_t wave_sum(uint32_t v) { return last_lane(wave_incl_scan(v)); }
