@@ -22,7 +22,7 @@
 // work (threshold, sums, publishing) is paid half as often, and a share still fits the registers. Measured against the
 // short-list kernel's shared rows (151936 fp32, microseconds a launch): one row, top-k 40: 20.6 -> 11.9; 64 rows of mixed
 // filters with 4096-id histories: 50 (126 when a row's min-p list ran over) -> 32.5; 32 rows of 50257, which went through
-// the three-pass kernel: 55.6 -> 15.4. Since then 11.8 -> 10.3, 30.8 -> 26.8 and 15.6 -> 14.5: a bit a token for those that lists name and a look a vector
+// the three-pass kernel: 55.6 -> 15.4. Since then 11.8 -> 9.9, 31.6 -> 28.4 and 15.6 -> 14.3: a bit a token for those that lists name and a look a vector
 // for those to list (64 rows 8 %, 40 rows 12 %), the waves' maxima and thresholds by a third of the instructions, the last part's exponentials by a quarter,
 // its places in the list by one addition a wave (one row 9 %), and a row's parts on one chiplet (1 to 2 %; 6 % of a row whose parameters come over the bus).
 #pragma once

@@ -5,7 +5,7 @@
 // whose last part counted the merged list once more (151936 fp32, microseconds a launch): 8 rows, K = 256: 19.6 -> 13.3;
 // a draft draw of 8 rows: 26.0 -> 11.6, of which the draw's one wave took 7 and takes 2.5. Since then 13.3 -> 11.8 (top_select, and what ws_few.h names), and of
 // the draw's one wave 6.5 K clocks -> 4.4 K: its parameters are asked for at the start, its sums end with the candidates, and the logarithms of the race
-// keys are another wave's. (A cycle of 8 sequences and 4 drafts, with its verification: 81.1 us -> 68.3.)
+// keys are another wave's. (A cycle of 8 sequences and 4 drafts, with its verification: 81.1 us -> 68.3, and 61.4 with ws_accept.h's kernels as they are.)
 #pragma once
 #include "ws_draft.h"
 #include "ws_few.h"
