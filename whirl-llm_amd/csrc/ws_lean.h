@@ -532,7 +532,7 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const uint32_t row,
                 vm = fmaxf(vm, x);                                                                                                           \
                 const float tc = bin_coord(aq, c64, x, tail_f);                                                                              \
                 bins[e] = static_cast<uint32_t>(tc);                                                                                         \
-                WSL_HIST_ADD(bins[e], tc);                                                                                                   \
+                atomicAdd(reinterpret_cast<unsigned long long*>(&myhist[bins[e]]), bin_word(tc));                                            \
             }                                                                                                                                \
             const uint32_t lo2 = __builtin_amdgcn_perm(bins[1], bins[0], 0x0c0c0400u);                                                       \
             uint32_t packed = __builtin_amdgcn_perm(bins[3], bins[2], 0x04000c0cu) | lo2;                                                    \
@@ -551,17 +551,6 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const uint32_t row,
             }                                                                                                                        \
         }                                                                                                                            \
     }
-#ifndef WS_EXP_NOATOMIC
-#define WSL_HIST_ADD(bin, tc) atomicAdd(reinterpret_cast<unsigned long long*>(&myhist[bin]), bin_word(tc))
-#else
-#define WSL_HIST_ADD(bin, tc) m = fmaxf(m, __uint_as_float(static_cast<uint32_t>(bin_word(tc))))
-#endif
-#ifndef WS_EXP_NOLOAD
-#define WSL_NEXT_LOAD(bt, slot) \
-    if ((bt) + kRing < NB) load((bt) + kRing, slot) /* the slot is free: the batch three ahead */
-#else
-#define WSL_NEXT_LOAD(bt, slot)
-#endif
     // ------------------------------------------------------------------ phase 0 (ws_sample.h): bitmap of the touched ids,
     // popcount prefix per word (rank of a touched id), per-rank history count and bias entries
     uint32_t n_touched = 0;
@@ -656,13 +645,10 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const uint32_t row,
 #pragma unroll
             for (int u = 0; u < kLeanBatch; ++u) cache[bt * kLeanBatch + u] = 0u;
         }
-        WSL_NEXT_LOAD(bt, bt % kRing);
+        if (bt + kRing < NB) load(bt + kRing, bt % kRing);  // the slot is free: the batch three ahead
     }
     if (t < 128) s_exp[t] = exp_tab;
 #undef WSL_SWEEP_BATCH
-#undef WSL_HIST_ADD
-#undef WSL_NEXT_LOAD
-    if (t < 128) s_exp[t] = exp_tab;
     __syncthreads();
     WSL_MARK(2);
     // Everything behind the sweep reads its arguments again, through a pointer the compiler cannot see through: none of
@@ -1539,16 +1525,11 @@ template <bool MASKED>
 __global__ void __launch_bounds__(WS_BLOCK) lean_batch_kernel(BatchArgs A) {
     __shared__ LeanShared shared;
     const uint32_t row = blockIdx.x;
-    const bool done = lean_row<MASKED>(A, row, shared);
-#ifndef WS_LEAN_NO_FALLBACK
-    if (done) return;
+    if (lean_row<MASKED>(A, row, shared)) return;
     __syncthreads();  // whatever the lean path left in LDS is dead
     LeanArgPtr Ap = (LeanArgPtr)__builtin_amdgcn_kernarg_segment_ptr();
     asm volatile("" : "+s"(Ap));
     three_pass_row<false>(Ap, row);
-#else
-    if (!done && threadIdx.x == 0) A.token[row] = -2;
-#endif
 }
 
 }  // namespace ws
