@@ -1502,22 +1502,22 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const uint32_t row,
 }
 
 // the three-pass code of ws_sample.h for one row, a function of its own: its registers and code stay out of the lean path.
-// It takes the kernel's argument segment and makes its own copy of the arguments with the three-pass layout of the LDS
-// (a copy made by the kernel would be made at the kernel's entry, on every row).
+// It takes the kernel's argument segment, and reads there where the three-pass layout of the LDS lies (RowLayout).
+// What it is handed comes in vector registers; said to be one value for the whole wave, so that everything that follows from it is scalar again. Not a tail
+// call: only then does the compiler leave out saving the callers' registers, which nobody reads any more - thirty-five scalar registers went to memory one by one,
+// each a round trip of a vector register that had to be free for it, and back at the end: 30 us of every handed-back row. (Before that, the arguments once
+// copied, and now, us: one row of 50257 without a filter 75 / 44, the same beside 255 others with one 94 / 54, ten rows of 256 of 151937 with sigma / T = 8
+// 137 / 95; ws_sample.h's own kernel takes 40, 48 and 88.)
 typedef const __attribute__((address_space(4))) BatchArgs* LeanArgPtr;
 template <bool KEPT>  // (KEPT: the build that can write the kept-set dump)
-__device__ __noinline__ void three_pass_row(LeanArgPtr Ap, const uint32_t row) {
-    BatchArgs B;
-    __builtin_memcpy(&B, (const void*)Ap, sizeof(BatchArgs));
-    B.lds_ab = B.fb_lds_ab;
-    B.lds_cnt = 0u;
-    B.lds_tie = B.fb_lds_tie;
-    B.two_sweep = 1;
-    B.work = nullptr;
-    B.split_log2 = 0u;
-    sample_row<false, false, KEPT>(B, row);
+__device__ __noinline__ __attribute__((not_tail_called)) void three_pass_row(LeanArgPtr Ap, const uint32_t row_) {
+    const uint64_t at = reinterpret_cast<uint64_t>(Ap);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(at)), hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(at >> 32));
+    const uint32_t row = __builtin_amdgcn_readfirstlane(row_);
+    const BatchArgs& A = *(const BatchArgs*)reinterpret_cast<LeanArgPtr>((static_cast<uint64_t>(hi) << 32) | lo);
+    sample_row<false, false, KEPT, true>(A, row);
     __syncthreads();  // (the row's flags are written by whichever thread finished it)
-    if (threadIdx.x == 0) B.flags[row] |= kRouteHandedBack;
+    if (threadIdx.x == 0) A.flags[row] |= kRouteHandedBack;
 }
 
 // MASKED: the batch has an allow mask (a kernel of its own: one build carrying both paths spilled far more registers)
