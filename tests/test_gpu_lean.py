@@ -204,3 +204,50 @@ def test_same_answers_as_the_kernel_that_takes_a_top_k():
     assert differ <= 2, differ
     assert torch.equal(a.stats[:, 0], b.stats[:, 0])
     assert torch.allclose(a.prob[sure], b.prob[sure], rtol=1e-6, atol=0)
+
+
+def _ragged(kind, sigma, V, rows, seed):
+    """Rows of V tokens on the GPU: N(0, sigma), a few tokens raised to 10 .. 14, or Zipfian."""
+    g = torch.Generator(device="cuda:0").manual_seed(seed)
+    x = torch.empty((rows, V), device="cuda:0").normal_(0.0, sigma, generator=g)
+    if kind == "raised":
+        ids = torch.randint(0, V, (rows, 20), device="cuda:0", generator=g)
+        x.scatter_(1, ids, torch.empty((rows, 20), device="cuda:0").uniform_(10.0, 14.0, generator=g))
+    elif kind == "zipf":
+        base = -1.1 * torch.log(torch.arange(1, V + 1, device="cuda:0", dtype=torch.float32))
+        x += base[torch.rand((rows, V), device="cuda:0", generator=g).argsort(dim=1)]
+    return x, torch.empty(rows, device="cuda:0").uniform_(0.7, 1.7, generator=g)
+
+
+def _sampled(x, inv_t, **more):
+    m, rows = gc.pkg(), x.shape[0]
+    steps = torch.arange(rows, dtype=torch.int64, device="cuda:0")
+    return m.BatchSampler(x, inv_t, steps * 77 + 5, steps, top_p=torch.full((rows,), 0.9, dtype=torch.float64, device="cuda:0"), rng=1, max_split=1, **more).run()
+
+
+@pytest.mark.parametrize("kind,sigma,V", [("normal", 3.0, 50257), ("normal", 1.5, 20483), ("raised", 2.0, 151937), ("raised", 3.0, 99991), ("zipf", 0.4, 151937)])
+def test_normaliser_as_close_as_three_sweeps(kind, sigma, V):
+    """Rows off every boundary, whose masses come from the bins: no further from 64 bits than where the same rows are swept three times (a kept-set dump takes
+    them there), and the same number on nearly every row - both count from eight units above the row's head, and only the order of the 64-bit sums is another.
+    The rows whose maximum lies above that (the three sweeps take it for the anchor then) are looked at by themselves: a coordinate of up to 256 is off by
+    2^-17, a mass by 2^-17 / 64 = 1.2e-7 at most, and the result's own rounding is 6e-8."""
+    m = gc.pkg()
+    x, inv_t = _ragged(kind, sigma, V, 128, V)
+    a, b = _sampled(x, inv_t), _sampled(x, inv_t, kept_cap=8)
+    torch.cuda.synchronize()
+    lean = (a.flags & m.FLAG_ROUTE_MASK) == m.FLAG_ROUTE_LEAN
+    assert int(lean.sum()) >= 120 and ((b.flags & m.FLAG_ROUTE_LEAN) == 0).all()
+    top = x.double().amax(1, keepdim=True)
+    z = torch.exp((x.double() - top) * inv_t.double()[:, None]).sum(1)
+    off = [s.stats[:, 1].double() / z - 1.0 for s in (a, b)]
+    lies = (top[:, 0] - x[:, :8192].double().amax(1)) * inv_t.double()
+    below, over = lean & (lies < 7.9), lean & (lies >= 7.9)
+    assert int(below.sum()) >= 64
+    rms = [float(o[below].square().mean().sqrt()) for o in off]
+    assert rms[0] <= 1.05 * rms[1] + 2e-9, rms
+    assert float((a.stats[below, 1] == b.stats[below, 1]).double().mean()) >= 0.95
+    if over.any():
+        assert float(off[0][over].abs().max()) <= 1.2e-7 + 6e-8
+    same = below & (((a.flags | b.flags) & m.FLAG_NEAR) == 0)
+    assert int(same.sum()) >= 32 and torch.equal(a.n_kept[same], b.n_kept[same]) and torch.equal(a.token[same], b.token[same])
+    print(kind, V, rms)

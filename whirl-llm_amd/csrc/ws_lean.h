@@ -35,20 +35,42 @@ constexpr uint32_t kLeanBuckets = 128u;   // words of the finish's tables in Lea
 constexpr uint32_t kLeanMaxList = 4096u;  // candidates of a row's ranges together: what the sort's 32 KiB hold
 // The bins the cut and the draw can fall in: as many as have eight different cache bytes, sixteen at most.
 constexpr uint32_t kLeanMaxBins = 16u;
-// Bins are counted down from an anchor this many units of the exponent above the largest of the row's first tokens
-// (the row's maximum may lie up to 16 above it before the row is handed back). Eight were too few for peaked rows: with
-// logits of sigma 4 at T = 0.5 the maximum of 151936 tokens lies 4.8 units above that of the first 8192 on average, and
-// more than 8 on a quarter of the rows.
-constexpr float kLeanAbove = 12.f;
+// A token's coordinate is measured from where ws_sample.h measures it, an anchor this many units of the exponent above the largest of the row's first tokens;
+// the bins begin kLeanRoom of them, four units, above the anchor, where coordinates are below zero. The room is for peaked rows: with logits of sigma 4 at T = 0.5
+// the maximum of 151936 tokens lies 4.8 units above that of the first 8192 on average, and more than 8 on a quarter of the rows. (Measured from
+// the first bin, tokens four to eight units below the head's largest have a bit less of their coordinate in 32 bits, and the mass that is taken from it has too. Rms error
+// of a normaliser against 64 bits, in 1e-8, from the first bin / from the anchor / ws_sample.h: 50257 tokens of N(0, 3) at T = 0.6 14.3 / 9.4 / 9.4,
+// 151937 of raised tokens 8.5 / 4.9 / 4.9, Zipfian 7.4 / 5.4 / 5.4; the sweep takes the same instructions either way.)
+constexpr float kLeanAbove = 8.f;
+constexpr int kLeanRoom = 256;
 // A range may span this many bins when few of them hold a token (the draw's range on a peaked row: two tokens fifty
 // bins apart); its bins then share the range's eight slots of the sort in order, several to a slot.
 constexpr uint32_t kLeanWide = 1024u;
-// The first bin of this kernel's tail, 48 units of the exponent below the anchor: the last 1024 bins, one to a thread,
+// The first bin of this kernel's tail, 48 units of the exponent below the first bin: the last 1024 bins, one to a thread,
 // take the tokens below that and the masked-out ones. (A scan of the bin cache for a bin finds the tokens of the tail
 // bins with the same cached bits as well: spread over 1024 bins, a 256th of the tail's tokens at most. In 64 bins a
 // row with nine tokens in ten masked out had up to a sixteenth of them found with every bin it asked for.)
 constexpr int kLeanTail = 3072;
-  // WS_FLAG_ROUTE_THREE_PASS
+
+// A token's height, bin_coord's coordinate with its sign turned round: what is above the anchor is above zero. What lies beyond the bins is put at their ends,
+// NaN at `low`, a negative number (of three values with a NaN among them the instruction takes the smallest).
+__device__ __forceinline__ float lean_height(float aq, float c64, float x, float low) {
+    return __builtin_amdgcn_fmed3f(__fmaf_rn(x, c64, -aq), low, static_cast<float>(kLeanRoom));
+}
+// its bin, counted from the anchor's: -kLeanRoom is the first (a floor and a conversion would be two instructions)
+__device__ __forceinline__ int lean_bin(float height) {
+    int b;
+    asm("v_cvt_flr_i32_f32 %0, -%1" : "=v"(b) : "v"(height));
+    return b;
+}
+// the same, and the histogram's word; at_anchor: the anchor's. (In one block: behind a written-out instruction the compiler puts a pause before the next that
+// reads its result.)
+typedef __attribute__((address_space(3))) uint64_t* LeanWord;
+__device__ __forceinline__ int lean_bin(float height, LeanWord at_anchor, LeanWord& word) {
+    int b;
+    asm("v_cvt_flr_i32_f32 %0, -%2\n\tv_lshl_add_u32 %1, %0, 3, %3" : "=&v"(b), "=v"(word) : "v"(height), "v"(at_anchor));
+    return b;
+}
 
 #ifdef WS_PHASE_TIMERS
 #define WSL_FAIL(code)                                                                                   \
@@ -458,9 +480,9 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const uint32_t row,
     }
     WSL_MARK(0);
 
-    // ------------------------------------------------------------------ the anchor: the head of the row + 8 exponent units
+    // ------------------------------------------------------------------ the anchor: the head of the row + kLeanAbove exponent units
     const float c64 = inv_t * 64.f;
-    float anchor, aq;
+    float aq;
     {
         float s = -INFINITY, allowed = -INFINITY;
 #pragma unroll
@@ -477,7 +499,7 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const uint32_t row,
         if (MASKED) block_max2(s, allowed, red_f, reinterpret_cast<float*>(red_u));
         else s = block_max(s, red_f);
         // (of the allowed tokens, where there are any: one that is masked out may lie so far above the others that their masses would be lost)
-        anchor = (MASKED && allowed > -INFINITY ? allowed : s) + kLeanAbove / inv_t;
+        const float anchor = (MASKED && allowed > -INFINITY ? allowed : s) + kLeanAbove / inv_t;
         aq = anchor_product(anchor, c64);
         if (!(anchor > -INFINITY && anchor < INFINITY)) WSL_FAIL(2);
     }
@@ -486,8 +508,8 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const uint32_t row,
     uint32_t cache[kLeanRegs];
     float m = -INFINITY;
     float vm_early[kEarly * kLeanBatch];  // maxima of the early batches' vectors, until the bitmap says which hold a touched token
-    const float tail_f = static_cast<float>(kLeanTail + static_cast<int>(t));  // this thread's own tail bin
-    uint64_t* myhist = (hist2 && (t & 1u)) ? hist2 : hist;
+    const float tail_f = static_cast<float>(kLeanRoom - kLeanTail - static_cast<int>(t));  // the height of this thread's own tail bin
+    const LeanWord at_anchor = (LeanWord)(((hist2 && (t & 1u)) ? hist2 : hist) + kLeanRoom);
     const uint32_t stage_cap = 2047u;
     const uint32_t n_full = (V >> kTokLog) / WS_BLOCK;  // rounds of whole vectors for every thread
     bool any_touched = false;               // uniform
@@ -524,16 +546,18 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const uint32_t row,
             const uint32_t w[4] = {q[slot][u].x, q[slot][u].y, q[slot][u].z, q[slot][u].w};                                          \
             const int32_t bw = MASKED ? static_cast<int32_t>(nal >> ((j * kTok) & 31u)) : 0;                                         \
             float vm = -INFINITY;                                                                                                    \
-            uint32_t bins[4];                                                                                                                \
+            int bins[4];                                                                                                                     \
             _Pragma("unroll") for (int e = 0; e < 4; ++e) {                                                                                  \
                 uint32_t bits = w[e];                                                                                                        \
                 if (MASKED) bits |= static_cast<uint32_t>((bw << (31 - e)) >> 31);                                                           \
                 const float x = __uint_as_float(bits);                                                                                       \
                 vm = fmaxf(vm, x);                                                                                                           \
-                const float tc = bin_coord(aq, c64, x, tail_f);                                                                              \
-                bins[e] = static_cast<uint32_t>(tc);                                                                                         \
-                atomicAdd(reinterpret_cast<unsigned long long*>(&myhist[bins[e]]), bin_word(tc));                                            \
+                const float h = lean_height(aq, c64, x, tail_f);                                                                             \
+                LeanWord word;                                                                                                               \
+                bins[e] = lean_bin(h, at_anchor, word);                                                                                      \
+                __hip_atomic_fetch_add(word, bin_word(-h), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);                                  \
             }                                                                                                                                \
+            /* (kLeanRoom is a multiple of 256: the low bytes are those of the histogram's indices) */                                       \
             const uint32_t lo2 = __builtin_amdgcn_perm(bins[1], bins[0], 0x0c0c0400u);                                                       \
             uint32_t packed = __builtin_amdgcn_perm(bins[3], bins[2], 0x04000c0cu) | lo2;                                                    \
             asm volatile("" : "+v"(packed)); /* (packed here, not where the tail first looks at it: four bins would stay live) */            \
@@ -668,7 +692,8 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const uint32_t row,
     float ma = -INFINITY, mu = -INFINITY;
     if (n_touched) {
         constexpr uint32_t kClaim = 0x80000000u;
-        const float tail_own = static_cast<float>(kLeanTail + static_cast<int>(t));
+        uint64_t* const anchors = hist + kLeanRoom;
+        const float tail_own = static_cast<float>(kLeanRoom - kLeanTail - static_cast<int>(t));
         const uint32_t stage_cap = 2047u;
         // K ids a thread and pass (a pass with nothing in its later slots would still issue their instructions)
         auto take = [&](auto kc, const int32_t* ids, uint32_t n, uint32_t j0, const uint32_t* kept_id) __attribute__((always_inline)) {
@@ -733,9 +758,9 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const uint32_t row,
                     pv[rk[k]] = x;
                     first[rk[k]] = i;  // the token id of the rank from here on
                     ma = fmaxf(ma, x);
-                    const float t0 = bin_coord(aq, c64, raw, tail_own), t1 = bin_coord(aq, c64, x, tail_own);
-                    atomicAdd(reinterpret_cast<unsigned long long*>(&hist[static_cast<uint32_t>(t0)]), 0ull - bin_word(t0));
-                    atomicAdd(reinterpret_cast<unsigned long long*>(&hist[static_cast<uint32_t>(t1)]), bin_word(t1));
+                    const float from = lean_height(aq, c64, raw, tail_own), to = lean_height(aq, c64, x, tail_own);
+                    atomicAdd(reinterpret_cast<unsigned long long*>(&anchors[lean_bin(from)]), 0ull - bin_word(-from));
+                    atomicAdd(reinterpret_cast<unsigned long long*>(&anchors[lean_bin(to)]), bin_word(-to));
                 }
             }
         };
@@ -757,12 +782,15 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const uint32_t row,
         float m_all = fmaxf(fmaxf(m, mu), ma);
         m = block_max(m_all, red_f);  // its barriers also end the moves in the histogram
     }
-    if (!(m <= anchor && (anchor - m) * c64 <= 1024.f)) WSL_FAIL(3);  // (also a row without any token: m = -inf)
+    {  // the sweep stands if no token lies above the first bin and that one is not wastefully high (and not on a row without any token: m = -inf)
+        const float above = __fmaf_rn(m, c64, -aq);
+        if (!(above <= static_cast<float>(kLeanRoom) && above >= static_cast<float>(kLeanRoom - 1024))) WSL_FAIL(3);
+    }
 
     // ------------------------------------------------------------------ scan of the histogram: four consecutive bins a thread,
     // the prefixes stay in registers
-    const double lift = static_cast<double>(aq) * (1.0 / 64.0) - static_cast<double>(m) * static_cast<double>(inv_t);  // >= 0
-    if (wv == 0u) {  // one wave: the factor that takes masses from the anchor to the maximum
+    const double lift = (static_cast<double>(aq) + kLeanRoom) * (1.0 / 64.0) - static_cast<double>(m) * static_cast<double>(inv_t);  // >= 0
+    if (wv == 0u) {  // one wave: the factor that takes masses from the first bin to the maximum
         const double tm = exp(lift);
         if (lane == 0u) s_d[7] = tm;
     }
@@ -1095,8 +1123,9 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const uint32_t row,
     constexpr uint32_t kListCap = 4096u;
     const uint32_t u0 = static_cast<uint32_t>(r0lo), w0 = nb0 - 1u;
     const uint32_t u1r = has_r1 ? static_cast<uint32_t>(r1lo) : 0xffff0000u, w1 = has_r1 ? nb1 - 1u : 0u;
+    auto bin_at = [&](float x) { return static_cast<uint32_t>(lean_bin(lean_height(aq, c64, x, static_cast<float>(kLeanRoom - 4095))) + kLeanRoom); };
     auto in_ranges = [&](float x) {
-        const uint32_t b = bin_of(aq, c64, x);
+        const uint32_t b = bin_at(x);
         return b - u0 <= w0 || b - u1r <= w1;
     };
     {
@@ -1171,7 +1200,7 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const uint32_t row,
     const uint32_t sh1 = nb1 > 8u ? 29u - static_cast<uint32_t>(__clz(static_cast<int>(nb1 - 1u))) : 0u;
     const uint32_t ns0 = ((nb0 - 1u) >> sh0) + 1u, ns1 = has_r1 ? ((nb1 - 1u) >> sh1) + 1u : 0u;  // slots of the ranges
     auto slot_of = [&](float x) {
-        const uint32_t b = static_cast<uint32_t>(bin_coord(aq, c64, x));
+        const uint32_t b = bin_at(x);
         const bool in1 = has_r1 && b - static_cast<uint32_t>(r1lo) < nb1;
         const uint32_t s_ = in1 ? (r1_first ? 0u : ns0) + ((b - static_cast<uint32_t>(r1lo)) >> sh1) : (r1_first ? ns1 : 0u) + ((b - static_cast<uint32_t>(r0lo)) >> sh0);
         return min(s_, kLeanMaxBins - 1u);
