@@ -251,3 +251,41 @@ def test_normaliser_as_close_as_three_sweeps(kind, sigma, V):
     same = below & (((a.flags | b.flags) & m.FLAG_NEAR) == 0)
     assert int(same.sum()) >= 32 and torch.equal(a.n_kept[same], b.n_kept[same]) and torch.equal(a.token[same], b.token[same])
     print(kind, V, rms)
+
+
+@pytest.mark.parametrize("V", [50257, 151936, 151937])
+@pytest.mark.parametrize("lists,masked", [(False, False), (True, False), (True, True)])
+def test_maximum_above_the_bins_is_swept_once_more(V, lists, masked):
+    """Rows whose maximum lies 11 to 31 units of the exponent above the largest of their first 8192 tokens - a token late in the row, alone or with others just
+    below it - are read a second time by the same code when it is more than 12, and not handed back. Their masses are as good as any: the
+    second sweep counts from the maximum."""
+    m = gc.pkg()
+    units = [11.0, 13.0, 16.0, 20.0, 25.0, 31.0]
+    c = _no_top_k(gc.make_cfg2(rows=6, V=V, n_hist=400 if lists else 0, n_bias=40 if lists else 0))
+    c["top_p"] = np.minimum(c["top_p"], 0.95)
+    c["min_p"][:] = 0.0
+    if masked:
+        rng = np.random.default_rng(V)
+        c["allow"] = rng.integers(0, 1 << 32, (6, (V + 31) // 32), dtype=np.uint64).astype(np.uint32)
+    for r in range(6):
+        late = V - 5 - 40 * r
+        allowed = np.unpackbits(c["allow"][r].view(np.uint8), bitorder="little")[:8192].astype(bool) if masked else np.ones(8192, bool)
+        head = float(c["logits"][r, :8192][allowed].max())
+        for j in range(6 if r % 2 else 1):
+            at = late - 7 * j
+            c["logits"][r, at] = head + (units[r] - 0.4 * j) / float(c["inv_t"][r])
+            if masked:
+                c["allow"][r, at >> 5] |= np.uint32(1 << (at & 31))
+            if lists:  # (nothing moves these tokens)
+                c["hist"][r][c["hist"][r] == at] = 0
+                c["bias_ids"][r][c["bias_ids"][r] == at] = 0
+    res, smp = run_lean(c, 1)
+    fl = smp.flags.cpu().numpy()
+    assert res["exact"] == 6 and res["handed_back"] == 0, res
+    again = (fl & m.FLAG_ROUTE_REDONE) != 0
+    assert not again[0] and again[1:].all(), fl
+    x = torch.from_numpy(c["logits"]).double()
+    if not lists:
+        z = torch.exp((x - x.amax(1, keepdim=True)) * torch.from_numpy(c["inv_t"]).double()[:, None]).sum(1).numpy()
+        off = smp.stats[:, 1].cpu().numpy().astype(np.float64) / z - 1.0
+        assert np.abs(off[again]).max() <= 2.4e-7, off  # (coordinates below 512: 2^-16 / 64 at most, and the result's rounding is 6e-8)

@@ -43,6 +43,11 @@ constexpr uint32_t kLeanMaxBins = 16u;
 // 151937 of raised tokens 8.5 / 4.9 / 4.9, Zipfian 7.4 / 5.4 / 5.4; the sweep takes the same instructions either way.)
 constexpr float kLeanAbove = 8.f;
 constexpr int kLeanRoom = 256;
+// A row whose maximum lies above the first bin is swept once more, from its maximum down (lean_rest): a second sweep where three would be made. Up to
+// this far above the anchor, that is: a maximum further up is a lone token with next to no mass below it, and such a row is handed back. (us, handed back / swept once more: ten rows
+// of 256 of 151937 with sigma / T = 8 95 / 67, 86 of 256 of raised tokens at T = 0.6 100 / 62, 18 of 256 of 50257 54 / 42. More room for the bins instead would take
+// masses from coordinates of up to 1024, at a fourth of their precision.)
+constexpr int kLeanFar = 1536;
 // A range may span this many bins when few of them hold a token (the draw's range on a peaked row: two tokens fifty
 // bins apart); its bins then share the range's eight slots of the sort in order, several to a slot.
 constexpr uint32_t kLeanWide = 1024u;
@@ -76,6 +81,7 @@ __device__ __forceinline__ int lean_bin(float height, LeanWord at_anchor, LeanWo
 #define WSL_FAIL(code)                                                                                   \
     do {                                                                                                 \
         if (threadIdx.x == 0 && A.entropy) A.entropy[row * 32 + 28] = (code) + 100.0 * sel_dbg(S);       \
+        if (threadIdx.x == 0) S.top = __uint_as_float(0x7fc00000u);                                      \
         return false;                                                                                    \
     } while (0)
 #define WSL_MARK(k)                                                \
@@ -83,7 +89,11 @@ __device__ __forceinline__ int lean_bin(float height, LeanWord at_anchor, LeanWo
         if (threadIdx.x == 0) S.marks[(k)] = clock64() - wsl_t0;   \
     } while (0)
 #else
-#define WSL_FAIL(code) return false
+#define WSL_FAIL(code)                                                 \
+    do {                                                               \
+        if (threadIdx.x == 0u) S.top = __uint_as_float(0x7fc00000u);   \
+        return false;                                                  \
+    } while (0)
 #define WSL_MARK(k) \
     do {            \
     } while (0)
@@ -282,9 +292,11 @@ __device__ __forceinline__ void bucket_sort_desc(uint64_t* keys, uint32_t n, uin
 // Every one of a row's parameters with one scalar load, all asked for together and waited for once. (Written as plain reads
 // they become vector loads, each behind the test of its pointer and each waited for on its own: a dozen trips to memory one
 // after the other.) An absent array is read at the kernel's argument segment instead and the value dropped.
-__device__ __forceinline__ LeanRowParams load_row_params(const BatchArgs& A, const uint32_t row) {
+// args: the kernel's argument segment.
+typedef const __attribute__((address_space(4))) BatchArgs* LeanArgPtr;
+__device__ __forceinline__ LeanRowParams load_row_params(const BatchArgs& A, const uint32_t row, const LeanArgPtr args) {
     LeanRowParams P;
-    const uint64_t dummy = reinterpret_cast<uint64_t>((const __attribute__((address_space(4))) void*)__builtin_amdgcn_kernarg_segment_ptr());
+    const uint64_t dummy = reinterpret_cast<uint64_t>(args);
     auto at = [&](const void* base, uint64_t byte_off) { return base ? reinterpret_cast<uint64_t>(base) + byte_off : dummy; };
     const uint64_t r4 = static_cast<uint64_t>(row) * 4u, r8 = static_cast<uint64_t>(row) * 8u;
     const uint64_t p_inv_t = at(A.inv_t, r4), p_top_k = at(A.top_k, r4), p_race = at(A.race, r4), p_top_p = at(A.top_p, r8), p_min_p = at(A.min_p, r8);
@@ -332,6 +344,10 @@ __device__ __forceinline__ LeanRowParams load_row_params(const BatchArgs& A, con
     return P;
 }
 
+__device__ __forceinline__ LeanRowParams load_row_params(const BatchArgs& A, const uint32_t row) {
+    return load_row_params(A, row, (LeanArgPtr)__builtin_amdgcn_kernarg_segment_ptr());
+}
+
 // what wave 0 works out from the searches' answers for everybody
 struct LeanSel {
     double X, m0base, m1base;
@@ -361,6 +377,7 @@ struct LeanShared {
     uint32_t s_w[16];
     uint32_t red_u[WS_WAVES];
     float red_f[WS_WAVES];
+    float top;  // what lean_row leaves when it returns false
 #ifdef WS_PHASE_TIMERS
     long long marks[32];
 #endif
@@ -369,9 +386,10 @@ struct LeanShared {
 #ifdef WS_PHASE_TIMERS
 __device__ __forceinline__ double sel_dbg(const LeanShared& S) { return S.sel.n_r0 + 1e5 * S.sel.n_r1 + 1e10 * (S.sel.r0hi - S.sel.r0lo + 1) + 1e12 * (S.sel.r1hi - S.sel.r1lo + 1); }
 #endif
-// One row. Returns false when the row is left to the three-pass code (nothing has been written for it then).
-template <bool MASKED>
-__device__ __forceinline__ bool lean_row(const BatchArgs& A, const uint32_t row, LeanShared& S) {
+// One row. Returns false when the row is left to others (nothing has been written for it then): S.top is NaN, and it is the three-pass code's; or the row's maximum,
+// and it is to be swept once more from there down (AGAIN; its arguments are at `args`).
+template <bool MASKED, bool AGAIN>
+__device__ __forceinline__ bool lean_row(const BatchArgs& A, const LeanArgPtr args, const uint32_t row, LeanShared& S) {
     constexpr uint32_t kTok = 4u, kTokLog = 2u;  // tokens in a 128-bit vector, which is one register of the bin cache: the low eight bits of each bin
     // (a scan for a bin also finds the tokens of the bins 256 apart, some hundreds each, and drops them afterwards)
 #ifdef WS_PHASE_TIMERS
@@ -447,7 +465,7 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const uint32_t row,
         }
     }
 
-    const LeanRowParams P = load_row_params(A, row);
+    const LeanRowParams P = load_row_params(A, row, AGAIN ? args : (LeanArgPtr)__builtin_amdgcn_kernarg_segment_ptr());
     const float inv_t = P.inv_t;
     const uint32_t top_k = P.top_k;
     const bool race = P.race;
@@ -499,7 +517,7 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const uint32_t row,
         if (MASKED) block_max2(s, allowed, red_f, reinterpret_cast<float*>(red_u));
         else s = block_max(s, red_f);
         // (of the allowed tokens, where there are any: one that is masked out may lie so far above the others that their masses would be lost)
-        const float anchor = (MASKED && allowed > -INFINITY ? allowed : s) + kLeanAbove / inv_t;
+        const float anchor = AGAIN ? S.top : (MASKED && allowed > -INFINITY ? allowed : s) + kLeanAbove / inv_t;
         aq = anchor_product(anchor, c64);
         if (!(anchor > -INFINITY && anchor < INFINITY)) WSL_FAIL(2);
     }
@@ -678,8 +696,7 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const uint32_t row,
     // Everything behind the sweep reads its arguments again, through a pointer the compiler cannot see through: none of
     // them stays in a register across the sweep (they spilled there, dozens of them, and every phase paid for it).
     // (the kernel's argument segment itself, where BatchArgs is the first and only argument: scalar loads, no copy)
-    typedef const __attribute__((address_space(4))) BatchArgs* ArgPtr;
-    ArgPtr Ap = (ArgPtr)__builtin_amdgcn_kernarg_segment_ptr();
+    LeanArgPtr Ap = AGAIN ? args : (LeanArgPtr)__builtin_amdgcn_kernarg_segment_ptr();
     asm volatile("" : "+s"(Ap));
     const float rep = P.rep, pres = P.pres, freq = P.freq;
     const int32_t* hist_ids2 = Ap->hist + h0;
@@ -784,7 +801,11 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const uint32_t row,
     }
     {  // the sweep stands if no token lies above the first bin and that one is not wastefully high (and not on a row without any token: m = -inf)
         const float above = __fmaf_rn(m, c64, -aq);
-        if (!(above <= static_cast<float>(kLeanRoom) && above >= static_cast<float>(kLeanRoom - 1024))) WSL_FAIL(3);
+        if (!(above <= static_cast<float>(kLeanRoom) && above >= static_cast<float>(kLeanRoom - 1024))) {
+            if (AGAIN || !(m > -INFINITY && above <= static_cast<float>(kLeanFar))) WSL_FAIL(3);
+            if (t == 0u) S.top = m;
+            return false;
+        }
     }
 
     // ------------------------------------------------------------------ scan of the histogram: four consecutive bins a thread,
@@ -1496,7 +1517,7 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const uint32_t row,
             if (mg_min_p < tol) flags |= kNearMinP;
             if (mg < tol) flags |= kNearDraw;
             Ap->token[row] = static_cast<int32_t>(cid[r]);
-            Ap->flags[row] = flags | kRouteLean;
+            Ap->flags[row] = flags | kRouteLean | (AGAIN ? kRouteRedone : 0u);
             if (Ap->prob) Ap->prob[row] = static_cast<float>(cem[r] / Zk);
             if (Ap->margin) Ap->margin[3 * row + 2] = mg;
         }
@@ -1508,7 +1529,7 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const uint32_t row,
             if (mg_top_p < tol) flags |= kNearTopP;
             if (mg_min_p < tol) flags |= kNearMinP;
             Ap->token[row] = static_cast<int32_t>(0xffffffffu - static_cast<uint32_t>(s_q[4]));
-            Ap->flags[row] = flags | kRouteLean;
+            Ap->flags[row] = flags | kRouteLean | (AGAIN ? kRouteRedone : 0u);
             if (Ap->prob) Ap->prob[row] = static_cast<float>(s_d[1] / Zk);
             if (Ap->margin) Ap->margin[3 * row + 2] = 0.0;
         }
@@ -1537,16 +1558,31 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const uint32_t row,
 // each a round trip of a vector register that had to be free for it, and back at the end: 30 us of every handed-back row. (Before that, the arguments once
 // copied, and now, us: one row of 50257 without a filter 75 / 44, the same beside 255 others with one 94 / 54, ten rows of 256 of 151937 with sigma / T = 8
 // 137 / 95; ws_sample.h's own kernel takes 40, 48 and 88.)
-typedef const __attribute__((address_space(4))) BatchArgs* LeanArgPtr;
-template <bool KEPT>  // (KEPT: the build that can write the kept-set dump)
-__device__ __noinline__ __attribute__((not_tail_called)) void three_pass_row(LeanArgPtr Ap, const uint32_t row_) {
+__device__ __forceinline__ LeanArgPtr wave_args(LeanArgPtr Ap) {
     const uint64_t at = reinterpret_cast<uint64_t>(Ap);
     const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(at)), hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(at >> 32));
+    return reinterpret_cast<LeanArgPtr>((static_cast<uint64_t>(hi) << 32) | lo);
+}
+template <bool KEPT>  // (KEPT: the build that can write the kept-set dump)
+__device__ __noinline__ __attribute__((not_tail_called)) void three_pass_row(LeanArgPtr Ap, const uint32_t row_) {
     const uint32_t row = __builtin_amdgcn_readfirstlane(row_);
-    const BatchArgs& A = *(const BatchArgs*)reinterpret_cast<LeanArgPtr>((static_cast<uint64_t>(hi) << 32) | lo);
+    const BatchArgs& A = *(const BatchArgs*)wave_args(Ap);
     sample_row<false, false, KEPT, true>(A, row);
     __syncthreads();  // (the row's flags are written by whichever thread finished it)
     if (threadIdx.x == 0) A.flags[row] |= kRouteHandedBack;
+}
+
+// What lean_row has left of a row. (A function of its own, as above: as a loop around that code in the kernel it cost the kernel some hundred spilled registers.)
+template <bool MASKED>
+__device__ __noinline__ __attribute__((not_tail_called)) void lean_rest(LeanArgPtr Ap_, const uint32_t row_, __attribute__((address_space(3))) LeanShared* S) {
+    LeanArgPtr Ap = wave_args(Ap_);
+    const uint32_t row = __builtin_amdgcn_readfirstlane(row_);
+    const float top = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(S->top)));
+    if (top == top) {
+        if (lean_row<MASKED, true>(*(const BatchArgs*)Ap, Ap, row, *(LeanShared*)S)) return;
+        __syncthreads();
+    }
+    three_pass_row<false>(Ap, row);
 }
 
 // MASKED: the batch has an allow mask (a kernel of its own: one build carrying both paths spilled far more registers)
@@ -1554,11 +1590,11 @@ template <bool MASKED>
 __global__ void __launch_bounds__(WS_BLOCK) lean_batch_kernel(BatchArgs A) {
     __shared__ LeanShared shared;
     const uint32_t row = blockIdx.x;
-    if (lean_row<MASKED>(A, row, shared)) return;
+    if (lean_row<MASKED, false>(A, nullptr, row, shared)) return;
     __syncthreads();  // whatever the lean path left in LDS is dead
     LeanArgPtr Ap = (LeanArgPtr)__builtin_amdgcn_kernarg_segment_ptr();
     asm volatile("" : "+s"(Ap));
-    three_pass_row<false>(Ap, row);
+    lean_rest<MASKED>(Ap, row, (__attribute__((address_space(3))) LeanShared*)&shared);
 }
 
 }  // namespace ws
