@@ -289,3 +289,23 @@ def test_maximum_above_the_bins_is_swept_once_more(V, lists, masked):
         z = torch.exp((x - x.amax(1, keepdim=True)) * torch.from_numpy(c["inv_t"]).double()[:, None]).sum(1).numpy()
         off = smp.stats[:, 1].cpu().numpy().astype(np.float64) / z - 1.0
         assert np.abs(off[again]).max() <= 2.4e-7, off  # (coordinates below 512: 2^-16 / 64 at most, and the result's rounding is 6e-8)
+
+
+@pytest.mark.parametrize("V", [50256, 50257, 151937])
+@pytest.mark.parametrize("lists", [False, True])
+def test_rows_without_any_filter(V, lists):
+    """A batch that has neither a top-p nor a min-p is nothing for this kernel, which would hand back every row. Rows off the vector boundaries go straight to
+    the three sweeps, with the workspace that takes their touched tokens' logits; the others to the single-sweep kernel."""
+    m = gc.pkg()
+    c = _no_top_k(gc.make_cfg2(rows=5, V=V, n_hist=600 if lists else 0, n_bias=30 if lists else 0))
+    c["top_p"][:], c["min_p"][:] = 1.0, 0.0
+    d = gc.upload(c, hints=True)
+    d["top_p"] = d["min_p"] = None
+    d["min_p_min"] = 0.0
+    smp = gc.sampler_for(c, d, 1, max_split=1).run()
+    res = gc.compare_rows(c, smp, range(5), 1, check_kept=False)
+    assert res["exact"] + res["differ"] == 5 and res["differ"] <= 1, res
+    assert not (smp.flags & (m.FLAG_ROUTE_LEAN | m.FLAG_ROUTE_HANDED_BACK)).any(), smp.flags
+    use = m.lib().ws_sample_batch_workspace_use(smp.desc)
+    tables = lists and V % 8 != 0
+    assert use == (m.WORK_TABLES if tables else m.WORK_NONE) and (not tables or smp.workspace.numel() >= 5 * 8 * 630)

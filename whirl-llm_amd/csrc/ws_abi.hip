@@ -344,8 +344,11 @@ BatchPlan plan_batch(const ws_batch* b, bool few = true) {
     //                256 rows: of 9001 19.7 / 20.3, 16387 23.3 / 20.7 and 21.7 / 20.7, 50257 37.9 / 25.2, 151937 67.1 / 40.0
     //     masked,      1 row:  of 20011 21.1 / 22.4, 32003 23.5 / 23.0 and 23.0 / 23.9;  256 rows of 20011 24.0 / 26.3, 32003 29.5 / 25.4
     //   with histories of 16 to 3400 ids: 1 row of 9001 22.2 / 22.2 and 21.3 / 22.0, 50257 38.7 / 24.5; 256 rows of 8003 27.0 / 23.0, 151937 77.9 / 42.8
+    //     masked too (180 shapes): 8192 to 12000 tokens 5 % slower here, to 16000 2 %, from there on faster, 27 % of the longest
+    // Rows without a filter are none of its own either: of a batch that has neither top-p nor min-p it would hand back every one (three sweeps and this kernel: 1 row of
+    // 50257 40 / 44, 256 rows 51 / 61, 256 of 151937 with 500 ids 117 / 125; the other single-sweep kernel and this one: 256 rows of 50256 52 / 61, of 151936 87 / 109).
     const uint32_t lean_least = vec_rows ? 8u : (cap ? 8192u : (b->allow ? 32768u : 20480u));
-    p.lean = (p.fused || !vec_rows) && b->dtype == WS_DTYPE_F32 && b->mode == WS_MODE_AUTO && !b->top_k && !b->kept_ids && !b->query_prob && !wants_entropy && !b->race &&
+    p.lean = (p.fused || !vec_rows) && (b->top_p || b->min_p) && b->dtype == WS_DTYPE_F32 && b->mode == WS_MODE_AUTO && !b->top_k && !b->kept_ids && !b->query_prob && !wants_entropy && !b->race &&
              b->vocab >= lean_least && b->vocab <= 163840u && (!b->bias_ids || b->max_bias <= 2047u) && fused_total + kStaticLean <= kMaxLds;
     if (p.lean) {
         p.lds_ab = 65536u;
