@@ -42,7 +42,7 @@ def kernels(tmp_path_factory):
         path = tmp_path_factory.mktemp("co") / f"{i}.elf"
         path.write_bytes(blob)
         names = re.findall(r"\.text\s+\S+\s+\S*\s*(\S+)$", subprocess.run([OBJDUMP, "-t", str(path)], capture_output=True, text=True, check=True).stdout, re.M)
-        names = [n for n in names if re.search(r"few_batch_kernel|topk_rows_shared|dflash_topk_shared|draft_sample_rows_shared|spec_verify_kernel|short_batch_kernelILi[01]ELb[01]ELb1E", n) and not n.endswith(".kd")]
+        names = [n for n in names if re.search(r"few_batch_kernel|few_own_kernel|topk_rows_shared|dflash_topk_shared|draft_sample_rows_shared|spec_verify_kernel|short_batch_kernelILi[01]ELb[01]ELb1E", n) and not n.endswith(".kd")]
         if not names:
             continue
         text = subprocess.run([OBJDUMP, "-d", "--no-show-raw-insn", f"--disassemble-symbols={','.join(names)}", str(path)], capture_output=True, text=True, check=True).stdout
@@ -64,8 +64,8 @@ def before_the_ticket(code):
 
 
 def test_stores_have_arrived_before_the_ticket_is_drawn(kernels):
-    # dtype x mask x size of the few-row sampler; three kernels of three sizes; the classic verification; the short-list kernel's shared rows
-    assert len(kernels) == 16 + 9 + 1 + 4, sorted(kernels)
+    # dtype x mask x size of the few-row sampler, and its two for a row that comes with the launch; three kernels of three sizes; the classic verification; the short-list kernel's shared rows
+    assert len(kernels) == 16 + 2 + 9 + 1 + 4, sorted(kernels)
     for name, code in kernels.items():
         back = before_the_ticket(code)
         assert "s_barrier" in back, name
