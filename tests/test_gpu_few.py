@@ -122,6 +122,34 @@ def test_ties_at_the_threshold_and_a_row_of_one_value():
     run(c, handed_back=3)
 
 
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("V,masked,by_p", [(32771, False, False), (50257, True, False), (32768, False, True), (151937, True, True)])
+def test_nan_of_either_kind_and_infinities_are_no_candidates(V, masked, by_p, dtype):
+    """NaN, quiet and signalling, of either sign: in the vectors of the row's largest tokens, on tokens that the lists name, all over a wave's chunk and at
+    the row's end; -inf in between, also at named tokens; and +inf under the mask. All of them count for -inf, none hands its row back."""
+    c = case(3, V, dtype, top_k=0 if by_p else 40, min_p=0.3 if by_p else 0.0, n_hist=900, n_bias=64, allowed=0.5 if masked else None)
+    rng = np.random.default_rng(V)
+    bits = c["logits"].view(np.uint32 if dtype == "f32" else np.uint16)
+    sh, per = (16, 4) if dtype == "f32" else (0, 8)
+    quiet, signalling, low = 0x7FC0 << sh, 0x7F81 << sh, 0xFF80 << sh
+    one_bit = signalling if dtype == "bf16" else 0x7F800001  # (a signalling NaN whose only set bit is the last)
+    kinds = np.array([quiet, quiet | 0x8000 << sh, signalling, signalling | 0x8000 << sh, one_bit, low], dtype=bits.dtype)
+    c["bias_vals"][:] = np.minimum(c["bias_vals"], 1.0)
+    for r in range(3):
+        top = np.argsort(gc.row_f32(c, r))[-60:]
+        beside = top[top // per * per + (top + 1) % per < V]
+        beside = beside // per * per + (beside + 1) % per  # another token of the vector
+        named = np.concatenate([c["hist"][r][::5], c["bias_ids"][r][::3]])
+        chunk = np.arange(7 * 8 * per, 15 * 8 * per)  # whole chunks of eight lanes: a wave's only vectors in a load
+        spoilt = np.concatenate([np.setdiff1d(beside, top[-50:]), named, chunk, rng.integers(0, V, 300), [V - 1 - r, V - 2 - r]])
+        bits[r, spoilt] = kinds[rng.integers(0, kinds.size, spoilt.size)]
+        if masked:
+            out = np.flatnonzero(~np.unpackbits(c["allow"][r].view(np.uint8), bitorder="little")[:V].astype(bool))
+            bits[r, out[rng.integers(0, out.size, 40)]] = 0x7F80 << sh
+            bits[r, np.intersect1d(out, c["hist"][r])[:5]] = 0x7F80 << sh
+    run(c, max_differ=1 if dtype == "bf16" else 0)
+
+
 @pytest.mark.parametrize("inv_t", [0.7, 1.25])
 def test_the_waves_sums_meet_in_64_bits(inv_t):
     """128 tokens, every one a different wave's only one (a wave's own sum is exactly one), so that the normaliser is made of the
