@@ -117,7 +117,7 @@ int ws_draft_sample_rows(void* stream, const float* x, int n, int* ctl_all, cons
                          const ws_dsamp_args* a, int* qbuf, unsigned rows);
 /* ws_draft_sample_rows with a workspace (same launch site): the draft head's rows come one draft position after the
  * other, a few rows at a time, so each launch leaves most of the GPU idle and its latency is paid up to 15 times a
- * cycle; with a workspace each row is shared by 2 to 16 workgroups (as ws_topk_rows_ws, K = 32). Same candidates; the
+ * cycle; with a workspace each row, of any length from 4096 tokens on, is shared by 2 to 16 workgroups. Same candidates; the
  * normaliser is summed in another order, so q's probabilities may differ in their last bits (the reference's own sum
  * depends on the order of its atomics). workspace: ws_draft_sample_rows_workspace() bytes (0: not split), 8-byte
  * aligned, zero-filled once, one launch at a time; without it this is ws_draft_sample_rows. */
@@ -279,7 +279,9 @@ typedef struct ws_batch {
                                includes a staging area per row; memory that holds only the rows' meeting places, 65792
                                bytes a row, still lets them be shared; short-list rows ask for 65536 bytes, which the
                                kernel that holds them in registers needs, and are shared with 33536 as well);
-                               (b) rows of the kernels that sweep the row twice (long or unaligned vocabularies)
+                               (b) rows of the kernels that sweep the row twice (long vocabularies; rows that are not
+                               whole aligned vectors, except of the batches that the one-sweep kernel takes:
+                               WS_FLAG_ROUTE_LEAN; ws_sample_batch_workspace_use says which)
                                that have a history or a bias: the first sweep leaves the raw logits of those tokens
                                here (8 bytes per history / bias entry) instead of gathering them one by one, and
                                leaves the memory with arbitrary contents - zero-fill it again before a batch of
@@ -353,9 +355,9 @@ int ws_sample_batch(void* stream, const ws_batch* b);
  * once everything the launch writes is visible to the host. Looking at those words costs some 5 us less than a stream wait;
  * a caller that looks in vain asks the stream (hipStreamQuery) for an error. */
 int ws_sample_batch_notify(void* stream, const ws_batch* b, uint32_t* done, uint32_t value);
-/* The same for a caller whose parameters and lists (inv_t .. freq, hist, bias_*, their offsets) lie in host memory that the device reads in place
- * (hipHostMalloc) and are as they should be when the call is made: the call may read them too, and send a lone row's along with the
- * launch. They stay as they are until the words have come. */
+/* The same for a caller whose parameters and lists (every array of the batch that goes in but `logits` and `allow`: inv_t .. freq, race, hist, hist_off,
+ * hist_len, bias_*) lie in host memory that the device reads in place (hipHostMalloc) and are as they should be when the call is made: the call may read
+ * them too, and send a lone row's along with the launch. They stay as they are until the words have come. */
 int ws_sample_batch_notify_host(void* stream, const ws_batch* b, uint32_t* done, uint32_t value);
 /* ws_sample_batch for callers that cannot allocate device memory - code under HIP graph capture, tight serving loops,
  * harnesses that forbid it; it has no counterpart in the reference. The split rows of a small batch meet in memory that is

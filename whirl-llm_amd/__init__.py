@@ -312,7 +312,8 @@ def draft_pick_rows(x, ctl_all, area, r, n_min, p_min, vmap=None, workspace=None
 
 
 def draft_sample_rows(x, ctl_all, area, r, args, qbuf, vmap=None, workspace=None):
-    """args: list of per-row dicts (on, top_k, qoff, inv_t, top_p, min_p, key). workspace: as for topk_rows (K = 32)."""
+    """args: list of per-row dicts (on, top_k, qoff, inv_t, top_p, min_p, key). workspace: a zero-filled uint8
+    device tensor of ws_draft_sample_rows_workspace(n, rows) bytes kept between calls (0: such rows are not shared)."""
     _dev_f32(x)
     ri, da = _row_idx(area), _dsamp_args(args)
     if workspace is not None:
