@@ -87,11 +87,6 @@ __device__ __forceinline__ T wave_incl_scan(T v) {
     return v;
 }
 
-// the same steps with a lane's own value where there is no source: lane 63 ends with the reduction of the wave
-template <int CTRL, int ROW_MASK>
-__device__ __forceinline__ float dpp_or_self(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), CTRL, ROW_MASK, 0xf, false));
-}
 __device__ __forceinline__ uint32_t last_lane(uint32_t v) { return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), 63)); }
 __device__ __forceinline__ float last_lane(float v) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63)); }
 __device__ __forceinline__ uint64_t last_lane(uint64_t v) {
@@ -148,6 +143,7 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
 #undef WS_WAVE_FOLD
 // The same in steps between which the compiler puts other work: where a wave has some (ws_code.h's, whose row is on its way: 256 rows of 151936, Zipfian, with the
 // folds above 40.0 us and with these 39.5).
+// (dpp_or_self: a lane's own value where there is no source, so that lane 63 ends with the reduction of the wave)
 template <int CTRL, int ROW_MASK>
 __device__ __forceinline__ uint32_t dpp_or_self(uint32_t v) {
     return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(static_cast<int>(v), static_cast<int>(v), CTRL, ROW_MASK, 0xf, false));

@@ -196,7 +196,7 @@ __device__ __forceinline__ double exp_neg(double a, const double* s_exp) {
     return s_exp[n >> 6] * s_exp[64u + (n & 63u)] * p;
 }
 
-// e^-a, of either sign: 2^k e^r with |r| <= ln 2 / 2, the series to r^13 (two units in the last place; a quarter of the library's instructions).
+// e^-a, of either sign: 2^k e^r with |r| <= ln 2 / 2, the series to r^13 (0.9 units in the last place at most over 2e7 arguments; a quarter of the library's instructions).
 // The reduction is Cody and Waite's, with ln 2 in the two parts that Sun's public fdlibm (e_exp.c) gives it.
 __device__ __forceinline__ double code_exp(double a) {
     const double k = __builtin_rint(a * -1.44269504088896340736);
@@ -218,7 +218,8 @@ __device__ __forceinline__ double code_exp(double a) {
     p = fma(p, r, 1.0);
     return __builtin_amdgcn_ldexp(p, static_cast<int>(k));
 }
-// the same of any a that is not below zero (2^30 e-folds and more would not fit the exponent's integer)
+// the same of any a that is not below zero (2^30 e-folds and more would not fit the exponent's integer). NaN, which an infinite inverse temperature makes of
+// the maximum's own distance, counts as no mass: such a row's probability is 0 / 0, NaN all the same
 __device__ __forceinline__ double exp_down(double a) { return code_exp(fmin(a, 1e6)); }
 
 // One of four values by number. The values come in as arguments, every one of them read before the choice: a chain
