@@ -309,3 +309,21 @@ def test_rows_without_any_filter(V, lists):
     use = m.lib().ws_sample_batch_workspace_use(smp.desc)
     tables = lists and V % 8 != 0
     assert use == (m.WORK_TABLES if tables else m.WORK_NONE) and (not tables or smp.workspace.numel() >= 5 * 8 * 630)
+
+
+@pytest.mark.parametrize("V,ids,masked,lean", [
+    (8191, 128, False, False), (8193, 127, False, False), (8193, 128, False, True), (16383, 127, False, False), (16385, 1, False, True), (20477, 0, False, False),
+    (20481, 0, False, True), (8193, 511, True, False), (8193, 512, True, True), (20479, 511, True, False), (20481, 1, True, True), (32767, 0, True, False), (32769, 0, True, True)])
+def test_short_rows_off_the_boundaries(V, ids, masked, lean):
+    """Either side of the lengths from which rows that are not whole aligned vectors go this way: with no lists, with a few ids, with more; masked and not."""
+    m = gc.pkg()
+    c = _no_top_k(gc.make_cfg2(rows=3, V=V, n_hist=ids, n_bias=0))
+    c["top_p"], c["min_p"][:] = np.minimum(c["top_p"], 0.95), 0.0
+    if masked:
+        c["allow"] = np.random.default_rng(V).integers(0, 1 << 32, (3, (V + 31) // 32), dtype=np.uint64).astype(np.uint32)
+    d = gc.upload(c, hints=True)
+    d["min_p_min"] = 0.0
+    smp = gc.sampler_for(c, d, 1, max_split=1).run()
+    res = gc.compare_rows(c, smp, range(3), 1, check_kept=False)
+    assert res["exact"] == 3, res
+    assert (((smp.flags & m.FLAG_ROUTE_LEAN) != 0) == lean).all(), smp.flags

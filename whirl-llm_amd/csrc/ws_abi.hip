@@ -345,9 +345,12 @@ BatchPlan plan_batch(const ws_batch* b, bool few = true) {
     //     masked,      1 row:  of 20011 21.1 / 22.4, 32003 23.5 / 23.0 and 23.0 / 23.9;  256 rows of 20011 24.0 / 26.3, 32003 29.5 / 25.4
     //   with histories of 16 to 3400 ids: 1 row of 9001 22.2 / 22.2 and 21.3 / 22.0, 50257 38.7 / 24.5; 256 rows of 8003 27.0 / 23.0, 151937 77.9 / 42.8
     //     masked too (180 shapes): 8192 to 12000 tokens 5 % slower here, to 16000 2 %, from there on faster, 27 % of the longest
+    //     raised tokens, 16 ids: 1 row of 8193 21.5 / 22.6, 14003 22.2 / 22.5, 16387 22.9 / 22.5; 256 rows of 9001 23.7 / 24.3, 16387 level; 64 ids: 1 row of 8193 21.6 / 22.5,
+    //     12001 22.3 / 22.6, 16387 23.5 / 22.7; 256 ids: 1 row of 8193 23.3 / 22.7
+    //     masked, 64 ids: 1 row of 8193 22.9 / 24.8, 12001 23.7 / 25.4, 16387 24.8 / 25.7, 24001 27.8 / 25.7; 256 rows of 8193 24.7 / 27.6, 16387 28.8 / 27.4; 500 ids: level at 8193
     // Rows without a filter are none of its own either: of a batch that has neither top-p nor min-p it would hand back every one (three sweeps and this kernel: 1 row of
     // 50257 40 / 44, 256 rows 51 / 61, 256 of 151937 with 500 ids 117 / 125; the other single-sweep kernel and this one: 256 rows of 50256 52 / 61, of 151936 87 / 109).
-    const uint32_t lean_least = vec_rows ? 8u : (cap ? 8192u : (b->allow ? 32768u : 20480u));
+    const uint32_t lean_least = vec_rows ? 8u : (cap >= (b->allow ? 512u : 128u) ? 8192u : (cap ? (b->allow ? 20480u : 16384u) : (b->allow ? 32768u : 20480u)));
     p.lean = (p.fused || !vec_rows) && (b->top_p || b->min_p) && b->dtype == WS_DTYPE_F32 && b->mode == WS_MODE_AUTO && !b->top_k && !b->kept_ids && !b->query_prob && !wants_entropy && !b->race &&
              b->vocab >= lean_least && b->vocab <= 163840u && (!b->bias_ids || b->max_bias <= 2047u) && fused_total + kStaticLean <= kMaxLds;
     if (p.lean) {
