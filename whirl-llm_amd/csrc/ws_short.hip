@@ -15,21 +15,27 @@ const ShortKernel kShortKernels[2][2][2] = {{{short_batch_kernel<0, false, false
                                             {{short_batch_kernel<1, false, false>, short_batch_kernel<1, false, true>},
                                              {short_batch_kernel<1, true, false>, short_batch_kernel<1, true, true>}}};
 // The rows that ws_twin.h has left to the three-pass code: launched behind it, with as many workgroups as compute units at most.
-// (the flags of all of a workgroup's rows are read at once: one after the other they took 3 us of 1000 rows that all were done)
-__global__ void __launch_bounds__(WS_BLOCK) short_rest_kernel(BatchArgs A) {
-    const uint32_t n = gridDim.x;
-    bool any = false;
-    for (uint32_t row = blockIdx.x + threadIdx.x * n; row < A.rows; row += WS_BLOCK * n) any |= A.flags[row] == kTwinRest;
-    if (!__syncthreads_or(any)) return;
-    for (uint32_t row = blockIdx.x; row < A.rows; row += n) {
-        const bool left = A.flags[row] == kTwinRest;
+// (The flags of all of a workgroup's rows are read at once: one after the other they took 3 us of 1000 rows that all were done. The rows are a function's of their own: around
+// its calls no register keeps the thread's number, and in the kernel that was a trip to scratch memory at its very start, 0.4 us of launches that had nothing to do.)
+__device__ __noinline__ __attribute__((not_tail_called)) void short_rest(LeanArgPtr Ap_, const uint32_t n_) {
+    LeanArgPtr Ap = wave_args(Ap_);
+    const uint32_t n = __builtin_amdgcn_readfirstlane(n_);
+    for (uint32_t row = blockIdx.x; row < Ap->rows; row += n) {
+        const bool left = Ap->flags[row] == kTwinRest;
         __syncthreads();  // (every wave has read the word before one of them writes the row's flags there; and the row before is done with LDS)
         if (!left) continue;  // uniform
-        LeanArgPtr Ap = (LeanArgPtr)__builtin_amdgcn_kernarg_segment_ptr();
-        asm volatile("" : "+s"(Ap));
         if (Ap->kept_ids) three_pass_row<true>(Ap, row);
         else three_pass_row<false>(Ap, row);
     }
+}
+__global__ void __launch_bounds__(WS_BLOCK) short_rest_kernel(BatchArgs A) {
+    const uint32_t n = gridDim.x, lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+    bool any = false;
+    for (uint32_t row = blockIdx.x + lane * n; row < A.rows; row += 64u * n) any |= A.flags[row] == kTwinRest;
+    if (!__ballot(any)) return;  // (every wave asks for itself, and all get the same: the first flag is written behind a barrier)
+    LeanArgPtr Ap = (LeanArgPtr)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(Ap));
+    short_rest(Ap, n);
 }
 }  // namespace
 
