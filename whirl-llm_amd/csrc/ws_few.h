@@ -17,7 +17,7 @@
 //     that about as many keys as top_k are left to sort.
 //   * a row's parts are on one chiplet where its compute units take all parts of its rows at once (few_place).
 // What bounds it is that chain: parameters, ids, their tokens' logits, the stores of the keys, headers and keys are six trips to
-// memory, between them some 2000 instructions of the slowest wave; with 64 rows and more the instructions a token, which two waves a SIMD
+// memory, between them some 1100 instructions of the average wave (582 vector, 538 scalar; the last part's do more); with 64 rows and more the instructions a token, which two waves a SIMD
 // issue one after the other. 512 threads rather than 1024: the cost of a wave's own
 // work (threshold, sums, publishing) is paid half as often, and a share still fits the registers. Measured against the
 // short-list kernel's shared rows (151936 fp32, microseconds a launch): one row, top-k 40: 20.6 -> 11.9; 64 rows of mixed
