@@ -1553,7 +1553,7 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const LeanArgPtr ar
 }
 
 // the three-pass code of ws_sample.h for one row, a function of its own: its registers and code stay out of the lean path.
-// It takes the kernel's argument segment, and reads there where the three-pass layout of the LDS lies (RowLayout).
+// It takes the kernel's argument segment, and reads there where the three-pass layout of the LDS lies (sample_row's BACK).
 // What it is handed comes in vector registers; said to be one value for the whole wave, so that everything that follows from it is scalar again. Not a tail
 // call: only then does the compiler leave out saving the callers' registers, which nobody reads any more - thirty-five scalar registers went to memory one by one,
 // each a round trip of a vector register that had to be free for it, and back at the end: 30 us of every handed-back row. (Before that, the arguments once

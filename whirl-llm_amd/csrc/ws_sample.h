@@ -1778,18 +1778,10 @@ __device__ __noinline__ ExactOut exact_row(const ExactIn in) {
 // that can write the kept-set dump; launches without kept_ids take the single-sweep builds that cannot, which keeps the
 // dump's flags and calls out of their register allocation (with them the tile cost 1-2 % more).
 // One row (or one part of a split row) by the workgroup that calls it: `block` = row * parts + part. The kernels below
-// are this function; the lean kernel (ws_lean.h) calls the three-pass instantiation for the rows it hands back (BACK: that layout of the LDS).
-template <bool BACK>
-struct RowLayout {
-    __device__ __forceinline__ static uint32_t lds_ab(const BatchArgs& A) { return BACK ? A.fb_lds_ab : A.lds_ab; }
-    __device__ __forceinline__ static uint32_t lds_cnt(const BatchArgs& A) { return BACK ? 0u : A.lds_cnt; }
-    __device__ __forceinline__ static uint32_t lds_tie(const BatchArgs& A) { return BACK ? A.fb_lds_tie : A.lds_tie; }
-    __device__ __forceinline__ static bool two_sweep(const BatchArgs& A) { return BACK || A.two_sweep; }
-    __device__ __forceinline__ static unsigned char* work(const BatchArgs& A) { return BACK ? nullptr : A.work; }
-};
+// are this function; the lean kernel (ws_lean.h) calls the three-pass instantiation for the rows it hands back (BACK: that layout of the LDS,
+// and no workspace. The choices stand where they are used: as functions of a struct they left the compiler another order of registers, and rows of the kernels here took 1 % longer).
 template <bool FUSED, bool SPLIT = false, bool KEPT = true, bool BACK = false>
 __device__ __forceinline__ void sample_row(const BatchArgs& A, const uint32_t block) {
-    using Lay = RowLayout<BACK>;
     int32_t* const kept_ids = KEPT ? A.kept_ids : nullptr;
 #ifdef WS_PHASE_TIMERS
     __shared__ long long ws_marks[64];
@@ -1823,9 +1815,9 @@ __device__ __forceinline__ void sample_row(const BatchArgs& A, const uint32_t bl
     uint64_t* hist = reinterpret_cast<uint64_t*>(lds);
     uint64_t* keys = hist;
     double* emass = reinterpret_cast<double*>(lds + 32768);
-    uint32_t* touched = reinterpret_cast<uint32_t*>(lds + Lay::lds_ab(A));
-    uint16_t* wprefix = reinterpret_cast<uint16_t*>(lds + Lay::lds_ab(A) + nW * 4u);
-    float* pv = reinterpret_cast<float*>(lds + Lay::lds_ab(A) + nW * 4u + ((nW * 2u + 15u) & ~15u));
+    uint32_t* touched = reinterpret_cast<uint32_t*>(lds + (BACK ? A.fb_lds_ab : A.lds_ab));
+    uint16_t* wprefix = reinterpret_cast<uint16_t*>(lds + (BACK ? A.fb_lds_ab : A.lds_ab) + nW * 4u);
+    float* pv = reinterpret_cast<float*>(lds + (BACK ? A.fb_lds_ab : A.lds_ab) + nW * 4u + ((nW * 2u + 15u) & ~15u));
 
     const float inv_t = A.inv_t[row];
     const uint32_t top_k = A.top_k ? A.top_k[row] : 0u;
@@ -1919,7 +1911,7 @@ __device__ __forceinline__ void sample_row(const BatchArgs& A, const uint32_t bl
                 run += __popc(touched[w]);
             }
         }
-        uint32_t* cnt = reinterpret_cast<uint32_t*>(lds + Lay::lds_cnt(A));  // low 20 bits: history count, high 12: bias entries
+        uint32_t* cnt = reinterpret_cast<uint32_t*>(lds + (BACK ? 0u : A.lds_cnt));  // low 20 bits: history count, high 12: bias entries
         uint32_t* first = cnt + A.patch_cap;               // index of the id's first bias entry
         for (uint32_t r = t; r < n_uniq; r += WS_BLOCK) {
             cnt[r] = 0u;
@@ -1994,8 +1986,8 @@ __device__ __forceinline__ void sample_row(const BatchArgs& A, const uint32_t bl
         for (uint32_t b = t; b < kBins; b += WS_BLOCK) gh[b] = 0ull;
         if (t < 4u) ctrl[t] = 0u;
     };
-    const float* praw = reinterpret_cast<const float*>(lds + Lay::lds_cnt(A));           // raw logits of the touched tokens, by rank
-    const uint32_t* pid = reinterpret_cast<const uint32_t*>(lds + Lay::lds_cnt(A)) + A.patch_cap;  // their token ids
+    const float* praw = reinterpret_cast<const float*>(lds + (BACK ? 0u : A.lds_cnt));           // raw logits of the touched tokens, by rank
+    const uint32_t* pid = reinterpret_cast<const uint32_t*>(lds + (BACK ? 0u : A.lds_cnt)) + A.patch_cap;  // their token ids
     // Raw logit of every touched token as the sweeps see it (NaN and masked-out -> -inf), one 4-byte gather per history
     // / bias entry (entries of one id store the same value), then its adjusted logit, once: bias, repetition, then
     // frequency and presence, each operation rounded to float. pv[r] <- adjusted, praw[r] (the dead count slot) <- raw,
@@ -2011,7 +2003,7 @@ __device__ __forceinline__ void sample_row(const BatchArgs& A, const uint32_t bl
         const int32_t* hist_ids = A.hist + h0;
         const int32_t* bias_ids = A.bias_ids + b0;
         const float* bias_vals = A.bias_vals + b0;
-        uint32_t* cnt = reinterpret_cast<uint32_t*>(lds + Lay::lds_cnt(A));
+        uint32_t* cnt = reinterpret_cast<uint32_t*>(lds + (BACK ? 0u : A.lds_cnt));
         uint32_t* first = cnt + A.patch_cap;
         float mu = -INFINITY;  // largest untouched, allowed logit among the vectors that hold touched tokens
         auto fetch4 = [&](const int32_t* ids, uint32_t n, bool in_regs) {  // four independent gathers per thread and round
@@ -2178,7 +2170,7 @@ __device__ __forceinline__ void sample_row(const BatchArgs& A, const uint32_t bl
         const int32_t* hist_ids = A.hist + h0;
         const int32_t* bias_ids = A.bias_ids + b0;
         const float* bias_vals = A.bias_vals + b0;
-        uint32_t* cnt = reinterpret_cast<uint32_t*>(lds + Lay::lds_cnt(A));
+        uint32_t* cnt = reinterpret_cast<uint32_t*>(lds + (BACK ? 0u : A.lds_cnt));
         uint32_t* first = cnt + A.patch_cap;
         const uint32_t whole_end = rv.vec ? (V & ~(per - 1u)) : 0u;  // tokens below this sit in whole 128-bit vectors
         const float tail_own = own_tail();
@@ -2325,7 +2317,7 @@ __device__ __forceinline__ void sample_row(const BatchArgs& A, const uint32_t bl
     };
     float m = -INFINITY;
     bool cached = false;
-    uint64_t* hist2 = FUSED && Lay::lds_tie(A) ? reinterpret_cast<uint64_t*>(lds + Lay::lds_tie(A)) : nullptr;  // second copy of the histogram
+    uint64_t* hist2 = FUSED && (BACK ? A.fb_lds_tie : A.lds_tie) ? reinterpret_cast<uint64_t*>(lds + (BACK ? A.fb_lds_tie : A.lds_tie)) : nullptr;  // second copy of the histogram
     // the split kernel's slices are at most half a row (two parts at least): half the registers, and room for everything else
     constexpr int kCR = SPLIT ? kCacheRegs / 2 : kCacheRegs;
     uint32_t cache[kCR];  // dead code (and no registers) in the exact instantiation
@@ -2458,7 +2450,7 @@ __device__ __forceinline__ void sample_row(const BatchArgs& A, const uint32_t bl
         if (!(m > -INFINITY)) flags |= kAllMasked;
     } else if (!(flags & kBadParam)) {
         bool adjusted = false;
-        if (Lay::two_sweep(A) && Lay::work(A) && n_touched) {
+        if ((BACK || A.two_sweep) && (BACK ? nullptr : A.work) && n_touched) {
             // ------------------------------------------------------------ with a workspace: the first sweep leaves the raw
             // logit of every touched token in pv, by rank, as the token goes by. Gathering them from the row pulls a
             // whole memory line per token - for a history of 8192 ids as much traffic as the sweep itself. The workspace
@@ -2466,10 +2458,10 @@ __device__ __forceinline__ void sample_row(const BatchArgs& A, const uint32_t bl
             // the histogram, so they move out first (the first-entry table as the bias value itself
             // where an id has one bias entry, as nearly all have: one dependent read less per rank afterwards).
             const uint32_t cap4 = (A.patch_cap + 3u) & ~3u;
-            uint32_t* gcnt = reinterpret_cast<uint32_t*>(Lay::work(A) + static_cast<size_t>(row) * capture_row_bytes(A.patch_cap));
+            uint32_t* gcnt = reinterpret_cast<uint32_t*>((BACK ? nullptr : A.work) + static_cast<size_t>(row) * capture_row_bytes(A.patch_cap));
             uint32_t* gbias = gcnt + cap4;
             {
-                const uint32_t* cnt = reinterpret_cast<const uint32_t*>(lds + Lay::lds_cnt(A));
+                const uint32_t* cnt = reinterpret_cast<const uint32_t*>(lds + (BACK ? 0u : A.lds_cnt));
                 const uint32_t* first = cnt + A.patch_cap;
                 const float* bias_vals = A.bias_vals + b0;
                 for (uint32_t r0 = 0; r0 < n_touched; r0 += 4u * WS_BLOCK) {
@@ -2520,7 +2512,7 @@ __device__ __forceinline__ void sample_row(const BatchArgs& A, const uint32_t bl
             }
         }
         if (!adjusted) gather_and_adjust(nullptr, 0u);
-        if (Lay::two_sweep(A) && !adjusted) {
+        if ((BACK || A.two_sweep) && !adjusted) {
             // ------------------------------------------------------------ maximum and histogram in one sweep, against a
             // bound above the maximum guessed from the adjusted tokens and the head of the row (as the single-sweep
             // mode does); rows the guess does not fit fall through to the two passes below
@@ -2901,12 +2893,12 @@ __device__ __forceinline__ void sample_row(const BatchArgs& A, const uint32_t bl
                 // scan's side arrays, idle by now) and places for keys and their masses: 32 per bucket where the spare LDS
                 // takes the masses, else 16 with keys and masses sharing the key region (idle until then)
                 constexpr uint32_t kLeanBuckets = 128u;  // 64 per range
-                const uint32_t lean_shift = Lay::lds_tie(A) ? 5u : 4u, lean_places = 1u << lean_shift;
-                const uint32_t lean_max = Lay::lds_tie(A) ? 800u : 448u;  // candidates per range: a bucket must not run out of places
+                const uint32_t lean_shift = (BACK ? A.fb_lds_tie : A.lds_tie) ? 5u : 4u, lean_places = 1u << lean_shift;
+                const uint32_t lean_max = (BACK ? A.fb_lds_tie : A.lds_tie) ? 800u : 448u;  // candidates per range: a bucket must not run out of places
                 uint64_t* lb_mass = reinterpret_cast<uint64_t*>(s_pool);
                 uint32_t* lb_cnt = reinterpret_cast<uint32_t*>(s_pool + 128);
                 uint64_t* lb_key = reinterpret_cast<uint64_t*>(lds);           // [bucket][place]
-                double* lb_e = reinterpret_cast<double*>(lds + (Lay::lds_tie(A) ? Lay::lds_tie(A) : 16384u));  // exact mass of lb_key
+                double* lb_e = reinterpret_cast<double*>(lds + ((BACK ? A.fb_lds_tie : A.lds_tie) ? (BACK ? A.fb_lds_tie : A.lds_tie) : 16384u));  // exact mass of lb_key
                 __shared__ unsigned long long s_q[2];
                 if (t < kLeanBuckets) {
                     lb_mass[t] = 0ull;
@@ -2971,7 +2963,7 @@ __device__ __forceinline__ void sample_row(const BatchArgs& A, const uint32_t bl
                             in.id0 = id0;
                             in.row_V = V;
                             in.dtype = rv.dtype;
-                            in.touched_at = rv.touched ? Lay::lds_ab(A) : 0xffffffffu;
+                            in.touched_at = rv.touched ? (BACK ? A.fb_lds_ab : A.lds_ab) : 0xffffffffu;
                             in.aq = aq;
                             in.c64 = c64;
                             in.last_bin = stage_last;
@@ -3677,9 +3669,9 @@ __device__ __forceinline__ void sample_row(const BatchArgs& A, const uint32_t bl
             // scanned and ranked like the first level. Counters: the spare LDS (n_big * kS2 + 1 words).
             constexpr uint32_t kS2 = 256;
             constexpr uint32_t kPB2 = (kMaxBig * kS2 + WS_BLOCK - 1) / WS_BLOCK;
-            uint32_t* c2 = reinterpret_cast<uint32_t*>(lds + Lay::lds_tie(A));
+            uint32_t* c2 = reinterpret_cast<uint32_t*>(lds + (BACK ? A.fb_lds_tie : A.lds_tie));
             uint32_t sub2[kCh], arr2[kCh];
-            if (!ok && n_big <= kMaxBig && Lay::lds_tie(A)) {  // uniform
+            if (!ok && n_big <= kMaxBig && (BACK ? A.fb_lds_tie : A.lds_tie)) {  // uniform
                 // one logit per big bucket?
 #pragma unroll
                 for (int q = 0; q < kCh; ++q) {
@@ -4133,7 +4125,7 @@ __device__ __forceinline__ void sample_row(const BatchArgs& A, const uint32_t bl
         in.allow = rv.allow;
         in.V = V;
         in.dtype = rv.dtype;
-        in.touched_at = rv.touched ? Lay::lds_ab(A) : 0xffffffffu;
+        in.touched_at = rv.touched ? (BACK ? A.fb_lds_ab : A.lds_ab) : 0xffffffffu;
         in.m = m;
         in.inv_t = inv_t;
         in.top_k = top_k;
@@ -4183,7 +4175,7 @@ __device__ __forceinline__ void sample_row(const BatchArgs& A, const uint32_t bl
             each_token([&](uint32_t i, float x) { term(key64(x, i)); });
         } else if (finished_lean) {  // the keys lie in the buckets' places
             const uint32_t* cnt_of = reinterpret_cast<const uint32_t*>(s_pool + 128);
-            const uint32_t shift = Lay::lds_tie(A) ? 5u : 4u;
+            const uint32_t shift = (BACK ? A.fb_lds_tie : A.lds_tie) ? 5u : 4u;
             for (uint32_t slot = t; slot < (128u << shift); slot += WS_BLOCK)
                 if ((slot & ((1u << shift) - 1u)) < cnt_of[slot >> shift]) term(reinterpret_cast<const uint64_t*>(lds)[slot]);
         } else {
@@ -4260,8 +4252,8 @@ __device__ __forceinline__ void sample_row(const BatchArgs& A, const uint32_t bl
         // after the bucket finish: the kept candidates go from the list to the room of the buckets' masses (done with)
         __syncthreads();
         if constexpr (FUSED)
-            dump_listed_candidates(rv.base, rv.dtype, rv.touched ? Lay::lds_ab(A) : 0xffffffffu, 32768u /* list */, listed_n, kept_key,
-                                   Lay::lds_tie(A) ? Lay::lds_tie(A) : 16384u /* lb_e */, kDumpListed, kept_ids + static_cast<size_t>(row) * A.kept_cap,
+            dump_listed_candidates(rv.base, rv.dtype, rv.touched ? (BACK ? A.fb_lds_ab : A.lds_ab) : 0xffffffffu, 32768u /* list */, listed_n, kept_key,
+                                   (BACK ? A.fb_lds_tie : A.lds_tie) ? (BACK ? A.fb_lds_tie : A.lds_tie) : 16384u /* lb_e */, kDumpListed, kept_ids + static_cast<size_t>(row) * A.kept_cap,
                                    A.kept_logits ? A.kept_logits + static_cast<size_t>(row) * A.kept_cap : nullptr, A.kept_cap);
         dumped = true;
     }
@@ -4271,7 +4263,7 @@ __device__ __forceinline__ void sample_row(const BatchArgs& A, const uint32_t bl
         in.allow = rv.allow;
         in.V = V;
         in.dtype = rv.dtype;
-        in.touched_at = rv.touched ? Lay::lds_ab(A) : 0xffffffffu;
+        in.touched_at = rv.touched ? (BACK ? A.fb_lds_ab : A.lds_ab) : 0xffffffffu;
         in.aq = aq;
         in.c64 = c64;
         in.kept_key = kept_key;
