@@ -34,11 +34,11 @@ KEPT_CAP = 0  # entries a row of the kept-set dump (--kept-cap), 0: no dump
 # of the kernel sources the counters were taken with), otherwise null. File names are relative to profiles/.
 TRAFFIC = {
     # (workload, mode): (bytes per launch, profiles/ file, kernel_digest() at the time)
-    ("tile", "auto"): (205089867, "lean_batch_kernel_tile_256x151936_f32.txt", "ddc84420ee437d5b"),
-    ("cfg1", "auto"): (776965, "few_batch_kernel_cfg1_1x151936_f32.txt", "ddc84420ee437d5b"),
-    ("cfg2", "auto"): (49984009, "few_batch_kernel_cfg2_64x151936_f32.txt", "ddc84420ee437d5b"),
-    ("cfg3", "auto"): (113147518, "code_batch_kernel_cfg3_256x151936_bf16.txt", "ddc84420ee437d5b"),
-    ("cfg5", "auto"): (1307123314, "twin_batch_kernel_cfg5_1024x262144_f32.txt", "ddc84420ee437d5b"),
+    ("tile", "auto"): (205089964, "lean_batch_kernel_tile_256x151936_f32.txt", "153c89e7a62af2dc"),
+    ("cfg1", "auto"): (765830, "few_batch_kernel_cfg1_1x151936_f32.txt", "153c89e7a62af2dc"),
+    ("cfg2", "auto"): (49972947, "few_batch_kernel_cfg2_64x151936_f32.txt", "153c89e7a62af2dc"),
+    ("cfg3", "auto"): (113236631, "code_batch_kernel_cfg3_256x151936_bf16.txt", "153c89e7a62af2dc"),
+    ("cfg5", "auto"): (1307120118, "twin_batch_kernel_cfg5_1024x262144_f32.txt", "153c89e7a62af2dc"),
 }
 
 
