@@ -161,3 +161,20 @@ def test_bf16_rows_either_side_of_the_lines_between_the_kernels(V, top_k, n_hist
     assert res["differ"] == 0 and res["exact"] == len(some(rows, 67)), res
     fl, m = smp.flags.cpu().numpy(), gc.pkg()
     assert (fl & m.FLAG_ROUTE_SHORT).all() and not (fl & m.FLAG_ROUTE_HANDED_BACK).any()
+
+
+@pytest.mark.parametrize("V,n_hist,n_bias,allowed,dtype", [(50257, 2047, 0, 0.5, "f32"), (50257, 2048, 0, 0.5, "f32"), (50257, 2049, 0, 0.5, "f32"), (50257, 1500, 548, 0.5, "f32"),
+                                                           (50257, 1500, 549, 0.5, "f32"), (12288, 2040, 8, 0.3, "bf16"), (262144, 8192, 500, 0.05, "f32"), (262144, 1542, 0, 0.5, "f32"),
+                                                           (262144, 5, 3, 0.1, "f32")])
+def test_masks_that_allow_the_whole_history(V, n_hist, n_bias, allowed, dtype):
+    """The list of the entries that a mask allows, to its last place and past it: the mask allows few tokens, but of every other row all that its
+    history and bias list name (so that more are listed than the mask let expect, and the row goes on without the list)."""
+    rows = rows_of()
+    c = _odd(rows, V, dtype, top_k=50, n_hist=n_hist, n_bias=max(n_bias, 1), allowed=allowed)
+    for r in range(0, rows, 2):
+        ids = np.concatenate([c["hist"][r], c["bias_ids"][r][:n_bias]]).astype(np.int64)
+        ids = ids[(ids >= 0) & (ids < V)]
+        np.bitwise_or.at(c["allow"][r], ids >> 5, (np.uint32(1) << (ids & 31).astype(np.uint32)).astype(c["allow"].dtype))
+    if not n_bias:
+        c["bias_ids"] = c["bias_vals"] = None
+    run_short(c if n_bias < 3 else twice_biased(c), 1, rows=some(rows, 41))

@@ -8,6 +8,13 @@
 // (280 since ws_common.h's search of bias lists), without history 266 / 239; top-k 50, 1000-id histories: 512 of 151936 83.8 / 73.3, 300 of 151936 77.2 / 63.9, 1000 of 50257 108 / 72.9, 1000 of 8000
 // 55.9 / 38.1; min-p alone, 1000 of 151936 149 / 139. (1024 of 262144 with a top-k of 50: 195, 5.5 TB/s.)
 //
+// While both rows sweep, the vector instructions of a unit are all in use (with the loads aimed at eight chunks in L2 a sweep took 84 us of the 91), so
+// what a listed token costs counts: 1850 of a row are one in five vectors out of six. A wave takes its places in the list thirty-two at a time, writes
+// logit and id as they are, and keeps its count in a scalar register (an atomic addition and its answer a token, the key made on the spot: 278 -> 270 us for
+// the rows above); the entries of a history that a mask rules out are looked at once (270 -> 253 with the registers below, 247 without a
+// spilled one): the sample's masked-out tokens become NaN in place, so that the mask's words are done with before the row is asked for. 512 rows of 151936, min-p
+// alone 108.8 -> 98.2, 300 of 262144 with a top-k of 1000 106.2 -> 101.2, 1000 bf16 rows of 12288 with a top-k of 200 52.3 -> 49.0, 300 of 151936 with a top-k of 300 and 4096 ids 86.5 -> 81.8.
+//
 // Against ws_short.h the touched tokens come before the sweep, not behind it: their tables are dead when it begins and can lie where the list
 // will be. A history entry's count, a token's bias marks and its claim are 16 bits, not 48: a token is claimed by clearing its word, and where a bias entry
 // names it only those claim it, so that nobody has to look the entry up. Rows for which a check fails are marked in `flags`, and a
@@ -20,6 +27,8 @@
 namespace ws {
 
 constexpr uint32_t kTwinHead = 8u;  // vectors a thread of the sample that the threshold is fitted to
+constexpr uint32_t kTwinPlaces = 32u;  // places of the list a wave takes at a time
+static_assert((kTwinPlaces - 1u) * WS_WAVES <= 256u, "the places left over: one a thread of the waves that close them");
 
 // LDS: the list at 0 (32 KiB; first the sample's bin counts), the bitmap of the touched tokens at lds_ab, and at lds_cnt its 16-bit popcount
 // prefixes and a 16-bit word per rank: history count | kBias | kBiases. These two are dead when the sweep begins, and where a second
@@ -106,6 +115,18 @@ __device__ __forceinline__ bool twin_row(const BatchArgs& A, const uint32_t row,
         for (uint32_t k = 0; k < kWords; ++k) aw[k] = allow[min(k * WS_BLOCK + t, nW - 1u)];
     }
 
+    constexpr uint32_t kFew = 4u, kFewShift = 20u, kFewId = (1u << kFewShift) - 1u;  // a listed entry: its id, and the number of a bias entry plus one
+    const uint32_t few_room = MASKED ? min(kFew * WS_BLOCK, (early_slots * 8u - kTwinBins * 4u) / 4u) : 0u;
+    uint32_t n_few = 0xffffffffu;
+    if (MASKED && n_all) {  // the tokens the mask allows: most rows' are few
+        uint32_t allowed = 0;
+#pragma unroll
+        for (uint32_t k = 0; k < kWords; ++k) allowed += k * WS_BLOCK + t < nW ? static_cast<uint32_t>(__popc(aw[k])) : 0u;
+        allowed = wave_sum(allowed);
+        if (lane == 0u) S.red_u[wv] = allowed;
+        if (t == 0u) S.s_w[4] = 0u;
+    }
+
     // the other whole chunks in order
     uint32_t c_next = spread == 1u ? kTwinHead : 1u, c_skip = spread == 1u ? 0xffffffffu : spread;
     auto next_chunk = [&]() __attribute__((always_inline)) {
@@ -141,17 +162,84 @@ __device__ __forceinline__ bool twin_row(const BatchArgs& A, const uint32_t row,
                 for (uint32_t k = 0; k < kMore; ++k) what(id[k], j0 + k * WS_BLOCK + t);
             }
         };
-#pragma unroll
-        for (uint32_t k = 0; k < kIds; ++k)
-            if (k * WS_BLOCK < n_all) mark(ids[k]);  // uniform
-        others([&](uint32_t id, uint32_t) { mark(id); });
-        __syncthreads();
+        // Of a masked row only the entries that its mask allows are gone on with - the mask where the bitmap will be, the entries listed behind the
+        // sample's counts, then in registers -, if they are few enough for it. (Nine in ten of 8692 masked out: 17 entries a thread, each looked up in
+        // three passes, were 25 us of a row's 125.)
+        bool by_list = false;
         if (MASKED) {
+            uint32_t n_allowed = 0;
+#pragma unroll
+            for (uint32_t w = 0; w < WS_WAVES; ++w) n_allowed += S.red_u[w];
+            by_list = nW <= kWords * WS_BLOCK && static_cast<float>(n_allowed) * static_cast<float>(n_all) * 1.1f + 64.f * static_cast<float>(V) < static_cast<float>(V) * static_cast<float>(few_room);  // uniform
+        }
+        if (MASKED && by_list) {
 #pragma unroll
             for (uint32_t k = 0; k < kWords; ++k)
-                if (k * WS_BLOCK + t < nW) touched[k * WS_BLOCK + t] &= aw[k];
-            for (uint32_t w = kWords * WS_BLOCK + t; w < nW; w += WS_BLOCK) touched[w] &= allow[w];
+                if (k * WS_BLOCK + t < nW) touched[k * WS_BLOCK + t] = aw[k];
             __syncthreads();
+            uint32_t* listed = head_cnt + kTwinBins;
+            auto list_allowed = [&](auto n, auto&& id_of, uint32_t j0) __attribute__((always_inline)) {
+                constexpr uint32_t N = decltype(n)::value;
+                uint32_t word[N], all = 0;
+                uint64_t on[N];
+#pragma unroll
+                for (uint32_t k = 0; k < N; ++k) word[k] = touched[min(id_of(k), V - 1u) >> 5] >> (id_of(k) & 31u);
+#pragma unroll
+                for (uint32_t k = 0; k < N; ++k) {
+                    on[k] = __ballot(id_of(k) < V && (word[k] & 1u));
+                    all += static_cast<uint32_t>(__popcll(on[k]));
+                }
+                uint32_t from = 0;
+                if (lane == 0u && all) from = atomicAdd(&S.s_w[4], all);
+                from = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(from)));
+#pragma unroll
+                for (uint32_t k = 0; k < N; ++k) {
+                    const uint32_t at = from + __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(on[k] >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(on[k]), 0u));
+                    const uint32_t j = j0 + k * WS_BLOCK + t;
+                    if (id_of(k) < V && (word[k] & 1u) && at < few_room) listed[at] = id_of(k) | (j < nh ? 0u : (j - nh + 1u) << kFewShift);
+                    from += static_cast<uint32_t>(__popcll(on[k]));
+                }
+            };
+            uint32_t next[kMore];
+#pragma unroll
+            for (uint32_t k = 0; k < kMore; ++k) next[k] = entry((kIds + k) * WS_BLOCK + t);
+            constexpr uint32_t kThird = kIds / 3u;
+#pragma unroll
+            for (uint32_t h = 0; h < 3u; ++h)
+                if (h * kThird * WS_BLOCK < n_all) list_allowed(std::integral_constant<uint32_t, kThird>{}, [&](uint32_t k) { return ids[h * kThird + k]; }, h * kThird * WS_BLOCK);  // uniform
+            for (uint32_t j0 = kIds * WS_BLOCK; j0 < n_all; j0 += kMore * WS_BLOCK) {
+                uint32_t id[kMore];
+#pragma unroll
+                for (uint32_t k = 0; k < kMore; ++k) {
+                    id[k] = next[k];
+                    next[k] = entry(j0 + (kMore + k) * WS_BLOCK + t);
+                }
+                list_allowed(std::integral_constant<uint32_t, kMore>{}, [&](uint32_t k) { return id[k]; }, j0);
+            }
+            __syncthreads();
+            n_few = S.s_w[4];
+            if (n_few <= few_room) {  // uniform
+#pragma unroll
+                for (uint32_t k = 0; k < kFew; ++k) ids[k] = k * WS_BLOCK + t < n_few ? listed[k * WS_BLOCK + t] : 0xffffffffu;
+            }
+            for (uint32_t w = t; w < nW; w += WS_BLOCK) touched[w] = 0u;
+            __syncthreads();
+        }
+        if (MASKED && n_few <= few_room) {  // uniform
+#pragma unroll
+            for (uint32_t k = 0; k < kFew; ++k)
+                if (k * WS_BLOCK < n_few) mark(ids[k] & kFewId);
+            __syncthreads();
+        } else {
+#pragma unroll
+            for (uint32_t k = 0; k < kIds; ++k)
+                if (k * WS_BLOCK < n_all) mark(ids[k]);  // uniform
+            others([&](uint32_t id, uint32_t) { mark(id); });
+            __syncthreads();
+            if (MASKED) {
+                for (uint32_t w = t; w < nW; w += WS_BLOCK) touched[w] &= allow[w];
+                __syncthreads();
+            }
         }
         {  // popcount prefixes: an odd number of consecutive words a thread (no two lanes of a read in one bank)
             const uint32_t per = ((nW + WS_BLOCK - 1u) / WS_BLOCK) | 1u, w0 = min(t * per, nW), w1 = min(w0 + per, nW);
@@ -170,10 +258,16 @@ __device__ __forceinline__ bool twin_row(const BatchArgs& A, const uint32_t row,
             if (j < nh) atomicAdd(&cnt[r >> 1], 1u << sh);
             else if ((atomicOr(&cnt[r >> 1], kBias << sh) >> sh) & kBias) atomicOr(&cnt[r >> 1], kBiases << sh);
         };
+        if (n_few <= few_room) {  // uniform
 #pragma unroll
-        for (uint32_t k = 0; k < kIds; ++k)
-            if (k * WS_BLOCK < n_all) count(ids[k], k * WS_BLOCK + t);  // uniform
-        others(count);
+            for (uint32_t k = 0; k < kFew; ++k)
+                if (k * WS_BLOCK < n_few) count(ids[k] & kFewId, ids[k] <= kFewId ? 0u : nh);  // uniform
+        } else {
+#pragma unroll
+            for (uint32_t k = 0; k < kIds; ++k)
+                if (k * WS_BLOCK < n_all) count(ids[k], k * WS_BLOCK + t);  // uniform
+            others(count);
+        }
     }
     WSS_MARK(1);  // bitmap done
     // one vector: its tokens as floats, masked-out / touched / NaN ones as -inf
@@ -190,6 +284,27 @@ __device__ __forceinline__ bool twin_row(const BatchArgs& A, const uint32_t row,
             x[e] = fmaxf(__uint_as_float(bits), -INFINITY);
         }
     };
+
+    // The sample without the tokens that do not count: they become NaN where they are, and the mask's words need no registers from here on.
+    auto values = [&](const uint4& q, float (&x)[TPV]) __attribute__((always_inline)) {
+        const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+        for (uint32_t e = 0; e < TPV; ++e)
+            x[e] = fmaxf(__uint_as_float(DT == 0 ? w[e] : ((e & 1u) ? (w[e >> 1] & 0xffff0000u) : (w[e >> 1] << 16))), -INFINITY);
+    };
+    if (MASKED || n_all) {
+#pragma unroll
+        for (uint32_t k = 0; k < kTwinHead; ++k) {
+            const uint32_t i0 = min(k * spread * WS_BLOCK + t, nv - 1u) * TPV;
+            uint32_t invalid = 0u;  // bit e: token e does not count here
+            if (MASKED) invalid = ~(hna[k] >> (i0 & 31u));
+            if (n_all) invalid |= touched[i0 >> 5] >> (i0 & 31u);
+            auto gone = [&](uint32_t e) { return static_cast<uint32_t>(static_cast<int32_t>(invalid << (31u - e)) >> 31); };
+            uint32_t* w = &hq[k].x;
+#pragma unroll
+            for (uint32_t e = 0; e < 4u; ++e) w[e] |= DT == 0 ? gone(e) : (gone(2u * e) & 0xffffu) | (gone(2u * e + 1u) << 16);
+        }
+    }
 
     // The first two batches behind the sample travel while the threshold is worked out. (A whole chunk's address is the
     // same register for every thread and a lane's offset: nothing to add or to clamp a vector.)
@@ -215,7 +330,7 @@ __device__ __forceinline__ bool twin_row(const BatchArgs& A, const uint32_t row,
         for (uint32_t k = 0; k < kTwinHead; ++k) {
             const uint32_t j = k * spread * WS_BLOCK + t;
             if (j < nv) {
-                unpack(hq[k], hna[k], j, x);
+                values(hq[k], x);
 #pragma unroll
                 for (uint32_t e = 0; e < TPV; ++e) ref = fmaxf(ref, x[e]);
             }
@@ -284,7 +399,7 @@ __device__ __forceinline__ bool twin_row(const BatchArgs& A, const uint32_t row,
             for (uint32_t k = 0; k < kTwinHead; ++k) {
                 const uint32_t j = k * spread * WS_BLOCK + t;
                 if (j < nv) {
-                    unpack(hq[k], hna[k], j, x);
+                    values(hq[k], x);
 #pragma unroll
                     for (uint32_t e = 0; e < TPV; ++e) {
                         const float d = fminf(__fmul_rn(__fsub_rn(top, x[e]), c32), kFar);
@@ -348,27 +463,29 @@ __device__ __forceinline__ bool twin_row(const BatchArgs& A, const uint32_t row,
         if (yes) {
             m = fmaxf(m, x);
             const uint32_t slot = atomicAdd(&S.s_w[1], 1u);
-            if (slot < (early ? early_slots : kShortCap)) list[slot] = key64(x, id);
+            if (slot < (early ? early_slots : kShortCap)) list[slot] = (static_cast<uint64_t>(__float_as_uint(x)) << 32) | id;
             else if (early) S.s_w[2] = 1u;
             if (early) atomicAdd(&S.s_w[3], 1u);
         }
     };
 
+    // (The list takes tokens as they are, logit and id; the sort's keys are made of them behind the sweep, all lanes at work.)
     // ---- the touched tokens: their adjusted logits (bias entries in list order, then repetition, then frequency / presence, as
     // ws_sample.h applies them), into the sum and - above the threshold - the list. A token is taken by the entry that finds its word there
     // and clears it: a bias entry where one names it, else one of its history.
     if (n_all) {
-        auto take_touched = [&](auto n, auto&& id_of, uint32_t j0) __attribute__((always_inline)) {
+        // (j_of: an entry's number; of a listed one that of a bias entry behind nh, or 0)
+        auto take_touched = [&](auto n, auto&& id_of, auto&& j_of, uint32_t j0, uint32_t n_of) __attribute__((always_inline)) {
             constexpr uint32_t N = decltype(n)::value;
             uint32_t word[N];
             float raw[N];
 #pragma unroll
             for (uint32_t k = 0; k < N; ++k) {
                 word[k] = 0u;
-                if (j0 + k * WS_BLOCK >= n_all) continue;  // uniform
+                if (j0 + k * WS_BLOCK >= n_of) continue;  // uniform
                 const uint32_t r = rank(id_of(k)), sh = (r & 1u) * 16u;
                 if (r == 0xffffffffu) continue;
-                if (j0 + k * WS_BLOCK + t < nh && ((cnt[r >> 1] >> sh) & kBias)) continue;
+                if (j_of(k) < nh && ((cnt[r >> 1] >> sh) & kBias)) continue;
                 word[k] = (atomicAnd(&cnt[r >> 1], ~(0xffffu << sh)) >> sh) & 0xffffu;
             }
 #pragma unroll
@@ -378,13 +495,13 @@ __device__ __forceinline__ bool twin_row(const BatchArgs& A, const uint32_t row,
             }
 #pragma unroll
             for (uint32_t k = 0; k < N; ++k) {
-                if (j0 + k * WS_BLOCK >= n_all) continue;  // uniform
+                if (j0 + k * WS_BLOCK >= n_of) continue;  // uniform
                 float x = -INFINITY;
                 if (word[k]) {
                     const uint32_t c = word[k] & (kBias - 1u);
                     x = fmaxf(raw[k], -INFINITY);
                     const bool several = (word[k] & kBiases) != 0u;
-                    if ((word[k] & kBias) && !several) x = __fadd_rn(x, bias_vals[j0 + k * WS_BLOCK + t - nh]);
+                    if ((word[k] & kBias) && !several) x = __fadd_rn(x, bias_vals[j_of(k) - nh]);
                     if (__ballot(several)) x = add_other_bias(several, id_of(k), 0xffffffffu, x, bias_ids, bias_vals, nb);  // (from the first of them)
                     if (c) {
                         x = x > 0.f ? __fdiv_rn(x, P.rep) : __fmul_rn(x, P.rep);
@@ -396,15 +513,22 @@ __device__ __forceinline__ bool twin_row(const BatchArgs& A, const uint32_t row,
                 push(x, id_of(k), word[k] && x > thr, true);
             }
         };
-        constexpr uint32_t kThird = kIds / 3u;
+        if (MASKED && n_few <= few_room) {  // uniform
+            take_touched(std::integral_constant<uint32_t, kFew>{}, [&](uint32_t k) { return ids[k] & kFewId; },
+                         [&](uint32_t k) { return ids[k] <= kFewId ? 0u : nh + (ids[k] >> kFewShift) - 1u; }, 0u, n_few);
+        } else {
+            constexpr uint32_t kThird = kIds / 3u;
 #pragma unroll
-        for (uint32_t h = 0; h < 3u; ++h)
-            if (h * kThird * WS_BLOCK < n_all) take_touched(std::integral_constant<uint32_t, kThird>{}, [&](uint32_t k) { return ids[h * kThird + k]; }, h * kThird * WS_BLOCK);
-        for (uint32_t j0 = kIds * WS_BLOCK; j0 < n_all; j0 += kMore * WS_BLOCK) {
-            uint32_t id[kMore];
+            for (uint32_t h = 0; h < 3u; ++h)
+                if (h * kThird * WS_BLOCK < n_all)
+                    take_touched(std::integral_constant<uint32_t, kThird>{}, [&](uint32_t k) { return ids[h * kThird + k]; },
+                                 [&](uint32_t k) { return (h * kThird + k) * WS_BLOCK + t; }, h * kThird * WS_BLOCK, n_all);
+            for (uint32_t j0 = kIds * WS_BLOCK; j0 < n_all; j0 += kMore * WS_BLOCK) {
+                uint32_t id[kMore];
 #pragma unroll
-            for (uint32_t k = 0; k < kMore; ++k) id[k] = entry(j0 + k * WS_BLOCK + t);
-            take_touched(std::integral_constant<uint32_t, kMore>{}, [&](uint32_t k) { return id[k]; }, j0);
+                for (uint32_t k = 0; k < kMore; ++k) id[k] = entry(j0 + k * WS_BLOCK + t);
+                take_touched(std::integral_constant<uint32_t, kMore>{}, [&](uint32_t k) { return id[k]; }, [&](uint32_t k) { return j0 + k * WS_BLOCK + t; }, j0, n_all);
+            }
         }
         __syncthreads();  // (the tables are done with: the list may take their place)
     }
@@ -416,6 +540,11 @@ __device__ __forceinline__ bool twin_row(const BatchArgs& A, const uint32_t row,
     q_part = vector_at(n_full * WS_BLOCK + t);
     // ---- the sweep: sum of exp, tokens above the threshold to the list
     const bool mapped = MASKED || n_all != 0u;  // uniform
+    // A wave lists its tokens at places that it takes thirty-two of at a time, so that most vectors need no word of the other waves; the few
+    // places left over at the end are filled from the list's end.
+    uint32_t my_next = 0, my_end = 0;  // uniform
+    float my_thr = thr;
+    auto wave_value = [](uint32_t v) __attribute__((always_inline)) { return static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(v))); };
     const float thr_a = __fsub_rn(thr, ref);  // (rounding is monotonous: x > thr makes x - ref, rounded, no smaller than this)
     auto take = [&](const uint4& q, uint32_t word, uint32_t shift, uint32_t i0) __attribute__((always_inline)) {
         const uint32_t w[4] = {q.x, q.y, q.z, q.w};
@@ -430,22 +559,66 @@ __device__ __forceinline__ bool twin_row(const BatchArgs& A, const uint32_t row,
             highest = fmaxf(highest, a);
             (e & 1u ? s1 : s0) += __builtin_amdgcn_exp2f(fmaf(a, k2lo, a * k2));
         }
-        if (__ballot(highest >= thr_a)) {  // uniform: a vector that may have a token for the list (a few per thousand)
+        if (__ballot(highest >= thr_a)) {  // uniform: a vector that may have a token for the list
+            uint64_t on[TPV];
+            uint32_t n = 0;
+            float top = x[0];
 #pragma unroll
-            for (uint32_t e = 0; e < TPV; ++e) push(x[e], i0 + e, x[e] > thr);
+            for (uint32_t e = 0; e < TPV; ++e) {
+                on[e] = __ballot(x[e] > my_thr);
+                n += static_cast<uint32_t>(__popcll(on[e]));
+                if (e) top = fmaxf(top, x[e]);
+            }
+            m = fmaxf(m, top);  // (whatever of it is not listed lies below what is)
+            auto list_at = [&](auto&& at) __attribute__((always_inline)) {
+                uint32_t i = 0;  // uniform
+#pragma unroll
+                for (uint32_t e = 0; e < TPV; ++e) {
+                    if (x[e] > my_thr) {
+                        const uint32_t k = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(on[e] >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(on[e]), 0u));
+                        uint32_t* to = reinterpret_cast<uint32_t*>(list) + 2u * at(k, i);
+                        to[0] = i0 + e;
+                        to[1] = __float_as_uint(x[e]);
+                    }
+                    i += static_cast<uint32_t>(__popcll(on[e]));
+                }
+            };
+            if (n <= my_end - my_next) {  // uniform
+                list_at([&](uint32_t k, uint32_t i) { return k + (my_next + i); });
+                my_next = wave_value(my_next + n);
+            } else {  // the rest of the wave's places, then new ones
+                const uint32_t left = my_end - my_next, more = max(n - left, kTwinPlaces);
+                uint32_t from = 0;
+                if (lane == 0u) from = atomicAdd(&S.s_w[1], more);
+                from = wave_value(from);
+                if (from + more > kShortCap) {
+                    my_thr = INFINITY;  // (the list is full: nothing more to it)
+                } else {
+                    list_at([&](uint32_t k, uint32_t i) { return k + i < left ? k + i + my_next : k + i + (from - left); });
+                    my_next = wave_value(from + (n - left));
+                    my_end = wave_value(from + more);
+                }
+            }
         }
     };
-    auto take_at = [&](const uint4& q, uint32_t j) __attribute__((always_inline)) { take(q, mapped ? invalid[(j * TPV) >> 5] : 0u, (j * TPV) & 31u, j * TPV); };
+    auto take_at = [&](uint4 q, uint32_t j) __attribute__((always_inline)) {  // (every lane of a wave: those past the row bring NaN)
+        if (j >= nv) q = make_uint4(0xffffffffu, 0xffffffffu, 0xffffffffu, 0xffffffffu);
+        take(q, mapped ? invalid[(min(j, nv - 1u) * TPV) >> 5] : 0u, (j * TPV) & 31u, j * TPV);
+    };
 #pragma unroll
     for (uint32_t k = 0; k < kTwinHead; ++k) {
-        const uint32_t j = k * spread * WS_BLOCK + t;
-        if (j < nv) take_at(hq[k], j);
+        uint32_t j0 = k * spread * WS_BLOCK;
+        asm volatile("" : "+s"(j0));  // (so that no vector's place in the bitmap waits in a register since the vector was asked for)
+        if (j0 < nv) take_at(hq[k], j0 + t);  // uniform
     }
     const uint32_t my_word = (t * TPV) >> 5, my_shift = (t * TPV) & 31u;
     auto eat = [&](const uint4 (&q)[KB], const uint32_t (&c)[KB]) __attribute__((always_inline)) {
+        uint32_t word[KB];
+#pragma unroll
+        for (uint32_t k = 0; k < KB; ++k) word[k] = mapped ? invalid[min(c[k], n_full - 1u) * (WS_BLOCK * TPV / 32u) + my_word] : 0u;
 #pragma unroll
         for (uint32_t k = 0; k < KB; ++k)
-            if (c[k] < n_full) take(q[k], mapped ? invalid[c[k] * (WS_BLOCK * TPV / 32u) + my_word] : 0u, my_shift, (c[k] * WS_BLOCK + t) * TPV);  // uniform
+            if (c[k] < n_full) take(q[k], word[k], my_shift, (c[k] * WS_BLOCK + t) * TPV);  // uniform
     };
     for (uint32_t i = kTwinHead; i < n_full; i += 2u * KB) {
         eat(qa, ca);
@@ -453,7 +626,7 @@ __device__ __forceinline__ bool twin_row(const BatchArgs& A, const uint32_t row,
         eat(qb, cb);
         load(qb, cb);
     }
-    if (!whole && n_full * WS_BLOCK + t < nv) take_at(q_part, n_full * WS_BLOCK + t);
+    if (!whole && n_full * WS_BLOCK < nv) take_at(q_part, n_full * WS_BLOCK + t);  // uniform
     if (n_odd) {  // uniform: the tokens behind the last whole vector
         float x = -INFINITY;
         const uint32_t id = nv * TPV + t;
@@ -474,6 +647,8 @@ __device__ __forceinline__ bool twin_row(const BatchArgs& A, const uint32_t row,
         if (lane == 0u) {
             S.red_f[wv] = wm_;
             S.red_d[wv] = ws_;
+            S.bstart[wv] = my_next;
+            S.bcnt[wv] = my_end - my_next;
         }
         __syncthreads();
         m = S.red_f[0];
@@ -485,11 +660,43 @@ __device__ __forceinline__ bool twin_row(const BatchArgs& A, const uint32_t row,
         }
     }
     WSS_MARK(5);
-    uint32_t n_list = S.s_w[1];
+    uint32_t n_list = S.s_w[1], n_left = 0;
+    {  // the places no wave has filled: the last n_left of the list take their contents to the others
+#pragma unroll
+        for (uint32_t w = 0; w < WS_WAVES; ++w) n_left += S.bcnt[w];
+        if (n_list <= kShortCap && n_left) {  // uniform
+            n_list -= n_left;
+            // (a wave has 64 of them; one wave for all of them took 1 us longer)
+            const uint32_t first = n_list + wv * 64u, from = first + lane;
+            if (wv * 64u < n_left) {  // uniform
+                bool filled = wv * 64u + lane < n_left;
+                uint32_t r = wv * 64u;  // how many of the waves before have contents
+#pragma unroll
+                for (uint32_t w = 0; w < WS_WAVES; ++w) {
+                    const uint32_t at = S.bstart[w], end = at + S.bcnt[w];
+                    filled = filled && !(from >= at && from < end);
+                    r -= max(min(end, first), n_list) - min(max(at, n_list), max(min(end, first), n_list));
+                }
+                const uint64_t on = __ballot(filled);
+                r += __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(on >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(on), 0u));
+                uint32_t to = from;
+#pragma unroll
+                for (uint32_t w = 0; w < WS_WAVES; ++w) {  // the r-th place that lies below the list's end
+                    const uint32_t at = S.bstart[w], n = at < n_list ? min(S.bcnt[w], n_list - at) : 0u;
+                    if (r < n) to = at + r;
+                    r = r < n ? 0xffffffffu : r - n;
+                }
+                if (filled) list[to] = list[from];
+            }
+            __syncthreads();
+        }
+    }
     if (by_p && n_list > kShortCap) {
         // A min-p row whose sample's maximum lies well below its own: the floor is known now, and the row is read once more, for the list alone.
         // (All of it, not what lies above the list's lowest: a row's sum has been taken. Of 65 rows of 50257 3 came this way.)
-        thr = fmaxf(thr, __fadd_rn(m, __fdiv_rn(static_cast<float>(log(min_p)) - 0.02f, inv_t)));
+        double floor_ = min_p;
+        asm volatile("" : "+v"(floor_));  // (so that nothing of its logarithm waits in registers from the threshold on)
+        thr = fmaxf(thr, __fadd_rn(m, __fdiv_rn(static_cast<float>(log(floor_)) - 0.02f, inv_t)));
         __syncthreads();
         if (t == 0) S.s_w[1] = S.s_w[3];
         __syncthreads();
@@ -516,6 +723,10 @@ __device__ __forceinline__ bool twin_row(const BatchArgs& A, const uint32_t row,
     }
     const uint32_t n_cand = by_k ? top_k : n_list;  // candidates the rules look at
     if (S.s_w[2] != 0u || n_list > kShortCap || !(m > -INFINITY) || !(__fsub_rn(m, ref) * inv_t < 80.f) || n_list < n_cand || n_cand == 0u) return false;
+    for (uint32_t k = t; k < n_list; k += WS_BLOCK) list[k] = key64(__uint_as_float(static_cast<uint32_t>(list[k] >> 32)), static_cast<uint32_t>(list[k]));
+    if (n_list <= WS_BLOCK / 4u) __syncthreads();  // (the sort of a short list begins with other threads' keys; a longer list's with a thread's own)
+    float inv_t_ = inv_t;
+    asm volatile("" : "+v"(inv_t_));  // (so that its 64-bit value does not wait in registers from the sweep on)
     // Tokens above `ref` can be most of the sum, and the larger the exponent, the less of a fraction 32 bits leave it (1.2e-6 of
     // the normaliser where the maximum lies 60 units above the sample's; 2e-7 up to the four units below which nothing is done):
     // they are all on the list, and their terms are taken out and put back in 64 bits.
@@ -523,7 +734,7 @@ __device__ __forceinline__ bool twin_row(const BatchArgs& A, const uint32_t row,
         double more = 0.0;
         for (uint32_t k = t; k < n_list; k += WS_BLOCK) {
             const float x = unkey32(static_cast<uint32_t>(list[k] >> 32));
-            if (x > ref) more += exp((static_cast<double>(x) - static_cast<double>(ref)) * static_cast<double>(inv_t)) - static_cast<double>(term(x));
+            if (x > ref) more += exp((static_cast<double>(x) - static_cast<double>(ref)) * static_cast<double>(inv_t_)) - static_cast<double>(term(x));
         }
         z += block_sum(more, S.red_d);
     }
@@ -537,8 +748,8 @@ __device__ __forceinline__ bool twin_row(const BatchArgs& A, const uint32_t row,
     R.top_p = top_p;
     R.min_p = min_p;
     R.u = batch_uniform(A.rng, P.seed, row, P.step, 0);
-    R.z = z * exp((static_cast<double>(ref) - static_cast<double>(m)) * static_cast<double>(inv_t));
-    R.inv_t = inv_t;
+    R.z = z * exp((static_cast<double>(ref) - static_cast<double>(m)) * static_cast<double>(inv_t_));
+    R.inv_t = inv_t_;
     R.m = m;
     R.n_cand = n_cand;
     R.by_k = by_k;
