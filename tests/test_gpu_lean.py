@@ -327,3 +327,17 @@ def test_short_rows_off_the_boundaries(V, ids, masked, lean):
     res = gc.compare_rows(c, smp, range(3), 1, check_kept=False)
     assert res["exact"] == 3, res
     assert (((smp.flags & m.FLAG_ROUTE_LEAN) != 0) == lean).all(), smp.flags
+
+
+@pytest.mark.parametrize("V,share", [(50257, 0.02), (151936, 0.17), (163837, 0.5)])
+def test_masked_out_tokens_under_every_byte(V, share):
+    """Nearly all of a row masked out, and cuts and draws under many different bytes (temperatures from 0.3 to 2): what is masked out is found with every one
+    of them and dropped."""
+    c = _no_top_k(gc.make_cfg2(rows=16, V=V, n_hist=100, n_bias=20))
+    c["top_p"] = np.linspace(0.5, 0.95, 16)
+    c["inv_t"] = np.linspace(0.5, 3.3, 16).astype(np.float32)
+    c["min_p"][:] = 0.0
+    rng = np.random.default_rng(V)
+    c["allow"] = np.ascontiguousarray(np.packbits(rng.random((16, (V + 31) // 32 * 32)) < share, axis=1, bitorder="little").view(np.uint32))
+    res, _ = run_lean(c, 1, max_differ=1, handed_back=1)
+    assert res["exact"] >= 15, res
