@@ -329,7 +329,56 @@ def test_short_rows_off_the_boundaries(V, ids, masked, lean):
     assert (((smp.flags & m.FLAG_ROUTE_LEAN) != 0) == lean).all(), smp.flags
 
 
-@pytest.mark.parametrize("V,share", [(50257, 0.02), (151936, 0.17), (163837, 0.5)])
+@pytest.mark.parametrize("V,masked,n_hist", [(V, masked, n_hist) for V in (163841, 163844, 163848, 172032, 200003, 262136, 262143, 262144) for masked in (False, True) for n_hist in (0, 700)] +
+                         [(262144, True, 3000), (200000, False, 4000)])
+def test_rows_longer_than_the_shorter_bin_cache(V, masked, n_hist):
+    """Rows of 163841 to 262144 tokens, one sweep as well: whole vectors and not, whole rounds and not, with touched tokens, the largest logits and masked-out
+    tokens in the last vector."""
+    c = _no_top_k(gc.make_cfg2(rows=5, V=V, n_hist=n_hist, n_bias=50 if n_hist else 0))
+    c["top_p"] = np.minimum(c["top_p"], 0.95)
+    for r in range(5):
+        if n_hist:
+            c["hist"][r][:2] = [V - 1, V - 1 - r % 4]
+        c["logits"][r, V - 1 - (r * 3) % 8] = 9.0 + r
+    if masked:
+        rng = np.random.default_rng(V)
+        c["allow"] = rng.integers(0, 1 << 32, (5, (V + 31) // 32), dtype=np.uint64).astype(np.uint32) | np.uint32(0x10000001)
+        c["logits"][:2, :500:40] = 14.0
+    res, _ = run_lean(c, 1, handed_back=1)
+    assert res["exact"] == 5, res
+
+
+@pytest.mark.parametrize("lists,masked", [(False, False), (True, True)])
+def test_long_rows_are_swept_once_more_as_well(lists, masked):
+    test_maximum_above_the_bins_is_swept_once_more(262144, lists, masked)
+
+
+@pytest.mark.parametrize("kind,sigma,V", [("normal", 2.0, 262144), ("zipf", 0.4, 200003)])
+def test_normaliser_of_long_rows(kind, sigma, V):
+    test_normaliser_as_close_as_three_sweeps(kind, sigma, V)
+
+
+@pytest.mark.parametrize("V,masked", [(262144, False), (200003, True)])
+def test_more_finds_than_the_list_holds(V, masked):
+    """The cut and the draw fall among 3000 tokens, and 20000 others lie 256 bins below those: their cached bytes are the same, and all are found. A long row
+    looks at each before it lists it; it is not handed back."""
+    c = _no_top_k(gc.make_cfg2(rows=4, V=V, n_hist=64, n_bias=8))
+    c["inv_t"][:], c["top_p"][:], c["min_p"][:] = 1.0, 0.8, 0.0
+    rng = np.random.default_rng(V)
+    for r in range(4):
+        x = np.full(V, -30.0, np.float32)
+        at = rng.permutation(V)[:23000]
+        x[at] = -1.0 + rng.uniform(0.0, 0.012, 23000).astype(np.float32)
+        x[at[3000:]] -= 4.0
+        c["logits"][r] = x
+    if masked:
+        c["allow"] = (rng.random((4, (V + 31) // 32 * 32)) < 0.9)
+        c["allow"] = np.ascontiguousarray(np.packbits(c["allow"], axis=1, bitorder="little").view(np.uint32))
+    res, _ = run_lean(c, 1)
+    assert res["exact"] == 4 and res["handed_back"] == 0, res
+
+
+@pytest.mark.parametrize("V,share", [(50257, 0.02), (151936, 0.17), (262144, 0.5)])
 def test_masked_out_tokens_under_every_byte(V, share):
     """Nearly all of a row masked out, and cuts and draws under many different bytes (temperatures from 0.3 to 2): what is masked out is found with every one
     of them and dropped."""

@@ -350,9 +350,13 @@ BatchPlan plan_batch(const ws_batch* b, bool few = true) {
     //     masked, 64 ids: 1 row of 8193 22.9 / 24.8, 12001 23.7 / 25.4, 16387 24.8 / 25.7, 24001 27.8 / 25.7; 256 rows of 8193 24.7 / 27.6, 16387 28.8 / 27.4; 500 ids: level at 8193
     // Rows without a filter are none of its own either: of a batch that has neither top-p nor min-p it would hand back every one (three sweeps and this kernel: 1 row of
     // 50257 40 / 44, 256 rows 51 / 61, 256 of 151937 with 500 ids 117 / 125; the other single-sweep kernel and this one: 256 rows of 50256 52 / 61, of 151936 87 / 109).
+    // Rows of 163841 to 262144 tokens, which no other single-sweep kernel takes, have their build of it with the longer bin cache (us, three sweeps and this; top-p 0.9):
+    //   1 row of 262144 69 / 47, 64 of 200000 with 500 ids 84 / 53, 32 of 163841 65 / 42, 256 of 262144 with 2000 ids 128 / 93, 200 Zipfian of 262144 with 3000 135 / 93, 100 of
+    //   200000 65 / 50; raised tokens: 16 of 256000 114 / 53, 256 of 163848 with 64 ids 83 / 67; masked: 88 of 248576, 17 % allowed, 94 / 58, 281 of 204976, 15 %, 150 / 119
+    //   Rows whose cut no list holds are handed back after a sweep in vain: 200 flat Zipfian rows of 262144, T up to 1.4, 845 / 891.
     const uint32_t lean_least = vec_rows ? 8u : (cap >= (b->allow ? 512u : 128u) ? 8192u : (cap ? (b->allow ? 20480u : 16384u) : (b->allow ? 32768u : 20480u)));
-    p.lean = (p.fused || !vec_rows) && (b->top_p || b->min_p) && b->dtype == WS_DTYPE_F32 && b->mode == WS_MODE_AUTO && !b->top_k && !b->kept_ids && !b->query_prob && !wants_entropy && !b->race &&
-             b->vocab >= lean_least && b->vocab <= 163840u && (!b->bias_ids || b->max_bias <= 2047u) && fused_total + kStaticLean <= kMaxLds;
+    p.lean = (p.fused || !vec_rows || b->vocab > 163840u) && (b->top_p || b->min_p) && b->dtype == WS_DTYPE_F32 && b->mode == WS_MODE_AUTO && !b->top_k && !b->kept_ids && !b->query_prob && !wants_entropy && !b->race &&
+             b->vocab >= lean_least && b->vocab <= 262144u && (!b->bias_ids || b->max_bias <= 2047u) && fused_total + kStaticLean <= kMaxLds;
     if (p.lean) {
         p.lds_ab = 65536u;
         p.lds_cnt = static_cast<uint32_t>(65536u + maps);

@@ -29,7 +29,9 @@
 
 namespace ws {
 
-constexpr int kLeanRegs = 40;   // bin-cache registers per thread: 160 tokens, rows of up to 163840 tokens
+// bin-cache registers per thread: 160 tokens, rows of up to 163840 tokens; or 256 tokens, rows of up to 262144 (a build of its own: a quarter of them lie in
+// scratch memory behind the sweep, which is still far from the two more sweeps that such rows took: see ws_abi.hip)
+constexpr int kLeanRegs = 40, kLeanRegsLong = 64;
 constexpr int kLeanBatch = 2;   // 128-bit loads per thread and batch
 constexpr uint32_t kLeanBuckets = 128u;   // words of the finish's tables in LeanShared
 constexpr uint32_t kLeanMaxList = 4096u;  // candidates of a row's ranges together: what the sort's 32 KiB hold
@@ -132,23 +134,27 @@ __device__ __forceinline__ uint32_t lean_flags(uint32_t y, const uint32_t (&c4)[
 
 // What a thread's scan of its bin cache found: per group of 8 registers (32 tokens) the first two tokens whose cached byte
 // equals one of the bytes asked for, with their logits requested right there (the loads travel while the scan goes on).
-constexpr int kLeanGroups = kLeanRegs / 8;
+template <int NREG>
 struct LeanHits {
-    uint32_t idx[2 * kLeanGroups];   // token index, 0xffffffff = none
-    uint32_t bits[2 * kLeanGroups];  // its logit as loaded
+    static constexpr int kGroups = NREG / 8;
+    uint32_t idx[2 * kGroups];   // token index, 0xffffffff = none
+    uint32_t bits[2 * kGroups];  // its logit as loaded
 };
 
 // A third token of a group and beyond goes to list[] as (token | kListNeedsLoad, 0), one LDS atomic each (rare). With
 // TO_LIST every find goes there (a second round of bytes). V: the row's tokens.
-template <int NT, bool TO_LIST>
-__device__ __forceinline__ void lean_scan(const uint32_t (&cache)[kLeanRegs], const uint32_t (&c4)[4], const void* __restrict__ xg, LeanHits& H,
-                                          uint2* list, uint32_t* n_list, uint32_t cap, uint32_t V) {
+// wanted(logit bits): only such a find goes to the list, with its logit (nullptr: as above).
+template <int NT, bool TO_LIST, int NREG, class WANTED = std::nullptr_t>
+__device__ __forceinline__ void lean_scan(const uint32_t (&cache)[NREG], const uint32_t (&c4)[4], const void* __restrict__ xg, LeanHits<NREG>& H,
+                                          uint2* list, uint32_t* n_list, uint32_t cap, uint32_t V, WANTED&& wanted = nullptr) {
+    constexpr bool LOOK = !std::is_same_v<std::decay_t<WANTED>, std::nullptr_t>;
+    constexpr int kGroups = LeanHits<NREG>::kGroups;
     const uint32_t t = threadIdx.x, nv = V >> 2;  // (whole vectors; of the one that the row may end in only the row's tokens are looked at)
     auto logit_bits = [&](uint32_t i) {
         return static_cast<const uint32_t*>(xg)[i];
     };
 #pragma unroll
-    for (int g = 0; g < kLeanGroups; ++g) {
+    for (int g = 0; g < kGroups; ++g) {
         // where the row ends is looked at per group, uniformly: a group past the row is skipped, the one group the end
         // falls in masks its finds, the others need no test
         uint32_t acc = 0;
@@ -170,8 +176,8 @@ __device__ __forceinline__ void lean_scan(const uint32_t (&cache)[kLeanRegs], co
             return ((reg * WS_BLOCK + t) << 2) + (bit >> 3);
         };
         if (!TO_LIST) {
-            H.idx[g] = H.idx[kLeanGroups + g] = 0xffffffffu;
-            H.bits[g] = H.bits[kLeanGroups + g] = 0u;
+            H.idx[g] = H.idx[kGroups + g] = 0xffffffffu;
+            H.bits[g] = H.bits[kGroups + g] = 0u;
             if (acc) {
                 const uint32_t i = token_of(static_cast<uint32_t>(__ffs(acc)) - 1u);
                 acc &= acc - 1u;
@@ -181,15 +187,20 @@ __device__ __forceinline__ void lean_scan(const uint32_t (&cache)[kLeanRegs], co
             if (acc) {
                 const uint32_t i = token_of(static_cast<uint32_t>(__ffs(acc)) - 1u);
                 acc &= acc - 1u;
-                H.idx[kLeanGroups + g] = i;
-                H.bits[kLeanGroups + g] = logit_bits(i);
+                H.idx[kGroups + g] = i;
+                H.bits[kGroups + g] = logit_bits(i);
             }
         }
         while (acc) {
             const uint32_t i = token_of(static_cast<uint32_t>(__ffs(acc)) - 1u);
             acc &= acc - 1u;
+            uint32_t bits = 0u;
+            if constexpr (LOOK) {
+                bits = logit_bits(i);
+                if (!wanted(bits)) continue;
+            }
             const uint32_t slot = atomicAdd(n_list, 1u);
-            if (slot < cap) list[slot] = make_uint2(i | kListNeedsLoad, 0u);
+            if (slot < cap) list[slot] = make_uint2(LOOK ? i : i | kListNeedsLoad, bits);
         }
     }
 }
@@ -404,7 +415,7 @@ __device__ __forceinline__ double sel_dbg(const LeanShared& S) { return S.sel.n_
 #endif
 // One row. Returns false when the row is left to others (nothing has been written for it then): S.top is NaN, and it is the three-pass code's; or the row's maximum,
 // and it is to be swept once more from there down (AGAIN; its arguments are at `args`).
-template <bool MASKED, bool AGAIN>
+template <bool MASKED, bool AGAIN, int NREG>
 __device__ __forceinline__ bool lean_row(const BatchArgs& A, const LeanArgPtr args, const uint32_t row, LeanShared& S) {
     constexpr uint32_t kTok = 4u, kTokLog = 2u;  // tokens in a 128-bit vector, which is one register of the bin cache: the low eight bits of each bin
     // (a scan for a bin also finds the tokens of the bins 256 apart, some hundreds each, and drops them afterwards)
@@ -445,7 +456,7 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const LeanArgPtr ar
     // the history ids are fetched, two dependent trips to memory; the first kEarly batches are binned before those ids
     // are looked at (what the ids touch there is put right afterwards), so that phase 0 costs its LDS work and no wait.
     constexpr int kRing = 3, kEarly = WS_LEAN_EARLY;
-    constexpr int NB = kLeanRegs / kLeanBatch;
+    constexpr int NB = NREG / kLeanBatch;
     uint4 q[kRing][kLeanBatch];
     uint32_t na[kRing][kLeanBatch];
     auto load = [&](int bt, int slot) __attribute__((always_inline)) {
@@ -539,7 +550,7 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const LeanArgPtr ar
     }
 
     // ------------------------------------------------------------------ the sweep
-    uint32_t cache[kLeanRegs];
+    uint32_t cache[NREG];
     float m = -INFINITY;
     float vm_early[kEarly * kLeanBatch];  // maxima of the early batches' vectors, until the bitmap says which hold a touched token
     const float tail_f = static_cast<float>(kLeanRoom - kLeanTail - static_cast<int>(t));  // the height of this thread's own tail bin
@@ -628,7 +639,7 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const LeanArgPtr ar
             if (id < V) atomicOr(&touched[id >> 5], 1u << (id & 31u));
         }
         __syncthreads();
-        constexpr uint32_t kChunk = 5;  // 163840 / 32 / 1024 words per thread
+        constexpr uint32_t kChunk = NREG / 8;  // words per thread: NREG * 4096 / 32 / 1024
         const uint32_t w0 = t * kChunk;
         uint32_t wd[kChunk], local = 0;
 #pragma unroll
@@ -1167,7 +1178,8 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const LeanArgPtr ar
         return b - u0 <= w0 || b - u1r <= w1;
     };
     {
-        LeanHits H;
+        LeanHits<NREG> H;
+        constexpr int kGroups = LeanHits<NREG>::kGroups;
         const void* xg = rv.base;
         const uint32_t nt = sel.n_bytes;
         const uint4 by0 = *reinterpret_cast<const uint4*>(&sel.bytes[0]);
@@ -1186,26 +1198,47 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const LeanArgPtr ar
         }
         WSL_MARK(20);
         // touched tokens whose adjusted logit lies in the ranges
-        for (uint32_t r = t; r < n_touched; r += WS_BLOCK) {
-            const float x = pv[r];
-            if (in_ranges(x)) {
-                const uint32_t slot = atomicAdd(&s_w[0], 1u);
-                if (slot < kListCap) list[slot] = make_uint2(first[r] | kListAdjusted, __float_as_uint(x));
+        auto list_touched = [&]() __attribute__((always_inline)) {
+            for (uint32_t r = t; r < n_touched; r += WS_BLOCK) {
+                const float x = pv[r];
+                if (in_ranges(x)) {
+                    const uint32_t slot = atomicAdd(&s_w[0], 1u);
+                    if (slot < kListCap) list[slot] = make_uint2(first[r] | kListAdjusted, __float_as_uint(x));
+                }
             }
-        }
+        };
+        list_touched();
         WSL_MARK(21);
         uint32_t mine = 0;
 #pragma unroll
-        for (int k = 0; k < 2 * kLeanGroups; ++k) mine += H.idx[k] != 0xffffffffu ? 1u : 0u;
+        for (int k = 0; k < 2 * kGroups; ++k) mine += H.idx[k] != 0xffffffffu ? 1u : 0u;
         const uint32_t inc = wave_incl_scan(mine);
         uint32_t base = 0;
         if (lane == 63u && inc) base = atomicAdd(&s_w[0], inc);
         uint32_t slot = __shfl(base, 63) + inc - mine;
 #pragma unroll
-        for (int k = 0; k < 2 * kLeanGroups; ++k) {
+        for (int k = 0; k < 2 * kGroups; ++k) {
             if (H.idx[k] == 0xffffffffu) continue;
             if (slot < kListCap) list[slot] = make_uint2(H.idx[k], H.bits[k]);
             ++slot;
+        }
+        if constexpr (NREG > kLeanRegs) {
+            // A long row whose finds are more than the list holds (a byte finds a thousand tokens of 262144): once more, and each find is looked at before it is
+            // listed, one after the other - 20 us, a quarter of what the three-pass code takes.
+            __syncthreads();
+            if (s_w[0] > kListCap) {  // uniform
+                __syncthreads();
+                if (t == 0u) s_w[0] = 0u;
+                __syncthreads();
+                auto wanted = [&](uint32_t bits) { return in_ranges(fmaxf(__uint_as_float(bits), -INFINITY)); };
+#pragma unroll 1
+                for (uint32_t b0_ = 0; b0_ < nt; b0_ += 4u) {
+                    const uint4 by = *reinterpret_cast<const uint4*>(&sel.bytes[b0_]);
+                    const uint32_t c4[4] = {by.x, nt > b0_ + 1u ? by.y : by.x, nt > b0_ + 2u ? by.z : by.x, nt > b0_ + 3u ? by.w : by.x};
+                    lean_scan<4, true>(cache, c4, xg, H, list, &s_w[0], kListCap, V, wanted);
+                }
+                list_touched();
+            }
         }
     }
     WSL_MARK(22);
@@ -1590,28 +1623,28 @@ __device__ __noinline__ __attribute__((not_tail_called)) void three_pass_row(Lea
 }
 
 // What lean_row has left of a row. (A function of its own, as above: as a loop around that code in the kernel it cost the kernel some hundred spilled registers.)
-template <bool MASKED>
+template <bool MASKED, int NREG>
 __device__ __noinline__ __attribute__((not_tail_called)) void lean_rest(LeanArgPtr Ap_, const uint32_t row_, __attribute__((address_space(3))) LeanShared* S) {
     LeanArgPtr Ap = wave_args(Ap_);
     const uint32_t row = __builtin_amdgcn_readfirstlane(row_);
     const float top = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(S->top)));
     if (top == top) {
-        if (lean_row<MASKED, true>(*(const BatchArgs*)Ap, Ap, row, *(LeanShared*)S)) return;
+        if (lean_row<MASKED, true, NREG>(*(const BatchArgs*)Ap, Ap, row, *(LeanShared*)S)) return;
         __syncthreads();
     }
     three_pass_row<false>(Ap, row);
 }
 
 // MASKED: the batch has an allow mask (a kernel of its own: one build carrying both paths spilled far more registers)
-template <bool MASKED>
+template <bool MASKED, int NREG>
 __global__ void __launch_bounds__(WS_BLOCK) lean_batch_kernel(BatchArgs A) {
     __shared__ LeanShared shared;
     const uint32_t row = blockIdx.x;
-    if (lean_row<MASKED, false>(A, nullptr, row, shared)) return;
+    if (lean_row<MASKED, false, NREG>(A, nullptr, row, shared)) return;
     __syncthreads();  // whatever the lean path left in LDS is dead
     LeanArgPtr Ap = (LeanArgPtr)__builtin_amdgcn_kernarg_segment_ptr();
     asm volatile("" : "+s"(Ap));
-    lean_rest<MASKED>(Ap, row, (__attribute__((address_space(3))) LeanShared*)&shared);
+    lean_rest<MASKED, NREG>(Ap, row, (__attribute__((address_space(3))) LeanShared*)&shared);
 }
 
 }  // namespace ws
