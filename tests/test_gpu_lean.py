@@ -390,3 +390,19 @@ def test_masked_out_tokens_under_every_byte(V, share):
     c["allow"] = np.ascontiguousarray(np.packbits(rng.random((16, (V + 31) // 32 * 32)) < share, axis=1, bitorder="little").view(np.uint32))
     res, _ = run_lean(c, 1, max_differ=1, handed_back=1)
     assert res["exact"] >= 15, res
+
+
+@pytest.mark.parametrize("V", [V + d for V in (32768, 49152, 65536, 98304, 131072, 155648, 163840) for d in (0, 1, 8)])
+@pytest.mark.parametrize("masked", [False, True])
+def test_rows_at_the_ends_of_the_bin_caches(V, masked):
+    """One token more than a build's bin cache holds, and a row that fills it: the largest logits and touched tokens in the last vector."""
+    c = _no_top_k(gc.make_cfg2(rows=3, V=V, n_hist=600, n_bias=30))
+    c["top_p"] = np.minimum(c["top_p"], 0.95)
+    for r in range(3):
+        c["hist"][r][:2] = [V - 1, V - 1 - r]
+        c["logits"][r, V - 1 - (r * 3) % 8] = 9.0 + r
+    if masked:
+        rng = np.random.default_rng(V)
+        c["allow"] = rng.integers(0, 1 << 32, (3, (V + 31) // 32), dtype=np.uint64).astype(np.uint32) | np.uint32(0x10000001)
+    res, _ = run_lean(c, 1, handed_back=1)
+    assert res["exact"] == 3, res

@@ -29,9 +29,13 @@
 
 namespace ws {
 
-// bin-cache registers per thread: 160 tokens, rows of up to 163840 tokens; or 256 tokens, rows of up to 262144 (a build of its own: a quarter of them lie in
-// scratch memory behind the sweep, which is still far from the two more sweeps that such rows took: see ws_abi.hip)
-constexpr int kLeanRegs = 40, kLeanRegsLong = 64;
+// Registers of the bin cache a thread, four tokens each: builds for rows of up to 32768, 49152, 65536, 98304, 131072 (ws_lean_short.hip), 155648, 163840 and 262144
+// tokens (ws_lean.hip), and a row gets the shortest that holds it. The loads past a row's end are asked for like the others - they may not lie behind a branch -, 64
+// lanes at one address each: a row of 25000 tokens waited 8 K clocks of 46 K for them in the build of 40 (us, that one and its own: 54 rows of 25792 20.1 / 17.3, 34 of
+// 35392 25.3 / 22.0, 256 of 32000 with 1000 ids 26.5 / 21.6, 200 of 50257 27.9 / 24.3, 100 of 98304 30.9 / 29.0). Of the longest a quarter of the cache lies in scratch
+// memory behind the sweep, which is still far from the two more sweeps that such rows took (ws_abi.hip).
+constexpr int kLeanRegsShort[] = {8, 12, 16, 24, 32}, kLeanRegsLong[] = {38, 40, 64};
+constexpr int kLeanLooks = 64;  // from here on finds are looked at before they are listed, when they are too many
 constexpr int kLeanBatch = 2;   // 128-bit loads per thread and batch
 constexpr uint32_t kLeanBuckets = 128u;   // words of the finish's tables in LeanShared
 constexpr uint32_t kLeanMaxList = 4096u;  // candidates of a row's ranges together: what the sort's 32 KiB hold
@@ -136,7 +140,7 @@ __device__ __forceinline__ uint32_t lean_flags(uint32_t y, const uint32_t (&c4)[
 // equals one of the bytes asked for, with their logits requested right there (the loads travel while the scan goes on).
 template <int NREG>
 struct LeanHits {
-    static constexpr int kGroups = NREG / 8;
+    static constexpr int kGroups = (NREG + 7) / 8;  // (the last may have fewer than eight registers)
     uint32_t idx[2 * kGroups];   // token index, 0xffffffff = none
     uint32_t bits[2 * kGroups];  // its logit as loaded
 };
@@ -161,11 +165,11 @@ __device__ __forceinline__ void lean_scan(const uint32_t (&cache)[NREG], const u
         const uint32_t g_lo = static_cast<uint32_t>(g * 8) * WS_BLOCK;
         if (g_lo + 8u * WS_BLOCK <= nv) {
 #pragma unroll
-            for (int r = 0; r < 8; ++r)  // bit 8 e + r: token e of register r
+            for (int r = 0; r < 8 && g * 8 + r < NREG; ++r)  // bit 8 e + r: token e of register r
                 acc = ((lean_flags<NT>(cache[g * 8 + r], c4) >> (7 - r)) & (0x01010101u << r)) | acc;
         } else if (g_lo * 4u < V) {
 #pragma unroll
-            for (int r = 0; r < 8; ++r) {
+            for (int r = 0; r < 8 && g * 8 + r < NREG; ++r) {
                 const uint32_t j = g_lo + static_cast<uint32_t>(r) * WS_BLOCK + t;
                 const uint32_t keep = (j < nv ? 0x01010101u : (j == nv ? 0x00010101u >> (8u * (3u - (V & 3u))) : 0u)) << r;
                 acc = ((lean_flags<NT>(cache[g * 8 + r], c4) >> (7 - r)) & keep) | acc;
@@ -639,7 +643,7 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const LeanArgPtr ar
             if (id < V) atomicOr(&touched[id >> 5], 1u << (id & 31u));
         }
         __syncthreads();
-        constexpr uint32_t kChunk = NREG / 8;  // words per thread: NREG * 4096 / 32 / 1024
+        constexpr uint32_t kChunk = (NREG + 7) / 8;  // words per thread: NREG * 4096 / 32 / 1024
         const uint32_t w0 = t * kChunk;
         uint32_t wd[kChunk], local = 0;
 #pragma unroll
@@ -706,7 +710,7 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const LeanArgPtr ar
             WSL_MARK(11);
             phase0();
         }
-        if (bt == NB - 4) exp_tab = t < 64 ? kExpHi[t] : (t < 128 ? kExpLo[t - 64] : 0.0);  // the histogram scan's tables: asked for now, parked in LDS after the sweep
+        if (bt == (NB > 4 ? NB - 4 : 0)) exp_tab = t < 64 ? kExpHi[t] : (t < 128 ? kExpLo[t - 64] : 0.0);  // the histogram scan's tables: asked for now, parked in LDS after the sweep
         if (bt < kEarly) {
             WSL_SWEEP_BATCH(bt, true)
         } else if (static_cast<uint32_t>(bt * kLeanBatch) * WS_BLOCK < nv) {  // uniform
@@ -717,6 +721,7 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const LeanArgPtr ar
         }
         if (bt + kRing < NB) load(bt + kRing, bt % kRing);  // the slot is free: the batch three ahead
     }
+    if constexpr (NB <= kEarly) phase0();
     if (t < 128) s_exp[t] = exp_tab;
 #undef WSL_SWEEP_BATCH
     __syncthreads();
@@ -1222,7 +1227,7 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const LeanArgPtr ar
             if (slot < kListCap) list[slot] = make_uint2(H.idx[k], H.bits[k]);
             ++slot;
         }
-        if constexpr (NREG > kLeanRegs) {
+        if constexpr (NREG >= kLeanLooks) {
             // A long row whose finds are more than the list holds (a byte finds a thousand tokens of 262144): once more, and each find is looked at before it is
             // listed, one after the other - 20 us, a quarter of what the three-pass code takes.
             __syncthreads();
