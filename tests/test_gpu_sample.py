@@ -372,3 +372,24 @@ def test_random_shapes_filters_and_masks_both_kernels():
         gc.workloads.DATA_SEED = seed0
     print(tot)
     assert tot["exact"] == tot["rows"], tot
+
+
+@pytest.mark.parametrize("V", [V + d for V in (16384, 32768, 65536, 98304, 131072) for d in (0, 8)])
+@pytest.mark.parametrize("masked", [False, True])
+def test_unhinted_rows_at_the_ends_of_the_bin_caches(V, masked):
+    """Batches of which nothing is known, rows with a top-k and without, unshared: a row that fills a build's bin cache and one of the next build's, with the largest
+    logits and touched tokens in the last vector."""
+    c = gc.make_cfg2(rows=6, V=V, n_hist=600, n_bias=30)
+    c["top_k"] = np.array([0, 50, 0, 1000, 20, 0], np.uint32).astype(c["top_k"].dtype)
+    c["top_p"] = np.minimum(c["top_p"], 0.95)
+    for r in range(6):
+        c["hist"][r][:2] = [V - 1, V - 1 - r]
+        c["logits"][r, V - 1 - (r * 3) % 8] = 9.0 + r
+    if masked:
+        rng = np.random.default_rng(V)
+        c["allow"] = rng.integers(0, 1 << 32, (6, (V + 31) // 32), dtype=np.uint64).astype(np.uint32) | np.uint32(0x10000001)
+    d = gc.upload(c)
+    smp = gc.sampler_for(c, d, 1, max_split=1).run()
+    res = gc.compare_rows(c, smp, range(6), 1, check_kept=False)
+    assert res["exact"] + res["differ"] == 6 and res["differ"] <= 1, res
+    assert not (smp.flags.cpu().numpy() & gc.pkg().FLAG_ROUTE_HANDED_BACK).any()

@@ -14,6 +14,7 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 SRC = os.path.join(HERE, "csrc", "ws_abi.hip")
 SRC_FUSED = os.path.join(HERE, "csrc", "ws_fused.hip")  # the single-sweep sampler kernel
+SRC_FUSED_SHORT = os.path.join(HERE, "csrc", "ws_fused_short.hip")  # the same for short rows
 SRC_SPLIT = os.path.join(HERE, "csrc", "ws_split.hip")  # the same kernel for rows split over several workgroups
 SRC_KEPT = [os.path.join(HERE, "csrc", f) for f in ("ws_fused_kept.hip", "ws_split_kept.hip")]  # both once more, with the kept-set dump
 SRC_SHORT = os.path.join(HERE, "csrc", "ws_short.hip")  # the short-list kernel for batches whose rows all have a bounded top-k
@@ -50,7 +51,7 @@ def build(verbose=True):
     # the translation units and the bare code object side by side (each takes a minute or two), then the link
     objdir = os.path.join(HERE, "csrc", "obj")
     os.makedirs(objdir, exist_ok=True)
-    srcs = (SRC, SRC_FUSED, SRC_SPLIT, *SRC_KEPT, *SRC_LEAN, SRC_CODE, SRC_SHORT, SRC_TWIN, SRC_FEW, SRC_TOP)
+    srcs = (SRC, SRC_FUSED, SRC_FUSED_SHORT, SRC_SPLIT, *SRC_KEPT, *SRC_LEAN, SRC_CODE, SRC_SHORT, SRC_TWIN, SRC_FEW, SRC_TOP)
     objs = [os.path.join(objdir, os.path.basename(src)[:-4] + ".o") for src in srcs]
     jobs = [[hipcc, *FLAGS, "-fPIC", "-c", "-o", obj, src] for obj, src in zip(objs, srcs)]
     jobs.append([hipcc, *FLAGS, "--genco", "-o", co, SRC])

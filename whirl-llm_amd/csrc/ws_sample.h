@@ -370,7 +370,8 @@ __device__ __forceinline__ void kept_bounds(double X, uint32_t c, double& zlo, d
 // with their raw logit and moved afterwards. For that their raw logits are needed: a 128-bit vector that holds a
 // touched token is copied as it is to stage[rank of its first touched token] (LDS, stage_cap + 1 slots of 16 bytes), which
 // costs two instructions per token and spares one scattered 4-byte read from HBM per touched token.
-constexpr int kCacheRegs = 163840 / WS_BLOCK / 2;  // 80 with 1024 threads, 160 with 512
+constexpr uint32_t kFusedShort = 131072u;  // rows of up to this many tokens have builds with shorter caches (ws_fused_short.hip)
+constexpr int kCacheTokens = 163840;  // (registers of the cache: 80 with 1024 threads, 160 with 512; half of them for a split row's slice)
 
 // Provisional anchor: the larger of `floor` and the maximum of the thread block's first batch of loads, plus 8 exponent
 // units of headroom; the same registers then feed the sweep. Returns false (nothing binned) when that is not finite.
@@ -1780,7 +1781,8 @@ __device__ __noinline__ ExactOut exact_row(const ExactIn in) {
 // One row (or one part of a split row) by the workgroup that calls it: `block` = row * parts + part. The kernels below
 // are this function; the lean kernel (ws_lean.h) calls the three-pass instantiation for the rows it hands back (BACK: that layout of the LDS,
 // and no workspace. The choices stand where they are used: as functions of a struct they left the compiler another order of registers, and rows of the kernels here took 1 % longer).
-template <bool FUSED, bool SPLIT = false, bool KEPT = true, bool BACK = false>
+// TOKENS: what the bin cache of an unsplit row holds.
+template <bool FUSED, bool SPLIT = false, bool KEPT = true, bool BACK = false, int TOKENS = kCacheTokens>
 __device__ __forceinline__ void sample_row(const BatchArgs& A, const uint32_t block) {
     int32_t* const kept_ids = KEPT ? A.kept_ids : nullptr;
 #ifdef WS_PHASE_TIMERS
@@ -2319,7 +2321,7 @@ __device__ __forceinline__ void sample_row(const BatchArgs& A, const uint32_t bl
     bool cached = false;
     uint64_t* hist2 = FUSED && (BACK ? A.fb_lds_tie : A.lds_tie) ? reinterpret_cast<uint64_t*>(lds + (BACK ? A.fb_lds_tie : A.lds_tie)) : nullptr;  // second copy of the histogram
     // the split kernel's slices are at most half a row (two parts at least): half the registers, and room for everything else
-    constexpr int kCR = SPLIT ? kCacheRegs / 2 : kCacheRegs;
+    constexpr int kCR = TOKENS / WS_BLOCK / (SPLIT ? 4 : 2);
     uint32_t cache[kCR];  // dead code (and no registers) in the exact instantiation
     if (FUSED && !(flags & kBadParam)) {
         // ---------------------------------------------------------------- fused sweep: anchor, histogram, max, bins
@@ -4279,9 +4281,9 @@ __device__ __forceinline__ void sample_row(const BatchArgs& A, const uint32_t bl
     }
 }
 
-template <bool FUSED, bool SPLIT = false, bool KEPT = true>
+template <bool FUSED, bool SPLIT = false, bool KEPT = true, int TOKENS = kCacheTokens>
 __global__ void __launch_bounds__(WS_BLOCK) sample_batch_kernel(BatchArgs A) {
-    sample_row<FUSED, SPLIT, KEPT>(A, blockIdx.x);
+    sample_row<FUSED, SPLIT, KEPT, false, TOKENS>(A, blockIdx.x);
 }
 
 }  // namespace ws
