@@ -178,3 +178,20 @@ def test_masks_that_allow_the_whole_history(V, n_hist, n_bias, allowed, dtype):
     if not n_bias:
         c["bias_ids"] = c["bias_vals"] = None
     run_short(c if n_bias < 3 else twice_biased(c), 1, rows=some(rows, 41))
+
+
+@pytest.mark.parametrize("V,top_k,step,allowed", [(50257, 513, 0.0, None), (50257, 1024, 0.0, 0.5), (700, 700, 0.0, None), (1500, 1000, 0.0, None), (50257, 1000, 0.25, None), (50257, 1000, 0.004, None),
+                                                  (262144, 1000, 0.0, 0.1)])
+def test_wide_top_k_without_an_order(V, top_k, step, allowed):
+    """A top-k of more than 512: cuts and draw by buckets - everything listed, more listed than kept, cuts by top-p, by min-p, by both and by neither; logits so
+    coarse that a bucket is too full and the list is sorted after all, and just not so."""
+    rows = rows_of()
+    c = _odd(rows, V, top_k=top_k, n_hist=min(300, V), n_bias=min(20, V), allowed=allowed)
+    if step:
+        c["logits"] = (np.round(c["logits"] / step) * step).astype(np.float32)
+    c["top_p"][::4] = 1.0
+    c["top_p"][1::4] = 0.3
+    c["min_p"][1::3] = 0.02
+    c["min_p"][2::6] = 1.0
+    c["inv_t"][::5] = 0.3
+    run_short(c, 1, rows=some(rows, 23), handed_back=2)

@@ -130,6 +130,253 @@ struct ShortRow {
     bool by_k;        // they are the row's top_k largest; else everything the min-p floor may let through
 };
 
+// a distance to a decision, and what it is measured in (divided only where somebody asks for the quotient: a division is some 200 clocks of the chain)
+struct ShortMargin {
+    double d, of;
+};
+// The row's answer, written by the lane that has the drawn token: its id, its mass, the running mass with and without it; the kept set's size and mass
+__device__ __forceinline__ void short_answer(const LeanArgPtr Ap, const uint32_t row, const ShortRow& R, uint32_t n3, uint32_t id, double e, double cin, double cex, double Zk, double target,
+                                             bool drawn, ShortMargin mg_top_p, ShortMargin mg_min_p, uint32_t pos) {
+    const ShortMargin mg = {drawn ? fmin(cin - target, pos > 0u ? target - cex : 1e300) : 0.0, Zk};
+    const double tol = Ap->tol;
+    uint32_t flags = kRouteShort;
+    if (mg_top_p.d < tol * mg_top_p.of) flags |= kNearTopP;
+    if (mg_min_p.d < tol * mg_min_p.of) flags |= kNearMinP;
+    if (mg.d < tol * mg.of) flags |= kNearDraw;
+    Ap->token[row] = static_cast<int32_t>(id);
+    Ap->flags[row] = flags;
+    if (Ap->prob) Ap->prob[row] = static_cast<float>(e / Zk);
+    if (Ap->n_kept) Ap->n_kept[row] = n3;
+    if (Ap->stats) {
+        Ap->stats[2 * row] = R.m;
+        Ap->stats[2 * row + 1] = static_cast<float>(R.z);
+    }
+    if (Ap->margin) {
+        Ap->margin[3 * row] = mg_top_p.d / mg_top_p.of;
+        Ap->margin[3 * row + 1] = mg_min_p.d / mg_min_p.of;
+        Ap->margin[3 * row + 2] = mg.d / mg.of;
+    }
+}
+
+// The same for a row with a top-k, without an order: the keys are dealt to 512 buckets as the sort would, with their masses, and one wave looks for the cuts and
+// the draw - a bucket by the buckets' running counts and masses, then a place among its few keys, which alone are put in order. What bounds a wide top-k's
+// finish where other rows sweep on the same unit (ws_twin.h) is the instructions: the rank and running mass of every key, sixteen waves in and out of a dozen barriers.
+// Masses are added up in fixed point against the maximum's, 2^-51 of it the last place: off by at most n 2^-52 of the normaliser, where running sums in 64-bit floats are
+// off by n 2^-53 of themselves. For 65 keys and more (n_list <= kShortCap - 1024: the buckets lie behind the list) of rows that are asked for neither a kept-set dump
+// nor an entropy or a query. Every thread calls it. Returns false when a bucket has more than a wave's lanes of keys (equal logits): the list still holds the same keys.
+// S.s_d[7]: the row's normaliser (R.z is not looked at: nobody has to keep it in registers meanwhile).
+__device__ __forceinline__ bool short_pick(uint64_t* list, const uint32_t n_list, const uint32_t row, const ShortRow& R, ShortShared& S) {
+    constexpr uint32_t K = (kShortCap - 1024u) / WS_BLOCK, NB = 512u;
+    static_assert(WS_BLOCK >= NB, "a thread a bucket");
+    const uint32_t t = threadIdx.x, lane = t & 63u;
+    const uint32_t wv = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(t >> 6)));
+    unsigned long long* mass = reinterpret_cast<unsigned long long*>(list + (kShortCap - 1024u));
+    uint32_t *cnt = reinterpret_cast<uint32_t*>(mass + NB), *start = cnt + NB;
+    const double inv_t = static_cast<double>(R.inv_t), min_p = R.min_p;
+    const bool use_top_p = R.top_p < 1.0, use_min_p = min_p > 0.0;
+    constexpr double kFix = 2251799813685248.0, kUnfix = 1.0 / kFix;  // 2^51: a mass is 1 at most, and there are 4096 of them
+    float d[K], dmax = 0.f, dsum = 0.f;
+#pragma unroll
+    for (uint32_t k = 0; k < K; ++k) {
+        d[k] = 0.f;
+        if (k * WS_BLOCK < n_list && k * WS_BLOCK + t < n_list) {
+            d[k] = fminf(__fsub_rn(R.m, unkey32(static_cast<uint32_t>(list[k * WS_BLOCK + t] >> 32))), 3e38f);
+            dmax = fmaxf(dmax, d[k]);
+            dsum += d[k];
+        }
+    }
+    if (t < NB) {
+        mass[t] = 0ull;
+        cnt[t] = 0u;
+    }
+    if (t == 0u) {
+        S.s_w[6] = 0u;
+        S.s_w[7] = 0xffffffffu;
+    }
+    dmax = wave_max(dmax);
+    dsum = wave_sum(dsum);
+    if (lane == 0u) {
+        S.bcnt[wv] = __float_as_uint(dmax);
+        S.bstart[wv] = __float_as_uint(dsum);
+    }
+    __syncthreads();  // (the buckets are clear as well)
+    float total = 0.f;
+    dmax = 0.f;
+#pragma unroll
+    for (uint32_t w = 0; w < WS_WAVES; ++w) {
+        dmax = fmaxf(dmax, __uint_as_float(S.bcnt[w]));
+        total += __uint_as_float(S.bstart[w]);
+    }
+    const float mean = fmaxf(dmax - total / static_cast<float>(n_list), dmax * 1e-6f + 1e-30f);
+    // (the scale of short_sort's buckets)
+    const float per = 1.f / mean;
+    auto level = [&](float d_) { return static_cast<float>(__float_as_uint(__fadd_rn(1.f, __fmul_rn(fmaxf(__fsub_rn(dmax, d_), 0.f), per))) - 0x3f800000u); };
+    const float scale = static_cast<float>(NB) / (level(0.f) + 1.f);
+    uint32_t at[K], pass = 0;  // bucket | place in it << 16
+    float near = INFINITY;
+#pragma unroll
+    for (uint32_t k = 0; k < K; ++k)
+        if (k * WS_BLOCK < n_list && k * WS_BLOCK + t < n_list) {
+            const double e = exp_down(static_cast<double>(d[k]) * inv_t);
+            const uint32_t b = NB - 1u - min(NB - 1u, static_cast<uint32_t>(level(d[k]) * scale));
+            at[k] = b | (atomicAdd(&cnt[b], 1u) << 16);
+            atomicAdd(&mass[b], static_cast<unsigned long long>(fma(e, kFix, 0.5)));
+            pass += e >= min_p ? 1u : 0u;
+            near = fminf(near, static_cast<float>(fabs(e - min_p)));
+        }
+    if (use_min_p) {
+        pass = wave_sum(pass);
+        const uint32_t nearest = ~wave_max_u32(~__float_as_uint(near));
+        if (lane == 0u && pass) atomicAdd(&S.s_w[6], pass);
+        if (lane == 0u) atomicMin(&S.s_w[7], nearest);
+    }
+    __syncthreads();
+    uint32_t c8[8], n_in = 0;
+    uint64_t g8[8], g_in = 0;
+    if (wv == 0u) {  // a lane has eight buckets
+#pragma unroll
+        for (uint32_t k = 0; k < 8u; ++k) {
+            c8[k] = cnt[lane * 8u + k];
+            g8[k] = mass[lane * 8u + k];
+        }
+        uint32_t most = 0;
+#pragma unroll
+        for (uint32_t k = 0; k < 8u; ++k) {
+            most = max(most, c8[k]);
+            n_in += c8[k];
+            g_in += g8[k];
+        }
+        uint32_t run = wave_incl_scan(n_in) - n_in;
+#pragma unroll
+        for (uint32_t k = 0; k < 8u; ++k) {
+            start[lane * 8u + k] = run;
+            run += c8[k];
+        }
+        n_in = run;
+        g_in = wave_incl_scan(g_in);
+        const bool crowded = __ballot(most > 64u) != 0ull;
+        if (lane == 0u) S.s_w[8] = crowded ? 1u : 0u;
+    }
+    __syncthreads();
+    if (S.s_w[8] != 0u) return false;
+    uint64_t key[K];  // (read again: the exponentials have the registers)
+#pragma unroll
+    for (uint32_t k = 0; k < K; ++k) key[k] = k * WS_BLOCK < n_list && k * WS_BLOCK + t < n_list ? list[k * WS_BLOCK + t] : 0ull;
+    __syncthreads();
+#pragma unroll
+    for (uint32_t k = 0; k < K; ++k)
+        if (k * WS_BLOCK < n_list && k * WS_BLOCK + t < n_list) list[start[at[k] & 0xffffu] + (at[k] >> 16)] = key[k];
+    __syncthreads();
+    if (wv != 0u) return true;
+
+    // ------------------------------------------------------------------ one wave
+    auto real = [&](uint64_t g) { return static_cast<double>(g) * kUnfix; };
+    // a bucket's keys in order, one a lane, with what is ranked before them
+    struct Place {
+        uint32_t n, before;  // keys in the bucket, and before it
+        uint64_t key;
+        double e, cin, cex;
+    };
+    // the first bucket with which the running count and mass satisfy `reached`; found: whether there is one
+    auto look = [&](auto&& reached, bool& found) __attribute__((always_inline)) {
+        Place R_;
+        const uint64_t any = __ballot(reached(n_in, real(g_in)));
+        found = any != 0ull;
+        const uint32_t f = found ? static_cast<uint32_t>(__ffsll(static_cast<unsigned long long>(any)) - 1) : 63u;
+        uint32_t run = f ? lane_value(n_in, f - 1u) : 0u, b = 0, n = 0, first = run;
+        uint64_t sum = f ? lane_value(g_in, f - 1u) : 0ull, before = sum;
+        bool done = false;
+#pragma unroll
+        for (uint32_t k = 0; k < 8u; ++k) {
+            const uint32_t c = lane_value(c8[k], f);
+            const uint64_t g = lane_value(g8[k], f);
+            if (!done && c) {  // uniform
+                b = f * 8u + k;
+                n = c;
+                first = run;
+                before = sum;
+                run += c;
+                sum += g;
+                done = reached(run, real(sum));
+            }
+        }
+        const uint32_t s0 = first;  // (the buckets lie one behind the other)
+        const uint64_t own = lane < n ? list[s0 + lane] : 0ull;
+        uint32_t above = 0;
+        for (uint32_t j = 0; j < n; ++j) above += lane_value(own, j) > own ? 1u : 0u;  // uniform
+        uint64_t* sorted = reinterpret_cast<uint64_t*>(mass);  // (the masses are in registers)
+        if (lane < n) sorted[above] = own;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        R_.n = n;
+        R_.before = first;
+        R_.key = lane < n ? sorted[lane] : 0ull;
+        R_.e = lane < n ? exp_down(static_cast<double>(__fsub_rn(R.m, unkey32(static_cast<uint32_t>(R_.key >> 32)))) * inv_t) : 0.0;
+        const double base = real(before), inc = wave_incl_scan(R_.e), up = __shfl_up(inc, 1);
+        R_.cin = base + inc;
+        R_.cex = base + (lane ? up : 0.0);
+        __builtin_amdgcn_wave_barrier();
+        return R_;
+    };
+    bool found;
+    const uint32_t n_cand = R.n_cand;
+    const double all = real(lane_value(g_in, 63u));
+    double Zk1 = all, e_last = -1.0;
+    if (n_list > n_cand) {
+        const Place at_k = look([&](uint32_t n, double) { return n >= n_cand; }, found);
+        const uint32_t j = n_cand - 1u - at_k.before;
+        Zk1 = lane_value(at_k.cin, j);
+        e_last = lane_value(at_k.e, j);
+    }
+    const double X = R.top_p * Zk1;
+    uint32_t n3 = n_cand;
+    double M = Zk1;
+    ShortMargin mg_top_p = {1.0, 1.0}, mg_min_p = {1.0, 1.0};
+    if (use_top_p) {
+        const Place at_p = look([&](uint32_t, double m_) { return m_ >= X; }, found);
+        mg_top_p = {0.0, X};  // (rounding: the running mass never reaches top_p of itself)
+        if (found) {
+            const uint64_t is = __ballot(lane < at_p.n && at_p.cin >= X);
+            const uint32_t j = is ? static_cast<uint32_t>(__ffsll(static_cast<unsigned long long>(is)) - 1) : at_p.n - 1u;
+            if (at_p.before + j < n_cand) {
+                n3 = at_p.before + j + 1u;
+                M = lane_value(at_p.cin, j);
+                const double ex = lane_value(at_p.cex, j);
+                mg_top_p = {fmin(M - X, n3 > 1u ? X - ex : X), X};
+            }
+        }
+    }
+    if (use_min_p) {
+        const uint32_t passed = S.s_w[6];
+        const double nearest = passed >= n_cand && e_last >= 0.0 ? fabs(e_last - min_p) : static_cast<double>(__uint_as_float(S.s_w[7]));
+        mg_min_p = {fmin(min_p, nearest), min_p};
+        if (passed < n3) {
+            n3 = max(passed, 1u);
+            const Place at_n = look([&](uint32_t n, double) { return n >= n3; }, found);
+            M = lane_value(at_n.cin, n3 - 1u - at_n.before);
+        }
+    }
+    const double target = R.u * M;
+    Place at_u = look([&](uint32_t, double m_) { return m_ > target; }, found);
+    uint32_t j;
+    {
+        const uint64_t is = __ballot(lane < at_u.n && at_u.cin > target);
+        j = is ? static_cast<uint32_t>(__ffsll(static_cast<unsigned long long>(is)) - 1) : at_u.n - 1u;
+    }
+    const bool drawn = found && at_u.before + j < n3;
+    if (!drawn) {  // (rounding: the walk falls through to the last kept, src/sampling/sampler.cpp:131)
+        at_u = look([&](uint32_t n, double) { return n >= n3; }, found);
+        j = n3 - 1u - at_u.before;
+    }
+    const LeanArgPtr Ap = (LeanArgPtr)__builtin_amdgcn_kernarg_segment_ptr();
+    ShortRow answer = R;
+    answer.z = S.s_d[7];
+    if (lane == j)
+        short_answer(Ap, row, answer, n3, 0xffffffffu - static_cast<uint32_t>(at_u.key), at_u.e, at_u.cin, at_u.cex, M, target, drawn, mg_top_p, mg_min_p, at_u.before + j);
+    return true;
+}
+
 // The reference's rules (src/sampling/sampler.cpp:31-74, :118-131) on the sorted candidates, and the row's results. Every
 // thread of the workgroup calls it.
 __device__ __forceinline__ void short_rules(uint64_t* list, const uint32_t row, const ShortRow& R, ShortShared& S) {
@@ -149,33 +396,11 @@ __device__ __forceinline__ void short_rules(uint64_t* list, const uint32_t row, 
     const uint64_t key = has ? list[t] : 0ull;
     const float x = has ? unkey32(static_cast<uint32_t>(key >> 32)) : -INFINITY;
     const uint32_t id = 0xffffffffu - static_cast<uint32_t>(key);
-    typedef const __attribute__((address_space(4))) BatchArgs* ArgPtr;
-    ArgPtr Ap = (ArgPtr)__builtin_amdgcn_kernarg_segment_ptr();
+    const LeanArgPtr Ap = (LeanArgPtr)__builtin_amdgcn_kernarg_segment_ptr();
     uint32_t n3;
-    // a distance to a decision, and what it is measured in (divided only where somebody asks for the quotient: a division is some 200 clocks of the chain)
-    struct Margin {
-        double d, of;
-    };
+    typedef ShortMargin Margin;
     auto write_out = [&](uint32_t id_, double e_, double cin_, double cex_, double Zk_, double target_, bool drawn, Margin mg_top_p_, Margin mg_min_p_, uint32_t pos) {
-        const Margin mg = {drawn ? fmin(cin_ - target_, pos > 0u ? target_ - cex_ : 1e300) : 0.0, Zk_};
-        const double tol = Ap->tol;
-        uint32_t flags = kRouteShort;
-        if (mg_top_p_.d < tol * mg_top_p_.of) flags |= kNearTopP;
-        if (mg_min_p_.d < tol * mg_min_p_.of) flags |= kNearMinP;
-        if (mg.d < tol * mg.of) flags |= kNearDraw;
-        Ap->token[row] = static_cast<int32_t>(id_);
-        Ap->flags[row] = flags;
-        if (Ap->prob) Ap->prob[row] = static_cast<float>(e_ / Zk_);
-        if (Ap->n_kept) Ap->n_kept[row] = n3;
-        if (Ap->stats) {
-            Ap->stats[2 * row] = m;
-            Ap->stats[2 * row + 1] = static_cast<float>(R.z);
-        }
-        if (Ap->margin) {
-            Ap->margin[3 * row] = mg_top_p_.d / mg_top_p_.of;
-            Ap->margin[3 * row + 1] = mg_min_p_.d / mg_min_p_.of;
-            Ap->margin[3 * row + 2] = mg.d / mg.of;
-        }
+        short_answer(Ap, row, R, n3, id_, e_, cin_, cex_, Zk_, target_, drawn, mg_top_p_, mg_min_p_, pos);
     };
     // optional outputs: -sum p ln p over the kept set with p = e / Zk and ln e = (x - m) / temperature, which is
     // ln Zk - (sum of e ln e) / Zk; and the share of one named token, 0 when it is not kept

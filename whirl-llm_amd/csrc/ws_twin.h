@@ -738,12 +738,6 @@ __device__ __forceinline__ bool twin_row(const BatchArgs& A, const uint32_t row,
         }
         z += block_sum(more, S.red_d);
     }
-    short_sort(list, n_list, m, S);
-    WSS_MARK(6);  // sorted
-    // the k-th largest has to lie above the threshold (below it, the sweep has left out tokens that rank before it); a min-p row's
-    // threshold lies below its floor by construction
-    const float x_k = unkey32(static_cast<uint32_t>(list[n_cand - 1u] >> 32));
-    if ((by_k && !(x_k > thr)) || !(x_k > -INFINITY)) return false;
     ShortRow R;
     R.top_p = top_p;
     R.min_p = min_p;
@@ -753,6 +747,22 @@ __device__ __forceinline__ bool twin_row(const BatchArgs& A, const uint32_t row,
     R.m = m;
     R.n_cand = n_cand;
     R.by_k = by_k;
+    // A wide top-k, two candidates a thread and more: its cuts and draw without an order (us, with the sort and without: 1024 masked rows of 262144, top-k 1000, 247.5 / 241.5, 300
+    // of 262144 101.6 / 97.9; level at a top-k of 100 to 500, and rows with a min-p alone, whose keys crowd at the floor, 86.7 / 95.4).
+    const LeanArgPtr Ap = (LeanArgPtr)__builtin_amdgcn_kernarg_segment_ptr();
+    if (DT == 0 && by_k && n_cand > WS_BLOCK && n_list <= kShortCap - 1024u && !Ap->kept_ids && !Ap->entropy && !Ap->query_prob) {  // uniform
+        if (t == 0u) S.s_d[7] = R.z;
+        __syncthreads();  // (the words that say which places were left over have been read as well)
+        if (short_pick(list, n_list, row, R, S)) return true;
+        R.z = S.s_d[7];
+        __syncthreads();
+    }
+    short_sort(list, n_list, m, S);
+    WSS_MARK(6);  // sorted
+    // the k-th largest has to lie above the threshold (below it, the sweep has left out tokens that rank before it); a min-p row's
+    // threshold lies below its floor by construction
+    const float x_k = unkey32(static_cast<uint32_t>(list[n_cand - 1u] >> 32));
+    if ((by_k && !(x_k > thr)) || !(x_k > -INFINITY)) return false;
     short_rules(list, row, R, S);
 #ifdef WS_SHORT_TIMERS
     WSS_MARK(8);
