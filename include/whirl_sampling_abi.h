@@ -359,6 +359,10 @@ int ws_sample_batch_notify(void* stream, const ws_batch* b, uint32_t* done, uint
  * hist_len, bias_*) lie in host memory that the device reads in place (hipHostMalloc) and are as they should be when the call is made: the call may read
  * them too, and send a lone row's along with the launch. They stay as they are until the words have come. */
 int ws_sample_batch_notify_host(void* stream, const ws_batch* b, uint32_t* done, uint32_t value);
+/* The same, but a batch of one row may come back undone: flags[0] is WS_FLAGS_LEFT then and nothing else has been written (the workspace is as every launch leaves it).
+ * The caller asks ws_sample_batch_notify_host for it. (A kernel that need not be able to do every row begins 1.2 us sooner on an idle GPU; a few rows in ten thousand come back.) */
+#define WS_FLAGS_LEFT 0xffffffffu
+int ws_sample_batch_try_host(void* stream, const ws_batch* b, uint32_t* done, uint32_t value);
 /* ws_sample_batch for callers that cannot allocate device memory - code under HIP graph capture, tight serving loops,
  * harnesses that forbid it; it has no counterpart in the reference. The split rows of a small batch meet in memory that is
  * part of the library's code object on every GPU (WS_STATIC_SPLIT_ROWS rows of it, about 4 MiB, held until the process

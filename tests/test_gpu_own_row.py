@@ -55,3 +55,41 @@ def test_the_row_of_the_arguments_is_the_row_of_memory(vocab, top_k, min_p, n_hi
             assert torch.equal(getattr(got, k), getattr(want, k)), k
     assert int(got.workspace.sum()) == 0 or not top_k and not min_p
     assert m.lib().ws_sample_batch_notify_host(None, m.C.byref(got.desc), None, 1) == -1
+
+
+@pytest.mark.parametrize("vocab,n_hist,declared,flat,left", [(151936, 256, 256, False, False), (40003, 0, 0, False, False), (19471, 40, 12, False, True), (40003, 64, 64, True, True)])
+def test_a_row_that_may_be_left(vocab, n_hist, declared, flat, left):
+    """ws_sample_batch_try_host: the same answers, or - a row with more history than the batch declares, a row of equal logits, of which no list holds the top-k's
+    ties - the mark in the flags and nothing else, the workspace zero; asked for again, the row is done as ever."""
+    m = gc.pkg()
+    rng = np.random.default_rng(vocab)
+    x = torch.from_numpy((np.zeros((1, vocab)) if flat else rng.normal(0, 2, (1, vocab))).astype(np.float32)).cuda()
+    args = dict(inv_t=np.full(1, 1.25, np.float32), top_p=np.full(1, 0.95), seed=np.full(1, 77 << 33, np.int64), step=np.full(1, 5, np.int64), top_k=np.full(1, 40, np.int32))
+    hints = dict(top_k_max=40)
+    if n_hist:
+        args.update(hist=(rng.random(n_hist) ** 2 * vocab).astype(np.int32), hist_off=np.array([0, n_hist], np.int32), rep=np.full(1, 1.3, np.float32))
+        hints.update(max_hist=declared)
+    args = {k: pinned(v) for k, v in args.items()}
+    make = lambda: m.BatchSampler(x, args["inv_t"], args["seed"], args["step"], kept_cap=64, **hints, **{k: v for k, v in args.items() if k not in ("inv_t", "seed", "step")})
+    want, got = make().run(), make()
+    got.token.fill_(-5)
+    torch.cuda.synchronize()
+    done = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+    words = done.numpy()
+
+    def ask(call, value):
+        m.check(getattr(m.lib(), call)(torch.cuda.current_stream().cuda_stream, m.C.byref(got.desc), done.data_ptr(), value), call)
+        until = time.monotonic() + 20.0
+        while words[0] != value and time.monotonic() < until:
+            pass
+        assert words[0] == value
+        torch.cuda.synchronize()
+
+    ask("ws_sample_batch_try_host", 1)
+    assert (int(got.flags[0]) == -1) == left
+    assert int(got.workspace.sum()) == 0
+    if left:
+        assert int(got.token[0]) == -5
+        ask("ws_sample_batch_notify_host", 2)
+    for k in ("token", "prob", "n_kept", "flags", "stats", "margin", "kept_ids", "kept_logits"):
+        assert torch.equal(getattr(got, k), getattr(want, k)), k

@@ -150,6 +150,7 @@ ABI = {
     "ws_sample_batch": (C.c_int, [C.c_void_p, C.POINTER(Batch)]),
     "ws_sample_batch_notify": (C.c_int, [C.c_void_p, C.POINTER(Batch), C.c_void_p, C.c_uint32]),
     "ws_sample_batch_notify_host": (C.c_int, [C.c_void_p, C.POINTER(Batch), C.c_void_p, C.c_uint32]),
+    "ws_sample_batch_try_host": (C.c_int, [C.c_void_p, C.POINTER(Batch), C.c_void_p, C.c_uint32]),
     "ws_sample_batch_static": (C.c_int, [C.c_void_p, C.POINTER(Batch)]),
     "ws_adjust_rows": (C.c_int, [C.c_void_p, C.POINTER(Adjust)]),
     "ws_accept_sampled": (C.c_int, [C.c_void_p, C.POINTER(Accept)]),

@@ -46,7 +46,8 @@ int launch_code(hipStream_t stream, const BatchArgs& a, unsigned rows, unsigned 
 int prepare_code(unsigned lds_limit);
 uint64_t code_lds_bytes(uint32_t vocab, uint32_t cap, uint32_t copies);
 // ws_few.hip: the same rows shared between workgroups that hold them in registers
-int launch_few(hipStream_t stream, const BatchArgs& a, unsigned lds_bytes, unsigned lds_limit, const OwnRow* own);
+// (leave: a row that `own` takes along may be left undone, marked in its flags)
+int launch_few(hipStream_t stream, const BatchArgs& a, unsigned lds_bytes, unsigned lds_limit, const OwnRow* own, bool leave);
 int prepare_few(unsigned lds_limit);
 // ws_top.hip: topk_rows, dflash_topk and draft_sample_rows with rows shared between workgroups
 int launch_topk_shared(hipStream_t stream, const float* x, int n, int K, float inv_t, int* ids, float* vals, float* stats, unsigned rows, unsigned parts,
@@ -775,7 +776,7 @@ BatchPlan plan_for(const ws_batch* b, uint64_t work_bytes) {
 
 // done: a word per row that gets `value` once the row's results are visible to the host, or nullptr (ws_sample_batch_notify)
 int sample_batch_on(void* stream, const ws_batch* b, const BatchPlan& p, unsigned char* work, uint64_t work_bytes, uint32_t* done_at = nullptr,
-                    uint32_t done_value = 0u, const ws::OwnRow* own = nullptr) {
+                    uint32_t done_value = 0u, const ws::OwnRow* own = nullptr, bool leave = false) {
     const bool can_split = split_fits(p, work, work_bytes);
     const bool staged = can_split && work_bytes >= p.workspace && p.workspace > p.workspace_min;
     ws::BatchArgs a{};
@@ -837,7 +838,7 @@ int sample_batch_on(void* stream, const ws_batch* b, const BatchPlan& p, unsigne
         a.work = work;
         a.fb_lds_tie = 0u;
         a.fb_lds_ab = p.short_fb_ab;
-        return ws::launch_few(S(stream), a, p.few_total, kMaxLds - kStaticFew, own);
+        return ws::launch_few(S(stream), a, p.few_total, kMaxLds - kStaticFew, own, leave);
     }
     if (p.code) {
         a.lds_tie = p.code_copies > 1u;
@@ -908,7 +909,7 @@ void own_row(const ws_batch* b, ws::OwnRow& o) {
     if (o.n_ids) std::memcpy(o.ids, b->hist + P.h0, o.n_ids * sizeof(int32_t));
 }
 
-int notify_on(void* stream, const ws_batch* b, uint32_t* done, uint32_t value, bool host_inputs) {
+int notify_on(void* stream, const ws_batch* b, uint32_t* done, uint32_t value, bool host_inputs, bool leave = false) {
     if (!done) return WS_E_INVALID;
     const BatchPlan p = plan_for(b, b ? b->workspace_bytes : 0);
     if (p.err != WS_OK) return p.err;
@@ -916,7 +917,7 @@ int notify_on(void* stream, const ws_batch* b, uint32_t* done, uint32_t value, b
     const bool few = p.few_parts && split_fits(p, work, b->workspace_bytes), with_row = host_inputs && few && b->rows == 1u;
     ws::OwnRow own;
     if (with_row) own_row(b, own);
-    if (const int e = sample_batch_on(stream, b, p, work, b->workspace_bytes, done, value, with_row ? &own : nullptr); e != WS_OK) return e;
+    if (const int e = sample_batch_on(stream, b, p, work, b->workspace_bytes, done, value, with_row ? &own : nullptr, leave); e != WS_OK) return e;
     if (few) return WS_OK;  // (that kernel writes the words itself)
     if (!b->rows) return WS_OK;
     for (uint32_t r = 0; r + 1u < b->rows; ++r) done[r] = value;
@@ -927,6 +928,8 @@ int notify_on(void* stream, const ws_batch* b, uint32_t* done, uint32_t value, b
 int ws_sample_batch_notify(void* stream, const ws_batch* b, uint32_t* done, uint32_t value) { return notify_on(stream, b, done, value, false); }
 
 int ws_sample_batch_notify_host(void* stream, const ws_batch* b, uint32_t* done, uint32_t value) { return notify_on(stream, b, done, value, true); }
+
+int ws_sample_batch_try_host(void* stream, const ws_batch* b, uint32_t* done, uint32_t value) { return notify_on(stream, b, done, value, true, true); }
 
 int ws_sample_batch_static(void* stream, const ws_batch* b) {
     const BatchPlan p = plan_for(b, sizeof(scratch));

@@ -681,7 +681,8 @@ __device__ __forceinline__ bool few_row(const BatchArgs& A, const OwnRow* own, c
     return true;
 }
 
-template <int DT, bool MASKED, int NV, bool OWN>
+// LEAVE: a row for which a check fails is marked in `flags` and left to another launch.
+template <int DT, bool MASKED, int NV, bool OWN, bool LEAVE>
 __device__ __forceinline__ void few_batch(const BatchArgs& A, const OwnRow* own) {
     __shared__ FewShared shared;
     uint32_t row, part;
@@ -691,8 +692,12 @@ __device__ __forceinline__ void few_batch(const BatchArgs& A, const OwnRow* own)
         __syncthreads();
         LeanArgPtr Ap = (LeanArgPtr)__builtin_amdgcn_kernarg_segment_ptr();
         asm volatile("" : "+s"(Ap));
-        if (Ap->kept_ids) three_pass_row<true>(Ap, row);
-        else three_pass_row<false>(Ap, row);
+        if constexpr (LEAVE) {
+            if (threadIdx.x == 0) Ap->flags[row] = kRowLeft;
+        } else {
+            if (Ap->kept_ids) three_pass_row<true>(Ap, row);
+            else three_pass_row<false>(Ap, row);
+        }
     }
     if (A.done && finisher) {  // a host looks at this word instead of waiting for the stream: everything written for the row first
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -702,13 +707,15 @@ __device__ __forceinline__ void few_batch(const BatchArgs& A, const OwnRow* own)
 }
 template <int DT, bool MASKED, int NV>
 __global__ void __launch_bounds__(WS_BLOCK) few_batch_kernel(BatchArgs A) {
-    few_batch<DT, MASKED, NV, false>(A, nullptr);
+    few_batch<DT, MASKED, NV, false, false>(A, nullptr);
 }
 // A lone row whose parameters and ids lie in host memory: as arguments they come with the launch, where the kernel above makes two trips over the bus, one behind
 // the other, before it knows its touched tokens (a decode step of 151936 tokens and 256 ids through the host API: 19.4 -> 16.6 us; of 700 ids 17.2, of 2000, which stay where they are, 19.3).
-template <int DT, int NV>
+// LEAVE: without the three-pass code, which takes the kernel from 99 registers to 248 and gives it scratch memory: 1.2 us of a launch on an idle GPU (32 decode steps of 151936
+// tokens and 256 ids 566 / 527 us).
+template <int DT, int NV, bool LEAVE>
 __global__ void __launch_bounds__(WS_BLOCK) few_own_kernel(BatchArgs A, OwnRow own) {
-    few_batch<DT, false, NV, true>(A, &own);
+    few_batch<DT, false, NV, true, LEAVE>(A, &own);
 }
 
 }  // namespace ws

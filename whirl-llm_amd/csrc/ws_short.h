@@ -30,7 +30,8 @@ constexpr uint32_t kShortMaxK = 1024u;  // largest top-k: one candidate a thread
 constexpr uint32_t kShortHead = 8u;     // head of a slice: vectors a thread asked for before anything else
 constexpr uint32_t kShortSample = 8u;   // of those, the vectors a thread whose tokens the threshold is fitted to (32768 tokens of fp32)
 constexpr uint32_t kRouteShort = 0x2000u;
-constexpr uint32_t kTwinRest = 0xffffffffu;  // in `flags`, between two kernels: a row of ws_twin.h's left to the three-pass code (no set of flags has every bit)
+constexpr uint32_t kRowLeft = 0xffffffffu;  // in `flags`: a row left to another launch (WS_FLAGS_LEFT; no set of flags has every bit)
+constexpr uint32_t kTwinRest = kRowLeft;  // in `flags`, between two kernels: a row of ws_twin.h's left to the three-pass code (no set of flags has every bit)
 
 
 #ifdef WS_SHORT_TIMERS

@@ -4,7 +4,7 @@
 // No vocabulary-sized work happens here unless the device flags the row.
 // Parameters, penalty lists, results and kept sets live in pinned host memory that the device addresses directly
 // (hipHostMalloc): the host writes the few hundred bytes a row needs, the kernel reads them over the bus (a lone row's come with the
-// launch), writes what it kept straight back and then a word the host looks at (ws_sample_batch_notify_host), and no copy command sits before or after
+// launch), writes what it kept straight back and then a word the host looks at (ws_sample_batch_try_host), and no copy command sits before or after
 // the launch - a decode step is one launch and one wait for that word, which comes some 5 us before a stream wait would end.
 // Everything here has waited for what it launched before it returns, so the host never rewrites a block that a launch
 // still reads.
@@ -336,8 +336,12 @@ void DeviceRows::filterOnDevice(const Sampler& s, std::uint32_t gr0, std::uint32
     b.workspace = d.work.at;
     b.workspace_bytes = d.work.bytes;
     d.in_flight = true;
-    check(ws_sample_batch_notify_host(stream_, &b, d.done, ++d.turn), "ws_sample_batch");
+    check(ws_sample_batch_try_host(stream_, &b, d.done, ++d.turn), "ws_sample_batch");
     waitForRows(n);  // results and kept sets are in host memory now
+    if (n == 1 && o.flags[0] == WS_FLAGS_LEFT) {  // (a lone row that the quick kernel has left)
+        check(ws_sample_batch_notify_host(stream_, &b, d.done, ++d.turn), "ws_sample_batch");
+        waitForRows(n);
+    }
     d.in_flight = false;
     const Dev::ResultView& h = o;
     ready_.clear();
