@@ -71,3 +71,21 @@ def test_stores_have_arrived_before_the_ticket_is_drawn(kernels):
         assert "s_barrier" in back, name
         waits = [op for op in back[back.index("s_barrier"):] if op.startswith("s_waitcnt") and "vmcnt(0)" in op]
         assert waits, f"{name}: its stores may still be on their way"
+
+
+def test_the_kernels_that_may_leave_a_row_wait_as_well(tmp_path):
+    """The builds of the lone row's kernel without the three-pass code (few_try_kernel), looked at the same way."""
+    if not os.path.exists(OBJDUMP):
+        pytest.skip("no llvm-objdump")
+    found = 0
+    for i, blob in enumerate(code_objects(LIB)):
+        path = tmp_path / f"{i}.elf"
+        path.write_bytes(blob)
+        names = re.findall(r"\.text\s+\S+\s+\S*\s*(\S*few_try_kernel\S*)$", subprocess.run([OBJDUMP, "-t", str(path)], capture_output=True, text=True, check=True).stdout, re.M)
+        for name in (n for n in names if not n.endswith(".kd")):
+            text = subprocess.run([OBJDUMP, "-d", "--no-show-raw-insn", f"--disassemble-symbols={name}", str(path)], capture_output=True, text=True, check=True).stdout
+            back = before_the_ticket([line.split("//")[0].strip() for line in text.splitlines() if line.startswith("\t")])
+            assert "s_barrier" in back, name
+            assert any(op.startswith("s_waitcnt") and "vmcnt(0)" in op for op in back[back.index("s_barrier"):]), name
+            found += 1
+    assert found == 2

@@ -22,7 +22,7 @@ SRC_TWIN = os.path.join(HERE, "csrc", "ws_twin.hip")  # the same for rows that a
 SRC_CODE = os.path.join(HERE, "csrc", "ws_code.hip")  # bf16 rows, held in registers and counted by value
 SRC_FEW = os.path.join(HERE, "csrc", "ws_few.hip")  # short-list rows shared between workgroups that hold them in registers
 SRC_TOP = os.path.join(HERE, "csrc", "ws_top.hip")  # top-k lists and draft draws of few rows, shared the same way
-SRC_LEAN = [os.path.join(HERE, "csrc", f) for f in ("ws_lean.hip", "ws_lean_short.hip")]  # the lean single-sweep kernel for batches of unsplit rows, long and short ones
+SRC_LEAN = os.path.join(HERE, "csrc", "ws_lean.hip")  # the lean single-sweep kernel for batches of unsplit rows
 # packed FP32 instructions are switched off for every device compile of this repository
 FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
          # the fused sweep is one fully unrolled loop of ~20 batches (its bin cache must stay in registers)
@@ -51,7 +51,7 @@ def build(verbose=True):
     # the translation units and the bare code object side by side (each takes a minute or two), then the link
     objdir = os.path.join(HERE, "csrc", "obj")
     os.makedirs(objdir, exist_ok=True)
-    srcs = (SRC, SRC_FUSED, SRC_FUSED_SHORT, SRC_SPLIT, *SRC_KEPT, *SRC_LEAN, SRC_CODE, SRC_SHORT, SRC_TWIN, SRC_FEW, SRC_TOP)
+    srcs = (SRC_LEAN, SRC_FEW, SRC, SRC_FUSED_SHORT, SRC_CODE, SRC_FUSED, SRC_SPLIT, *SRC_KEPT, SRC_SHORT, SRC_TWIN, SRC_TOP)  # the longest first
     objs = [os.path.join(objdir, os.path.basename(src)[:-4] + ".o") for src in srcs]
     jobs = [[hipcc, *FLAGS, "-fPIC", "-c", "-o", obj, src] for obj, src in zip(objs, srcs)]
     jobs.append([hipcc, *FLAGS, "--genco", "-o", co, SRC])

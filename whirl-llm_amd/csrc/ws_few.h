@@ -711,11 +711,15 @@ __global__ void __launch_bounds__(WS_BLOCK) few_batch_kernel(BatchArgs A) {
 }
 // A lone row whose parameters and ids lie in host memory: as arguments they come with the launch, where the kernel above makes two trips over the bus, one behind
 // the other, before it knows its touched tokens (a decode step of 151936 tokens and 256 ids through the host API: 19.4 -> 16.6 us; of 700 ids 17.2, of 2000, which stay where they are, 19.3).
-// LEAVE: without the three-pass code, which takes the kernel from 99 registers to 248 and gives it scratch memory: 1.2 us of a launch on an idle GPU (32 decode steps of 151936
-// tokens and 256 ids 566 / 527 us).
-template <int DT, int NV, bool LEAVE>
+template <int DT, int NV>
 __global__ void __launch_bounds__(WS_BLOCK) few_own_kernel(BatchArgs A, OwnRow own) {
-    few_batch<DT, false, NV, true, LEAVE>(A, &own);
+    few_batch<DT, false, NV, true, false>(A, &own);
+}
+// Without the three-pass code, which takes the kernel from 99 registers to 248 and gives it scratch memory: 1 us of a launch on an idle GPU (32 decode steps of 151936
+// tokens and 256 ids 568 / 540 us).
+template <int DT, int NV>
+__global__ void __launch_bounds__(WS_BLOCK) few_try_kernel(BatchArgs A, OwnRow own) {
+    few_batch<DT, false, NV, true, true>(A, &own);
 }
 
 }  // namespace ws

@@ -18,7 +18,7 @@ const FewKernel kFewKernels[2][2][4] = {
      {few_batch_kernel<1, true, 3>, few_batch_kernel<1, true, 5>, few_batch_kernel<1, true, 10>, few_batch_kernel<1, true, 14>}}};
 // a lone row of up to 16 parts: fp32, unmasked; rows beyond 327680 tokens go the other way
 constexpr int kOwnSizes = 2;
-void (*const kOwnKernels[2][kOwnSizes])(BatchArgs, OwnRow) = {{few_own_kernel<0, 5, false>, few_own_kernel<0, 10, false>}, {few_own_kernel<0, 5, true>, few_own_kernel<0, 10, true>}};
+void (*const kOwnKernels[2][kOwnSizes])(BatchArgs, OwnRow) = {{few_own_kernel<0, 5>, few_own_kernel<0, 10>}, {few_try_kernel<0, 5>, few_try_kernel<0, 10>}};
 }  // namespace
 
 int prepare_few(unsigned lds_limit) {

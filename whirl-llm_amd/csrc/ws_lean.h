@@ -29,12 +29,12 @@
 
 namespace ws {
 
-// Registers of the bin cache a thread, four tokens each: builds for rows of up to 32768, 49152, 65536, 98304, 131072 (ws_lean_short.hip), 155648, 163840 and 262144
-// tokens (ws_lean.hip), and a row gets the shortest that holds it. The loads past a row's end are asked for like the others - they may not lie behind a branch -, 64
+// Registers of the bin cache a thread, four tokens each: builds for rows of up to 32768, 49152, 65536, 98304, 155648, 163840 and 262144
+// tokens, and a row gets the shortest that holds it. The loads past a row's end are asked for like the others - they may not lie behind a branch -, 64
 // lanes at one address each: a row of 25000 tokens waited 8 K clocks of 46 K for them in the build of 40 (us, that one and its own: 54 rows of 25792 20.1 / 17.3, 34 of
 // 35392 25.3 / 22.0, 256 of 32000 with 1000 ids 26.5 / 21.6, 200 of 50257 27.9 / 24.3, 100 of 98304 30.9 / 29.0). Of the longest a quarter of the cache lies in scratch
 // memory behind the sweep, which is still far from the two more sweeps that such rows took (ws_abi.hip).
-constexpr int kLeanRegsShort[] = {8, 12, 16, 24, 32}, kLeanRegsLong[] = {38, 40, 64};
+constexpr int kLeanRegs[] = {8, 12, 16, 24, 38, 40, 64};
 constexpr int kLeanLooks = 64;  // from here on finds are looked at before they are listed, when they are too many
 constexpr int kLeanBatch = 2;   // 128-bit loads per thread and batch
 constexpr uint32_t kLeanBuckets = 128u;   // words of the finish's tables in LeanShared
@@ -1649,7 +1649,7 @@ __global__ void __launch_bounds__(WS_BLOCK) lean_batch_kernel(BatchArgs A) {
     __syncthreads();  // whatever the lean path left in LDS is dead
     LeanArgPtr Ap = (LeanArgPtr)__builtin_amdgcn_kernarg_segment_ptr();
     asm volatile("" : "+s"(Ap));
-    lean_rest<MASKED, NREG>(Ap, row, (__attribute__((address_space(3))) LeanShared*)&shared);
+    lean_rest<MASKED, (NREG <= 40 ? 40 : 64)>(Ap, row, (__attribute__((address_space(3))) LeanShared*)&shared);  // (one for all shorter rows: few are swept twice)
 }
 
 }  // namespace ws
