@@ -6,7 +6,7 @@
 // words, the same decision rules (src/sampling/sampler.cpp:15-78, :118-131) and margins.
 //
 // What is different from that kernel, and why:
-//   * every token's bin is remembered as eight of its bits, four tokens per register (40 registers instead of 160): a
+//   * every token's bin is remembered as eight of its bits, four tokens per register (of 163840 tokens 40 registers instead of 160): a
 //     scan for the tokens of a few bins tests four tokens with three instructions per bin; a token of another bin with
 //     the same bits is found as well and dropped when its logit has been read again. The registers this frees let the
 //     first two batches of the row travel while phase 0 builds its tables, and four waves per SIMD hide the tail's
@@ -32,7 +32,7 @@ namespace ws {
 // Registers of the bin cache a thread, four tokens each: builds for rows of up to 32768, 49152, 65536, 98304, 155648, 163840 and 262144
 // tokens, and a row gets the shortest that holds it. The loads past a row's end are asked for like the others - they may not lie behind a branch -, 64
 // lanes at one address each: a row of 25000 tokens waited 8 K clocks of 46 K for them in the build of 40 (us, that one and its own: 54 rows of 25792 20.1 / 17.3, 34 of
-// 35392 25.3 / 22.0, 256 of 32000 with 1000 ids 26.5 / 21.6, 200 of 50257 27.9 / 24.3, 100 of 98304 30.9 / 29.0). Of the longest a quarter of the cache lies in scratch
+// 35392 24.3 / 20.5, 256 of 32000 with 1000 ids 26.5 / 21.6, 200 of 50257 27.9 / 24.3, 100 of 98304 30.9 / 29.0). Of the longest a quarter of the cache lies in scratch
 // memory behind the sweep, which is still far from the two more sweeps that such rows took (ws_abi.hip).
 constexpr int kLeanRegs[] = {8, 12, 16, 24, 38, 40, 64};
 constexpr int kLeanLooks = 64;  // from here on finds are looked at before they are listed, when they are too many
