@@ -195,3 +195,23 @@ def test_wide_top_k_without_an_order(V, top_k, step, allowed):
     c["min_p"][2::6] = 1.0
     c["inv_t"][::5] = 0.3
     run_short(c, 1, rows=some(rows, 23), handed_back=2)
+
+
+@pytest.mark.parametrize("V,n_bias,n_hist,allowed", [(262144, 4096, 3, 0.1), (262144, 5000, 1, 0.05), (50257, 4095, 4, 0.02), (50257, 6000, 2, 0.02), (50257, 4097, 0, 0.02)])
+def test_masked_rows_with_more_bias_entries_than_the_batch_declares(V, n_bias, n_hist, allowed):
+    """Lists that fit max_hist + max_bias together, of which the bias list is by far the longer one: a masked row takes each entry's own value, however many
+    there are, and counts none as history."""
+    rows = rows_of()
+    c = _odd(rows, V, top_k=50, n_hist=max(n_hist, 1), n_bias=n_bias, allowed=allowed)
+    if not n_hist:
+        c["hist"] = np.full((rows, 1), -1, np.int32)
+    for r in range(rows):  # (the last entries are allowed, and their tokens among the largest)
+        ids = np.unique(c["bias_ids"][r, -40:]).astype(np.int64)
+        np.bitwise_or.at(c["allow"][r], ids >> 5, (np.uint32(1) << (ids & 31).astype(np.uint32)).astype(c["allow"].dtype))
+        c["logits"][r, ids[::2]] = 8.0
+    d = gc.upload(c, hints=True)
+    d["max_hist"], d["max_bias"] = 7700, 1000
+    smp = gc.sampler_for(c, d, 1, kept_cap=1024).run()
+    res = gc.compare_rows(c, smp, some(rows, 23), 1)
+    m = gc.pkg()
+    assert res["differ"] == 0 and (smp.flags.cpu().numpy() & m.FLAG_ROUTE_MASK == m.FLAG_ROUTE_SHORT).all(), res

@@ -115,7 +115,9 @@ __device__ __forceinline__ bool twin_row(const BatchArgs& A, const uint32_t row,
         for (uint32_t k = 0; k < kWords; ++k) aw[k] = allow[min(k * WS_BLOCK + t, nW - 1u)];
     }
 
-    constexpr uint32_t kFew = 4u, kFewShift = 20u, kFewId = (1u << kFewShift) - 1u;  // a listed entry: its id, and the number of a bias entry plus one
+    // a listed entry: its id, and the number of a bias entry plus one
+    constexpr uint32_t kFew = 4u, kFewShift = 20u, kFewId = (1u << kFewShift) - 1u, kFewBias = (1u << (32u - kFewShift)) - 1u;
+    static_assert(kWords * WS_BLOCK * 32u <= kFewId, "an id of a row that is listed, and none that is 0xffffffff");
     const uint32_t few_room = MASKED ? min(kFew * WS_BLOCK, (early_slots * 8u - kTwinBins * 4u) / 4u) : 0u;
     uint32_t n_few = 0xffffffffu;
     if (MASKED && n_all) {  // the tokens the mask allows: most rows' are few
@@ -170,7 +172,8 @@ __device__ __forceinline__ bool twin_row(const BatchArgs& A, const uint32_t row,
             uint32_t n_allowed = 0;
 #pragma unroll
             for (uint32_t w = 0; w < WS_WAVES; ++w) n_allowed += S.red_u[w];
-            by_list = nW <= kWords * WS_BLOCK && static_cast<float>(n_allowed) * static_cast<float>(n_all) * 1.1f + 64.f * static_cast<float>(V) < static_cast<float>(V) * static_cast<float>(few_room);  // uniform
+            // (a row may have more bias entries than the number has room for: only history and bias list together are bounded by the launch's tables)
+            by_list = nW <= kWords * WS_BLOCK && nb <= kFewBias && static_cast<float>(n_allowed) * static_cast<float>(n_all) * 1.1f + 64.f * static_cast<float>(V) < static_cast<float>(V) * static_cast<float>(few_room);  // uniform
         }
         if (MASKED && by_list) {
 #pragma unroll
