@@ -215,3 +215,36 @@ def test_masked_rows_with_more_bias_entries_than_the_batch_declares(V, n_bias, n
     res = gc.compare_rows(c, smp, some(rows, 23), 1)
     m = gc.pkg()
     assert res["differ"] == 0 and (smp.flags.cpu().numpy() & m.FLAG_ROUTE_MASK == m.FLAG_ROUTE_SHORT).all(), res
+
+
+@pytest.mark.parametrize("V,n_hist", [(50257, 0), (50260, 64), (262144, 8192), (384930, 262)])
+def test_top_k_rows_whose_list_just_fits(V, n_hist):
+    """Rows with 3840 to 4096 tokens above the threshold, all within a bin of it, spread over the row, in one stretch of it or in the last waves' share of every
+    chunk: the list holds them, whatever places the waves had taken. With one more it does not."""
+    rows = rows_of()
+    c = _odd(rows, V, top_k=1000, n_hist=max(n_hist, 1), n_bias=0)
+    c["bias_ids"] = c["bias_vals"] = None
+    rng = np.random.default_rng(V)
+    c["logits"][:] = (rng.standard_normal((rows, V), dtype=np.float32) - 30).astype(np.float32)
+    c["inv_t"][:], c["top_p"][:], c["min_p"][:] = 1.0, 0.95, 0.0
+    if not n_hist:
+        c["hist"] = None
+    listed = np.array([3840, 3849, 3900, 4000, 4064, 4090, 4095, 4096, 4097, 4200])[np.arange(rows) % 10]
+    for r in range(rows):
+        kind = r // 10 % 3
+        if kind == 0:
+            at = rng.permutation(V)[:listed[r]]
+        elif kind == 1:
+            at = rng.integers(0, V - listed[r]) + np.arange(listed[r])
+        else:
+            at = np.flatnonzero(np.arange(V) % 2048 >= 1536)
+            at = at[rng.permutation(at.size)[:listed[r]]]
+        if n_hist:  # (none of them touched)
+            c["hist"][r] = rng.permutation(np.setdiff1d(np.arange(20000), at))[:n_hist]
+        c["logits"][r, at] = 2.0 + rng.uniform(0.0, 0.028, at.size).astype(np.float32)
+    _, smp = run_short(c, 1, rows=some(rows), handed_back=rows)
+    back = (smp.flags.cpu().numpy() & gc.pkg().FLAG_ROUTE_HANDED_BACK) != 0
+    # (a stretch that the sample misses puts the threshold far below, where everything is listed)
+    sampled = np.arange(rows) // 10 % 3 != 1
+    assert not back[(listed <= 4096) & sampled].any(), listed[back & (listed <= 4096) & sampled]
+    assert back[listed > 4096].all()

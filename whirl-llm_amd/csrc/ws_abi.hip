@@ -260,13 +260,18 @@ void code_or_short(const ws_batch* b, uint64_t cap, BatchPlan& p) {
     if (p.code) p.workspace = p.workspace_min = 0;
 }
 
-// LDS of a row of ws_twin.h: the list, the bitmap, the tables behind it; or, where that is more than half a compute unit's and the
+// LDS of a row of ws_twin.h: the list and its spare places, the bitmap, the tables behind it; or, where that is more than half a compute unit's and the
 // other way is not, the tables below the bitmap, in the upper part of the list's place as far as they have to (not over the sample's bin
-// counts, which are in use with them; the touched tokens above the threshold are listed in what is left below the tables).
+// counts, which are in use with them; the touched tokens above the threshold are listed in what is left below the tables). Two rows a unit
+// come before spare places: without them the sweep takes its places one by one.
 void twin_plan(uint32_t nW, uint64_t cap, BatchPlan& p) {
     const uint64_t map = uint64_t{nW} * 4u, tabs = ((uint64_t{nW} * 2u + 3u) & ~uint64_t{3}) + ((cap * 2u + 3u) & ~uint64_t{3});
     const uint64_t half = kMaxLds / 2u - kStaticTwin, list = 32768u;
-    uint64_t ab = list, tabs_at = list + map, total = list + map + tabs;
+    uint64_t ab = list, total = list + map + tabs;
+    const uint64_t spare = ws::kTwinSpare * 8u, room = total <= half ? half - total : spare;  // (a row that has the unit to itself: plan_batch has seen to more than this)
+    ab += room < spare ? room & ~uint64_t{15} : spare;
+    uint64_t tabs_at = ab + map;
+    total = tabs_at + tabs;
     if (total > half && map + list <= half) {
         const uint64_t low_ab = (half - map) & ~uint64_t{15}, counts = ws::kTwinBins * 4u;
         if (low_ab >= tabs + counts + 3u) {

@@ -148,6 +148,7 @@ __host__ inline dim3 few_grid(uint32_t parts, uint32_t rows, uint32_t together) 
 }
 constexpr uint32_t kFewKeys = 7648u;  // keys of a row in its workspace (ws_few.h)
 constexpr uint32_t kTwinBins = 2048u;  // ws_twin.h: bins of the sample's logits, 1/32 e-fold each
+constexpr uint32_t kTwinSpare = 256u;  // and places behind its list, for those that its waves take and do not fill
 constexpr uint32_t kShortSplitCtrl = kShortCap * 8u, kShortSplitRowBytes = kShortSplitCtrl + 768u;  // the same of ws_short.h's shared rows
 // Workspace of one row of the three-pass kernel: per history / bias entry a word of each of phase 0's two rank
 // tables, which sit out the first sweep there. Whole memory lines, so that rows share none.

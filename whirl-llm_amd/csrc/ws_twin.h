@@ -27,8 +27,8 @@
 namespace ws {
 
 constexpr uint32_t kTwinHead = 8u;  // vectors a thread of the sample that the threshold is fitted to
-constexpr uint32_t kTwinPlaces = 32u;  // places of the list a wave takes at a time
-static_assert((kTwinPlaces - 1u) * WS_WAVES <= 256u, "the places left over: one a thread of the waves that close them");
+constexpr uint32_t kTwinPlaces = 32u;  // places of the list a wave takes at a time, where the list has kTwinSpare places more than the tokens it may hold
+static_assert((kTwinPlaces - 1u) * WS_WAVES <= kTwinSpare && kTwinSpare <= 64u * WS_WAVES, "room for the places that are taken and not filled; a thread each to close them");
 
 // LDS: the list at 0 (32 KiB; first the sample's bin counts), the bitmap of the touched tokens at lds_ab, and at lds_cnt its 16-bit popcount
 // prefixes and a 16-bit word per rank: history count | kBias | kBiases. These two are dead when the sweep begins, and where a second
@@ -54,6 +54,7 @@ __device__ __forceinline__ bool twin_row(const BatchArgs& A, const uint32_t row,
     uint32_t* invalid = touched;  // (what it holds from the sweep on)
     uint16_t* wprefix = reinterpret_cast<uint16_t*>(lds + A.lds_cnt);
     uint32_t* cnt = reinterpret_cast<uint32_t*>(lds + A.lds_cnt + ((nW * 2u + 3u) & ~3u));  // two ranks a word
+    const uint32_t spare = min(kTwinSpare, (A.lds_ab >> 3) - kShortCap);  // places behind the list's
     const uint32_t early_slots = A.lds_cnt < A.lds_ab ? min(kShortCap, A.lds_cnt >> 3) : kShortCap;  // of the list, while the tables are needed
 
     // The row: chunks of a vector a thread, whole ones and at most one that is not, and a few tokens behind the last vector
@@ -466,7 +467,7 @@ __device__ __forceinline__ bool twin_row(const BatchArgs& A, const uint32_t row,
         if (yes) {
             m = fmaxf(m, x);
             const uint32_t slot = atomicAdd(&S.s_w[1], 1u);
-            if (slot < (early ? early_slots : kShortCap)) list[slot] = (static_cast<uint64_t>(__float_as_uint(x)) << 32) | id;
+            if (slot < (early ? early_slots : kShortCap + spare)) list[slot] = (static_cast<uint64_t>(__float_as_uint(x)) << 32) | id;
             else if (early) S.s_w[2] = 1u;
             if (early) atomicAdd(&S.s_w[3], 1u);
         }
@@ -544,7 +545,10 @@ __device__ __forceinline__ bool twin_row(const BatchArgs& A, const uint32_t row,
     // ---- the sweep: sum of exp, tokens above the threshold to the list
     const bool mapped = MASKED || n_all != 0u;  // uniform
     // A wave lists its tokens at places that it takes thirty-two of at a time, so that most vectors need no word of the other waves; the few
-    // places left over at the end are filled from the list's end.
+    // places left over at the end are filled from the list's end. What is taken and not filled - one place less than that a wave, at most - has to
+    // fit beside a full list: fewer at a time where there is no such room (rows of 370000 tokens and more, two a unit). 300 rows of 100000, us, with a list of
+    // 4096 tokens: top-k 97.9, min-p 99.3 (a place a token 110 and 112; what is not filled counted against the list 236, handed back, and 134, read twice).
+    const uint32_t places = min(kTwinPlaces, spare / WS_WAVES + 1u);  // uniform
     uint32_t my_next = 0, my_end = 0;  // uniform
     float my_thr = thr;
     auto wave_value = [](uint32_t v) __attribute__((always_inline)) { return static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(v))); };
@@ -590,12 +594,12 @@ __device__ __forceinline__ bool twin_row(const BatchArgs& A, const uint32_t row,
                 list_at([&](uint32_t k, uint32_t i) { return k + (my_next + i); });
                 my_next = wave_value(my_next + n);
             } else {  // the rest of the wave's places, then new ones
-                const uint32_t left = my_end - my_next, more = max(n - left, kTwinPlaces);
+                const uint32_t left = my_end - my_next, more = max(n - left, places);
                 uint32_t from = 0;
                 if (lane == 0u) from = atomicAdd(&S.s_w[1], more);
                 from = wave_value(from);
-                if (from + more > kShortCap) {
-                    my_thr = INFINITY;  // (the list is full: nothing more to it)
+                if (from + more > kShortCap + spare) {
+                    my_thr = INFINITY;  // (more tokens than the list may hold: nothing more to it)
                 } else {
                     list_at([&](uint32_t k, uint32_t i) { return k + i < left ? k + i + my_next : k + i + (from - left); });
                     my_next = wave_value(from + (n - left));
@@ -667,7 +671,7 @@ __device__ __forceinline__ bool twin_row(const BatchArgs& A, const uint32_t row,
     {  // the places no wave has filled: the last n_left of the list take their contents to the others
 #pragma unroll
         for (uint32_t w = 0; w < WS_WAVES; ++w) n_left += S.bcnt[w];
-        if (n_list <= kShortCap && n_left) {  // uniform
+        if (n_list <= kShortCap + spare && n_left) {  // uniform
             n_list -= n_left;
             // (a wave has 64 of them; one wave for all of them took 1 us longer)
             const uint32_t first = n_list + wv * 64u, from = first + lane;
