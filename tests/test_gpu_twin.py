@@ -180,12 +180,11 @@ def test_masks_that_allow_the_whole_history(V, n_hist, n_bias, allowed, dtype):
     run_short(c if n_bias < 3 else twice_biased(c), 1, rows=some(rows, 41))
 
 
-@pytest.mark.parametrize("V,top_k,step,allowed", [(50257, 513, 0.0, None), (50257, 1024, 0.0, 0.5), (700, 700, 0.0, None), (1500, 1000, 0.0, None), (50257, 1000, 0.25, None), (50257, 1000, 0.004, None),
-                                                  (262144, 1000, 0.0, 0.1)])
-def test_wide_top_k_without_an_order(V, top_k, step, allowed):
-    """A top-k of more than 512: cuts and draw by buckets - everything listed, more listed than kept, cuts by top-p, by min-p, by both and by neither; logits so
-    coarse that a bucket is too full and the list is sorted after all, and just not so."""
-    rows = rows_of()
+WIDE = [(50257, 513, 0.0, None), (50257, 1024, 0.0, 0.5), (700, 700, 0.0, None), (1500, 1000, 0.0, None), (50257, 1000, 0.25, None), (50257, 1000, 0.004, None), (262144, 1000, 0.0, 0.1)]
+
+
+def _wide(rows, V, top_k, step, allowed):
+    """Rows cut by top-k alone, by top-p (0.3 too), by min-p and by both, cold ones among them; step: the grid the logits lie on."""
     c = _odd(rows, V, top_k=top_k, n_hist=min(300, V), n_bias=min(20, V), allowed=allowed)
     if step:
         c["logits"] = (np.round(c["logits"] / step) * step).astype(np.float32)
@@ -194,7 +193,35 @@ def test_wide_top_k_without_an_order(V, top_k, step, allowed):
     c["min_p"][1::3] = 0.02
     c["min_p"][2::6] = 1.0
     c["inv_t"][::5] = 0.3
-    run_short(c, 1, rows=some(rows, 23), handed_back=2)
+    return c
+
+
+@pytest.mark.parametrize("V,top_k,step,allowed", WIDE)
+def test_wide_top_k_without_an_order(V, top_k, step, allowed):
+    """A top-k of more than 512 in a batch that asks for no dump, which is when cuts and draw go by buckets: everything listed, more listed than kept, cuts by
+    top-p, by min-p, by both and by neither; logits so coarse that a bucket is too full and the list is sorted after all, and just not so."""
+    rows = rows_of()
+    run_short(_wide(rows, V, top_k, step, allowed), 1, rows=some(rows, 23), kept_cap=0, handed_back=2)
+
+
+@pytest.mark.parametrize("V,top_k,step,allowed", WIDE)
+def test_wide_top_k_by_buckets_and_by_the_sort(V, top_k, step, allowed):
+    """The same rows with the dump, which are sorted: tokens, counts and flags are the same, and so are probabilities and distances to the decisions but for
+    the rounding of 64-bit sums. A running mass of up to 2048 terms that reach it by chains of at most 30 additions is off by 30 x 2^-53 of itself on either side,
+    a distance to a cut by that much of the cut's mass, which is what it is divided by: 8e-15, 1e-14 with the quotients' own roundings."""
+    rows = rows_of()
+    c = _wide(rows, V, top_k, step, allowed)
+    got, want = (gc.sampler_for(c, gc.upload(c, hints=True), 1, kept_cap=cap).run() for cap in (0, 1024))
+    m = gc.pkg()
+    assert torch.equal(got.flags, want.flags)
+    # (a min-p of 1 is the largest token's own mass: reported as near, and decided the same way)
+    near = ((got.flags & m.FLAG_NEAR) != 0) & torch.from_numpy(c["min_p"] != 1.0).cuda()
+    assert int(near.sum()) <= 2
+    for k in ("token", "n_kept"):
+        assert torch.equal(getattr(got, k)[~near], getattr(want, k)[~near]), k
+    assert torch.allclose(got.prob, want.prob, rtol=3e-7, atol=0)  # (two roundings to 32 bits)
+    # (a draw of the first or last token has 1e300 or 0 in the place of one distance on both sides)
+    assert (got.margin - want.margin)[~near].abs().max().item() <= 1e-14
 
 
 @pytest.mark.parametrize("V,n_bias,n_hist,allowed", [(262144, 4096, 3, 0.1), (262144, 5000, 1, 0.05), (50257, 4095, 4, 0.02), (50257, 6000, 2, 0.02), (50257, 4097, 0, 0.02)])

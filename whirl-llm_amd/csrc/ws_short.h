@@ -162,9 +162,12 @@ __device__ __forceinline__ void short_answer(const LeanArgPtr Ap, const uint32_t
 // The same for a row with a top-k, without an order: the keys are dealt to 512 buckets as the sort would, with their masses, and one wave looks for the cuts and
 // the draw - a bucket by the buckets' running counts and masses, then a place among its few keys, which alone are put in order. What bounds a wide top-k's
 // finish where other rows sweep on the same unit (ws_twin.h) is the instructions: the rank and running mass of every key, sixteen waves in and out of a dozen barriers.
-// Masses are added up in fixed point against the maximum's, 2^-51 of it the last place: off by at most n 2^-52 of the normaliser, where running sums in 64-bit floats are
-// off by n 2^-53 of themselves. For 65 keys and more (n_list <= kShortCap - 1024: the buckets lie behind the list) of rows that are asked for neither a kept-set dump
-// nor an entropy or a query. Every thread calls it. Returns false when a bucket has more than a wave's lanes of keys (equal logits): the list still holds the same keys.
+// Masses are added up in fixed point against the maximum's, in whole units of 2^-51 and what is left of each in units of 2^-77: the order of the additions does not
+// matter, and a running mass is as good as exact until it becomes a 64-bit float. (Worked out on the CPU for 3000 lists of 600 to 2000 keys, the error of a running mass in
+// units of 2^-53 of itself: 0.5 on average and 2.9 at most; short_rules' sums 1.3 and 9.3.)
+// For 65 keys and more (n_list <= kShortCap - 1024: the buckets lie behind the list) of rows that are asked for neither a kept-set dump
+// nor an entropy or a query. Every thread calls it. Returns false when a bucket has more than a wave's lanes of keys (equal logits; where logits were 16-bit
+// floats once, hundreds are equal): the list still holds the same keys.
 // S.s_d[7]: the row's normaliser (R.z is not looked at: nobody has to keep it in registers meanwhile).
 __device__ __forceinline__ bool short_pick(uint64_t* list, const uint32_t n_list, const uint32_t row, const ShortRow& R, ShortShared& S) {
     constexpr uint32_t K = (kShortCap - 1024u) / WS_BLOCK, NB = 512u;
@@ -172,10 +175,11 @@ __device__ __forceinline__ bool short_pick(uint64_t* list, const uint32_t n_list
     const uint32_t t = threadIdx.x, lane = t & 63u;
     const uint32_t wv = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(t >> 6)));
     unsigned long long* mass = reinterpret_cast<unsigned long long*>(list + (kShortCap - 1024u));
-    uint32_t *cnt = reinterpret_cast<uint32_t*>(mass + NB), *start = cnt + NB;
+    uint32_t *rest = reinterpret_cast<uint32_t*>(mass + NB), *cnt = rest + NB, *start = cnt;  // (the buckets' first places, once their counts are read)
     const double inv_t = static_cast<double>(R.inv_t), min_p = R.min_p;
     const bool use_top_p = R.top_p < 1.0, use_min_p = min_p > 0.0;
-    constexpr double kFix = 2251799813685248.0, kUnfix = 1.0 / kFix;  // 2^51: a mass is 1 at most, and there are 4096 of them
+    // (2^51 and 2^26: a mass is 1 at most, and there are 4096 of them; the rests of a bucket's 64 keys are 32 bits together)
+    constexpr double kFix = 2251799813685248.0, kUnfix = 1.0 / kFix, kRest = 67108864.0, kUnrest = kUnfix / kRest;
     float d[K], dmax = 0.f, dsum = 0.f;
 #pragma unroll
     for (uint32_t k = 0; k < K; ++k) {
@@ -188,11 +192,13 @@ __device__ __forceinline__ bool short_pick(uint64_t* list, const uint32_t n_list
     }
     if (t < NB) {
         mass[t] = 0ull;
+        rest[t] = 0u;
         cnt[t] = 0u;
     }
     if (t == 0u) {
         S.s_w[6] = 0u;
-        S.s_w[7] = 0xffffffffu;
+        S.s_w[8] = 0u;
+        S.s_q[0] = ~0ull;
     }
     dmax = wave_max(dmax);
     dsum = wave_sum(dsum);
@@ -213,39 +219,40 @@ __device__ __forceinline__ bool short_pick(uint64_t* list, const uint32_t n_list
     const float per = 1.f / mean;
     auto level = [&](float d_) { return static_cast<float>(__float_as_uint(__fadd_rn(1.f, __fmul_rn(fmaxf(__fsub_rn(dmax, d_), 0.f), per))) - 0x3f800000u); };
     const float scale = static_cast<float>(NB) / (level(0.f) + 1.f);
-    uint32_t at[K], pass = 0;  // bucket | place in it << 16
-    float near = INFINITY;
+    uint32_t at[K];  // bucket | place in it << 16
 #pragma unroll
     for (uint32_t k = 0; k < K; ++k)
         if (k * WS_BLOCK < n_list && k * WS_BLOCK + t < n_list) {
-            const double e = exp_down(static_cast<double>(d[k]) * inv_t);
-            const uint32_t b = NB - 1u - min(NB - 1u, static_cast<uint32_t>(level(d[k]) * scale));
-            at[k] = b | (atomicAdd(&cnt[b], 1u) << 16);
-            atomicAdd(&mass[b], static_cast<unsigned long long>(fma(e, kFix, 0.5)));
+            const uint32_t b = NB - 1u - min(NB - 1u, static_cast<uint32_t>(level(d[k]) * scale)), place = atomicAdd(&cnt[b], 1u);
+            at[k] = b | (place << 16);
+            if (place >= 64u) S.s_w[8] = 1u;
+        }
+    uint32_t pass = 0;
+    double near = INFINITY;
+#pragma unroll
+    for (uint32_t k = 0; k < K; ++k)
+        if (k * WS_BLOCK < n_list && k * WS_BLOCK + t < n_list) {
+            const double e = exp_down(static_cast<double>(d[k]) * inv_t), fixed = e * kFix, whole = floor(fixed);
+            const uint32_t b = at[k] & 0xffffu;
+            atomicAdd(&mass[b], static_cast<unsigned long long>(whole));
+            atomicAdd(&rest[b], static_cast<uint32_t>((fixed - whole) * kRest));
             pass += e >= min_p ? 1u : 0u;
-            near = fminf(near, static_cast<float>(fabs(e - min_p)));
+            near = fmin(near, fabs(e - min_p));
         }
     if (use_min_p) {
         pass = wave_sum(pass);
-        const uint32_t nearest = ~wave_max_u32(~__float_as_uint(near));
         if (lane == 0u && pass) atomicAdd(&S.s_w[6], pass);
-        if (lane == 0u) atomicMin(&S.s_w[7], nearest);
+        const unsigned long long bits = static_cast<unsigned long long>(__double_as_longlong(near));  // (of numbers that are not negative: in their order)
+        if (bits < S.s_q[0]) atomicMin(&S.s_q[0], bits);
     }
     __syncthreads();
+    if (S.s_w[8] != 0u) return false;
     uint32_t c8[8], n_in = 0;
-    uint64_t g8[8], g_in = 0;
     if (wv == 0u) {  // a lane has eight buckets
 #pragma unroll
         for (uint32_t k = 0; k < 8u; ++k) {
             c8[k] = cnt[lane * 8u + k];
-            g8[k] = mass[lane * 8u + k];
-        }
-        uint32_t most = 0;
-#pragma unroll
-        for (uint32_t k = 0; k < 8u; ++k) {
-            most = max(most, c8[k]);
             n_in += c8[k];
-            g_in += g8[k];
         }
         uint32_t run = wave_incl_scan(n_in) - n_in;
 #pragma unroll
@@ -254,12 +261,7 @@ __device__ __forceinline__ bool short_pick(uint64_t* list, const uint32_t n_list
             run += c8[k];
         }
         n_in = run;
-        g_in = wave_incl_scan(g_in);
-        const bool crowded = __ballot(most > 64u) != 0ull;
-        if (lane == 0u) S.s_w[8] = crowded ? 1u : 0u;
     }
-    __syncthreads();
-    if (S.s_w[8] != 0u) return false;
     uint64_t key[K];  // (read again: the exponentials have the registers)
 #pragma unroll
     for (uint32_t k = 0; k < K; ++k) key[k] = k * WS_BLOCK < n_list && k * WS_BLOCK + t < n_list ? list[k * WS_BLOCK + t] : 0ull;
@@ -271,7 +273,18 @@ __device__ __forceinline__ bool short_pick(uint64_t* list, const uint32_t n_list
     if (wv != 0u) return true;
 
     // ------------------------------------------------------------------ one wave
-    auto real = [&](uint64_t g) { return static_cast<double>(g) * kUnfix; };
+    double m8[8];  // the running mass with each of the lane's buckets
+    {
+        uint64_t g8[8], l8[8], g = 0, l = 0;
+#pragma unroll
+        for (uint32_t k = 0; k < 8u; ++k) {
+            g8[k] = g += mass[lane * 8u + k];
+            l8[k] = l += rest[lane * 8u + k];
+        }
+        const uint64_t g0 = wave_incl_scan(g) - g, l0 = wave_incl_scan(l) - l;
+#pragma unroll
+        for (uint32_t k = 0; k < 8u; ++k) m8[k] = fma(static_cast<double>(l0 + l8[k]), kUnrest, static_cast<double>(g0 + g8[k]) * kUnfix);
+    }
     // a bucket's keys in order, one a lane, with what is ranked before them
     struct Place {
         uint32_t n, before;  // keys in the bucket, and before it
@@ -281,28 +294,26 @@ __device__ __forceinline__ bool short_pick(uint64_t* list, const uint32_t n_list
     // the first bucket with which the running count and mass satisfy `reached`; found: whether there is one
     auto look = [&](auto&& reached, bool& found) __attribute__((always_inline)) {
         Place R_;
-        const uint64_t any = __ballot(reached(n_in, real(g_in)));
+        const uint64_t any = __ballot(reached(n_in, m8[7]));
         found = any != 0ull;
         const uint32_t f = found ? static_cast<uint32_t>(__ffsll(static_cast<unsigned long long>(any)) - 1) : 63u;
-        uint32_t run = f ? lane_value(n_in, f - 1u) : 0u, b = 0, n = 0, first = run;
-        uint64_t sum = f ? lane_value(g_in, f - 1u) : 0ull, before = sum;
+        uint32_t run = f ? lane_value(n_in, f - 1u) : 0u, n = 0, first = run;
+        double sum = f ? lane_value(m8[7], f - 1u) : 0.0, before = sum;
         bool done = false;
 #pragma unroll
         for (uint32_t k = 0; k < 8u; ++k) {
             const uint32_t c = lane_value(c8[k], f);
-            const uint64_t g = lane_value(g8[k], f);
+            const double with = lane_value(m8[k], f);
             if (!done && c) {  // uniform
-                b = f * 8u + k;
                 n = c;
                 first = run;
                 before = sum;
                 run += c;
-                sum += g;
-                done = reached(run, real(sum));
+                sum = with;
+                done = reached(run, sum);
             }
         }
-        const uint32_t s0 = first;  // (the buckets lie one behind the other)
-        const uint64_t own = lane < n ? list[s0 + lane] : 0ull;
+        const uint64_t own = lane < n ? list[first + lane] : 0ull;  // (the buckets lie one behind the other)
         uint32_t above = 0;
         for (uint32_t j = 0; j < n; ++j) above += lane_value(own, j) > own ? 1u : 0u;  // uniform
         uint64_t* sorted = reinterpret_cast<uint64_t*>(mass);  // (the masses are in registers)
@@ -314,15 +325,15 @@ __device__ __forceinline__ bool short_pick(uint64_t* list, const uint32_t n_list
         R_.before = first;
         R_.key = lane < n ? sorted[lane] : 0ull;
         R_.e = lane < n ? exp_down(static_cast<double>(__fsub_rn(R.m, unkey32(static_cast<uint32_t>(R_.key >> 32)))) * inv_t) : 0.0;
-        const double base = real(before), inc = wave_incl_scan(R_.e), up = __shfl_up(inc, 1);
-        R_.cin = base + inc;
-        R_.cex = base + (lane ? up : 0.0);
+        const double inc = wave_incl_scan(R_.e), up = __shfl_up(inc, 1);
+        R_.cin = before + inc;
+        R_.cex = before + (lane ? up : 0.0);
         __builtin_amdgcn_wave_barrier();
         return R_;
     };
     bool found;
     const uint32_t n_cand = R.n_cand;
-    const double all = real(lane_value(g_in, 63u));
+    const double all = lane_value(m8[7], 63u);
     double Zk1 = all, e_last = -1.0;
     if (n_list > n_cand) {
         const Place at_k = look([&](uint32_t n, double) { return n >= n_cand; }, found);
@@ -350,7 +361,7 @@ __device__ __forceinline__ bool short_pick(uint64_t* list, const uint32_t n_list
     }
     if (use_min_p) {
         const uint32_t passed = S.s_w[6];
-        const double nearest = passed >= n_cand && e_last >= 0.0 ? fabs(e_last - min_p) : static_cast<double>(__uint_as_float(S.s_w[7]));
+        const double nearest = passed >= n_cand && e_last >= 0.0 ? fabs(e_last - min_p) : __longlong_as_double(static_cast<long long>(S.s_q[0]));
         mg_min_p = {fmin(min_p, nearest), min_p};
         if (passed < n3) {
             n3 = max(passed, 1u);
