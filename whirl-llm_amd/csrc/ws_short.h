@@ -54,8 +54,13 @@ struct ShortShared {
     alignas(16) uint32_t bcnt[64], bstart[64];  // the bucket sort's counts and starts
 };
 
+// How far the keys of a list lie below its largest: the largest such distance, and their sum (known: somebody has looked).
+struct ShortSpan {
+    float dmax = 0.f, total = 0.f;
+    bool known = false;
+};
 // Puts the n_list (<= kShortCap) different keys in descending order. m: the largest of their logits. Every thread calls it.
-__device__ __forceinline__ void short_sort(uint64_t* list, const uint32_t n_list, const float m, ShortShared& S) {
+__device__ __forceinline__ void short_sort(uint64_t* list, const uint32_t n_list, const float m, ShortShared& S, const ShortSpan span = {}) {
     const uint32_t t = threadIdx.x;
     if (n_list <= WS_BLOCK / 4u) {
         // A short list (a lone row's top-k 40 lists some 200 keys): every key against every other, four threads a key,
@@ -85,26 +90,30 @@ __device__ __forceinline__ void short_sort(uint64_t* list, const uint32_t n_list
         // list is the tail of a row's logits, dense at its lower end, with a few tokens far above as a rule. (On a linear
         // scale a third of the keys could share a bucket, and each of them counts the others: 871 of 8 rows' keys took 12K
         // clocks, 8K of them there.)
-        float dmax = 0.f, dsum = 0.f;
-        for (uint32_t k = t; k < n_list; k += WS_BLOCK) {
-            const float d = fminf(__fsub_rn(m, unkey32(static_cast<uint32_t>(list[k] >> 32))), 3e38f);
-            dmax = fmaxf(dmax, d);
-            dsum += d;
-        }
-        dmax = wave_max(dmax);
-        dsum = wave_sum(dsum);
-        __syncthreads();  // (the row's maximum and sum were read from these words, and not every wave need have come by)
-        if ((t & 63u) == 0u) {
-            S.red_f[t >> 6] = dmax;
-            S.red_d[t >> 6] = static_cast<double>(dsum);
-        }
-        __syncthreads();
-        dmax = S.red_f[0];
-        double total = S.red_d[0];
+        float dmax = span.dmax;
+        double total = static_cast<double>(span.total);
+        if (!span.known) {
+            float dsum = 0.f;
+            for (uint32_t k = t; k < n_list; k += WS_BLOCK) {
+                const float d = fminf(__fsub_rn(m, unkey32(static_cast<uint32_t>(list[k] >> 32))), 3e38f);
+                dmax = fmaxf(dmax, d);
+                dsum += d;
+            }
+            dmax = wave_max(dmax);
+            dsum = wave_sum(dsum);
+            __syncthreads();  // (the row's maximum and sum were read from these words, and not every wave need have come by)
+            if ((t & 63u) == 0u) {
+                S.red_f[t >> 6] = dmax;
+                S.red_d[t >> 6] = static_cast<double>(dsum);
+            }
+            __syncthreads();
+            dmax = S.red_f[0];
+            total = S.red_d[0];
 #pragma unroll
-        for (uint32_t w = 1; w < WS_WAVES; ++w) {
-            dmax = fmaxf(dmax, S.red_f[w]);
-            total += S.red_d[w];
+            for (uint32_t w = 1; w < WS_WAVES; ++w) {
+                dmax = fmaxf(dmax, S.red_f[w]);
+                total += S.red_d[w];
+            }
         }
         const float mean = fmaxf(dmax - static_cast<float>(total) / static_cast<float>(n_list), dmax * 1e-6f + 1e-30f);
         // (512 buckets, their counters behind the keys, while the list leaves that room; else 64 in the static words)
@@ -167,9 +176,9 @@ __device__ __forceinline__ void short_answer(const LeanArgPtr Ap, const uint32_t
 // units of 2^-53 of itself: 0.5 on average and 2.9 at most; short_rules' sums 1.3 and 9.3.)
 // For 65 keys and more (n_list <= kShortCap - 1024: the buckets lie behind the list) of rows that are asked for neither a kept-set dump
 // nor an entropy or a query. Every thread calls it. Returns false when a bucket has more than a wave's lanes of keys (equal logits; where logits were 16-bit
-// floats once, hundreds are equal): the list still holds the same keys.
+// floats once, hundreds are equal), which the counts tell before anybody has worked out a mass: the list still holds the same keys, and `span` is known.
 // S.s_d[7]: the row's normaliser (R.z is not looked at: nobody has to keep it in registers meanwhile).
-__device__ __forceinline__ bool short_pick(uint64_t* list, const uint32_t n_list, const uint32_t row, const ShortRow& R, ShortShared& S) {
+__device__ __forceinline__ bool short_pick(uint64_t* list, const uint32_t n_list, const uint32_t row, const ShortRow& R, ShortShared& S, ShortSpan& span) {
     constexpr uint32_t K = (kShortCap - 1024u) / WS_BLOCK, NB = 512u;
     static_assert(WS_BLOCK >= NB, "a thread a bucket");
     const uint32_t t = threadIdx.x, lane = t & 63u;
@@ -214,6 +223,7 @@ __device__ __forceinline__ bool short_pick(uint64_t* list, const uint32_t n_list
         dmax = fmaxf(dmax, __uint_as_float(S.bcnt[w]));
         total += __uint_as_float(S.bstart[w]);
     }
+    span = {dmax, total, true};
     const float mean = fmaxf(dmax - total / static_cast<float>(n_list), dmax * 1e-6f + 1e-30f);
     // (the scale of short_sort's buckets)
     const float per = 1.f / mean;
@@ -227,6 +237,8 @@ __device__ __forceinline__ bool short_pick(uint64_t* list, const uint32_t n_list
             at[k] = b | (place << 16);
             if (place >= 64u) S.s_w[8] = 1u;
         }
+    __syncthreads();
+    if (S.s_w[8] != 0u) return false;
     uint32_t pass = 0;
     double near = INFINITY;
 #pragma unroll
@@ -245,8 +257,6 @@ __device__ __forceinline__ bool short_pick(uint64_t* list, const uint32_t n_list
         const unsigned long long bits = static_cast<unsigned long long>(__double_as_longlong(near));  // (of numbers that are not negative: in their order)
         if (bits < S.s_q[0]) atomicMin(&S.s_q[0], bits);
     }
-    __syncthreads();
-    if (S.s_w[8] != 0u) return false;
     uint32_t c8[8], n_in = 0;
     if (wv == 0u) {  // a lane has eight buckets
 #pragma unroll

@@ -754,17 +754,20 @@ __device__ __forceinline__ bool twin_row(const BatchArgs& A, const uint32_t row,
     R.m = m;
     R.n_cand = n_cand;
     R.by_k = by_k;
-    // A wide top-k, two candidates a thread and more: its cuts and draw without an order (us, with the sort and without: 1024 masked rows of 262144, top-k 1000, 247.5 / 241.5, 300
-    // of 262144 101.6 / 97.9; level at a top-k of 100 to 500, and rows with a min-p alone, whose keys crowd at the floor, 86.7 / 95.4).
+    // A wide top-k, two candidates a thread and more: its cuts and draw without an order (us, with the sort and without, top-k 1000: 1024 masked rows of 262144 248 / 243, 300
+    // of 262144 91.9 / 88.6, 512 of 151936 74.6 / 71.2, 1000 of 32000 67.9 / 63.7; level at a top-k of 100 to 500, and rows with a min-p alone, whose keys crowd at the floor, slower: 86.7 / 95.4).
+    // Rows with a bucket too full for it are sorted after all: of fp32 logits that were bf16 once 512 rows of 151936, nearly all of which have one, take 84.9 / 85.8, 300 of 262144,
+    // half of which have, 102.6 / 103.2, 1024 masked ones, few of which have, 260 / 247.
+    ShortSpan span;
     const LeanArgPtr Ap = (LeanArgPtr)__builtin_amdgcn_kernarg_segment_ptr();
     if (DT == 0 && by_k && n_cand > WS_BLOCK && n_list <= kShortCap - 1024u && !Ap->kept_ids && !Ap->entropy && !Ap->query_prob) {  // uniform
         if (t == 0u) S.s_d[7] = R.z;
         __syncthreads();  // (the words that say which places were left over have been read as well)
-        if (short_pick(list, n_list, row, R, S)) return true;
+        if (short_pick(list, n_list, row, R, S, span)) return true;
         R.z = S.s_d[7];
         __syncthreads();
     }
-    short_sort(list, n_list, m, S);
+    short_sort(list, n_list, m, S, span);
     WSS_MARK(6);  // sorted
     // the k-th largest has to lie above the threshold (below it, the sweep has left out tokens that rank before it); a min-p row's
     // threshold lies below its floor by construction
