@@ -1351,14 +1351,15 @@ struct Walk {
     uint32_t before_c, found;
 };
 // The first key, in descending order, at which the running total - counts (by_mass 0) or masses - reaches `want`;
-// before_c / before_m: what ranks before it. found 0: the whole row, of mass `total`, stays below `want`.
+// before_c / before_m: what ranks before it. found 0: the whole row, of mass `total`, stays below `want`. Where at least `enough` tokens rank before
+// the key's bin nobody asks for the key: before_c says so, and the rest is not looked for (key 0).
 // The bin is read off the prefixes. Inside it a token is K, its order key without the id's twelve idle bits: while the bin, or
 // what is left of it, has more tokens than LDS has room for, a pass finds the span of their keys and a pass divides it by 1024
 // (thousands of equal logits: the span is one of ids); then a pass lists them and every key is compared with every other.
 // Radix passes over all of the row from the top of the key - up to six a question, an exp of every token in each, and nearly
 // all tokens meeting in a few words of the first - took 7.2 ms
 // a launch with such rows (151936 bf16 tokens, Zipfian, top-p 0.9 and up); now 1.0 ms.
-__device__ __noinline__ Walk exact_walk(const ExactIn in, const uint64_t total, const uint32_t by_mass, const uint64_t want) {
+__device__ __noinline__ Walk exact_walk(const ExactIn in, const uint64_t total, const uint32_t by_mass, const uint64_t want, const uint32_t enough) {
     extern __shared__ __align__(16) unsigned char lds[];
     // its few words lie behind the last bin's prefix (static LDS of its own would come off what a batch may ask for)
     static_assert(kTail + 8 + 6 + 16 + 8 + 1 <= kBins && WS_WAVES <= 16, "room behind the prefixes");
@@ -1390,6 +1391,10 @@ __device__ __noinline__ Walk exact_walk(const ExactIn in, const uint64_t total, 
             if (bin == 0xffffffffu) return Walk{0ull, total, 0ull, V, 0u};
             uint64_t base_m = hm[bin];
             uint32_t base_c = hc[bin], n_in = end_c(bin) - base_c;
+            if (base_c >= enough) {  // uniform
+                __syncthreads();  // (the caller may call again)
+                return Walk{0ull, base_m, 0ull, base_c, 1u};
+            }
             uint64_t lo = 0ull, hi = ~0ull;
             auto each_inside = [&](auto&& f) __attribute__((always_inline)) {
                 R.each_token([&](uint32_t i, float x) __attribute__((always_inline)) {
@@ -1590,7 +1595,7 @@ __device__ __noinline__ ExactOut exact_row(const ExactIn in) {
     }
     __syncthreads();
 
-    auto walk = [&](bool by_mass, uint64_t want) __attribute__((always_inline)) { return exact_walk(in, Zfx, by_mass ? 1u : 0u, want); };
+    auto walk = [&](bool by_mass, uint64_t want, uint32_t enough = 0xffffffffu) __attribute__((always_inline)) { return exact_walk(in, Zfx, by_mass ? 1u : 0u, want, enough); };
     // smallest race key of the block, the candidate that is earlier in sorted order (the larger `who`) on equal keys
     const double inf = __longlong_as_double(0x7FF0000000000000ll);
     auto block_first = [&](double& k, uint64_t& who) {
@@ -1677,11 +1682,14 @@ __device__ __noinline__ ExactOut exact_row(const ExactIn in) {
     if (!open_row) {
         if (use_top_p) {
             double Xf = in.top_p * (prefix_mode ? static_cast<double>(kept_fx) : (in.top_k > 0 ? Zs : Zfs) * kFx);
-            auto cut_at = [&](double xf) { return walk(true, xf > 1.0 ? static_cast<uint64_t>(ceil(xf)) : 1ull); };
-            Walk w2 = cut_at(Xf);
-            if (!prefix_mode && in.top_k == 0 && (!w2.found || w2.before_c >= 16384u)) {  // past the engine's candidates: the complete row
+            auto cut_at = [&](double xf, uint32_t enough) { return walk(true, xf > 1.0 ? static_cast<uint64_t>(ceil(xf)) : 1ull, enough); };
+            // past the engine's candidates it is the complete row, whose mass is another: which it is the bins' counts tell, as a rule, without the six passes over the
+            // row that the key takes (us, top-p 0.9: 64 rows of 151936 with logits in steps of 0.5 948 / 697, 256 of 200000 N(0, 0.5) at T 1.4 848 / 668)
+            const bool engine = !prefix_mode && in.top_k == 0;
+            Walk w2 = cut_at(Xf, engine ? 16384u : 0xffffffffu);
+            if (engine && (!w2.found || w2.before_c >= 16384u)) {
                 Xf = in.top_p * static_cast<double>(Zfx);
-                w2 = cut_at(Xf);
+                w2 = cut_at(Xf, 0xffffffffu);
             }
             if (w2.found && w2.before_c < nk) {
                 const double inc = static_cast<double>(w2.before_m + w2.own_m), exc = static_cast<double>(w2.before_m);
