@@ -406,3 +406,29 @@ def test_rows_at_the_ends_of_the_bin_caches(V, masked):
         c["allow"] = rng.integers(0, 1 << 32, (3, (V + 31) // 32), dtype=np.uint64).astype(np.uint32) | np.uint32(0x10000001)
     res, _ = run_lean(c, 1, handed_back=1)
     assert res["exact"] == 3, res
+
+
+@pytest.mark.parametrize("V,masked,n_hist", [(32000, False, 0), (50257, True, 300), (151936, False, 2000), (163844, True, 0), (262144, False, 700), (262144, True, 3000)])
+def test_rows_whose_cut_no_list_holds(V, masked, n_hist):
+    """Logits on a grid, thousands of tokens each step, the cut and the draw among them: answered by the exact path from what the sweep has left - with touched tokens
+    in the ties and above them, before and behind the 16384th token, by top-p, min-p and both."""
+    rows = 12
+    c = _no_top_k(gc.make_cfg2(rows=rows, V=V, n_hist=n_hist, n_bias=50 if n_hist else 0))
+    rng = np.random.default_rng(V)
+    c["logits"] = (np.round(rng.standard_normal((rows, V)) * 4) / 2).astype(np.float32)
+    c["inv_t"] = np.linspace(0.6, 1.2, rows).astype(np.float32)
+    c["top_p"] = np.array([0.3, 0.5, 0.6, 0.7, 0.8, 0.9, 0.95, 0.99, 1.0, 1.0, 0.6, 0.9])
+    c["min_p"] = np.array([0.0] * 8 + [0.02, 0.3, 0.05, 0.01])
+    for r in range(rows):
+        if n_hist:
+            c["hist"][r][:2] = [V - 1, V - 1 - r % 4]
+        c["logits"][r, V - 1 - r % 4] = 5.0
+    if masked:
+        on = rng.random((rows, (V + 31) // 32 * 32)) < 0.8
+        c["allow"] = np.ascontiguousarray(np.packbits(on, axis=1, bitorder="little").view(np.uint32))
+    res, smp = run_lean(c, 1, max_differ=1, handed_back=rows)
+    fl, m = smp.flags.cpu().numpy(), gc.pkg()
+    assert ((fl & m.FLAG_ROUTE_EXACT) != 0).sum() >= (1 if V < 100000 else 6), fl
+    assert (((fl & m.FLAG_ROUTE_EXACT) != 0) <= ((fl & m.FLAG_ROUTE_HANDED_BACK) != 0)).all()
+    nk = smp.n_kept.cpu().numpy()
+    assert V < 100000 or (nk < 16384).any() and (nk > 16384).any()

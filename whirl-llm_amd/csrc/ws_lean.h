@@ -408,7 +408,10 @@ struct LeanShared {
     uint32_t s_w[16];
     uint32_t red_u[WS_WAVES];
     float red_f[WS_WAVES];
-    float top;  // what lean_row leaves when it returns false
+    // what lean_row leaves when it returns false: which way the row goes, its maximum, the tokens its history and bias list touch, its normaliser
+    float top, m_left;
+    uint32_t touched_left;
+    double z_left;
 #ifdef WS_PHASE_TIMERS
     long long marks[32];
 #endif
@@ -417,8 +420,9 @@ struct LeanShared {
 #ifdef WS_PHASE_TIMERS
 __device__ __forceinline__ double sel_dbg(const LeanShared& S) { return S.sel.n_r0 + 1e5 * S.sel.n_r1 + 1e10 * (S.sel.r0hi - S.sel.r0lo + 1) + 1e12 * (S.sel.r1hi - S.sel.r1lo + 1); }
 #endif
-// One row. Returns false when the row is left to others (nothing has been written for it then): S.top is NaN, and it is the three-pass code's; or the row's maximum,
-// and it is to be swept once more from there down (AGAIN; its arguments are at `args`).
+// One row. Returns false when the row is left to others (nothing has been written for it then): S.top is NaN, and it is the three-pass code's; or infinite, and the exact
+// path is to answer it (the touched tokens' tables are where that looks for them); or the row's maximum, and it is to be swept once more from there down (AGAIN; its
+// arguments are at `args`).
 template <bool MASKED, bool AGAIN, int NREG>
 __device__ __forceinline__ bool lean_row(const BatchArgs& A, const LeanArgPtr args, const uint32_t row, LeanShared& S) {
     constexpr uint32_t kTok = 4u, kTokLog = 2u;  // tokens in a 128-bit vector, which is one register of the bin cache: the low eight bits of each bin
@@ -1154,7 +1158,22 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const LeanArgPtr ar
         }
     }
     __syncthreads();
-    if (!sel.ok) WSL_FAIL(5);
+    if (!sel.ok) {
+        // Tied or flat rows. The three-pass code would count the row once more, to find that its list does not hold the tokens either: its bins lie elsewhere, but what
+        // one bin has too many of it has as well, and half as many again of several bins are taken to be too many for both.
+        const BinRec dlo = found(2u), dhi = found(3u);
+        BinRec cut = found(0u);
+        if (cut.b != 0xffffffffu && cut.cex >= 16384u) cut = found(1u);
+        const uint32_t most = max(max(dlo.c, dhi.c), sel.topp_in_list ? cut.c : 0u);
+        if (dlo.b == 0xffffffffu || dhi.b == 0xffffffffu || dhi.b < dlo.b || sel.r0hi >= kLeanTail || (most <= kLeanMaxList && sel.n_r0 + sel.n_r1 <= kLeanMaxList + kLeanMaxList / 2u)) WSL_FAIL(5);
+        if (t == 0u) {
+            S.top = INFINITY;
+            S.m_left = m;
+            S.touched_left = n_touched;
+            S.z_left = Z;
+        }
+        return false;
+    }
     const int r0lo = sel.r0lo, r0hi = sel.r0hi, r1lo = sel.r1lo, r1hi = sel.r1hi;
     const bool has_r1 = r1hi >= r1lo;
     const uint32_t nb0 = static_cast<uint32_t>(r0hi - r0lo + 1), nb1 = has_r1 ? static_cast<uint32_t>(r1hi - r1lo + 1) : 0u;
@@ -1627,17 +1646,61 @@ __device__ __noinline__ __attribute__((not_tail_called)) void three_pass_row(Lea
     if (threadIdx.x == 0) A.flags[row] |= kRouteHandedBack;
 }
 
+// A row whose cut or draw falls among more tokens than a list holds: answered by the exact path as the three-pass code would have it done, from the sweep's maximum and normaliser
+// and with the touched tokens' tables that the sweep has left. (Logits in steps of 0.5, us, by way of the
+// three-pass code and straight: 64 rows of 262144 at top-p 0.9 1157 / 1030, at 0.6 1072 / 947, a lone one 806 / 682; without the sweep in vain, as they were before this kernel took rows of that
+// length, 954 and 692 at top-p 0.6.)
+__device__ __noinline__ __attribute__((not_tail_called)) void exact_left_row(LeanArgPtr Ap_, const uint32_t row_, __attribute__((address_space(3))) LeanShared* S) {
+    const LeanArgPtr Ap = wave_args(Ap_);
+    const uint32_t row = __builtin_amdgcn_readfirstlane(row_);
+    const BatchArgs& A = *(const BatchArgs*)Ap;
+    const LeanRowParams P = load_row_params(A, row, Ap);
+    ExactIn in;
+    in.base = static_cast<const unsigned char*>(A.logits) + static_cast<size_t>(row) * A.row_stride * 4u;
+    in.allow = A.allow ? A.allow + static_cast<size_t>(row) * A.allow_stride : nullptr;
+    in.V = A.vocab;
+    in.dtype = 0;
+    in.touched_at = __builtin_amdgcn_readfirstlane(S->touched_left) ? A.lds_ab : 0xffffffffu;
+    in.m = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(S->m_left)));
+    in.inv_t = P.inv_t;
+    in.top_k = in.n1_asked = 0u;
+    in.top_p = P.top_p;
+    in.min_p = P.min_p;
+    in.u = batch_uniform(A.rng, P.seed, row, P.step, 0);
+    in.rbase = 0ull;
+    in.mode = (P.top_p < 1.0 ? 4u : 0u) | (P.min_p > 0.0 ? 8u : 0u);
+    const float m = in.m, z = static_cast<float>(S->z_left);
+    const ExactOut out = exact_row(in);
+    if (threadIdx.x == 0) {
+        A.token[row] = out.token;
+        A.flags[row] = kRouteHandedBack | kRouteExact | (out.mg_top_p < A.tol ? kNearTopP : 0u) | (out.mg_min_p < A.tol ? kNearMinP : 0u) | (out.mg_draw < A.tol ? kNearDraw : 0u);
+        if (A.prob) A.prob[row] = static_cast<float>(out.ptok);
+        if (A.n_kept) A.n_kept[row] = out.n3;
+        if (A.stats) {
+            A.stats[2 * row] = m;
+            A.stats[2 * row + 1] = z;
+        }
+        if (A.margin) {
+            A.margin[3 * row] = out.mg_top_p;
+            A.margin[3 * row + 1] = out.mg_min_p;
+            A.margin[3 * row + 2] = out.mg_draw;
+        }
+    }
+}
+
 // What lean_row has left of a row. (A function of its own, as above: as a loop around that code in the kernel it cost the kernel some hundred spilled registers.)
 template <bool MASKED, int NREG>
 __device__ __noinline__ __attribute__((not_tail_called)) void lean_rest(LeanArgPtr Ap_, const uint32_t row_, __attribute__((address_space(3))) LeanShared* S) {
     LeanArgPtr Ap = wave_args(Ap_);
     const uint32_t row = __builtin_amdgcn_readfirstlane(row_);
-    const float top = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(S->top)));
-    if (top == top) {
+    float top = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(S->top)));
+    if (top < INFINITY) {
         if (lean_row<MASKED, true, NREG>(*(const BatchArgs*)Ap, Ap, row, *(LeanShared*)S)) return;
         __syncthreads();
+        top = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(S->top)));
     }
-    three_pass_row<false>(Ap, row);
+    if (top == INFINITY) exact_left_row(Ap, row, S);
+    else three_pass_row<false>(Ap, row);
 }
 
 // MASKED: the batch has an allow mask (a kernel of its own: one build carrying both paths spilled far more registers)
