@@ -136,6 +136,7 @@ struct DeviceRows::Dev {
     std::uint32_t* done = nullptr;     // [row_cap]
     std::uint32_t turn = 0;            // what the last launch writes there
     bool in_flight = false;            // a launch has not been waited for (an exception came first)
+    bool was_left = false;             // the last lone row was one that the quick kernel leaves: as a rule so is the request's next
     std::int32_t* kept_ids = nullptr;  // [row_cap][cap]
     float* kept_logits = nullptr;
     std::int32_t* hist = nullptr;      // the history, once per row
@@ -336,13 +337,15 @@ void DeviceRows::filterOnDevice(const Sampler& s, std::uint32_t gr0, std::uint32
     b.workspace = d.work.at;
     b.workspace_bytes = d.work.bytes;
     d.in_flight = true;
-    check(ws_sample_batch_try_host(stream_, &b, d.done, ++d.turn), "ws_sample_batch");
+    const bool quick = n == 1 && !d.was_left;
+    check((quick ? ws_sample_batch_try_host : ws_sample_batch_notify_host)(stream_, &b, d.done, ++d.turn), "ws_sample_batch");
     waitForRows(n);  // results and kept sets are in host memory now
-    if (n == 1 && o.flags[0] == WS_FLAGS_LEFT) {  // (a lone row that the quick kernel has left)
+    if (quick && o.flags[0] == WS_FLAGS_LEFT) {
         check(ws_sample_batch_notify_host(stream_, &b, d.done, ++d.turn), "ws_sample_batch");
         waitForRows(n);
     }
     d.in_flight = false;
+    if (n == 1) d.was_left = (o.flags[0] & WS_FLAG_ROUTE_HANDED_BACK) != 0;
     const Dev::ResultView& h = o;
     ready_.clear();
     ready_.resize(n);
