@@ -21,11 +21,10 @@ def run_short(c, rng_mode, rows=None, kept_cap=1024, max_differ=0, handed_back=0
         d["top_k_max"] = top_k_max
     assert d["top_k_max"] >= 1 or d["min_p_min"] > 0
     smp = gc.sampler_for(c, d, rng_mode, kept_cap=kept_cap, **more)
-    if kept_cap:  # (0: a batch without the dump, which some rows have a finish of their own for)
-        smp.kept_ids.fill_(-7)
+    smp.kept_ids.fill_(-7)
     smp.run()
     rows = range(c["rows"]) if rows is None else rows
-    res = gc.compare_rows(c, smp, rows, rng_mode, check_kept=bool(kept_cap))
+    res = gc.compare_rows(c, smp, rows, rng_mode)
     assert res["differ"] <= max_differ and res["exact"] + res["differ"] == res["rows"], res
     fl = smp.flags.cpu().numpy()
     short = int(((fl & m.FLAG_ROUTE_SHORT) != 0).sum())

@@ -180,6 +180,24 @@ def test_masks_that_allow_the_whole_history(V, n_hist, n_bias, allowed, dtype):
     run_short(c if n_bias < 3 else twice_biased(c), 1, rows=some(rows, 41))
 
 
+@pytest.mark.parametrize("V,top_k,step,allowed", [(50257, 513, 0.0, None), (50257, 1024, 0.0, 0.5), (700, 700, 0.0, None), (1500, 1000, 0.0, None), (50257, 1000, 0.25, None), (50257, 1000, 0.004, None),
+                                                  (262144, 1000, 0.0, 0.1)])
+def test_wide_top_k_without_an_order(V, top_k, step, allowed):
+    """A top-k of more than 512: cuts and draw by buckets - everything listed, more listed than kept, cuts by top-p, by min-p, by both and by neither; logits so
+    coarse that a bucket is too full and the list is sorted after all, and just not so."""
+    rows = rows_of()
+    c = _odd(rows, V, top_k=top_k, n_hist=min(300, V), n_bias=min(20, V), allowed=allowed)
+    if step:
+        c["logits"] = (np.round(c["logits"] / step) * step).astype(np.float32)
+    c["top_p"][::4] = 1.0
+    c["top_p"][1::4] = 0.3
+    c["min_p"][1::3] = 0.02
+    c["min_p"][2::6] = 1.0
+    c["inv_t"][::5] = 0.3
+    run_short(c, 1, rows=some(rows, 23), handed_back=2)
+
+
+# (The rows above are asked for a dump, and so they are sorted. The finish by buckets is for batches that ask for none.)
 WIDE = [(50257, 513, 0.0, None), (50257, 1024, 0.0, 0.5), (700, 700, 0.0, None), (1500, 1000, 0.0, None), (50257, 1000, 0.25, None), (50257, 1000, 0.004, None), (262144, 1000, 0.0, 0.1)]
 
 
@@ -197,11 +215,16 @@ def _wide(rows, V, top_k, step, allowed):
 
 
 @pytest.mark.parametrize("V,top_k,step,allowed", WIDE)
-def test_wide_top_k_without_an_order(V, top_k, step, allowed):
+def test_wide_top_k_by_buckets(V, top_k, step, allowed):
     """A top-k of more than 512 in a batch that asks for no dump, which is when cuts and draw go by buckets: everything listed, more listed than kept, cuts by
     top-p, by min-p, by both and by neither; logits so coarse that a bucket is too full and the list is sorted after all, and just not so."""
     rows = rows_of()
-    run_short(_wide(rows, V, top_k, step, allowed), 1, rows=some(rows, 23), kept_cap=0, handed_back=2)
+    c = _wide(rows, V, top_k, step, allowed)
+    smp = gc.sampler_for(c, gc.upload(c, hints=True), 1, kept_cap=0).run()
+    res = gc.compare_rows(c, smp, some(rows, 23), 1, check_kept=False)
+    m, fl = gc.pkg(), smp.flags.cpu().numpy()
+    short, back = (int(((fl & bit) != 0).sum()) for bit in (m.FLAG_ROUTE_SHORT, m.FLAG_ROUTE_HANDED_BACK))
+    assert res["differ"] == 0 and short + back == rows and back <= 2, (res, short, back)
 
 
 @pytest.mark.parametrize("V,top_k,step,allowed", WIDE)
