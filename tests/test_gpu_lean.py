@@ -432,3 +432,26 @@ def test_rows_whose_cut_no_list_holds(V, masked, n_hist):
     assert (((fl & m.FLAG_ROUTE_EXACT) != 0) <= ((fl & m.FLAG_ROUTE_HANDED_BACK) != 0)).all()
     nk = smp.n_kept.cpu().numpy()
     assert V < 100000 or (nk < 16384).any() and (nk > 16384).any()
+
+
+@pytest.mark.parametrize("V", [50257, 163848, 200003])
+@pytest.mark.parametrize("n_bias,named", [(2047, 2047), (2048, 2048), (3000, 2100)])
+def test_more_bias_entries_than_the_batch_declares(V, n_bias, named):
+    """Bias lists that fit max_hist + max_bias together, most of whose entries name one token, of the history too: it takes all of them, in their order, whatever
+    room the count of a token's entries has in a kernel of those that batches with shorter lists get."""
+    c = _no_top_k(gc.make_cfg2(rows=4, V=V, n_hist=4, n_bias=n_bias))
+    c["inv_t"][:], c["top_p"][:], c["min_p"][:] = 1.0, 0.9, 0.0
+    rng = np.random.default_rng(n_bias)
+    for r in range(4):
+        tok = V - 1 - 7 * r
+        c["hist"][r][0] = tok
+        c["bias_ids"][r, rng.permutation(n_bias)[:named]] = tok
+        c["bias_vals"][r] = np.round(c["bias_vals"][r] * 64) / 65536  # (their sum lifts or lowers the token by some tenths)
+        c["logits"][r, tok] = 7.0
+    d = gc.upload(c, hints=True)
+    d["max_hist"], d["max_bias"], d["min_p_min"] = 2500, 1000, 0.0
+    smp = gc.sampler_for(c, d, 1, max_split=1).run()
+    res = gc.compare_rows(c, smp, range(4), 1, check_kept=False)
+    m, fl = gc.pkg(), smp.flags.cpu().numpy()
+    assert res["differ"] == 0 and ((fl & (m.FLAG_ROUTE_LEAN | m.FLAG_ROUTE_HANDED_BACK)) != 0).all(), (res, fl)
+    assert n_bias > 2047 or ((fl & m.FLAG_ROUTE_LEAN) != 0).all(), fl

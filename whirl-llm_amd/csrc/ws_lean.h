@@ -509,8 +509,9 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const LeanArgPtr ar
     double neg_log_min_p = 0.0;  // wave 15 only (for the select, which has no time for a logarithm)
     if (wv == WS_WAVES - 1u && use_min_p) neg_log_min_p = -log(min_p);
     const uint32_t h0 = P.h0, nh = P.nh, b0 = P.b0, nb = P.nb;
-    // rows this code does not take: a top-k, no filter at all, the race draw, parameters the three-pass code reports
-    if (top_k != 0u || !(use_top_p || use_min_p) || race || !(inv_t > 0.f) || nh + nb > A.patch_cap) WSL_FAIL(1);
+    // rows this code does not take: a top-k, no filter at all, the race draw, parameters the three-pass code reports, more bias entries than the eleven bits
+    // behind the claim's count (a row may have them: only history and bias list together are bounded by the launch's tables)
+    if (top_k != 0u || !(use_top_p || use_min_p) || race || !(inv_t > 0.f) || nh + nb > A.patch_cap || nb > 2047u) WSL_FAIL(1);
 
     const int32_t* hist_ids = A.hist + h0;
     const int32_t* bias_ids = A.bias_ids + b0;
