@@ -121,7 +121,8 @@ __device__ __forceinline__ bool twin_row(const BatchArgs& A, const uint32_t row,
     static_assert(kWords * WS_BLOCK * 32u <= kFewId, "an id of a row that is listed, and none that is 0xffffffff");
     const uint32_t few_room = MASKED ? min(kFew * WS_BLOCK, (early_slots * 8u - kTwinBins * 4u) / 4u) : 0u;
     uint32_t n_few = 0xffffffffu;
-    if (MASKED && n_all) {  // the tokens the mask allows: most rows' are few
+    const bool long_lists = MASKED && n_all > kFew * WS_BLOCK;  // uniform: more entries than the listed ones' rounds take as they are
+    if (long_lists) {  // the tokens the mask allows: most rows' are few
         uint32_t allowed = 0;
 #pragma unroll
         for (uint32_t k = 0; k < kWords; ++k) allowed += k * WS_BLOCK + t < nW ? static_cast<uint32_t>(__popc(aw[k])) : 0u;
@@ -167,9 +168,10 @@ __device__ __forceinline__ bool twin_row(const BatchArgs& A, const uint32_t row,
         };
         // Of a masked row only the entries that its mask allows are gone on with - the mask where the bitmap will be, the entries listed behind the
         // sample's counts, then in registers -, if they are few enough for it. (Nine in ten of 8692 masked out: 17 entries a thread, each looked up in
-        // three passes, were 25 us of a row's 125.)
+        // three passes, were 25 us of a row's 125.) Lists of up to four entries a thread are as fast without: 257 rows of 10496 with 606 ids took 18.7 us and 20.0 by
+        // the list, 700 of 13952 with 32 bias entries 31 and 33.
         bool by_list = false;
-        if (MASKED) {
+        if (long_lists) {
             uint32_t n_allowed = 0;
 #pragma unroll
             for (uint32_t w = 0; w < WS_WAVES; ++w) n_allowed += S.red_u[w];
@@ -241,7 +243,10 @@ __device__ __forceinline__ bool twin_row(const BatchArgs& A, const uint32_t row,
             others([&](uint32_t id, uint32_t) { mark(id); });
             __syncthreads();
             if (MASKED) {
-                for (uint32_t w = t; w < nW; w += WS_BLOCK) touched[w] &= allow[w];
+#pragma unroll
+                for (uint32_t k = 0; k < kWords; ++k)
+                    if (k * WS_BLOCK + t < nW) touched[k * WS_BLOCK + t] &= aw[k];
+                for (uint32_t w = kWords * WS_BLOCK + t; w < nW; w += WS_BLOCK) touched[w] &= allow[w];
                 __syncthreads();
             }
         }
@@ -500,13 +505,13 @@ __device__ __forceinline__ bool twin_row(const BatchArgs& A, const uint32_t row,
 #pragma unroll
             for (uint32_t k = 0; k < N; ++k) {
                 if (j0 + k * WS_BLOCK >= n_of) continue;  // uniform
-                float x = -INFINITY;
+                float x = fmaxf(raw[k], -INFINITY);
+                const bool several = (word[k] & kBiases) != 0u;
+                if ((word[k] & kBias) && !several) x = __fadd_rn(x, bias_vals[j_of(k) - nh]);
+                // (from the first of them; all lanes, which share the search: the few with an allowed token alone took 5 us)
+                if (__ballot(several)) x = add_other_bias(several, id_of(k), 0xffffffffu, x, bias_ids, bias_vals, nb);
                 if (word[k]) {
                     const uint32_t c = word[k] & (kBias - 1u);
-                    x = fmaxf(raw[k], -INFINITY);
-                    const bool several = (word[k] & kBiases) != 0u;
-                    if ((word[k] & kBias) && !several) x = __fadd_rn(x, bias_vals[j_of(k) - nh]);
-                    if (__ballot(several)) x = add_other_bias(several, id_of(k), 0xffffffffu, x, bias_ids, bias_vals, nb);  // (from the first of them)
                     if (c) {
                         x = x > 0.f ? __fdiv_rn(x, P.rep) : __fmul_rn(x, P.rep);
                         x = __fsub_rn(x, __fadd_rn(__fmul_rn(P.freq, static_cast<float>(c)), P.pres));
