@@ -298,3 +298,39 @@ def test_top_k_rows_whose_list_just_fits(V, n_hist):
     sampled = np.arange(rows) // 10 % 3 != 1
     assert not back[(listed <= 4096) & sampled].any(), listed[back & (listed <= 4096) & sampled]
     assert back[listed > 4096].all()
+
+
+@pytest.mark.parametrize("V,dtype,n_hist", [(16384, "f32", 0), (20483, "f32", 40), (50260, "f32", 700), (33001, "bf16", 0), (12289, "bf16", 64)])
+def test_lists_of_few_places(V, dtype, n_hist):
+    """Rows whose list takes up to 512 places, a few more or many more, by a min-p alone or a small top-k: tokens spread over the row, in one wave's share of every
+    chunk, in one vector, in the tokens behind the last vector."""
+    rows = rows_of()
+    c = _odd(rows, V, top_k=0, n_hist=max(n_hist, 1), n_bias=0)
+    c["bias_ids"] = c["bias_vals"] = None
+    if not n_hist:
+        c["hist"] = None
+    rng = np.random.default_rng(V)
+    x = (rng.standard_normal((rows, V), dtype=np.float32) - 30).astype(np.float32)
+    c["inv_t"][:], c["top_p"][:], c["min_p"][:] = 1.0, 0.95, 0.05
+    listed = np.array([1, 2, 8, 31, 32, 33, 63, 64, 65, 127, 129, 250, 256, 257, 300, 400, 480, 511, 513, 700])[np.arange(rows) % 20]
+    for r in range(rows):
+        kind = r // 20 % 4
+        if kind == 0:
+            at = rng.permutation(V)[:listed[r]]
+        elif kind == 1:
+            at = np.flatnonzero(np.arange(V) % 2048 < 256)
+            at = at[rng.permutation(at.size)[:listed[r]]]
+        elif kind == 2:
+            at = rng.integers(0, V - listed[r]) + np.arange(listed[r])
+        else:
+            at = V - 1 - np.arange(listed[r])
+        if n_hist:
+            c["hist"][r][:min(5, at.size)] = at[:5]  # (a few of them touched)
+        x[r, at] = 4.0 + rng.uniform(0.0, 2.5, at.size).astype(np.float32)
+    c["logits"] = x
+    if dtype == "bf16":
+        c["logits"], c["dtype"] = gc.f32_to_bf16_bits(x), "bf16"
+    run_short(c, 1, rows=some(rows, 3), handed_back=1)
+    c["top_k"][:] = 8
+    c["min_p"][:] = 0.0
+    run_short(c, 1, rows=some(rows, 7), handed_back=1)

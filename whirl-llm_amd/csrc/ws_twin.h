@@ -27,6 +27,7 @@
 namespace ws {
 
 constexpr uint32_t kTwinHead = 8u;  // vectors a thread of the sample that the threshold is fitted to
+constexpr uint32_t kTwinEmpty = 0xffffffffu;  // in the place of an id
 constexpr uint32_t kTwinPlaces = 32u;  // places of the list a wave takes at a time, where the list has kTwinSpare places more than the tokens it may hold
 static_assert((kTwinPlaces - 1u) * WS_WAVES <= kTwinSpare && kTwinSpare <= 64u * WS_WAVES, "room for the places that are taken and not filled; a thread each to close them");
 
@@ -304,6 +305,7 @@ __device__ __forceinline__ bool twin_row(const BatchArgs& A, const uint32_t row,
     if (MASKED || n_all) {
 #pragma unroll
         for (uint32_t k = 0; k < kTwinHead; ++k) {
+            if (k * spread * WS_BLOCK >= nv) break;  // uniform
             const uint32_t i0 = min(k * spread * WS_BLOCK + t, nv - 1u) * TPV;
             uint32_t invalid = 0u;  // bit e: token e does not count here
             if (MASKED) invalid = ~(hna[k] >> (i0 & 31u));
@@ -652,17 +654,22 @@ __device__ __forceinline__ bool twin_row(const BatchArgs& A, const uint32_t row,
     if (lane == 0u) atomicMax(reinterpret_cast<int*>(&S.marks[13]), __float_as_int(static_cast<float>(clock64() - wss_t0)));  // the slowest wave's
 #endif
     double z;  // the sum against `ref`
+    uint64_t my_token;  // what lies at the thread's own place of the list
+    uint32_t n_list, no_room;
     {          // the block's maximum and sum with one barrier between them
         const float wm_ = wave_max(m);
         const double ws_ = wave_sum(static_cast<double>(s0) + static_cast<double>(s1));
-        __syncthreads();
-        if (lane == 0u) {
+        if (lane < my_end - my_next) reinterpret_cast<uint32_t*>(list)[2u * (my_next + lane)] = kTwinEmpty;
+        if (lane == 0u) {  // (words that nobody has looked at since the threshold's barriers)
             S.red_f[wv] = wm_;
             S.red_d[wv] = ws_;
             S.bstart[wv] = my_next;
             S.bcnt[wv] = my_end - my_next;
         }
         __syncthreads();
+        my_token = list[t];
+        n_list = S.s_w[1];
+        no_room = S.s_w[2];
         m = S.red_f[0];
         z = S.red_d[0];
 #pragma unroll
@@ -672,8 +679,28 @@ __device__ __forceinline__ bool twin_row(const BatchArgs& A, const uint32_t row,
         }
     }
     WSS_MARK(5);
-    uint32_t n_list = S.s_w[1], n_left = 0;
-    {  // the places no wave has filled: the last n_left of the list take their contents to the others
+    auto as_key = [](uint64_t token) __attribute__((always_inline)) { return key64(__uint_as_float(static_cast<uint32_t>(token >> 32)), static_cast<uint32_t>(token)); };
+    // Few places, most of them empty as a rule (a confident row's, with a min-p alone): a place a thread, and what is filled moves up, as a key. (us, a place a token / the
+    // way below / this: 300 rows of 10292, Zipfian, min-p 0.03, 13.5 / 14.4 / 14.0; 512 bf16 rows of 12452 with 34 ids 16.6 / 18.9 / 17.8; 400 of 16320 14.5 / 16.2 / 15.7. Places taken one at
+    // a time at first, or moved by the wave that has filled them: slower where lists are longer, 400 of 35044 39.3 / 41.4.)
+    const bool few_places = n_list <= WS_BLOCK;  // uniform
+    if (few_places) {
+        const bool filled = t < n_list && static_cast<uint32_t>(my_token) != kTwinEmpty;
+        const uint64_t on = __ballot(filled);
+        if (lane == 0u) S.red_u[wv] = static_cast<uint32_t>(__popcll(on));
+        __syncthreads();
+        uint32_t at = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(on >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(on), 0u));
+        n_list = 0;
+#pragma unroll
+        for (uint32_t w = 0; w < WS_WAVES; ++w) {
+            const uint32_t n = S.red_u[w];
+            at += w < wv ? n : 0u;
+            n_list += n;
+        }
+        if (filled) list[at] = as_key(my_token);
+        __syncthreads();
+    } else {  // the places no wave has filled: the last n_left of the list take their contents to the others
+        uint32_t n_left = 0;
 #pragma unroll
         for (uint32_t w = 0; w < WS_WAVES; ++w) n_left += S.bcnt[w];
         if (n_list <= kShortCap + spare && n_left) {  // uniform
@@ -734,9 +761,11 @@ __device__ __forceinline__ bool twin_row(const BatchArgs& A, const uint32_t row,
         n_list = S.s_w[1];
     }
     const uint32_t n_cand = by_k ? top_k : n_list;  // candidates the rules look at
-    if (S.s_w[2] != 0u || n_list > kShortCap || !(m > -INFINITY) || !(__fsub_rn(m, ref) * inv_t < 80.f) || n_list < n_cand || n_cand == 0u) return false;
-    for (uint32_t k = t; k < n_list; k += WS_BLOCK) list[k] = key64(__uint_as_float(static_cast<uint32_t>(list[k] >> 32)), static_cast<uint32_t>(list[k]));
-    if (n_list <= WS_BLOCK / 4u) __syncthreads();  // (the sort of a short list begins with other threads' keys; a longer list's with a thread's own)
+    if (no_room != 0u || n_list > kShortCap || !(m > -INFINITY) || !(__fsub_rn(m, ref) * inv_t < 80.f) || n_list < n_cand || n_cand == 0u) return false;
+    if (!few_places) {  // uniform
+        for (uint32_t k = t; k < n_list; k += WS_BLOCK) list[k] = as_key(list[k]);
+        if (n_list <= WS_BLOCK / 4u) __syncthreads();  // (the sort of a short list begins with other threads' keys; a longer list's with a thread's own)
+    }
     float inv_t_ = inv_t;
     asm volatile("" : "+v"(inv_t_));  // (so that its 64-bit value does not wait in registers from the sweep on)
     // Tokens above `ref` can be most of the sum, and the larger the exponent, the less of a fraction 32 bits leave it (1.2e-6 of
@@ -750,15 +779,18 @@ __device__ __forceinline__ bool twin_row(const BatchArgs& A, const uint32_t row,
         }
         z += block_sum(more, S.red_d);
     }
-    ShortRow R;
-    R.top_p = top_p;
-    R.min_p = min_p;
-    R.u = batch_uniform(A.rng, P.seed, row, P.step, 0);
-    R.z = z * exp((static_cast<double>(ref) - static_cast<double>(m)) * static_cast<double>(inv_t_));
-    R.inv_t = inv_t_;
-    R.m = m;
-    R.n_cand = n_cand;
-    R.by_k = by_k;
+    auto rules_of = [&]() __attribute__((always_inline)) {
+        ShortRow R;
+        R.top_p = top_p;
+        R.min_p = min_p;
+        R.u = batch_uniform(A.rng, P.seed, row, P.step, 0);
+        R.z = z * exp((static_cast<double>(ref) - static_cast<double>(m)) * static_cast<double>(inv_t_));
+        R.inv_t = inv_t_;
+        R.m = m;
+        R.n_cand = n_cand;
+        R.by_k = by_k;
+        return R;
+    };
     // A wide top-k, two candidates a thread and more: its cuts and draw without an order (us, with the sort and without, top-k 1000: 1024 masked rows of 262144 248 / 243, 300
     // of 262144 91.9 / 88.6, 512 of 151936 74.6 / 71.2, 1000 of 32000 67.9 / 63.7; level at a top-k of 100 to 500, and rows with a min-p alone, whose keys crowd at the floor, slower: 86.7 / 95.4).
     // Rows with a bucket too full for it are sorted after all: of fp32 logits that were bf16 once 512 rows of 151936, nearly all of which have one, take 84.9 / 85.8, 300 of 262144,
@@ -766,10 +798,10 @@ __device__ __forceinline__ bool twin_row(const BatchArgs& A, const uint32_t row,
     ShortSpan span;
     const LeanArgPtr Ap = (LeanArgPtr)__builtin_amdgcn_kernarg_segment_ptr();
     if (DT == 0 && by_k && n_cand > WS_BLOCK && n_list <= kShortCap - 1024u && !Ap->kept_ids && !Ap->entropy && !Ap->query_prob) {  // uniform
+        const ShortRow R = rules_of();
         if (t == 0u) S.s_d[7] = R.z;
         __syncthreads();  // (the words that say which places were left over have been read as well)
         if (short_pick(list, n_list, row, R, S, span)) return true;
-        R.z = S.s_d[7];
         __syncthreads();
     }
     short_sort(list, n_list, m, S, span);
@@ -778,7 +810,7 @@ __device__ __forceinline__ bool twin_row(const BatchArgs& A, const uint32_t row,
     // threshold lies below its floor by construction
     const float x_k = unkey32(static_cast<uint32_t>(list[n_cand - 1u] >> 32));
     if ((by_k && !(x_k > thr)) || !(x_k > -INFINITY)) return false;
-    short_rules(list, row, R, S);
+    short_rules(list, row, rules_of(), S);
 #ifdef WS_SHORT_TIMERS
     WSS_MARK(8);
     __syncthreads();
