@@ -420,9 +420,9 @@ struct LeanShared {
 #ifdef WS_PHASE_TIMERS
 __device__ __forceinline__ double sel_dbg(const LeanShared& S) { return S.sel.n_r0 + 1e5 * S.sel.n_r1 + 1e10 * (S.sel.r0hi - S.sel.r0lo + 1) + 1e12 * (S.sel.r1hi - S.sel.r1lo + 1); }
 #endif
-// One row. Returns false when the row is left to others (nothing has been written for it then): S.top is NaN, and it is the three-pass code's; or infinite, and the exact
-// path is to answer it (the touched tokens' tables are where that looks for them); or the row's maximum, and it is to be swept once more from there down (AGAIN; its
-// arguments are at `args`).
+// One row. Returns false when the row is left to others (nothing has been written for it then): S.top is NaN, and it is the three-pass code's; or infinite, and its cut or its
+// draw lies among tokens that the list does not take (the touched tokens' tables are where the exact path looks for them); or the row's maximum, and it is to be swept once
+// more from there down (AGAIN; its arguments are at `args`).
 template <bool MASKED, bool AGAIN, int NREG>
 __device__ __forceinline__ bool lean_row(const BatchArgs& A, const LeanArgPtr args, const uint32_t row, LeanShared& S) {
     constexpr uint32_t kTok = 4u, kTokLog = 2u;  // tokens in a 128-bit vector, which is one register of the bin cache: the low eight bits of each bin
@@ -509,9 +509,10 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const LeanArgPtr ar
     double neg_log_min_p = 0.0;  // wave 15 only (for the select, which has no time for a logarithm)
     if (wv == WS_WAVES - 1u && use_min_p) neg_log_min_p = -log(min_p);
     const uint32_t h0 = P.h0, nh = P.nh, b0 = P.b0, nb = P.nb;
-    // rows this code does not take: a top-k, no filter at all, the race draw, parameters the three-pass code reports, more bias entries than the eleven bits
-    // behind the claim's count (a row may have them: only history and bias list together are bounded by the launch's tables)
-    if (top_k != 0u || !(use_top_p || use_min_p) || race || !(inv_t > 0.f) || nh + nb > A.patch_cap || nb > 2047u) WSL_FAIL(1);
+    // Rows this code does not take: a top-k, no filter at all, the race draw, parameters the three-pass code reports; and more than 2047 bias entries, which a row may have -
+    // only history and bias list together are bounded by the launch's tables - and which the eleven bits below a claim's do not count. (As a condition of its own that
+    // one made the masked build of 38 registers spill 17, 3 to 8 % of its rows' time.)
+    if ((top_k | (nb >> 11)) != 0u || !(use_top_p || use_min_p) || race || !(inv_t > 0.f) || nh + nb > A.patch_cap) WSL_FAIL(1);
 
     const int32_t* hist_ids = A.hist + h0;
     const int32_t* bias_ids = A.bias_ids + b0;
@@ -922,7 +923,12 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const LeanArgPtr ar
             rm += ms[k];
         }
         me[4] = base_m + im;  // (what the next thread starts from, bit for bit)
-        if (t == WS_BLOCK - 1u) me[4] = Z;
+        if (t == WS_BLOCK - 1u) {
+            me[4] = Z;
+            S.m_left = m;  // (for lean_rest; written here, where they are at hand: on the way out they cost the longest build registers)
+            S.z_left = Z;
+            S.touched_left = n_touched;
+        }
     }
     WSL_MARK(4);
     const double Zf = static_cast<double>(static_cast<float>(Z));  // Sampler::sum is a float (src/sampling/sampler.h:38)
@@ -1159,20 +1165,8 @@ __device__ __forceinline__ bool lean_row(const BatchArgs& A, const LeanArgPtr ar
         }
     }
     __syncthreads();
-    if (!sel.ok) {
-        // Tied or flat rows. The three-pass code would count the row once more, to find that its list does not hold the tokens either: its bins lie elsewhere, but what
-        // one bin has too many of it has as well, and half as many again of several bins are taken to be too many for both.
-        const BinRec dlo = found(2u), dhi = found(3u);
-        BinRec cut = found(0u);
-        if (cut.b != 0xffffffffu && cut.cex >= 16384u) cut = found(1u);
-        const uint32_t most = max(max(dlo.c, dhi.c), sel.topp_in_list ? cut.c : 0u);
-        if (dlo.b == 0xffffffffu || dhi.b == 0xffffffffu || dhi.b < dlo.b || sel.r0hi >= kLeanTail || (most <= kLeanMaxList && sel.n_r0 + sel.n_r1 <= kLeanMaxList + kLeanMaxList / 2u)) WSL_FAIL(5);
-        if (t == 0u) {
-            S.top = INFINITY;
-            S.m_left = m;
-            S.touched_left = n_touched;
-            S.z_left = Z;
-        }
+    if (!sel.ok) {  // (what follows from it is worked out by lean_rest, for the same reason)
+        if (t == 0u) S.top = INFINITY;
         return false;
     }
     const int r0lo = sel.r0lo, r0hi = sel.r0hi, r1lo = sel.r1lo, r1hi = sel.r1hi;
@@ -1700,7 +1694,33 @@ __device__ __noinline__ __attribute__((not_tail_called)) void lean_rest(LeanArgP
         __syncthreads();
         top = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(S->top)));
     }
-    if (top == INFINITY) exact_left_row(Ap, row, S);
+    bool ties = top == INFINITY;  // uniform
+    if (ties) {
+        // Tied or flat rows. The three-pass code would count the row once more, to find that its list does not hold the tokens either: its bins lie elsewhere, but what
+        // one bin has too many of it has as well, and half as many again of several bins are taken to be too many for both.
+        auto found = [&](uint32_t search) {  // the first wave's record that holds a bin
+            LeanBinRec r;
+            r.b = 0xffffffffu;
+            r.c = 0u;
+            r.cex = 0u;
+            for (uint32_t w = 0; w < WS_WAVES && r.b == 0xffffffffu; ++w) {
+                r.b = S->rec[search * WS_WAVES + w].b;
+                r.cex = S->rec[search * WS_WAVES + w].cex;
+                r.c = S->rec[search * WS_WAVES + w].c;
+            }
+            return r;
+        };
+        const LeanBinRec dlo = found(2u), dhi = found(3u);
+        uint32_t most = max(dlo.c, dhi.c);
+        if (S->sel.topp_in_list) {
+            LeanBinRec cut = found(0u);
+            if (cut.b != 0xffffffffu && cut.cex >= 16384u) cut = found(1u);
+            if (cut.b != 0xffffffffu) most = max(most, cut.c);
+        }
+        ties = dlo.b != 0xffffffffu && dhi.b != 0xffffffffu && dhi.b >= dlo.b && S->sel.r0hi < kLeanTail && (most > kLeanMaxList || S->sel.n_r0 + S->sel.n_r1 > kLeanMaxList + kLeanMaxList / 2u);
+        ties = __builtin_amdgcn_readfirstlane(ties ? 1 : 0) != 0;
+    }
+    if (ties) exact_left_row(Ap, row, S);
     else three_pass_row<false>(Ap, row);
 }
 
