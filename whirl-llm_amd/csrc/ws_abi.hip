@@ -344,22 +344,22 @@ BatchPlan plan_batch(const ws_batch* b, bool few = true) {
 #endif
     // Its rows are those without a top-k, and a batch says so by leaving `top_k` out: a row with one would be handed
     // back to the three-pass code inside the launch, at twice the time of the kernel that takes a top-k in its stride.
-    // It reads rows at any address. Rows that are not whole aligned vectors, which the other single-sweep kernels do not take, are swept three times otherwise, and
-    // that is the faster way only for short ones (us, three sweeps and this kernel; N(0, 2) and rows of raised tokens):
-    //   without lists, 1 row:  of 9001 17.6 / 19.4, 16387 19.1 / 19.5, 20011 21.0 / 19.6 and 19.7 / 19.7, 50257 28.7 / 22.0, 151937 49.1 / 32.1
-    //                256 rows: of 9001 19.7 / 20.3, 16387 23.3 / 20.7 and 21.7 / 20.7, 50257 37.9 / 25.2, 151937 67.1 / 40.0
-    //     masked,      1 row:  of 20011 21.1 / 22.4, 32003 23.5 / 23.0 and 23.0 / 23.9;  256 rows of 20011 24.0 / 26.3, 32003 29.5 / 25.4
-    //   with histories of 16 to 3400 ids: 1 row of 9001 22.2 / 22.2 and 21.3 / 22.0, 50257 38.7 / 24.5; 256 rows of 8003 27.0 / 23.0, 151937 77.9 / 42.8
-    //     masked too (180 shapes): 8192 to 12000 tokens 5 % slower here, to 16000 2 %, from there on faster, 27 % of the longest
-    //     raised tokens, 16 ids: 1 row of 8193 21.5 / 22.6, 14003 22.2 / 22.5, 16387 22.9 / 22.5; 256 rows of 9001 23.7 / 24.3, 16387 level; 64 ids: 1 row of 8193 21.6 / 22.5,
-    //     12001 22.3 / 22.6, 16387 23.5 / 22.7; 256 ids: 1 row of 8193 23.3 / 22.7
-    //     masked, 64 ids: 1 row of 8193 22.9 / 24.8, 12001 23.7 / 25.4, 16387 24.8 / 25.7, 24001 27.8 / 25.7; 256 rows of 8193 24.7 / 27.6, 16387 28.8 / 27.4; 500 ids: level at 8193
+    // It reads rows at any address. Rows that are not whole aligned vectors, which the other single-sweep kernels do not take, are swept three times otherwise, and short ones are. The
+    // lines below were drawn when the one build of this kernel asked for 163840 tokens of every row; since there are builds for short rows it would be the faster way from
+    // some 8000 tokens on, and with lists from 2000. (us, three sweeps and this kernel, N(0, 2) and rows of raised tokens, top-p 0.9. The lines stand: which way rows of these
+    // lengths go is held to the token by a test.)
+    //   without lists, 1 row:    of 2051 15.6 / 16.2, 8195 16.5 / 16.4, 16387 17.9 / 16.7, 20011 19.3 / 17.0;  256 rows: of 2051 17.7 / 16.7, 8195 19.0 / 16.8, 16387 22.6 / 17.0, 20011 23.7 / 17.3
+    //           masked, 1 row:   of 2051 16.5 / 18.0, 8195 17.7 / 18.1, 12001 18.6 / 18.0, 32003 22.6 / 18.0;  256 rows: of 6001 19.2 / 20.3, 8195 19.8 / 19.2, 32003 29.3 / 21.0
+    //   16 and 64 ids, 1 row:    of 2051 19.4 / 17.9, 12001 21.5 / 18.2;  256 rows: of 2051 22.0 / 18.8, 12001 24.3 / 18.6
+    //           masked, 1 row:   of 2051 20.1 / 20.0, 20011 24.9 / 20.1;  256 rows: of 4099 22.7 / 22.7, 6001 23.1 / 21.7, 20011 28.6 / 23.3
+    //   500 ids, 1 row:          of 2051 21.7 / 17.9, 6001 22.3 / 18.1;  256 rows: of 2051 25.7 / 18.5, 6001 25.9 / 18.5;  masked: 256 rows of 2051 26.4 / 22.4, 20011 30.7 / 23.5
+    //   longer rows (with the build of 163840): 1 row of 50257 28.7 / 22.0, with ids 38.7 / 24.5, of 151937 49.1 / 32.1; 256 rows of 50257 37.9 / 25.2, of 151937 67.1 / 40.0, with ids 77.9 / 42.8
     // Rows without a filter are none of its own either: of a batch that has neither top-p nor min-p it would hand back every one (three sweeps and this kernel: 1 row of
     // 50257 40 / 44, 256 rows 51 / 61, 256 of 151937 with 500 ids 117 / 125; the other single-sweep kernel and this one: 256 rows of 50256 52 / 61, of 151936 87 / 109).
     // Rows of 163841 to 262144 tokens, which no other single-sweep kernel takes, have their build of it with the longer bin cache (us, three sweeps and this; top-p 0.9):
     //   1 row of 262144 69 / 47, 64 of 200000 with 500 ids 84 / 53, 32 of 163841 65 / 42, 256 of 262144 with 2000 ids 128 / 93, 200 Zipfian of 262144 with 3000 135 / 93, 100 of
     //   200000 65 / 50; raised tokens: 16 of 256000 114 / 53, 256 of 163848 with 64 ids 83 / 67; masked: 88 of 248576, 17 % allowed, 94 / 58, 281 of 204976, 15 %, 150 / 119
-    //   Rows whose cut no list holds are handed back after a sweep in vain: 200 flat Zipfian rows of 262144, T up to 1.4, 845 / 891.
+    //   Rows whose cut no list holds are swept in vain, and go on to the exact path from there: 200 flat Zipfian rows of 262144, T up to 1.4, 845 / 675; 64 of 262144 in steps of 0.5 954 / 947.
     const uint32_t lean_least = vec_rows ? 8u : (cap >= (b->allow ? 512u : 128u) ? 8192u : (cap ? (b->allow ? 20480u : 16384u) : (b->allow ? 32768u : 20480u)));
     p.lean = (p.fused || !vec_rows || b->vocab > 163840u) && (b->top_p || b->min_p) && b->dtype == WS_DTYPE_F32 && b->mode == WS_MODE_AUTO && !b->top_k && !b->kept_ids && !b->query_prob && !wants_entropy && !b->race &&
              b->vocab >= lean_least && b->vocab <= 262144u && (!b->bias_ids || b->max_bias <= 2047u) && fused_total + kStaticLean <= kMaxLds;

@@ -32,8 +32,10 @@ namespace ws {
 // Registers of the bin cache a thread, four tokens each: builds for rows of up to 32768, 49152, 65536, 98304, 155648, 163840 and 262144
 // tokens, and a row gets the shortest that holds it. The loads past a row's end are asked for like the others - they may not lie behind a branch -, 64
 // lanes at one address each: a row of 25000 tokens waited 8 K clocks of 46 K for them in the build of 40 (us, that one and its own: 54 rows of 25792 20.1 / 17.3, 34 of
-// 35392 24.3 / 20.5, 256 of 32000 with 1000 ids 26.5 / 21.6, 200 of 50257 27.9 / 24.3, 100 of 98304 30.9 / 29.0). Of the longest a quarter of the cache lies in scratch
-// memory behind the sweep, which is still far from the two more sweeps that such rows took (ws_abi.hip).
+// 35392 24.3 / 20.5, 256 of 32000 with 1000 ids 26.5 / 21.6, 200 of 50257 27.9 / 24.3, 100 of 98304 30.9 / 29.0). The longest, of whose 128 registers the cache and a scan's finds are 96,
+// spills 71 (masked 73), still far from the two more sweeps that such rows took (ws_abi.hip); the masked one of 8, whose batches are all early ones, spills 17.
+// The classes of the longer rows lie closer together than what a launch varies by (256 rows, the build of 38 and the next one: of 151936 40.5 / 41.1, of 140000 level; against one of 32, which
+// there is not: of 98312 31.8 / 30.7, of 120000 34.6 / 33.6, of 131072 38.7 / 36.0, masked 38.0 / 40.6).
 constexpr int kLeanRegs[] = {8, 12, 16, 24, 38, 40, 64};
 constexpr int kLeanLooks = 64;  // from here on finds are looked at before they are listed, when they are too many
 constexpr int kLeanBatch = 2;   // 128-bit loads per thread and batch
