@@ -34,11 +34,11 @@ KEPT_CAP = 0  # entries a row of the kept-set dump (--kept-cap), 0: no dump
 # of the kernel sources the counters were taken with), otherwise null. File names are relative to profiles/.
 TRAFFIC = {
     # (workload, mode): (bytes per launch, profiles/ file, kernel_digest() at the time)
-    ("tile", "auto"): (205094664, "lean_batch_kernel_tile_256x151936_f32.txt", "857feb9f3972c3f6"),
-    ("cfg1", "auto"): (791881, "few_batch_kernel_cfg1_1x151936_f32.txt", "857feb9f3972c3f6"),
-    ("cfg2", "auto"): (49988725, "few_batch_kernel_cfg2_64x151936_f32.txt", "857feb9f3972c3f6"),
-    ("cfg3", "auto"): (113244996, "code_batch_kernel_cfg3_256x151936_bf16.txt", "857feb9f3972c3f6"),
-    ("cfg5", "auto"): (1286183907, "twin_batch_kernel_cfg5_1024x262144_f32.txt", "857feb9f3972c3f6"),
+    ("tile", "auto"): (205064514, "lean_batch_kernel_tile_256x151936_f32.txt", "be97aea6c77f29a0"),
+    ("cfg1", "auto"): (790915, "few_batch_kernel_cfg1_1x151936_f32.txt", "be97aea6c77f29a0"),
+    ("cfg2", "auto"): (49993829, "few_batch_kernel_cfg2_64x151936_f32.txt", "be97aea6c77f29a0"),
+    ("cfg3", "auto"): (113042427, "code_batch_kernel_cfg3_256x151936_bf16.txt", "be97aea6c77f29a0"),
+    ("cfg5", "auto"): (1286253971, "twin_batch_kernel_cfg5_1024x262144_f32.txt", "be97aea6c77f29a0"),
 }
 
 
