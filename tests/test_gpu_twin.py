@@ -334,3 +334,14 @@ def test_lists_of_few_places(V, dtype, n_hist):
     c["top_k"][:] = 8
     c["min_p"][:] = 0.0
     run_short(c, 1, rows=some(rows, 7), handed_back=1)
+
+
+@pytest.mark.parametrize("n_hist,n_bias", [(2040, 8), (2040, 9), (1, 2047), (2, 2047), (2048, 0), (2049, 0)])
+@pytest.mark.parametrize("V,allowed,dtype", [(9792, 0.05, "f32"), (50257, 0.3, "bf16")])
+def test_masked_rows_at_the_length_from_which_allowed_entries_are_listed(V, allowed, dtype, n_hist, n_bias):
+    """Lists of 2048 entries and of one more, with tokens that several bias entries name."""
+    rows = rows_of()
+    c = _odd(rows, V, dtype, top_k=30, n_hist=n_hist, n_bias=n_bias, allowed=allowed)
+    if not n_bias:
+        c["bias_ids"] = c["bias_vals"] = None
+    run_short(c if n_bias < 3 else twice_biased(c), 1, rows=some(rows, 41), handed_back=1)
